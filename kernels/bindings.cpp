@@ -16,11 +16,11 @@ void launch_fused_add_rms_norm(T*, T*, const T*, float, int, int, hipStream_t);
 template <typename T>
 void launch_silu_and_mul(T*, const T*, int, int, hipStream_t);
 template <typename T>
-void launch_rotary_embedding(const long*, T*, T*, const float*, int, int, int,
-                             int, hipStream_t);
+void launch_rotary_embedding(const long*, T*, const T*, T*, const float*, int, int,
+                             int, int, long, long, hipStream_t);
 template <typename T>
 void launch_reshape_and_cache(const T*, const T*, T*, T*, const long*, int,
-                              int, hipStream_t);
+                              int, long, long, hipStream_t);
 template <typename T>
 void launch_paged_decode(T*, const T*, const T*, const T*, const int*,
                          const int*, float, int, int, int, int, int, int,
@@ -64,8 +64,8 @@ void launch_paged_prefill_mfma_v2_fp8(__hip_bfloat16*, const __hip_bfloat16*,
                                       int, int, int, int, int, hipStream_t);
 void launch_reshape_and_cache_fp8(const __hip_bfloat16*,
                                   const __hip_bfloat16*, unsigned char*,
-                                  unsigned char*, const long*, int, int,
-                                  hipStream_t);
+                                  unsigned char*, const long*, int, int, long,
+                                  long, hipStream_t);
 void launch_gemm_skinny_q(__hip_bfloat16*, float*, const __hip_bfloat16*,
                           const unsigned char*, const float*, int, int, int,
                           int, int, hipStream_t);
@@ -168,7 +168,18 @@ void silu_and_mul(torch::Tensor out, torch::Tensor x) {
   });
 }
 
-void rotary_embedding(torch::Tensor positions, torch::Tensor q,
+// Elements between the starts of a [rows, ...] tensor's rows, whose own elements
+// are dense.
+int64_t row_stride(const torch::Tensor& t, const char* name) {
+  int64_t want = 1;
+  for (int64_t d = t.dim() - 1; d > 0; --d) {
+    TORCH_CHECK(t.size(d) == 1 || t.stride(d) == want, name, ": rows must be dense");
+    want *= t.size(d);
+  }
+  return t.size(0) > 1 ? t.stride(0) : want;
+}
+
+void rotary_embedding(torch::Tensor positions, torch::Tensor q_out, torch::Tensor q,
                       torch::Tensor k, int64_t head_dim,
                       torch::Tensor cos_sin_cache) {
   const int tokens = positions.size(0);
@@ -176,11 +187,15 @@ void rotary_embedding(torch::Tensor positions, torch::Tensor q,
   const int nk = k.size(-1) / head_dim;
   TORCH_CHECK(positions.scalar_type() == at::ScalarType::Long);
   TORCH_CHECK(cos_sin_cache.scalar_type() == at::ScalarType::Float);
+  TORCH_CHECK(q.dim() == 2 && k.dim() == 2 && q.size(0) == tokens && k.size(0) == tokens,
+              "q and k must be [tokens, heads * head_dim]");
+  TORCH_CHECK(q_out.is_contiguous() && q_out.sizes() == q.sizes() &&
+              q_out.scalar_type() == q.scalar_type() && k.scalar_type() == q.scalar_type());
   DISPATCH_FLOATING(q.scalar_type(), {
     launch_rotary_embedding<scalar_t>(
-        positions.data_ptr<long>(), ptr<scalar_t>(q), ptr<scalar_t>(k),
-        cos_sin_cache.data_ptr<float>(), tokens, nq, nk, (int)head_dim,
-        current_stream());
+        positions.data_ptr<long>(), ptr<scalar_t>(q_out), cptr<scalar_t>(q),
+        ptr<scalar_t>(k), cos_sin_cache.data_ptr<float>(), tokens, nq, nk, (int)head_dim,
+        row_stride(q, "q"), row_stride(k, "k"), current_stream());
   });
 }
 
@@ -189,6 +204,15 @@ void reshape_and_cache(torch::Tensor k, torch::Tensor v, torch::Tensor k_cache,
   const int tokens = k.size(0);
   const int row_elems = k_cache.size(2) * k_cache.size(3);
   TORCH_CHECK(slot_mapping.scalar_type() == at::ScalarType::Long);
+  // the copies are 16 bytes wide
+  const int64_t wide = 16 / k.element_size();
+  auto lined_up = [&](const torch::Tensor& t) {
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 &&
+           (t.size(0) <= 1 || t.stride(0) % wide == 0);
+  };
+  if (!lined_up(k)) k = k.contiguous();
+  if (!lined_up(v)) v = v.contiguous();
+  const int64_t ks = row_stride(k, "k"), vs = row_stride(v, "v");
   if (k_cache.scalar_type() == at::ScalarType::Byte) {
     TORCH_CHECK(k.scalar_type() == at::ScalarType::BFloat16,
                 "fp8 KV cache takes bf16 K/V inputs");
@@ -198,14 +222,14 @@ void reshape_and_cache(torch::Tensor k, torch::Tensor v, torch::Tensor k_cache,
         reinterpret_cast<const __hip_bfloat16*>(v.data_ptr()),
         reinterpret_cast<unsigned char*>(k_cache.data_ptr()),
         reinterpret_cast<unsigned char*>(v_cache.data_ptr()),
-        slot_mapping.data_ptr<long>(), tokens, row_elems, current_stream());
+        slot_mapping.data_ptr<long>(), tokens, row_elems, ks, vs, current_stream());
     return;
   }
   DISPATCH_FLOATING(k.scalar_type(), {
     launch_reshape_and_cache<scalar_t>(
         cptr<scalar_t>(k), cptr<scalar_t>(v), ptr<scalar_t>(k_cache),
         ptr<scalar_t>(v_cache), slot_mapping.data_ptr<long>(), tokens,
-        row_elems, current_stream());
+        row_elems, ks, vs, current_stream());
   });
 }
 
@@ -460,7 +484,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fused_add_rms_norm", &fused_add_rms_norm,
         "in-place residual-add + RMSNorm (CDNA4)");
   m.def("silu_and_mul", &silu_and_mul, "SwiGLU activation (CDNA4)");
-  m.def("rotary_embedding", &rotary_embedding, "NeoX rotary, in place (CDNA4)");
+  m.def("rotary_embedding", &rotary_embedding, "NeoX rotary: q into dense rows, k in place (CDNA4)");
   m.def("reshape_and_cache", &reshape_and_cache, "paged KV cache write (CDNA4)");
   register_attention_ops(m);
   m.def("xar_alloc", &xar_alloc,

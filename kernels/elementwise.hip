@@ -40,7 +40,9 @@ void launch_silu_and_mul(T* out, const T* x, int rows, int d, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------------------
-// NeoX rotary embedding, in place on q and k.
+// NeoX rotary embedding: q into q_out (dense rows, may be q itself), k in place.
+// Rows of q and k may lie further apart than they are long (column slices of one
+// projection).
 // cos_sin_cache: [max_pos, head_dim] f32, first half cos, second half sin.
 // One block per token; threads cover (head, i<half) pairs for q then k.
 // ---------------------------------------------------------------------------
@@ -48,44 +50,48 @@ void launch_silu_and_mul(T* out, const T* x, int rows, int d, hipStream_t s) {
 template <typename T>
 __global__ void rotary_embedding_kernel(
     const long* __restrict__ positions,  // [T]
-    T* __restrict__ q,                   // [T, nq * hd]
-    T* __restrict__ k,                   // [T, nk * hd]
+    T* q_out,                            // [T, nq * hd]
+    const T* q,                          // [T, nq * hd], rows q_stride apart
+    T* __restrict__ k,                   // [T, nk * hd], rows k_stride apart
     const float* __restrict__ cos_sin,   // [max_pos, hd]
-    const int nq, const int nk, const int hd) {
+    const int nq, const int nk, const int hd, const long q_stride, const long k_stride) {
   const int token = blockIdx.x;
   const long pos = positions[token];
   const float* cs = cos_sin + pos * hd;
   const int half = hd / 2;
 
-  T* q_row = q + (long)token * nq * hd;
-  T* k_row = k + (long)token * nk * hd;
+  const T* q_row = q + token * q_stride;
+  T* o_row = q_out + (long)token * nq * hd;
+  T* k_row = k + token * k_stride;
   const int total = (nq + nk) * half;
   for (int idx = threadIdx.x; idx < total; idx += blockDim.x) {
     const int h = idx / half;
     const int i = idx % half;
-    T* row = h < nq ? q_row + h * hd : k_row + (h - nq) * hd;
+    const T* row = h < nq ? q_row + h * hd : k_row + (h - nq) * hd;
+    T* out = h < nq ? o_row + h * hd : k_row + (h - nq) * hd;
     const float c = cs[i];
     const float s = cs[half + i];
     const float x1 = ScalarOps<T>::to_f32(row[i]);
     const float x2 = ScalarOps<T>::to_f32(row[i + half]);
-    row[i] = ScalarOps<T>::from_f32(x1 * c - x2 * s);
-    row[i + half] = ScalarOps<T>::from_f32(x2 * c + x1 * s);
+    out[i] = ScalarOps<T>::from_f32(x1 * c - x2 * s);
+    out[i + half] = ScalarOps<T>::from_f32(x2 * c + x1 * s);
   }
 }
 
 template <typename T>
-void launch_rotary_embedding(const long* positions, T* q, T* k,
+void launch_rotary_embedding(const long* positions, T* q_out, const T* q, T* k,
                              const float* cos_sin, int tokens, int nq, int nk,
-                             int hd, hipStream_t s) {
+                             int hd, long q_stride, long k_stride, hipStream_t s) {
   int threads = 256;
   hipLaunchKernelGGL(rotary_embedding_kernel<T>, dim3(tokens), dim3(threads), 0,
-                     s, positions, q, k, cos_sin, nq, nk, hd);
+                     s, positions, q_out, q, k, cos_sin, nq, nk, hd, q_stride, k_stride);
 }
 
 // ---------------------------------------------------------------------------
 // reshape_and_cache: scatter per-token K/V rows into the paged cache.
 // cache layout: [num_blocks, block_size, kv_heads, head_dim] — a token's
-// (kv_heads*head_dim) row is contiguous, so this is a straight 16-B copy.
+// (kv_heads*head_dim) row is contiguous, so this is a straight 16-B copy.  Rows
+// of k and v may lie k_stride / v_stride elements apart.
 // ---------------------------------------------------------------------------
 
 template <typename T>
@@ -95,13 +101,13 @@ __global__ void reshape_and_cache_kernel(
     T* __restrict__ k_cache,      // [nb * bs, kvh * hd] flattened
     T* __restrict__ v_cache,
     const long* __restrict__ slots,  // [T]
-    const int row_elems) {
+    const int row_elems, const long k_stride, const long v_stride) {
   constexpr int V = Vec16<T>::kElems;
   const int token = blockIdx.x;
   const long slot = slots[token];
   if (slot < 0) return;
-  const T* k_src = k + (long)token * row_elems;
-  const T* v_src = v + (long)token * row_elems;
+  const T* k_src = k + token * k_stride;
+  const T* v_src = v + token * v_stride;
   T* k_dst = k_cache + slot * row_elems;
   T* v_dst = v_cache + slot * row_elems;
   for (int i = threadIdx.x * V; i < row_elems; i += blockDim.x * V) {
@@ -113,10 +119,10 @@ __global__ void reshape_and_cache_kernel(
 template <typename T>
 void launch_reshape_and_cache(const T* k, const T* v, T* kc, T* vc,
                               const long* slots, int tokens, int row_elems,
-                              hipStream_t s) {
+                              long k_stride, long v_stride, hipStream_t s) {
   int threads = 128;
   hipLaunchKernelGGL(reshape_and_cache_kernel<T>, dim3(tokens), dim3(threads),
-                     0, s, k, v, kc, vc, slots, row_elems);
+                     0, s, k, v, kc, vc, slots, row_elems, k_stride, v_stride);
 }
 
 // fp8 KV cache (SURVEY E5 + E18 adjacency): bf16 K/V quantized to OCP e4m3
@@ -128,12 +134,12 @@ __global__ void reshape_and_cache_fp8_kernel(
     unsigned char* __restrict__ k_cache,   // [nb * bs, kvh * hd] e4m3
     unsigned char* __restrict__ v_cache,
     const long* __restrict__ slots,
-    const int row_elems) {
+    const int row_elems, const long k_stride, const long v_stride) {
   const int token = blockIdx.x;
   const long slot = slots[token];
   if (slot < 0) return;
-  const __hip_bfloat16* k_src = k + (long)token * row_elems;
-  const __hip_bfloat16* v_src = v + (long)token * row_elems;
+  const __hip_bfloat16* k_src = k + token * k_stride;
+  const __hip_bfloat16* v_src = v + token * v_stride;
   unsigned char* k_dst = k_cache + slot * row_elems;
   unsigned char* v_dst = v_cache + slot * row_elems;
   for (int i = threadIdx.x * 8; i < row_elems; i += blockDim.x * 8) {
@@ -147,17 +153,20 @@ __global__ void reshape_and_cache_fp8_kernel(
 void launch_reshape_and_cache_fp8(const __hip_bfloat16* k,
                                   const __hip_bfloat16* v, unsigned char* kc,
                                   unsigned char* vc, const long* slots,
-                                  int tokens, int row_elems, hipStream_t s) {
+                                  int tokens, int row_elems, long k_stride,
+                                  long v_stride, hipStream_t s) {
   hipLaunchKernelGGL(reshape_and_cache_fp8_kernel, dim3(tokens), dim3(128), 0,
-                     s, k, v, kc, vc, slots, row_elems);
+                     s, k, v, kc, vc, slots, row_elems, k_stride, v_stride);
 }
 
 #define INSTANTIATE(T)                                                         \
   template void launch_silu_and_mul<T>(T*, const T*, int, int, hipStream_t);   \
-  template void launch_rotary_embedding<T>(const long*, T*, T*, const float*,  \
-                                           int, int, int, int, hipStream_t);   \
+  template void launch_rotary_embedding<T>(const long*, T*, const T*, T*,      \
+                                           const float*, int, int, int, int,   \
+                                           long, long, hipStream_t);           \
   template void launch_reshape_and_cache<T>(const T*, const T*, T*, T*,        \
-                                            const long*, int, int, hipStream_t);
+                                            const long*, int, int, long, long, \
+                                            hipStream_t);
 
 INSTANTIATE(float)
 INSTANTIATE(__hip_bfloat16)

@@ -101,10 +101,14 @@ def rotary_embedding(
     head_dim: int,
     cos_sin_cache: torch.Tensor,
 ) -> tuple[torch.Tensor, torch.Tensor]:
-    """NeoX rotary; in place on GPU, out-of-place on CPU."""
+    """NeoX rotary; in place on GPU, out-of-place on CPU.  q and k may be column
+    slices of one projection's rows: k is turned where it lies, q (which the
+    attention kernels read as dense rows) into rows of its own."""
     if _native(q):
-        _C.rotary_embedding(positions, q, k, head_dim, cos_sin_cache)
-        return q, k
+        out = q if q.is_contiguous() else torch.empty(
+            q.shape, dtype=q.dtype, device=q.device)
+        _C.rotary_embedding(positions, out, q, k, head_dim, cos_sin_cache)
+        return out, k
     return reference.rotary_embedding(positions, q, k, head_dim, cos_sin_cache)
 
 
