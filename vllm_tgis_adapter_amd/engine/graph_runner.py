@@ -75,6 +75,9 @@ class DecodeGraphRunner:
     @torch.inference_mode()
     def capture(self) -> None:
         stream = torch.cuda.Stream()
+        # weights, cache and the static inputs may still be on their way: the
+        # side stream would gather with ids and tables that hold anything
+        stream.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(stream):
             # one eager warmup pass (cuBLAS/hipBLASLt workspace init etc.)
             b = self.buckets[-1]
