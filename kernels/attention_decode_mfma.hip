@@ -1,5 +1,5 @@
-// MFMA paged decode attention — replaces the VALU decode
-// kernel for bf16 head_dim 64/128, GQA group <= 8.
+// MFMA paged decode attention with a window, sinks, chunks, prefixes or capped
+// scores: bf16, GQA group <= 8 (plain attention: attention_decode_stream.hip).
 //
 // The VALU kernel spent its time in per-slot cross-lane reduction chains
 // (rocprofv3 r1: 155 us/call vs a ~17 us HBM roofline at batch 64, ctx 512).
@@ -24,36 +24,22 @@
 typedef __attribute__((ext_vector_type(8))) short bf16x8_t;
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 
-// 8 consecutive KV elements as bf16: direct for bf16 caches, hardware
-// cvt_pk_f32_fp8 for e4m3 caches (fp8 KV halves the decode HBM stream)
-template <typename CT>
-DEVINLINE bf16x8_t load_kv8(const CT* p);
-template <>
-DEVINLINE bf16x8_t load_kv8<__hip_bfloat16>(const __hip_bfloat16* p) {
-  return *reinterpret_cast<const bf16x8_t*>(p);
-}
-template <>
-DEVINLINE bf16x8_t load_kv8<unsigned char>(const unsigned char* p) {
-  return __builtin_bit_cast(
-      bf16x8_t, fp8x8_to_bf16x8(*reinterpret_cast<const u32x2_vec_t*>(p)));
-}
-
 #define KVT 32     // kv slots per mfma tile
 #define NWAVES 4   // waves per workgroup
 
-// WS (window + sink variant): the query (position seq_len - 1) sees the last
-// `window` keys only (window 0: all), and the probabilities enter the value
-// product as the sum of two bf16 terms (rounded value + rounded remainder);
-// the sink joins the denominator in the merge kernel.
-// CH (chunk variant, on top of WS): the query sees the keys of its own chunk
+// The query (position seq_len - 1) sees the last `window` keys only (window 0:
+// all), and the probabilities enter the value product as the sum of two bf16 terms
+// (rounded value + rounded remainder); a sink joins the denominator in the merge
+// kernel.
+// CH (chunk variant): the query sees the keys of its own chunk
 // of `chunk` positions only; the value cache holds v_heads <= kvh heads and
 // key head g reads value head g mod v_heads.
-// PX (prefix variants, on top of WS): keys ahead of the window, in tiles of
+// PX (prefix variants): keys ahead of the window, in tiles of
 // their own before the window's tiles.  PX_KEEP: the sequence's first `keep`
 // tokens.  PX_POOL: one pooled key and value per block of `pool` positions that
 // ends at or before seq_len - 1 - window; pooled block b is kept in the cache
 // block that holds its last token (per_block places each).
-// CAP (capped variants, on top of WS): scores become softcap tanh(score / softcap)
+// CAP (capped variants): scores become softcap tanh(score / softcap)
 // (softcap 0: as they are).  CAP_FIXED: up to kFixedMaxCap the cap bounds them well
 // enough that the exponentials are taken without a running maximum.
 enum { PX_NONE = 0, PX_KEEP = 1, PX_POOL = 2 };
@@ -65,14 +51,14 @@ struct SpanKeys {
   const __hip_bfloat16* v_pool;
 };
 
-template <int HEAD_DIM, typename CT, bool WS, bool CH = false, int PX = PX_NONE,
-          int CAP = CAP_NONE, int VD = HEAD_DIM>
+template <int HEAD_DIM, bool CH = false, int PX = PX_NONE, int CAP = CAP_NONE,
+          int VD = HEAD_DIM>
 __global__ __launch_bounds__(256, 2) void paged_decode_mfma_kernel(
     float* __restrict__ part_acc,   // [nseq, nheads, P, VD] f32
     float* __restrict__ part_ml,    // [nseq, nheads, P, 2] f32 (m, l)
     const __hip_bfloat16* __restrict__ q,        // [nseq, nheads, HD]
-    const CT* __restrict__ k_cache,  // [nb, bs, kvh, HD] bf16 | e4m3
-    const CT* __restrict__ v_cache,
+    const __hip_bfloat16* __restrict__ k_cache,  // [nb, bs, kvh, HD] bf16 | e4m3
+    const __hip_bfloat16* __restrict__ v_cache,
     const int* __restrict__ block_tables,  // [nseq, max_blocks]
     const int* __restrict__ seq_lens,      // [nseq]
     const float scale,
@@ -86,10 +72,8 @@ __global__ __launch_bounds__(256, 2) void paged_decode_mfma_kernel(
     const int v_heads = 0,
     const SpanKeys sp = SpanKeys{},
     const float softcap = 0.f) {
-  static_assert(CAP == CAP_NONE || (WS && !CH && PX == PX_NONE),
-                "the capped variant builds on the window variant");
-  static_assert(!CH || WS, "the chunk variant builds on the window variant");
-  static_assert(PX == PX_NONE || (WS && !CH), "prefixes build on the window variant");
+  static_assert(CAP == CAP_NONE || (!CH && PX == PX_NONE), "capped: window only");
+  static_assert(PX == PX_NONE || !CH, "prefixes: window only");
   constexpr int KCH = HEAD_DIM / 16;  // k-chunks for the QK^T mfma
   constexpr int DT = VD / 32;         // 32-col output tiles
   static_assert(HEAD_DIM % 16 == 0 && (VD == 64 || VD == 128), "head sizes");
@@ -109,7 +93,7 @@ __global__ __launch_bounds__(256, 2) void paged_decode_mfma_kernel(
   // this partition's tile range; waves stride by NWAVES inside it
   const int tiles_total = (seq_len + KVT - 1) / KVT;
   const int first_pos = (CH && chunk > 0) ? max(0, seq_len - 1) / chunk * chunk
-                        : (WS && window > 0) ? max(0, seq_len - window) : 0;
+                        : window > 0 ? max(0, seq_len - window) : 0;
   const int tile_first = first_pos / KVT;
   // prefix tiles come first in this workgroup range's numbering
   int pre_len = 0;
@@ -168,8 +152,8 @@ __global__ __launch_bounds__(256, 2) void paged_decode_mfma_kernel(
       const int block = btable[pos / block_size];
       return (long)block * block_size + pos % block_size;
     };
-    const CT* k_src = k_cache;
-    const CT* v_src = v_cache;
+    const __hip_bfloat16* k_src = k_cache;
+    const __hip_bfloat16* v_src = v_cache;
     if constexpr (PX == PX_POOL) {
       if (prefix) { k_src = sp.k_pool; v_src = sp.v_pool; }
     }
@@ -184,10 +168,10 @@ __global__ __launch_bounds__(256, 2) void paged_decode_mfma_kernel(
     {
       const int pos = kv_base + col;
       if (pos < limit) {
-        const CT* k_row = k_src + row_of(pos) * kv_row_stride + (long)kv_head * HEAD_DIM;
+        const __hip_bfloat16* k_row = k_src + row_of(pos) * kv_row_stride + (long)kv_head * HEAD_DIM;
 #pragma unroll
         for (int ks = 0; ks < KCH; ++ks)
-          ka[ks] = load_kv8<CT>(k_row + ks * 16 + half * 8);
+          ka[ks] = *reinterpret_cast<const bf16x8_t*>(k_row + ks * 16 + half * 8);
       } else {
 #pragma unroll
         for (int ks = 0; ks < KCH; ++ks) ka[ks] = bf16x8_t{};
@@ -206,7 +190,7 @@ __global__ __launch_bounds__(256, 2) void paged_decode_mfma_kernel(
         vv[pass] = bf16x8_t{};
         if (pos < limit) {
           const long row = row_of(pos) * v_row_stride + (long)v_head * VD + d8;
-          vv[pass] = load_kv8<CT>(v_src + row);
+          vv[pass] = *reinterpret_cast<const bf16x8_t*>(v_src + row);
         }
       }
 #pragma unroll
@@ -245,7 +229,7 @@ __global__ __launch_bounds__(256, 2) void paged_decode_mfma_kernel(
     for (int r = 0; r < 16; ++r) {
       const int kv_pos = kv_base + (r & 3) + 8 * (r >> 2) + 4 * half;
       float sv = acc_s[r] * (CAP != CAP_NONE && capped ? softcap : scale);
-      if (kv_pos >= limit || (WS && !prefix && kv_pos < first_pos)) sv = -FLT_MAX;
+      if (kv_pos >= limit || (!prefix && kv_pos < first_pos)) sv = -FLT_MAX;
       s_val[r] = sv;
       local_max = fmaxf(local_max, sv);
     }
@@ -282,7 +266,7 @@ __global__ __launch_bounds__(256, 2) void paged_decode_mfma_kernel(
     }
 
     // ---- pack P to bf16 A-fragments (cvt_pk + permlane32_swap) -----------
-    constexpr int PASSES = WS ? 2 : 1;   // pass 1: what the first rounding left over
+    constexpr int PASSES = 2;   // pass 1: what the first rounding left over
     bf16x8_t pa[PASSES][2];
 #pragma unroll
     for (int ps = 0; ps < PASSES; ++ps) {
@@ -291,7 +275,7 @@ __global__ __launch_bounds__(256, 2) void paged_decode_mfma_kernel(
       for (int i = 0; i < 8; ++i) {
         asm volatile("v_cvt_pk_bf16_f32 %0, %1, %2"
                      : "=v"(pk[i]) : "v"(p[2 * i]), "v"(p[2 * i + 1]));
-        if (WS && ps == 0) {
+        if (ps == 0) {
           p[2 * i] -= __uint_as_float(pk[i] << 16);
           p[2 * i + 1] -= __uint_as_float(pk[i] & 0xffff0000u);
         }
@@ -323,9 +307,7 @@ __global__ __launch_bounds__(256, 2) void paged_decode_mfma_kernel(
           b[j] = *reinterpret_cast<const short*>(
               v_lds + (c * 16 + half * 8 + j) * VD + dt * 32 + col);
         acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[0][c], b, acc_o[dt], 0, 0, 0);
-        if (WS)
-          acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[PASSES - 1][c], b,
-                                                              acc_o[dt], 0, 0, 0);
+        acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[1][c], b, acc_o[dt], 0, 0, 0);
       }
     }
   }
@@ -411,84 +393,6 @@ int decode_mfma_num_partitions(int nseq, int kvh, int max_context) {
   return npart;
 }
 
-template <typename CT>
-static void launch_decode_ct(__hip_bfloat16* out, float* part_acc,
-                             float* part_ml, const __hip_bfloat16* q,
-                             const CT* kc, const CT* vc, const int* bt,
-                             const int* sl, float scale, int nseq, int nheads,
-                             int kvh, int head_dim, int block_size,
-                             int max_blocks, int npart, hipStream_t stream,
-                             int window = 0, int has_sink = 0, float sink = 0.f,
-                             bool ws = false) {
-  const int group = nheads / kvh;
-  dim3 grid(nseq, kvh, npart);
-  dim3 block(256);
-  dim3 mgrid(nseq, nheads);
-  const int P = npart * NWAVES;
-  if (ws) {
-    switch (head_dim) {
-      case 64:
-        hipLaunchKernelGGL((paged_decode_mfma_kernel<64, CT, true>), grid, block, 0,
-                           stream, part_acc, part_ml, q, kc, vc, bt, sl, scale,
-                           nheads, kvh, group, block_size, max_blocks, window);
-        hipLaunchKernelGGL((decode_merge_kernel<64>), mgrid, dim3(64), 0, stream,
-                           out, part_acc, part_ml, nheads, P, has_sink, sink, nullptr, nullptr);
-        break;
-      case 128:
-        hipLaunchKernelGGL((paged_decode_mfma_kernel<128, CT, true>), grid, block, 0,
-                           stream, part_acc, part_ml, q, kc, vc, bt, sl, scale,
-                           nheads, kvh, group, block_size, max_blocks, window);
-        hipLaunchKernelGGL((decode_merge_kernel<128>), mgrid, dim3(128), 0, stream,
-                           out, part_acc, part_ml, nheads, P, has_sink, sink, nullptr, nullptr);
-        break;
-      default:
-        abort();
-    }
-    return;
-  }
-  switch (head_dim) {
-    case 64:
-      hipLaunchKernelGGL((paged_decode_mfma_kernel<64, CT, false>), grid, block, 0,
-                         stream, part_acc, part_ml, q, kc, vc, bt, sl, scale,
-                         nheads, kvh, group, block_size, max_blocks, 0);
-      hipLaunchKernelGGL((decode_merge_kernel<64>), mgrid, dim3(64), 0, stream,
-                         out, part_acc, part_ml, nheads, P, 0, 0.f, nullptr, nullptr);
-      break;
-    case 128:
-      hipLaunchKernelGGL((paged_decode_mfma_kernel<128, CT, false>), grid, block, 0,
-                         stream, part_acc, part_ml, q, kc, vc, bt, sl, scale,
-                         nheads, kvh, group, block_size, max_blocks, 0);
-      hipLaunchKernelGGL((decode_merge_kernel<128>), mgrid, dim3(128), 0, stream,
-                         out, part_acc, part_ml, nheads, P, 0, 0.f, nullptr, nullptr);
-      break;
-    default:
-      abort();
-  }
-}
-
-void launch_paged_decode_mfma(__hip_bfloat16* out, float* part_acc,
-                              float* part_ml, const __hip_bfloat16* q,
-                              const __hip_bfloat16* kc, const __hip_bfloat16* vc,
-                              const int* bt, const int* sl, float scale,
-                              int nseq, int nheads, int kvh, int head_dim,
-                              int block_size, int max_blocks, int npart,
-                              hipStream_t stream) {
-  launch_decode_ct<__hip_bfloat16>(out, part_acc, part_ml, q, kc, vc, bt, sl,
-                                   scale, nseq, nheads, kvh, head_dim,
-                                   block_size, max_blocks, npart, stream);
-}
-
-void launch_paged_decode_mfma_fp8(
-    __hip_bfloat16* out, float* part_acc, float* part_ml,
-    const __hip_bfloat16* q, const unsigned char* kc, const unsigned char* vc,
-    const int* bt, const int* sl, float scale, int nseq, int nheads, int kvh,
-    int head_dim, int block_size, int max_blocks, int npart,
-    hipStream_t stream) {
-  launch_decode_ct<unsigned char>(out, part_acc, part_ml, q, kc, vc, bt, sl,
-                                  scale, nseq, nheads, kvh, head_dim,
-                                  block_size, max_blocks, npart, stream);
-}
-
 // window + sink variant (bf16 cache)
 void launch_paged_decode_mfma_ws(__hip_bfloat16* out, float* part_acc,
                                  float* part_ml, const __hip_bfloat16* q,
@@ -498,10 +402,27 @@ void launch_paged_decode_mfma_ws(__hip_bfloat16* out, float* part_acc,
                                  int block_size, int max_blocks, int npart,
                                  int window, int has_sink, float sink,
                                  hipStream_t stream) {
-  launch_decode_ct<__hip_bfloat16>(out, part_acc, part_ml, q, kc, vc, bt, sl,
-                                   scale, nseq, nheads, kvh, head_dim,
-                                   block_size, max_blocks, npart, stream, window,
-                                   has_sink, sink, true);
+  const int group = nheads / kvh;
+  const dim3 grid(nseq, kvh, npart), mgrid(nseq, nheads);
+  const int P = npart * NWAVES;
+  switch (head_dim) {
+    case 64:
+      hipLaunchKernelGGL((paged_decode_mfma_kernel<64>), grid, dim3(256), 0, stream, part_acc,
+                         part_ml, q, kc, vc, bt, sl, scale, nheads, kvh, group, block_size,
+                         max_blocks, window);
+      hipLaunchKernelGGL((decode_merge_kernel<64>), mgrid, dim3(64), 0, stream, out, part_acc,
+                         part_ml, nheads, P, has_sink, sink, nullptr, nullptr);
+      break;
+    case 128:
+      hipLaunchKernelGGL((paged_decode_mfma_kernel<128>), grid, dim3(256), 0, stream, part_acc,
+                         part_ml, q, kc, vc, bt, sl, scale, nheads, kvh, group, block_size,
+                         max_blocks, window);
+      hipLaunchKernelGGL((decode_merge_kernel<128>), mgrid, dim3(128), 0, stream, out, part_acc,
+                         part_ml, nheads, P, has_sink, sink, nullptr, nullptr);
+      break;
+    default:
+      abort();
+  }
 }
 
 // chunk variant with shared value heads and f32 output (bf16 cache)
@@ -520,7 +441,7 @@ void launch_paged_decode_mfma_chunk(float* out, float* part_acc, float* part_ml,
   switch (head_dim) {
     case 64:
       hipLaunchKernelGGL(
-          (paged_decode_mfma_kernel<64, __hip_bfloat16, true, true>), grid, dim3(256),
+          (paged_decode_mfma_kernel<64, true>), grid, dim3(256),
           0, stream, part_acc, part_ml, q, kc, vc, bt, sl, scale, nheads, kvh, group,
           block_size, max_blocks, 0, chunk, v_heads);
       hipLaunchKernelGGL((decode_merge_kernel<64, float>), mgrid, dim3(64), 0, stream,
@@ -528,7 +449,7 @@ void launch_paged_decode_mfma_chunk(float* out, float* part_acc, float* part_ml,
       break;
     case 128:
       hipLaunchKernelGGL(
-          (paged_decode_mfma_kernel<128, __hip_bfloat16, true, true>), grid,
+          (paged_decode_mfma_kernel<128, true>), grid,
           dim3(256), 0, stream, part_acc, part_ml, q, kc, vc, bt, sl, scale, nheads,
           kvh, group, block_size, max_blocks, 0, chunk, v_heads);
       hipLaunchKernelGGL((decode_merge_kernel<128, float>), mgrid, dim3(128), 0,
@@ -551,11 +472,11 @@ static void launch_decode_span(__hip_bfloat16* out, float* part_acc, float* part
   const dim3 grid(nseq, kvh, npart), mgrid(nseq, nheads);
   const int P = npart * NWAVES;
   if (sp.pool > 0)
-    hipLaunchKernelGGL((paged_decode_mfma_kernel<HD, __hip_bfloat16, true, false, PX_POOL>),
+    hipLaunchKernelGGL((paged_decode_mfma_kernel<HD, false, PX_POOL>),
                        grid, dim3(256), 0, stream, part_acc, part_ml, q, kc, vc, bt, sl,
                        scale, nheads, kvh, group, block_size, max_blocks, window, 0, 0, sp);
   else
-    hipLaunchKernelGGL((paged_decode_mfma_kernel<HD, __hip_bfloat16, true, false, PX_KEEP>),
+    hipLaunchKernelGGL((paged_decode_mfma_kernel<HD, false, PX_KEEP>),
                        grid, dim3(256), 0, stream, part_acc, part_ml, q, kc, vc, bt, sl,
                        scale, nheads, kvh, group, block_size, max_blocks, window, 0, 0, sp);
   if (back != nullptr)
@@ -599,7 +520,7 @@ static void launch_decode_capped(__hip_bfloat16* out, float* part_acc, float* pa
                                  float softcap, hipStream_t stream) {
   const dim3 grid(nseq, kvh, npart), mgrid(nseq, nheads);
   hipLaunchKernelGGL(
-      (paged_decode_mfma_kernel<HD, __hip_bfloat16, true, false, PX_NONE, CAP, VD>), grid,
+      (paged_decode_mfma_kernel<HD, false, PX_NONE, CAP, VD>), grid,
       dim3(256), 0, stream, part_acc, part_ml, q, kc, vc, bt, sl, scale, nheads, kvh,
       nheads / kvh, block_size, max_blocks, window, 0, 0, SpanKeys{}, softcap);
   hipLaunchKernelGGL((decode_merge_kernel<VD>), mgrid, dim3(VD), 0, stream, out, part_acc,

@@ -1,0 +1,366 @@
+// Paged decode attention, one query row per sequence: bf16 or e4m3 cache, heads of
+// 64 or 128, up to 8 query heads per key head.
+//
+// Bound by the cache's bytes.  Every wave walks 32-key tiles: keys and values are
+// loaded as whole rows (a tile of both in registers while the one before is worked
+// on, its block ids a tile earlier still), keys, then values, go through the wave's
+// own LDS tile.  v_mfma_f32_16x16x32_bf16 takes S^T = K Q^T, so a lane keeps one
+// query's statistics and accumulators and no shuffle rescales them; the two 16-key
+// score tiles take the second product's slots in the order the score layout has
+// them, so probabilities are packed where they are, and the values come back
+// transposed (ds_read_b64_tr_b16), swizzled so that neither way has bank conflicts.
+// The rows are read once: loads that leave no trace in the caches (nontemporal).
+//
+// The keys of a sequence are cut over up to npart workgroups (a pure function of
+// shapes, so that a captured launch stays valid) of at least four tiles each, the
+// four waves merge in LDS, and only a sequence that was cut goes through the merge
+// kernel.
+//
+// Measured (MI355X, 32/8 heads of 128, two layers with their cache writes): 512
+// sequences of ~520 keys, bf16: 794 -> 361 us (2.8 -> 6.1 TB/s; a plain read
+// reaches 6.3); 41 of ~4800 keys, e4m3: 1365 -> 167 us (the former kernel ran 328
+// workgroups there).  On the way: three workgroups a CU instead of two spill, 427;
+// cached loads, 407; keys loaded straight into the operand's layout, 398.
+
+#include "common.h"
+#include <float.h>
+
+typedef __attribute__((ext_vector_type(8))) short bf16x8_t;
+typedef __attribute__((ext_vector_type(4))) short s16x4_t;
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+typedef __attribute__((ext_vector_type(4))) unsigned int u32x4_t;
+typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
+
+namespace {
+
+constexpr int kTile = 32;    // keys per wave and step
+constexpr int kWaves = 4;
+constexpr int kMinTiles = kWaves;   // a workgroup's share is no smaller
+constexpr float kLog2e = 1.4426950408889634f;
+
+DEVINLINE unsigned pack_bf16(float a, float b) {
+  unsigned r;
+  asm volatile("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
+// tiles of a sequence that one workgroup takes, a multiple of the waves
+DEVINLINE int tiles_per_part(int tiles, int npart) {
+  const int per = (tiles + npart - 1) / npart;
+  return max(kMinTiles, (per + kWaves - 1) / kWaves * kWaves);
+}
+
+template <int HD, typename CT>
+__global__ __launch_bounds__(256, 2) void paged_decode_stream_kernel(
+    __hip_bfloat16* __restrict__ out,       // [nseq, nheads, HD]
+    float* __restrict__ part_acc,           // [nseq, nheads, npart, HD] (npart > 1)
+    float* __restrict__ part_ml,            // [nseq, nheads, npart, 2]  (npart > 1)
+    const __hip_bfloat16* __restrict__ q,   // [nseq, nheads, HD]
+    const CT* __restrict__ k_cache,         // [blocks, block_size, kvh, HD]
+    const CT* __restrict__ v_cache,
+    const int* __restrict__ block_tables,   // [nseq, max_blocks]
+    const int* __restrict__ seq_lens,       // [nseq]
+    const float scale_log2, const int nheads, const int kvh, const int group,
+    const int block_size, const int block_shift, const int max_blocks) {
+  constexpr bool FP8 = sizeof(CT) == 1;
+  constexpr int KS = HD / 32;              // contraction steps of a score tile
+  constexpr int DT = HD / 16;              // 16-wide tiles of the result
+  constexpr int PER = 16 / sizeof(CT);     // elements of a 16-byte load
+  constexpr int LPR = HD / PER;            // lanes per value row
+  constexpr int RPP = 64 / LPR;            // value rows per pass
+  constexpr int VP = kTile / RPP;          // passes
+
+  const int seq = blockIdx.x, kv_head = blockIdx.y, part = blockIdx.z;
+  const int npart = gridDim.z;
+  const int seq_len = seq_lens[seq];
+  const int tiles = (seq_len + kTile - 1) / kTile;
+  const int tpp = tiles_per_part(tiles, npart);
+  const int lo = part * tpp;
+  // a sequence without keys (padding) still gets its zeros from part 0
+  if (lo >= tiles && part > 0) return;
+  const int hi = min(lo + tpp, tiles);
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int col = lane & 15, quad = lane >> 4;
+  const int head0 = kv_head * group;
+  const int* table = block_tables + (long)seq * max_blocks;
+  const long row_elems = (long)kvh * HD;
+
+  __shared__ __align__(16) __hip_bfloat16 tile_all[kWaves][kTile * HD];
+  __shared__ float ml_all[kWaves][2][16];
+  __hip_bfloat16* tile_lds = tile_all[wave];
+
+  bf16x8_t qf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    qf[ks] = bf16x8_t{};
+    if (col < group)
+      qf[ks] = *reinterpret_cast<const bf16x8_t*>(
+          q + ((long)seq * nheads + head0 + col) * HD + ks * 32 + quad * 8);
+  }
+
+  // cache row of key (tile * 32 + lane % 32); past the end: of the last key
+  auto slot_of = [&](int tile) {
+    const int pos = min(tile * kTile + (lane & 31), seq_len - 1);
+    const int page = block_shift >= 0 ? pos >> block_shift : pos / block_size;
+    return table[page] * block_size + (pos - page * block_size);
+  };
+
+  u32x4_t kr[VP], vr[VP];
+  auto issue = [&](int slot) {
+    long at[VP];
+#pragma unroll
+    for (int ps = 0; ps < VP; ++ps)
+      at[ps] = __shfl(slot, ps * RPP + lane / LPR, 64) * row_elems + kv_head * HD +
+               (lane % LPR) * PER;
+#pragma unroll
+    for (int ps = 0; ps < VP; ++ps) kr[ps] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(k_cache + at[ps]));
+#pragma unroll
+    for (int ps = 0; ps < VP; ++ps) vr[ps] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(v_cache + at[ps]));
+  };
+  // 16-byte chunk c of row r lies at chunk c ^ swizzle(r): a pair of chunks stays a
+  // pair, the 16 rows of a transposed read cover all banks twice, and eight rows'
+  // equal chunks lie in different banks
+  auto swizzle = [](int r) { return HD == 128 ? (r & 7) * 2 : ((r >> 1) & 3) * 2; };
+  auto stage = [&](const u32x4_t (&from)[VP]) {
+#pragma unroll
+    for (int ps = 0; ps < VP; ++ps) {
+      const int r = ps * RPP + lane / LPR;
+      char* row = reinterpret_cast<char*>(tile_lds) + r * HD * 2;
+      if constexpr (FP8) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          u32x2_vec_t u;
+          u[0] = from[ps][2 * h];
+          u[1] = from[ps][2 * h + 1];
+          *reinterpret_cast<bf16x8_vec_t*>(
+              row + (((lane % LPR) * 2 + h) ^ swizzle(r)) * 16) = fp8x8_to_bf16x8(u);
+        }
+      } else {
+        *reinterpret_cast<u32x4_t*>(row + ((lane % LPR) ^ swizzle(r)) * 16) = from[ps];
+      }
+    }
+    // other lanes of this wave read it: LDS keeps a wave's order, the compiler has to
+    asm volatile("" ::: "memory");
+  };
+
+  float m_state = -FLT_MAX, l_state = 0.f;   // of query `col`; l: this lane's keys
+  f32x4_t acc[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x4_t{};
+
+  int t = lo + wave, slot_next = 0;
+  if (t < hi) {
+    issue(slot_of(t));
+    if (t + kWaves < hi) slot_next = slot_of(t + kWaves);
+  }
+  for (; t < hi; t += kWaves) {
+    f32x4_t s[2] = {f32x4_t{}, f32x4_t{}};
+    stage(kr);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt) {
+        const int r = rt * 16 + col;
+        const bf16x8_t kf = *reinterpret_cast<const bf16x8_t*>(
+            reinterpret_cast<const char*>(tile_lds) + r * HD * 2 +
+            ((ks * 4 + quad) ^ swizzle(r)) * 16);
+        s[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[ks], s[rt], 0, 0, 0);
+      }
+    asm volatile("" ::: "memory");
+    stage(vr);
+    if (t + kWaves < hi) {
+      issue(slot_next);
+      if (t + 2 * kWaves < hi) slot_next = slot_of(t + 2 * kWaves);
+    }
+
+    // ---- softmax: lane has keys rt*16 + quad*4 + r of query col ----------
+    const int base = t * kTile + quad * 4;
+    float big = -FLT_MAX;
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float v = s[rt][r] * scale_log2;
+        if (base + rt * 16 + r >= seq_len) v = -FLT_MAX;
+        s[rt][r] = v;
+        big = fmaxf(big, v);
+      }
+    big = fmaxf(big, __shfl_xor(big, 16, 64));
+    big = fmaxf(big, __shfl_xor(big, 32, 64));
+    const float m_new = fmaxf(m_state, big);
+    if (!__all(m_new == m_state)) {
+      const float f = __builtin_amdgcn_exp2f(m_state - m_new);
+      l_state *= f;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[dt][r] *= f;
+      m_state = m_new;
+    }
+    union { unsigned u[4]; bf16x8_t v; } p;
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+      float e[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        e[r] = s[rt][r] == -FLT_MAX ? 0.f : __builtin_amdgcn_exp2f(s[rt][r] - m_state);
+        l_state += e[r];
+      }
+      p.u[2 * rt] = pack_bf16(e[0], e[1]);
+      p.u[2 * rt + 1] = pack_bf16(e[2], e[3]);
+    }
+
+    // ---- O^T += V^T P^T, values read back transposed ---------------------
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      union { s16x4_t h[2]; bf16x8_t v; } vf;
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt) {
+        const int r = rt * 16 + quad * 4 + (col >> 2);
+        char* at = reinterpret_cast<char*>(tile_lds) + r * HD * 2 +
+                   ((dt * 2 + ((col & 3) >> 1)) ^ swizzle(r)) * 16 + (col & 1) * 8;
+        vf.h[rt] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)at);
+      }
+      acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, p.v, acc[dt], 0, 0, 0);
+    }
+    asm volatile("" ::: "memory");
+  }
+
+  // ---- the waves' results become one ---------------------------------------
+  l_state += __shfl_xor(l_state, 16, 64);
+  l_state += __shfl_xor(l_state, 32, 64);
+  if (lane < 16) {
+    ml_all[wave][0][lane] = m_state;
+    ml_all[wave][1][lane] = l_state;
+  }
+  __syncthreads();
+  float M = ml_all[0][0][col];
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w) M = fmaxf(M, ml_all[w][0][col]);
+  const float f = __builtin_amdgcn_exp2f(m_state - M);
+  float* mine = reinterpret_cast<float*>(tile_all[wave]);   // [16][HD]
+  static_assert(kTile * 2 >= 16 * 4, "a wave's tile holds its result");
+  if (col < group) {
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+      *reinterpret_cast<f32x4_t*>(mine + col * HD + dt * 16 + quad * 4) = acc[dt] * f;
+  }
+  __syncthreads();
+  const bool whole = tpp >= tiles;
+  for (int i = tid; i < group * HD; i += 256) {
+    const int g = i / HD, d = i % HD;
+    float top = ml_all[0][0][g];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) top = fmaxf(top, ml_all[w][0][g]);
+    float a = 0.f, l = 0.f;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      a += reinterpret_cast<const float*>(tile_all[w])[i];
+      l += ml_all[w][1][g] * __builtin_amdgcn_exp2f(ml_all[w][0][g] - top);
+    }
+    const long row = (long)seq * nheads + head0 + g;
+    if (whole) {
+      out[row * HD + d] = __float2bfloat16(a * (l > 0.f ? 1.f / l : 0.f));
+    } else {
+      part_acc[(row * npart + part) * HD + d] = a;
+      if (d == 0) {
+        part_ml[(row * npart + part) * 2] = top;
+        part_ml[(row * npart + part) * 2 + 1] = l;
+      }
+    }
+  }
+}
+
+// Sequences that were cut: out = sum_p f_p acc_p / sum_p f_p l_p.
+template <int HD>
+__global__ __launch_bounds__(HD) void decode_stream_merge_kernel(
+    __hip_bfloat16* __restrict__ out, const float* __restrict__ part_acc,
+    const float* __restrict__ part_ml, const int* __restrict__ seq_lens,
+    const int nheads, const int npart) {
+  const int seq = blockIdx.x, d = threadIdx.x;
+  const int tiles = (seq_lens[seq] + kTile - 1) / kTile;
+  const int tpp = tiles_per_part(tiles, npart);
+  if (tpp >= tiles) return;
+  const int used = (tiles + tpp - 1) / tpp;   // <= npart <= 64
+  const long row = (long)seq * nheads + blockIdx.y;
+  const int lane = d & 63;
+  const float* ml = part_ml + row * npart * 2;
+  const float m = lane < used ? ml[2 * lane] : -FLT_MAX;
+  const float l = lane < used ? ml[2 * lane + 1] : 0.f;
+  const float M = wave_reduce_max(m);
+  const float f = lane < used ? __builtin_amdgcn_exp2f(m - M) : 0.f;
+  const float L = wave_reduce_sum(f * l);
+  const float* acc = part_acc + row * npart * HD + d;
+  float a = 0.f;
+  for (int p0 = 0; p0 < used; p0 += 8) {   // eight loads on their way at a time
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = acc[(long)min(p0 + i, used - 1) * HD];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (p0 + i < used) a += __shfl(f, p0 + i, 64) * v[i];
+  }
+  out[row * HD + d] = __float2bfloat16(a * (L > 0.f ? 1.f / L : 0.f));
+}
+
+template <int HD, typename CT>
+void launch(__hip_bfloat16* out, float* part_acc, float* part_ml, const __hip_bfloat16* q,
+            const CT* kc, const CT* vc, const int* bt, const int* sl, float scale, int nseq,
+            int nheads, int kvh, int block_size, int max_blocks, int npart,
+            hipStream_t stream) {
+  int shift = -1;
+  if ((block_size & (block_size - 1)) == 0) shift = __builtin_ctz(block_size);
+  hipLaunchKernelGGL((paged_decode_stream_kernel<HD, CT>), dim3(nseq, kvh, npart), dim3(256), 0,
+                     stream, out, part_acc, part_ml, q, kc, vc, bt, sl, scale * kLog2e, nheads,
+                     kvh, nheads / kvh, block_size, shift, max_blocks);
+  if (npart > 1)
+    hipLaunchKernelGGL((decode_stream_merge_kernel<HD>), dim3(nseq, nheads), dim3(HD), 0, stream,
+                       out, part_acc, part_ml, sl, nheads, npart);
+}
+
+}  // namespace
+
+// Workgroups a sequence and key head may be cut over: enough for some six per CU
+// where the batch alone has fewer (twice as many measured the same), at least four
+// tiles each at the longest context.
+int decode_stream_num_partitions(int nseq, int kvh, int max_context) {
+  const int heads = nseq * kvh > 0 ? nseq * kvh : 1;
+  const int tiles = (max_context + kTile - 1) / kTile;
+  const int most = tiles / kMinTiles > 0 ? tiles / kMinTiles : 1;
+  int npart = (1536 + heads - 1) / heads;
+  if (npart > 64) npart = 64;
+  return npart < most ? npart : most;
+}
+
+template <typename CT>
+static void launch_hd(__hip_bfloat16* out, float* part_acc, float* part_ml,
+                      const __hip_bfloat16* q, const CT* kc, const CT* vc, const int* bt,
+                      const int* sl, float scale, int nseq, int nheads, int kvh, int head_dim,
+                      int block_size, int max_blocks, int npart, hipStream_t stream) {
+  if (head_dim == 64)
+    launch<64, CT>(out, part_acc, part_ml, q, kc, vc, bt, sl, scale, nseq, nheads, kvh,
+                   block_size, max_blocks, npart, stream);
+  else
+    launch<128, CT>(out, part_acc, part_ml, q, kc, vc, bt, sl, scale, nseq, nheads, kvh,
+                    block_size, max_blocks, npart, stream);
+}
+
+void launch_paged_decode_stream(__hip_bfloat16* out, float* part_acc, float* part_ml,
+                                const __hip_bfloat16* q, const __hip_bfloat16* kc,
+                                const __hip_bfloat16* vc, const int* bt, const int* sl,
+                                float scale, int nseq, int nheads, int kvh, int head_dim,
+                                int block_size, int max_blocks, int npart, hipStream_t stream) {
+  launch_hd(out, part_acc, part_ml, q, kc, vc, bt, sl, scale, nseq, nheads, kvh, head_dim,
+            block_size, max_blocks, npart, stream);
+}
+
+void launch_paged_decode_stream_fp8(__hip_bfloat16* out, float* part_acc, float* part_ml,
+                                    const __hip_bfloat16* q, const unsigned char* kc,
+                                    const unsigned char* vc, const int* bt, const int* sl,
+                                    float scale, int nseq, int nheads, int kvh, int head_dim,
+                                    int block_size, int max_blocks, int npart,
+                                    hipStream_t stream) {
+  launch_hd(out, part_acc, part_ml, q, kc, vc, bt, sl, scale, nseq, nheads, kvh, head_dim,
+            block_size, max_blocks, npart, stream);
+}

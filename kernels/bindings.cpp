@@ -42,7 +42,6 @@ void launch_paged_prefill_mfma(__hip_bfloat16*, const __hip_bfloat16*,
                                const __hip_bfloat16*, const __hip_bfloat16*,
                                const int*, const int*, const int*, float, int,
                                int, int, int, int, int, int, hipStream_t);
-int decode_mfma_num_partitions(int nseq, int kvh, int max_context);
 int gemm_skinny_num_ksplit(int N, int K, int M);
 void launch_logsoftmax_topk(float*, int*, float*, int*,
                             const __hip_bfloat16*, const long*, int, int,
@@ -52,11 +51,6 @@ void launch_gemm_tile(__hip_bfloat16*, const __hip_bfloat16*,
 void launch_xgmi_allreduce(const unsigned long long*, __hip_bfloat16*,
                            const __hip_bfloat16*, long, long, int, int,
                            hipStream_t);
-void launch_paged_decode_mfma_fp8(__hip_bfloat16*, float*, float*,
-                                  const __hip_bfloat16*, const unsigned char*,
-                                  const unsigned char*, const int*,
-                                  const int*, float, int, int, int, int, int,
-                                  int, int, hipStream_t);
 void launch_paged_prefill_mfma_v2_fp8(__hip_bfloat16*, const __hip_bfloat16*,
                                       const unsigned char*,
                                       const unsigned char*, const int*,
@@ -74,11 +68,6 @@ void launch_gemm_skinny(__hip_bfloat16*, float*, const __hip_bfloat16*,
                         hipStream_t);
 void launch_gemm_skinny_gated(__hip_bfloat16*, float*, const __hip_bfloat16*,
                               const __hip_bfloat16*, int, int, int, int,
-                              hipStream_t);
-void launch_paged_decode_mfma(__hip_bfloat16*, float*, float*,
-                              const __hip_bfloat16*, const __hip_bfloat16*,
-                              const __hip_bfloat16*, const int*, const int*,
-                              float, int, int, int, int, int, int, int,
                               hipStream_t);
 template <typename T>
 void launch_lora_shrink(float*, const T*, const T*, const int*, int, int, int,

@@ -36,22 +36,20 @@ void launch_paged_decode_mfma_capped(__hip_bfloat16*, float*, float*, const __hi
                                      const int*, float, int, int, int, int, int, int, int, int,
                                      int, const float*, float, hipStream_t);
 int decode_mfma_num_partitions(int nseq, int kvh, int max_context);
-void launch_paged_decode_mfma_fp8(__hip_bfloat16*, float*, float*,
-                                  const __hip_bfloat16*, const unsigned char*,
-                                  const unsigned char*, const int*,
-                                  const int*, float, int, int, int, int, int,
-                                  int, int, hipStream_t);
+int decode_stream_num_partitions(int nseq, int kvh, int max_context);
+void launch_paged_decode_stream(__hip_bfloat16*, float*, float*, const __hip_bfloat16*,
+                                const __hip_bfloat16*, const __hip_bfloat16*, const int*,
+                                const int*, float, int, int, int, int, int, int, int,
+                                hipStream_t);
+void launch_paged_decode_stream_fp8(__hip_bfloat16*, float*, float*, const __hip_bfloat16*,
+                                    const unsigned char*, const unsigned char*, const int*,
+                                    const int*, float, int, int, int, int, int, int, int,
+                                    hipStream_t);
 void launch_paged_prefill_mfma_v2_fp8(__hip_bfloat16*, const __hip_bfloat16*,
                                       const unsigned char*,
                                       const unsigned char*, const int*,
                                       const int*, const int*, float, int, int,
                                       int, int, int, int, int, hipStream_t);
-void launch_paged_decode_mfma(__hip_bfloat16*, float*, float*,
-                              const __hip_bfloat16*, const __hip_bfloat16*,
-                              const __hip_bfloat16*, const int*, const int*,
-                              float, int, int, int, int, int, int, int,
-                              hipStream_t);
-
 void launch_paged_prefill_mfma_v2_ws(__hip_bfloat16*, const __hip_bfloat16*,
                                      const __hip_bfloat16*, const __hip_bfloat16*,
                                      const int*, const int*, const int*, float,
@@ -137,45 +135,44 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
     const char* e = getenv("VTA_DECODE_VALU");
     return e && e[0] == '1';
   }();
+  if (nseq == 0) return;
+  if (!q.is_contiguous()) q = q.contiguous();   // the kernels read dense rows
+  auto stream_decode = [&](bool fp8) {
+    const int npart = decode_stream_num_partitions(nseq, kvh, max_blocks * block_size);
+    torch::Tensor part_acc, part_ml;
+    if (npart > 1) {   // only a sequence that is cut leaves partial results
+      auto opts = q.options().dtype(at::ScalarType::Float);
+      part_acc = at::empty({nseq, nheads, npart, head_dim}, opts);
+      part_ml = at::empty({nseq, nheads, npart, 2}, opts);
+    }
+    float* pa = npart > 1 ? part_acc.data_ptr<float>() : nullptr;
+    float* pm = npart > 1 ? part_ml.data_ptr<float>() : nullptr;
+    if (fp8)
+      launch_paged_decode_stream_fp8(
+          ptr<__hip_bfloat16>(out), pa, pm, cptr<__hip_bfloat16>(q),
+          cptr<unsigned char>(k_cache), cptr<unsigned char>(v_cache),
+          block_tables.data_ptr<int>(), seq_lens.data_ptr<int>(), (float)scale, nseq, nheads,
+          kvh, head_dim, block_size, max_blocks, npart, current_stream());
+    else
+      launch_paged_decode_stream(
+          ptr<__hip_bfloat16>(out), pa, pm, cptr<__hip_bfloat16>(q),
+          cptr<__hip_bfloat16>(k_cache), cptr<__hip_bfloat16>(v_cache),
+          block_tables.data_ptr<int>(), seq_lens.data_ptr<int>(), (float)scale, nseq, nheads,
+          kvh, head_dim, block_size, max_blocks, npart, current_stream());
+  };
   const bool kv_fp8 = k_cache.scalar_type() == at::ScalarType::Byte;
   if (kv_fp8) {
     TORCH_CHECK(q.scalar_type() == at::ScalarType::BFloat16 &&
                     (head_dim == 64 || head_dim == 128) && group >= 1 &&
                     group <= 8,
                 "fp8 KV cache requires the bf16 MFMA decode path");
-    const int npart = decode_mfma_num_partitions(nseq, kvh, max_blocks * block_size);
-    const int P = npart * 4;
-    auto opts = q.options().dtype(at::ScalarType::Float);
-    auto part_acc = at::empty({nseq, nheads, P, head_dim}, opts);
-    auto part_ml = at::empty({nseq, nheads, P, 2}, opts);
-    launch_paged_decode_mfma_fp8(
-        reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
-        part_acc.data_ptr<float>(), part_ml.data_ptr<float>(),
-        reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()),
-        reinterpret_cast<const unsigned char*>(k_cache.data_ptr()),
-        reinterpret_cast<const unsigned char*>(v_cache.data_ptr()),
-        block_tables.data_ptr<int>(), seq_lens.data_ptr<int>(), (float)scale,
-        nseq, nheads, kvh, head_dim, block_size, max_blocks, npart,
-        current_stream());
+    stream_decode(true);
     return;
   }
   if (!force_valu && q.scalar_type() == at::ScalarType::BFloat16 &&
       (head_dim == 64 || head_dim == 128) && group >= 1 && group <= 8 &&
-      nheads == kvh * group && nseq > 0) {
-    const int npart = decode_mfma_num_partitions(nseq, kvh, max_blocks * block_size);
-    const int P = npart * 4;
-    auto opts = q.options().dtype(at::ScalarType::Float);
-    auto part_acc = at::empty({nseq, nheads, P, head_dim}, opts);
-    auto part_ml = at::empty({nseq, nheads, P, 2}, opts);
-    launch_paged_decode_mfma(
-        reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
-        part_acc.data_ptr<float>(), part_ml.data_ptr<float>(),
-        reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()),
-        reinterpret_cast<const __hip_bfloat16*>(k_cache.data_ptr()),
-        reinterpret_cast<const __hip_bfloat16*>(v_cache.data_ptr()),
-        block_tables.data_ptr<int>(), seq_lens.data_ptr<int>(), (float)scale,
-        nseq, nheads, kvh, head_dim, block_size, max_blocks, npart,
-        current_stream());
+      nheads == kvh * group) {
+    stream_decode(false);
     return;
   }
   DISPATCH_FLOATING(q.scalar_type(), {
@@ -199,6 +196,7 @@ void paged_attention_prefill(torch::Tensor out, torch::Tensor q,
   const int kvh = k_cache.size(2);
   const int block_size = k_cache.size(1);
   const int max_blocks = block_tables.size(1);
+  if (!q.is_contiguous()) q = q.contiguous();   // the kernels read dense rows
   static const bool force_valu = [] {
     const char* e = getenv("VTA_PREFILL_VALU");
     return e && e[0] == '1';

@@ -46,7 +46,7 @@ _SEQ_SOURCES = ["stream_ops.hip", "canon_conv.hip", "layer_norm_stream.hip",
 # kernels without torch types that more than one extension links
 _SHARED_SOURCES = ["moe_gemm.hip"]
 _LAT_SOURCES = ["latent_attention.hip", "latent_attention_mfma.hip"]
-_ATTN_SOURCES = ["attention.hip", "attention_decode_mfma.hip",
+_ATTN_SOURCES = ["attention.hip", "attention_decode_mfma.hip", "attention_decode_stream.hip",
                  "attention_prefill_mfma.hip", "attention_prefill_mfma_v2.hip"]
 
 EXTENSIONS = {

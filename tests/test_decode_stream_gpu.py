@@ -1,0 +1,62 @@
+"""Decode attention kernel (attention_decode_stream.hip) against the reference op:
+tile, page and split edges, both caches."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# around the 32-key tile, the four-tile share of a workgroup, and a cut sequence;
+# 0: a padding row of a captured batch
+EDGES = [1, 15, 16, 17, 31, 32, 33, 0, 63, 65, 127, 128, 129, 255, 257, 700]
+
+
+def _caches(lens, block, kvh, hd, fp8, seed, width):
+    g = torch.Generator().manual_seed(seed)
+    need = [-(-n // block) for n in lens]
+    ids = torch.randperm(sum(need) + 3, generator=g).tolist()
+    tables = torch.zeros(len(lens), width, dtype=torch.int32)
+    for i, n in enumerate(need):
+        tables[i, :n] = torch.tensor([ids.pop() for _ in range(n)], dtype=torch.int32)
+    kc, vc = (torch.randn(sum(need) + 3, block, kvh, hd, generator=g).bfloat16() for _ in "kv")
+    if fp8:
+        kc, vc = (c.to(torch.float8_e4m3fn).view(torch.uint8) for c in (kc, vc))
+    return kc, vc, tables
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize(("kvh", "group", "hd", "block", "lens", "width"), [
+    (8, 4, 128, 16, EDGES, 512),        # cut by the longest context the table takes
+    (8, 4, 128, 16, EDGES, 44),         # fewer cuts
+    (2, 8, 64, 16, EDGES, 512),
+    (1, 1, 128, 8, [5000], 640),        # one head: as many cuts as there can be
+    (1, 7, 64, 24, [3, 1000, 2999], 128),   # pages of no power of two
+    (32, 1, 64, 1, [40, 77], 80),
+    (8, 4, 128, 16, [97] * 200, 8),     # a batch that fills the chip: no cuts
+])
+def test_matches_the_reference(fp8, kvh, group, hd, block, lens, width):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from vllm_tgis_adapter_amd import ops
+    from vllm_tgis_adapter_amd.ops import reference as R
+
+    kc, vc, tables = _caches(lens, block, kvh, hd, fp8, 3, width)
+    q = torch.randn(len(lens), kvh * group, hd,
+                    generator=torch.Generator().manual_seed(4)).bfloat16()
+    seq_lens = torch.tensor(lens, dtype=torch.int32)
+    out = ops.paged_attention_decode(q.cuda(), kc.cuda(), vc.cuda(), tables.cuda(),
+                                     seq_lens.cuda(), hd ** -0.5, max(lens)).float().cpu()
+    if fp8:
+        kc, vc = (c.view(torch.float8_e4m3fn) for c in (kc, vc))
+    live = [i for i, n in enumerate(lens) if n]
+    want = R.paged_attention(
+        q[live].float(), kc.float(), vc.float(), tables[live],
+        torch.arange(len(live) + 1, dtype=torch.int32), seq_lens[live], hd ** -0.5)
+    # probabilities and the result are rounded to bf16: half a unit in the last of 8
+    # bits each, of a weighted mean of values
+    bound = 2 ** -8 * vc.float().abs().max()
+    assert (out[live] - want).abs().max() <= bound
+    assert torch.equal(out[[i for i, n in enumerate(lens) if not n]],
+                       torch.zeros(len(lens) - len(live), kvh * group, hd))
