@@ -60,9 +60,13 @@ void launch_reshape_and_cache_fp8(const __hip_bfloat16*,
                                   const __hip_bfloat16*, unsigned char*,
                                   unsigned char*, const long*, int, int, long,
                                   long, hipStream_t);
-void launch_gemm_skinny_q(__hip_bfloat16*, float*, const __hip_bfloat16*,
-                          const unsigned char*, const float*, int, int, int,
-                          int, int, hipStream_t);
+int gemm_stream_parts(int M, int N, int K, bool gated);
+void launch_gemm_stream(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hip_bfloat16*,
+                        int, int, int, int, hipStream_t);
+void launch_gemm_stream_gated(__hip_bfloat16*, float*, const __hip_bfloat16*,
+                              const __hip_bfloat16*, int, int, int, int, hipStream_t);
+void launch_gemm_stream_q(__hip_bfloat16*, float*, const __hip_bfloat16*, const unsigned char*,
+                          const float*, int, int, int, int, int, hipStream_t);
 void launch_gemm_skinny(__hip_bfloat16*, float*, const __hip_bfloat16*,
                         const __hip_bfloat16*, int, int, int, int,
                         hipStream_t);
@@ -276,6 +280,13 @@ void gemm_tile(torch::Tensor y, torch::Tensor x, torch::Tensor w) {
                    K, current_stream());
 }
 
+// f32 space for the parts of a result that the streaming products leave for a merge
+float* stream_parts(torch::Tensor& space, const torch::Tensor& x, int parts, int64_t elems) {
+  if (parts <= 1) return nullptr;
+  space = at::empty({parts, elems}, x.options().dtype(at::ScalarType::Float));
+  return space.data_ptr<float>();
+}
+
 void gemm_skinny(torch::Tensor y, torch::Tensor x, torch::Tensor w) {
   const int M = x.size(0);
   const int K = x.size(1);
@@ -285,8 +296,15 @@ void gemm_skinny(torch::Tensor y, torch::Tensor x, torch::Tensor w) {
   TORCH_CHECK(x.is_contiguous() && w.is_contiguous() && y.is_contiguous());
   TORCH_CHECK(M >= 1 && N % 128 == 0 && K % 64 == 0);
   TORCH_CHECK(w.size(1) == K && y.size(0) == M && y.size(1) == N);
-  const int KS = gemm_skinny_num_ksplit(N, K, M);
   torch::Tensor part;
+  if (M <= 64) {
+    const int parts = gemm_stream_parts(M, N, K, false);
+    launch_gemm_stream(ptr<__hip_bfloat16>(y), stream_parts(part, x, parts, (int64_t)M * N),
+                       cptr<__hip_bfloat16>(x), cptr<__hip_bfloat16>(w), M, N, K, parts,
+                       current_stream());
+    return;
+  }
+  const int KS = gemm_skinny_num_ksplit(N, K, M);
   float* pp = nullptr;
   if (KS > 1) {
     part = at::empty({KS, M, N}, x.options().dtype(at::ScalarType::Float));
@@ -312,18 +330,13 @@ void gemm_skinny_q(torch::Tensor y, torch::Tensor x, torch::Tensor wq,
   TORCH_CHECK(M >= 1 && M <= 64 && N % 128 == 0 && K % 128 == 0);
   TORCH_CHECK(qbits == 8 || qbits == 4);
   TORCH_CHECK(wq.size(1) == (qbits == 8 ? K : K / 2));
-  const int KS = gemm_skinny_num_ksplit(N, K, M);
+  TORCH_CHECK(y.size(0) == M && y.size(1) == N && x.size(1) == K);
+  TORCH_CHECK(wscale.numel() == (qbits == 8 ? (int64_t)N : (int64_t)N * (K / 128)));
+  const int parts = gemm_stream_parts(M, N, K, false);
   torch::Tensor part;
-  float* pp = nullptr;
-  if (KS > 1) {
-    part = at::empty({KS, M, N}, x.options().dtype(at::ScalarType::Float));
-    pp = part.data_ptr<float>();
-  }
-  launch_gemm_skinny_q(
-      reinterpret_cast<__hip_bfloat16*>(y.data_ptr()), pp,
-      reinterpret_cast<const __hip_bfloat16*>(x.data_ptr()),
-      reinterpret_cast<const unsigned char*>(wq.data_ptr()),
-      wscale.data_ptr<float>(), (int)qbits, M, N, K, KS, current_stream());
+  launch_gemm_stream_q(ptr<__hip_bfloat16>(y), stream_parts(part, x, parts, (int64_t)M * N),
+                       cptr<__hip_bfloat16>(x), cptr<unsigned char>(wq),
+                       wscale.data_ptr<float>(), (int)qbits, M, N, K, parts, current_stream());
 }
 
 void gemm_skinny_gated(torch::Tensor y, torch::Tensor x, torch::Tensor w13) {
@@ -336,8 +349,16 @@ void gemm_skinny_gated(torch::Tensor y, torch::Tensor x, torch::Tensor w13) {
   TORCH_CHECK(M >= 1 && I % 128 == 0 && K % 64 == 0);
   TORCH_CHECK(w13.size(0) % 2 == 0 && w13.size(1) == K);
   TORCH_CHECK(y.size(0) == M && y.size(1) == I);
-  const int KS = gemm_skinny_num_ksplit(I, K, M);
   torch::Tensor part;
+  if (M <= 64) {
+    const int parts = gemm_stream_parts(M, I, K, true);
+    launch_gemm_stream_gated(ptr<__hip_bfloat16>(y),
+                             stream_parts(part, x, parts, (int64_t)2 * M * I),
+                             cptr<__hip_bfloat16>(x), cptr<__hip_bfloat16>(w13), M, I, K, parts,
+                             current_stream());
+    return;
+  }
+  const int KS = gemm_skinny_num_ksplit(I, K, M);
   float* pp = nullptr;
   if (KS > 1) {
     part = at::empty({KS, 2, M, I}, x.options().dtype(at::ScalarType::Float));

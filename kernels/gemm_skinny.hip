@@ -1,24 +1,8 @@
 #include <cstdlib>
-// Skinny decode GEMM (M <= 64): y[M,N] = x[M,K] · W[N,K]^T, bf16 in/out.
-//
-// hipBLASLt's picks for the llama decode shapes run at 22-43% of the HBM
-// roofline (tools/gemm_bench.py, r1).  v1 of this kernel read MFMA fragments
-// straight from HBM; per-lane 16B pieces of 16 rows made every access a
-// scattered line request and each workgroup re-read all of x (the W stream
-// evicts x from L2), so useful bandwidth capped at ~1.8 TB/s.  v2 is a real
-// tiled GEMM shaped for the streaming bound:
-//   - grid (N/128, KS): each workgroup owns 128 W rows and 1/KS of K.
-//     KS (pure shape function, hipGraph-safe) tops the grid up to >=512
-//     workgroups; KS>1 writes f32 partials merged by a tiny second kernel.
-//   - per 64-k chunk, W[128, 64] (16 KB) and x[64, 64] (8 KB) tiles are
-//     staged HBM->LDS with 128B-contiguous-per-row coalescing, XOR-swizzled
-//     ((row&7)<<4, guide G4) so the 16-rows-per-lane fragment reads are
-//     bank-conflict-free; double-buffered so chunk c+1 streams while c
-//     computes.  x is read once per WG (amortized over 128 N rows).
-//   - each wave owns NT=2 16-row n-tiles; per 32-k slice it does
-//     NT*MT v_mfma_f32_16x16x32_bf16 with both operands from LDS.
-//
-// x rows past M are staged as zeros; output rows past M are never written.
+// bf16 products of more than 64 rows that are sent here and not to the library
+// (gemm_stream.hip has the smaller ones): a 128x128 macro-tile, and its gated form.
+// Chunks of 64 inputs go through registers into swizzled, double-buffered LDS; K is
+// cut over workgroups until there are 512 of them, with a merge kernel.
 
 #include "common.h"
 
@@ -36,137 +20,6 @@ typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 DEVINLINE int swz(int row, int byte_in_row) {
   return row * (GS_KB * 2) + (byte_in_row ^ ((row & 7) << 4));
 }
-
-template <int MT>  // m tiles of 16 rows per workgroup (up to 8 = 128 rows)
-__global__ __launch_bounds__(256, 2) void gemm_skinny_kernel(
-    __hip_bfloat16* __restrict__ y,  // [M, N]   (KS == 1)
-    float* __restrict__ part,        // [KS, M, N] f32 (KS > 1; else null)
-    const __hip_bfloat16* __restrict__ x,  // [M, K]
-    const __hip_bfloat16* __restrict__ w,  // [N, K]
-    const int M,
-    const int N,
-    const int K) {
-  const int n_blk = blockIdx.x;      // which 128-row block of W
-  const int ks = blockIdx.y;
-  const int m0 = blockIdx.z * (MT * 16);  // this workgroup's m rows
-  const int KS = gridDim.y;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int row16 = lane & 15;
-  const int kq = lane >> 4;
-
-  const int k_per_wg = K / KS;
-  const int k_lo = ks * k_per_wg;
-  const int nchunks = k_per_wg / GS_KB;
-  const long n_base = (long)n_blk * GS_ROWS;
-
-  constexpr int XROWS = MT * 16;
-  constexpr int XPASS = (XROWS + 31) / 32;
-  __shared__ __hip_bfloat16 w_lds[2][GS_ROWS * GS_KB];
-  __shared__ __hip_bfloat16 x_lds[2][XROWS * GS_KB];
-
-  // ---- staging: 256 threads, 8 per row (8 x 16 B = 128 B contiguous) -----
-  const int st_row = tid / 8;        // 0..31 per pass
-  const int st_byte = (tid & 7) * 16;
-  const __hip_bfloat16* w_base = w + (n_base + st_row) * (long)K + k_lo + st_byte / 2;
-  const __hip_bfloat16* x_base =
-      x + (long)(m0 + st_row) * K + k_lo + st_byte / 2;
-
-  bf16x8_t st_w[GS_ROWS / 32];       // 4 passes of W
-  bf16x8_t st_x[XPASS];              // x rows m0 .. m0+XROWS
-  auto stage_load = [&](int chunk) {
-    const int koff = chunk * GS_KB;
-#pragma unroll
-    for (int p = 0; p < GS_ROWS / 32; ++p)
-      st_w[p] = *reinterpret_cast<const bf16x8_t*>(w_base + (long)(p * 32) * K + koff);
-#pragma unroll
-    for (int p = 0; p < XPASS; ++p) {
-      const int r = p * 32 + st_row;
-      st_x[p] = bf16x8_t{};
-      if (r < XROWS && m0 + r < M)
-        st_x[p] = *reinterpret_cast<const bf16x8_t*>(x_base + (long)(p * 32) * K + koff);
-    }
-  };
-  auto stage_write = [&](int buf) {
-#pragma unroll
-    for (int p = 0; p < GS_ROWS / 32; ++p)
-      *reinterpret_cast<bf16x8_t*>(
-          reinterpret_cast<char*>(w_lds[buf]) + swz(p * 32 + st_row, st_byte)) = st_w[p];
-#pragma unroll
-    for (int p = 0; p < XPASS; ++p) {
-      const int r = p * 32 + st_row;
-      if (r < XROWS)
-        *reinterpret_cast<bf16x8_t*>(
-            reinterpret_cast<char*>(x_lds[buf]) + swz(r, st_byte)) = st_x[p];
-    }
-  };
-
-  f32x4_t acc[GS_NT][MT];
-#pragma unroll
-  for (int nt = 0; nt < GS_NT; ++nt)
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = f32x4_t{};
-
-  // T14 pipeline (guide §5): write chunk c from regs (its loads had a full
-  // iteration to land), immediately re-issue loads for c+1 into the same
-  // regs, barrier, compute c.  No load-latency stall inside the loop.
-  stage_load(0);
-
-  for (int c = 0; c < nchunks; ++c) {
-    const int buf = c & 1;
-    stage_write(buf);
-    if (c + 1 < nchunks) stage_load(c + 1);
-    __syncthreads();  // chunk c staged for everyone
-
-#pragma unroll
-    for (int kc = 0; kc < 2; ++kc) {
-      const int byte = kc * 64 + kq * 16;
-      bf16x8_t a[GS_NT], b[MT];
-#pragma unroll
-      for (int nt = 0; nt < GS_NT; ++nt) {
-        const int r = (wave * GS_NT + nt) * 16 + row16;
-        a[nt] = *reinterpret_cast<const bf16x8_t*>(
-            reinterpret_cast<const char*>(w_lds[buf]) + swz(r, byte));
-      }
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        b[mt] = *reinterpret_cast<const bf16x8_t*>(
-            reinterpret_cast<const char*>(x_lds[buf]) + swz(mt * 16 + row16, byte));
-      }
-#pragma unroll
-      for (int nt = 0; nt < GS_NT; ++nt)
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-          acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[nt], b[mt], acc[nt][mt], 0, 0, 0);
-    }
-  }
-
-  // ---- epilogue: C frag D[n_local = kq*4+reg][m = row16] per (nt, mt) ----
-#pragma unroll
-  for (int nt = 0; nt < GS_NT; ++nt) {
-    const long n0 = n_base + (wave * GS_NT + nt) * 16 + kq * 4;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int m = m0 + mt * 16 + row16;
-      if (m >= M) continue;
-      if (part == nullptr) {
-        // pack 4 f32 -> 4 bf16 (8 B) at y[m][n0..n0+4)
-        union { unsigned u[2]; } o;
-        asm volatile("v_cvt_pk_bf16_f32 %0, %1, %2"
-                     : "=v"(o.u[0]) : "v"(acc[nt][mt][0]), "v"(acc[nt][mt][1]));
-        asm volatile("v_cvt_pk_bf16_f32 %0, %1, %2"
-                     : "=v"(o.u[1]) : "v"(acc[nt][mt][2]), "v"(acc[nt][mt][3]));
-        *reinterpret_cast<unsigned*>(y + (long)m * N + n0) = o.u[0];
-        *reinterpret_cast<unsigned*>(y + (long)m * N + n0 + 2) = o.u[1];
-      } else {
-        float* p = part + ((long)ks * M + m) * N + n0;
-        *reinterpret_cast<f32x4_t*>(p) = acc[nt][mt];
-      }
-    }
-  }
-}
-
 
 // ---------------------------------------------------------------------------
 // Large-M tiled GEMM (M > 64): classic 128x128 macro-tile on
@@ -322,17 +175,8 @@ void launch_gemm_skinny(__hip_bfloat16* y, float* part, const __hip_bfloat16* x,
                         hipStream_t stream) {
   dim3 block(256);
   float* p = KS > 1 ? part : nullptr;
-#define GS_CASE(MT, ZB)                                                      \
-  hipLaunchKernelGGL(gemm_skinny_kernel<MT>, dim3(N / GS_ROWS, KS, ZB),      \
-                     block, 0, stream, y, p, x, w, M, N, K)
-  if (M <= 16) GS_CASE(1, 1);
-  else if (M <= 32) GS_CASE(2, 1);
-  else if (M <= 64) GS_CASE(4, 1);
-  else
-    hipLaunchKernelGGL(gemm_tile_kernel,
-                       dim3(N / 128, KS, (M + 127) / 128), block, 0, stream,
-                       y, p, x, w, M, N, K);
-#undef GS_CASE
+  hipLaunchKernelGGL(gemm_tile_kernel, dim3(N / 128, KS, (M + 127) / 128), block, 0, stream, y,
+                     p, x, w, M, N, K);
   if (KS > 1) {
     const long total = (long)M * N;
     hipLaunchKernelGGL(gemm_skinny_merge_kernel,
@@ -510,15 +354,8 @@ void launch_gemm_skinny_gated(__hip_bfloat16* y, float* part,
                               int KS, hipStream_t stream) {
   dim3 block(256);
   float* p = KS > 1 ? part : nullptr;
-#define GG_CASE(MT, ZB)                                                       \
-  hipLaunchKernelGGL(gemm_skinny_gated_kernel<MT>,                            \
-                     dim3(I / GS_ROWS, KS, ZB), block, 0, stream, y,          \
-                     p, x, w13, M, I, K)
-  if (M <= 16) GG_CASE(1, 1);
-  else if (M <= 32) GG_CASE(2, 1);
-  else if (M <= 64) GG_CASE(4, 1);
-  else GG_CASE(8, (M + 127) / 128);
-#undef GG_CASE
+  hipLaunchKernelGGL(gemm_skinny_gated_kernel<8>, dim3(I / GS_ROWS, KS, (M + 127) / 128), block,
+                     0, stream, y, p, x, w13, M, I, K);
   if (KS > 1) {
     const long total = (long)M * I;
     hipLaunchKernelGGL(gemm_gated_merge_kernel,

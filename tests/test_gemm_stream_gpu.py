@@ -1,0 +1,81 @@
+"""Products of few rows (gemm_stream.hip) against float64: every way of cutting them,
+edges of the 16-row tiles, K that ends in half a tile."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+ROWS = [1, 15, 16, 17, 23, 32, 33, 61, 64]
+# N, K: one workgroup's columns, K of a single tile and of half a last one, as many
+# columns as the other cuts take
+SHAPES = [(128, 64), (128, 128), (256, 192), (384, 1088), (5120, 256), (8192, 320), (256, 8192),
+          (1152, 4160)]
+
+
+def _need():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+
+
+def _x(m, k, seed):
+    g = torch.Generator("cuda").manual_seed(seed)
+    return torch.randn((m, k), generator=g, device="cuda").bfloat16()
+
+
+def _check(got, want, terms):
+    """Sums of `terms` products in float32, one rounding to bf16: half a unit in the
+    last of 8 bits of the value, and 2**-20 of the terms' size for the sums."""
+    assert got.dtype == torch.bfloat16
+    err = (got.double() - want).abs()
+    assert (err <= 2 ** -8 * want.abs() + 2 ** -20 * terms).all(), err.max().item()
+
+
+@pytest.mark.parametrize("m", ROWS)
+@pytest.mark.parametrize(("n", "k"), SHAPES)
+def test_plain(m, n, k):
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    x, w = _x(m, k, 1), _x(n, k, 2)
+    _check(ops.linear(x, w), x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t())
+
+
+@pytest.mark.parametrize("m", ROWS)
+@pytest.mark.parametrize(("n", "k"), SHAPES)
+def test_gated(m, n, k):
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    x, w = _x(m, k, 3), _x(2 * n, k, 4) / k ** 0.5
+    g, u = (x.double() @ w.double().t()).chunk(2, dim=1)
+    got = ops.gated_mlp_up(x, w)
+    # float32 sums are off by far less than the last rounding; exp and the division
+    # are good to 1e-5
+    want = torch.nn.functional.silu(g) * u
+    _check(got, want, 30 * (1 + g.abs()) * (1 + u.abs()))
+
+
+@pytest.mark.parametrize("qbits", [8, 4])
+@pytest.mark.parametrize("m", ROWS)
+@pytest.mark.parametrize(("n", "k"), [s for s in SHAPES if s[1] % 128 == 0])
+def test_rounded(qbits, m, n, k):
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    x, w = _x(m, k, 5), _x(n, k, 6)
+    w[0] = 0.0                      # a row of zeros has the smallest scale
+    w[1, : k // 2] = 64.0           # one group or half of a row far above the rest
+    wq, scale = ops.quantize_weight(w, qbits)
+    if qbits == 8:
+        exact = wq.double() * scale.double()[:, None]
+    else:
+        q = torch.stack([wq & 0xF, wq >> 4], dim=2).view(n, k // 128, 128).double() - 8.0
+        exact = (q * scale.double()[:, :, None]).view(n, k)
+    got = ops.linear_quant(x, wq, scale, qbits)
+    # 4 bits: sums of 8 + n/2 in place of n - 8, up to five times their size
+    _check(got, x.double() @ exact.t(), 5 * (x.double().abs() @ exact.abs().t()
+                                             + 4 * x.double().abs().sum(1, keepdim=True)
+                                             * exact.abs().amax(1) / 4))
