@@ -82,9 +82,15 @@ void launch_lora_expand(T*, const float*, const T*, const int*, const float*,
 template <typename T>
 void launch_sample_argmax(long*, const T*, const float*, const float*, int,
                           int, hipStream_t);
-void launch_moe_gemm(__hip_bfloat16*, const __hip_bfloat16*,
-                     const __hip_bfloat16*, const int*, int, int, int, int,
+void launch_moe_gemm(__hip_bfloat16*, const __hip_bfloat16*, const __hip_bfloat16*, const int*,
+                     const int*, int, int, int, int, int, hipStream_t);
+int moe_topk_max_experts();
+int moe_topk_max_top();
+void launch_moe_topk(int*, float*, const __hip_bfloat16*, const __hip_bfloat16*, int, int, int,
                      int, hipStream_t);
+void launch_moe_group(int*, int*, int*, const int*, int, int, int, hipStream_t);
+void launch_moe_sum(__hip_bfloat16*, const __hip_bfloat16*, const int*, const float*, int, int,
+                    int, hipStream_t);
 
 // paged attention (bindings_attn.cpp, shared with the `_C_attn` extension)
 void register_attention_ops(pybind11::module& m);
@@ -402,9 +408,10 @@ void lora_bgmv(torch::Tensor out, torch::Tensor x, torch::Tensor a_stack,
 }
 
 void moe_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w,
-              torch::Tensor seg_off, int64_t mode) {
+              torch::Tensor seg_off, int64_t mode, c10::optional<torch::Tensor> rows) {
   // mode 0: plain, 1: silu(first half) * second half, 2: squared relu
-  const int T = x.size(0);
+  // rows: sorted row r is x[rows[r]]; without it x is sorted itself
+  const int T = rows.has_value() ? rows->numel() : x.size(0);
   const int K = x.size(1);
   const int E = w.size(0);
   const long wn = w.size(1);
@@ -419,12 +426,55 @@ void moe_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w,
   TORCH_CHECK(N % 128 == 0 && K % 64 == 0 && w.size(2) == K);
   TORCH_CHECK(y.size(0) == T && y.size(1) == N);
   TORCH_CHECK(x.is_contiguous() && w.is_contiguous() && y.is_contiguous());
+  const int* rp = nullptr;
+  if (rows.has_value()) {
+    TORCH_CHECK(rows->is_cuda() && rows->scalar_type() == at::ScalarType::Int &&
+                rows->is_contiguous());
+    rp = rows->data_ptr<int>();
+  }
   if (T == 0) return;
-  launch_moe_gemm(reinterpret_cast<__hip_bfloat16*>(y.data_ptr()),
-                  reinterpret_cast<const __hip_bfloat16*>(x.data_ptr()),
-                  reinterpret_cast<const __hip_bfloat16*>(w.data_ptr()),
-                  seg_off.data_ptr<int>(), E, N, K, T, (int)mode,
-                  current_stream());
+  launch_moe_gemm(ptr<__hip_bfloat16>(y), cptr<__hip_bfloat16>(x), cptr<__hip_bfloat16>(w),
+                  seg_off.data_ptr<int>(), rp, E, N, K, T, (int)mode, current_stream());
+}
+
+void moe_topk(torch::Tensor ids, torch::Tensor weights, torch::Tensor x, torch::Tensor gate) {
+  const int T = x.size(0), K = x.size(1), E = gate.size(0), top = ids.size(1);
+  TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::ScalarType::BFloat16 && x.is_contiguous() &&
+              gate.scalar_type() == at::ScalarType::BFloat16 && gate.is_contiguous() &&
+              gate.size(1) == K && K % 8 == 0);
+  TORCH_CHECK(E >= 1 && E <= moe_topk_max_experts() && top >= 1 && top <= E &&
+              top <= moe_topk_max_top());
+  TORCH_CHECK(ids.scalar_type() == at::ScalarType::Int && ids.is_contiguous() &&
+              ids.size(0) == T && weights.scalar_type() == at::ScalarType::Float &&
+              weights.is_contiguous() && weights.sizes() == ids.sizes());
+  if (T == 0) return;
+  launch_moe_topk(ids.data_ptr<int>(), weights.data_ptr<float>(), cptr<__hip_bfloat16>(x),
+                  cptr<__hip_bfloat16>(gate), T, E, K, top, current_stream());
+}
+
+void moe_group(torch::Tensor rows, torch::Tensor pos, torch::Tensor seg, torch::Tensor ids) {
+  // ids hold experts 0 .. seg.numel() - 2 only
+  const int pairs = ids.numel(), E = seg.numel() - 1;
+  for (const auto& t : {rows, pos, seg, ids})
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::ScalarType::Int && t.is_contiguous());
+  TORCH_CHECK(rows.numel() == pairs && pos.numel() == pairs && ids.dim() == 2 && E >= 1 &&
+              E <= moe_topk_max_experts());
+  launch_moe_group(rows.data_ptr<int>(), pos.data_ptr<int>(), seg.data_ptr<int>(),
+                   ids.data_ptr<int>(), pairs, E, (int)ids.size(1), current_stream());
+}
+
+void moe_sum(torch::Tensor out, torch::Tensor ye, torch::Tensor pos, torch::Tensor weights) {
+  const int T = pos.size(0), top = pos.size(1), H = ye.size(1);
+  TORCH_CHECK(ye.is_cuda() && ye.scalar_type() == at::ScalarType::BFloat16 &&
+              ye.is_contiguous() && ye.size(0) == (int64_t)T * top && H % 8 == 0);
+  TORCH_CHECK(out.scalar_type() == at::ScalarType::BFloat16 && out.is_contiguous() &&
+              out.size(0) == T && out.size(1) == H);
+  TORCH_CHECK(pos.scalar_type() == at::ScalarType::Int && pos.is_contiguous() &&
+              weights.scalar_type() == at::ScalarType::Float && weights.is_contiguous() &&
+              weights.sizes() == pos.sizes());
+  if (T == 0) return;
+  launch_moe_sum(ptr<__hip_bfloat16>(out), cptr<__hip_bfloat16>(ye), pos.data_ptr<int>(),
+                 weights.data_ptr<float>(), T, H, top, current_stream());
 }
 
 void sample_argmax(torch::Tensor out, torch::Tensor logits,
@@ -511,7 +561,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_skinny_gated", &gemm_skinny_gated,
         "fused gate/up skinny GEMM + SiLU-mul, M <= 64 (CDNA4 MFMA)");
   m.def("moe_gemm", &moe_gemm,
-        "grouped MoE GEMM over expert segments (CDNA4 MFMA)");
+        "grouped MoE GEMM over expert segments (CDNA4 MFMA)", py::arg("y"), py::arg("x"),
+        py::arg("w"), py::arg("seg_off"), py::arg("mode"), py::arg("rows") = py::none());
+  m.def("moe_topk", &moe_topk, "router product, choice and weights of a softmax router");
+  m.def("moe_group", &moe_group, "token-expert pairs grouped by expert");
+  m.def("moe_sum", &moe_sum, "weighted sum of each token's expert results");
+  m.def("moe_topk_max_experts", &moe_topk_max_experts);
+  m.def("moe_topk_max_top", &moe_topk_max_top);
   m.def("logsoftmax_topk", &logsoftmax_topk,
         "fused log-softmax + top-K + sampled-token rank (one HBM pass)");
   m.def("sample_argmax", &sample_argmax,

@@ -33,9 +33,8 @@ int moe_sort_small_pairs();
 template <typename T>
 void launch_moe_sort(T*, int*, int*, int*, const T*, long, const int*, int, int,
                      int, int, const float*, hipStream_t);
-void launch_moe_gemm(__hip_bfloat16*, const __hip_bfloat16*,
-                     const __hip_bfloat16*, const int*, int, int, int, int, int,
-                     hipStream_t);
+void launch_moe_gemm(__hip_bfloat16*, const __hip_bfloat16*, const __hip_bfloat16*, const int*,
+                     const int*, int, int, int, int, int, hipStream_t);
 void launch_moe_gemm_clamped(__hip_bfloat16*, const __hip_bfloat16*, const __hip_bfloat16*,
                              const int*, int, int, int, int, float, hipStream_t);
 
@@ -341,7 +340,7 @@ void moe_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w,
   TORCH_CHECK(x.is_contiguous() && w.is_contiguous() && y.is_contiguous());
   if (T == 0) return;
   launch_moe_gemm(ptr<__hip_bfloat16>(y), ptr<__hip_bfloat16>(x),
-                  ptr<__hip_bfloat16>(w), ptr<int>(seg_off), E, N, K, T, (int)mode,
+                  ptr<__hip_bfloat16>(w), ptr<int>(seg_off), nullptr, E, N, K, T, (int)mode,
                   stream());
 }
 

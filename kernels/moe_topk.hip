@@ -1,0 +1,208 @@
+// What surrounds the expert products of a softmax-routed mixture: router product and
+// choice, grouping of the token-expert pairs, and the weighted sum of the results.
+//
+// These took some 20 launches of tensor ops a layer (product, softmax, selection, sort,
+// histogram, prefix, gathers, scatter-add): all of them latency at decode sizes, and
+// several passes over [T k, H] at prompt sizes.  Three launches instead; the expert
+// product reads its rows through the list made here, so the gathered copy is gone, and
+// the sum is taken in f32 and rounded once.
+
+#include "common.h"
+
+namespace {
+
+constexpr int kTokens = 4;        // tokens of a workgroup
+constexpr int kMaxExperts = 64;
+constexpr int kMaxTop = 8;
+
+// ids, weights [T, top]: the top largest x[t]·gate[e] and their softmax among themselves.
+// The four waves cut K; a workgroup's tokens share what it reads of the gate matrix.
+// Bound by the latency of a few dependent loads at decode sizes, by x and the gate
+// matrix from L2 at prompt sizes.
+__global__ __launch_bounds__(256) void moe_topk_kernel(
+    int* __restrict__ ids, float* __restrict__ weights,
+    const __hip_bfloat16* __restrict__ x,     // [T, K]
+    const __hip_bfloat16* __restrict__ gate,  // [E, K]
+    const int T, const int E, const int K, const int top) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int t0 = blockIdx.x * kTokens;
+  __shared__ float part[4][kTokens][8];
+  __shared__ float logits[kTokens][kMaxExperts];
+
+  const int per = ((K / 8 + 3) / 4) * 8;      // inputs of a wave, in runs of 8
+  const int lo = wave * per, hi = min(lo + per, K);
+  for (int e0 = 0; e0 < E; e0 += 8) {
+    float acc[kTokens][8];
+#pragma unroll
+    for (int t = 0; t < kTokens; ++t)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[t][e] = 0.f;
+    for (int k = lo + lane * 8; k < hi; k += 512) {
+      Vec16<__hip_bfloat16> xv[kTokens], gv[8];
+#pragma unroll
+      for (int t = 0; t < kTokens; ++t) xv[t] = load16(x + (long)min(t0 + t, T - 1) * K + k);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) gv[e] = load16(gate + (long)min(e0 + e, E - 1) * K + k);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        float xf[kTokens];
+#pragma unroll
+        for (int t = 0; t < kTokens; ++t) xf[t] = __bfloat162float(xv[t].data[j]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float g = __bfloat162float(gv[e].data[j]);
+#pragma unroll
+          for (int t = 0; t < kTokens; ++t) acc[t][e] = __builtin_fmaf(xf[t], g, acc[t][e]);
+        }
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < kTokens; ++t)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float v = wave_reduce_sum(acc[t][e]);
+        if (lane == 0) part[wave][t][e] = v;
+      }
+    __syncthreads();
+    if (threadIdx.x < kTokens * 8) {
+      const int t = threadIdx.x / 8, e = threadIdx.x % 8;
+      if (e0 + e < E)
+        logits[t][e0 + e] = (part[0][t][e] + part[1][t][e]) + (part[2][t][e] + part[3][t][e]);
+    }
+    __syncthreads();
+  }
+
+  const int t = threadIdx.x;
+  if (t >= kTokens || t0 + t >= T) return;
+  // ties and NaN: the lowest expert that is left, so that every id is an expert
+  unsigned long long taken = 0;
+  int chosen[kMaxTop];
+  float value[kMaxTop], sum = 0.f;
+#pragma unroll
+  for (int j = 0; j < kMaxTop; ++j) {
+    if (j >= top) break;
+    int best = -1;
+    float v = 0.f;
+    for (int e = 0; e < E; ++e) {
+      if (taken >> e & 1) continue;
+      const float l = logits[t][e];
+      if (best < 0 || l > v) {
+        best = e;
+        v = l;
+      }
+    }
+    taken |= 1ull << best;
+    chosen[j] = best;
+    value[j] = v;
+  }
+  const float most = value[0];
+#pragma unroll
+  for (int j = 0; j < kMaxTop; ++j) {
+    if (j >= top) break;
+    value[j] = __expf(value[j] - most);
+    sum += value[j];
+  }
+#pragma unroll
+  for (int j = 0; j < kMaxTop; ++j) {
+    if (j >= top) break;
+    ids[(long)(t0 + t) * top + j] = chosen[j];
+    weights[(long)(t0 + t) * top + j] = value[j] / sum;
+  }
+}
+
+// Pairs p = t * top + j grouped by expert: seg [E + 1], pos[p] the sorted row of a pair,
+// rows[pos[p]] = t.  One workgroup: a few thousand pairs are less than a second launch.
+// A wave counts and claims places for all its lanes of one expert at a time.
+__global__ __launch_bounds__(1024) void moe_group_kernel(
+    int* __restrict__ rows, int* __restrict__ pos, int* __restrict__ seg,
+    const int* __restrict__ ids, const int pairs, const int E, const int top) {
+  __shared__ int count[kMaxExperts], next[kMaxExperts];
+  const int tid = threadIdx.x, lane = tid & 63;
+  for (int e = tid; e < E; e += 1024) count[e] = 0;
+  __syncthreads();
+  auto for_each = [&](auto take) {
+    for (int base = 0; base < pairs; base += 1024) {
+      const int p = base + tid;
+      const int e = p < pairs ? ids[p] : -1;
+      unsigned long long left = __ballot(e >= 0);
+      while (left) {
+        const int lead = __builtin_ctzll(left);
+        const int which = __shfl(e, lead, 64);
+        const unsigned long long same = __ballot(e == which);
+        take(p, e == which, which, same, lead);
+        left &= ~same;
+      }
+    }
+  };
+  for_each([&](int, bool, int which, unsigned long long same, int lead) {
+    if (lane == lead) atomicAdd(&count[which], __popcll(same));
+  });
+  __syncthreads();
+  if (tid == 0) {
+    int at = 0;
+    for (int e = 0; e < E; ++e) {
+      seg[e] = at;
+      next[e] = at;
+      at += count[e];
+    }
+    seg[E] = at;
+  }
+  __syncthreads();
+  for_each([&](int p, bool mine, int which, unsigned long long same, int lead) {
+    int at = 0;
+    if (lane == lead) at = atomicAdd(&next[which], __popcll(same));
+    at = __shfl(at, lead, 64);
+    if (mine) {
+      const int row = at + __popcll(same & ((1ull << lane) - 1));
+      pos[p] = row;
+      rows[row] = p / top;
+    }
+  });
+}
+
+// out[t] = sum_j weights[t, j] ye[pos[t, j]], in f32, rounded once.  Bound by the bytes
+// of ye and out.
+__global__ __launch_bounds__(256) void moe_sum_kernel(
+    __hip_bfloat16* __restrict__ out,       // [T, H]
+    const __hip_bfloat16* __restrict__ ye,  // [T * top, H]
+    const int* __restrict__ pos, const float* __restrict__ weights, const int H,
+    const int top) {
+  const long t = blockIdx.x;
+  for (int h = threadIdx.x * 8; h < H; h += 2048) {
+    float acc[8] = {};
+    for (int j = 0; j < top; ++j) {
+      const float w = weights[t * top + j];
+      const Vec16<__hip_bfloat16> v = load16(ye + (long)pos[t * top + j] * H + h);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc[i] = __builtin_fmaf(w, __bfloat162float(v.data[i]), acc[i]);
+    }
+    Vec16<__hip_bfloat16> o;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o.data[i] = __float2bfloat16(acc[i]);
+    store16(out + t * H + h, o);
+  }
+}
+
+}  // namespace
+
+int moe_topk_max_experts() { return kMaxExperts; }
+int moe_topk_max_top() { return kMaxTop; }
+
+void launch_moe_topk(int* ids, float* weights, const __hip_bfloat16* x,
+                     const __hip_bfloat16* gate, int T, int E, int K, int top,
+                     hipStream_t stream) {
+  hipLaunchKernelGGL(moe_topk_kernel, dim3((T + kTokens - 1) / kTokens), dim3(256), 0, stream,
+                     ids, weights, x, gate, T, E, K, top);
+}
+
+void launch_moe_group(int* rows, int* pos, int* seg, const int* ids, int pairs, int E, int top,
+                      hipStream_t stream) {
+  hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(1024), 0, stream, rows, pos, seg, ids,
+                     pairs, E, top);
+}
+
+void launch_moe_sum(__hip_bfloat16* out, const __hip_bfloat16* ye, const int* pos,
+                    const float* weights, int T, int H, int top, hipStream_t stream) {
+  hipLaunchKernelGGL(moe_sum_kernel, dim3(T), dim3(256), 0, stream, out, ye, pos, weights, H,
+                     top);
+}

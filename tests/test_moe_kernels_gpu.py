@@ -1,0 +1,115 @@
+"""Expert products and what surrounds them: every way the products are cut, empty and
+uneven segments, rows through a list, against float64 and the reference ops."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _need_gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+
+
+def _segments(counts):
+    seg = torch.zeros(len(counts) + 1, dtype=torch.int32)
+    seg[1:] = torch.tensor(counts).cumsum(0)
+    return seg
+
+
+# rows per expert: one pair, means at and around each line of the rule (9, 18, 52, 250),
+# empty experts, one expert with everything, more experts than lanes of a wave
+COUNTS = [
+    [0, 1, 0], [9, 9], [16, 1, 0, 17, 11], [18, 20, 16], [19, 19, 40, 0], [52, 52], [53, 130, 0],
+    [64, 65, 127, 1], [249, 250], [250, 250], [300, 1, 513, 256], [0, 0, 700],
+    [3] * 70, [0] * 65 + [40, 0, 2],
+]
+
+
+@pytest.mark.parametrize("mode", ["plain", "silu", "relu2", "clamped"])
+@pytest.mark.parametrize("counts", COUNTS, ids=str)
+@pytest.mark.parametrize(("n", "k"), [(128, 64), (256, 320)])
+@pytest.mark.parametrize("listed", [False, True])
+def test_products(mode, counts, n, k, listed):
+    from vllm_tgis_adapter_amd import ops
+
+    g = torch.Generator("cuda").manual_seed(len(counts) + n)
+    seg = _segments(counts)
+    total, experts = int(seg[-1]), len(counts)
+    gated = mode in ("silu", "clamped")
+    w = torch.randn((experts, (2 if gated else 1) * n, k), generator=g,
+                    device="cuda").bfloat16() / k ** 0.5
+    rows = None
+    if listed:
+        x = torch.randn((max(total // 2, 1), k), generator=g, device="cuda").bfloat16()
+        rows = torch.randint(len(x), (total,), generator=g, device="cuda", dtype=torch.int32)
+        xs = x[rows.long()]
+    else:
+        x = xs = torch.randn((total, k), generator=g, device="cuda").bfloat16()
+    act = {"relu2": "relu2", "clamped": "clamped"}.get(mode)
+    got = ops.moe_gemm(x, w, seg.cuda(), gated, act=act, limit=1.5, rows=rows)
+    assert got.shape == (total, n)
+    for e in range(experts):
+        lo, hi = int(seg[e]), int(seg[e + 1])
+        s = xs[lo:hi].double() @ w[e].double().t()
+        if gated:
+            a, u = s.chunk(2, dim=1)
+            if mode == "clamped":
+                a, u = a.clamp(max=1.5), u.clamp(-1.5, 1.5)
+                s = a * torch.sigmoid(1.702 * a) * (u + 1)
+            else:
+                s = torch.nn.functional.silu(a) * u
+        elif mode == "relu2":
+            s = s.clamp(min=0).square()
+        # one rounding to bf16; float32 sums of up to 320 terms and exp below 1e-5
+        err = (got[lo:hi].double() - s).abs()
+        assert (err <= 2 ** -8 * s.abs() + 1e-4).all(), (e, err.max().item())
+
+
+@pytest.mark.parametrize("tokens", [1, 3, 4, 5, 33, 1030])
+@pytest.mark.parametrize(("experts", "top", "k"), [(8, 2, 4096), (1, 1, 64), (9, 3, 200),
+                                                   (64, 8, 512)])
+def test_router_grouping_and_sum(tokens, experts, top, k):
+    from vllm_tgis_adapter_amd import ops
+
+    g = torch.Generator("cuda").manual_seed(tokens)
+    x = torch.randn((tokens, k), generator=g, device="cuda").bfloat16()
+    gate = torch.randn((experts, k), generator=g, device="cuda").bfloat16() / k ** 0.5
+    ids, weights = ops.moe_topk(x, gate, top)
+    logits = x.double() @ gate.double().t()
+    assert (ids.sort(dim=1).values.diff(dim=1) > 0).all()       # no expert twice
+    chosen = logits.gather(1, ids.long())
+    # float32 sums: what was chosen is the largest up to their error
+    assert (chosen - logits.topk(top, dim=1).values).abs().max() <= 1e-5 * k ** 0.5
+    torch.testing.assert_close(weights.double(), chosen.softmax(dim=1), atol=1e-5, rtol=1e-4)
+
+    rows, pos, seg = ops.moe_group(ids, experts)
+    count = torch.bincount(ids.view(-1).long(), minlength=experts)
+    assert torch.equal(seg[1:].long(), count.cumsum(0)) and seg[0] == 0
+    flat = pos.view(-1).long()
+    assert torch.equal(flat.sort().values, torch.arange(tokens * top, device="cuda"))
+    assert torch.equal(rows[flat].long(),
+                       torch.arange(tokens, device="cuda").repeat_interleave(top))
+    e = ids.view(-1).long()
+    assert (flat >= seg[e]).all() and (flat < seg[e + 1]).all()
+
+    ye = torch.randn((tokens * top, 264), generator=g, device="cuda").bfloat16()
+    got = ops.moe_sum(ye, pos, weights)
+    want = (ye[pos.long()].double() * weights.double()[..., None]).sum(dim=1)
+    assert ((got.double() - want).abs() <= 2 ** -8 * want.abs() + 1e-5).all()
+
+
+def test_router_of_equal_and_undefined_scores_names_experts():
+    from vllm_tgis_adapter_amd import ops
+
+    gate = torch.ones((8, 64), device="cuda").bfloat16()
+    x = torch.ones((3, 64), device="cuda").bfloat16()
+    x[1, 0] = float("nan")
+    x[2, 0] = float("inf")
+    ids, weights = ops.moe_topk(x, gate, 2)
+    assert ids.tolist() == [[0, 1]] * 3
+    assert weights[0].tolist() == [0.5, 0.5] and weights[1].isnan().all()

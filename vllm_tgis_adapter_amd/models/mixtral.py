@@ -104,6 +104,14 @@ class MoEBlock(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:  # [T, H]
         t = x.shape[0]
+        if (not self.ep and ops.moe_gemm_usable(x, self.hidden, self.inter)
+                and ops.moe_route_usable(x, self.gate, self.top_k)):
+            # the products read their rows through the list of the grouping
+            ids, weights = ops.moe_topk(x, self.gate, self.top_k)
+            rows, pos, seg = ops.moe_group(ids, self.num_experts)
+            h = ops.moe_gemm(x, self.w13, seg, gated=True, rows=rows)
+            ye = ops.moe_gemm(h, self.w2, seg, gated=False)
+            return tp_all_reduce(ops.moe_sum(ye, pos, weights))
         router_logits = F.linear(x, self.gate)           # [T, E]
         weights, ids = ops.topk_softmax(router_logits, self.top_k)  # [T, k]
         out = torch.zeros_like(x)

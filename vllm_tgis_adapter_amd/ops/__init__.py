@@ -384,6 +384,7 @@ def moe_gemm(
     gated: bool,
     act: str | None = None,
     limit: float = 0.0,
+    rows: torch.Tensor | None = None,  # [T] int32: sorted row r is x[rows[r]]
 ) -> torch.Tensor:
     """Grouped GEMM over expert segments (E16); gated fuses SiLU(g)*u, or with
     act "clamped" the clamped gate (see clamped_glu); a plain product may be
@@ -392,8 +393,15 @@ def moe_gemm(
     if act not in ((None, "clamped") if gated else (None, "relu2")):
         raise ValueError(f"unknown activation {act!r}")
     n = w.shape[1] // 2 if gated else w.shape[1]
+    if rows is not None and (x.device.type != "cuda" or _FORCE_REFERENCE or _C is None
+                             or act == "clamped"):
+        x, rows = x[rows.long()], None
     if x.device.type != "cuda" or _FORCE_REFERENCE:
         return reference.moe_gemm(x, w, seg_off.cpu(), gated, act, limit)
+    if rows is not None:
+        out = torch.empty((rows.shape[0], n), dtype=x.dtype, device=x.device)
+        _C.moe_gemm(out, x, w, seg_off, 1 if gated else (2 if act == "relu2" else 0), rows)
+        return out
     out = torch.empty((x.shape[0], n), dtype=x.dtype, device=x.device)
     if act == "clamped":
         _native_seq(x)
@@ -412,6 +420,47 @@ def moe_gemm_usable(x: torch.Tensor, hidden: int, inter: int) -> bool:
         and hidden % 128 == 0
         and hidden % 64 == 0
     )
+
+
+def moe_route_usable(x: torch.Tensor, gate: torch.Tensor, top_k: int) -> bool:
+    """Whether moe_topk and moe_group take this router (a softmax over up to 64
+    experts, up to 8 chosen)."""
+    return (
+        native_enabled(x)
+        and x.dtype == torch.bfloat16
+        and gate.dtype == torch.bfloat16
+        and x.shape[1] % 8 == 0
+        and gate.shape[0] <= _C.moe_topk_max_experts()
+        and 1 <= top_k <= min(gate.shape[0], _C.moe_topk_max_top())
+    )
+
+
+def moe_topk(x: torch.Tensor, gate: torch.Tensor, top_k: int):
+    """Router of a mixture: ids [T, top_k] int32 of the largest x @ gate^T and the
+    softmax among them [T, top_k] f32; one launch (GPU only)."""
+    t = x.shape[0]
+    ids = torch.empty((t, top_k), dtype=torch.int32, device=x.device)
+    w = torch.empty((t, top_k), dtype=torch.float32, device=x.device)
+    _C.moe_topk(ids, w, x.contiguous(), gate)
+    return ids, w
+
+
+def moe_group(ids: torch.Tensor, experts: int):
+    """The pairs ids [T, k] grouped by expert (GPU only): rows [T * k] int32, the token
+    of each sorted row; pos [T, k] int32, the sorted row of each pair; seg [experts + 1]
+    int32.  The order inside a segment is not specified."""
+    rows = torch.empty(ids.numel(), dtype=torch.int32, device=ids.device)
+    pos = torch.empty_like(ids)
+    seg = torch.empty(experts + 1, dtype=torch.int32, device=ids.device)
+    _C.moe_group(rows, pos, seg, ids)
+    return rows, pos, seg
+
+
+def moe_sum(ye: torch.Tensor, pos: torch.Tensor, weights: torch.Tensor) -> torch.Tensor:
+    """out[t] = sum_k weights[t, k] * ye[pos[t, k]], f32 inside (GPU only)."""
+    out = torch.empty((pos.shape[0], ye.shape[1]), dtype=ye.dtype, device=ye.device)
+    _C.moe_sum(out, ye, pos, weights)
+    return out
 
 
 def topk_softmax(gate_logits: torch.Tensor, top_k: int):
