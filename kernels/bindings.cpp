@@ -60,7 +60,7 @@ void launch_reshape_and_cache_fp8(const __hip_bfloat16*,
                                   const __hip_bfloat16*, unsigned char*,
                                   unsigned char*, const long*, int, int, long,
                                   long, hipStream_t);
-int gemm_stream_parts(int M, int N, int K, bool gated);
+int gemm_stream_parts(int qbits, int M, int N, int K, bool gated);
 void launch_gemm_stream(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hip_bfloat16*,
                         int, int, int, int, hipStream_t);
 void launch_gemm_stream_gated(__hip_bfloat16*, float*, const __hip_bfloat16*,
@@ -73,6 +73,10 @@ void launch_gemm_skinny(__hip_bfloat16*, float*, const __hip_bfloat16*,
 void launch_gemm_skinny_gated(__hip_bfloat16*, float*, const __hip_bfloat16*,
                               const __hip_bfloat16*, int, int, int, int,
                               hipStream_t);
+void launch_gemm_block_q(__hip_bfloat16*, const __hip_bfloat16*, const unsigned char*,
+                         const float*, int, int, int, int, hipStream_t);
+void launch_widen_weight(__hip_bfloat16*, const unsigned char*, const float*, int, long, int,
+                         hipStream_t);
 template <typename T>
 void launch_lora_shrink(float*, const T*, const T*, const int*, int, int, int,
                         hipStream_t);
@@ -304,7 +308,7 @@ void gemm_skinny(torch::Tensor y, torch::Tensor x, torch::Tensor w) {
   TORCH_CHECK(w.size(1) == K && y.size(0) == M && y.size(1) == N);
   torch::Tensor part;
   if (M <= 64) {
-    const int parts = gemm_stream_parts(M, N, K, false);
+    const int parts = gemm_stream_parts(16, M, N, K, false);
     launch_gemm_stream(ptr<__hip_bfloat16>(y), stream_parts(part, x, parts, (int64_t)M * N),
                        cptr<__hip_bfloat16>(x), cptr<__hip_bfloat16>(w), M, N, K, parts,
                        current_stream());
@@ -322,27 +326,49 @@ void gemm_skinny(torch::Tensor y, torch::Tensor x, torch::Tensor w) {
                      N, K, KS, current_stream());
 }
 
-void gemm_skinny_q(torch::Tensor y, torch::Tensor x, torch::Tensor wq,
-                   torch::Tensor wscale, int64_t qbits) {
-  const int M = x.size(0);
-  const int K = x.size(1);
-  const int N = wq.size(0);
-  TORCH_CHECK(x.scalar_type() == at::ScalarType::BFloat16);
+void check_rounded(const torch::Tensor& wq, const torch::Tensor& wscale, int64_t qbits,
+                   int64_t N, int64_t K) {
+  TORCH_CHECK(qbits == 8 || qbits == 4);
   TORCH_CHECK(wq.scalar_type() == at::ScalarType::Byte ||
               wq.scalar_type() == at::ScalarType::Char);
   TORCH_CHECK(wscale.scalar_type() == at::ScalarType::Float);
-  TORCH_CHECK(x.is_contiguous() && wq.is_contiguous() &&
-              wscale.is_contiguous() && y.is_contiguous());
-  TORCH_CHECK(M >= 1 && M <= 64 && N % 128 == 0 && K % 128 == 0);
-  TORCH_CHECK(qbits == 8 || qbits == 4);
-  TORCH_CHECK(wq.size(1) == (qbits == 8 ? K : K / 2));
-  TORCH_CHECK(y.size(0) == M && y.size(1) == N && x.size(1) == K);
-  TORCH_CHECK(wscale.numel() == (qbits == 8 ? (int64_t)N : (int64_t)N * (K / 128)));
-  const int parts = gemm_stream_parts(M, N, K, false);
+  TORCH_CHECK(wq.is_cuda() && wq.is_contiguous() && wscale.is_contiguous());
+  TORCH_CHECK(N % 128 == 0 && K % 128 == 0);
+  TORCH_CHECK(wq.size(0) == N && wq.size(1) == (qbits == 8 ? K : K / 2));
+  TORCH_CHECK(wscale.numel() == (qbits == 8 ? N : N * (K / 128)));
+}
+
+// y = x W^T for rounded weights, any number of rows
+void gemm_q(torch::Tensor y, torch::Tensor x, torch::Tensor wq, torch::Tensor wscale,
+            int64_t qbits) {
+  const int M = x.size(0), K = x.size(1), N = wq.size(0);
+  check_rounded(wq, wscale, qbits, N, K);
+  TORCH_CHECK(x.scalar_type() == at::ScalarType::BFloat16 &&
+              y.scalar_type() == at::ScalarType::BFloat16);
+  TORCH_CHECK(x.is_contiguous() && y.is_contiguous() && M >= 1);
+  TORCH_CHECK(y.size(0) == M && y.size(1) == N);
+  // rows of a block of W are found by 32 bits
+  TORCH_CHECK((int64_t)128 * K < (1LL << 31));
+  if (M > 64) {
+    launch_gemm_block_q(ptr<__hip_bfloat16>(y), cptr<__hip_bfloat16>(x), cptr<unsigned char>(wq),
+                        wscale.data_ptr<float>(), (int)qbits, M, N, K, current_stream());
+    return;
+  }
+  const int parts = gemm_stream_parts((int)qbits, M, N, K, false);
   torch::Tensor part;
   launch_gemm_stream_q(ptr<__hip_bfloat16>(y), stream_parts(part, x, parts, (int64_t)M * N),
                        cptr<__hip_bfloat16>(x), cptr<unsigned char>(wq),
                        wscale.data_ptr<float>(), (int)qbits, M, N, K, parts, current_stream());
+}
+
+// out [N, K] bf16 = the weights that (wq, wscale) round
+void widen_weight(torch::Tensor out, torch::Tensor wq, torch::Tensor wscale, int64_t qbits) {
+  const int64_t N = out.size(0), K = out.size(1);
+  check_rounded(wq, wscale, qbits, N, K);
+  TORCH_CHECK(out.is_cuda() && out.is_contiguous() &&
+              out.scalar_type() == at::ScalarType::BFloat16);
+  launch_widen_weight(ptr<__hip_bfloat16>(out), cptr<unsigned char>(wq),
+                      wscale.data_ptr<float>(), (int)qbits, N * K, (int)K, current_stream());
 }
 
 void gemm_skinny_gated(torch::Tensor y, torch::Tensor x, torch::Tensor w13) {
@@ -357,7 +383,7 @@ void gemm_skinny_gated(torch::Tensor y, torch::Tensor x, torch::Tensor w13) {
   TORCH_CHECK(y.size(0) == M && y.size(1) == I);
   torch::Tensor part;
   if (M <= 64) {
-    const int parts = gemm_stream_parts(M, I, K, true);
+    const int parts = gemm_stream_parts(16, M, I, K, true);
     launch_gemm_stream_gated(ptr<__hip_bfloat16>(y),
                              stream_parts(part, x, parts, (int64_t)2 * M * I),
                              cptr<__hip_bfloat16>(x), cptr<__hip_bfloat16>(w13), M, I, K, parts,
@@ -554,8 +580,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "in-place one-shot all-reduce over peer-mapped xGMI buffers");
   m.def("gemm_tile", &gemm_tile,
         "128x128-tile glds-staged bf16 GEMM for decode batches (CDNA4)");
-  m.def("gemm_skinny_q", &gemm_skinny_q,
-        "weight-only-quantized (int8 / int4-g128) skinny decode GEMM");
+  m.def("gemm_q", &gemm_q, "product with int8 / 4-bit weights");
+  m.def("widen_weight", &widen_weight, "int8 / 4-bit weights to bf16");
   m.def("gemm_skinny", &gemm_skinny,
         "skinny decode GEMM y = x @ w^T, M <= 64 (CDNA4 MFMA)");
   m.def("gemm_skinny_gated", &gemm_skinny_gated,

@@ -1,0 +1,299 @@
+// Products of more than 64 rows with rounded weights: y[m, n] = sum_k x[m, k] W[n, k],
+// W in int8 (a scale per row) or in 4 bits (offset 8, a scale per row and 128 inputs).
+//
+// The weights used to be widened by tensor ops (for 4 bits: masks, shifts, casts, a stack,
+// two products, all in f32 in memory) ahead of a library product: 1.0 ms of 1.3 ms a
+// llama-3-8b layer at 301 rows.  Now
+//  - up to some hundreds of rows the product widens a tile's weights itself, between LDS
+//    and the matrix unit: W crosses memory once, at its own size;
+//  - above, one kernel writes the widened matrix (bf16(q scale), bound by its bytes) for
+//    the library's product, which is then the larger part and the faster one.
+//
+// In the product weights are whole numbers and scales are applied to 32-bit sums, as in
+// gemm_stream.hip: int8 by conversion to f32 of which the upper half is all; 4 bits as the
+// bf16 pattern of 8 + n/2, with -12 times the sum of x added by a constant operand and the
+// scale doubled.  A lane's 16 (8) bytes hold two matrix steps' inputs, x is read to match.
+// x and W reach LDS without registers; x chunks are swizzled as in block_gemm.h, W rows of
+// 64 (32) bytes by r / 4 (r / 8).
+//
+// Measured: four llama-3-8b layers around attention, 301 rows, int8: 5101 -> 1061 us.
+// Widening 28672 x 4096: 61 us (5.8 TB/s).
+
+#include "block_gemm.h"
+
+namespace {
+
+using block_gemm::bf16x8_t;
+using block_gemm::f32x4_t;
+
+typedef __attribute__((ext_vector_type(4))) unsigned int u32x4_t;
+typedef __attribute__((ext_vector_type(2))) unsigned int u32x2_t;
+
+// DEPTH: inputs of a tile (4 bits: 128, a group of one scale).
+template <int QB, int DEPTH, int BM, int BN, int WM, int WN, int STAGES>
+__global__ __launch_bounds__(WM * WN * 64, 2) void gemm_block_q_kernel(
+    __hip_bfloat16* __restrict__ y,         // [M, N]
+    const __hip_bfloat16* __restrict__ x,   // [M, K]
+    const unsigned char* __restrict__ w,    // int8 [N, K] | packed [N, K / 2]
+    const float* __restrict__ scale,        // [N] | [N, K / 128]
+    const int M, const int N, const int K) {
+  static_assert(QB == 8 || DEPTH == 128, "a tile of 4-bit weights is a group");
+  constexpr int WAVES = WM * WN;
+  constexpr int TM = BM / WM / 16, TN = BN / WN / 16;
+  constexpr int AL = DEPTH / 8;                  // lanes (16 bytes) of an x row in a tile
+  constexpr int WB = DEPTH * QB / 8;             // bytes of a W row in a tile
+  constexpr int WL = WB / 16;                    // lanes a W row
+  constexpr int CHUNKS = WL / 4;                 // 16-byte chunks of a lane's W row
+  constexpr int STEPS = 16 * 8 / QB / 8;         // matrix steps of a chunk
+  constexpr int A_PASS = BM * AL / 64 / WAVES;
+  constexpr int B_LOADS = BN * WL / 64;          // 1 KB each, shared out over the waves
+  constexpr int B_PASS = (B_LOADS + WAVES - 1) / WAVES;
+  constexpr int S_PASS = QB == 4 ? 1 : 0;        // scales: 64 columns a load
+  constexpr int A_BYTES = BM * DEPTH * 2, B_BYTES = BN * WB;
+  constexpr int STAGE = A_BYTES + B_BYTES + (QB == 4 ? BN * 4 : 0);
+  static_assert(BM * AL % (64 * WAVES) == 0 && BN * WL % 64 == 0 && BN % 64 == 0, "whole loads");
+  __shared__ __align__(16) char lds[STAGES * STAGE];
+
+  // neighbours in a run of blocks that one XCD gets share their columns of W
+  const int m_tiles = (M + BM - 1) / BM, blocks = m_tiles * (N / BN);
+  const int per_xcd = (blocks + 7) / 8, slot = blockIdx.x / 8;
+  const int id = (blockIdx.x % 8) * per_xcd + slot;
+  if (slot >= per_xcd || id >= blocks) return;
+  const int m0 = id % m_tiles * BM, n0 = id / m_tiles * BN;
+
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int col = lane & 15, quad = lane >> 4;
+  const int wm = wave / WN, wn = wave % WN;
+  // a chunk's place in its row is turned by the row: rows of 256, 128, 64 bytes
+  auto swz = [](int lanes, int r) { return lanes == 16 ? r % 16 : lanes == 8 ? r / 2 % 8 : r / 4 % 4; };
+
+  unsigned long a_off[A_PASS];
+  unsigned b_off[B_PASS], s_off = 0;
+#pragma unroll
+  for (int p = 0; p < A_PASS; ++p) {
+    const int r = (p * WAVES + wave) * (64 / AL) + lane / AL;
+    a_off[p] = (unsigned long)min(m0 + r, M - 1) * K * 2 + ((lane % AL) ^ swz(AL, r)) * 16;
+  }
+  // (where there are fewer loads than waves some are made twice: all waves wait alike)
+#pragma unroll
+  for (int p = 0; p < B_PASS; ++p) {
+    const int r = (p * WAVES + wave) % B_LOADS * (64 / WL) + lane / WL;
+    b_off[p] = r * (K * QB / 8) + ((lane % WL) ^ swz(WL, r)) * 16;
+  }
+  if constexpr (QB == 4) s_off = (unsigned)(wave % (BN / 64) * 64 + lane) * (K / 128);
+  const char* xa = reinterpret_cast<const char*>(x);
+  const char* wb = reinterpret_cast<const char*>(w) + (long)n0 * (K * QB / 8);
+  const float* sb = QB == 4 ? scale + (long)n0 * (K / 128) : scale;
+  auto stage = [&](int buf, int tile) {
+    char* to = lds + buf * STAGE;
+#pragma unroll
+    for (int p = 0; p < A_PASS; ++p)
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) unsigned*)(xa + (long)tile * (DEPTH * 2) +
+                                                              a_off[p]),
+          (__attribute__((address_space(3))) unsigned*)(to + (p * WAVES + wave) * 1024), 16, 0, 0);
+#pragma unroll
+    for (int p = 0; p < B_PASS; ++p)
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) unsigned*)(wb + (long)tile * WB + b_off[p]),
+          (__attribute__((address_space(3))) unsigned*)(to + A_BYTES +
+                                                        (p * WAVES + wave) % B_LOADS * 1024),
+          16, 0, 0);
+    if constexpr (QB == 4)
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) unsigned*)(sb + s_off + tile),
+          (__attribute__((address_space(3))) unsigned*)(to + A_BYTES + B_BYTES +
+                                                        wave % (BN / 64) * 256),
+          4, 0, 0);
+  };
+
+  f32x4_t acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4_t{};
+  bf16x8_t off;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) off[j] = (short)0xc140;   // -12
+
+  const int tiles = K / DEPTH;
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < tiles) stage(s, s);
+  int buf = 0;
+  for (int t = 0; t < tiles; ++t) {
+    if (STAGES > 2 && t + 1 < tiles)
+      block_gemm::wait_loads<(STAGES - 2) * (A_PASS + B_PASS + S_PASS)>();
+    else
+      block_gemm::wait_loads<0>();
+    block_gemm::meet();
+    if (t + STAGES - 1 < tiles) {
+      int ahead = buf + STAGES - 1;
+      if (ahead >= STAGES) ahead -= STAGES;
+      stage(ahead, t + STAGES - 1);
+    }
+    const char* al = lds + buf * STAGE;
+    const char* bl = al + A_BYTES;
+    f32x4_t part[QB == 4 ? TM : 1][QB == 4 ? TN : 1], base[QB == 4 ? TM : 1];
+    if constexpr (QB == 4) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        base[i] = f32x4_t{};
+#pragma unroll
+        for (int j = 0; j < TN; ++j) part[i][j] = f32x4_t{};
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < CHUNKS; ++h) {
+      u32x4_t c[TN];
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int r = (wn * TN + j) * 16 + col;
+        c[j] = *reinterpret_cast<const u32x4_t*>(bl + r * WB + ((h * 4 + quad) ^ swz(WL, r)) * 16);
+      }
+#pragma unroll
+      for (int st = 0; st < STEPS; ++st) {
+        bf16x8_t xf[TM];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const int r = (wm * TM + i) * 16 + col;
+          xf[i] = *reinterpret_cast<const bf16x8_t*>(
+              al + r * (DEPTH * 2) + (((h * 4 + quad) * STEPS + st) ^ swz(AL, r)) * 16);
+          if constexpr (QB == 4)
+            base[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[i], off, base[i], 0, 0, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          union { unsigned u[4]; bf16x8_t v; } wf;
+          if constexpr (QB == 8) {
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+              const unsigned two = c[j][2 * st + d / 2] >> (d % 2 * 16);
+              const float a = (float)(signed char)(two & 0xff);
+              const float b = (float)(signed char)((two >> 8) & 0xff);
+              wf.u[d] = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302);
+            }
+          } else {
+            // even and odd weights to bits 3..6 of every byte, then to pairs
+            const unsigned even = (c[j][st] << 3) & 0x78787878u;
+            const unsigned odd = (c[j][st] >> 1) & 0x78787878u;
+            wf.u[0] = __builtin_amdgcn_perm(odd, even, 0x0c040c00) | 0x41004100u;
+            wf.u[1] = __builtin_amdgcn_perm(odd, even, 0x0c050c01) | 0x41004100u;
+            wf.u[2] = __builtin_amdgcn_perm(odd, even, 0x0c060c02) | 0x41004100u;
+            wf.u[3] = __builtin_amdgcn_perm(odd, even, 0x0c070c03) | 0x41004100u;
+          }
+#pragma unroll
+          for (int i = 0; i < TM; ++i) {
+            f32x4_t& to = QB == 4 ? part[QB == 4 ? i : 0][QB == 4 ? j : 0] : acc[i][j];
+            to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[i], wf.v, to, 0, 0, 0);
+          }
+        }
+      }
+    }
+    if constexpr (QB == 4) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const float s =
+            2.f * reinterpret_cast<const float*>(bl + B_BYTES)[(wn * TN + j) * 16 + col];
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            acc[i][j][r] = __builtin_fmaf(s, part[i][j][r] + base[i][r], acc[i][j][r]);
+      }
+    }
+    if (++buf == STAGES) buf = 0;
+  }
+
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int n = n0 + (wn * TN + j) * 16 + col;
+    const float s = QB == 8 ? scale[n] : 1.f;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int m = m0 + (wm * TM + i) * 16 + quad * 4 + r;
+        if (m < M) y[(long)m * N + n] = __float2bfloat16(QB == 8 ? acc[i][j][r] * s : acc[i][j][r]);
+      }
+  }
+}
+
+// out[n, k] = bf16(q scale), 16 weights a thread; bound by the bytes in and out.
+template <int QB>
+__global__ __launch_bounds__(256) void widen_weight_kernel(
+    __hip_bfloat16* __restrict__ out, const unsigned char* __restrict__ w,
+    const float* __restrict__ scale, const long total, const int K) {
+  for (long i = ((long)blockIdx.x * 256 + threadIdx.x) * 16; i < total;
+       i += (long)gridDim.x * 4096) {
+    const float s = QB == 8 ? scale[i / K] : scale[i / 128];
+    Vec16<__hip_bfloat16> o[2];
+    if constexpr (QB == 8) {
+      const u32x4_t q = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(w + i));
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        o[j / 8].data[j % 8] =
+            __float2bfloat16((float)(signed char)((q[j / 4] >> (j % 4 * 8)) & 0xff) * s);
+    } else {
+      const u32x2_t q = __builtin_nontemporal_load(reinterpret_cast<const u32x2_t*>(w + i / 2));
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        o[j / 8].data[j % 8] =
+            __float2bfloat16(((float)((q[j / 8] >> (j % 8 * 4)) & 15) - 8.f) * s);
+    }
+    store16(out + i, o[0]);
+    store16(out + i + 8, o[1]);
+  }
+}
+
+// Tiles by how many blocks there are to fill 256 CUs with (us of what is chosen and the
+// next best; columns x inputs 6144 x 4096, 4096 x 4096, 28672 x 4096, 4096 x 14336):
+//   int8, 100 rows: 32x64 20.6 (64x64 22.4), 32x64 16.2 (21.4), 64x128 48.3, 32x64 49.0 (65.1)
+//         301 rows: 64x64 29.4 (64x128 31.9), 64x64 26.8 (29.9), 64x128 99, 64x64 81.5 (88.9)
+//         700 rows: 64x128 57 (58.6), 64x64 36 (42.2), 64x128 200, 64x64 118 (132)
+//        1500 rows: 64x128 102, 64, 128x128 375 (64x128 440), 64x128 212
+//   4 bits, 100 rows: 32x64 24.5 (64x64 23.9), 18.4 (23.4), 64x128 53, 32x64 56.4 (74.7)
+//         301 rows: 64x128 34.1, 32x64 31.2 (33.2), 64x128 123, 32x64 101 (107)
+//         700 rows: 64x128 77, 48.5, 247, 167
+template <int QB>
+void launch_block(__hip_bfloat16* y, const __hip_bfloat16* x, const unsigned char* w,
+                  const float* scale, int M, int N, int K, hipStream_t stream) {
+#define GO(DEPTH, BM, BN, WM, WN, ST)                                                        \
+  hipLaunchKernelGGL((gemm_block_q_kernel<QB, DEPTH, BM, BN, WM, WN, ST>),                   \
+                     dim3(((M + BM - 1) / BM * (N / BN) + 7) / 8 * 8), dim3(WM * WN * 64), 0, \
+                     stream, y, x, w, scale, M, N, K)
+  const long wide = (M + 63L) / 64 * (N / 128);   // blocks of 64x128
+  if constexpr (QB == 4) {
+    if (wide >= 230) GO(128, 64, 128, 1, 4, 3);
+    else GO(128, 32, 64, 1, 4, 3);
+  } else {
+    if (wide >= 4096) GO(64, 128, 128, 2, 2, 2);
+    else if (wide >= 448) GO(64, 64, 128, 1, 4, 3);
+    else if (wide >= 150) GO(128, 64, 64, 1, 4, 2);
+    else GO(128, 32, 64, 1, 4, 3);
+  }
+#undef GO
+}
+
+}  // namespace
+
+// M >= 1, N % 128 == 0, K % 128 == 0
+void launch_gemm_block_q(__hip_bfloat16* y, const __hip_bfloat16* x, const unsigned char* w,
+                         const float* scale, int qbits, int M, int N, int K,
+                         hipStream_t stream) {
+  if (qbits == 8)
+    launch_block<8>(y, x, w, scale, M, N, K, stream);
+  else
+    launch_block<4>(y, x, w, scale, M, N, K, stream);
+}
+
+// total = N * K, K % 128 == 0
+void launch_widen_weight(__hip_bfloat16* out, const unsigned char* w, const float* scale,
+                         int qbits, long total, int K, hipStream_t stream) {
+  const long blocks = (total / 16 + 255) / 256;
+  const dim3 grid(blocks < 16384 ? blocks : 16384);
+  if (qbits == 8)
+    hipLaunchKernelGGL(widen_weight_kernel<8>, grid, dim3(256), 0, stream, out, w, scale, total, K);
+  else
+    hipLaunchKernelGGL(widen_weight_kernel<4>, grid, dim3(256), 0, stream, out, w, scale, total, K);
+}

@@ -54,51 +54,63 @@ __global__ __launch_bounds__(256) void gemm_stream_merge_kernel(
   *reinterpret_cast<uint2*>(y + at) = o.u;
 }
 
-// How a product is cut.  The lines are where they measured fastest (us, bf16 unless
-// said; M = 1..16 | 23 | 61):
+// How a product is cut (waves along N x waves along K, workgroups along K).  The lines
+// are where they measured fastest (us; bf16 unless said; N x K):
 //   up to 16 rows of x, x is a small part of what is read and waves work alone:
-//     4096 x 4096: WK 8 8.1, WK 4 9.5; 14336 x 4096 gated: WK 4 39.8, WK 8 42.0.
-//   17..32: 14336 x 4096 gated: 2 x 2 43.4, 1 x 4 45.5; 4096 x 4096: 1 x 8 11.2, 4 x 2
-//     over four workgroups and a merge 12.1; 4096 x 14336: the same two 27.4, 25.4.
-//   33..64: every wave's own copy of x would cost more than W, 4 x 2 waves share it:
-//     4096 x 14336: over four workgroups 34.9, 1 x 8 43.5; 14336 x 4096 gated: 2 x 2
-//     48.4, 4 x 2 49.7; 28672 x 4096 int8: 4 x 2 42.8; 2048 x 2048: 1 x 8 9.4, 4 x 2 10.3.
-enum class Cut { kWave8, kWave4, kShare22, kShare42 };
+//     4096 x 4096: 1x8 8.1, 1x4 9.5; 14336 x 4096 gated: 1x4 39.8, 1x8 42.0.
+//   17..32, plain: 4096 x 4096: 1x8 11.2, 4x2 over 4 12.1; 4096 x 14336: 27.4, 25.4;
+//     8192 x 8192: 4x2 over 2 30.4, 2x4 31.4; 28672 x 4096 int8: 4x2 27.3, 4x1 30.9.
+//     gated: 14336 x 4096: 2x2 43.4, 1x4 45.5, 4x1 47.5; 28672 x 8192: 4x1 158, 2x2 171.
+//   33..64, every wave's own copy of x would cost more than W: 4096 x 14336: 4x2 over 4
+//     34.9, 1x8 43.5; 2048 x 2048: 1x8 9.4, 4x2 10.3; 28672 x 4096: int8 4x2 42, 8x1 over
+//     2 45, 4 bits 8x1 over 2 41, 4x2 47 (more of x is turned per weight);
+//     8192 x 28672: 4x2 over 4 93, over 2 109.  gated: 14336 x 4096: 2x2 48.4, 4x2 49.7;
+//     28672 x 8192: 4x1 158, 2x2 189; 8192 x 2048: 2x4 18.0, 2x2 21.5.
+enum class Cut { kWave8, kWave4, kShare22, kShare24, kShare41, kShare42, kShare81 };
 
-Cut cut_of(int M, int N, int K, bool gated) {
+Cut cut_of(int qbits, int M, int N, int K, bool gated) {
   if (M <= 16) return N / 16 < 512 ? Cut::kWave8 : Cut::kWave4;
-  if (M <= 32) {
-    if (N >= 8192) return Cut::kShare22;
-    if (K >= 8192) return Cut::kShare42;
-    return N / 16 < 320 ? Cut::kWave8 : Cut::kWave4;
+  if (gated) {
+    if (K >= 8192) return Cut::kShare41;
+    return K < 4096 && M > 32 ? Cut::kShare24 : Cut::kShare22;
   }
-  if (K < 4096 && N < 8192) return Cut::kWave8;
-  return gated ? Cut::kShare22 : Cut::kShare42;
+  if ((long)N * K <= 1L << (M <= 32 ? 24 : 23)) return Cut::kWave8;
+  if (qbits == 4 && M > 32 && N >= 16384 && K >= 4096) return Cut::kShare81;
+  return Cut::kShare42;
+}
+
+template <int QB, int MT, bool GATED, int WN, int WK>
+void launch_cut(__hip_bfloat16* y, float* part, const __hip_bfloat16* x, const void* w,
+                const float* s, int M, int N, int K, int parts, hipStream_t stream) {
+  constexpr int kCols = 16 * WN;   // of a workgroup; N is a multiple of 128
+  static_assert(128 % kCols == 0, "whole workgroups");
+  hipLaunchKernelGGL(
+      (gemm_stream_kernel<QB, MT, 1, WN, WK, GATED ? moe::kSilu : moe::kPlain>),
+      dim3(N / kCols, parts), dim3(64 * WN * WK), 0, stream, y, part, x, w, s, M, N, K);
 }
 
 template <int QB, int MT, bool GATED>
 void launch_mt(__hip_bfloat16* y, float* part, const __hip_bfloat16* x, const void* w,
                const float* s, int M, int N, int K, int parts, hipStream_t stream) {
-#define GO(WN, WK)                                                                            \
-  hipLaunchKernelGGL((gemm_stream_kernel<QB, MT, 1, WN, WK, GATED ? moe::kSilu : moe::kPlain>),                          \
-                     dim3(N / (16 * WN), parts), dim3(64 * WN * WK), 0, stream, y, part, x, w, \
-                     s, M, N, K)
-  const Cut cut = cut_of(M, N, K, GATED);
+  const Cut cut = cut_of(QB, M, N, K, GATED);
+  auto run = [&](auto launch) { launch(y, part, x, w, s, M, N, K, parts, stream); };
   if constexpr (MT == 1) {
-    if (cut == Cut::kWave8) GO(1, 8);
-    else GO(1, 4);
+    if (cut == Cut::kWave8) run(launch_cut<QB, MT, GATED, 1, 8>);
+    else run(launch_cut<QB, MT, GATED, 1, 4>);
+  } else if constexpr (GATED) {
+    if (cut == Cut::kShare41) run(launch_cut<QB, MT, GATED, 4, 1>);
+    else if (cut == Cut::kShare24) run(launch_cut<QB, MT, GATED, 2, 4>);
+    else run(launch_cut<QB, MT, GATED, 2, 2>);
+  } else if (cut == Cut::kWave8) {
+    run(launch_cut<QB, MT, GATED, 1, 8>);
   } else {
-    switch (cut) {
-      case Cut::kWave8: GO(1, 8); break;
-      case Cut::kWave4: GO(1, 4); break;
-      case Cut::kShare22: GO(2, 2); break;
-      case Cut::kShare42:
-        // the gated form takes this cut for few columns only
-        GO(4, 2);
-        break;
+    if constexpr (QB == 4) {
+      if (cut == Cut::kShare81) run(launch_cut<QB, MT, GATED, 8, 1>);
+      else run(launch_cut<QB, MT, GATED, 4, 2>);
+    } else {
+      run(launch_cut<QB, MT, GATED, 4, 2>);
     }
   }
-#undef GO
   if (parts > 1) {
     const long plane = (long)M * N;
     hipLaunchKernelGGL((gemm_stream_merge_kernel<GATED>), dim3((plane / 4 + 255) / 256),
@@ -117,17 +129,20 @@ void launch_q(__hip_bfloat16* y, float* part, const __hip_bfloat16* x, const voi
 }  // namespace
 
 // Workgroups that K is cut over besides the waves (each leaves a part of the result):
-// as many as make one a CU.  A function of shapes.
-int gemm_stream_parts(int M, int N, int K, bool gated) {
-  if (cut_of(M, N, K, gated) != Cut::kShare42) return 1;
-  const int wgs = N / 64;
-  int parts = (256 + wgs - 1) / wgs;
+// as many as make one a CU, two where K is long and the columns are many.  A function of
+// shapes.
+int gemm_stream_parts(int qbits, int M, int N, int K, bool gated) {
+  const Cut cut = cut_of(qbits, M, N, K, gated);
+  if (gated || (cut != Cut::kShare42 && cut != Cut::kShare81)) return 1;
+  const int wgs = N / (cut == Cut::kShare81 ? 128 : 64);
+  const int want = M > 32 && N >= 8192 && K >= 8192 ? 512 : 256;
+  int parts = (want + wgs - 1) / wgs;
   if (parts > 8) parts = 8;
   const int most = K / 1024 > 0 ? K / 1024 : 1;   // four tiles of 128 a wave at least
   return parts < most ? parts : most;
 }
 
-// M <= 64, N % 64 == 0, K % 64 == 0 (rounded weights: K % 128 == 0)
+// M <= 64, N % 128 == 0, K % 64 == 0 (rounded weights: K % 128 == 0)
 void launch_gemm_stream(__hip_bfloat16* y, float* part, const __hip_bfloat16* x,
                         const __hip_bfloat16* w, int M, int N, int K, int parts,
                         hipStream_t stream) {

@@ -12,7 +12,7 @@ ROWS = [1, 15, 16, 17, 23, 32, 33, 61, 64]
 # N, K: one workgroup's columns, K of a single tile and of half a last one, as many
 # columns as the other cuts take
 SHAPES = [(128, 64), (128, 128), (256, 192), (384, 1088), (5120, 256), (8192, 320), (256, 8192),
-          (1152, 4160)]
+          (1152, 4160), (4096, 4224), (16384, 4096), (9216, 8192)]
 
 
 def _need():
@@ -79,3 +79,37 @@ def test_rounded(qbits, m, n, k):
     _check(got, x.double() @ exact.t(), 5 * (x.double().abs() @ exact.abs().t()
                                              + 4 * x.double().abs().sum(1, keepdim=True)
                                              * exact.abs().amax(1) / 4))
+
+
+@pytest.mark.parametrize("qbits", [8, 4])
+@pytest.mark.parametrize("m", [65, 127, 128, 129, 301, 460, 900])
+# blocks for every choice of tile: narrow, 64 wide, 128 wide, and many
+@pytest.mark.parametrize(("n", "k"), [(128, 128), (512, 384), (4096, 256), (8192, 640),
+                                      (36864, 256)])
+def test_rounded_many_rows(qbits, m, n, k):
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    x, w = _x(m, k, 7), _x(n, k, 8)
+    wq, scale = ops.quantize_weight(w, qbits)
+    exact = ops.dequantize_weight(wq, scale, qbits, torch.float32).double()
+    got = ops.linear_quant(x, wq, scale, qbits)
+    terms = x.double().abs() @ exact.abs().t()
+    # above the line of the product's own widening the weights are rounded to bf16
+    wide = m > ops._quant_rows(qbits, n, k)
+    err = (got.double() - x.double() @ exact.t()).abs()
+    bound = 2 ** -8 * (x.double() @ exact.t()).abs() + (2 ** -9 if wide else 2 ** -17) * terms
+    assert (err <= bound).all(), (err - bound).max().item()
+
+
+@pytest.mark.parametrize("qbits", [8, 4])
+def test_widened_weights_are_the_rounded_ones(qbits):
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    w = _x(384, 640, 9)
+    wq, scale = ops.quantize_weight(w, qbits)
+    x = _x(2100, 640, 10)
+    got = ops.linear_quant(x, wq, scale, qbits)
+    want = torch.nn.functional.linear(x, ops.dequantize_weight(wq, scale, qbits))
+    assert torch.equal(got, want)

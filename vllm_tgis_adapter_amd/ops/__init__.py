@@ -273,28 +273,38 @@ def dequantize_weight(wq: torch.Tensor, scales: torch.Tensor, qbits: int,
     return (q.view(n, k // 128, 128) * scales.unsqueeze(2)).view(n, k).to(dtype)
 
 
+def _quant_rows(qbits: int, n: int, k: int) -> int:
+    """Most rows of a product that widens its weights itself.  Above, the second pass
+    over the widened matrix costs less than the library's faster product saves (us, own
+    | widened for the library): int8 28672 x 4096 448 rows 141 | 148, 600 rows 192 | 186,
+    2048 x 2048 1500 rows 23 | 28; 4 bits 28672 x 4096 301 rows 129 | 136, 448 rows
+    176 | 157, 4096 x 14336 80 rows 58 | 67, 150 rows 78 | 72."""
+    if n * k <= 1 << 23:
+        return 1500 if qbits == 8 else 1000
+    if qbits == 8:
+        return 560
+    return 320 if k < 8192 else 128
+
+
 def linear_quant(x: torch.Tensor, wq: torch.Tensor, scales: torch.Tensor,
                  qbits: int, bias: torch.Tensor | None = None) -> torch.Tensor:
-    """W8A16/W4A16 linear: native dequant-GEMM for decode batches, dequant +
-    hipBLASLt above (prefill is compute-bound; the quant win is the weight
-    stream at small M)."""
+    """W8A16/W4A16 linear.  Up to ``_quant_rows`` rows the product widens the
+    weights on their way to the matrix unit; above, one launch writes them in bf16
+    for the library's product."""
     x2 = x.reshape(-1, x.shape[-1])
     m = x2.shape[0]
     n = wq.shape[0]
     k = x2.shape[1]
-    if (
-        bias is None
-        and _native(x)
-        and x.dtype == torch.bfloat16
-        and 1 <= m <= 64
-        and n % 128 == 0
-        and k % 128 == 0
-        and x2.is_contiguous()
-    ):
-        out = torch.empty((m, n), dtype=x.dtype, device=x.device)
-        _C.gemm_skinny_q(out, x2, wq, scales, qbits)
-        return out.view(*x.shape[:-1], n)
-    w = dequantize_weight(wq, scales, qbits, x.dtype)
+    if _native(x) and x.dtype == torch.bfloat16 and n % 128 == 0 and k % 128 == 0:
+        if (bias is None and 1 <= m <= _quant_rows(qbits, n, k) and x2.is_contiguous()
+                and wq.is_contiguous() and scales.is_contiguous()):
+            out = torch.empty((m, n), dtype=x.dtype, device=x.device)
+            _C.gemm_q(out, x2, wq, scales, qbits)
+            return out.view(*x.shape[:-1], n)
+        w = torch.empty((n, k), dtype=x.dtype, device=x.device)
+        _C.widen_weight(w, wq.contiguous(), scales.contiguous(), qbits)
+    else:
+        w = dequantize_weight(wq, scales, qbits, x.dtype)
     return torch.nn.functional.linear(x, w, bias)
 
 
