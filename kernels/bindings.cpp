@@ -77,6 +77,14 @@ void launch_gemm_block_q(__hip_bfloat16*, const __hip_bfloat16*, const unsigned 
                          const float*, int, int, int, int, hipStream_t);
 void launch_widen_weight(__hip_bfloat16*, const unsigned char*, const float*, int, long, int,
                          hipStream_t);
+struct LoraCols {
+  int end[3], shift[3];
+};
+int lora_shrink_cuts(int T, int K);
+void launch_lora_tiles(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hip_bfloat16*,
+                       const __hip_bfloat16*, const int*, const float*, const LoraCols&, int,
+                       int, int, int, int, int, int, int, hipStream_t);
+void launch_lora_slots(int*, const int*, const int*, int, int, hipStream_t);
 template <typename T>
 void launch_lora_shrink(float*, const T*, const T*, const int*, int, int, int,
                         hipStream_t);
@@ -433,6 +441,57 @@ void lora_bgmv(torch::Tensor out, torch::Tensor x, torch::Tensor a_stack,
   });
 }
 
+// bf16: out[t, start_p ...] += scale · B_p A_p x[t] for up to three projections of x, whose
+// adapters' weights are stacked side by side: a [L, P R, K], b [L, V, R], spans[p] = (start,
+// end) in out's columns, V = the sum of their widths.
+void lora_delta(torch::Tensor out, torch::Tensor x, torch::Tensor a, torch::Tensor b,
+                torch::Tensor slots, torch::Tensor scales,
+                const std::vector<std::pair<int64_t, int64_t>>& spans) {
+  const int T = x.size(0), K = x.size(1), L = a.size(0), PR = a.size(1), R = b.size(2);
+  const int V = b.size(1), out_w = out.size(1), P = spans.size();
+  for (const auto& t : {out, x, a, b})
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::ScalarType::BFloat16 && t.is_contiguous());
+  TORCH_CHECK(P >= 1 && P <= 3 && PR == P * R && (R == 8 || R == 16 || R == 32 || R == 64));
+  TORCH_CHECK(a.size(2) == K && K % 8 == 0 && b.size(0) == L && out.size(0) == T);
+  TORCH_CHECK(slots.is_cuda() && slots.scalar_type() == at::ScalarType::Int &&
+              slots.numel() == T);
+  TORCH_CHECK(scales.is_cuda() && scales.scalar_type() == at::ScalarType::Float &&
+              scales.numel() >= L);
+  slots = slots.contiguous();
+  scales = scales.contiguous();
+  LoraCols cols;
+  int64_t v = 0;
+  for (int p = 0; p < 3; ++p) {
+    const auto& span = spans[p < P ? p : P - 1];
+    if (p < P) {
+      TORCH_CHECK(0 <= span.first && span.first <= span.second && span.second <= out_w);
+      cols.shift[p] = (int)(span.first - v);
+      v += span.second - span.first;
+    } else {
+      cols.shift[p] = cols.shift[P - 1];
+    }
+    cols.end[p] = (int)v;
+  }
+  TORCH_CHECK(v == V);
+  if (T == 0 || V == 0 || L == 0) return;
+  const int cuts = lora_shrink_cuts(T, K);
+  auto tmp = at::empty({cuts, T, PR}, x.options().dtype(at::ScalarType::Float));
+  launch_lora_tiles(ptr<__hip_bfloat16>(out), tmp.data_ptr<float>(), cptr<__hip_bfloat16>(x),
+                    cptr<__hip_bfloat16>(a), cptr<__hip_bfloat16>(b), slots.data_ptr<int>(),
+                    scales.data_ptr<float>(), cols, T, L, R, PR, V, K, out_w, cuts,
+                    current_stream());
+}
+
+// slots[t] = the place of token_ids[t] among ids (64 at most), or -1
+void lora_slots(torch::Tensor slots, torch::Tensor token_ids, const std::vector<int>& ids) {
+  for (const auto& t : {slots, token_ids})
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::ScalarType::Int && t.is_contiguous());
+  TORCH_CHECK(slots.numel() == token_ids.numel() && ids.size() <= 64);
+  if (slots.numel() == 0) return;
+  launch_lora_slots(slots.data_ptr<int>(), token_ids.data_ptr<int>(), ids.data(),
+                    (int)ids.size(), (int)slots.numel(), current_stream());
+}
+
 void moe_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w,
               torch::Tensor seg_off, int64_t mode, c10::optional<torch::Tensor> rows) {
   // mode 0: plain, 1: silu(first half) * second half, 2: squared relu
@@ -598,6 +657,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "fused log-softmax + top-K + sampled-token rank (one HBM pass)");
   m.def("sample_argmax", &sample_argmax,
         "fused temperature/gumbel-race sampling + greedy argmax (CDNA4)");
+  m.def("lora_delta", &lora_delta,
+        "bf16 multi-LoRA of up to three projections of one input");
+  m.def("lora_slots", &lora_slots, "adapter slot of every token");
   m.def("lora_bgmv", &lora_bgmv,
         "batched multi-LoRA shrink+expand for mixed-adapter batches (CDNA4)");
 }

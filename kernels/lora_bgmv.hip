@@ -1,19 +1,30 @@
-// Batched multi-LoRA shrink/expand kernels.
+// Batched multi-LoRA products.
 //
-// Mixed-adapter batches carry a per-token adapter slot (-1 = no adapter);
-// weights for the active adapters are stacked host-side into
-//   A_stack [L, R, K]   (shrink:  tmp[t] = A[slot(t)] · x[t])
-//   B_stack [L, N, R]   (expand:  out[t, off:off+N] += scale_s · B[slot(t)] · tmp[t])
-// with R padded to the max rank (padded rows/cols are zero).
+// Mixed-adapter batches carry a per-token adapter slot (-1 = no adapter); weights of the
+// active adapters are stacked host-side, for up to three projections of one input side
+// by side (q, k, v; gate, up):
+//   A_stack [L, P R, K]   (shrink:  tmp[t] = A[slot(t)] · x[t])
+//   B_stack [L, V, R]     (expand:  out[t, col(v)] += scale_s · B[slot(t), v] · tmp[t, p(v)])
+// with R padded to the largest rank (padded rows / columns are zero) and V the columns of
+// the projections one after the other.
 //
-// BGMV geometry — one token per workgroup:
+// bf16, shrink: 16 tokens and one adapter a workgroup (it ends at once where none of the
+// tokens has it), K cut over workgroups and waves, both operands straight from L2 into
+// v_mfma_f32_16x16x32_bf16.  The former kernel took a token a workgroup and a rank at a
+// time, each with its own wave reduction.  expand: one column a thread, the tokens of a
+// workgroup in turn, a row of B kept while the adapter stays the same, f32 sums in f32.
+// Both are bound by launch and load latency at decode sizes; at prompt sizes expand by the
+// read and write of out.
+//
+// Layers of 4096 wide rows, 61 tokens of 4 adapters of rank 16: 7 + 7 launches of 25 and
+// 5 us were 4 + 4 of 4.7 and 6.5.  2048 tokens: shrink 23 us, expand into 4096 columns 14
+// and into 28672 102, where reading and writing out takes 51.
+//
+// f32 and f16: one token per workgroup in both,
 //   shrink: 4 waves split K; each (wave, r) pair accumulates a partial dot,
 //           folded across lanes by shfl and across waves in LDS.  tmp is f32.
 //   expand: R <= 64 fits a lane-resident tmp row; each thread owns one
 //           output column and walks r with the B row loads coalesced.
-// Decode batches are tiny (T <= a few hundred) and A/B stay L2-resident, so
-// per-token re-reads are cheap; grouping tokens by adapter (true SGMV) only
-// pays at prefill sizes, where the torch grouped path still applies.
 
 #include "common.h"
 
@@ -119,6 +130,218 @@ void launch_lora_expand(T* out, const float* tmp, const T* b_stack,
   hipLaunchKernelGGL(lora_expand_kernel<T>, dim3(Tn, (N + 255) / 256),
                      dim3(256), 0, stream, out, tmp, b_stack, slots, scales, R,
                      N, out_w, off);
+}
+
+// ---------------------------------------------------------------------------
+// bf16
+// ---------------------------------------------------------------------------
+
+typedef __attribute__((ext_vector_type(8))) short bf16x8_t;
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+
+// virtual column v of projection p (v < end[p]) is column v + shift[p] of out
+struct LoraCols {
+  int end[3], shift[3];
+};
+
+namespace {
+
+constexpr int kShrinkWaves = 4;
+
+// grid (token tiles of 16, adapters, cuts of K).  tmp [cuts, T, PR]; tokens without an
+// adapter are left unwritten.
+template <int TILES>   // 16-wide tiles of PR
+__global__ __launch_bounds__(64 * kShrinkWaves) void lora_shrink_tile_kernel(
+    float* __restrict__ tmp, const __hip_bfloat16* __restrict__ x,
+    const __hip_bfloat16* __restrict__ a_stack, const int* __restrict__ slots, const int T,
+    const int PR, const int K) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int col = lane & 15, quad = lane >> 4;
+  const int t0 = blockIdx.x * 16, slot = blockIdx.y;
+  const int own = t0 + col < T ? slots[t0 + col] : -1;
+  if (__ballot(own == slot) == 0) return;
+
+  const __hip_bfloat16* xr = x + (long)min(t0 + col, T - 1) * K + quad * 8;
+  const __hip_bfloat16* ar[TILES];
+#pragma unroll
+  for (int j = 0; j < TILES; ++j)
+    ar[j] = a_stack + ((long)slot * PR + min(j * 16 + col, PR - 1)) * K + quad * 8;
+  f32x4_t acc[TILES];
+#pragma unroll
+  for (int j = 0; j < TILES; ++j) acc[j] = f32x4_t{};
+
+  const int steps = (K + 31) / 32, stride = gridDim.z * kShrinkWaves;
+  constexpr int AHEAD = TILES <= 4 ? 4 : 2;
+  for (int s0 = blockIdx.z * kShrinkWaves + wave; s0 < steps; s0 += AHEAD * stride) {
+    bf16x8_t xf[AHEAD], af[AHEAD][TILES];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      const int k = (s0 + u * stride) * 32;
+      const bool in = k + quad * 8 < K;   // K % 8 == 0: a lane's eight inputs are in or out
+      xf[u] = in ? *reinterpret_cast<const bf16x8_t*>(xr + k) : bf16x8_t{};
+#pragma unroll
+      for (int j = 0; j < TILES; ++j)
+        af[u][j] = in ? *reinterpret_cast<const bf16x8_t*>(ar[j] + k) : bf16x8_t{};
+    }
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+#pragma unroll
+      for (int j = 0; j < TILES; ++j)
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[u], af[u][j], acc[j], 0, 0, 0);
+  }
+
+  __shared__ f32x4_t all[kShrinkWaves][TILES][64];
+#pragma unroll
+  for (int j = 0; j < TILES; ++j) all[wave][j][lane] = acc[j];
+  __syncthreads();
+  for (int j = wave; j < TILES; j += kShrinkWaves) {
+    f32x4_t v = all[0][j][lane];
+#pragma unroll
+    for (int w = 1; w < kShrinkWaves; ++w) v += all[w][j][lane];
+    const int r = j * 16 + col;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int m = quad * 4 + i;
+      if (__shfl(own, m, 64) == slot && r < PR)
+        tmp[((long)blockIdx.z * T + t0 + m) * PR + r] = v[i];
+    }
+  }
+}
+
+// grid (ceil(V / 256), ceil(T / TOKENS))
+template <int R, int TOKENS>
+__global__ __launch_bounds__(256) void lora_expand_tile_kernel(
+    __hip_bfloat16* __restrict__ out,            // [T, out_w]
+    const float* __restrict__ tmp,               // [cuts, T, PR]
+    const __hip_bfloat16* __restrict__ b_stack,  // [L, V, R]
+    const int* __restrict__ slots, const float* __restrict__ scales, const LoraCols cols,
+    const int T, const int PR, const int V, const int out_w, const int cuts) {
+  __shared__ float sums[TOKENS][3 * R];
+  __shared__ int own[TOKENS];
+  const int t0 = blockIdx.y * TOKENS, v = blockIdx.x * 256 + threadIdx.x;
+  const int tokens = min(TOKENS, T - t0);
+  if (threadIdx.x < TOKENS)
+    own[threadIdx.x] = threadIdx.x < tokens ? slots[t0 + threadIdx.x] : -1;
+  __syncthreads();
+  for (int i = threadIdx.x; i < tokens * PR; i += 256) {
+    const int t = i / PR;
+    float s = 0.f;
+    if (own[t] >= 0)
+      for (int c = 0; c < cuts; ++c) s += tmp[((long)c * T + t0) * PR + i];
+    sums[t][i % PR] = s;
+  }
+  __syncthreads();
+  if (v >= V) return;
+  const int p = v < cols.end[0] ? 0 : v < cols.end[1] ? 1 : 2;
+  __hip_bfloat16* o = out + (long)t0 * out_w + v + cols.shift[p];
+  float was[TOKENS];
+#pragma unroll
+  for (int t = 0; t < TOKENS; ++t)
+    was[t] = t < tokens ? __bfloat162float(o[(long)t * out_w]) : 0.f;
+
+  Vec16<__hip_bfloat16> b[R / 8];
+  float scale = 0.f;
+  int cur = -1;
+#pragma unroll
+  for (int t = 0; t < TOKENS; ++t) {
+    const int slot = __builtin_amdgcn_readfirstlane(own[t]);
+    if (slot < 0) continue;
+    if (slot != cur) {
+      cur = slot;
+      scale = scales[slot];
+#pragma unroll
+      for (int j = 0; j < R / 8; ++j) b[j] = load16(b_stack + ((long)slot * V + v) * R + j * 8);
+    }
+    float acc = 0.f;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      acc = __builtin_fmaf(__bfloat162float(b[r / 8].data[r % 8]), sums[t][p * R + r], acc);
+    o[(long)t * out_w] = __float2bfloat16(was[t] + acc * scale);
+  }
+}
+
+template <int R>
+void launch_expand(__hip_bfloat16* out, const float* tmp, const __hip_bfloat16* b,
+                   const int* slots, const float* scales, const LoraCols& cols, int T, int PR,
+                   int V, int out_w, int cuts, hipStream_t stream) {
+  auto go = [&](auto kernel, int tokens) {
+    hipLaunchKernelGGL(kernel, dim3((V + 255) / 256, (T + tokens - 1) / tokens), dim3(256), 0,
+                       stream, out, tmp, b, slots, scales, cols, T, PR, V, out_w, cuts);
+  };
+  // Tokens a workgroup: few keep the chip full, many share the sums' way through LDS and
+  // the rows of B.  Rank 16, by 256-column tiles of all tokens (us at 2, 4, 8, 16 tokens):
+  // 976 3.7 4.4 5.6 8.2, 6832 7.0 5.9 6.6 9.7, 14336 12.1 9.6 8.7 11.5, 67200 67 50 41 44,
+  // 229376 157 123 106 102; ranks 8 and 64 cross at the same places.
+  const long tiles = (V + 255L) / 256 * T;
+  if (tiles <= 2560) go(lora_expand_tile_kernel<R, 2>, 2);
+  else if (tiles <= 8192) go(lora_expand_tile_kernel<R, 4>, 4);
+  else if (tiles <= 98304) go(lora_expand_tile_kernel<R, 8>, 8);
+  else go(lora_expand_tile_kernel<R, 16>, 16);
+}
+
+// slot of every token: the place of its adapter's id among `ids`, or -1
+struct LoraIds {
+  int n, id[64];
+};
+
+__global__ __launch_bounds__(256) void lora_slots_kernel(int* __restrict__ slots,
+                                                         const int* __restrict__ token_ids,
+                                                         const LoraIds ids, const int T) {
+  const int t = blockIdx.x * 256 + threadIdx.x;
+  if (t >= T) return;
+  const int id = token_ids[t];
+  int s = -1;
+  for (int i = 0; i < ids.n; ++i)
+    if (ids.id[i] == id) s = i;
+  slots[t] = s;
+}
+
+}  // namespace
+
+void launch_lora_slots(int* slots, const int* token_ids, const int* ids, int n, int T,
+                       hipStream_t stream) {
+  LoraIds by_value{};
+  by_value.n = n;
+  for (int i = 0; i < n && i < 64; ++i) by_value.id[i] = ids[i];
+  hipLaunchKernelGGL(lora_slots_kernel, dim3((T + 255) / 256), dim3(256), 0, stream, slots,
+                     token_ids, by_value, T);
+}
+
+// Workgroups K is cut over: enough for one a CU, four steps a wave at least (K 14336, rank
+// 16, 61 tokens: 29.5 us uncut, 6.1 in 8, 4.2 in 16; K 4096: 12.5, 3.7, 3.1, and as much
+// again in expand's sums; 2048 tokens: 23 us uncut and in 16).
+int lora_shrink_cuts(int T, int K) {
+  const int tiles = (T + 15) / 16;
+  int cuts = (256 + tiles - 1) / tiles;
+  if (cuts > 16) cuts = 16;
+  const int most = K >= 1024 ? K / (32 * kShrinkWaves * 4) : 1;
+  return cuts < most ? cuts : most;
+}
+
+// R in {8, 16, 32, 64}, PR = projections * R; tmp [cuts, T, PR]
+void launch_lora_tiles(__hip_bfloat16* out, float* tmp, const __hip_bfloat16* x,
+                       const __hip_bfloat16* a, const __hip_bfloat16* b, const int* slots,
+                       const float* scales, const LoraCols& cols, int T, int L, int R, int PR,
+                       int V, int K, int out_w, int cuts, hipStream_t stream) {
+  auto shrink = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((T + 15) / 16, L, cuts), dim3(64 * kShrinkWaves), 0, stream,
+                       tmp, x, a, slots, T, PR, K);
+  };
+  const int tiles = (PR + 15) / 16;
+  if (tiles <= 1) shrink(lora_shrink_tile_kernel<1>);
+  else if (tiles <= 2) shrink(lora_shrink_tile_kernel<2>);
+  else if (tiles <= 3) shrink(lora_shrink_tile_kernel<3>);
+  else if (tiles <= 4) shrink(lora_shrink_tile_kernel<4>);
+  else if (tiles <= 6) shrink(lora_shrink_tile_kernel<6>);
+  else if (tiles <= 8) shrink(lora_shrink_tile_kernel<8>);
+  else shrink(lora_shrink_tile_kernel<12>);
+#define EXPAND(RR) \
+  launch_expand<RR>(out, tmp, b, slots, scales, cols, T, PR, V, out_w, cuts, stream)
+  if (R == 8) EXPAND(8);
+  else if (R == 16) EXPAND(16);
+  else if (R == 32) EXPAND(32);
+  else EXPAND(64);
+#undef EXPAND
 }
 
 #define INSTANTIATE_LORA(T)                                                  \

@@ -5,9 +5,9 @@ onto the serving model and applies them per request in mixed batches.
 
 Application model: each step batch carries a per-token adapter id; for every
 active adapter the delta  x @ A^T @ B^T * (alpha/r)  is added onto the
-matching projection outputs.  Today this runs as batched torch GEMMs grouped
-by adapter (shrink+expand per adapter — fine for a handful of live adapters);
-the batched SGMV HIP kernel replaces the inner loop next.
+matching projection outputs: on a GPU by the batched kernels of
+kernels/lora_bgmv.hip over stacks of the active adapters, else grouped by
+adapter.
 
 TP sharding follows the base layer: column-parallel projections
 (q/k/v/gate/up) shard B on the output dim; row-parallel projections (o/down)
@@ -57,7 +57,7 @@ class LoRAContext:
 
 CTX = LoRAContext()
 
-# (slot_ids, layer, proj, N, dtype) -> (a_stack, b_stack, scales) for lora_bgmv
+# (slot_ids, layer, projections, dtype) -> (a_stack, b_stack, scales, spans)
 _STACK_CACHE: dict = {}
 
 
@@ -90,11 +90,9 @@ def set_context(token_lora_ids: Optional[torch.Tensor], adapters: dict[int, LoRA
     CTX.slot_ids = new_slot_ids
     CTX.token_slots = None
     if token_lora_ids is not None and adapters:
-        id2slot = {lid: s for s, lid in enumerate(CTX.slot_ids)}
-        slots = torch.full_like(token_lora_ids, -1)
-        for lid, s in id2slot.items():
-            slots[token_lora_ids == lid] = s
-        CTX.token_slots = slots.to(torch.int32)
+        from .. import ops
+
+        CTX.token_slots = ops.lora_slots(token_lora_ids, CTX.slot_ids)
 
 
 def clear_context() -> None:
@@ -104,35 +102,40 @@ def clear_context() -> None:
     CTX.slot_ids = ()
 
 
-def _get_stacks(layer_idx: int, proj: str, n_out: int, in_size: int,
-                dtype: torch.dtype, device) -> tuple:
-    """Stacked, rank-padded (A, B, scales) tensors for the active adapter set."""
-    key = (CTX.slot_ids, layer_idx, proj, n_out, dtype)
-    hit = _STACK_CACHE.get(key)
-    if hit is not None:
-        return hit
+def _get_stacks(layer_idx: int, projs: list[tuple[str, int, int]], in_size: int,
+                dtype: torch.dtype, device) -> Optional[tuple]:
+    """Stacked, rank-padded (A, B, scales, spans) of the active adapter set for the
+    projections of one input: A [L, P * R, in_size], B [L, V, R] (the projections'
+    columns one after the other) and their spans of the output.  Projections that no
+    adapter has are left out; None when that leaves none."""
+    key = (CTX.slot_ids, layer_idx, tuple(projs), dtype)
+    if key in _STACK_CACHE:
+        return _STACK_CACHE[key]
     adapters = [CTX.adapters[lid] for lid in CTX.slot_ids]
-    rmax = max(
-        (a.weights[(layer_idx, proj)][0].shape[0]
-         for a in adapters if (layer_idx, proj) in a.weights),
-        default=0,
-    )
-    if rmax == 0:
+    have = [(name, lo, hi) for name, lo, hi in projs
+            if any((layer_idx, name) in a.weights for a in adapters)]
+    if not have:
         _STACK_CACHE[key] = None
         return None
-    L = len(adapters)
-    a_stack = torch.zeros((L, rmax, in_size), dtype=dtype, device=device)
-    b_stack = torch.zeros((L, n_out, rmax), dtype=dtype, device=device)
-    scales = torch.zeros((L,), dtype=torch.float32, device=device)
+    rank = max(a.weights[(layer_idx, name)][0].shape[0]
+               for a in adapters for name, _, _ in have if (layer_idx, name) in a.weights)
+    from .. import ops
+
+    rank = next((r for r in ops.LORA_RANKS if r >= rank), rank)
+    L, width = len(adapters), sum(hi - lo for _, lo, hi in have)
+    a_stack = torch.zeros((L, len(have) * rank, in_size), dtype=dtype, device=device)
+    b_stack = torch.zeros((L, width, rank), dtype=dtype, device=device)
+    scales = torch.tensor([ad.scaling for ad in adapters], dtype=torch.float32, device=device)
     for s, ad in enumerate(adapters):
-        ab = ad.weights.get((layer_idx, proj))
-        scales[s] = ad.scaling
-        if ab is None:
-            continue
-        a, b = ab
-        a_stack[s, : a.shape[0]] = a
-        b_stack[s, :, : b.shape[1]] = b
-    _STACK_CACHE[key] = (a_stack, b_stack, scales)
+        v = 0
+        for p, (name, lo, hi) in enumerate(have):
+            ab = ad.weights.get((layer_idx, name))
+            if ab is not None:
+                a, b = ab
+                a_stack[s, p * rank: p * rank + a.shape[0]] = a
+                b_stack[s, v: v + hi - lo, : b.shape[1]] = b
+            v += hi - lo
+    _STACK_CACHE[key] = (a_stack, b_stack, scales, [(lo, hi) for _, lo, hi in have])
     return _STACK_CACHE[key]
 
 
@@ -155,13 +158,18 @@ def apply_lora(
         and x.shape[1] % 8 == 0
         and all(a.rank <= 64 for a in CTX.adapters.values())
     ):
-        for name, start, end in projs:
-            stacks = _get_stacks(layer_idx, name, end - start, x.shape[1],
-                                 x.dtype, x.device)
+        if x.dtype == torch.bfloat16 and len(projs) <= 3:
+            stacks = _get_stacks(layer_idx, projs, x.shape[1], x.dtype, x.device)
+            if stacks is not None:
+                a_stack, b_stack, scales, spans = stacks
+                ops.lora_delta(out, x, a_stack, b_stack, CTX.token_slots, scales, spans)
+            return out
+        for proj in projs:
+            stacks = _get_stacks(layer_idx, [proj], x.shape[1], x.dtype, x.device)
             if stacks is None:
                 continue
-            a_stack, b_stack, scales = stacks
-            ops.lora_bgmv(out, x, a_stack, b_stack, CTX.token_slots, scales, start)
+            a_stack, b_stack, scales, _ = stacks
+            ops.lora_bgmv(out, x, a_stack, b_stack, CTX.token_slots, scales, proj[1])
         return out
     token_ids = CTX.token_lora_ids
     for lora_id, adapter in CTX.adapters.items():

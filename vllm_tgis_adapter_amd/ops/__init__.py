@@ -344,10 +344,46 @@ def lora_bgmv(
 ) -> None:
     """Batched LoRA delta for a mixed-adapter batch (GPU only)."""
     assert _native(x), "lora_bgmv is the GPU path; CPU uses the torch loop"
+    rank = a_stack.shape[1]
+    if (x.dtype == torch.bfloat16 and rank in LORA_RANKS
+            and all(t.data_ptr() % 16 == 0 for t in (x, a_stack, b_stack))):
+        lora_delta(out, x, a_stack, b_stack, slots, scales, [(off, off + b_stack.shape[1])])
+        return
     tmp = torch.empty(
-        (x.shape[0], a_stack.shape[1]), dtype=torch.float32, device=x.device
+        (x.shape[0], rank), dtype=torch.float32, device=x.device
     )
     _C.lora_bgmv(out, x, a_stack, b_stack, tmp, slots, scales, off)
+
+
+# what lora_delta's stacks are padded to
+LORA_RANKS = (8, 16, 32, 64)
+
+
+def lora_delta(
+    out: torch.Tensor,      # [T, out_w] bf16, updated in place
+    x: torch.Tensor,        # [T, K]
+    a_stack: torch.Tensor,  # [L, P * R, K]
+    b_stack: torch.Tensor,  # [L, V, R]: the projections' columns one after the other
+    slots: torch.Tensor,    # [T] int32, -1 = no adapter
+    scales: torch.Tensor,   # [L] float32
+    spans: list[tuple[int, int]],  # each projection's columns of out
+) -> None:
+    """lora_bgmv for up to three projections of one input at once (GPU, bf16, R in
+    LORA_RANKS)."""
+    assert _native(x), "lora_delta is the GPU path; CPU uses the torch loop"
+    _C.lora_delta(out, x, a_stack, b_stack, slots, scales, spans)
+
+
+def lora_slots(token_ids: torch.Tensor, ids: tuple[int, ...]) -> torch.Tensor:
+    """Place of every token's adapter id among ``ids``, -1 where it is none of them."""
+    if native_enabled(token_ids) and token_ids.dtype == torch.int32 and len(ids) <= 64:
+        slots = torch.empty_like(token_ids, memory_format=torch.contiguous_format)
+        _C.lora_slots(slots, token_ids.contiguous(), list(ids))
+        return slots
+    slots = torch.full_like(token_ids, -1)
+    for s, lid in enumerate(ids):
+        slots[token_ids == lid] = s
+    return slots.to(torch.int32)
 
 
 def sample_argmax(
