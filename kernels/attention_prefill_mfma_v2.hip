@@ -1,9 +1,8 @@
-// MFMA prefill attention v2: flash-style causal attention over
-// the paged KV cache, rebuilt on the CDNA4 ladder that lifts the r1 kernel's
-// 11-16% MFU: KVBLK=64 tiles, a zero-conflict XOR-16 K image, hardware
-// transpose reads (ds_read_b64_tr_b16) for the V fragments, async staging
-// (global loads issued under softmax+PV), defer-max rescaling, and exp2 with
-// the softmax scale folded into the logits.
+// Prompt attention with a window, sinks, chunks, prefixes or capped scores over the paged
+// KV cache (plain causal attention: attention_prefill_tile.hip): KVBLK=64
+// tiles, a zero-conflict XOR-16 K image, hardware transpose reads (ds_read_b64_tr_b16) for
+// the V fragments, async staging (global loads issued under softmax+PV), defer-max
+// rescaling, and exp2 with the softmax scale folded into the logits.
 //
 // Geometry: one workgroup = 8 waves = one 256-row query tile per (seq, head);
 // each wave owns 32 q rows.  K/V tiles of 64 kv slots x HEAD_DIM are staged
@@ -14,8 +13,7 @@
 //      hit 16 distinct banks per lane group (zero conflict).
 //   V: 16 subtiles [32 kv][16 d] row-major, stride 1152 B (1024 + 128 pad so
 //      d0-adjacent subtiles sit 32 dword-banks apart) -> each 16-lane quarter
-//      tr-reads a [4 kv][16 d] window, conflict-free, B-fragments at b64 rate
-//      (the r1 kernel's per-element V gathers were 64 ds_read_u16 per tile).
+//      tr-reads a [4 kv][16 d] window, conflict-free, B-fragments at b64 rate.
 //
 // Swapped-operand score MFMA (S^T = K.Q^T) keeps each lane's P row local:
 // row stats need one fmax chain + one shfl_xor(32); P packs to bf16 with
@@ -27,16 +25,8 @@
 typedef __attribute__((ext_vector_type(8))) short bf16x8_t;
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 
-template <typename CT>
-DEVINLINE bf16x8_t load_kv8_v2(const CT* p);
-template <>
-DEVINLINE bf16x8_t load_kv8_v2<__hip_bfloat16>(const __hip_bfloat16* p) {
+DEVINLINE bf16x8_t load_kv8_v2(const __hip_bfloat16* p) {
   return *reinterpret_cast<const bf16x8_t*>(p);
-}
-template <>
-DEVINLINE bf16x8_t load_kv8_v2<unsigned char>(const unsigned char* p) {
-  return __builtin_bit_cast(
-      bf16x8_t, fp8x8_to_bf16x8(*reinterpret_cast<const u32x2_vec_t*>(p)));
 }
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4_b;
 typedef __attribute__((address_space(3))) bf16x4_b* lds_tr_ptr;
@@ -58,23 +48,23 @@ __device__ inline float cross_half_sum(float v) {
   return v + __shfl_xor(v, 32, 64);
 }
 
-// WS (window + sink variant): a query at position i sees keys j with
+// Window and sink: a query at position i sees keys j with
 // 0 <= i - j < window (window 0: all j <= i); with has_sink the denominator
 // also holds exp(sink); and the probabilities enter the value product as the
 // sum of two bf16 terms (rounded value + rounded remainder), so that they
 // carry 16 mantissa bits instead of 8.
-// CH (chunk variant, on top of WS with window 0): a query at position i sees
+// CH (chunk variant, window 0): a query at position i sees
 // keys j <= i of its own chunk only, floor(j / chunk) = floor(i / chunk); the
 // value cache holds v_heads <= kvh heads and key head g reads value head
 // g mod v_heads; the output is f32.
-// PX (prefix variants, on top of WS without a sink): keys ahead of the window,
+// PX (prefix variants, no sink): keys ahead of the window,
 // in tiles of their own before the window's tiles.  PX_KEEP: the sequence's
 // first `keep` tokens.  PX_POOL: one pooled key and value per block of `pool`
 // positions that ends at or before i - window; pooled block b is kept in the
 // cache block that holds its last token (per_block places each).  back (cos,
 // sin per query row and pair): the output's dims m and m + HEAD_DIM/2 are turned
 // back by the row's angles before they are rounded.
-// CAP (capped variants, on top of WS): the sink is one per head, and scores
+// CAP (capped variants): the sink is one per head, and scores
 // become softcap tanh(score / softcap) before the softmax (softcap 0: as they are).
 // CAP_FIXED: a cap also bounds the scores; up to kFixedMaxCap the exponentials are
 // taken as they are, without a running maximum or a rescale (e^60 and its inverse
@@ -132,14 +122,14 @@ DEVINLINE void cap_scores(f32x16_t* s, float scale, float softcap) {
   }
 }
 
-template <int HEAD_DIM, typename CT, int NW, bool WS, bool CH = false,
+template <int HEAD_DIM, int NW, bool CH = false,
           typename OT = __hip_bfloat16, int PX = PX_NONE, int CAP = CAP_NONE,
           int VD = HEAD_DIM>
 __global__ __launch_bounds__(NW * 64, 512 / (NW * 64)) void paged_prefill_mfma_v2_kernel(
     OT* __restrict__ out,                        // [total_q, nheads, HD]
     const __hip_bfloat16* __restrict__ q,        // [total_q, nheads, HD]
-    const CT* __restrict__ k_cache,  // [nb, bs, kvh, HD] bf16 | e4m3
-    const CT* __restrict__ v_cache,
+    const __hip_bfloat16* __restrict__ k_cache,  // [nb, bs, kvh, HD]
+    const __hip_bfloat16* __restrict__ v_cache,
     const int* __restrict__ block_tables,     // [nseq, max_blocks]
     const int* __restrict__ query_start_loc,  // [nseq+1]
     const int* __restrict__ seq_lens,         // [nseq]
@@ -155,13 +145,12 @@ __global__ __launch_bounds__(NW * 64, 512 / (NW * 64)) void paged_prefill_mfma_v
     const int v_heads = 0,
     const SpanTiles sp = SpanTiles{},
     const Capped cap = Capped{}) {
-  static_assert(CAP == CAP_NONE || (WS && !CH && PX == PX_NONE),
-                "the capped variant builds on the window variant");
+  static_assert(CAP == CAP_NONE || (!CH && PX == PX_NONE),
+                "the capped variant has a window only");
   static_assert((HEAD_DIM == 128 && VD == 128) || CAP != CAP_NONE,
                 "other head sizes are built for the capped variants only");
   static_assert(HEAD_DIM % 16 == 0 && HEAD_DIM <= 256 && (VD == 64 || VD == 128), "head sizes");
-  static_assert(PX == PX_NONE || (WS && !CH), "prefixes build on the window variant");
-  static_assert(!CH || WS, "the chunk variant builds on the window variant");
+  static_assert(PX == PX_NONE || !CH, "prefixes go with a window");
   constexpr int KCH = HEAD_DIM / 16;  // QK^T k-chunks (8)
   constexpr int DT = VD / 32;         // 32-col output tiles (4)
   constexpr int KS = (HEAD_DIM + 127) / 128 * 128;   // K image row stride (elements)
@@ -234,7 +223,7 @@ __global__ __launch_bounds__(NW * 64, 512 / (NW * 64)) void paged_prefill_mfma_v
   // first key tile any row of the workgroup sees, lowest key position any
   // row of this wave sees
   int kv_first = 0, wave_win_lo = 0;
-  if (WS && window > 0) {
+  if (window > 0) {
     kv_first = max(0, seq_len - q_len + tile_base - window + 1) / KVT2 * KVT2;
     wave_win_lo = max(0, wave_q_pos_min - window + 1);
   }
@@ -282,17 +271,17 @@ __global__ __launch_bounds__(NW * 64, 512 / (NW * 64)) void paged_prefill_mfma_v
           const int page = (pos * sp.pool + sp.pool - 1) / block_size;
           const long at = (long)btable[page] * sp.per_block +
                           (pos - page * block_size / sp.pool);
-          st_k[pass] = load_kv8_v2<__hip_bfloat16>(sp.k_pool + at * kv_row_stride +
+          st_k[pass] = load_kv8_v2(sp.k_pool + at * kv_row_stride +
                                                    (long)kv_head * HEAD_DIM + st_d8);
-          st_v[pass] = load_kv8_v2<__hip_bfloat16>(sp.v_pool + at * kv_row_stride +
+          st_v[pass] = load_kv8_v2(sp.v_pool + at * kv_row_stride +
                                                    (long)kv_head * HEAD_DIM + st_d8);
           continue;
         }
         const int block = btable[pos / block_size];
         const long tok = (long)block * block_size + pos % block_size;
-        st_k[pass] = load_kv8_v2<CT>(k_cache + tok * kv_row_stride +
+        st_k[pass] = load_kv8_v2(k_cache + tok * kv_row_stride +
                                      (long)kv_head * HEAD_DIM + st_d8);
-        st_v[pass] = load_kv8_v2<CT>(v_cache + tok * v_row_stride +
+        st_v[pass] = load_kv8_v2(v_cache + tok * v_row_stride +
                                      (long)v_head * VD + st_d8);
       }
     }
@@ -302,7 +291,7 @@ __global__ __launch_bounds__(NW * 64, 512 / (NW * 64)) void paged_prefill_mfma_v
       if (x_d8 < HEAD_DIM && pos < limit) {
         const int block = btable[pos / block_size];
         const long tok = (long)block * block_size + pos % block_size;
-        st_x = load_kv8_v2<CT>(k_cache + tok * kv_row_stride + (long)kv_head * HEAD_DIM + x_d8);
+        st_x = load_kv8_v2(k_cache + tok * kv_row_stride + (long)kv_head * HEAD_DIM + x_d8);
       }
     }
   };
@@ -345,7 +334,7 @@ __global__ __launch_bounds__(NW * 64, 512 / (NW * 64)) void paged_prefill_mfma_v
         (tile_base + wave * 32 < q_len) &&
         (prefix ? kv_base < pre_hi
                 : (kv_base <= wave_max_pos) &&
-                      (!WS || kv_base + KVT2 > wave_win_lo ||
+                      (kv_base + KVT2 > wave_win_lo ||
                        (PX == PX_KEEP && kv_base < sp.keep)));
     const char* k_lds = reinterpret_cast<const char*>(k_lds2[buf]);
     const char* v_lds = v_lds2[buf];
@@ -384,7 +373,7 @@ __global__ __launch_bounds__(NW * 64, 512 / (NW * 64)) void paged_prefill_mfma_v
           (prefix ? kv_base + KVT2 <= pre_lo
                   : (kv_base + KVT2 - 1 <= wave_q_pos_min) &&
                         (kv_base + KVT2 <= seq_len) &&
-                        (!WS || window == 0 ||
+                        (window == 0 ||
                          kv_base > wave_q_pos_min + 31 - window) &&
                         (!CH || chunk == 0 ||
                          kv_base >= (wave_q_pos_min + 31) / chunk * chunk));
@@ -408,7 +397,7 @@ __global__ __launch_bounds__(NW * 64, 512 / (NW * 64)) void paged_prefill_mfma_v
             const bool hidden =
                 prefix ? kv_pos >= q_pre
                        : kv_pos > q_pos || kv_pos >= seq_len ||
-                             (WS && window > 0 && kv_pos + window <= q_pos &&
+                             (window > 0 && kv_pos + window <= q_pos &&
                               (PX != PX_KEEP || kv_pos >= sp.keep)) ||
                              (CH && kv_pos < q_lo);
             if (!q_valid || hidden) v = -FLT_MAX;
@@ -459,8 +448,8 @@ __global__ __launch_bounds__(NW * 64, 512 / (NW * 64)) void paged_prefill_mfma_v
       l_state += cross_half_sum(local_sum);
 
       // ---- P -> bf16 A-fragments (cvt_pk + permlane32_swap, T12) -------
-      // PASSES 2 (WS): pass 1 packs what the first rounding left over
-      constexpr int PASSES = WS ? 2 : 1;
+      // pass 1 packs what the first rounding left over
+      constexpr int PASSES = 2;
       bf16x8_t pa[PASSES][4];
 #pragma unroll
       for (int ps = 0; ps < PASSES; ++ps) {
@@ -472,7 +461,7 @@ __global__ __launch_bounds__(NW * 64, 512 / (NW * 64)) void paged_prefill_mfma_v
             asm volatile("v_cvt_pk_bf16_f32 %0, %1, %2"
                          : "=v"(pk[i])
                          : "v"(p[kb * 16 + 2 * i]), "v"(p[kb * 16 + 2 * i + 1]));
-            if (WS && ps == 0) {
+            if (ps == 0) {
               p[kb * 16 + 2 * i] -= __uint_as_float(pk[i] << 16);
               p[kb * 16 + 2 * i + 1] -= __uint_as_float(pk[i] & 0xffff0000u);
             }
@@ -517,9 +506,8 @@ __global__ __launch_bounds__(NW * 64, 512 / (NW * 64)) void paged_prefill_mfma_v
           u.h[1] = rb[c];
           acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
               pa[0][c], u.v, acc_o[dt], 0, 0, 0);
-          if (WS)
-            acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                pa[PASSES - 1][c], u.v, acc_o[dt], 0, 0, 0);
+          acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              pa[PASSES - 1][c], u.v, acc_o[dt], 0, 0, 0);
         }
       }
     }
@@ -534,7 +522,7 @@ __global__ __launch_bounds__(NW * 64, 512 / (NW * 64)) void paged_prefill_mfma_v
   // (q_local check below), not per lane.
   float l_fin = l_state, o_scale = 1.f;
   const float sink_h = CAP != CAP_NONE && cap.sinks != nullptr ? cap.sinks[head] : sink;
-  if (WS && has_sink) {
+  if (has_sink) {
     // the sink joins the denominator; both terms relative to the larger of
     // the running max and the sink (log2 domain)
     const float a2 = m2_state == -FLT_MAX ? -FLT_MAX : m2_state * sc2;
@@ -574,66 +562,6 @@ __global__ __launch_bounds__(NW * 64, 512 / (NW * 64)) void paged_prefill_mfma_v
   }
 }
 
-#include <cstdlib>
-
-template <typename CT>
-static void launch_prefill_v2_ct(
-    __hip_bfloat16* out, const __hip_bfloat16* q, const CT* kc, const CT* vc,
-    const int* bt, const int* qsl, const int* sl, float scale, int nseq,
-    int nheads, int kvh, int head_dim, int block_size, int max_blocks,
-    int max_query_len, hipStream_t stream, int window = 0, int has_sink = 0,
-    float sink = 0.f, bool ws = false) {
-  if (head_dim != 128) abort();
-  if (ws) {
-    const int qtiles = (max_query_len + 255) / 256;
-    hipLaunchKernelGGL((paged_prefill_mfma_v2_kernel<128, CT, 8, true>),
-                       dim3(nseq, nheads, qtiles), dim3(512), 0, stream, out,
-                       q, kc, vc, bt, qsl, sl, scale, nheads, kvh, block_size,
-                       max_blocks, window, has_sink, sink, 0, 0, SpanTiles{}, Capped{});
-    return;
-  }
-  static const int nw = [] {
-    const char* e = getenv("VTA_PREFILL_WAVES");
-    // measured: 8-wave/256-row wins (317/560 TF vs 302/498 for 4-wave —
-    // the doubled per-CU staging traffic outweighs the causal-skew saving)
-    return (e && e[0] == '4') ? 4 : 8;
-  }();
-  if (nw == 8) {
-    const int qtiles = (max_query_len + 255) / 256;
-    hipLaunchKernelGGL((paged_prefill_mfma_v2_kernel<128, CT, 8, false>),
-                       dim3(nseq, nheads, qtiles), dim3(512), 0, stream, out,
-                       q, kc, vc, bt, qsl, sl, scale, nheads, kvh, block_size,
-                       max_blocks, 0, 0, 0.f, 0, 0, SpanTiles{}, Capped{});
-  } else {
-    const int qtiles = (max_query_len + 127) / 128;
-    hipLaunchKernelGGL((paged_prefill_mfma_v2_kernel<128, CT, 4, false>),
-                       dim3(nseq, nheads, qtiles), dim3(256), 0, stream, out,
-                       q, kc, vc, bt, qsl, sl, scale, nheads, kvh, block_size,
-                       max_blocks, 0, 0, 0.f, 0, 0, SpanTiles{}, Capped{});
-  }
-}
-
-void launch_paged_prefill_mfma_v2(
-    __hip_bfloat16* out, const __hip_bfloat16* q, const __hip_bfloat16* kc,
-    const __hip_bfloat16* vc, const int* bt, const int* qsl, const int* sl,
-    float scale, int nseq, int nheads, int kvh, int head_dim, int block_size,
-    int max_blocks, int max_query_len, hipStream_t stream) {
-  launch_prefill_v2_ct<__hip_bfloat16>(out, q, kc, vc, bt, qsl, sl, scale,
-                                       nseq, nheads, kvh, head_dim,
-                                       block_size, max_blocks, max_query_len,
-                                       stream);
-}
-
-void launch_paged_prefill_mfma_v2_fp8(
-    __hip_bfloat16* out, const __hip_bfloat16* q, const unsigned char* kc,
-    const unsigned char* vc, const int* bt, const int* qsl, const int* sl,
-    float scale, int nseq, int nheads, int kvh, int head_dim, int block_size,
-    int max_blocks, int max_query_len, hipStream_t stream) {
-  launch_prefill_v2_ct<unsigned char>(out, q, kc, vc, bt, qsl, sl, scale,
-                                      nseq, nheads, kvh, head_dim, block_size,
-                                      max_blocks, max_query_len, stream);
-}
-
 // window + sink variant (bf16 cache, HD = 128)
 void launch_paged_prefill_mfma_v2_ws(
     __hip_bfloat16* out, const __hip_bfloat16* q, const __hip_bfloat16* kc,
@@ -641,10 +569,10 @@ void launch_paged_prefill_mfma_v2_ws(
     float scale, int nseq, int nheads, int kvh, int head_dim, int block_size,
     int max_blocks, int max_query_len, int window, int has_sink, float sink,
     hipStream_t stream) {
-  launch_prefill_v2_ct<__hip_bfloat16>(out, q, kc, vc, bt, qsl, sl, scale,
-                                       nseq, nheads, kvh, head_dim,
-                                       block_size, max_blocks, max_query_len,
-                                       stream, window, has_sink, sink, true);
+  hipLaunchKernelGGL((paged_prefill_mfma_v2_kernel<128, 8>),
+                     dim3(nseq, nheads, (max_query_len + 255) / 256), dim3(512), 0, stream, out,
+                     q, kc, vc, bt, qsl, sl, scale, nheads, kvh, block_size, max_blocks, window,
+                     has_sink, sink, 0, 0, SpanTiles{}, Capped{});
 }
 
 // chunk variant with shared value heads and f32 output (bf16 cache, HD = 128)
@@ -655,7 +583,7 @@ void launch_paged_prefill_mfma_v2_chunk(
     int max_blocks, int max_query_len, int chunk, hipStream_t stream) {
   const int qtiles = (max_query_len + 255) / 256;
   hipLaunchKernelGGL(
-      (paged_prefill_mfma_v2_kernel<128, __hip_bfloat16, 8, true, true, float>),
+      (paged_prefill_mfma_v2_kernel<128, 8, true, float>),
       dim3(nseq, nheads, qtiles), dim3(512), 0, stream, out, q, kc, vc, bt, qsl,
       sl, scale, nheads, kvh, block_size, max_blocks, 0, 0, 0.f, chunk, v_heads,
       SpanTiles{}, Capped{});
@@ -674,13 +602,13 @@ void launch_paged_prefill_mfma_v2_span(
   sp.k_pool = kp; sp.v_pool = vp;
   sp.back = reinterpret_cast<const float2*>(back);
   if (pool > 0)
-    hipLaunchKernelGGL((paged_prefill_mfma_v2_kernel<128, __hip_bfloat16, 8, true, false,
+    hipLaunchKernelGGL((paged_prefill_mfma_v2_kernel<128, 8, false,
                                                      __hip_bfloat16, PX_POOL>),
                        grid, dim3(512), 0, stream, out, q, kc, vc, bt, qsl, sl, scale,
                        nheads, kvh, block_size, max_blocks, window, 0, 0.f, 0, 0, sp,
                        Capped{});
   else
-    hipLaunchKernelGGL((paged_prefill_mfma_v2_kernel<128, __hip_bfloat16, 8, true, false,
+    hipLaunchKernelGGL((paged_prefill_mfma_v2_kernel<128, 8, false,
                                                      __hip_bfloat16, PX_KEEP>),
                        grid, dim3(512), 0, stream, out, q, kc, vc, bt, qsl, sl, scale,
                        nheads, kvh, block_size, max_blocks, window, 0, 0.f, 0, 0, sp,
@@ -696,7 +624,7 @@ static void launch_prefill_capped(
     int nseq, int nheads, int kvh, int block_size, int max_blocks, int max_query_len,
     int window, const Capped& cap, hipStream_t stream) {
   const dim3 grid(nseq, nheads, (max_query_len + 255) / 256);
-  hipLaunchKernelGGL((paged_prefill_mfma_v2_kernel<HD, __hip_bfloat16, 8, true, false,
+  hipLaunchKernelGGL((paged_prefill_mfma_v2_kernel<HD, 8, false,
                                                    __hip_bfloat16, PX_NONE, CAP, VD>),
                      grid, dim3(512), 0, stream, out, q, kc, vc, bt, qsl, sl, scale, nheads,
                      kvh, block_size, max_blocks, window, cap.sinks != nullptr ? 1 : 0, 0.f, 0,

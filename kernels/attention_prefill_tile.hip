@@ -1,0 +1,501 @@
+// Paged causal prompt attention: bf16 or e4m3 cache, heads of 64 or 128.
+//
+// A workgroup takes NW waves of 32 query rows of one key head: as many of its query heads
+// as divide the waves, and the tokens that are left over of them, so that the keys of a
+// tile serve all heads and the rows of a workgroup end at nearly the same key.  Tiles of
+// 64 keys and values are staged once for all of them, bf16 straight HBM -> LDS
+// (global_load_lds), the block ids a tile ahead of the loads.
+//
+// v_mfma_f32_32x32x16_bf16 takes S^T = K Q^T, so a lane keeps one query's statistics and
+// accumulators; 16 keys of the scores enter the second product in the order the score
+// layout has them, so probabilities are packed where they are, and the values come back
+// transposed (ds_read_b64_tr_b16).  The products of the next tile's scores alternate with
+// this tile's exponentials: keys are staged a tile ahead of values.
+//
+// Bound by the matrix unit and the vector unit taking turns (heads of 128: 1024 and 1060
+// cycles of a wave and tile, 2270 taken) where the chip is full; by a wave's own chain,
+// 1.6 us a tile, where it is not, hence the cut over keys.
+//
+// Measured (MI355X, 32/8 heads of 128, before -> after): 3500 tokens of 7 prompts after
+// 700 each, bf16: 182 -> 87 us, 625 TFLOP/s; one prompt of 8192 tokens 975 TFLOP/s, 512
+// tokens after 5000 65 us.  On the way: eight waves of one head (256 tokens) leave early
+// rows' waves idle; the second product a tile behind the first, both among the exponentials,
+// 564 -> 590 us at 8192 tokens, with register staging 630; transposed reads as asm 584.
+
+#include "common.h"
+#include <float.h>
+
+typedef __attribute__((ext_vector_type(8))) short bf16x8_t;
+typedef __attribute__((ext_vector_type(4))) short s16x4_t;
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+typedef __attribute__((ext_vector_type(16))) float f32x16_t;
+typedef __attribute__((ext_vector_type(4))) unsigned int u32x4_t;
+typedef __attribute__((ext_vector_type(2))) unsigned int u32x2_t;
+typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
+
+namespace {
+
+constexpr int kTile = 64;   // keys of a step
+constexpr int kMinTiles = 6;   // a part is no shorter
+constexpr float kLog2e = 1.4426950408889634f;
+// A maximum that grew by less than this (log2) is not followed: sums and probabilities
+// stay in range, their relative precision is the same.
+constexpr float kDefer = 11.5f;
+
+typedef __attribute__((ext_vector_type(2))) float f32x2_t;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf2_t;
+DEVINLINE unsigned pack_bf16(float a, float b) {
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2_t{a, b}, bf2_t));
+}
+
+typedef __attribute__((address_space(3))) bf16x8_t lds_bf16x8_t;
+
+// Through a restrict parameter: without it the compiler takes the builtin for a read of
+// whatever is on its way to LDS, and has it wait for the loads of the next tile.
+DEVINLINE s16x4_t read_transposed(lds_s16x4_t* __restrict__ at) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(at);
+}
+
+// 16-byte chunk c of row r of a tile lies at chunk c ^ swizzle(r).  Keys: the 16 rows of
+// equal chunks cover all banks.  Values: pairs of chunks stay pairs, the four rows of a
+// transposed read lie in different banks.
+template <int HD> DEVINLINE int k_swizzle(int r) { return HD == 128 ? r & 15 : (r >> 1) & 7; }
+template <int HD> DEVINLINE int v_swizzle(int r) {
+  return HD == 128 ? (r & 7) * 2 : ((r >> 1) & 3) * 2;
+}
+
+// tiles of keys that one part takes
+DEVINLINE int tiles_per_part(int tiles, int parts) {
+  return max(kMinTiles, (tiles + parts - 1) / parts);
+}
+
+template <int HD, typename CT, int NW>
+__global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
+    __hip_bfloat16* __restrict__ out,         // [total_q, nheads, HD]
+    const __hip_bfloat16* __restrict__ q,     // [total_q, nheads, HD]
+    const CT* __restrict__ k_cache,           // [blocks, block_size, kvh, HD]
+    const CT* __restrict__ v_cache,
+    const int* __restrict__ block_tables,     // [nseq, max_blocks]
+    const int* __restrict__ query_start_loc,  // [nseq + 1]
+    const int* __restrict__ seq_lens,         // [nseq]
+    const float scale_log2, const int nheads, const int kvh, const int heads,  // of a workgroup
+    const int block_size, const int block_shift, const int max_blocks, const int parts,
+    float* __restrict__ part_acc,             // [parts, total_q, nheads, HD] (parts > 1)
+    float* __restrict__ part_ml) {            // [parts, total_q, nheads, 2]  (parts > 1)
+  constexpr bool FP8 = sizeof(CT) == 1;
+  constexpr int KS = HD / 16;          // contraction steps of a score tile
+  constexpr int DT = HD / 32;          // 32-wide tiles of the result
+  constexpr int CPR = HD / 8;          // 16-byte chunks of a row in LDS
+  constexpr int LPR = HD * sizeof(CT) / 16;   // lanes a cache row takes
+  constexpr int RPP = 64 / LPR;               // rows of a wave's load
+  constexpr int PASS = kTile / RPP / NW;      // loads of a thread, keys or values
+  constexpr int BYTES = kTile * HD * 2;
+  static_assert(PASS * RPP * NW == kTile, "whole passes");
+
+  const int seq = blockIdx.y;
+  const int q_start = query_start_loc[seq];
+  const int q_len = query_start_loc[seq + 1] - q_start;
+  const int seq_len = seq_lens[seq];
+  const int tokens = NW / heads * 32;
+  // the last tokens see the most keys: they go first
+  const int tile = (q_len + tokens - 1) / tokens - 1 - (int)blockIdx.z / parts;
+  if (tile < 0) return;
+
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int col = lane & 31, half = lane >> 5;
+  const int group = nheads / kvh, per_kv = group / heads;   // workgroups of a key head
+  const int kv_head = blockIdx.x / per_kv;
+  const int head = kv_head * group + blockIdx.x % per_kv * heads + wave % heads;
+  const int token0 = tile * tokens + wave / heads * 32;
+  const int token = min(token0 + col, q_len - 1);
+  const int past = seq_len - q_len;
+  const int keys = min(seq_len, past + min((tile + 1) * tokens, q_len));
+  const int tiles = (keys + kTile - 1) / kTile, per = tiles_per_part(tiles, parts);
+  const int first = blockIdx.z % parts * per;
+  // no keys at all: part 0 writes the zeros
+  if (first >= tiles && first > 0) return;
+  const int n = min(per, tiles - first), origin = first * kTile;
+  // positions from the part's first key on
+  const int q_pos = past + token - origin;
+  const int wave_min = past + token0 - origin;
+  const int wave_max = token0 < q_len ? past + min(token0 + 31, q_len - 1) - origin : -1;
+
+  extern __shared__ __align__(16) char lds_all[];   // keys twice, values twice
+  char* const k_lds[2] = {lds_all, lds_all + BYTES};
+  char* const v_lds[2] = {lds_all + 2 * BYTES, lds_all + 3 * BYTES};
+
+  const __hip_bfloat16* q_row = q + ((long)(q_start + token) * nheads + head) * HD + half * 8;
+  bf16x8_t qf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const bf16x8_t*>(q_row + ks * 16);
+
+  // ---- staging -----------------------------------------------------------
+  const int* table = block_tables + (long)seq * max_blocks;
+  const long row_bytes = (long)kvh * HD * sizeof(CT);
+  const char* k_at = reinterpret_cast<const char*>(k_cache) + kv_head * HD * sizeof(CT);
+  const char* v_at = reinterpret_cast<const char*>(v_cache) + kv_head * HD * sizeof(CT);
+  auto row_of = [&](int ps) { return (ps * NW + wave) * RPP + lane / LPR; };
+  // block ids of a tile's keys (past the end: of the last key), and the cache rows that
+  // they lead to: apart, so that nothing waits for the ids before the next step
+  auto pos_of = [&](int ps, int t) { return min(origin + t * kTile + row_of(ps), keys - 1); };
+  auto page_of = [&](int pos) {
+    return block_shift >= 0 ? pos >> block_shift : pos / block_size;
+  };
+  auto ids_of = [&](int (&ids)[PASS], int t) {
+#pragma unroll
+    for (int ps = 0; ps < PASS; ++ps) ids[ps] = table[page_of(pos_of(ps, t))];
+  };
+  auto slots_of = [&](int (&slots)[PASS], const int (&ids)[PASS], int t) {
+#pragma unroll
+    for (int ps = 0; ps < PASS; ++ps) {
+      const int pos = pos_of(ps, t);
+      slots[ps] = ids[ps] * block_size + (pos - page_of(pos) * block_size);
+    }
+  };
+  u32x4_t kr[FP8 ? PASS : 1], vr[FP8 ? PASS : 1];
+  auto issue = [&](const char* cache, const int (&slots)[PASS], char* lds, auto& regs,
+                   auto swizzle) {
+#pragma unroll
+    for (int ps = 0; ps < PASS; ++ps) {
+      const char* row = cache + slots[ps] * row_bytes;
+      if constexpr (FP8)
+        regs[ps] = *reinterpret_cast<const u32x4_t*>(row + lane % LPR * 16);
+      else
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) unsigned*)(row + ((lane % LPR) ^
+                                                                       swizzle(row_of(ps))) * 16),
+            (__attribute__((address_space(3))) unsigned*)(lds + (ps * NW + wave) * 1024), 16, 0,
+            0);
+    }
+  };
+  auto unpack = [&](char* lds, const auto& regs, auto swizzle) {
+#pragma unroll
+    for (int ps = 0; ps < PASS; ++ps)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        u32x2_vec_t u;
+        u[0] = regs[ps][2 * h];
+        u[1] = regs[ps][2 * h + 1];
+        const int r = row_of(ps);
+        *reinterpret_cast<bf16x8_vec_t*>(
+            lds + r * HD * 2 + ((lane % LPR * 2 + h) ^ swizzle(r)) * 16) = fp8x8_to_bf16x8(u);
+      }
+  };
+  auto k_swz = [](int r) { return k_swizzle<HD>(r); };
+  auto v_swz = [](int r) { return v_swizzle<HD>(r); };
+  // own loads have landed (or are written to LDS), everybody's have
+  auto meet = [&] {
+    if constexpr (FP8) {
+      __syncthreads();
+    } else {
+      __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
+  };
+
+  // ---- the two products ----------------------------------------------------
+  float m_state = -FLT_MAX, l_state = 0.f;   // of query `col`, raw scores; l: this half's keys
+  f32x16_t acc[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x16_t{};
+
+  // LDS addresses in the first tile of keys and of values; kept out of the compiler's sight,
+  // which would rather compute them again than keep them (where there are registers for it)
+  constexpr bool KEEP = !FP8 && NW == 8;
+  unsigned k_lane[KS], v_lane[DT];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    k_lane[ks] = col * HD * 2 + ((ks * 2 + half) ^ k_swizzle<HD>(col)) * 16;
+    if constexpr (KEEP) asm volatile("" : "+v"(k_lane[ks]));
+  }
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) {
+    const int i = lane & 15, side = lane >> 4 & 1, r = half * 4 + (i >> 2);
+    v_lane[dt] = 2 * BYTES + r * HD * 2 +
+                 (((dt * 2 + side) * 2 + ((i & 3) >> 1)) ^ v_swizzle<HD>(r)) * 16 + (i & 1) * 8;
+    if constexpr (KEEP) asm volatile("" : "+v"(v_lane[dt]));
+  }
+  auto key_frag = [&](int at, int g) {   // g: 32-key half g % 2, 16 dims g / 2
+    return *(const lds_bf16x8_t*)(k_lane[g >> 1] + (at + (g & 1) * 32 * HD * 2));
+  };
+  // next = scores of the tile in lds; between its products, work(i), i = 0..15
+  auto scores = [&](f32x16_t (&next)[2], int at, auto work) {
+    constexpr int AHEAD = 3;
+    bf16x8_t kf[AHEAD];
+#pragma unroll
+    for (int g = 0; g < AHEAD; ++g) kf[g] = key_frag(at, g);
+#pragma unroll
+    for (int g = 0; g < 2 * KS; ++g) {
+      next[g & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          kf[g % AHEAD], qf[g >> 1], g < 2 ? f32x16_t{} : next[g & 1], 0, 0, 0);
+      if (g + AHEAD < 2 * KS) kf[g % AHEAD] = key_frag(at, g + AHEAD);
+#pragma unroll
+      for (int i = 0; i < 8 / KS; ++i) work(g * (8 / KS) + i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  const float defer = kDefer / scale_log2;
+  // lane: keys base + 32 kb + 8 (r / 4) + 4 half + r % 4 of query col
+  auto follow = [&](f32x16_t (&s)[2], const int base) {
+    if (base + kTile - 1 > wave_min) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (base + kb * 32 + (r >> 2) * 8 + half * 4 + (r & 3) > q_pos) s[kb][r] = -FLT_MAX;
+    }
+    float big = fmaxf(s[0][0], s[1][0]);
+#pragma unroll
+    for (int r = 1; r < 16; ++r) big = fmaxf(fmaxf(big, s[0][r]), s[1][r]);
+    const auto sides = __builtin_amdgcn_permlane32_swap(
+        __builtin_bit_cast(unsigned, big), __builtin_bit_cast(unsigned, big), false, false);
+    big = fmaxf(__builtin_bit_cast(float, sides[0]), __builtin_bit_cast(float, sides[1]));
+    if (!__all(m_state != -FLT_MAX && big <= m_state + defer)) {
+      const float m_new = fmaxf(m_state, big);
+      const float f = __builtin_amdgcn_exp2f((m_state - m_new) * scale_log2);
+      l_state *= f;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[dt][r] *= f;
+      m_state = m_new;
+    }
+  };
+  union Probs { unsigned u[4]; bf16x8_t v; };
+  // two of 32 probabilities
+  float bias;
+  auto weigh = [&](const f32x16_t (&s)[2], Probs (&p)[4], int i) {
+    const int kb = i >> 3, r = i % 8 * 2;
+    const float a = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kb][r], scale_log2, bias));
+    const float b = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kb][r + 1], scale_log2, bias));
+    l_state += a + b;
+    p[i / 4].u[i % 4] = pack_bf16(a, b);
+  };
+  auto values = [&](const Probs (&p)[4], int buf) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        union { s16x4_t h[2]; bf16x8_t v; } vf;
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+          vf.h[x] = read_transposed(
+              (lds_s16x4_t*)(v_lane[dt] + (buf * BYTES + (2 * c + x) * 8 * HD * 2)));
+        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.v, p[c].v, acc[dt], 0, 0, 0);
+      }
+  };
+
+  f32x16_t s0[2], s1[2];
+  int slots[PASS], ids[PASS];   // rows of tile t + 1, block ids of tile t + 2
+  auto step = [&](int t, f32x16_t (&now)[2], f32x16_t (&next)[2], int buf) {
+    meet();
+    const bool more_k = t + 2 < n, more_v = t + 1 < n;
+    if (more_v) issue(v_at, slots, v_lds[buf ^ 1], vr, v_swz);
+    if (more_k) {
+      slots_of(slots, ids, t + 2);
+      issue(k_at, slots, k_lds[buf], kr, k_swz);
+      if (t + 3 < n) ids_of(ids, t + 3);
+    }
+    // wave-uniform: the matrix unit wants all lanes
+    if (t * kTile <= wave_max) {
+      Probs p[4];
+      follow(now, t * kTile);
+      bias = m_state == -FLT_MAX ? 0.f : -m_state * scale_log2;
+      auto work = [&](int i) { weigh(now, p, i); };
+      if (more_v && (t + 1) * kTile <= wave_max) {
+        scores(next, (buf ^ 1) * BYTES, work);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) work(i);
+      }
+      values(p, buf);
+    }
+    if constexpr (FP8) {
+      if (more_v) unpack(v_lds[buf ^ 1], vr, v_swz);
+      if (more_k) unpack(k_lds[buf], kr, k_swz);
+    }
+  };
+  if (n > 0) {
+    ids_of(ids, 0);
+    slots_of(slots, ids, 0);
+    issue(k_at, slots, k_lds[0], kr, k_swz);
+    issue(v_at, slots, v_lds[0], vr, v_swz);
+    if constexpr (FP8) {
+      unpack(k_lds[0], kr, k_swz);
+      unpack(v_lds[0], vr, v_swz);
+    }
+    if (n > 1) {
+      ids_of(ids, 1);
+      slots_of(slots, ids, 1);
+      issue(k_at, slots, k_lds[1], kr, k_swz);
+      if constexpr (FP8) unpack(k_lds[1], kr, k_swz);
+      if (n > 2) ids_of(ids, 2);
+    }
+    meet();
+    if (0 <= wave_max) scores(s0, 0, [](int) {});
+    for (int t = 0; t < n; t += 2) {
+      step(t, s0, s1, 0);
+      if (t + 1 < n) step(t + 1, s1, s0, 1);
+    }
+  }
+
+  l_state += __shfl_xor(l_state, 32, 64);
+  if (token0 + col >= q_len) return;
+  const long row = (long)(q_start + token) * nheads + head;
+  if (per < tiles) {
+    const long at = blockIdx.z % parts * ((long)query_start_loc[gridDim.y] * nheads) + row;
+    float* o = part_acc + at * HD + half * 4;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; r += 4)
+        *reinterpret_cast<f32x4_t*>(o + dt * 32 + r * 2) =
+            f32x4_t{acc[dt][r], acc[dt][r + 1], acc[dt][r + 2], acc[dt][r + 3]};
+    if (half == 0) {
+      part_ml[at * 2] = m_state == -FLT_MAX ? -FLT_MAX : m_state * scale_log2;
+      part_ml[at * 2 + 1] = l_state;
+    }
+    return;
+  }
+  const float inv = l_state > 0.f ? 1.f / l_state : 0.f;
+  __hip_bfloat16* o = out + row * HD + half * 4;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; r += 4) {
+      u32x2_t w;
+      w[0] = pack_bf16(acc[dt][r] * inv, acc[dt][r + 1] * inv);
+      w[1] = pack_bf16(acc[dt][r + 2] * inv, acc[dt][r + 3] * inv);
+      *reinterpret_cast<u32x2_t*>(o + dt * 32 + r * 2) = w;
+    }
+}
+
+// Tokens whose keys were cut: out = sum_p f_p acc_p / sum_p f_p l_p.  grid (tokens of the
+// longest prompt, sequences, heads / 4), a wave a head; parts <= 16.
+template <int HD>
+__global__ __launch_bounds__(256) void prefill_tile_merge_kernel(
+    __hip_bfloat16* __restrict__ out, const float* __restrict__ part_acc,
+    const float* __restrict__ part_ml, const int* __restrict__ query_start_loc,
+    const int* __restrict__ seq_lens, const int nheads, const int tokens, const int parts) {
+  const int seq = blockIdx.y, token = blockIdx.x;
+  const int head = blockIdx.z * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int q_start = query_start_loc[seq], q_len = query_start_loc[seq + 1] - q_start;
+  if (token >= q_len || head >= nheads) return;
+  const int seq_len = seq_lens[seq], past = seq_len - q_len;
+  const int keys = min(seq_len, past + min((token / tokens + 1) * tokens, q_len));
+  const int tiles = (keys + kTile - 1) / kTile, per = tiles_per_part(tiles, parts);
+  if (per >= tiles) return;
+  const int used = (tiles + per - 1) / per;
+  const long rows = (long)query_start_loc[gridDim.y] * nheads;
+  const long row = (long)(q_start + token) * nheads + head;
+  const float* ml = part_ml + (min(lane, used - 1) * rows + row) * 2;
+  const float m = lane < used ? ml[0] : -FLT_MAX, l = lane < used ? ml[1] : 0.f;
+  constexpr int V = HD / 64;
+  const float* acc = part_acc + row * HD + lane * V;
+  float a[V] = {};
+  const float top = wave_reduce_max(m);
+  const float f = lane < used ? __builtin_amdgcn_exp2f(m - top) : 0.f;
+  const float sum = wave_reduce_sum(f * l);
+  for (int p0 = 0; p0 < used; p0 += 4) {   // four loads on their way at a time
+    float v[4][V];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < V; ++j) v[i][j] = acc[min(p0 + i, used - 1) * rows * HD + j];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (p0 + i < used)
+#pragma unroll
+        for (int j = 0; j < V; ++j) a[j] += __shfl(f, p0 + i, 64) * v[i][j];
+  }
+  const float inv = sum > 0.f ? 1.f / sum : 0.f;
+#pragma unroll
+  for (int j = 0; j < V; ++j) out[row * HD + lane * V + j] = __float2bfloat16(a[j] * inv);
+}
+
+struct Cut {
+  int waves, heads, tokens, parts;   // of a workgroup; workgroups a tile's keys are cut over
+};
+
+// Eight waves share every tile of keys where their workgroups, with the keys cut into parts
+// where there are few, fill more than half the chip; else four do, two such workgroups a
+// CU.  Measured, heads 32/8 of 128 (us, waves/parts): 3500 tokens of 7 prompts after 700
+// each 8/1 87, 4/1 88, 8/2 133; 512 after 5000 8/1 167, 4/1 146, 8/2 99, 8/4 65, 4/4 69, 8/8
+// 77; 1000 after 3000 8/1 130, 8/2 87, 8/4 91; 64 after 6000 4/1 157, 4/8 34, 4/16 29, 8/16
+// 33; 4 of 100 after 1000 8/1 41, 4/1 36, 4/2 34; 4 of 50 after 500 (9 tiles) 4/1 21, 4/2 26;
+// one of 300 8/1 17, 4/1 14.5.
+Cut cut_of(int nseq, int nheads, int kvh, int max_query_len, int max_keys) {
+  const int group = nheads / kvh, most = max_keys / (kTile * kMinTiles);
+  Cut c{};
+  for (c.waves = 8;; c.waves = 4) {
+    c.heads = c.waves;
+    while (group % c.heads) c.heads /= 2;
+    c.tokens = c.waves / c.heads * 32;
+    const long blocks =
+        (long)nheads / c.heads * nseq * ((max_query_len + c.tokens - 1) / c.tokens);
+    const long fit = 256 * 8 / c.waves / (blocks > 0 ? blocks : 1);
+    c.parts = fit < 16 ? (int)fit : 16;
+    if (c.parts > most) c.parts = most;
+    if (c.parts < 1) c.parts = 1;
+    if (c.waves == 4 || blocks * c.parts > 128) return c;
+  }
+}
+
+template <int HD, typename CT>
+void launch(__hip_bfloat16* out, float* part_acc, float* part_ml, const __hip_bfloat16* q,
+            const CT* kc, const CT* vc, const int* bt, const int* qsl, const int* sl,
+            float scale, int nseq, int nheads, int kvh, int block_size, int max_blocks,
+            int max_query_len, const Cut& c, hipStream_t stream) {
+  const int shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz(block_size) : -1;
+  const int tiles = (max_query_len + c.tokens - 1) / c.tokens;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(nheads / c.heads, nseq, tiles * c.parts),
+                       dim3(c.waves * 64), 4 * kTile * HD * 2, stream, out, q, kc, vc, bt, qsl,
+                       sl, scale * kLog2e, nheads, kvh, c.heads, block_size, shift, max_blocks,
+                       c.parts, part_acc, part_ml);
+  };
+  if (c.waves == 8) go(paged_prefill_tile_kernel<HD, CT, 8>);
+  else go(paged_prefill_tile_kernel<HD, CT, 4>);
+  if (c.parts > 1)
+    hipLaunchKernelGGL((prefill_tile_merge_kernel<HD>), dim3(max_query_len, nseq, (nheads + 3) / 4),
+                       dim3(256), 0, stream, out, part_acc, part_ml, qsl, sl, nheads, c.tokens, c.parts);
+}
+
+}  // namespace
+
+// Workgroups that a prompt's keys may be cut over (a function of shapes only): 1, or the
+// launch needs part_acc [parts, tokens, nheads, head_dim] and part_ml [parts, tokens,
+// nheads, 2].
+int prefill_tile_parts(int nseq, int nheads, int kvh, int max_query_len, int max_keys) {
+  return cut_of(nseq, nheads, kvh, max_query_len, max_keys).parts;
+}
+
+void launch_paged_prefill_tile(__hip_bfloat16* out, float* part_acc, float* part_ml,
+                               const __hip_bfloat16* q, const __hip_bfloat16* kc,
+                               const __hip_bfloat16* vc, const int* bt, const int* qsl,
+                               const int* sl, float scale, int nseq, int nheads, int kvh,
+                               int head_dim, int block_size, int max_blocks, int max_query_len,
+                               int max_keys, hipStream_t stream) {
+  const Cut c = cut_of(nseq, nheads, kvh, max_query_len, max_keys);
+  auto go = [&](auto launch) {
+    launch(out, part_acc, part_ml, q, kc, vc, bt, qsl, sl, scale, nseq, nheads, kvh, block_size,
+           max_blocks, max_query_len, c, stream);
+  };
+  if (head_dim == 128) go(launch<128, __hip_bfloat16>);
+  else go(launch<64, __hip_bfloat16>);
+}
+
+// heads of 128
+void launch_paged_prefill_tile_fp8(__hip_bfloat16* out, float* part_acc, float* part_ml,
+                                   const __hip_bfloat16* q, const unsigned char* kc,
+                                   const unsigned char* vc, const int* bt, const int* qsl,
+                                   const int* sl, float scale, int nseq, int nheads, int kvh,
+                                   int block_size, int max_blocks, int max_query_len,
+                                   int max_keys, hipStream_t stream) {
+  launch<128, unsigned char>(out, part_acc, part_ml, q, kc, vc, bt, qsl, sl, scale, nseq, nheads,
+                             kvh, block_size, max_blocks, max_query_len,
+                             cut_of(nseq, nheads, kvh, max_query_len, max_keys),
+                             stream);
+}

@@ -17,15 +17,15 @@ template <typename T>
 void launch_paged_prefill(T*, const T*, const T*, const T*, const int*,
                           const int*, const int*, float, int, int, int, int,
                           int, int, int, hipStream_t);
-void launch_paged_prefill_mfma_v2(__hip_bfloat16*, const __hip_bfloat16*,
-                                  const __hip_bfloat16*, const __hip_bfloat16*,
-                                  const int*, const int*, const int*, float,
-                                  int, int, int, int, int, int, int,
-                                  hipStream_t);
-void launch_paged_prefill_mfma(__hip_bfloat16*, const __hip_bfloat16*,
-                               const __hip_bfloat16*, const __hip_bfloat16*,
-                               const int*, const int*, const int*, float, int,
-                               int, int, int, int, int, int, hipStream_t);
+int prefill_tile_parts(int nseq, int nheads, int kvh, int max_query_len, int max_keys);
+void launch_paged_prefill_tile(__hip_bfloat16*, float*, float*, const __hip_bfloat16*,
+                               const __hip_bfloat16*, const __hip_bfloat16*, const int*,
+                               const int*, const int*, float, int, int, int, int, int, int, int,
+                               int, hipStream_t);
+void launch_paged_prefill_tile_fp8(__hip_bfloat16*, float*, float*, const __hip_bfloat16*,
+                                   const unsigned char*, const unsigned char*, const int*,
+                                   const int*, const int*, float, int, int, int, int, int, int,
+                                   int, hipStream_t);
 void launch_paged_prefill_mfma_v2_capped(__hip_bfloat16*, const __hip_bfloat16*,
                                          const __hip_bfloat16*, const __hip_bfloat16*,
                                          const int*, const int*, const int*, float, int, int,
@@ -45,11 +45,6 @@ void launch_paged_decode_stream_fp8(__hip_bfloat16*, float*, float*, const __hip
                                     const unsigned char*, const unsigned char*, const int*,
                                     const int*, float, int, int, int, int, int, int, int,
                                     hipStream_t);
-void launch_paged_prefill_mfma_v2_fp8(__hip_bfloat16*, const __hip_bfloat16*,
-                                      const unsigned char*,
-                                      const unsigned char*, const int*,
-                                      const int*, const int*, float, int, int,
-                                      int, int, int, int, int, hipStream_t);
 void launch_paged_prefill_mfma_v2_ws(__hip_bfloat16*, const __hip_bfloat16*,
                                      const __hip_bfloat16*, const __hip_bfloat16*,
                                      const int*, const int*, const int*, float,
@@ -189,57 +184,60 @@ void paged_attention_prefill(torch::Tensor out, torch::Tensor q,
                              torch::Tensor block_tables,
                              torch::Tensor query_start_loc,
                              torch::Tensor seq_lens, double scale,
-                             int64_t max_query_len) {
+                             int64_t max_query_len, int64_t max_seq_len) {
   const int nseq = seq_lens.size(0);
   const int nheads = q.size(1);
   const int head_dim = q.size(2);
   const int kvh = k_cache.size(2);
   const int block_size = k_cache.size(1);
   const int max_blocks = block_tables.size(1);
+  if (nseq == 0 || max_query_len <= 0) return;
   if (!q.is_contiguous()) q = q.contiguous();   // the kernels read dense rows
   static const bool force_valu = [] {
     const char* e = getenv("VTA_PREFILL_VALU");
     return e && e[0] == '1';
   }();
-  static const bool force_v1 = [] {
-    const char* e = getenv("VTA_PREFILL_V1");
-    return e && e[0] == '1';
-  }();
+  const bool tiles = q.scalar_type() == at::ScalarType::BFloat16 &&
+                     (head_dim == 128 || (head_dim == 64 &&
+                                          k_cache.scalar_type() == at::ScalarType::BFloat16));
+  // the longest sequence only decides how the work is cut
+  const int max_keys = (int)std::min<int64_t>(max_seq_len, (int64_t)max_blocks * block_size);
+  const int64_t parts =
+      tiles && (!force_valu || k_cache.scalar_type() == at::ScalarType::Byte)
+          ? prefill_tile_parts(nseq, nheads, kvh, (int)max_query_len, max_keys)
+          : 1;
+  torch::Tensor part_acc, part_ml;
+  float *acc = nullptr, *ml = nullptr;
+  if (parts > 1) {
+    const auto opt = q.options().dtype(at::ScalarType::Float);
+    part_acc = at::empty({parts, q.size(0), nheads, head_dim}, opt);
+    part_ml = at::empty({parts, q.size(0), nheads, 2}, opt);
+    acc = part_acc.data_ptr<float>();
+    ml = part_ml.data_ptr<float>();
+  }
   if (k_cache.scalar_type() == at::ScalarType::Byte) {
     TORCH_CHECK(q.scalar_type() == at::ScalarType::BFloat16 && head_dim == 128,
-                "fp8 KV cache requires the bf16 v2 prefill path (hd=128)");
-    launch_paged_prefill_mfma_v2_fp8(
-        reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
+                "fp8 KV cache requires bf16 queries and heads of 128");
+    launch_paged_prefill_tile_fp8(
+        reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), acc, ml,
         reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()),
         reinterpret_cast<const unsigned char*>(k_cache.data_ptr()),
         reinterpret_cast<const unsigned char*>(v_cache.data_ptr()),
         block_tables.data_ptr<int>(), query_start_loc.data_ptr<int>(),
-        seq_lens.data_ptr<int>(), (float)scale, nseq, nheads, kvh, head_dim,
-        block_size, max_blocks, (int)max_query_len, current_stream());
-    return;
-  }
-  if (!force_valu && !force_v1 &&
-      q.scalar_type() == at::ScalarType::BFloat16 && head_dim == 128) {
-    launch_paged_prefill_mfma_v2(
-        reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
-        reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()),
-        reinterpret_cast<const __hip_bfloat16*>(k_cache.data_ptr()),
-        reinterpret_cast<const __hip_bfloat16*>(v_cache.data_ptr()),
-        block_tables.data_ptr<int>(), query_start_loc.data_ptr<int>(),
-        seq_lens.data_ptr<int>(), (float)scale, nseq, nheads, kvh, head_dim,
-        block_size, max_blocks, (int)max_query_len, current_stream());
+        seq_lens.data_ptr<int>(), (float)scale, nseq, nheads, kvh,
+        block_size, max_blocks, (int)max_query_len, max_keys, current_stream());
     return;
   }
   if (!force_valu && q.scalar_type() == at::ScalarType::BFloat16 &&
       (head_dim == 64 || head_dim == 128)) {
-    launch_paged_prefill_mfma(
-        reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
+    launch_paged_prefill_tile(
+        reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), acc, ml,
         reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()),
         reinterpret_cast<const __hip_bfloat16*>(k_cache.data_ptr()),
         reinterpret_cast<const __hip_bfloat16*>(v_cache.data_ptr()),
         block_tables.data_ptr<int>(), query_start_loc.data_ptr<int>(),
         seq_lens.data_ptr<int>(), (float)scale, nseq, nheads, kvh, head_dim,
-        block_size, max_blocks, (int)max_query_len, current_stream());
+        block_size, max_blocks, (int)max_query_len, max_keys, current_stream());
     return;
   }
   DISPATCH_FLOATING(q.scalar_type(), {

@@ -47,7 +47,7 @@ _SEQ_SOURCES = ["stream_ops.hip", "canon_conv.hip", "layer_norm_stream.hip",
 _SHARED_SOURCES = ["moe_gemm.hip"]
 _LAT_SOURCES = ["latent_attention.hip", "latent_attention_mfma.hip"]
 _ATTN_SOURCES = ["attention.hip", "attention_decode_mfma.hip", "attention_decode_stream.hip",
-                 "attention_prefill_mfma.hip", "attention_prefill_mfma_v2.hip"]
+                 "attention_prefill_mfma_v2.hip", "attention_prefill_tile.hip"]
 
 EXTENSIONS = {
     "_C": dict(

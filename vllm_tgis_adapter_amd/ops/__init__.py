@@ -177,7 +177,7 @@ def paged_attention_prefill(
         out = torch.empty_like(q)
         _C.paged_attention_prefill(
             out, q, k_cache, v_cache, block_tables, query_start_loc, seq_lens,
-            scale, max_query_len
+            scale, max_query_len, max_seq_len
         )
         return out
     if k_cache.dtype == torch.uint8:  # fp8 KV: dequantize for the reference
@@ -967,7 +967,8 @@ def gqa_attention_prefill(q, k_cache, v_cache, block_tables, query_start_loc,
             dst = out if out.is_contiguous() else torch.empty_like(q)
             _attn_ext().paged_attention_prefill(dst, q, k_cache, v_cache, block_tables,
                                        query_start_loc, seq_lens, float(scale),
-                                       int(max_query_len))
+                                       int(max_query_len),
+                                       block_tables.shape[1] * k_cache.shape[1])
             if dst is not out:
                 out.copy_(dst)
             return out
