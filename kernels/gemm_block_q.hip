@@ -16,7 +16,7 @@
 // x and W reach LDS without registers; x chunks are swizzled as in block_gemm.h, W rows of
 // 64 (32) bytes by r / 4 (r / 8).
 //
-// Measured: four llama-3-8b layers around attention, 301 rows, int8: 5101 -> 1061 us.
+// Measured: four llama-3-8b layers around attention, 301 rows, int8: 5101 -> 1046 us.
 // Widening 28672 x 4096: 61 us (5.8 TB/s).
 
 #include "block_gemm.h"
@@ -67,12 +67,11 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_block_q_kernel(
   // a chunk's place in its row is turned by the row: rows of 256, 128, 64 bytes
   auto swz = [](int lanes, int r) { return lanes == 16 ? r % 16 : lanes == 8 ? r / 2 % 8 : r / 4 % 4; };
 
-  unsigned long a_off[A_PASS];
-  unsigned b_off[B_PASS], s_off = 0;
+  unsigned a_off[A_PASS], b_off[B_PASS], s_off = 0;
 #pragma unroll
   for (int p = 0; p < A_PASS; ++p) {
     const int r = (p * WAVES + wave) * (64 / AL) + lane / AL;
-    a_off[p] = (unsigned long)min(m0 + r, M - 1) * K * 2 + ((lane % AL) ^ swz(AL, r)) * 16;
+    a_off[p] = (min(m0 + r, M - 1) - m0) * (K * 2) + ((lane % AL) ^ swz(AL, r)) * 16;
   }
   // (where there are fewer loads than waves some are made twice: all waves wait alike)
 #pragma unroll
@@ -80,31 +79,22 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_block_q_kernel(
     const int r = (p * WAVES + wave) % B_LOADS * (64 / WL) + lane / WL;
     b_off[p] = r * (K * QB / 8) + ((lane % WL) ^ swz(WL, r)) * 16;
   }
-  if constexpr (QB == 4) s_off = (unsigned)(wave % (BN / 64) * 64 + lane) * (K / 128);
-  const char* xa = reinterpret_cast<const char*>(x);
-  const char* wb = reinterpret_cast<const char*>(w) + (long)n0 * (K * QB / 8);
-  const float* sb = QB == 4 ? scale + (long)n0 * (K / 128) : scale;
+  if constexpr (QB == 4) s_off = (wave % (BN / 64) * 64 + lane) * (K / 128) * 4;
+  const auto x_from = block_gemm::resource(x + (long)m0 * K);
+  const auto w_from = block_gemm::resource(w + (long)n0 * (K * QB / 8));
+  const auto s_from = block_gemm::resource(QB == 4 ? scale + (long)n0 * (K / 128) : scale);
   auto stage = [&](int buf, int tile) {
     char* to = lds + buf * STAGE;
 #pragma unroll
     for (int p = 0; p < A_PASS; ++p)
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) unsigned*)(xa + (long)tile * (DEPTH * 2) +
-                                                              a_off[p]),
-          (__attribute__((address_space(3))) unsigned*)(to + (p * WAVES + wave) * 1024), 16, 0, 0);
+      block_gemm::load_lds(to + (p * WAVES + wave) * 1024, x_from, a_off[p], tile * (DEPTH * 2));
 #pragma unroll
     for (int p = 0; p < B_PASS; ++p)
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) unsigned*)(wb + (long)tile * WB + b_off[p]),
-          (__attribute__((address_space(3))) unsigned*)(to + A_BYTES +
-                                                        (p * WAVES + wave) % B_LOADS * 1024),
-          16, 0, 0);
+      block_gemm::load_lds(to + A_BYTES + (p * WAVES + wave) % B_LOADS * 1024, w_from, b_off[p],
+                           tile * WB);
     if constexpr (QB == 4)
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) unsigned*)(sb + s_off + tile),
-          (__attribute__((address_space(3))) unsigned*)(to + A_BYTES + B_BYTES +
-                                                        wave % (BN / 64) * 256),
-          4, 0, 0);
+      block_gemm::load_lds4(to + A_BYTES + B_BYTES + wave % (BN / 64) * 256, s_from, s_off,
+                              tile * 4);
   };
 
   f32x4_t acc[TM][TN];
