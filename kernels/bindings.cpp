@@ -61,6 +61,9 @@ void launch_reshape_and_cache_fp8(const __hip_bfloat16*,
                                   unsigned char*, const long*, int, int, long,
                                   long, hipStream_t);
 int gemm_stream_parts(int qbits, int M, int N, int K, bool gated);
+int gemm_block_parts(int M, int N, int K);
+void launch_gemm_block(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hip_bfloat16*, int,
+                       int, int, int, hipStream_t);
 void launch_gemm_stream(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hip_bfloat16*,
                         int, int, int, int, hipStream_t);
 void launch_gemm_stream_gated(__hip_bfloat16*, float*, const __hip_bfloat16*,
@@ -441,6 +444,27 @@ void lora_bgmv(torch::Tensor out, torch::Tensor x, torch::Tensor a_stack,
   });
 }
 
+// y = x w^T by large tiles, K cut over workgroups
+void gemm_block(torch::Tensor y, torch::Tensor x, torch::Tensor w) {
+  for (const auto& t : {y, x, w})
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::ScalarType::BFloat16 &&
+                t.is_contiguous() && t.dim() == 2);
+  const int64_t M = x.size(0), K = x.size(1), N = y.size(1);
+  TORCH_CHECK(y.size(0) == M && w.size(0) == N && w.size(1) == K);
+  TORCH_CHECK(N % 128 == 0 && K % 64 == 0 && M < (1 << 24) && N < (1 << 24) && K < (1 << 23));
+  if (M == 0 || N == 0) return;
+  if (K == 0) {
+    y.zero_();
+    return;
+  }
+  const int parts = gemm_block_parts((int)M, (int)N, (int)K);
+  torch::Tensor part;
+  if (parts > 1) part = at::empty({parts, M, N}, x.options().dtype(at::ScalarType::Float));
+  launch_gemm_block(ptr<__hip_bfloat16>(y), parts > 1 ? part.data_ptr<float>() : nullptr,
+                    cptr<__hip_bfloat16>(x), cptr<__hip_bfloat16>(w), (int)M, (int)N, (int)K,
+                    parts, current_stream());
+}
+
 // bf16: out[t, start_p ...] += scale · B_p A_p x[t] for up to three projections of x, whose
 // adapters' weights are stacked side by side: a [L, P R, K], b [L, V, R], spans[p] = (start,
 // end) in out's columns, V = the sum of their widths.
@@ -657,6 +681,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "fused log-softmax + top-K + sampled-token rank (one HBM pass)");
   m.def("sample_argmax", &sample_argmax,
         "fused temperature/gumbel-race sampling + greedy argmax (CDNA4)");
+  m.def("gemm_block", &gemm_block, "product of more than 64 rows, large tiles");
   m.def("lora_delta", &lora_delta,
         "bf16 multi-LoRA of up to three projections of one input");
   m.def("lora_slots", &lora_slots, "adapter slot of every token");

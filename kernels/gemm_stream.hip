@@ -54,6 +54,22 @@ __global__ __launch_bounds__(256) void gemm_stream_merge_kernel(
   *reinterpret_cast<uint2*>(y + at) = o.u;
 }
 
+}  // namespace
+
+// y = the sum of parts of a product (of silu of the first half times the second)
+void launch_gemm_merge(__hip_bfloat16* y, const float* part, long plane, int parts, bool gated,
+                       hipStream_t stream) {
+  const dim3 grid((plane / 4 + 255) / 256);
+  if (gated)
+    hipLaunchKernelGGL(gemm_stream_merge_kernel<true>, grid, dim3(256), 0, stream, y, part, plane,
+                       parts);
+  else
+    hipLaunchKernelGGL(gemm_stream_merge_kernel<false>, grid, dim3(256), 0, stream, y, part,
+                       plane, parts);
+}
+
+namespace {
+
 // How a product is cut (waves along N x waves along K, workgroups along K).  The lines
 // are where they measured fastest (us; bf16 unless said; N x K):
 //   up to 16 rows of x, x is a small part of what is read and waves work alone:
@@ -111,11 +127,7 @@ void launch_mt(__hip_bfloat16* y, float* part, const __hip_bfloat16* x, const vo
       run(launch_cut<QB, MT, GATED, 4, 2>);
     }
   }
-  if (parts > 1) {
-    const long plane = (long)M * N;
-    hipLaunchKernelGGL((gemm_stream_merge_kernel<GATED>), dim3((plane / 4 + 255) / 256),
-                       dim3(256), 0, stream, y, part, plane, parts);
-  }
+  if (parts > 1) launch_gemm_merge(y, part, (long)M * N, parts, GATED, stream);
 }
 
 template <int QB, bool GATED>

@@ -1,0 +1,55 @@
+"""bf16 products by large tiles with a cut K (gemm_block.hip) against float64: rows around
+the tiles of 128, a K of one tile, of uneven and of equal parts, and the rule that sends a
+product there."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# N, K: one part, parts of unequal length (193 tiles in 8), eight equal ones, two a CU
+SHAPES = [(128, 64), (384, 960), (128, 12352), (2048, 8192), (4096, 14336), (10240, 8192)]
+
+
+def _need():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+
+
+def _inputs(m, n, k):
+    g = torch.Generator("cuda").manual_seed(m + n + k)
+    return [torch.randn((r, k), generator=g, device="cuda").bfloat16() for r in (m, n)]
+
+
+def _check(got, x, w):
+    """float32 sums, one rounding to bf16: half a unit in the last of 8 bits of the
+    value, and 2**-20 of the terms' size."""
+    want = x.double() @ w.double().t()
+    terms = x.double().abs() @ w.double().abs().t()
+    err = (got.double() - want).abs()
+    assert (err <= 2 ** -8 * want.abs() + 2 ** -20 * terms).all(), err.max().item()
+
+
+@pytest.mark.parametrize("m", [1, 65, 127, 128, 129, 257, 512])
+@pytest.mark.parametrize(("n", "k"), SHAPES)
+def test_tiles(m, n, k):
+    _need()
+    from vllm_tgis_adapter_amd.ops import _C
+
+    x, w = _inputs(m, n, k)
+    y = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    _C.gemm_block(y, x, w)
+    _check(y, x, w)
+
+
+@pytest.mark.parametrize(("m", "n", "k"), [
+    (64, 4096, 14336), (65, 4096, 14336), (512, 4096, 14336), (513, 4096, 14336),
+    (256, 8192, 8192), (257, 8192, 8192), (128, 2048, 8192), (129, 2048, 8192)])
+def test_rule(m, n, k):
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    x, w = _inputs(m, n, k)
+    _check(ops.linear(x, w), x, w)

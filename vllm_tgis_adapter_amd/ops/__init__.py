@@ -195,8 +195,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
     hipBLASLt runs the M<=64 llama decode shapes at 22-43% of the HBM
     roofline (tools/gemm_bench.py); the hand-written MFMA kernel streams the
     weight matrix once with waves splitting K in-workgroup.  Larger M stays
-    on hipBLASLt (the in-tree tile kernel only reached parity there —
-    VTA_GEMM_MAX_M raises the cutover for experiments).
+    on hipBLASLt (VTA_GEMM_MAX_M raises the cutover for experiments) but for
+    the rows and inputs of ``_block_rows``.
     """
     max_m = int(os.environ.get("VTA_GEMM_MAX_M", "64"))
     tile_max_m = int(os.environ.get("VTA_GEMM_TILE_MAX_M", "0"))
@@ -224,7 +224,26 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
             )
             _C.gemm_tile(out, x, weight)
             return out
+        if m > max_m and m in _block_rows(weight.shape[0], x.shape[1]):
+            out = torch.empty(
+                (m, weight.shape[0]), dtype=x.dtype, device=x.device
+            )
+            _C.gemm_block(out, x, weight)
+            return out
     return torch.nn.functional.linear(x, weight, bias)
+
+
+def _block_rows(n: int, k: int) -> range:
+    """Rows of a product past 64 that the tiles with a cut K take from the library:
+    where K is so long that its few tiles leave the chip idle.  us, library | tiles:
+    2048 x 8192 128 rows 21.3 | 23.7, 160 25.8 | 24.4, 700 44 | 38, 1000 49 | 48;
+    8192 x 8192 65 rows 35.1 | 34.5, 256 76 | 55, 301 66 | 71; 4096 x 14336 65 rows
+    48.6 | 40.8, 512 89 | 85, 700 101 | 112; 4096 x 4096 65 rows 16 | 18, 512 29 | 32."""
+    if k < 8192:
+        return range(0)
+    if n * k <= 1 << 24:
+        return range(129, 701)
+    return range(65, 257 if k < 12288 else 513)
 
 
 def gemm_tile(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
