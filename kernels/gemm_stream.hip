@@ -1,4 +1,5 @@
-// Products of few rows with a whole weight matrix (decode, M <= 64):
+// Products of few rows with a whole weight matrix (decode, M <= 64; a single row with bf16
+// or 4-bit weights: gemm_row.hip):
 //   y[m, n] = sum_k x[m, k] W[n, k],  or  silu(x Wg^T) * (x Wu^T) for W = [Wg; Wu],
 // with W in bf16, in int8 (a scale per row) or in 4 bits (offset 8, a scale per row
 // and 128 inputs).
@@ -26,8 +27,6 @@
 //   23 rows, 14336 x 4096 gated 55.2 -> 43.4; the mean of 6144 x 4096, 4096 x 4096 and
 //     4096 x 14336 23.9 -> 17.5 (a llama-3-8b layer reads W at 4.5 TB/s);
 //   61 rows, the mean of these three and 28672 x 4096: 38.1 -> 30;
-//   1 row, 4 bits, the mean of the same four: 26.9 -> 10.9 (28672 x 4096: 18.3);
-//   a llama-1b step of one stream 727 -> 486 us, a llama-3-8b one in 4 bits 1139 -> 753.
 
 #include "gemm_stream.h"
 
@@ -154,23 +153,36 @@ int gemm_stream_parts(int qbits, int M, int N, int K, bool gated) {
   return parts < most ? parts : most;
 }
 
+bool gemm_row_fits(int qbits, int K);
+void launch_gemm_row(__hip_bfloat16* y, const __hip_bfloat16* x, const void* w,
+                     const float* scale, int qbits, int N, int K, bool gated,
+                     hipStream_t stream);
+
 // M <= 64, N % 128 == 0, K % 64 == 0 (rounded weights: K % 128 == 0)
 void launch_gemm_stream(__hip_bfloat16* y, float* part, const __hip_bfloat16* x,
                         const __hip_bfloat16* w, int M, int N, int K, int parts,
                         hipStream_t stream) {
-  launch_q<16, false>(y, part, x, w, nullptr, M, N, K, parts, stream);
+  if (M == 1 && gemm_row_fits(16, K))
+    launch_gemm_row(y, x, w, nullptr, 16, N, K, false, stream);
+  else
+    launch_q<16, false>(y, part, x, w, nullptr, M, N, K, parts, stream);
 }
 
 void launch_gemm_stream_gated(__hip_bfloat16* y, float* part, const __hip_bfloat16* x,
                               const __hip_bfloat16* w13, int M, int I, int K, int parts,
                               hipStream_t stream) {
-  launch_q<16, true>(y, part, x, w13, nullptr, M, I, K, parts, stream);
+  if (M == 1 && gemm_row_fits(16, K))
+    launch_gemm_row(y, x, w13, nullptr, 16, I, K, true, stream);
+  else
+    launch_q<16, true>(y, part, x, w13, nullptr, M, I, K, parts, stream);
 }
 
 void launch_gemm_stream_q(__hip_bfloat16* y, float* part, const __hip_bfloat16* x,
                           const unsigned char* wq, const float* scale, int qbits, int M, int N,
                           int K, int parts, hipStream_t stream) {
-  if (qbits == 8)
+  if (M == 1 && gemm_row_fits(qbits, K))
+    launch_gemm_row(y, x, wq, scale, qbits, N, K, false, stream);
+  else if (qbits == 8)
     launch_q<8, false>(y, part, x, wq, scale, M, N, K, parts, stream);
   else
     launch_q<4, false>(y, part, x, wq, scale, M, N, K, parts, stream);

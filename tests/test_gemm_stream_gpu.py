@@ -113,3 +113,24 @@ def test_widened_weights_are_the_rounded_ones(qbits):
     got = ops.linear_quant(x, wq, scale, qbits)
     want = torch.nn.functional.linear(x, ops.dequantize_weight(wq, scale, qbits))
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize(("n", "k"), [(128, 28672), (128, 28800), (256, 6272), (33024, 2176)])
+def test_one_row(n, k):
+    """Rows as long as are kept in LDS, longer ones, and more rows of W than workgroups."""
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    x, w = _x(1, k, 11), _x(n, k, 12) / k ** 0.5
+    terms = x.double().abs() @ w.double().abs().t()
+    _check(ops.linear(x, w), x.double() @ w.double().t(), terms)
+    g, u = (x.double() @ w.double().t()).chunk(2, dim=1)
+    if n % 256 == 0:
+        _check(ops.gated_mlp_up(x, w), torch.nn.functional.silu(g) * u,
+               30 * (1 + g.abs()) * (1 + u.abs()))
+    wq, scale = ops.quantize_weight(w, 4)
+    exact = ops.dequantize_weight(wq, scale, 4, torch.float32).double()
+    # sums of 8 + n/2 in place of n - 8 (see test_rounded)
+    size = x.double().abs().sum(1, keepdim=True) * exact.abs().amax(1)
+    _check(ops.linear_quant(x, wq, scale, 4), x.double() @ exact.t(),
+           5 * (x.double().abs() @ exact.abs().t() + size))
