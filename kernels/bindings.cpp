@@ -185,6 +185,7 @@ void silu_and_mul(torch::Tensor out, torch::Tensor x) {
 // Elements between the starts of a [rows, ...] tensor's rows, whose own elements
 // are dense.
 int64_t row_stride(const torch::Tensor& t, const char* name) {
+  if (t.is_contiguous() && t.size(0) > 0) return t.numel() / t.size(0);
   int64_t want = 1;
   for (int64_t d = t.dim() - 1; d > 0; --d) {
     TORCH_CHECK(t.size(d) == 1 || t.stride(d) == want, name, ": rows must be dense");
@@ -222,7 +223,7 @@ void reshape_and_cache(torch::Tensor k, torch::Tensor v, torch::Tensor k_cache,
   const int64_t wide = 16 / k.element_size();
   auto lined_up = [&](const torch::Tensor& t) {
     return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 &&
-           (t.size(0) <= 1 || t.stride(0) % wide == 0);
+           (t.is_contiguous() || t.size(0) <= 1 || t.stride(0) % wide == 0);
   };
   if (!lined_up(k)) k = k.contiguous();
   if (!lined_up(v)) v = v.contiguous();
