@@ -61,6 +61,9 @@ void launch_reshape_and_cache_fp8(const __hip_bfloat16*,
                                   unsigned char*, const long*, int, int, long,
                                   long, hipStream_t);
 int gemm_stream_parts(int qbits, int M, int N, int K, bool gated);
+void launch_rotary_cache(const long*, __hip_bfloat16*, const __hip_bfloat16*,
+                         const __hip_bfloat16*, const __hip_bfloat16*, const float*, void*, void*,
+                         const long*, int, int, int, int, long, long, long, bool, hipStream_t);
 int gemm_block_parts(int M, int N, int K);
 void launch_gemm_block(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hip_bfloat16*, int,
                        int, int, int, hipStream_t);
@@ -246,6 +249,36 @@ void reshape_and_cache(torch::Tensor k, torch::Tensor v, torch::Tensor k_cache,
         ptr<scalar_t>(v_cache), slot_mapping.data_ptr<long>(), tokens,
         row_elems, ks, vs, current_stream());
   });
+}
+
+// q turned into q_out, k turned and v into the cache, in one launch (bf16)
+void rotary_cache(torch::Tensor positions, torch::Tensor q_out, torch::Tensor q, torch::Tensor k,
+                  torch::Tensor v, int64_t head_dim, torch::Tensor cos_sin_cache,
+                  torch::Tensor k_cache, torch::Tensor v_cache, torch::Tensor slot_mapping) {
+  const int64_t tokens = positions.size(0), nq = q.size(-1) / head_dim, nk = k.size(-1) / head_dim;
+  for (const auto& t : {q_out, q, k, v})
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::ScalarType::BFloat16 && t.dim() == 2 &&
+                t.size(0) == tokens && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0);
+  TORCH_CHECK(head_dim % 16 == 0 && nq * head_dim == q.size(1) && nk * head_dim == k.size(1) &&
+              v.size(1) == k.size(1) && q_out.size(1) == q.size(1) && q_out.is_contiguous());
+  const int64_t qs = row_stride(q, "q"), ks = row_stride(k, "k"), vs = row_stride(v, "v");
+  TORCH_CHECK(qs % 8 == 0 && ks % 8 == 0 && vs % 8 == 0, "rows start at 16 bytes");
+  TORCH_CHECK(positions.scalar_type() == at::ScalarType::Long && positions.is_contiguous() &&
+              slot_mapping.scalar_type() == at::ScalarType::Long && slot_mapping.is_contiguous() &&
+              slot_mapping.numel() >= tokens);
+  TORCH_CHECK(cos_sin_cache.scalar_type() == at::ScalarType::Float &&
+              cos_sin_cache.is_contiguous() && cos_sin_cache.size(-1) == head_dim);
+  const bool fp8 = k_cache.scalar_type() == at::ScalarType::Byte;
+  TORCH_CHECK(k_cache.scalar_type() == v_cache.scalar_type() &&
+              (fp8 || k_cache.scalar_type() == at::ScalarType::BFloat16));
+  TORCH_CHECK(k_cache.is_contiguous() && v_cache.is_contiguous() && k_cache.size(2) == nk &&
+              k_cache.size(3) == head_dim);
+  if (tokens == 0) return;
+  launch_rotary_cache(positions.data_ptr<long>(), ptr<__hip_bfloat16>(q_out),
+                      cptr<__hip_bfloat16>(q), cptr<__hip_bfloat16>(k), cptr<__hip_bfloat16>(v),
+                      cos_sin_cache.data_ptr<float>(), k_cache.data_ptr(), v_cache.data_ptr(),
+                      slot_mapping.data_ptr<long>(), (int)tokens, (int)nq, (int)nk, (int)head_dim,
+                      qs, ks, vs, fp8, current_stream());
 }
 
 // ---- direct-xGMI all-reduce plumbing (E15) --------------------------------
@@ -682,6 +715,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "fused log-softmax + top-K + sampled-token rank (one HBM pass)");
   m.def("sample_argmax", &sample_argmax,
         "fused temperature/gumbel-race sampling + greedy argmax (CDNA4)");
+  m.def("rotary_cache", &rotary_cache, "rotation of q and k with the cache write");
   m.def("gemm_block", &gemm_block, "product of more than 64 rows, large tiles");
   m.def("lora_delta", &lora_delta,
         "bf16 multi-LoRA of up to three projections of one input");

@@ -71,14 +71,10 @@ class Attention(nn.Module):
     ) -> torch.Tensor:
         qkv = self.qkv_proj(hidden, lora=self._qkv_lora)
         q, k, v = qkv.split([self.q_local, self.kv_local, self.kv_local], dim=-1)
-        q, k = ops.rotary_embedding(positions, q, k, self.head_dim, cos_sin_cache)
-        t = hidden.shape[0]
-        q = q.view(t, self.num_heads, self.head_dim)
-        k = k.view(t, self.num_kv_heads, self.head_dim)
-        v = v.view(t, self.num_kv_heads, self.head_dim)
-
         k_cache, v_cache = kv_cache
-        ops.reshape_and_cache(k, v, k_cache, v_cache, meta.slot_mapping)
+        q = ops.rotary_and_cache(positions, q, k, v, self.head_dim, cos_sin_cache,
+                                 k_cache, v_cache, meta.slot_mapping)
+        q = q.view(hidden.shape[0], self.num_heads, self.head_dim)
 
         out = torch.empty_like(q)
         npt = meta.num_prefill_tokens
@@ -95,7 +91,7 @@ class Attention(nn.Module):
                 meta.decode_block_tables, meta.decode_seq_lens,
                 self.scale, meta.max_decode_seq_len, out=out[npt:],
             )
-        return self.o_proj(out.view(t, -1), lora=self._o_lora)
+        return self.o_proj(out.view(hidden.shape[0], -1), lora=self._o_lora)
 
 
 class LlamaMLP(nn.Module):

@@ -131,6 +131,34 @@ def reshape_and_cache(
     reference.reshape_and_cache(k, v, k_cache, v_cache, slot_mapping)
 
 
+def rotary_and_cache(
+    positions: torch.Tensor,
+    q: torch.Tensor,             # [T, num_heads * head_dim]
+    k: torch.Tensor,             # [T, num_kv_heads * head_dim]
+    v: torch.Tensor,
+    head_dim: int,
+    cos_sin_cache: torch.Tensor,
+    k_cache: torch.Tensor,
+    v_cache: torch.Tensor,
+    slot_mapping: torch.Tensor,
+) -> torch.Tensor:
+    """rotary_embedding of q and k, and reshape_and_cache of the turned k and of v; returns
+    q turned.  One launch for bf16 rows that start at 16 bytes (k is then left as it is)."""
+    if (_native(q) and q.dtype == torch.bfloat16 and head_dim % 16 == 0
+            and k_cache.dtype in (torch.bfloat16, torch.uint8)
+            and cos_sin_cache.dtype == torch.float32
+            and all(t.data_ptr() % 16 == 0 and t.stride(0) % 8 == 0 and t.stride(1) == 1
+                    for t in (q, k, v))):
+        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+        _C.rotary_cache(positions, out, q, k, v, head_dim, cos_sin_cache, k_cache, v_cache,
+                        slot_mapping)
+        return out
+    q, k = rotary_embedding(positions, q, k, head_dim, cos_sin_cache)
+    shape = (k.shape[0], k.shape[1] // head_dim, head_dim)
+    reshape_and_cache(k.view(shape), v.view(shape), k_cache, v_cache, slot_mapping)
+    return q
+
+
 def paged_attention_decode(
     q: torch.Tensor,            # [N, num_heads, head_dim] — one token per seq
     k_cache: torch.Tensor,
