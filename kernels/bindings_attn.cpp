@@ -113,6 +113,18 @@ const T* cptr(const torch::Tensor& t) {
       TORCH_CHECK(false, "unsupported dtype");                           \
   }
 
+// The prompt kernels on the matrix cores follow the largest unscaled score, give hidden keys
+// the lowest float and fold the scale into the exponent: right for a scale that is positive
+// and not so small that it lifts that mark into range.  Of other scales the queries take the
+// sign (exact), a power of two that the smallest of them lack, or the zero.
+void positive_scale(torch::Tensor& q, double& scale) {
+  if (!(scale < 0x1p-100)) return;   // (NaN stays as it is)
+  double turn = scale < 0 ? -1.0 : scale > 0 ? 1.0 : 0.0;
+  if (scale > -0x1p-100) turn *= 0x1p-64;
+  q = q * turn;
+  scale = turn == 0.0 ? 1.0 : scale / turn;
+}
+
 void paged_attention_decode(torch::Tensor out, torch::Tensor q,
                             torch::Tensor k_cache, torch::Tensor v_cache,
                             torch::Tensor block_tables, torch::Tensor seq_lens,
@@ -200,6 +212,7 @@ void paged_attention_prefill(torch::Tensor out, torch::Tensor q,
   const bool tiles = q.scalar_type() == at::ScalarType::BFloat16 &&
                      (head_dim == 128 || (head_dim == 64 &&
                                           k_cache.scalar_type() == at::ScalarType::BFloat16));
+  if (tiles) positive_scale(q, scale);
   // the longest sequence only decides how the work is cut
   const int max_keys = (int)std::min<int64_t>(max_seq_len, (int64_t)max_blocks * block_size);
   const int64_t parts =
@@ -291,6 +304,7 @@ void windowed_attention_prefill(torch::Tensor out, torch::Tensor q,
               query_start_loc.scalar_type() == at::ScalarType::Int &&
               query_start_loc.numel() == nseq + 1 && max_query_len >= 1);
   if (q.size(0) == 0 || nseq == 0) return;
+  positive_scale(q, scale);
   launch_paged_prefill_mfma_v2_ws(
       reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
       reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()),
@@ -375,6 +389,7 @@ void capped_attention_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor 
               query_start_loc.scalar_type() == at::ScalarType::Int &&
               query_start_loc.numel() == nseq + 1 && max_query_len >= 1);
   if (q.size(0) == 0 || nseq == 0) return;
+  positive_scale(q, scale);
   launch_paged_prefill_mfma_v2_capped(
       reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
       reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()),
@@ -457,6 +472,7 @@ void chunk_attention_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor k
               query_start_loc.scalar_type() == at::ScalarType::Int &&
               query_start_loc.numel() == nseq + 1 && max_query_len >= 1);
   if (q.size(0) == 0 || nseq == 0) return;
+  positive_scale(q, scale);
   launch_paged_prefill_mfma_v2_chunk(
       out.data_ptr<float>(), reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()),
       reinterpret_cast<const __hip_bfloat16*>(k_cache.data_ptr()),
@@ -549,6 +565,7 @@ void span_attention_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor k_
               query_start_loc.scalar_type() == at::ScalarType::Int &&
               query_start_loc.numel() == nseq + 1 && max_query_len >= 1);
   if (q.size(0) == 0 || nseq == 0) return;
+  positive_scale(q, scale);
   launch_paged_prefill_mfma_v2_span(
       reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
       reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()),

@@ -77,3 +77,75 @@ def test_prefill(shape, heads, kv_heads, dim, dtype, block):
         # unit in the last of 8 bits: by 2**-8 of the value just above a power of two
         err = (got[rows].double() - want).abs()
         assert (err <= 1.01 * 2 ** -7 * terms + 1e-6).all(), (i, err.max().item())
+
+
+def _paged(lens, kv_heads, dim, gen, block=16, fp8=False, unowned=None):
+    """Caches and tables of sequences of these lengths; unowned: what the rows hold that
+    no sequence has."""
+    need = [-(-n // block) for n in lens]
+    ids = torch.randperm(sum(need) + 1, generator=torch.Generator().manual_seed(7)).tolist()
+    tables, at = torch.zeros((len(lens), max(need)), dtype=torch.int32), 0
+    own = torch.zeros((sum(need) + 1, block), dtype=torch.bool)
+    for i, n in enumerate(lens):
+        tables[i, :need[i]] = torch.tensor(ids[at:at + need[i]])
+        own[tables[i, :need[i]].long()] = torch.arange(need[i] * block).view(-1, block) < n
+        at += need[i]
+    cache = [torch.randn((len(own), block, kv_heads, dim), generator=gen, device="cuda")
+             for _ in "kv"]
+    cache = [c.to(torch.float8_e4m3fn) if fp8 else c.bfloat16() for c in cache]
+    if unowned is not None:
+        for c in cache:
+            c.view(torch.uint8 if fp8 else torch.bfloat16)[~own.cuda()] = unowned
+    return cache, tables
+
+
+def _ints(v):
+    return torch.tensor(v, dtype=torch.int32, device="cuda")
+
+
+def _close(got, want, terms):
+    """Probabilities and the result are rounded to bf16 once each (see above)."""
+    err = (got.cpu().double() - want.double()).abs()
+    assert (err <= 1.01 * 2 ** -7 * terms.double() + 1e-6).all(), err.max().item()
+
+
+@pytest.mark.parametrize("scale", [-0.11, 0.0, -0.0, 1e-38, -1e-42])
+@pytest.mark.parametrize(("kind", "dim"), [
+    ("plain", 64), ("plain", 128), ("fp8", 128), ("windowed", 128), ("capped", 64),
+    ("capped", 128), ("chunk", 128)])
+def test_scale_of_any_sign(kind, dim, scale):
+    """A row sees its own keys only, whatever the scale's sign."""
+    _need()
+    from vllm_tgis_adapter_amd import ops
+    from vllm_tgis_adapter_amd.ops import reference as R
+
+    gen = torch.Generator("cuda").manual_seed(dim)
+    new, lens, heads, kv_heads = [70, 129], [135, 129], 8, 2
+    (kc, vc), tables = _paged(lens, kv_heads, dim, gen, fp8=kind == "fp8")
+    q = torch.randn((sum(new), heads, dim), generator=gen, device="cuda").bfloat16()
+    start = [0, 70, 199]
+    where = (tables.cuda(), _ints(start), _ints(lens))
+    sinks = torch.linspace(-1, 1, heads)
+    out = torch.full_like(q, float("nan"), dtype=torch.float32 if kind == "chunk" else None)
+    if kind in ("plain", "fp8"):
+        kb, vb = (c.view(torch.uint8) if kind == "fp8" else c for c in (kc, vc))
+        out = ops.paged_attention_prefill(q, kb, vb, *where, scale, max(new), max(lens))
+    elif kind == "windowed":
+        ops.gqa_attention_prefill(q, kc, vc, *where, scale, max(new), out, window=40, sink=0.3)
+    elif kind == "capped":
+        ops.gqa_attention_prefill(q, kc, vc, *where, scale, max(new), out, window=40,
+                                  sinks=sinks.cuda(), softcap=2.0)
+    else:
+        ops.chunk_attention_prefill(q, kc, vc, *where, scale, max(new), 48, out)
+
+    def plain(v):
+        args = (q.float().cpu(), kc.float().cpu(), v, tables, torch.tensor(start),
+                torch.tensor(lens), scale)
+        if kind == "chunk":
+            return R.chunk_attention(*args, 48)
+        if kind == "windowed":
+            return R.paged_attention(*args, 40, 0.3)
+        return R.paged_attention(*args, 40, sinks, 2.0) if kind == "capped" \
+            else R.paged_attention(*args)
+
+    _close(out, plain(vc.float().cpu()), plain(vc.float().abs().cpu()))
