@@ -142,6 +142,7 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
     const char* e = getenv("VTA_DECODE_VALU");
     return e && e[0] == '1';
   }();
+  TORCH_CHECK(out.is_contiguous() && out.numel() >= q.numel(), "out: dense rows, as many as q");
   if (nseq == 0) return;
   if (!q.is_contiguous()) q = q.contiguous();   // the kernels read dense rows
   auto stream_decode = [&](bool fp8) {
@@ -203,6 +204,7 @@ void paged_attention_prefill(torch::Tensor out, torch::Tensor q,
   const int kvh = k_cache.size(2);
   const int block_size = k_cache.size(1);
   const int max_blocks = block_tables.size(1);
+  TORCH_CHECK(out.is_contiguous() && out.numel() >= q.numel(), "out: dense rows, as many as q");
   if (nseq == 0 || max_query_len <= 0) return;
   if (!q.is_contiguous()) q = q.contiguous();   // the kernels read dense rows
   static const bool force_valu = [] {

@@ -149,3 +149,71 @@ def test_scale_of_any_sign(kind, dim, scale):
             else R.paged_attention(*args)
 
     _close(out, plain(vc.float().cpu()), plain(vc.float().abs().cpu()))
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("step", ["prompt", "decode", "decode into"])
+def test_queries_and_results_in_any_order(step, dim):
+    """Heads ahead of rows in memory: queries are read, and results written, by their
+    strides."""
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    gen = torch.Generator("cuda").manual_seed(dim)
+    lens = [33, 100, 7]
+    (kc, vc), tables = _paged(lens, 2, dim, gen)
+    new = [20, 100, 1] if step == "prompt" else [1] * 3
+    q = torch.randn((sum(new), 8, dim), generator=gen, device="cuda").bfloat16()
+    turned = q.transpose(0, 1).contiguous().transpose(0, 1)
+    start = _ints([sum(new[:i]) for i in range(len(new) + 1)])
+
+    def run(q, **kw):
+        if step == "prompt":
+            return ops.paged_attention_prefill(q, kc, vc, tables.cuda(), start, _ints(lens), 0.1,
+                                               max(new), max(lens))
+        return ops.paged_attention_decode(q, kc, vc, tables.cuda(), _ints(lens), 0.1, max(lens),
+                                          **kw)
+
+    want = run(q)
+    if step == "decode into":
+        out = torch.full_like(turned, float("nan"))
+        assert not out.is_contiguous() and run(q, out=out) is out
+        assert torch.equal(out, want)
+    else:
+        assert torch.equal(run(turned), want)
+        out = torch.full_like(turned, float("nan"))
+        if step == "prompt":
+            ops.gqa_attention_prefill(turned, kc, vc, tables.cuda(), start, _ints(lens), 0.1,
+                                      max(new), out)
+        else:
+            ops.gqa_attention_decode(turned, kc, vc, tables.cuda(), _ints(lens), 0.1, out)
+        assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize(("dim", "fp8"), [(64, False), (128, False), (128, True)])
+@pytest.mark.parametrize("step", ["prompt", "decode"])
+def test_rows_that_no_sequence_owns(step, dim, fp8):
+    """Free blocks, the rest of a last block and rows past the longest prompt's hold NaN."""
+    _need()
+    from vllm_tgis_adapter_amd import ops
+    from vllm_tgis_adapter_amd.ops import reference as R
+
+    gen = torch.Generator("cuda").manual_seed(dim)
+    lens = [1, 17, 200, 65]
+    new = [1, 3, 130, 65] if step == "prompt" else [1] * 4
+    (kc, vc), tables = _paged(lens, 2, dim, gen, fp8=fp8, unowned=0x7f if fp8 else float("nan"))
+    q = torch.randn((sum(new), 8, dim), generator=gen, device="cuda").bfloat16()
+    start = [sum(new[:i]) for i in range(len(new) + 1)]
+    kb, vb = (c.view(torch.uint8) if fp8 else c for c in (kc, vc))
+    if step == "prompt":
+        got = ops.paged_attention_prefill(q, kb, vb, tables.cuda(), _ints(start), _ints(lens),
+                                          0.1, max(new), max(lens))
+    else:
+        got = ops.paged_attention_decode(q, kb, vb, tables.cuda(), _ints(lens), 0.1, max(lens))
+
+    def plain(v):
+        return R.paged_attention(q.float().cpu(), kc.float().cpu().nan_to_num(), v, tables,
+                                 torch.tensor(start), torch.tensor(lens), 0.1)
+
+    v = vc.float().cpu().nan_to_num()
+    _close(got, plain(v), plain(v.abs()))

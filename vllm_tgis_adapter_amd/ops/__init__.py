@@ -159,6 +159,11 @@ def rotary_and_cache(
     return q
 
 
+def _dense_like(q: torch.Tensor) -> torch.Tensor:
+    """Room for a result that kernels write as dense rows, whatever q's strides."""
+    return torch.empty_like(q, memory_format=torch.contiguous_format)
+
+
 def paged_attention_decode(
     q: torch.Tensor,            # [N, num_heads, head_dim] — one token per seq
     k_cache: torch.Tensor,
@@ -170,11 +175,14 @@ def paged_attention_decode(
     out: torch.Tensor | None = None,
 ) -> torch.Tensor:
     if _native(q):
-        if out is None:
-            out = torch.empty_like(q)
+        dst = out if out is not None and out.is_contiguous() else _dense_like(q)
         _C.paged_attention_decode(
-            out, q, k_cache, v_cache, block_tables, seq_lens, scale
+            dst, q, k_cache, v_cache, block_tables, seq_lens, scale
         )
+        if out is None:
+            return dst
+        if dst is not out:
+            out.copy_(dst)
         return out
     n = q.shape[0]
     qsl = torch.arange(n + 1, dtype=torch.int32)
@@ -202,7 +210,7 @@ def paged_attention_prefill(
     max_seq_len: int,
 ) -> torch.Tensor:
     if _native(q):
-        out = torch.empty_like(q)
+        out = _dense_like(q)
         _C.paged_attention_prefill(
             out, q, k_cache, v_cache, block_tables, query_start_loc, seq_lens,
             scale, max_query_len, max_seq_len
@@ -997,7 +1005,7 @@ def gqa_attention_prefill(q, k_cache, v_cache, block_tables, query_start_loc,
             return out
         if window > 0 or sink is not None:
             if _windowed_matrix_core_fits(q, k_cache, v_cache, single=False):
-                dst = out if out.is_contiguous() else torch.empty_like(q)
+                dst = out if out.is_contiguous() else _dense_like(q)
                 _attn_ext().windowed_attention_prefill(
                     dst, q, k_cache, v_cache, block_tables, query_start_loc, seq_lens,
                     float(scale), int(max_query_len), int(window), sink is not None,
@@ -1011,7 +1019,7 @@ def gqa_attention_prefill(q, k_cache, v_cache, block_tables, query_start_loc,
                                    sink is not None, float(sink or 0.0))
             return out
         if _matrix_core_attention_fits(q, k_cache, v_cache):
-            dst = out if out.is_contiguous() else torch.empty_like(q)
+            dst = out if out.is_contiguous() else _dense_like(q)
             _attn_ext().paged_attention_prefill(dst, q, k_cache, v_cache, block_tables,
                                        query_start_loc, seq_lens, float(scale),
                                        int(max_query_len),
@@ -1051,7 +1059,7 @@ def gqa_attention_decode(q, k_cache, v_cache, block_tables, seq_lens, scale,
             return out
         if window > 0 or sink is not None:
             if _windowed_matrix_core_fits(q, k_cache, v_cache, single=True):
-                dst = out if out.is_contiguous() else torch.empty_like(q)
+                dst = out if out.is_contiguous() else _dense_like(q)
                 _attn_ext().windowed_attention_decode(
                     dst, q, k_cache, v_cache, block_tables, seq_lens, float(scale),
                     int(window), sink is not None, float(sink or 0.0))
@@ -1067,7 +1075,7 @@ def gqa_attention_decode(q, k_cache, v_cache, block_tables, seq_lens, scale,
                 _attn_ext().paged_attention_decode(out, q, k_cache, v_cache,
                                                    block_tables, seq_lens, float(scale))
             else:
-                tmp = torch.empty_like(q)
+                tmp = _dense_like(q)
                 _attn_ext().paged_attention_decode(tmp, q, k_cache, v_cache,
                                                    block_tables, seq_lens, float(scale))
                 out.copy_(tmp)
