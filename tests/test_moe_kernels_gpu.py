@@ -113,3 +113,54 @@ def test_router_of_equal_and_undefined_scores_names_experts():
     ids, weights = ops.moe_topk(x, gate, 2)
     assert ids.tolist() == [[0, 1]] * 3
     assert weights[0].tolist() == [0.5, 0.5] and weights[1].isnan().all()
+
+
+@pytest.mark.parametrize("layout", ["dense", "slice", "turned", "odd offset", "odd gate"])
+@pytest.mark.parametrize("rows", [1, 33, 700])
+def test_mixture_of_rows_in_any_layout(layout, rows):
+    """The whole block, for rows as callers may have them, against float64."""
+    from vllm_tgis_adapter_amd.engine.config import ModelConfig
+    from vllm_tgis_adapter_amd.models.mixtral import MoEBlock
+
+    mc = ModelConfig(model="m", architecture="mixtral", vocab_size=64, hidden_size=256,
+                     intermediate_size=384, num_layers=1, num_heads=2, num_kv_heads=1,
+                     head_dim=128, max_model_len=64, dtype=torch.bfloat16, num_experts=8,
+                     num_experts_per_tok=2)
+    torch.manual_seed(rows)
+    with torch.device("cuda"):
+        block = MoEBlock(mc)
+    for w in (block.gate, block.w13, block.w2):
+        w.data.normal_(0, 0.06)
+    x = torch.randn((rows, 256), device="cuda").bfloat16()
+    if layout == "slice":
+        given = torch.zeros((rows, 300), dtype=x.dtype, device="cuda")[:, 16:272]
+    elif layout == "turned":
+        given = torch.zeros((256, rows), dtype=x.dtype, device="cuda").t()
+    elif layout == "odd offset":
+        given = torch.zeros(rows * 256 + 1, dtype=x.dtype, device="cuda")[1:].view(rows, 256)
+    else:
+        given = x.clone()
+    if layout == "odd gate":
+        wide = torch.zeros((8, 257), dtype=x.dtype, device="cuda")
+        wide[:, 1:] = block.gate.data
+        block.gate.data = wide[:, 1:]
+    given.copy_(x)
+    with torch.inference_mode():
+        got = block(given)
+    logits = x.double() @ block.gate.double().t()
+    score, pick = logits.topk(2, dim=1)
+    # f32 router sums: only rows whose second and third scores they cannot swap
+    third = logits.topk(3, dim=1).values[:, 2]
+    clear = score[:, 1] - third > 1e-3
+    score = score.softmax(1)
+    want, terms = (torch.zeros((rows, 256), dtype=torch.float64, device="cuda") for _ in "wt")
+    for j in range(2):
+        for e in range(8):
+            at = (pick[:, j] == e).nonzero().view(-1)
+            a, u = (x[at].double() @ block.w13[e].double().t()).chunk(2, dim=1)
+            h = torch.nn.functional.silu(a) * u
+            want[at] += score[at, j, None] * (h @ block.w2[e].double().t())
+            terms[at] += score[at, j, None] * (h.abs() @ block.w2[e].double().abs().t())
+    # roundings to bf16 of h, of an expert's result and of the sum
+    err = (got.double() - want).abs()[clear]
+    assert (err <= 3 * 2 ** -8 * terms[clear] + 1e-4).all(), err.max().item()

@@ -159,6 +159,13 @@ def rotary_and_cache(
     return q
 
 
+def _dense16(t: torch.Tensor) -> torch.Tensor:
+    """t, or a copy, with dense rows from a 16-byte boundary on, as wide loads take them."""
+    if t.is_contiguous() and t.data_ptr() % 16 == 0:
+        return t
+    return t.clone(memory_format=torch.contiguous_format)
+
+
 def _dense_like(q: torch.Tensor) -> torch.Tensor:
     """Room for a result that kernels write as dense rows, whatever q's strides."""
     return torch.empty_like(q, memory_format=torch.contiguous_format)
@@ -499,10 +506,14 @@ def moe_gemm(
         x, rows = x[rows.long()], None
     if x.device.type != "cuda" or _FORCE_REFERENCE:
         return reference.moe_gemm(x, w, seg_off.cpu(), gated, act, limit)
+    if w.data_ptr() % 16:
+        w = w.clone()
     if rows is not None:
         out = torch.empty((rows.shape[0], n), dtype=x.dtype, device=x.device)
-        _C.moe_gemm(out, x, w, seg_off, 1 if gated else (2 if act == "relu2" else 0), rows)
+        _C.moe_gemm(out, _dense16(x), w, seg_off, 1 if gated else (2 if act == "relu2" else 0), rows)
         return out
+    if x.data_ptr() % 16:
+        x = x.clone()
     out = torch.empty((x.shape[0], n), dtype=x.dtype, device=x.device)
     if act == "clamped":
         _native_seq(x)
@@ -542,7 +553,7 @@ def moe_topk(x: torch.Tensor, gate: torch.Tensor, top_k: int):
     t = x.shape[0]
     ids = torch.empty((t, top_k), dtype=torch.int32, device=x.device)
     w = torch.empty((t, top_k), dtype=torch.float32, device=x.device)
-    _C.moe_topk(ids, w, x.contiguous(), gate)
+    _C.moe_topk(ids, w, _dense16(x), _dense16(gate))
     return ids, w
 
 
