@@ -395,6 +395,9 @@ void gemm_q(torch::Tensor y, torch::Tensor x, torch::Tensor wq, torch::Tensor ws
   // rows of a block of W are found by 32 bits
   TORCH_CHECK((int64_t)128 * K < (1LL << 31));
   if (M > 64) {
+    // both reach LDS in 16-byte pieces
+    TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+                reinterpret_cast<uintptr_t>(wq.data_ptr()) % 16 == 0);
     launch_gemm_block_q(ptr<__hip_bfloat16>(y), cptr<__hip_bfloat16>(x), cptr<unsigned char>(wq),
                         wscale.data_ptr<float>(), (int)qbits, M, N, K, current_stream());
     return;
@@ -411,7 +414,8 @@ void widen_weight(torch::Tensor out, torch::Tensor wq, torch::Tensor wscale, int
   const int64_t N = out.size(0), K = out.size(1);
   check_rounded(wq, wscale, qbits, N, K);
   TORCH_CHECK(out.is_cuda() && out.is_contiguous() &&
-              out.scalar_type() == at::ScalarType::BFloat16);
+              out.scalar_type() == at::ScalarType::BFloat16 &&
+              reinterpret_cast<uintptr_t>(wq.data_ptr()) % 16 == 0);
   launch_widen_weight(ptr<__hip_bfloat16>(out), cptr<unsigned char>(wq),
                       wscale.data_ptr<float>(), (int)qbits, N * K, (int)K, current_stream());
 }
@@ -486,6 +490,9 @@ void gemm_block(torch::Tensor y, torch::Tensor x, torch::Tensor w) {
   const int64_t M = x.size(0), K = x.size(1), N = y.size(1);
   TORCH_CHECK(y.size(0) == M && w.size(0) == N && w.size(1) == K);
   TORCH_CHECK(N % 128 == 0 && K % 64 == 0 && M < (1 << 24) && N < (1 << 24) && K < (1 << 23));
+  // both reach LDS in 16-byte pieces
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+              reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0);
   if (M == 0 || N == 0) return;
   if (K == 0) {
     y.zero_();

@@ -53,3 +53,39 @@ def test_rule(m, n, k):
 
     x, w = _inputs(m, n, k)
     _check(ops.linear(x, w), x, w)
+
+
+@pytest.mark.parametrize("which", ["x", "w"])
+def test_any_address(which):
+    """Tensors that start off a 16-byte boundary."""
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    x, w = _inputs(200, 4096, 8192)
+
+    def moved(t):
+        flat = torch.zeros(t.numel() + 1, dtype=t.dtype, device="cuda")
+        return flat[1:].view(t.shape).copy_(t)
+
+    x, w = (moved(x), w) if which == "x" else (x, moved(w))
+    _check(ops.linear(x, w), x, w)
+
+
+@pytest.mark.parametrize("which", ["x", "w"])
+def test_gradient(which):
+    """A differentiated product has its gradient at every number of rows."""
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    x, w = _inputs(200, 4096, 8192)
+    (x if which == "x" else w).requires_grad_()
+    y = ops.linear(x, w)
+    back = torch.ones_like(y)
+    y.backward(back)
+    if which == "x":
+        want = back.float() @ w.float()
+    else:
+        want = back.float().t() @ x.float()
+    got = (x if which == "x" else w).grad.float()
+    # float32 sums, one rounding to bf16
+    assert (got - want).norm() <= 2 ** -8 * want.norm()

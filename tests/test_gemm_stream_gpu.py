@@ -134,3 +134,46 @@ def test_one_row(n, k):
     size = x.double().abs().sum(1, keepdim=True) * exact.abs().amax(1)
     _check(ops.linear_quant(x, wq, scale, 4), x.double() @ exact.t(),
            5 * (x.double().abs() @ exact.abs().t() + size))
+
+
+def _at_odd_offset(t):
+    flat = torch.zeros(t.numel() + 1, dtype=t.dtype, device=t.device)
+    out = flat[1:].view(t.shape)
+    return out.copy_(t)
+
+
+@pytest.mark.parametrize("qbits", [8, 4])
+@pytest.mark.parametrize("which", ["x", "codes"])
+@pytest.mark.parametrize("m", [65, 300, 1200])
+def test_rounded_many_rows_from_any_address(qbits, which, m):
+    """Tensors that start off a 16-byte boundary, in both forms of the product."""
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    x, w = _x(m, 256, 13), _x(256, 256, 14)
+    wq, scale = ops.quantize_weight(w, qbits)
+    want = ops.linear_quant(x, wq, scale, qbits)
+    if which == "x":
+        x = _at_odd_offset(x)
+    else:
+        wq = _at_odd_offset(wq)
+    got = ops.linear_quant(x, wq, scale, qbits)
+    exact = x.double() @ ops.dequantize_weight(wq, scale, qbits, torch.float32).double().t()
+    terms = x.double().abs() @ ops.dequantize_weight(wq, scale, qbits, torch.float32).double(
+        ).abs().t()
+    # weights are rounded to bf16 on some of the ways
+    for y in (want, got):
+        assert ((y.double() - exact).abs() <= 2 ** -8 * exact.abs() + 2 ** -9 * terms).all()
+
+
+@pytest.mark.parametrize("qbits", [8, 4])
+def test_rounded_many_rows_keep_the_gradient(qbits):
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    x = _x(100, 256, 17).requires_grad_()
+    wq, scale = ops.quantize_weight(_x(256, 256, 18), qbits)
+    back = _x(100, 256, 19)
+    ops.linear_quant(x, wq, scale, qbits).backward(back)
+    want = back @ ops.dequantize_weight(wq, scale, qbits)
+    assert torch.equal(x.grad, want)

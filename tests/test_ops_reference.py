@@ -137,3 +137,33 @@ def test_topk_softmax():
     w, ids = R.topk_softmax(logits, 2)
     assert ids[0].tolist() == [1, 2]
     assert abs(w.sum().item() - 1.0) < 1e-6
+
+
+def test_calls_that_stay_with_the_library():
+    """Products that are differentiated, mapped, traced or off a 16-byte boundary."""
+    from torch.autograd import forward_ad
+
+    from vllm_tgis_adapter_amd import ops
+
+    seen = []
+
+    def look(x):
+        seen.append(ops._plain_tensors(x))
+        return x * 1
+
+    x = torch.randn(2, 8)
+    look(x)
+    look(torch.nn.Parameter(x, requires_grad=False))
+    assert seen == [True, True]
+    seen.clear()
+    look(x.clone().requires_grad_())
+    torch.func.vmap(look)(x)
+    torch.func.jvp(look, (x,), (x,))
+    torch.func.grad(lambda t: look(t).sum())(x)
+    with forward_ad.dual_level():
+        look(forward_ad.make_dual(x, x))
+    torch.jit.trace(look, x, check_trace=False)
+    look(torch.randn(17)[1:])
+    assert len(seen) == 7 and not any(seen)
+    with torch.no_grad():
+        assert ops._plain_tensors(x.clone().requires_grad_())

@@ -13,6 +13,7 @@ from __future__ import annotations
 import os
 
 import torch
+from torch.autograd import forward_ad
 
 from . import reference
 
@@ -267,13 +268,27 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
             )
             _C.gemm_tile(out, x, weight)
             return out
-        if m > max_m and m in _block_rows(weight.shape[0], x.shape[1]):
+        if (m > max_m and m in _block_rows(weight.shape[0], x.shape[1])
+                and _plain_tensors(x, weight)):
             out = torch.empty(
                 (m, weight.shape[0]), dtype=x.dtype, device=x.device
             )
             _C.gemm_block(out, x, weight)
             return out
     return torch.nn.functional.linear(x, weight, bias)
+
+
+def _plain_tensors(*tensors: torch.Tensor) -> bool:
+    """Whether a kernel here may stand in for a library product: tensors with memory of
+    their own, from a 16-byte boundary on (it is loaded into LDS in such pieces), and
+    nothing that would differentiate, map or trace the call."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return False
+    if (forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None
+            or torch._C._functorch.peek_interpreter_stack() is not None):
+        return False
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.data_ptr() % 16 == 0
+               for t in tensors)
 
 
 def _block_rows(n: int, k: int) -> range:
@@ -359,12 +374,13 @@ def linear_quant(x: torch.Tensor, wq: torch.Tensor, scales: torch.Tensor,
     k = x2.shape[1]
     if _native(x) and x.dtype == torch.bfloat16 and n % 128 == 0 and k % 128 == 0:
         if (bias is None and 1 <= m <= _quant_rows(qbits, n, k) and x2.is_contiguous()
-                and wq.is_contiguous() and scales.is_contiguous()):
+                and wq.is_contiguous() and scales.is_contiguous()
+                and (m <= 64 or _plain_tensors(x2, wq))):
             out = torch.empty((m, n), dtype=x.dtype, device=x.device)
             _C.gemm_q(out, x2, wq, scales, qbits)
             return out.view(*x.shape[:-1], n)
         w = torch.empty((n, k), dtype=x.dtype, device=x.device)
-        _C.widen_weight(w, wq.contiguous(), scales.contiguous(), qbits)
+        _C.widen_weight(w, _dense16(wq), scales.contiguous(), qbits)
     else:
         w = dequantize_weight(wq, scales, qbits, x.dtype)
     return torch.nn.functional.linear(x, w, bias)
