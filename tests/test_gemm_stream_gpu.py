@@ -166,6 +166,22 @@ def test_rounded_many_rows_from_any_address(qbits, which, m):
         assert ((y.double() - exact).abs() <= 2 ** -8 * exact.abs() + 2 ** -9 * terms).all()
 
 
+@pytest.mark.parametrize("form", ["unsigned codes", "bf16 scales"])
+def test_rounded_many_rows_of_other_types(form):
+    """What dequantize_weight makes of codes and scales that quantize_weight does not make."""
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    x, w = _x(100, 256, 15), _x(384, 256, 16)
+    wq, scale = ops.quantize_weight(w, 8)
+    if form == "unsigned codes":
+        wq = (wq.to(torch.int16) + 127).to(torch.uint8)
+    else:
+        scale = scale.bfloat16()
+    want = torch.nn.functional.linear(x, ops.dequantize_weight(wq, scale, 8))
+    assert torch.equal(ops.linear_quant(x, wq, scale, 8), want)
+
+
 @pytest.mark.parametrize("qbits", [8, 4])
 def test_rounded_many_rows_keep_the_gradient(qbits):
     _need()

@@ -373,12 +373,18 @@ def linear_quant(x: torch.Tensor, wq: torch.Tensor, scales: torch.Tensor,
     n = wq.shape[0]
     k = x2.shape[1]
     if _native(x) and x.dtype == torch.bfloat16 and n % 128 == 0 and k % 128 == 0:
+        # what quantize_weight makes; dequantize_weight reads other types its own way
+        made = (scales.dtype == torch.float32
+                and wq.dtype == (torch.int8 if qbits == 8 else torch.uint8))
         if (bias is None and 1 <= m <= _quant_rows(qbits, n, k) and x2.is_contiguous()
                 and wq.is_contiguous() and scales.is_contiguous()
-                and (m <= 64 or _plain_tensors(x2, wq))):
+                and (m <= 64 or made and _plain_tensors(x2, wq))):
             out = torch.empty((m, n), dtype=x.dtype, device=x.device)
             _C.gemm_q(out, x2, wq, scales, qbits)
             return out.view(*x.shape[:-1], n)
+    else:
+        made = False
+    if made:
         w = torch.empty((n, k), dtype=x.dtype, device=x.device)
         _C.widen_weight(w, _dense16(wq), scales.contiguous(), qbits)
     else:
