@@ -78,6 +78,7 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(
   unsigned long long taken = 0;
   int chosen[kMaxTop];
   float value[kMaxTop], sum = 0.f;
+  bool undefined = false;   // a NaN anywhere makes every weight one, as in a full softmax
 #pragma unroll
   for (int j = 0; j < kMaxTop; ++j) {
     if (j >= top) break;
@@ -86,6 +87,7 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(
     for (int e = 0; e < E; ++e) {
       if (taken >> e & 1) continue;
       const float l = logits[t][e];
+      if (j == 0) undefined |= l != l;
       if (best < 0 || l > v) {
         best = e;
         v = l;
@@ -95,7 +97,7 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(
     chosen[j] = best;
     value[j] = v;
   }
-  const float most = value[0];
+  const float most = undefined ? __builtin_nanf("") : value[0];
 #pragma unroll
   for (int j = 0; j < kMaxTop; ++j) {
     if (j >= top) break;

@@ -164,3 +164,15 @@ def test_mixture_of_rows_in_any_layout(layout, rows):
     # roundings to bf16 of h, of an expert's result and of the sum
     err = (got.double() - want).abs()[clear]
     assert (err <= 3 * 2 ** -8 * terms[clear] + 1e-4).all(), err.max().item()
+
+
+def test_router_keeps_an_undefined_score():
+    """One expert's score is NaN: so is every weight, as a softmax over all experts says."""
+    from vllm_tgis_adapter_amd import ops
+
+    g = torch.Generator("cuda").manual_seed(0)
+    x = torch.randn((5, 64), generator=g, device="cuda").bfloat16()
+    gate = torch.randn((8, 64), generator=g, device="cuda").bfloat16()
+    gate[3, 10] = float("nan")
+    ids, weights = ops.moe_topk(x, gate, 2)
+    assert weights.isnan().all() and ((ids >= 0) & (ids < 8)).all()
