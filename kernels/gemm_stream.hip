@@ -26,7 +26,7 @@
 // merge where there is one:
 //   23 rows, 14336 x 4096 gated 55.2 -> 43.4; the mean of 6144 x 4096, 4096 x 4096 and
 //     4096 x 14336 23.9 -> 17.5 (a llama-3-8b layer reads W at 4.5 TB/s);
-//   61 rows, the mean of these three and 28672 x 4096: 38.1 -> 30;
+//   61 rows, the mean of these three and 28672 x 4096: 38.1 -> 30.
 
 #include "gemm_stream.h"
 
@@ -70,27 +70,39 @@ void launch_gemm_merge(__hip_bfloat16* y, const float* part, long plane, int par
 namespace {
 
 // How a product is cut (waves along N x waves along K, workgroups along K).  The lines
-// are where they measured fastest (us; bf16 unless said; N x K):
+// are where they measured fastest (us from cold weights; bf16 unless said; N x K):
 //   up to 16 rows of x, x is a small part of what is read and waves work alone:
-//     4096 x 4096: 1x8 8.1, 1x4 9.5; 14336 x 4096 gated: 1x4 39.8, 1x8 42.0.
-//   17..32, plain: 4096 x 4096: 1x8 11.2, 4x2 over 4 12.1; 4096 x 14336: 27.4, 25.4;
-//     8192 x 8192: 4x2 over 2 30.4, 2x4 31.4; 28672 x 4096 int8: 4x2 27.3, 4x1 30.9.
-//     gated: 14336 x 4096: 2x2 43.4, 1x4 45.5, 4x1 47.5; 28672 x 8192: 4x1 158, 2x2 171.
-//   33..64, every wave's own copy of x would cost more than W: 4096 x 14336: 4x2 over 4
-//     34.9, 1x8 43.5; 2048 x 2048: 1x8 9.4, 4x2 10.3; 28672 x 4096: int8 4x2 42, 8x1 over
-//     2 45, 4 bits 8x1 over 2 41, 4x2 47 (more of x is turned per weight);
-//     8192 x 28672: 4x2 over 4 93, over 2 109.  gated: 14336 x 4096: 2x2 48.4, 4x2 49.7;
-//     28672 x 8192: 4x1 158, 2x2 189; 8192 x 2048: 2x4 18.0, 2x2 21.5.
+//     4096 x 4096: 1x8 8.1, 1x4 9.5; 6144 x 4096: 1x4 13.2, 1x8 13.9; 5120 x 8192: 22.0,
+//     25.0; 14336 x 4096 gated: 39.8, 42.0.
+//   25 rows, plain: 4096 x 4096: 1x8 11.8, 4x2 over 4 12.4; 4096 x 14336: 28.6, 25.8;
+//     8192 x 8192: 4x2 over 2 29.7, 1x8 34.6; 28672 x 4096 int8: 4x2 27.4, 4x1 31.0.
+//   49 rows, every wave's own copy of x would cost more than W: 4096 x 14336: 4x2 over 8
+//     32.6, 1x8 39.8; 2048 x 2048: 1x8 8.8, 4x2 over 4 9.9; 4 bits, where more of x is
+//     turned per weight: 28672 x 4096: 8x1 over 2 44.3, 4x2 60; 8192 x 8192: 8x1 over 8
+//     30.1, 4x2 over 2 35.9.
+//   gated, 25 | 49 rows, by how many columns there are to share out (a whole layer's to an
+//   eighth of one's):
+//     28672 x 8192: 4x1 156 | 157, 2x2 173 | 191; 14336 x 8192: 2x2 79 | 91, 4x1 89 | 119;
+//     14336 x 4096: 2x2 42.6 | 47.8, 4x1 47.7 | 62;
+//     7168 x 4096: 1x4 26.0 | 30.8, 2x4 27.1 | 28.6, 2x2 28.5 | 35.0; 8064 x 8192: 1x4 47.9
+//     | 57.6, 2x4 54.9 | 57.7, 2x2 54 | 68; 5120 x 4096: 2x4 22.8 | 25.9, 1x4 24.2 | 28.9;
+//     3584 x 8192: 1x8 27.2 | 31.2, 2x4 37 | 45, 4x1 68 | 104; 2048 x 2048: 9.4 | 12.1,
+//     2x4 12.3 | 14.5;
+//     1280 x 8192: 2x4 over 6 16.7 | 18.4, 1x8 21.2 | 27.2; 1792 x 4096: over 4 13.5 | 15.1,
+//     14.1 | 17.3; 64 rows, 2560 x 8192: over 3 26.8, 1x8 32.1; 4096 x 14336: over 2 53, 62.
 enum class Cut { kWave8, kWave4, kShare22, kShare24, kShare41, kShare42, kShare81 };
 
 Cut cut_of(int qbits, int M, int N, int K, bool gated) {
-  if (M <= 16) return N / 16 < 512 ? Cut::kWave8 : Cut::kWave4;
+  if (M <= 16) return N / 16 <= 256 ? Cut::kWave8 : Cut::kWave4;
   if (gated) {
-    if (K >= 8192) return Cut::kShare41;
-    return K < 4096 && M > 32 ? Cut::kShare24 : Cut::kShare22;
+    if (N >= 20480 && K >= 8192) return Cut::kShare41;
+    if (N >= 12288) return Cut::kShare22;
+    if (N > 4096) return M <= 32 && N >= 6144 ? Cut::kWave4 : Cut::kShare24;
+    return (N <= 2048 ? K >= 4096 : M > 32 && K >= 3 * N) ? Cut::kShare24 : Cut::kWave8;
   }
   if ((long)N * K <= 1L << (M <= 32 ? 24 : 23)) return Cut::kWave8;
-  if (qbits == 4 && M > 32 && N >= 16384 && K >= 4096) return Cut::kShare81;
+  if (qbits == 4 && M > 32 && (N >= 16384 ? K >= 4096 : N >= 8192 && K >= 8192))
+    return Cut::kShare81;
   return Cut::kShare42;
 }
 
@@ -115,6 +127,8 @@ void launch_mt(__hip_bfloat16* y, float* part, const __hip_bfloat16* x, const vo
   } else if constexpr (GATED) {
     if (cut == Cut::kShare41) run(launch_cut<QB, MT, GATED, 4, 1>);
     else if (cut == Cut::kShare24) run(launch_cut<QB, MT, GATED, 2, 4>);
+    else if (cut == Cut::kWave8) run(launch_cut<QB, MT, GATED, 1, 8>);
+    else if (cut == Cut::kWave4) run(launch_cut<QB, MT, GATED, 1, 4>);
     else run(launch_cut<QB, MT, GATED, 2, 2>);
   } else if (cut == Cut::kWave8) {
     run(launch_cut<QB, MT, GATED, 1, 8>);
@@ -139,18 +153,32 @@ void launch_q(__hip_bfloat16* y, float* part, const __hip_bfloat16* x, const voi
 
 }  // namespace
 
-// Workgroups that K is cut over besides the waves (each leaves a part of the result):
-// as many as make one a CU, two where K is long and the columns are many.  A function of
-// shapes.
+// Workgroups that K is cut over besides the waves (each leaves a part of the result), of four
+// tiles of 128 a wave at least: what fills whole rounds of one workgroup a CU best, up to two
+// rounds.  us, 25 | 49 rows, waves 4x2 over 2, 3, 4 workgroups: 6144 x 4096 (96 columns of
+// workgroups) 15.4 18.7 17.1 | 20.3 20.4 19.3; 7168 x 8192 (112) 26.7 30.4 27.7 | 34.6 34.0
+// 30.5; 10240 x 4096 (160) 24.3 21.3 22.5 | 27.2 23.3 29.1; 16384 x 2048 (256), over 1 and 2,
+// 15.7 18.7 | 18.9 22.0.  Two rounds rather than one as full go with more rows of x, in 4 bits
+// with fewer (8192 x 8192 over 2, 4: 28.5 22.7 | 35.9 37.7).  A function of shapes.
 int gemm_stream_parts(int qbits, int M, int N, int K, bool gated) {
   const Cut cut = cut_of(qbits, M, N, K, gated);
-  if (gated || (cut != Cut::kShare42 && cut != Cut::kShare81)) return 1;
+  if (gated) {   // columns that are few are cut over as many workgroups as there are CUs
+    const int fill = cut == Cut::kShare24 && N <= 4096 ? 256 / (N / 32) : 1;
+    const int most = K / 1024 < 8 ? K / 1024 : 8;
+    return fill < most ? fill : most > 0 ? most : 1;
+  }
+  if (cut != Cut::kShare42 && cut != Cut::kShare81) return 1;
   const int wgs = N / (cut == Cut::kShare81 ? 128 : 64);
-  const int want = M > 32 && N >= 8192 && K >= 8192 ? 512 : 256;
-  int parts = (want + wgs - 1) / wgs;
-  if (parts > 8) parts = 8;
-  const int most = K / 1024 > 0 ? K / 1024 : 1;   // four tiles of 128 a wave at least
-  return parts < most ? parts : most;
+  const bool two = wgs < 256 && (cut == Cut::kShare81 || (qbits == 4) == (M <= 32));
+  int parts = 1, best = 0;
+  for (int p = 1; p <= 8 && (p == 1 || (p <= K / 1024 && wgs * p <= 512)); ++p) {
+    const int rounds = (wgs * p + 255) / 256, full = wgs * p / rounds;
+    if (full > best || (full == best && two)) {
+      parts = p;
+      best = full;
+    }
+  }
+  return parts;
 }
 
 bool gemm_row_fits(int qbits, int K);

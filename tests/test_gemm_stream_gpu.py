@@ -193,3 +193,37 @@ def test_rounded_many_rows_keep_the_gradient(qbits):
     ops.linear_quant(x, wq, scale, qbits).backward(back)
     want = back @ ops.dequantize_weight(wq, scale, qbits)
     assert torch.equal(x.grad, want)
+
+
+@pytest.mark.parametrize("m", [16, 17, 32, 33, 64])
+# columns on both sides of every line of the cut, K of whole, half and uneven shares
+@pytest.mark.parametrize(("n", "k"), [(128, 4096), (2048, 4160), (2176, 6464), (2176, 6528),
+                                      (1024, 4032), (1280, 8192), (4096, 12288), (4096, 640),
+                                      (4224, 640), (6016, 320), (6144, 320),
+                                      (12160, 192), (12288, 192), (20480, 8192)])
+def test_gated_cuts(m, n, k):
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    x, w = _x(m, k, 20), _x(2 * n, k, 21) / k ** 0.5
+    g, u = (x.double() @ w.double().t()).chunk(2, dim=1)
+    _check(ops.gated_mlp_up(x, w), torch.nn.functional.silu(g) * u,
+           30 * (1 + g.abs()) * (1 + u.abs()))
+
+
+@pytest.mark.parametrize("m", [17, 49])
+# K over 1 to 8 workgroups, of equal and of unequal numbers of tiles
+@pytest.mark.parametrize(("n", "k"), [(6144, 4096), (7168, 4224), (10240, 3200), (5120, 8192),
+                                      (2560, 7040), (16384, 2048), (4096, 8320)])
+def test_parts_of_k(m, n, k):
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    x, w = _x(m, k, 22), _x(n, k, 23)
+    _check(ops.linear(x, w), x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t())
+    if k % 128 == 0:
+        wq, scale = ops.quantize_weight(w, 4)
+        exact = ops.dequantize_weight(wq, scale, 4, torch.float32).double()
+        size = x.double().abs().sum(1, keepdim=True) * exact.abs().amax(1)
+        _check(ops.linear_quant(x, wq, scale, 4), x.double() @ exact.t(),
+               5 * (x.double().abs() @ exact.abs().t() + size))
