@@ -6,7 +6,7 @@
 // K less and leaves most of the chip idle.  us in a captured graph over weights that are
 // not in the caches (library -> here), N x K:
 //   4096 x 14336: 65 rows 48.6 -> 40.8, 128 75 -> 40, 256 63 -> 53, 512 89 -> 85
-//   8192 x 28672: 65 rows 193 -> 103, 128 203 -> 123, 256 317 -> 171, 512 308 -> 302
+//   8192 x 28672: 65 rows 193 -> 103, 128 203 -> 123, 256 317 -> 171
 //   10240 x 8192: 128 rows 59 -> 50, 256 89 -> 67;  8192 x 8192: 48 -> 41, 76 -> 55
 
 #include "block_gemm.h"

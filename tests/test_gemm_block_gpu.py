@@ -44,15 +44,26 @@ def test_tiles(m, n, k):
     _check(y, x, w)
 
 
-@pytest.mark.parametrize(("m", "n", "k"), [
-    (64, 4096, 14336), (65, 4096, 14336), (512, 4096, 14336), (513, 4096, 14336),
-    (256, 8192, 8192), (257, 8192, 8192), (128, 2048, 8192), (129, 2048, 8192)])
-def test_rule(m, n, k):
+# the last row below and the first row of the rule, the last row of it and the first above
+LINES = [(4096, 14336, 65, 640), (8192, 8192, 65, 256), (2048, 8192, 129, 700),
+         (1024, 8192, 257, 700), (2560, 8192, 200, 512), (12288, 8192, 65, 128)]
+
+
+@pytest.mark.parametrize(("m", "n", "k", "own"), [
+    (m, n, k, own) for n, k, lo, hi in LINES
+    for m, own in ((lo - 1, False), (lo, True), (hi, True), (hi + 1, False))] + [
+    (128, 12416, 8192, False), (128, 4096, 8128, False), (512, 57344, 8192, False)])
+def test_rule(m, n, k, own, monkeypatch):
+    """Which product a call gets, and that it is right."""
     _need()
     from vllm_tgis_adapter_amd import ops
 
+    calls, run = [], ops._C.gemm_block
+    monkeypatch.setattr(ops._C, "gemm_block", lambda *a: (calls.append(a), run(*a)))
     x, w = _inputs(m, n, k)
-    _check(ops.linear(x, w), x, w)
+    y = ops.linear(x, w)
+    assert bool(calls) == own
+    _check(y, x, w)
 
 
 @pytest.mark.parametrize("which", ["x", "w"])

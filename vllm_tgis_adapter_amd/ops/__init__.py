@@ -292,16 +292,22 @@ def _plain_tensors(*tensors: torch.Tensor) -> bool:
 
 
 def _block_rows(n: int, k: int) -> range:
-    """Rows of a product past 64 that the tiles with a cut K take from the library:
-    where K is so long that its few tiles leave the chip idle.  us, library | tiles:
-    2048 x 8192 128 rows 21.3 | 23.7, 160 25.8 | 24.4, 700 44 | 38, 1000 49 | 48;
-    8192 x 8192 65 rows 35.1 | 34.5, 256 76 | 55, 301 66 | 71; 4096 x 14336 65 rows
-    48.6 | 40.8, 512 89 | 85, 700 101 | 112; 4096 x 4096 65 rows 16 | 18, 512 29 | 32."""
-    if k < 8192:
+    """Rows of a product past 64 that the tiles with a cut K take from the library: where K
+    is so long, and 128 x 128 tiles so few, that K can be cut over three workgroups and
+    more.  Time over the library's, cold weights, N x K: rows:
+      1024 x 8192: 160 1.13, 257 0.94, 512 1.04, 700 0.86;  2048 x 8192: 128 1.11, 129 0.91,
+      700 0.87;  2560 x 8192: 160 1.00, 200 0.91, 512 0.85, 513 1.16;  4096 x 14336: 65 0.84,
+      128 0.56, 512 0.96, 640 0.83, 700 1.15;  5120 x 8192: 65 1.06, 129 1.03, 256 0.60, 512
+      0.95, 513 1.24;  8192 x 8192: 65 0.99, 144 1.05, 256 0.72, 300 1.10;  8192 x 28672: 65
+      0.54, 256 0.53, 384 1.20;  10240 x 8192: 128 0.85, 256 0.77, 257 1.17;  12288 x 8192:
+      128 0.90, 129 1.08;  14336 x 8192: 65 1.07, 128 1.13;  57344 x 8192: 160 1.32."""
+    if k < 8192 or n > 12288:
         return range(0)
-    if n * k <= 1 << 24:
-        return range(129, 701)
-    return range(65, 257 if k < 12288 else 513)
+    if n < 2048:
+        return range(257, 701)
+    if n < 3072:
+        return range(129, 701) if n < 2560 else range(200, 513)
+    return range(65, min(700, 168 // (n // 128) * 128) + 1)
 
 
 def gemm_tile(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
