@@ -435,10 +435,17 @@ struct Cut {
 // 77; 1000 after 3000 8/1 130, 8/2 87, 8/4 91; 64 after 6000 4/1 157, 4/8 34, 4/16 29, 8/16
 // 33; 4 of 100 after 1000 8/1 41, 4/1 36, 4/2 34; 4 of 50 after 500 (9 tiles) 4/1 21, 4/2 26;
 // one of 300 8/1 17, 4/1 14.5.
-Cut cut_of(int nseq, int nheads, int kvh, int max_query_len, int max_keys) {
+//
+// With few query heads a key head the waves take tokens, and half as many waves go where the
+// longest prompt leaves half of them idle: heads 12/12 of 64 (us, 8 | 4 | 2 waves): 64 prompts
+// of 17 tokens 13.1 | 9.1 | 6.7, 300 of 9 | 29.6 | 18.3.  Idle waves still stage keys: with
+// long contexts all eight are worth it (16/16 heads of 128, 64 tokens after 4000 22.6 | 24.2),
+// two do for a few tiles only (16/8, 100 of 5 after 500 | 55 | 66), and e4m3 keys, which are
+// widened, take more (16/16, 16 of 128 11.5 | 12.6, 8 of 30 | 7.2 | 8.5).
+Cut cut_of(bool fp8, int nseq, int nheads, int kvh, int max_query_len, int max_keys) {
   const int group = nheads / kvh, most = max_keys / (kTile * kMinTiles);
   Cut c{};
-  for (c.waves = 8;; c.waves = 4) {
+  for (c.waves = 8;; c.waves /= 2) {
     c.heads = c.waves;
     while (group % c.heads) c.heads /= 2;
     c.tokens = c.waves / c.heads * 32;
@@ -448,7 +455,10 @@ Cut cut_of(int nseq, int nheads, int kvh, int max_query_len, int max_keys) {
     c.parts = fit < 16 ? (int)fit : 16;
     if (c.parts > most) c.parts = most;
     if (c.parts < 1) c.parts = 1;
-    if (c.waves == 4 || blocks * c.parts > 128) return c;
+    const bool idle = c.tokens > 32 && max_keys <= 8 * kTile &&
+                      max_query_len <= c.tokens / (fp8 ? 8 : 2);
+    const bool least = c.waves == (fp8 || max_keys > 2 * kTile ? 4 : 2);
+    if (least || (!idle && (c.waves == 4 || blocks * c.parts > 128))) return c;
   }
 }
 
@@ -466,7 +476,8 @@ void launch(__hip_bfloat16* out, float* part_acc, float* part_ml, const __hip_bf
                        c.parts, part_acc, part_ml);
   };
   if (c.waves == 8) go(paged_prefill_tile_kernel<HD, CT, 8>);
-  else go(paged_prefill_tile_kernel<HD, CT, 4>);
+  else if (c.waves == 4) go(paged_prefill_tile_kernel<HD, CT, 4>);
+  else go(paged_prefill_tile_kernel<HD, CT, 2>);
   if (c.parts > 1)
     hipLaunchKernelGGL((prefill_tile_merge_kernel<HD>), dim3(max_query_len, nseq, (nheads + 3) / 4),
                        dim3(256), 0, stream, out, part_acc, part_ml, qsl, sl, nheads, c.tokens, c.parts);
@@ -477,8 +488,9 @@ void launch(__hip_bfloat16* out, float* part_acc, float* part_ml, const __hip_bf
 // Workgroups that a prompt's keys may be cut over (a function of shapes only): 1, or the
 // launch needs part_acc [parts, tokens, nheads, head_dim] and part_ml [parts, tokens,
 // nheads, 2].
-int prefill_tile_parts(int nseq, int nheads, int kvh, int max_query_len, int max_keys) {
-  return cut_of(nseq, nheads, kvh, max_query_len, max_keys).parts;
+int prefill_tile_parts(bool fp8, int nseq, int nheads, int kvh, int max_query_len,
+                       int max_keys) {
+  return cut_of(fp8, nseq, nheads, kvh, max_query_len, max_keys).parts;
 }
 
 void launch_paged_prefill_tile(__hip_bfloat16* out, float* part_acc, float* part_ml,
@@ -487,7 +499,7 @@ void launch_paged_prefill_tile(__hip_bfloat16* out, float* part_acc, float* part
                                const int* sl, float scale, int nseq, int nheads, int kvh,
                                int head_dim, int block_size, int max_blocks, int max_query_len,
                                int max_keys, hipStream_t stream) {
-  const Cut c = cut_of(nseq, nheads, kvh, max_query_len, max_keys);
+  const Cut c = cut_of(false, nseq, nheads, kvh, max_query_len, max_keys);
   auto go = [&](auto launch) {
     launch(out, part_acc, part_ml, q, kc, vc, bt, qsl, sl, scale, nseq, nheads, kvh, block_size,
            max_blocks, max_query_len, c, stream);
@@ -505,6 +517,5 @@ void launch_paged_prefill_tile_fp8(__hip_bfloat16* out, float* part_acc, float* 
                                    int max_keys, hipStream_t stream) {
   launch<128, unsigned char>(out, part_acc, part_ml, q, kc, vc, bt, qsl, sl, scale, nseq, nheads,
                              kvh, block_size, max_blocks, max_query_len,
-                             cut_of(nseq, nheads, kvh, max_query_len, max_keys),
-                             stream);
+                             cut_of(true, nseq, nheads, kvh, max_query_len, max_keys), stream);
 }

@@ -217,3 +217,37 @@ def test_rows_that_no_sequence_owns(step, dim, fp8):
 
     v = vc.float().cpu().nan_to_num()
     _close(got, plain(v), plain(v.abs()))
+
+
+@pytest.mark.parametrize(("heads", "kv_heads", "dim", "fp8"), [
+    (4, 4, 64, False), (4, 4, 128, False), (8, 4, 128, False), (4, 4, 128, True),
+    (6, 2, 64, False)])
+# the longest prompt and the keys on both sides of the lines of the waves: 16, 32, 64 and 128
+# rows of 8, 4 and 2 waves, 128 and 512 keys
+@pytest.mark.parametrize(("seqs", "longest", "past"), [
+    (40, 9, 0), (40, 32, 96), (40, 33, 95), (40, 32, 97), (12, 64, 0), (12, 65, 63), (12, 128, 0),
+    (12, 129, 0), (6, 64, 448), (6, 64, 449)])
+def test_waves(heads, kv_heads, dim, fp8, seqs, longest, past):
+    """Many short prompts: workgroups of two, four and eight waves."""
+    _need()
+    from vllm_tgis_adapter_amd import ops
+    from vllm_tgis_adapter_amd.ops import reference as R
+
+    gen = torch.Generator("cuda").manual_seed(longest)
+    new = [1 + (7 * i) % longest for i in range(seqs - 1)] + [longest]
+    lens = [n + past * (i % 2) for i, n in enumerate(new)]
+    lens[-1] = longest + past
+    (kc, vc), tables = _paged(lens, kv_heads, dim, gen, fp8=fp8,
+                              unowned=0x7f if fp8 else float("nan"))
+    q = torch.randn((sum(new), heads, dim), generator=gen, device="cuda").bfloat16()
+    start = [sum(new[:i]) for i in range(seqs + 1)]
+    kb, vb = (c.view(torch.uint8) if fp8 else c for c in (kc, vc))
+    got = ops.paged_attention_prefill(q, kb, vb, tables.cuda(), _ints(start), _ints(lens), 0.1,
+                                      longest, max(lens))
+
+    def plain(v):
+        return R.paged_attention(q.float().cpu(), kc.float().cpu().nan_to_num(), v, tables,
+                                 torch.tensor(start), torch.tensor(lens), 0.1)
+
+    v = vc.float().cpu().nan_to_num()
+    _close(got, plain(v), plain(v.abs()))
