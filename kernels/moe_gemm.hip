@@ -105,13 +105,23 @@ void launch_mode(__hip_bfloat16* y, const __hip_bfloat16* x, const __hip_bfloat1
   //       (<2,2,2> 316, 197);  50: <4,4,2> 323, 173 (128 x 128: 351, 228);
   //   64: 128 x 128 349, 232 (<4,4,2> 480, 332);  125: 128 x 128 449, 299 (256 x 256: 458,
   //       335);  250: 256 x 256 609, 382 (128 x 128: 671, 480);  737: 1258, 726 (1442, 738).
+  //
+  // That is with even loads.  The streaming form's workgroups, a chunk of 64 rows an expert and
+  // two a CU, fill whole rounds at usual widths, and a few experts with more rows start another
+  // round: plain products that are brim-full go to the large tiles earlier, where these fill
+  // the chip or K is short.  16 experts of 4096 out and 3584 between, 128 tokens (mean 32) even |
+  // by rank^-0.6: <4,4,2> 83 | 112, 128 x 128 85 | 85; 2048 and 2048: 33 | 47, 37 | 36; 8 of
+  // 4096 and 3584, 128 x 128 at one workgroup a CU: <4,4,2> 46 | 49, 66 | 66.
   const int mean = T / E;
   // rows of a block are found by 32 bits
   const bool far = (long)N * cols * K * 2 >= 1L << 32 || (long)T * K * 2 >= 1L << 32;
+  const long one = (long)E * (N / 64), last = one % 512;   // streaming workgroups
+  const bool brim = !moe::gated(MODE) && (last == 0 || last > 460) &&
+                    (K <= 2048 || (one >= 1024 && K <= 8192));
   if (mean <= 9 && moe::gated(MODE)) STREAM(1, 1, 4);
   else if (mean <= 9) STREAM(1, 2, 2);
   else if (mean <= 18 && moe::gated(MODE)) STREAM(2, 2, 2);
-  else if (mean <= 52 || far) STREAM(4, 4, 2);
+  else if (far || (mean <= 52 && !brim)) STREAM(4, 4, 2);
   else if (mean < 250 || N * cols % 256 != 0) BLOCK(128, 128, 2, 2, 2);
   else BLOCK(256, 256, 2, 4, 2);
 #undef STREAM

@@ -176,3 +176,29 @@ def test_router_keeps_an_undefined_score():
     gate[3, 10] = float("nan")
     ids, weights = ops.moe_topk(x, gate, 2)
     assert weights.isnan().all() and ((ids >= 0) & (ids < 8)).all()
+
+
+@pytest.mark.parametrize("mode", ["plain", "relu2"])
+# widths that fill whole rounds of streaming workgroups and ones that do not, short and long K
+@pytest.mark.parametrize(("experts", "n", "k"), [(16, 4096, 128), (16, 4096, 2112), (8, 4096, 2048),
+                                                 (8, 4096, 2112), (16, 3712, 192), (15, 2048, 64)])
+@pytest.mark.parametrize("mean", [9, 10, 30, 53])
+def test_products_that_fill_whole_rounds(mode, experts, n, k, mean):
+    """Uneven loads on both ways of cutting a plain product."""
+    from vllm_tgis_adapter_amd import ops
+
+    g = torch.Generator("cuda").manual_seed(n + k + mean)
+    counts = [0, 3 * mean - 1 + mean // 2, mean - mean // 2, 1] + [mean] * (experts - 4)
+    seg = _segments(counts)
+    assert int(seg[-1]) == experts * mean
+    w = torch.randn((experts, n, k), generator=g, device="cuda").bfloat16() / k ** 0.5
+    x = torch.randn((int(seg[-1]), k), generator=g, device="cuda").bfloat16()
+    got = ops.moe_gemm(x, w, seg.cuda(), False, act="relu2" if mode == "relu2" else None)
+    for e in range(experts):
+        lo, hi = int(seg[e]), int(seg[e + 1])
+        s = x[lo:hi].double() @ w[e].double().t()
+        if mode == "relu2":
+            s = s.clamp(min=0).square()
+        err = (got[lo:hi].double() - s).abs()
+        # one rounding to bf16; float32 sums of up to 2112 terms of size 1 / sqrt(k)
+        assert (err <= 2 ** -8 * s.abs() + 1e-4).all(), (e, err.max().item())
