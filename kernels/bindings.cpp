@@ -21,27 +21,10 @@ void launch_rotary_embedding(const long*, T*, const T*, T*, const float*, int, i
 template <typename T>
 void launch_reshape_and_cache(const T*, const T*, T*, T*, const long*, int,
                               int, long, long, hipStream_t);
-template <typename T>
-void launch_paged_decode(T*, const T*, const T*, const T*, const int*,
-                         const int*, float, int, int, int, int, int, int,
-                         hipStream_t);
-template <typename T>
-void launch_paged_prefill(T*, const T*, const T*, const T*, const int*,
-                          const int*, const int*, float, int, int, int, int,
-                          int, int, int, hipStream_t);
 void launch_mfma_probe_32(const unsigned short*, const unsigned short*, float*,
                           hipStream_t);
 void launch_mfma_probe_16(const unsigned short*, const unsigned short*, float*,
                           hipStream_t);
-void launch_paged_prefill_mfma_v2(__hip_bfloat16*, const __hip_bfloat16*,
-                                  const __hip_bfloat16*, const __hip_bfloat16*,
-                                  const int*, const int*, const int*, float,
-                                  int, int, int, int, int, int, int,
-                                  hipStream_t);
-void launch_paged_prefill_mfma(__hip_bfloat16*, const __hip_bfloat16*,
-                               const __hip_bfloat16*, const __hip_bfloat16*,
-                               const int*, const int*, const int*, float, int,
-                               int, int, int, int, int, int, hipStream_t);
 int gemm_skinny_num_ksplit(int N, int K, int M);
 void launch_logsoftmax_topk(float*, int*, float*, int*,
                             const __hip_bfloat16*, const long*, int, int,
@@ -51,11 +34,6 @@ void launch_gemm_tile(__hip_bfloat16*, const __hip_bfloat16*,
 void launch_xgmi_allreduce(const unsigned long long*, __hip_bfloat16*,
                            const __hip_bfloat16*, long, long, int, int,
                            hipStream_t);
-void launch_paged_prefill_mfma_v2_fp8(__hip_bfloat16*, const __hip_bfloat16*,
-                                      const unsigned char*,
-                                      const unsigned char*, const int*,
-                                      const int*, const int*, float, int, int,
-                                      int, int, int, int, int, hipStream_t);
 void launch_reshape_and_cache_fp8(const __hip_bfloat16*,
                                   const __hip_bfloat16*, unsigned char*,
                                   unsigned char*, const long*, int, int, long,

@@ -81,8 +81,7 @@ struct Block {
     const int wm = wave / WN, wn = wave % WN;
 
     // this lane's rows and chunk of every pass: eight rows a wave and instruction
-    unsigned long a_off[kAPass];
-    unsigned b_off[kBPass];
+    unsigned a_off[kAPass], b_off[kBPass];
 #pragma unroll
     for (int p = 0; p < kAPass; ++p) {
       const int r = (p * kWaves + wave) * 8 + lane / 8;

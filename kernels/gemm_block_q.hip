@@ -12,9 +12,9 @@
 // In the product weights are whole numbers and scales are applied to 32-bit sums, as in
 // gemm_stream.hip: int8 by conversion to f32 of which the upper half is all; 4 bits as the
 // bf16 pattern of 8 + n/2, with -12 times the sum of x added by a constant operand and the
-// scale doubled.  A lane's 16 (8) bytes hold two matrix steps' inputs, x is read to match.
-// x and W reach LDS without registers; x chunks are swizzled as in block_gemm.h, W rows of
-// 64 (32) bytes by r / 4 (r / 8).
+// scale doubled.  A lane's 16 bytes of W hold the inputs of two matrix steps in int8, of four
+// in 4 bits, and x is read to match.  x and W reach LDS without registers; chunks of a row are
+// turned by the row: x by r (256-byte rows) or r / 2 (128), W by r / 2 (128) or r / 4 (64).
 //
 // Measured: four llama-3-8b layers around attention, 301 rows, int8: 5101 -> 1046 us.
 // Widening 28672 x 4096: 61 us (5.8 TB/s).
@@ -242,6 +242,8 @@ __global__ __launch_bounds__(256) void widen_weight_kernel(
 //         301 rows: 64x64 29.4 (64x128 31.9), 64x64 26.8 (29.9), 64x128 99, 64x64 81.5 (88.9)
 //         700 rows: 64x128 57 (58.6), 64x64 36 (42.2), 64x128 200, 64x64 118 (132)
 //        1500 rows: 64x128 102, 64, 128x128 375 (64x128 440), 64x128 212
+//   (past 560 rows only matrices of up to 2^23 weights come here, so that the lines above hold
+//   where they are wide and short)
 //   4 bits, 100 rows: 32x64 24.5 (64x64 23.9), 18.4 (23.4), 64x128 53, 32x64 56.4 (74.7)
 //         301 rows: 64x128 34.1, 32x64 31.2 (33.2), 64x128 123, 32x64 101 (107)
 //         700 rows: 64x128 77, 48.5, 247, 167

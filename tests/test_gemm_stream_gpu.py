@@ -83,7 +83,8 @@ def test_rounded(qbits, m, n, k):
 
 @pytest.mark.parametrize("qbits", [8, 4])
 @pytest.mark.parametrize("m", [65, 127, 128, 129, 301, 460, 900])
-# blocks for every choice of tile: narrow, 64 wide, 128 wide, and many
+# blocks for the choices of tile: narrow, 64 wide, 128 wide, and many (the largest tiles:
+# test_rounded_largest_tiles)
 @pytest.mark.parametrize(("n", "k"), [(128, 128), (512, 384), (4096, 256), (8192, 640),
                                       (36864, 256)])
 def test_rounded_many_rows(qbits, m, n, k):
@@ -227,3 +228,17 @@ def test_parts_of_k(m, n, k):
         size = x.double().abs().sum(1, keepdim=True) * exact.abs().amax(1)
         _check(ops.linear_quant(x, wq, scale, 4), x.double() @ exact.t(),
                5 * (x.double().abs() @ exact.abs().t() + size))
+
+
+@pytest.mark.parametrize("m", [1025, 1041])
+def test_rounded_largest_tiles(m):
+    """Wide matrices of few inputs, past 4096 blocks: 128 x 128 in int8."""
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    n, k = 32768, 256
+    assert m <= ops._quant_rows(8, n, k) and (m + 63) // 64 * (n // 128) >= 4096
+    x, w = _x(m, k, 24), _x(n, k, 25)
+    wq, scale = ops.quantize_weight(w, 8)
+    exact = (wq.double() * scale.double()[:, None]).t()
+    _check(ops.linear_quant(x, wq, scale, 8), x.double() @ exact, x.double().abs() @ exact.abs())
