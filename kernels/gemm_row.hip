@@ -11,11 +11,12 @@
 // v_dot2_f32_bf16 into f32.  4-bit weights enter as 8 + n / 2, -12 times the sum of x
 // takes the offset out, the doubled scale goes onto the f32 sum of a lane's 32 inputs.
 //
-// us over weights that are not in the caches, gemm_stream.h -> here (at 6.2 TB/s), N x K:
-//   4 bits: 28672 x 4096 23.7 -> 17.0 (9.5), 6144 x 4096 8.9 -> 7.0 (2.0), 4096 x 4096 6.7 ->
-//     5.8 (1.4), 4096 x 14336 17.4 -> 12.6 (4.7);
-//   bf16: 14336 x 4096 gated 41.7 -> 36.3 (38), 8192 x 2048 gated 15.7 -> 12.9 (10.8), 2048 x
-//     8192 11.4 -> 8.8 (5.4), 2048 x 2048 5.1 -> 4.2 (1.4), 32000 x 2048 27.8 -> 21.7 (21);
+// us over 1.5 GB of weights in turn, gemm_stream.h -> here (at 6.2 TB/s; reads in sequence
+// reach 6.4), N x K:
+//   4 bits: 28672 x 4096 23.7 -> 18.1 (10.1), 6144 x 4096 8.9 -> 7.2 (2.2), 4096 x 4096 6.7 ->
+//     5.8 (1.4), 4096 x 14336 17.4 -> 13.6 (5.0);
+//   bf16: 14336 x 4096 gated 41.7 -> 36.9 (37.9), 8192 x 2048 gated 15.7 -> 13.4 (10.8), 2048 x
+//     8192 11.4 -> 8.9 (5.4), 2048 x 2048 5.1 -> 4.2 (1.4), 32000 x 2048 27.8 -> 22.8 (21.1);
 //   a llama-1b step 486 -> 433 us, a llama-3-8b one in 4 bits 751 -> 638.
 // With two rows the same way is no faster (28672 x 4096 23.7, bf16 4096 x 4096 9.9 against
 // 8.8), in int8 it is slower with one (28672 x 4096 26 against 25).

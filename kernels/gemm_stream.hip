@@ -19,7 +19,7 @@
 // becomes 8 + n/2 by two logical operations a pair (n in the upper bits of a bf16
 // mantissa); x is put in the order that this leaves the weights in, -12 times the sum
 // of x, which the matrix unit adds by a constant operand, takes the offset out again
-// and the scale is doubled.
+// and the scale is doubled.  (An infinite x, or one above 2^123, makes its row NaN there.)
 //
 // Measured against the kernels before (barriers around 64-input chunks, weights rounded
 // to bf16 with their scale, a merge launch for every matrix), us a product with the

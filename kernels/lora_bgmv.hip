@@ -17,7 +17,7 @@
 // read and write of out.
 //
 // Layers of 4096 wide rows, 61 tokens of 4 adapters of rank 16: 7 + 7 launches of 25 and
-// 5 us were 4 + 4 of 4.7 and 6.5.  2048 tokens: shrink 23 us, expand into 4096 columns 14
+// 5 us were 4 + 4 of 4.4 and 6.3.  2048 tokens: shrink 23 us, expand into 4096 columns 14
 // and into 28672 102, where reading and writing out takes 51.
 //
 // f32 and f16: one token per workgroup in both,
