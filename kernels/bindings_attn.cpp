@@ -119,6 +119,7 @@ const T* cptr(const torch::Tensor& t) {
 // and not so small that it lifts that mark into range.  Of other scales the queries take the
 // sign (exact), a power of two that the smallest of them lack, or the zero.
 void positive_scale(torch::Tensor& q, double& scale) {
+  scale = (float)scale;   // as the kernels take it: what is below its range is zero
   if (!(scale < 0x1p-100)) return;   // (NaN stays as it is)
   double turn = scale < 0 ? -1.0 : scale > 0 ? 1.0 : 0.0;
   if (scale > -0x1p-100) turn *= 0x1p-64;

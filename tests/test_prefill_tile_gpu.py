@@ -109,7 +109,7 @@ def _close(got, want, terms):
     assert (err <= 1.01 * 2 ** -7 * terms.double() + 1e-6).all(), err.max().item()
 
 
-@pytest.mark.parametrize("scale", [-0.11, 0.0, -0.0, 1e-38, -1e-42])
+@pytest.mark.parametrize("scale", [-0.11, 0.0, -0.0, 1e-38, -1e-42, 1e-60, -1e-300])
 @pytest.mark.parametrize(("kind", "dim"), [
     ("plain", 64), ("plain", 128), ("fp8", 128), ("windowed", 128), ("capped", 64),
     ("capped", 128), ("chunk", 128)])
