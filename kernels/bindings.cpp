@@ -47,6 +47,14 @@ void launch_gemm_block(__hip_bfloat16*, float*, const __hip_bfloat16*, const __h
                        int, int, int, hipStream_t);
 void launch_gemm_stream(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hip_bfloat16*,
                         int, int, int, int, hipStream_t);
+bool gemm_row_fits(int qbits, int K);
+void launch_gemm_row_norm_gated(__hip_bfloat16*, __hip_bfloat16*, const __hip_bfloat16*,
+                                const __hip_bfloat16*, const __hip_bfloat16*, float, const void*,
+                                const float*, int, int, int, hipStream_t);
+void launch_gemm_row_norm_turn(__hip_bfloat16*, __hip_bfloat16*, const __hip_bfloat16*,
+                               const __hip_bfloat16*, const __hip_bfloat16*, float, const void*,
+                               const float*, int, int, const long*, const long*, const float*,
+                               void*, void*, int, int, int, bool, hipStream_t);
 void launch_gemm_stream_gated(__hip_bfloat16*, float*, const __hip_bfloat16*,
                               const __hip_bfloat16*, int, int, int, int, hipStream_t);
 void launch_gemm_stream_q(__hip_bfloat16*, float*, const __hip_bfloat16*, const unsigned char*,
@@ -398,6 +406,88 @@ void widen_weight(torch::Tensor out, torch::Tensor wq, torch::Tensor wscale, int
                       wscale.data_ptr<float>(), (int)qbits, N * K, (int)K, current_stream());
 }
 
+// What the products of one normed row share: x [1, K] (+ residual) -> norm -> w [rows, K] in
+// qbits; returns the sum's place (null without a residual).
+__hip_bfloat16* check_row_norm(const torch::Tensor& x, const c10::optional<torch::Tensor>& residual,
+                               c10::optional<torch::Tensor>& sum, const torch::Tensor& weight,
+                               const torch::Tensor& w, const c10::optional<torch::Tensor>& scales,
+                               int64_t qbits, int64_t rows) {
+  const int64_t K = x.numel();
+  auto row = [&](const torch::Tensor& t) {
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::ScalarType::BFloat16 && t.is_contiguous() &&
+                    t.numel() == K && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0,
+                "one dense bf16 row from a 16-byte boundary on");
+  };
+  row(x);
+  row(weight);
+  TORCH_CHECK(residual.has_value() == sum.has_value());
+  if (residual.has_value()) {
+    row(*residual);
+    row(*sum);
+    TORCH_CHECK(sum->data_ptr() != residual->data_ptr() && sum->data_ptr() != x.data_ptr());
+  }
+  TORCH_CHECK(rows % 128 == 0 && K % 64 == 0 && gemm_row_fits((int)qbits, (int)K));
+  TORCH_CHECK(w.is_cuda() && w.dim() == 2 && w.size(0) == rows && w.is_contiguous() &&
+              reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0);
+  if (qbits == 16) {
+    TORCH_CHECK(w.scalar_type() == at::ScalarType::BFloat16 && w.size(1) == K);
+  } else {
+    TORCH_CHECK(scales.has_value() && scales->is_cuda());
+    check_rounded(w, *scales, qbits, rows, K);
+  }
+  return sum.has_value() ? ptr<__hip_bfloat16>(*sum) : nullptr;
+}
+
+const __hip_bfloat16* optional_row(const c10::optional<torch::Tensor>& t) {
+  return t.has_value() ? cptr<__hip_bfloat16>(*t) : nullptr;
+}
+
+const float* optional_scales(const c10::optional<torch::Tensor>& t, int64_t qbits) {
+  return qbits == 16 ? nullptr : t->data_ptr<float>();
+}
+
+// y [1, I] = silu(n Wg^T) * (n Wu^T), n = rmsnorm(x + residual), sum = x + residual
+void row_norm_gated(torch::Tensor y, c10::optional<torch::Tensor> sum, torch::Tensor x,
+                    c10::optional<torch::Tensor> residual, torch::Tensor weight, double eps,
+                    torch::Tensor w, c10::optional<torch::Tensor> scales, int64_t qbits) {
+  const int64_t I = y.numel();
+  __hip_bfloat16* to = check_row_norm(x, residual, sum, weight, w, scales, qbits, 2 * I);
+  TORCH_CHECK(y.is_cuda() && y.scalar_type() == at::ScalarType::BFloat16 && y.is_contiguous() &&
+              I % 128 == 0);
+  launch_gemm_row_norm_gated(ptr<__hip_bfloat16>(y), to, cptr<__hip_bfloat16>(x),
+                             optional_row(residual), cptr<__hip_bfloat16>(weight), (float)eps,
+                             w.data_ptr(), optional_scales(scales, qbits), (int)qbits, (int)I,
+                             (int)x.numel(), current_stream());
+}
+
+// q [1, heads * hd] = the turned queries of n W^T, its turned keys and its values in the cache
+void row_norm_turn(torch::Tensor q, c10::optional<torch::Tensor> sum, torch::Tensor x,
+                   c10::optional<torch::Tensor> residual, torch::Tensor weight, double eps,
+                   torch::Tensor w, c10::optional<torch::Tensor> scales, int64_t qbits,
+                   torch::Tensor positions, torch::Tensor slots, torch::Tensor cos_sin,
+                   torch::Tensor k_cache, torch::Tensor v_cache) {
+  TORCH_CHECK(k_cache.dim() == 4 && k_cache.sizes() == v_cache.sizes());
+  const int64_t kvh = k_cache.size(2), hd = k_cache.size(3), heads = q.numel() / hd;
+  TORCH_CHECK(q.is_cuda() && q.scalar_type() == at::ScalarType::BFloat16 && q.is_contiguous() &&
+              heads * hd == q.numel() && hd >= 32 && (hd & (hd - 1)) == 0);
+  __hip_bfloat16* to =
+      check_row_norm(x, residual, sum, weight, w, scales, qbits, (heads + 2 * kvh) * hd);
+  const bool fp8 = k_cache.scalar_type() == at::ScalarType::Byte;
+  for (const auto& c : {k_cache, v_cache})
+    TORCH_CHECK(c.is_cuda() && c.is_contiguous() &&
+                c.scalar_type() == (fp8 ? at::ScalarType::Byte : at::ScalarType::BFloat16));
+  for (const auto& i : {positions, slots})
+    TORCH_CHECK(i.is_cuda() && i.scalar_type() == at::ScalarType::Long && i.numel() == 1);
+  TORCH_CHECK(cos_sin.is_cuda() && cos_sin.scalar_type() == at::ScalarType::Float &&
+              cos_sin.is_contiguous() && cos_sin.size(-1) == hd);
+  launch_gemm_row_norm_turn(
+      ptr<__hip_bfloat16>(q), to, cptr<__hip_bfloat16>(x), optional_row(residual),
+      cptr<__hip_bfloat16>(weight), (float)eps, w.data_ptr(), optional_scales(scales, qbits),
+      (int)qbits, (int)x.numel(), positions.data_ptr<long>(), slots.data_ptr<long>(),
+      cos_sin.data_ptr<float>(), k_cache.data_ptr(), v_cache.data_ptr(), (int)heads, (int)kvh,
+      __builtin_ctzl(hd) - 1, fp8, current_stream());
+}
+
 void gemm_skinny_gated(torch::Tensor y, torch::Tensor x, torch::Tensor w13) {
   const int M = x.size(0);
   const int K = x.size(1);
@@ -689,6 +779,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("widen_weight", &widen_weight, "int8 / 4-bit weights to bf16");
   m.def("gemm_skinny", &gemm_skinny,
         "skinny decode GEMM y = x @ w^T, M <= 64 (CDNA4 MFMA)");
+  m.def("row_norm_gated", &row_norm_gated, "norm and gated product of one row (CDNA4)");
+  m.def("row_norm_turn", &row_norm_turn,
+        "norm, query / key / value product, rotation and cache write of one row (CDNA4)");
   m.def("gemm_skinny_gated", &gemm_skinny_gated,
         "fused gate/up skinny GEMM + SiLU-mul, M <= 64 (CDNA4 MFMA)");
   m.def("moe_gemm", &moe_gemm,

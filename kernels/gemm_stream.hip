@@ -1,5 +1,5 @@
-// Products of few rows with a whole weight matrix (decode, M <= 64; a single row with bf16
-// or 4-bit weights: gemm_row.hip):
+// Products of few rows with a whole weight matrix (decode, M <= 64; a single row:
+// gemm_row.hip):
 //   y[m, n] = sum_k x[m, k] W[n, k],  or  silu(x Wg^T) * (x Wu^T) for W = [Wg; Wu],
 // with W in bf16, in int8 (a scale per row) or in 4 bits (offset 8, a scale per row
 // and 128 inputs).

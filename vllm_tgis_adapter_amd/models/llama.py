@@ -26,6 +26,20 @@ from ..parallel.layers import (
 )
 
 
+def lora_active() -> bool:
+    from ..engine.lora import CTX
+
+    return CTX.active
+
+
+def stored_weight(linear: nn.Module):
+    """A projection's weight as it is stored: (weight, scales or None, bits)."""
+    bits = getattr(linear, "quant_bits", None)
+    if bits is None:
+        return linear.weight, None, 16
+    return linear.weight_q, linear.weight_scale, bits
+
+
 class RMSNorm(nn.Module):
     def __init__(self, hidden: int, eps: float, dtype: torch.dtype):
         super().__init__()
@@ -74,8 +88,22 @@ class Attention(nn.Module):
         k_cache, v_cache = kv_cache
         q = ops.rotary_and_cache(positions, q, k, v, self.head_dim, cos_sin_cache,
                                  k_cache, v_cache, meta.slot_mapping)
-        q = q.view(hidden.shape[0], self.num_heads, self.head_dim)
+        return self.attend(q, kv_cache, meta)
 
+    def row_inputs(self, hidden, residual, norm, positions, kv_cache, meta, cos_sin_cache):
+        """The norm, the projections, the rotation and the cache write of a step of one row
+        in one launch: (q, residual), or None where that doesn't apply."""
+        qkv = self.qkv_proj
+        if hidden.shape[0] != 1 or qkv.bias is not None or lora_active():
+            return None
+        return ops.row_norm_qkv(
+            hidden, residual, norm.weight, norm.eps, *stored_weight(qkv), self.num_heads,
+            positions, cos_sin_cache, *kv_cache, meta.slot_mapping)
+
+    def attend(self, q, kv_cache, meta: AttnMetadata) -> torch.Tensor:
+        """Attention over the cache, which has the step's keys and values, and o_proj."""
+        k_cache, v_cache = kv_cache
+        q = q.view(q.shape[0], self.num_heads, self.head_dim)
         out = torch.empty_like(q)
         npt = meta.num_prefill_tokens
         if npt:
@@ -91,7 +119,7 @@ class Attention(nn.Module):
                 meta.decode_block_tables, meta.decode_seq_lens,
                 self.scale, meta.max_decode_seq_len, out=out[npt:],
             )
-        return self.o_proj(out.view(hidden.shape[0], -1), lora=self._o_lora)
+        return self.o_proj(out.view(q.shape[0], -1), lora=self._o_lora)
 
 
 class LlamaMLP(nn.Module):
@@ -109,14 +137,37 @@ class LlamaMLP(nn.Module):
         self._down_lora = (layer_idx, [("down_proj", 0, cfg.hidden_size)])
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        from ..engine.lora import CTX as _lora_ctx
-
-        if not _lora_ctx.active and getattr(self.gate_up, "quant_bits", None) is None:
+        if not lora_active() and getattr(self.gate_up, "quant_bits", None) is None:
             h = ops.gated_mlp_up(x, self.gate_up.weight)
             if h is not None:
                 return self.down(h, lora=self._down_lora)
         h = ops.silu_and_mul(self.gate_up(x, lora=self._gu_lora))
         return self.down(h, lora=self._down_lora)
+
+    def row(self, hidden, residual, norm):
+        """The norm and the feed-forward of a step of one row, the norm and the gate in the
+        first product's launch: (hidden, residual), or None where that doesn't apply."""
+        if hidden.shape[0] != 1 or self.gate_up.bias is not None or lora_active():
+            return None
+        made = ops.row_norm_gated(hidden, residual, norm.weight, norm.eps,
+                                  *stored_weight(self.gate_up))
+        if made is None:
+            return None
+        return self.down(made[0], lora=self._down_lora), made[1]
+
+
+def attention_sublayer(layer, hidden, residual, positions, kv_cache, meta, cos_sin_cache):
+    """A layer's first norm and attention: (hidden, residual) for the second norm."""
+    made = layer.attn.row_inputs(hidden, residual, layer.input_norm, positions, kv_cache, meta,
+                                 cos_sin_cache)
+    if made is not None:
+        return layer.attn.attend(made[0], kv_cache, meta), made[1]
+    if residual is None:
+        residual = hidden
+        hidden = layer.input_norm(hidden)
+    else:
+        hidden, residual = layer.input_norm(hidden, residual)
+    return layer.attn(hidden, positions, kv_cache, meta, cos_sin_cache), residual
 
 
 class LlamaDecoderLayer(nn.Module):
@@ -128,12 +179,11 @@ class LlamaDecoderLayer(nn.Module):
         self.mlp = LlamaMLP(cfg, layer_idx)
 
     def forward(self, hidden, residual, positions, kv_cache, meta, cos_sin_cache):
-        if residual is None:
-            residual = hidden
-            hidden = self.input_norm(hidden)
-        else:
-            hidden, residual = self.input_norm(hidden, residual)
-        hidden = self.attn(hidden, positions, kv_cache, meta, cos_sin_cache)
+        hidden, residual = attention_sublayer(
+            self, hidden, residual, positions, kv_cache, meta, cos_sin_cache)
+        made = self.mlp.row(hidden, residual, self.post_norm)
+        if made is not None:
+            return made
         hidden, residual = self.post_norm(hidden, residual)
         hidden = self.mlp(hidden)
         return hidden, residual

@@ -21,7 +21,7 @@ from .. import ops
 from ..engine.config import ModelConfig
 from ..parallel import divide, get_tp_world_size, tp_all_reduce
 from ..parallel.layers import ParallelLMHead, VocabParallelEmbedding, _init_weight
-from .llama import Attention, RMSNorm
+from .llama import Attention, RMSNorm, attention_sublayer
 
 
 class MoEBlock(nn.Module):
@@ -158,12 +158,8 @@ class MixtralDecoderLayer(nn.Module):
         self.moe = MoEBlock(cfg)
 
     def forward(self, hidden, residual, positions, kv_cache, meta, cos_sin_cache):
-        if residual is None:
-            residual = hidden
-            hidden = self.input_norm(hidden)
-        else:
-            hidden, residual = self.input_norm(hidden, residual)
-        hidden = self.attn(hidden, positions, kv_cache, meta, cos_sin_cache)
+        hidden, residual = attention_sublayer(
+            self, hidden, residual, positions, kv_cache, meta, cos_sin_cache)
         hidden, residual = self.post_norm(hidden, residual)
         hidden = self.moe(hidden)
         return hidden, residual

@@ -423,6 +423,85 @@ def gated_mlp_up(x: torch.Tensor, w13: torch.Tensor) -> torch.Tensor | None:
     return None
 
 
+def _row_norm_usable(x, residual, norm_weight, weight, scales, qbits: int) -> bool:
+    """Whether a norm and the product of its one row are one launch: what the kernels of a
+    single row take, and where gated_mlp_up and linear_quant would take their kernels too."""
+    if (x.dim() != 2 or x.shape[0] != 1 or not native_enabled(x)
+            or int(os.environ.get("VTA_GEMM_MAX_M", "64")) < 1):
+        return False
+    k = x.shape[1]
+    rows = [x, norm_weight] if residual is None else [x, norm_weight, residual]
+    if not all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.numel() == k for t in rows):
+        return False
+    if qbits == 16:
+        if weight.dtype != torch.bfloat16 or weight.shape[1] != k:
+            return False
+    elif (scales.dtype != torch.float32 or not scales.is_contiguous() or k % 128
+          or weight.dtype != (torch.int8 if qbits == 8 else torch.uint8)):
+        return False
+    return (weight.shape[0] % 128 == 0 and k % 64 == 0 and k <= 28672
+            and weight.is_contiguous() and _plain_tensors(*rows, weight))
+
+
+def row_norm_gated(
+    x: torch.Tensor,                 # [1, K]
+    residual: torch.Tensor | None,   # [1, K]
+    norm_weight: torch.Tensor,
+    eps: float,
+    weight: torch.Tensor,            # [gate; up] as it is or rounded
+    scales: torch.Tensor | None,
+    qbits: int = 16,
+) -> tuple[torch.Tensor, torch.Tensor] | None:
+    """A step of one row: fused_add_rms_norm, the merged product and silu_and_mul in one
+    launch.  Returns (h, x + residual), the latter a tensor of its own (x itself without a
+    residual), or None where the kernel doesn't apply."""
+    if not _row_norm_usable(x, residual, norm_weight, weight, scales, qbits):
+        return None
+    inter = weight.shape[0] // 2
+    if inter % 128:
+        return None
+    out = torch.empty((1, inter), dtype=x.dtype, device=x.device)
+    total = None if residual is None else torch.empty_like(x)
+    _C.row_norm_gated(out, total, x, residual, norm_weight, eps, weight, scales, qbits)
+    return out, x if total is None else total
+
+
+def row_norm_qkv(
+    x: torch.Tensor,                 # [1, K]
+    residual: torch.Tensor | None,
+    norm_weight: torch.Tensor,
+    eps: float,
+    weight: torch.Tensor,            # [queries; keys; values]
+    scales: torch.Tensor | None,
+    qbits: int,
+    heads: int,
+    positions: torch.Tensor,
+    cos_sin_cache: torch.Tensor,
+    k_cache: torch.Tensor,
+    v_cache: torch.Tensor,
+    slot_mapping: torch.Tensor,
+) -> tuple[torch.Tensor, torch.Tensor] | None:
+    """A step of one row: fused_add_rms_norm, the merged product and rotary_and_cache in one
+    launch.  Returns (q turned, x + residual) as row_norm_gated does, or None."""
+    if k_cache.dim() != 4 or not _row_norm_usable(x, residual, norm_weight, weight, scales, qbits):
+        return None
+    kvh, hd = k_cache.shape[2:]
+    if (weight.shape[0] != (heads + 2 * kvh) * hd or hd < 32 or hd & (hd - 1)
+            or k_cache.shape != v_cache.shape
+            or k_cache.dtype not in (torch.bfloat16, torch.uint8) or k_cache.dtype != v_cache.dtype
+            or not k_cache.is_contiguous() or not v_cache.is_contiguous()
+            or cos_sin_cache.dtype != torch.float32 or cos_sin_cache.shape[-1] != hd
+            or not cos_sin_cache.is_contiguous()
+            or positions.dtype != torch.int64 or slot_mapping.dtype != torch.int64
+            or positions.numel() != 1 or slot_mapping.numel() != 1):
+        return None
+    q = torch.empty((1, heads * hd), dtype=x.dtype, device=x.device)
+    total = None if residual is None else torch.empty_like(x)
+    _C.row_norm_turn(q, total, x, residual, norm_weight, eps, weight, scales, qbits, positions,
+                     slot_mapping, cos_sin_cache, k_cache, v_cache)
+    return q, x if total is None else total
+
+
 def lora_bgmv(
     out: torch.Tensor,      # [T, out_w] updated in place
     x: torch.Tensor,        # [T, K]
