@@ -65,8 +65,9 @@ void launch_gemm_skinny(__hip_bfloat16*, float*, const __hip_bfloat16*,
 void launch_gemm_skinny_gated(__hip_bfloat16*, float*, const __hip_bfloat16*,
                               const __hip_bfloat16*, int, int, int, int,
                               hipStream_t);
-void launch_gemm_block_q(__hip_bfloat16*, const __hip_bfloat16*, const unsigned char*,
-                         const float*, int, int, int, int, hipStream_t);
+int gemm_panel_plan(int M, int N, int K);
+void launch_gemm_block_q(__hip_bfloat16*, float*, const __hip_bfloat16*, const unsigned char*,
+                         const float*, int, int, int, int, int, hipStream_t);
 void launch_widen_weight(__hip_bfloat16*, const unsigned char*, const float*, int, long, int,
                          hipStream_t);
 struct LoraCols {
@@ -384,8 +385,11 @@ void gemm_q(torch::Tensor y, torch::Tensor x, torch::Tensor wq, torch::Tensor ws
     // both reach LDS in 16-byte pieces
     TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
                 reinterpret_cast<uintptr_t>(wq.data_ptr()) % 16 == 0);
-    launch_gemm_block_q(ptr<__hip_bfloat16>(y), cptr<__hip_bfloat16>(x), cptr<unsigned char>(wq),
-                        wscale.data_ptr<float>(), (int)qbits, M, N, K, current_stream());
+    const int plan = qbits == 8 ? gemm_panel_plan(M, N, K) : 1;
+    torch::Tensor part;
+    launch_gemm_block_q(ptr<__hip_bfloat16>(y), stream_parts(part, x, plan & 255, (int64_t)M * N),
+                        cptr<__hip_bfloat16>(x), cptr<unsigned char>(wq),
+                        wscale.data_ptr<float>(), (int)qbits, M, N, K, plan, current_stream());
     return;
   }
   const int parts = gemm_stream_parts((int)qbits, M, N, K, false);
@@ -779,6 +783,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("widen_weight", &widen_weight, "int8 / 4-bit weights to bf16");
   m.def("gemm_skinny", &gemm_skinny,
         "skinny decode GEMM y = x @ w^T, M <= 64 (CDNA4 MFMA)");
+  m.def("gemm_panel_plan", &gemm_panel_plan,
+        "which panel int8 products of many rows take, and parts of K (panel << 8 | parts)");
   m.def("row_norm_gated", &row_norm_gated, "norm and gated product of one row (CDNA4)");
   m.def("row_norm_turn", &row_norm_turn,
         "norm, query / key / value product, rotation and cache write of one row (CDNA4)");

@@ -5,7 +5,8 @@
 // two products, all in f32 in memory) ahead of a library product: 1.0 ms of 1.3 ms a
 // llama-3-8b layer at 301 rows.  Now
 //  - up to some hundreds of rows the product widens a tile's weights itself, between LDS
-//    and the matrix unit: W crosses memory once, at its own size;
+//    and the matrix unit: W crosses memory once, at its own size (int8: gemm_panel_q.h, but
+//    for small matrices);
 //  - above, one kernel writes the widened matrix (bf16(q scale), bound by its bytes) for
 //    the library's product, which is then the larger part and the faster one.
 //
@@ -16,10 +17,11 @@
 // in 4 bits, and x is read to match.  x and W reach LDS without registers; chunks of a row are
 // turned by the row: x by r (256-byte rows) or r / 2 (128), W by r / 2 (128) or r / 4 (64).
 //
-// Measured: four llama-3-8b layers around attention, 301 rows, int8: 5101 -> 1046 us.
+// Measured: four llama-3-8b layers around attention, 301 rows, int8: 5101 -> 1064 us with tiles of
+// up to 64 x 128 whose weights every 64 rows widened again, -> 739 us with panels.
 // Widening 28672 x 4096: 61 us (5.8 TB/s).
 
-#include "block_gemm.h"
+#include "gemm_panel_q.h"
 
 namespace {
 
@@ -238,15 +240,12 @@ __global__ __launch_bounds__(256) void widen_weight_kernel(
 
 // Tiles by how many blocks there are to fill 256 CUs with (us of what is chosen and the
 // next best; columns x inputs 6144 x 4096, 4096 x 4096, 28672 x 4096, 4096 x 14336):
-//   int8, 100 rows: 32x64 20.6 (64x64 22.4), 32x64 16.2 (21.4), 64x128 48.3, 32x64 49.0 (65.1)
-//         301 rows: 64x64 29.4 (64x128 31.9), 64x64 26.8 (29.9), 64x128 99, 64x64 81.5 (88.9)
-//         700 rows: 64x128 57 (58.6), 64x64 36 (42.2), 64x128 200, 64x64 118 (132)
-//        1500 rows: 64x128 102, 64, 128x128 375 (64x128 440), 64x128 212
-//   (past 560 rows only matrices of up to 2^23 weights come here, so that the lines above hold
-//   where they are wide and short)
 //   4 bits, 100 rows: 32x64 24.5 (64x64 23.9), 18.4 (23.4), 64x128 53, 32x64 56.4 (74.7)
 //         301 rows: 64x128 34.1, 32x64 31.2 (33.2), 64x128 123, 32x64 101 (107)
 //         700 rows: 64x128 77, 48.5, 247, 167
+//   int8, small matrices of short K (64x64, and 32x64 where fewer, | panels): 2048 x 2048, 100
+//         rows 10.3 | 10.2, 256 rows 10.5 | 12.3; 3072 x 2048, 128 rows 10.5 | 12.0, 301 rows
+//         12.6 | 12.8, 384 rows 15.5 | 13.2
 template <int QB>
 void launch_block(__hip_bfloat16* y, const __hip_bfloat16* x, const unsigned char* w,
                   const float* scale, int M, int N, int K, hipStream_t stream) {
@@ -259,24 +258,95 @@ void launch_block(__hip_bfloat16* y, const __hip_bfloat16* x, const unsigned cha
     if (wide >= 230) GO(128, 64, 128, 1, 4, 3);
     else GO(128, 32, 64, 1, 4, 3);
   } else {
-    if (wide >= 4096) GO(64, 128, 128, 2, 2, 2);
-    else if (wide >= 448) GO(64, 64, 128, 1, 4, 3);
-    else if (wide >= 150) GO(128, 64, 64, 1, 4, 2);
+    if (wide >= 150) GO(128, 64, 64, 1, 4, 2);
     else GO(128, 32, 64, 1, 4, 3);
   }
 #undef GO
 }
 
+// Panels (gemm_panel_q.h) and how their time adds up, us: what a tile of 64 inputs takes with
+// one workgroup on a CU and with as many as share one.  Fitted to some 5000 times (ten matrices
+// from 1024 x 4096 to 28672 x 4096, 70 to 2048 rows, K cut over one to eight workgroups; 7 % rms);
+// what it chooses is 1.1 % off the fastest panel in the mean.
+struct Panel {
+  int tm, tn, per_cu;
+  float one, full;
+};
+constexpr Panel kPanels[] = {{5, 1, 2, .232f, .423f}, {5, 2, 2, .347f, .598f},
+                             {6, 2, 2, .373f, .648f}, {8, 1, 2, .319f, .551f},
+                             {8, 2, 2, .582f, .784f}, {8, 2, 1, .482f, .482f},
+                             {10, 2, 1, .550f, .550f}, {10, 4, 1, .985f, .985f}};
+
+float panel_us(const Panel& p, int M, int N, int K, int parts) {
+  const int wgs = (M + p.tm * 16 - 1) / (p.tm * 16) * (N / (p.tn * 64)) * parts;
+  const int tiles = (K / 64 + parts - 1) / parts, round = 256 * p.per_cu, left = wgs % round;
+  float us = 2.6f + wgs / round * (p.full * tiles + 3.4f);
+  if (left > 0) us += (left > 256 ? p.full : p.one) * tiles + 3.4f;
+  if (parts > 1) us += 2.1f + 1.6e-6f * parts * M * N;   // their merge
+  return us;
+}
+
 }  // namespace
 
-// M >= 1, N % 128 == 0, K % 128 == 0
-void launch_gemm_block_q(__hip_bfloat16* y, const __hip_bfloat16* x, const unsigned char* w,
-                         const float* scale, int qbits, int M, int N, int K,
-                         hipStream_t stream) {
-  if (qbits == 8)
-    launch_block<8>(y, x, w, scale, M, N, K, stream);
-  else
+// Which panel, and how many workgroups K is cut over (each leaves a part of the result in f32),
+// of eight tiles of 64 inputs at least: (panel << 8 | parts), or 1 where tiles of
+// gemm_block_q_kernel do.  A function of shapes.
+int gemm_panel_plan(int M, int N, int K) {
+  if (K <= 2048 && (long)N * K <= 1 << 23 && M <= 320) return 1;
+  int plan = 0;
+  float least = 0.f;
+  for (int i = 0; i < (int)(sizeof(kPanels) / sizeof(kPanels[0])); ++i) {
+    if (N % (kPanels[i].tn * 64) != 0) continue;
+    for (int parts = 1; parts <= 8 && (parts == 1 || K / parts >= 512); ++parts) {
+      const int depth = (K / 64 + parts - 1) / parts;
+      if ((K / 64 + depth - 1) / depth != parts) continue;   // no part is empty
+      const float us = panel_us(kPanels[i], M, N, K, parts);
+      if (plan == 0 || us < least) {
+        plan = (i + 1) << 8 | parts;
+        least = us;
+      }
+    }
+  }
+  return plan;
+}
+
+void launch_gemm_merge(__hip_bfloat16* y, const float* part, long plane, int parts, bool gated,
+                       hipStream_t stream);
+
+namespace {
+
+void launch_panel(__hip_bfloat16* y, float* part, const __hip_bfloat16* x, const unsigned char* w,
+                  const float* scale, int M, int N, int K, int plan, hipStream_t stream) {
+  const int parts = plan & 255, panel = (plan >> 8) - 1;
+  const int depth = (K / 64 + parts - 1) / parts * 64;
+#define GO(I, STAGES)                                                                         \
+  case I: {                                                                                   \
+    constexpr Panel p = kPanels[I];                                                           \
+    const int blocks = (M + p.tm * 16 - 1) / (p.tm * 16) * (N / (p.tn * 64));                 \
+    hipLaunchKernelGGL((gemm_panel::gemm_panel_q_kernel<p.tm, p.tn, STAGES, p.per_cu>),       \
+                       dim3((blocks + 7) / 8 * 8, parts), dim3(64 * gemm_panel::kWaves), 0,   \
+                       stream, y, part, x, w, scale, M, N, K, depth);                         \
+    break;                                                                                    \
+  }
+  switch (panel) {
+    GO(0, 5) GO(1, 4) GO(2, 4) GO(3, 4) GO(4, 3) GO(5, 5) GO(6, 4) GO(7, 4)
+  }
+#undef GO
+  if (parts > 1) launch_gemm_merge(y, part, (long)M * N, parts, false, stream);
+}
+
+}  // namespace
+
+// M >= 1, N % 128 == 0, K % 128 == 0; int8: plan of gemm_panel_plan, its parts [parts, M, N]
+void launch_gemm_block_q(__hip_bfloat16* y, float* part, const __hip_bfloat16* x,
+                         const unsigned char* w, const float* scale, int qbits, int M, int N,
+                         int K, int plan, hipStream_t stream) {
+  if (qbits == 4)
     launch_block<4>(y, x, w, scale, M, N, K, stream);
+  else if (plan > 1)
+    launch_panel(y, part, x, w, scale, M, N, K, plan, stream);
+  else
+    launch_block<8>(y, x, w, scale, M, N, K, stream);
 }
 
 // total = N * K, K % 128 == 0

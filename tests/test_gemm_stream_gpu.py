@@ -83,7 +83,7 @@ def test_rounded(qbits, m, n, k):
 
 @pytest.mark.parametrize("qbits", [8, 4])
 @pytest.mark.parametrize("m", [65, 127, 128, 129, 301, 460, 900])
-# blocks for the choices of tile: narrow, 64 wide, 128 wide, and many (the largest tiles:
+# blocks for the choices of tile: narrow, 64 wide, 128 wide, and many (more of them:
 # test_rounded_largest_tiles)
 @pytest.mark.parametrize(("n", "k"), [(128, 128), (512, 384), (4096, 256), (8192, 640),
                                       (36864, 256)])
@@ -232,7 +232,7 @@ def test_parts_of_k(m, n, k):
 
 @pytest.mark.parametrize("m", [1025, 1041])
 def test_rounded_largest_tiles(m):
-    """Wide matrices of few inputs, past 4096 blocks: 128 x 128 in int8."""
+    """Wide matrices of few inputs, past 4096 blocks of 64 x 128."""
     _need()
     from vllm_tgis_adapter_amd import ops
 
@@ -241,4 +241,24 @@ def test_rounded_largest_tiles(m):
     x, w = _x(m, k, 24), _x(n, k, 25)
     wq, scale = ops.quantize_weight(w, 8)
     exact = (wq.double() * scale.double()[:, None]).t()
+    _check(ops.linear_quant(x, wq, scale, 8), x.double() @ exact, x.double().abs() @ exact.abs())
+
+
+# every panel with whole K and with K cut over workgroups, evenly and unevenly, last panels
+# with one row and nearly full
+@pytest.mark.parametrize(("m", "n", "k", "panel", "parts"), [
+    (321, 128, 128, 0, 1), (65, 128, 2176, 0, 4), (161, 1024, 4096, 0, 5), (65, 28672, 384, 1, 1),
+    (65, 6144, 4096, 1, 5), (321, 8192, 128, 2, 1), (161, 2048, 4224, 2, 6), (511, 4096, 128, 3, 1),
+    (127, 2048, 6272, 3, 7), (511, 16384, 128, 4, 1), (511, 4096, 14336, 4, 4),
+    (97, 28672, 384, 5, 1), (97, 6144, 4096, 5, 5), (129, 28672, 384, 6, 1), (257, 4096, 8192, 6, 4),
+    (1199, 8192, 128, 7, 1), (301, 6144, 8192, 7, 5)])
+def test_int8_panels(m, n, k, panel, parts):
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    assert m <= ops._quant_rows(8, n, k)
+    assert ops._C.gemm_panel_plan(m, n, k) == (panel + 1) << 8 | parts
+    x, w = _x(m, k, 26), _x(n, k, 27)
+    wq, scale = ops.quantize_weight(w, 8)
+    exact = (wq.double() * scale.double()[:, None]).t().contiguous()
     _check(ops.linear_quant(x, wq, scale, 8), x.double() @ exact, x.double().abs() @ exact.abs())
