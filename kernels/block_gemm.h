@@ -32,6 +32,12 @@ template <int N> DEVINLINE void wait_loads() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0f70);
 }
 
+// vmcnt(N) and lgkmcnt(0)
+template <int N> DEVINLINE void wait_loads_and_reads() {
+  static_assert(N < 64, "vmcnt has six bits");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0070);
+}
+
 // The waves meet; loads on their way to LDS stay on their way (a fence would wait for
 // all of them).
 DEVINLINE void meet() {
@@ -40,13 +46,13 @@ DEVINLINE void meet() {
   asm volatile("" ::: "memory");
 }
 
-// 4 GB from a wave-uniform address on
-DEVINLINE __amdgpu_buffer_rsrc_t resource(const void* from) {
+// 4 GB (or less) from a wave-uniform address on
+DEVINLINE __amdgpu_buffer_rsrc_t resource(const void* from, unsigned size = 0xffffffff) {
   const unsigned long long at = reinterpret_cast<unsigned long long>(from);
   const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)at);
   const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(at >> 32));
   return __builtin_amdgcn_make_buffer_rsrc(
-      reinterpret_cast<void*>((unsigned long long)hi << 32 | lo), 0, 0xffffffff, 0x00027000);
+      reinterpret_cast<void*>((unsigned long long)hi << 32 | lo), 0, size, 0x00027000);
 }
 
 // 16 (4) bytes a lane from `from` + offset (+ the uniform ahead) to lds + 16 (4) lane.

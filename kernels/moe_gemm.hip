@@ -11,15 +11,18 @@
 // sorted rows need not exist: with a list of rows (x_rows) row r is x[x_rows[r]].
 //
 // Few rows an expert: bound by the bytes of W, the streaming kernel of gemm_stream.h.
-// More: block_gemm.h's tiles; the gated form takes half of a tile's columns from each
-// half of W, arranged so that a wave holds the gate and the up sum of the same output.
+// More: tiles of 128 x 128 by block_gemm.h, from 250 rows an expert on of 256 x 256 by
+// ring_gemm.h; the gated form takes half of a tile's columns from each half of W, arranged
+// so that a wave holds the gate and the up sum of the same output.
 //
 // Measured, 8 experts of 14336 x 4096 (two experts a token, MI355X): a layer's three
-// products and its routing, 33 tokens 723 -> 452 us (4.7 -> 6.2 TB/s), 2949 tokens 3164 ->
-// 1920 us (0.66 -> 1.08 PFLOP/s).
+// products and its routing, 33 tokens 723 -> 452 us (4.7 -> 6.2 TB/s), 2949 tokens 1950 (256 x
+// 256 by block_gemm.h) -> 1707 us (1.22 PFLOP/s; the second product's 400 tiles are 1.6 rounds
+// of 256 CUs).
 
 #include "block_gemm.h"
 #include "gemm_stream.h"
+#include "ring_gemm.h"
 
 namespace {
 
@@ -85,6 +88,56 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void moe_block_kernel(
 }
 
 template <int MODE>
+__global__ __launch_bounds__(256, 1) void moe_ring_kernel(
+    __hip_bfloat16* __restrict__ y,        // [T, N]
+    const __hip_bfloat16* __restrict__ x,  // [T, K] sorted by expert, or what segs.rows lists
+    const __hip_bfloat16* __restrict__ w,  // [E, (gated ? 2 N : N), K]
+    const moe::Segments segs, const int N, const int K, const float limit) {
+  using R = ring_gemm::Ring<256, 256, 2, 2, 4>;
+  constexpr bool GATED = moe::gated(MODE);
+  constexpr int COLS = GATED ? 128 : 256;          // outputs of a block
+  constexpr int OUT = GATED ? 4 : 8;               // output tiles of a wave
+  __shared__ __align__(16) char lds[R::kLds];
+
+  const moe::Tile at = moe::find_tile(segs, 256, N / COLS);
+  if (at.rows == 0) return;
+  const int n0 = at.n * COLS;
+  const unsigned row_bytes = K * 2;
+  f32x4_t acc[R::kTM][R::kTN];
+  R::clear(acc);
+  R::run(acc, lds, reinterpret_cast<const char*>(x),
+         reinterpret_cast<const char*>(w + ((long)at.expert * (GATED ? 2 : 1) * N + n0) * K), K,
+         // rows past the segment: its last one, whose results are not written
+         [&](int r) {
+           const int row = at.row0 + min(r, at.rows - 1);
+           return (segs.rows != nullptr ? segs.rows[row] : row) * row_bytes;
+         },
+         [&](int r) {   // a wave's output tiles of gates, then of the other half
+           const int wave = r / 128, in = r % 128;
+           const int half = in / (OUT * 16);
+           return (half * N + wave * (OUT * 16) + R::out_col(in % (OUT * 16))) * row_bytes;
+         });
+
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int col = lane & 15, quad = lane >> 4, wm = wave / 2, wn = wave % 2;
+#pragma unroll
+  for (int i = 0; i < R::kTM; ++i) {
+    const int m = (wm * R::kTM + i) * 16 + col;
+    if (m >= at.rows) continue;
+    __hip_bfloat16* to = y + (long)(at.row0 + m) * N + n0 + wn * OUT * 16 + quad * 8;
+#pragma unroll
+    for (int j = 0; j < OUT; j += 2) {
+      union { __hip_bfloat16 h[8]; uint4 u; } o;
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+        o.h[r] = __float2bfloat16(moe::finish<MODE>(
+            acc[i][j + r / 4][r % 4], acc[i][(GATED ? OUT : 0) + j + r / 4][r % 4], limit));
+      *reinterpret_cast<uint4*>(to + j * 16) = o.u;
+    }
+  }
+}
+
+template <int MODE>
 void launch_mode(__hip_bfloat16* y, const __hip_bfloat16* x, const __hip_bfloat16* w,
                  const int* seg_off, const int* x_rows, int E, int N, int K, int T,
                  float limit, hipStream_t stream) {
@@ -105,6 +158,7 @@ void launch_mode(__hip_bfloat16* y, const __hip_bfloat16* x, const __hip_bfloat1
   //       (<2,2,2> 316, 197);  50: <4,4,2> 323, 173 (128 x 128: 351, 228);
   //   64: 128 x 128 349, 232 (<4,4,2> 480, 332);  125: 128 x 128 449, 299 (256 x 256: 458,
   //       335);  250: 256 x 256 609, 382 (128 x 128: 671, 480);  737: 1258, 726 (1442, 738).
+  // (256 x 256 there with block_gemm.h's loop; ring_gemm.h's takes a fifth less.)
   //
   // That is with even loads.  The streaming form's workgroups, a chunk of 64 rows an expert and
   // two a CU, fill whole rounds at usual widths, and a few experts with more rows start another
@@ -123,7 +177,9 @@ void launch_mode(__hip_bfloat16* y, const __hip_bfloat16* x, const __hip_bfloat1
   else if (mean <= 18 && moe::gated(MODE)) STREAM(2, 2, 2);
   else if (far || (mean <= 52 && !brim)) STREAM(4, 4, 2);
   else if (mean < 250 || N * cols % 256 != 0) BLOCK(128, 128, 2, 2, 2);
-  else BLOCK(256, 256, 2, 4, 2);
+  else
+    hipLaunchKernelGGL(moe_ring_kernel<MODE>, dim3(moe::max_blocks(T, E, 256, N * cols / 256)),
+                       dim3(256), 0, stream, y, x, w, segs, N, K, limit);
 #undef STREAM
 #undef BLOCK
 }
