@@ -42,9 +42,11 @@ int gemm_stream_parts(int qbits, int M, int N, int K, bool gated);
 void launch_rotary_cache(const long*, __hip_bfloat16*, const __hip_bfloat16*,
                          const __hip_bfloat16*, const __hip_bfloat16*, const float*, void*, void*,
                          const long*, int, int, int, int, long, long, long, bool, hipStream_t);
-int gemm_block_parts(int M, int N, int K);
-void launch_gemm_block(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hip_bfloat16*, int,
-                       int, int, int, hipStream_t);
+int gemm_ring_plan(int M, int N, int K, bool gated);
+bool gemm_ring_takes(int N, int K, int plan, bool gated);
+bool gemm_ring_wins(long M, long N, long K, bool gated);
+void launch_gemm_ring(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hip_bfloat16*, int,
+                      int, int, int, bool, hipStream_t);
 void launch_gemm_stream(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hip_bfloat16*,
                         int, int, int, int, hipStream_t);
 bool gemm_row_fits(int qbits, int K);
@@ -329,6 +331,10 @@ float* stream_parts(torch::Tensor& space, const torch::Tensor& x, int parts, int
   return space.data_ptr<float>();
 }
 
+bool on16(const torch::Tensor& t);
+void run_ring(torch::Tensor& y, const torch::Tensor& x, const torch::Tensor& w, int64_t M,
+              int64_t N, int64_t K, bool gated, int plan);
+
 void gemm_skinny(torch::Tensor y, torch::Tensor x, torch::Tensor w) {
   const int M = x.size(0);
   const int K = x.size(1);
@@ -340,6 +346,10 @@ void gemm_skinny(torch::Tensor y, torch::Tensor x, torch::Tensor w) {
   TORCH_CHECK(w.size(1) == K && y.size(0) == M && y.size(1) == N);
   torch::Tensor part;
   if (M <= 64) {
+    if (gemm_ring_wins(M, N, K, false) && on16(x) && on16(w) && on16(y)) {
+      run_ring(y, x, w, M, N, K, false, gemm_ring_plan(M, N, K, false));
+      return;
+    }
     const int parts = gemm_stream_parts(16, M, N, K, false);
     launch_gemm_stream(ptr<__hip_bfloat16>(y), stream_parts(part, x, parts, (int64_t)M * N),
                        cptr<__hip_bfloat16>(x), cptr<__hip_bfloat16>(w), M, N, K, parts,
@@ -554,28 +564,42 @@ void lora_bgmv(torch::Tensor out, torch::Tensor x, torch::Tensor a_stack,
   });
 }
 
-// y = x w^T by large tiles, K cut over workgroups
-void gemm_block(torch::Tensor y, torch::Tensor x, torch::Tensor w) {
+bool on16(const torch::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+
+// checked: y = x w^T, or the gated product, by gemm_ring.hip's tiles
+void run_ring(torch::Tensor& y, const torch::Tensor& x, const torch::Tensor& w, int64_t M,
+              int64_t N, int64_t K, bool gated, int plan) {
+  torch::Tensor part;
+  launch_gemm_ring(ptr<__hip_bfloat16>(y), stream_parts(part, x, plan & 15, M * N),
+                   cptr<__hip_bfloat16>(x), cptr<__hip_bfloat16>(w), (int)M, (int)N, (int)K, plan,
+                   gated, current_stream());
+}
+
+// y = x w^T, or silu(x wg^T) * (x wu^T) for w = [wg; wu], by large tiles; plan: as
+// gemm_ring_plan gives it, 0: that one
+void gemm_ring(torch::Tensor y, torch::Tensor x, torch::Tensor w, bool gated, int64_t plan) {
   for (const auto& t : {y, x, w})
     TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::ScalarType::BFloat16 &&
                 t.is_contiguous() && t.dim() == 2);
   const int64_t M = x.size(0), K = x.size(1), N = y.size(1);
-  TORCH_CHECK(y.size(0) == M && w.size(0) == N && w.size(1) == K);
+  TORCH_CHECK(y.size(0) == M && w.size(0) == (gated ? 2 : 1) * N && w.size(1) == K);
   TORCH_CHECK(N % 128 == 0 && K % 64 == 0 && M < (1 << 24) && N < (1 << 24) && K < (1 << 23));
-  // both reach LDS in 16-byte pieces
-  TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
-              reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0);
+  TORCH_CHECK(!gated || (N + 128) * K * 2 < (int64_t)1 << 32, "W is found by 32 bits");
+  // x and w reach LDS, y memory, in 16-byte pieces
+  TORCH_CHECK(on16(x) && on16(w) && on16(y));
   if (M == 0 || N == 0) return;
   if (K == 0) {
     y.zero_();
     return;
   }
-  const int parts = gemm_block_parts((int)M, (int)N, (int)K);
-  torch::Tensor part;
-  if (parts > 1) part = at::empty({parts, M, N}, x.options().dtype(at::ScalarType::Float));
-  launch_gemm_block(ptr<__hip_bfloat16>(y), parts > 1 ? part.data_ptr<float>() : nullptr,
-                    cptr<__hip_bfloat16>(x), cptr<__hip_bfloat16>(w), (int)M, (int)N, (int)K,
-                    parts, current_stream());
+  if (plan == 0) plan = gemm_ring_plan((int)M, (int)N, (int)K, gated);
+  TORCH_CHECK(gemm_ring_takes((int)N, (int)K, (int)plan, gated), "no such plan");
+  run_ring(y, x, w, M, N, K, gated, (int)plan);
+}
+
+// y = x w^T by large tiles, K cut over workgroups
+void gemm_block(torch::Tensor y, torch::Tensor x, torch::Tensor w) {
+  gemm_ring(y, x, w, false, 0);
 }
 
 // bf16: out[t, start_p ...] += scale · B_p A_p x[t] for up to three projections of x, whose
@@ -804,7 +828,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sample_argmax", &sample_argmax,
         "fused temperature/gumbel-race sampling + greedy argmax (CDNA4)");
   m.def("rotary_cache", &rotary_cache, "rotation of q and k with the cache write");
-  m.def("gemm_block", &gemm_block, "product of more than 64 rows, large tiles");
+  m.def("gemm_block", &gemm_block, "product of many rows, large tiles");
+  m.def("gemm_ring", &gemm_ring, "product of many rows, large tiles, also gated", py::arg("y"),
+        py::arg("x"), py::arg("w"), py::arg("gated") = false, py::arg("plan") = 0);
+  m.def("gemm_ring_wins", &gemm_ring_wins, "whether the large tiles are the faster product");
   m.def("lora_delta", &lora_delta,
         "bf16 multi-LoRA of up to three projections of one input");
   m.def("lora_slots", &lora_slots, "adapter slot of every token");

@@ -148,9 +148,14 @@ struct Ring {
       for (int q = 0; q < kProducts; ++q) {
         const int ks = q / (kHM * kHN), i = q / kHN % kHM, jj = q % kHN;
         const int j = i % 2 ? kHN - 1 - jj : jj;
-        if (q % 2 == 0 && q / 2 < reads) read(q / 2);
+#pragma unroll
+        for (int r = 0; r < reads; ++r)   // in the first half of the products, if they fit
+          if (r * (2 * reads > kProducts ? kProducts : kProducts / 2) / reads == q) read(r);
         const int each = kProducts / (last - first);
-        if (q % each == each / 2 + 1 && first + q / each < last) ask(first + q / each);
+#pragma unroll
+        for (int l = first; l < last; ++l)
+          if (min((l - first) * kProducts / (last - first) + each / 2 + 1, kProducts - 1) == q)
+            ask(l);
         multiply(acc[i0 + i][j0 + j], fb[ks * kHN + j], fa[ks * kHM + i]);
         if (q % 2 == 1) __builtin_amdgcn_sched_barrier(0);
       }

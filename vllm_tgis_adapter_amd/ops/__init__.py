@@ -240,7 +240,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
     roofline (tools/gemm_bench.py); the hand-written MFMA kernel streams the
     weight matrix once with waves splitting K in-workgroup.  Larger M stays
     on hipBLASLt (VTA_GEMM_MAX_M raises the cutover for experiments) but for
-    the rows and inputs of ``_block_rows``.
+    the rows and inputs of ``_block_rows`` and where ``gemm_ring_wins``
+    (gemm_ring.hip) says that the tiles here are faster.
     """
     max_m = int(os.environ.get("VTA_GEMM_MAX_M", "64"))
     tile_max_m = int(os.environ.get("VTA_GEMM_TILE_MAX_M", "0"))
@@ -274,6 +275,13 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
                 (m, weight.shape[0]), dtype=x.dtype, device=x.device
             )
             _C.gemm_block(out, x, weight)
+            return out
+        if (m > max(max_m, 64) and _C.gemm_ring_wins(m, weight.shape[0], x.shape[1], False)
+                and _plain_tensors(x, weight)):
+            out = torch.empty(
+                (m, weight.shape[0]), dtype=x.dtype, device=x.device
+            )
+            _C.gemm_ring(out, x, weight)
             return out
     return torch.nn.functional.linear(x, weight, bias)
 
@@ -408,7 +416,7 @@ def gated_mlp_up(x: torch.Tensor, w13: torch.Tensor) -> torch.Tensor | None:
     max_m = int(os.environ.get("VTA_GEMM_MAX_M", "64"))
     if (
         x.dim() == 2
-        and 1 <= x.shape[0] <= max_m
+        and x.shape[0] >= 1
         and x.dtype == torch.bfloat16
         and w13.dtype == torch.bfloat16
         and w13.shape[0] % 256 == 0
@@ -417,10 +425,16 @@ def gated_mlp_up(x: torch.Tensor, w13: torch.Tensor) -> torch.Tensor | None:
         and w13.is_contiguous()
         and _native(x)
     ):
-        inter = w13.shape[0] // 2
-        out = torch.empty((x.shape[0], inter), dtype=x.dtype, device=x.device)
-        _C.gemm_skinny_gated(out, x, w13)
-        return out
+        rows, inter = x.shape[0], w13.shape[0] // 2
+        if rows <= max_m:
+            out = torch.empty((rows, inter), dtype=x.dtype, device=x.device)
+            _C.gemm_skinny_gated(out, x, w13)
+            return out
+        if (rows > 64 and _C.gemm_ring_wins(rows, inter, x.shape[1], True)
+                and _plain_tensors(x, w13)):
+            out = torch.empty((rows, inter), dtype=x.dtype, device=x.device)
+            _C.gemm_ring(out, x, w13, True)
+            return out
     return None
 
 
