@@ -8,35 +8,34 @@
 // silu_and_mul: out[t, i] = silu(x[t, i]) * x[t, d + i]
 // ---------------------------------------------------------------------------
 
+// grid (rows, pieces of a row): a vector a thread, so that a few rows are not a chain of
+// loads (61 rows of 14336: 5.4 -> 4.1 us)
 template <typename T>
-__global__ void silu_and_mul_kernel(
+__global__ __launch_bounds__(256) void silu_and_mul_kernel(
     T* __restrict__ out,        // [rows, d]
     const T* __restrict__ x,    // [rows, 2*d]
     const int d) {
   constexpr int V = Vec16<T>::kElems;
-  const int row = blockIdx.x;
+  const int row = blockIdx.x, i = (blockIdx.y * 256 + threadIdx.x) * V;
+  if (i >= d) return;
   const T* a_row = x + (long)row * 2 * d;
-  const T* b_row = a_row + d;
-  T* out_row = out + (long)row * d;
-  for (int i = threadIdx.x * V; i < d; i += blockDim.x * V) {
-    Vec16<T> a = load16(a_row + i);
-    Vec16<T> b = load16(b_row + i);
+  Vec16<T> a = load16(a_row + i);
+  Vec16<T> b = load16(a_row + d + i);
 #pragma unroll
-    for (int j = 0; j < V; ++j) {
-      float av = ScalarOps<T>::to_f32(a.data[j]);
-      float bv = ScalarOps<T>::to_f32(b.data[j]);
-      float s = av / (1.f + __expf(-av));
-      a.data[j] = ScalarOps<T>::from_f32(s * bv);
-    }
-    store16(out_row + i, a);
+  for (int j = 0; j < V; ++j) {
+    float av = ScalarOps<T>::to_f32(a.data[j]);
+    float bv = ScalarOps<T>::to_f32(b.data[j]);
+    float s = av / (1.f + __expf(-av));
+    a.data[j] = ScalarOps<T>::from_f32(s * bv);
   }
+  store16(out + (long)row * d + i, a);
 }
 
 template <typename T>
 void launch_silu_and_mul(T* out, const T* x, int rows, int d, hipStream_t s) {
-  int threads = 256;
-  hipLaunchKernelGGL(silu_and_mul_kernel<T>, dim3(rows), dim3(threads), 0, s,
-                     out, x, d);
+  constexpr int kPiece = 256 * Vec16<T>::kElems;
+  hipLaunchKernelGGL(silu_and_mul_kernel<T>, dim3(rows, (d + kPiece - 1) / kPiece), dim3(256), 0,
+                     s, out, x, d);
 }
 
 // ---------------------------------------------------------------------------

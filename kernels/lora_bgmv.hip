@@ -17,7 +17,7 @@
 // read and write of out.
 //
 // Layers of 4096 wide rows, 61 tokens of 4 adapters of rank 16: 7 + 7 launches of 25 and
-// 5 us were 4 + 4 of 4.4 and 6.3.  2048 tokens: shrink 23 us, expand into 4096 columns 14
+// 5 us were 4 + 4 of 4.6 and 4.0 to 7.8.  2048 tokens: shrink 23 us, expand into 4096 columns 14
 // and into 28672 102, where reading and writing out takes 51.
 //
 // f32 and f16: one token per workgroup in both,
@@ -231,7 +231,9 @@ __global__ __launch_bounds__(64 * kShrinkWaves) void lora_shrink_tile_kernel(
   }
 }
 
-// grid (ceil(V / 256), ceil(T / TOKENS))
+// grid (ceil(V / 256), ceil(T / TOKENS)).  Few tokens are a chain of latencies: what was in
+// out, the cuts' sums and, where they fit, the rows of B for all tokens are asked for at once
+// (61 tokens, rank 16, 4096 columns: 6.5 -> 4.0 us).
 template <int R, int TOKENS>
 __global__ __launch_bounds__(256) void lora_expand_tile_kernel(
     __hip_bfloat16* __restrict__ out,            // [T, out_w]
@@ -239,47 +241,63 @@ __global__ __launch_bounds__(256) void lora_expand_tile_kernel(
     const __hip_bfloat16* __restrict__ b_stack,  // [L, V, R]
     const int* __restrict__ slots, const float* __restrict__ scales, const LoraCols cols,
     const int T, const int PR, const int V, const int out_w, const int cuts) {
+  constexpr bool AHEAD = TOKENS * R <= 64;
   __shared__ float sums[TOKENS][3 * R];
-  __shared__ int own[TOKENS];
   const int t0 = blockIdx.y * TOKENS, v = blockIdx.x * 256 + threadIdx.x;
   const int tokens = min(TOKENS, T - t0);
-  if (threadIdx.x < TOKENS)
-    own[threadIdx.x] = threadIdx.x < tokens ? slots[t0 + threadIdx.x] : -1;
-  __syncthreads();
+  int own[TOKENS];
+#pragma unroll
+  for (int t = 0; t < TOKENS; ++t)
+    own[t] = __builtin_amdgcn_readfirstlane(t < tokens ? slots[t0 + t] : -1);
+  const int p = v < cols.end[0] ? 0 : v < cols.end[1] ? 1 : 2;
+  __hip_bfloat16* o = out + (long)t0 * out_w + v + cols.shift[p];
+  __hip_bfloat16 was[TOKENS];
+  Vec16<__hip_bfloat16> b[AHEAD ? TOKENS : 1][R / 8];
+  float scale[TOKENS];
+#pragma unroll
+  for (int t = 0; t < TOKENS; ++t) {
+    if (own[t] < 0) continue;
+    scale[t] = scales[own[t]];
+    if (v >= V) continue;
+    was[t] = o[(long)t * out_w];
+    if constexpr (AHEAD) {
+#pragma unroll
+      for (int j = 0; j < R / 8; ++j) b[t][j] = load16(b_stack + ((long)own[t] * V + v) * R + j * 8);
+    }
+  }
+  // (tokens without an adapter: whatever is there, which is not used)
   for (int i = threadIdx.x; i < tokens * PR; i += 256) {
-    const int t = i / PR;
     float s = 0.f;
-    if (own[t] >= 0)
-      for (int c = 0; c < cuts; ++c) s += tmp[((long)c * T + t0) * PR + i];
-    sums[t][i % PR] = s;
+    for (int c0 = 0; c0 < cuts; c0 += 8) {
+      float part[8];
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+        part[c] = tmp[((long)min(c0 + c, cuts - 1) * T + t0) * PR + i];
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+        if (c0 + c < cuts) s += part[c];
+    }
+    sums[i / PR][i % PR] = s;
   }
   __syncthreads();
   if (v >= V) return;
-  const int p = v < cols.end[0] ? 0 : v < cols.end[1] ? 1 : 2;
-  __hip_bfloat16* o = out + (long)t0 * out_w + v + cols.shift[p];
-  float was[TOKENS];
-#pragma unroll
-  for (int t = 0; t < TOKENS; ++t)
-    was[t] = t < tokens ? __bfloat162float(o[(long)t * out_w]) : 0.f;
-
-  Vec16<__hip_bfloat16> b[R / 8];
-  float scale = 0.f;
   int cur = -1;
 #pragma unroll
   for (int t = 0; t < TOKENS; ++t) {
-    const int slot = __builtin_amdgcn_readfirstlane(own[t]);
-    if (slot < 0) continue;
-    if (slot != cur) {
-      cur = slot;
-      scale = scales[slot];
+    if (own[t] < 0) continue;
+    if constexpr (!AHEAD) {
+      if (own[t] != cur) {
+        cur = own[t];
 #pragma unroll
-      for (int j = 0; j < R / 8; ++j) b[j] = load16(b_stack + ((long)slot * V + v) * R + j * 8);
+        for (int j = 0; j < R / 8; ++j) b[0][j] = load16(b_stack + ((long)cur * V + v) * R + j * 8);
+      }
     }
     float acc = 0.f;
 #pragma unroll
     for (int r = 0; r < R; ++r)
-      acc = __builtin_fmaf(__bfloat162float(b[r / 8].data[r % 8]), sums[t][p * R + r], acc);
-    o[(long)t * out_w] = __float2bfloat16(was[t] + acc * scale);
+      acc = __builtin_fmaf(__bfloat162float(b[AHEAD ? t : 0][r / 8].data[r % 8]),
+                           sums[t][p * R + r], acc);
+    o[(long)t * out_w] = __float2bfloat16(__bfloat162float(was[t]) + acc * scale[t]);
   }
 }
 

@@ -1,8 +1,91 @@
 // Fused RMSNorm kernels.
 // Memory-bound: one workgroup per row, 16-B vector loads (guide G13 — scalar
 // bf16 loads cost ~2x), sum-of-squares in f32, one pass read + one pass write.
+//
+// Of a step's rows what counts is the chain of latencies.  Rows of up to 8192 (f32: 4096)
+// stay in registers, CHUNKS vectors a thread, the weight is asked for with the row, and the
+// waves' sums meet once: 61 rows of 4096 4.3 -> 3.7 us, 8192 rows 44.5 -> 42.8 (they were read
+// again after the sum, which waited for the store and then for a cold weight).
 
 #include "common.h"
+
+namespace {
+
+constexpr int kThreads = 256;
+
+// the workgroup's sum, in one meeting
+DEVINLINE float sum_of_waves(float x, float* lds) {
+  x = wave_reduce_sum(x);
+  if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = x;
+  __syncthreads();
+  return (lds[0] + lds[1]) + (lds[2] + lds[3]);
+}
+
+// x <- rmsnorm(x + residual) w, residual <- x + residual, or (ADD false) out <- rmsnorm(x) w;
+// hidden is a multiple of a vector and at most CHUNKS of them a thread
+template <typename T, int CHUNKS, bool ADD>
+__global__ __launch_bounds__(kThreads) void rms_norm_row_kernel(
+    T* out, const T* x, T* residual, const T* __restrict__ weight, const float eps,
+    const int hidden) {
+  constexpr int V = Vec16<T>::kElems;
+  const long row = (long)blockIdx.x * hidden;
+  Vec16<T> v[CHUNKS], r[CHUNKS], w[CHUNKS];
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int i = (c * kThreads + threadIdx.x) * V;
+    if (i >= hidden) continue;
+    v[c] = load16(x + row + i);
+    if (ADD) r[c] = load16(residual + row + i);
+    w[c] = load16(weight + i);
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int i = (c * kThreads + threadIdx.x) * V;
+    if (i >= hidden) continue;
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      // the norm is of the rounded sum, which is what is stored
+      if (ADD)
+        v[c].data[j] = ScalarOps<T>::from_f32(ScalarOps<T>::to_f32(v[c].data[j]) +
+                                              ScalarOps<T>::to_f32(r[c].data[j]));
+      const float s = ScalarOps<T>::to_f32(v[c].data[j]);
+      ss += s * s;
+    }
+    if (ADD) store16(residual + row + i, v[c]);
+  }
+  __shared__ float lds[kThreads / 64];
+  const float inv = rsqrtf(sum_of_waves(ss, lds) / hidden + eps);
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int i = (c * kThreads + threadIdx.x) * V;
+    if (i >= hidden) continue;
+#pragma unroll
+    for (int j = 0; j < V; ++j)
+      v[c].data[j] = ScalarOps<T>::from_f32(ScalarOps<T>::to_f32(v[c].data[j]) * inv *
+                                            ScalarOps<T>::to_f32(w[c].data[j]));
+    store16(out + row + i, v[c]);
+  }
+}
+
+template <typename T, bool ADD>
+bool launch_row(T* out, const T* x, T* residual, const T* w, float eps, int rows, int hidden,
+                hipStream_t stream) {
+  constexpr int V = Vec16<T>::kElems;
+  if (hidden % V != 0) return false;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(rows), dim3(kThreads), 0, stream, out, x, residual, w, eps,
+                       hidden);
+    return true;
+  };
+  const int chunks = (hidden / V + kThreads - 1) / kThreads;
+  if (chunks <= 1) return go(rms_norm_row_kernel<T, 1, ADD>);
+  if (chunks <= 2) return go(rms_norm_row_kernel<T, 2, ADD>);
+  if (chunks <= 4) return go(rms_norm_row_kernel<T, 4, ADD>);
+  return false;
+}
+
+}  // namespace
 
 template <typename T>
 __global__ void rms_norm_kernel(
@@ -89,6 +172,7 @@ __global__ void fused_add_rms_norm_kernel(
 template <typename T>
 void launch_rms_norm(T* out, const T* in, const T* w, float eps, int rows,
                      int hidden, hipStream_t stream) {
+  if (launch_row<T, false>(out, in, nullptr, w, eps, rows, hidden, stream)) return;
   const int threads = 256;
   hipLaunchKernelGGL(rms_norm_kernel<T>, dim3(rows), dim3(threads), 0, stream,
                      out, in, w, eps, hidden);
@@ -97,6 +181,7 @@ void launch_rms_norm(T* out, const T* in, const T* w, float eps, int rows,
 template <typename T>
 void launch_fused_add_rms_norm(T* x, T* res, const T* w, float eps, int rows,
                                int hidden, hipStream_t stream) {
+  if (launch_row<T, true>(x, x, res, w, eps, rows, hidden, stream)) return;
   const int threads = 256;
   hipLaunchKernelGGL(fused_add_rms_norm_kernel<T>, dim3(rows), dim3(threads), 0,
                      stream, x, res, w, eps, hidden);
