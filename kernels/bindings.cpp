@@ -43,6 +43,8 @@ void launch_rotary_cache(const long*, __hip_bfloat16*, const __hip_bfloat16*,
                          const __hip_bfloat16*, const __hip_bfloat16*, const float*, void*, void*,
                          const long*, int, int, int, int, long, long, long, bool, hipStream_t);
 int gemm_ring_plan(int M, int N, int K, bool gated);
+void launch_gemm_ring_parts(__hip_bfloat16*, float*, const __hip_bfloat16*,
+                            const __hip_bfloat16*, int, int, int, int, hipStream_t);
 bool gemm_ring_takes(int N, int K, int plan, bool gated);
 bool gemm_ring_wins(long M, long N, long K, bool gated);
 void launch_gemm_ring(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hip_bfloat16*, int,
@@ -76,6 +78,11 @@ struct LoraCols {
   int end[3], shift[3];
 };
 int lora_shrink_cuts(int T, int K);
+void launch_lora_shrink_tiles(float*, const __hip_bfloat16*, const __hip_bfloat16*, const int*,
+                              int, int, int, int, int, hipStream_t);
+void launch_lora_finish(__hip_bfloat16*, const __hip_bfloat16*, const float*, const float*,
+                        const __hip_bfloat16*, const int*, const float*, const LoraCols&, int, int,
+                        int, int, int, int, int, bool, hipStream_t);
 void launch_lora_tiles(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hip_bfloat16*,
                        const __hip_bfloat16*, const int*, const float*, const LoraCols&, int,
                        int, int, int, int, int, int, int, hipStream_t);
@@ -602,6 +609,25 @@ void gemm_block(torch::Tensor y, torch::Tensor x, torch::Tensor w) {
   gemm_ring(y, x, w, false, 0);
 }
 
+LoraCols lora_cols(const std::vector<std::pair<int64_t, int64_t>>& spans, int V, int out_w) {
+  LoraCols cols;
+  const int P = spans.size();
+  int64_t v = 0;
+  for (int p = 0; p < 3; ++p) {
+    const auto& span = spans[p < P ? p : P - 1];
+    if (p < P) {
+      TORCH_CHECK(0 <= span.first && span.first <= span.second && span.second <= out_w);
+      cols.shift[p] = (int)(span.first - v);
+      v += span.second - span.first;
+    } else {
+      cols.shift[p] = cols.shift[P - 1];
+    }
+    cols.end[p] = (int)v;
+  }
+  TORCH_CHECK(v == V);
+  return cols;
+}
+
 // bf16: out[t, start_p ...] += scale · B_p A_p x[t] for up to three projections of x, whose
 // adapters' weights are stacked side by side: a [L, P R, K], b [L, V, R], spans[p] = (start,
 // end) in out's columns, V = the sum of their widths.
@@ -620,20 +646,7 @@ void lora_delta(torch::Tensor out, torch::Tensor x, torch::Tensor a, torch::Tens
               scales.numel() >= L);
   slots = slots.contiguous();
   scales = scales.contiguous();
-  LoraCols cols;
-  int64_t v = 0;
-  for (int p = 0; p < 3; ++p) {
-    const auto& span = spans[p < P ? p : P - 1];
-    if (p < P) {
-      TORCH_CHECK(0 <= span.first && span.first <= span.second && span.second <= out_w);
-      cols.shift[p] = (int)(span.first - v);
-      v += span.second - span.first;
-    } else {
-      cols.shift[p] = cols.shift[P - 1];
-    }
-    cols.end[p] = (int)v;
-  }
-  TORCH_CHECK(v == V);
+  const LoraCols cols = lora_cols(spans, V, out_w);
   if (T == 0 || V == 0 || L == 0) return;
   const int cuts = lora_shrink_cuts(T, K);
   auto tmp = at::empty({cuts, T, PR}, x.options().dtype(at::ScalarType::Float));
@@ -641,6 +654,62 @@ void lora_delta(torch::Tensor out, torch::Tensor x, torch::Tensor a, torch::Tens
                     cptr<__hip_bfloat16>(a), cptr<__hip_bfloat16>(b), slots.data_ptr<int>(),
                     scales.data_ptr<float>(), cols, T, L, R, PR, V, K, out_w, cuts,
                     current_stream());
+}
+
+// bf16: out = the product of x and its deltas as in lora_delta, for all W columns, gated: silu
+// of the first half of them times the second.  The product is given (y [T, W]) or made from w
+// [W, K] by gemm_ring.hip's tiles.
+void lora_product(torch::Tensor out, torch::Tensor x, c10::optional<torch::Tensor> w,
+                  c10::optional<torch::Tensor> y, torch::Tensor a, torch::Tensor b,
+                  torch::Tensor slots, torch::Tensor scales,
+                  const std::vector<std::pair<int64_t, int64_t>>& spans, bool gated) {
+  const int T = x.size(0), K = x.size(1), L = a.size(0), PR = a.size(1), R = b.size(2);
+  const int V = b.size(1), P = spans.size();
+  TORCH_CHECK(w.has_value() != y.has_value());
+  const torch::Tensor& given = w.has_value() ? *w : *y;
+  for (const auto& t : {out, x, a, b, given})
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::ScalarType::BFloat16 && t.is_contiguous() &&
+                on16(t));
+  const int W = w.has_value() ? w->size(0) : y->size(1);
+  TORCH_CHECK(P >= 1 && P <= 3 && PR == P * R && (R == 8 || R == 16 || R == 32 || R == 64));
+  TORCH_CHECK(a.size(2) == K && K % 8 == 0 && b.size(0) == L && L >= 1);
+  TORCH_CHECK(out.dim() == 2 && out.size(0) == T && W % 2 == 0 &&
+              out.size(1) == (gated ? W / 2 : W));
+  TORCH_CHECK(slots.is_cuda() && slots.scalar_type() == at::ScalarType::Int &&
+              slots.is_contiguous() && slots.numel() == T);
+  TORCH_CHECK(scales.is_cuda() && scales.scalar_type() == at::ScalarType::Float &&
+              scales.is_contiguous() && scales.numel() >= L);
+  for (int p = 1; p < P; ++p) TORCH_CHECK(spans[p - 1].second <= spans[p].first, "spans in order");
+  const LoraCols cols = lora_cols(spans, V, W);
+  if (T == 0) return;
+  const auto f32 = x.options().dtype(at::ScalarType::Float);
+  torch::Tensor base, part;
+  int parts = 0;
+  if (y.has_value()) {
+    TORCH_CHECK(y->size(0) == T);
+    base = *y;
+  } else {
+    TORCH_CHECK(w->size(1) == K && W % 128 == 0 && K % 64 == 0 && K > 0 && K < (1 << 23));
+    const int plan = gemm_ring_plan(T, W, K, false);
+    if ((plan & 15) > 1) {
+      parts = plan & 15;
+      part = at::empty({parts, T, W}, f32);
+    } else {
+      base = at::empty({T, W}, x.options());
+    }
+    launch_gemm_ring_parts(parts ? nullptr : ptr<__hip_bfloat16>(base),
+                           parts ? part.data_ptr<float>() : nullptr, cptr<__hip_bfloat16>(x),
+                           cptr<__hip_bfloat16>(*w), T, W, K, plan, current_stream());
+  }
+  const int cuts = lora_shrink_cuts(T, K);
+  auto tmp = at::empty({cuts, T, PR}, f32);
+  launch_lora_shrink_tiles(tmp.data_ptr<float>(), cptr<__hip_bfloat16>(x),
+                           cptr<__hip_bfloat16>(a), slots.data_ptr<int>(), T, L, PR, K, cuts,
+                           current_stream());
+  launch_lora_finish(ptr<__hip_bfloat16>(out), parts ? nullptr : cptr<__hip_bfloat16>(base),
+                     parts ? part.data_ptr<float>() : nullptr, tmp.data_ptr<float>(),
+                     cptr<__hip_bfloat16>(b), slots.data_ptr<int>(), scales.data_ptr<float>(),
+                     cols, T, R, PR, V, W, cuts, parts, gated, current_stream());
 }
 
 // slots[t] = the place of token_ids[t] among ids (64 at most), or -1
@@ -832,6 +901,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_ring", &gemm_ring, "product of many rows, large tiles, also gated", py::arg("y"),
         py::arg("x"), py::arg("w"), py::arg("gated") = false, py::arg("plan") = 0);
   m.def("gemm_ring_wins", &gemm_ring_wins, "whether the large tiles are the faster product");
+  m.def("lora_product", &lora_product, "a product with its LoRA deltas, also gated");
   m.def("lora_delta", &lora_delta,
         "bf16 multi-LoRA of up to three projections of one input");
   m.def("lora_slots", &lora_slots, "adapter slot of every token");

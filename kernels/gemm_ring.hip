@@ -214,3 +214,10 @@ void launch_gemm_ring(__hip_bfloat16* y, float* part, const __hip_bfloat16* x,
   else launch_plan<false>(y, part, x, w, M, N, K, plan, stream);
   if ((plan & 15) > 1) launch_gemm_merge(y, part, (long)M * N, plan & 15, false, stream);
 }
+
+// the same, plain; parts of K are left as they are
+void launch_gemm_ring_parts(__hip_bfloat16* y, float* part, const __hip_bfloat16* x,
+                            const __hip_bfloat16* w, int M, int N, int K, int plan,
+                            hipStream_t stream) {
+  launch_plan<false>(y, part, x, w, M, N, K, plan, stream);
+}

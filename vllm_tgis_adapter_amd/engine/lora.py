@@ -139,6 +139,51 @@ def _get_stacks(layer_idx: int, projs: list[tuple[str, int, int]], in_size: int,
     return _STACK_CACHE[key]
 
 
+def _batched(x: torch.Tensor) -> bool:
+    """Whether the batched kernels take the deltas of this input."""
+    from .. import ops
+
+    return (
+        CTX.token_slots is not None
+        and ops.native_enabled(x)
+        and x.is_contiguous()
+        and x.shape[1] % 8 == 0
+        and all(a.rank <= 64 for a in CTX.adapters.values())
+    )
+
+
+def lora_linear(
+    layer_idx: int,
+    projs: list[tuple[str, int, int]],
+    x: torch.Tensor,
+    weight: Optional[torch.Tensor],  # of the base linear, without a bias; None: not as it is
+    base,                            # () -> its product, for a weight that is None
+    gated: bool = False,
+) -> Optional[torch.Tensor]:
+    """The base linear's product and the adapters' deltas made together, gated: and silu of
+    the first half of its columns times the second.  None where that does not apply: the
+    caller has the product made, then apply_lora."""
+    if not (CTX.active and x.dim() == 2 and x.dtype == torch.bfloat16 and len(projs) <= 3
+            and _batched(x)):
+        return None
+    stacks = _get_stacks(layer_idx, projs, x.shape[1], x.dtype, x.device)
+    if stacks is None:
+        return None
+    from .. import ops
+
+    a_stack, b_stack, scales, spans = stacks
+    out = None
+    if weight is not None:
+        out = ops.lora_product(x, weight, None, a_stack, b_stack, CTX.token_slots, scales, spans,
+                               gated)
+    if out is None and gated:
+        y = base()
+        out = ops.lora_product(x, None, y, a_stack, b_stack, CTX.token_slots, scales, spans, True)
+        if out is None:
+            out = ops.silu_and_mul(apply_lora(layer_idx, projs, x, y))
+    return out
+
+
 def apply_lora(
     layer_idx: int,
     projs: list[tuple[str, int, int]],  # (proj name, out-slice start, out-slice end)
@@ -150,14 +195,7 @@ def apply_lora(
     from .. import ops
 
     # GPU: batched BGMV shrink/expand HIP kernels over the mixed batch (E12)
-    if (
-        CTX.token_slots is not None
-        and ops.native_enabled(x)
-        and x.is_contiguous()
-        and out.is_contiguous()
-        and x.shape[1] % 8 == 0
-        and all(a.rank <= 64 for a in CTX.adapters.values())
-    ):
+    if _batched(x) and out.is_contiguous():
         if x.dtype == torch.bfloat16 and len(projs) <= 3:
             stacks = _get_stacks(layer_idx, projs, x.shape[1], x.dtype, x.device)
             if stacks is not None:

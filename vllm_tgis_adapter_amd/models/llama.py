@@ -141,7 +141,7 @@ class LlamaMLP(nn.Module):
             h = ops.gated_mlp_up(x, self.gate_up.weight)
             if h is not None:
                 return self.down(h, lora=self._down_lora)
-        h = ops.silu_and_mul(self.gate_up(x, lora=self._gu_lora))
+        h = self.gate_up.gated(x, lora=self._gu_lora)
         return self.down(h, lora=self._down_lora)
 
     def row(self, hidden, residual, norm):

@@ -558,6 +558,33 @@ def lora_delta(
     _C.lora_delta(out, x, a_stack, b_stack, slots, scales, spans)
 
 
+def lora_product(
+    x: torch.Tensor,               # [T, K] bf16
+    weight: torch.Tensor | None,   # [W, K] bf16, or
+    y: torch.Tensor | None,        # [T, W], the product itself
+    a_stack: torch.Tensor, b_stack: torch.Tensor, slots: torch.Tensor, scales: torch.Tensor,
+    spans: list[tuple[int, int]],  # in order, as lora_delta
+    gated: bool = False,
+) -> torch.Tensor | None:
+    """A product and its LoRA deltas in one, gated: and silu of the first half of its columns
+    times the second.  None where the tiles of gemm_ring.hip are not what would run the
+    product, or where tensors do not suit."""
+    given = weight if y is None else y
+    rows, width = x.shape[0], given.shape[0 if y is None else 1]
+    if (not native_enabled(x) or given.dtype != torch.bfloat16 or not given.is_contiguous()
+            or width % 2 or not slots.is_contiguous() or not scales.is_contiguous()
+            or not _plain_tensors(x, given, a_stack, b_stack)):
+        return None
+    if y is None and not (_C.gemm_ring_wins(rows, width, x.shape[1], False)
+                          or (rows > 64 and rows in _block_rows(width, x.shape[1])
+                              and width % 128 == 0 and x.shape[1] % 64 == 0)):
+        return None
+    out = torch.empty((rows, width // 2 if gated else width), dtype=x.dtype, device=x.device)
+    _C.lora_product(out, x, None if y is not None else weight, y, a_stack, b_stack, slots, scales,
+                    spans, gated)
+    return out
+
+
 def lora_slots(token_ids: torch.Tensor, ids: tuple[int, ...]) -> torch.Tensor:
     """Place of every token's adapter id among ``ids``, -1 where it is none of them."""
     if native_enabled(token_ids) and token_ids.dtype == torch.int32 and len(ids) <= 64:

@@ -38,6 +38,11 @@ def _linear_fwd(mod: nn.Module, x: torch.Tensor) -> torch.Tensor:
     return ops.linear(x, mod.weight, mod.bias)
 
 
+def _as_it_is(mod: nn.Module) -> torch.Tensor | None:
+    """A layer's weight unless it is rounded."""
+    return mod.weight if getattr(mod, "quant_bits", None) is None else None
+
+
 def _init_weight(shape, dtype, std: float = 0.006) -> nn.Parameter:
     # Random-init path for synthetic benchmarking (BASELINE measures on
     # random-init weights); real checkpoints overwrite via load_weights.
@@ -87,13 +92,28 @@ class MergedColumnParallelLinear(nn.Module):
         self.bias = _init_weight((total,), dtype, std=0.0) if bias else None
 
     def forward(self, x: torch.Tensor, lora=None) -> torch.Tensor:
-        y = _linear_fwd(self, x)
         if lora is not None:
-            from ..engine.lora import apply_lora
+            from ..engine.lora import apply_lora, lora_linear
 
             layer_idx, projs = lora
-            apply_lora(layer_idx, projs, x, y)
-        return y
+            y = lora_linear(layer_idx, projs, x, _as_it_is(self) if self.bias is None else None,
+                            None)
+            if y is None:
+                y = apply_lora(layer_idx, projs, x, _linear_fwd(self, x))
+            return y
+        return _linear_fwd(self, x)
+
+    def gated(self, x: torch.Tensor, lora=None) -> torch.Tensor:
+        """silu of the first half of the outputs times the second."""
+        if lora is not None:
+            from ..engine.lora import lora_linear
+
+            layer_idx, projs = lora
+            h = lora_linear(layer_idx, projs, x, _as_it_is(self) if self.bias is None else None,
+                            lambda: _linear_fwd(self, x), gated=True)
+            if h is not None:
+                return h
+        return ops.silu_and_mul(self(x, lora=lora))
 
     def load_full_weights(self, ws: list[torch.Tensor]) -> None:
         r = get_tp_rank()
@@ -117,18 +137,22 @@ class RowParallelLinear(nn.Module):
         self.bias = _init_weight((out_size,), dtype, std=0.0) if bias else None
 
     def forward(self, x: torch.Tensor, lora=None) -> torch.Tensor:
-        qbits = getattr(self, "quant_bits", None)
-        if qbits is not None:
-            y = ops.linear_quant(x, self.weight_q, self.weight_scale, qbits)
-        else:
-            y = ops.linear(x, self.weight)
+        y = None
         if lora is not None:
             # delta added BEFORE the all-reduce: A is input-sharded, so the
             # per-rank partial deltas sum to the full LoRA delta
-            from ..engine.lora import apply_lora
+            from ..engine.lora import apply_lora, lora_linear
 
             layer_idx, projs = lora
-            apply_lora(layer_idx, projs, x, y)
+            y = lora_linear(layer_idx, projs, x, _as_it_is(self), None)
+        if y is None:
+            qbits = getattr(self, "quant_bits", None)
+            if qbits is not None:
+                y = ops.linear_quant(x, self.weight_q, self.weight_scale, qbits)
+            else:
+                y = ops.linear(x, self.weight)
+            if lora is not None:
+                apply_lora(layer_idx, projs, x, y)
         y = tp_all_reduce(y)
         if self.bias is not None:
             y = y + self.bias
