@@ -58,9 +58,10 @@ DEVINLINE __amdgpu_buffer_rsrc_t resource(const void* from, unsigned size = 0xff
 // 16 (4) bytes a lane from `from` + offset (+ the uniform ahead) to lds + 16 (4) lane.
 // Buffer loads: with a global one on its way the compiler has every read of LDS wait for
 // all reads before it.
+template <int HINT = 0>
 DEVINLINE void load_lds(char* lds, __amdgpu_buffer_rsrc_t from, unsigned offset, int ahead) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(
-      from, (__attribute__((address_space(3))) void*)lds, 16, offset, ahead, 0, 0);
+      from, (__attribute__((address_space(3))) void*)lds, 16, offset, ahead, 0, HINT);
 }
 DEVINLINE void load_lds4(char* lds, __amdgpu_buffer_rsrc_t from, unsigned offset, int ahead) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(

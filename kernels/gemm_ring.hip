@@ -22,12 +22,12 @@ namespace {
 using ring_gemm::f32x4_t;
 
 // grid (tiles of y, parts of K); part [parts, M, N] (gridDim.y > 1); depth: K of a part
-template <int BM, int BN, int SLOTS, int OCC, bool GATED>
+template <int BM, int BN, int SLOTS, int OCC, bool GATED, int HINT = 0>
 __global__ __launch_bounds__(256, OCC) void gemm_ring_kernel(
     __hip_bfloat16* __restrict__ y, float* __restrict__ part,
     const __hip_bfloat16* __restrict__ x, const __hip_bfloat16* __restrict__ w, const int M,
     const int N, const int K, const int depth) {
-  using R = ring_gemm::Ring<BM, BN, 2, 2, SLOTS>;
+  using R = ring_gemm::Ring<BM, BN, 2, 2, SLOTS, HINT>;
   constexpr int COLS = GATED ? BN / 2 : BN;              // outputs of a block
   constexpr int OUT = GATED ? R::kTN / 2 : R::kTN;       // output tiles of a wave
   __shared__ __align__(16) char lds[R::kLds];
@@ -91,15 +91,39 @@ constexpr Form kForms[] = {
     {128, 128, 2, 1.5, 0.3, 0.48, 1.00, 3.9, 0.20, 0.21},
     {64, 128, 2, 2.3, 0.0, 0.34, 0.77, 3.2, 0.21, 0.20},
 };
+// The fifth form, 64 x 64 for up to 64 rows, is not fitted: few_rows below.
+constexpr int kFew = 4, kForm4Cols = 64;
 
 struct Plan {
   int form, parts;
   double us;
 };
 
+// Up to 64 rows x is one tile and W comes by once: workgroups of 64 rows of W, as many as there
+// are CUs (K cut), or two a CU where that leaves a quarter of them idle or K stays long, and W
+// past the caches.  us, the streaming kernel | 64 x 128 by the model below | here, N x K, 24 |
+// 64 rows: 28672 x 4096 44.7 48.8 39.9 | 52.2 49.9 47.3; 4096 x 14336 26.8 27.7 24.1 | 37.3 29.4
+// 28.8; 6144 x 4096 15.9 15.4 14.8 | 21.6 17.3 18.1; 4096 x 4096 12.1 12.7 11.5 | 16.5 14.2 12.6;
+// 16384 x 2048 16.6 17.1 15.5 | 20.6 19.2 16.5; 8192 x 28672 83 83 75 | 101 90 96.  Workgroups 128,
+// 256, 512 at 8192 x 28672, 24 rows: 130, 90, 75; at 4096 x 14336 64, 128, 256, 512: 54, 33, 24, 27.
+int few_rows(int M, int N, int K) {
+  if (M > 64 || (M > 48 && K >= 8192 && (long)N * K > 80000000)) return 0;
+  const int cols = N / 64, tiles = K / 64;
+  int parts = 256 / cols;
+  if (parts < 1) parts = 1;
+  if (cols * parts < 192) parts = 512 / cols;
+  if (tiles / parts > 128 && cols * parts <= 256) parts *= 2;
+  if (parts > 8) parts = 8;
+  if (parts > tiles / 6) parts = tiles / 6;
+  if (parts < 1) parts = 1;
+  const int depth = (tiles + parts - 1) / parts;
+  return (tiles + depth - 1) / depth;
+}
+
 // The form and the parts of K (of six tiles at least) that the model gives the least time.  It
 // picks what is 3 % slower than the best of all at the mean of the measured sizes, 1 % gated.
 Plan plan_of(int M, int N, int K, bool gated) {
+  if (const int parts = gated ? 0 : few_rows(M, N, K)) return Plan{kFew, parts, 0.0};
   Plan best{0, 1, 1e30};
   const double cols = gated ? 2.0 * N : N, w_mb = cols * K * 2e-6;
   for (int f = 0; f < 4; ++f) {
@@ -126,12 +150,12 @@ Plan plan_of(int M, int N, int K, bool gated) {
   return best;
 }
 
-template <int BM, int BN, int SLOTS, int OCC, bool GATED>
+template <int BM, int BN, int SLOTS, int OCC, bool GATED, int HINT = 0>
 void launch_form(__hip_bfloat16* y, float* part, const __hip_bfloat16* x, const __hip_bfloat16* w,
                  int M, int N, int K, int parts, hipStream_t stream) {
   const long blocks = (M + BM - 1) / BM * (long)(N / (GATED ? BN / 2 : BN));
   const int depth = (K / 64 + parts - 1) / parts * 64;
-  hipLaunchKernelGGL((gemm_ring_kernel<BM, BN, SLOTS, OCC, GATED>),
+  hipLaunchKernelGGL((gemm_ring_kernel<BM, BN, SLOTS, OCC, GATED, HINT>),
                      dim3((blocks + 7) / 8 * 8, parts), dim3(256), 0, stream, y, part, x, w, M, N,
                      K, depth);
 }
@@ -144,7 +168,16 @@ void launch_plan(__hip_bfloat16* y, float* part, const __hip_bfloat16* x, const 
     case 0: launch_form<256, 256, 4, 1, GATED>(y, part, x, w, M, N, K, parts, stream); break;
     case 1: launch_form<128, 256, 4, 1, GATED>(y, part, x, w, M, N, K, parts, stream); break;
     case 2: launch_form<128, 128, 4, 2, GATED>(y, part, x, w, M, N, K, parts, stream); break;
-    default: launch_form<64, 128, 6, 2, GATED>(y, part, x, w, M, N, K, parts, stream);
+    case 3: launch_form<64, 128, 6, 2, GATED>(y, part, x, w, M, N, K, parts, stream); break;
+    default:
+      if constexpr (!GATED) {
+        // W that is read once and is large goes past the caches (24 rows: 28672 x 4096 46.4 ->
+        // 39.9 us, 8192 x 3584 15.6 -> 13.8, 4096 x 4096 11.5 -> 11.5; 64 rows 12.6 -> 13.5)
+        if (M <= 64 && (long)N * K >= 20000000)
+          launch_form<64, 64, 8, 2, false, 2>(y, part, x, w, M, N, K, parts, stream);
+        else
+          launch_form<64, 64, 8, 2, false>(y, part, x, w, M, N, K, parts, stream);
+      }
   }
 }
 
@@ -168,18 +201,18 @@ int gemm_ring_plan(int M, int N, int K, bool gated) {
 // Whether a plan is one: a tile's columns fit, no part of K is empty.
 bool gemm_ring_takes(int N, int K, int plan, bool gated) {
   const int form = plan >> 4, parts = plan & 15;
-  if (plan < 0 || form > 3 || parts < 1 || parts > (gated ? 1 : 8)) return false;
+  if (plan < 0 || form > (gated ? 3 : kFew) || parts < 1 || parts > (gated ? 1 : 8)) return false;
   const int depth = (K / 64 + parts - 1) / parts;
-  return (gated ? 2L : 1L) * N % kForms[form].bn == 0 && (K / 64 + depth - 1) / depth == parts;
+  const int bn = form == kFew ? kForm4Cols : kForms[form].bn;
+  return (gated ? 2L : 1L) * N % bn == 0 && (K / 64 + depth - 1) / depth == parts;
 }
 
 // Whether these tiles take a product from what would run it otherwise.  Time over that one's,
 // cold weights, N x K: rows.
-//  Against gemm_stream.hip's (up to 64 rows, where x costs it more than W does):
-//   4096 x 4096: 32 1.01, 48 0.85, 64 0.85; 6144 x 4096: 48 0.79, 64 0.86; 4096 x 14336: 24
-//   1.02, 48 0.88; 8192 x 8192: 24 1.19, 48 0.93; 12288 x 8192: 36 1.00, 64 0.92; not cut, 28672
-//   x 4096: 48 1.02, 64 0.95, 12288 x 4096: 64 1.22; 1024 x 8192: 17 0.85, 64 0.57;
-//   2048 x 2048: 32 1.24, 64 1.02; few columns and long K, 1280 and 2048 x 8192: 17 0.85 0.88.
+//  Against gemm_stream.hip's, 17 to 64 rows: 28672 x 4096 0.90 to 0.94; 4096 x 14336 0.77 to
+//   0.90; 4096 x 4096 17 0.98, 64 0.76; 512 x 4096 0.96 to 0.66; 3072 x 2048 17 1.08, 40 0.95, 64
+//   0.91; 2048 x 2048 32 1.12, 40 0.97; 12 rows: 6144 x 4096 1.08, 4096 x 4096 1.09, 28672 x 4096
+//   0.93.
 //  Against the library's:
 //   65 to 256 rows: 4096 x 4096 0.60 to 0.99; 6144 x 4096 0.76 to 1.00; 4096 x 14336 0.82 to
 //   0.97; 8192 x 8192 0.89 to 1.02; 2560 x 8192 0.54 to 0.90; 12288 and 14336 x 4096 and 8192
@@ -198,10 +231,9 @@ bool gemm_ring_wins(long M, long N, long K, bool gated) {
     const double library = 12.9 + sqrt(tf * tf + mb * mb) + 0.6e-6 * M * N;
     return plan_of(M, N, K, true).us < 0.92 * library;
   }
-  if (M <= 16 || N * K < 6000000) return false;
-  if (M <= 32) return 4 * N <= K;
-  if (M <= 64)   // K is cut, or one round is nearly full
-    return K >= 3584 && ((M > 48 && N >= 24576) || plan_of(M, N, K, false).parts > 1);
+  if (M <= 64)
+    return M > 16 && N * K >= 2000000 && (K >= 4096 || N * K >= 16000000 || M >= 40);
+  if (N * K < 6000000) return false;
   if (M <= 256) return K >= 3584 && N <= 10240;
   return M <= 1024 && 2 * K >= 7 * N;
 }

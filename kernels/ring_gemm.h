@@ -30,7 +30,8 @@ using block_gemm::f32x4_t;
 
 constexpr int kDepth = 64;   // inputs of a tile
 
-template <int BM, int BN, int WM, int WN, int SLOTS>
+// HINT: of the loads of B (2: not to be kept in the caches)
+template <int BM, int BN, int WM, int WN, int SLOTS, int HINT = 0>
 struct Ring {
   static constexpr int kWaves = WM * WN;
   static constexpr int kThreads = kWaves * 64;
@@ -110,7 +111,7 @@ struct Ring {
         block_gemm::load_lds(to + p * kWaves * 1024, block_gemm::resource(a, bytes),
                              a_off[ha][p < kAPass ? p : 0], tile * (kDepth * 2));
       else
-        block_gemm::load_lds(to + kABytes + (p - kAPass) * kWaves * 1024,
+        block_gemm::load_lds<HINT>(to + kABytes + (p - kAPass) * kWaves * 1024,
                              block_gemm::resource(b, bytes),
                              b_off[hb][p < kAPass ? 0 : p - kAPass], tile * (kDepth * 2));
     };

@@ -10,7 +10,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 # rows and columns of W of a form's tile
-FORMS = [(256, 256), (128, 256), (128, 128), (64, 128)]
+FORMS = [(256, 256), (128, 256), (128, 128), (64, 128), (64, 64)]
 
 
 @pytest.fixture(autouse=True)
@@ -39,15 +39,17 @@ def _check(got, x, w, gated):
     assert (err <= 2 ** -8 * s.abs() + off).all(), err.max().item()
 
 
-@pytest.mark.parametrize("form", range(4))
+@pytest.mark.parametrize("form", range(5))
 @pytest.mark.parametrize("gated", [False, True])
 @pytest.mark.parametrize("k", [64, 128, 448, 832])
 def test_forms(form, gated, k):
     from vllm_tgis_adapter_amd.ops import _C
 
     bm, bn = FORMS[form]
+    if gated and form == 4:
+        pytest.skip("plain only")
     for m in (1, bm - 1, bm, bm + 1, 9 * bm + 17):      # nine tiles: a band and one more
-        for cols in (1, 3):
+        for cols in (1, 2, 3):
             n = bn * cols if not gated else bn * cols // 2
             if n % 128:
                 continue
@@ -57,7 +59,7 @@ def test_forms(form, gated, k):
             _check(y, x, w, gated)
 
 
-@pytest.mark.parametrize("form", range(4))
+@pytest.mark.parametrize("form", range(5))
 @pytest.mark.parametrize(("parts", "k"), [(2, 128), (2, 192), (3, 448), (5, 2112), (8, 12352)])
 def test_parts(form, parts, k):
     from vllm_tgis_adapter_amd.ops import _C
@@ -73,17 +75,18 @@ def test_plans_that_are_none():
 
     x, w = _inputs(8, 128, 192)
     y = torch.empty((8, 128), dtype=torch.bfloat16, device="cuda")
-    for plan in (-1, 0x41, 0x20, 0x29, 0x24, 0x01):   # form, parts, empty parts, columns
+    for plan in (-1, 0x51, 0x20, 0x29, 0x24, 0x01):   # form, parts, empty parts, columns
         with pytest.raises(RuntimeError):
             _C.gemm_ring(y, x, w, False, plan)
 
 
 # first and last rows of the rule and the ones beside them: rows, N, K, whether it takes them
-LINES = [(32, 4096, 4096, False), (33, 4096, 4096, True), (64, 4096, 4096, True),
-         (64, 12288, 4096, False), (33, 512, 8192, False), (16, 2048, 8192, False), (17, 2048, 8192, True), (48, 28672, 4096, False),
-         (49, 28672, 4096, True), (256, 4096, 4096, True), (257, 4096, 4096, False),
-         (128, 4096, 3520, False), (65, 2048, 8192, True), (1024, 2048, 8192, True),
-         (1025, 2048, 8192, False)]
+LINES = [(16, 4096, 4096, False), (17, 4096, 4096, True), (64, 4096, 4096, True),
+         (33, 128, 8192, False), (17, 512, 4096, True), (39, 3072, 2048, False),
+         (40, 3072, 2048, True), (64, 8192, 28672, True), (64, 28672, 4096, True),
+         (17, 28672, 4096, True), (65, 28672, 4096, False), (256, 4096, 4096, True),
+         (257, 4096, 4096, False), (128, 4096, 3520, False), (65, 2048, 8192, True),
+         (1024, 2048, 8192, True), (1025, 2048, 8192, False)]
 
 
 @pytest.mark.parametrize(("m", "n", "k", "own"), LINES)
