@@ -11,95 +11,35 @@
 // sorted rows need not exist: with a list of rows (x_rows) row r is x[x_rows[r]].
 //
 // Few rows an expert: bound by the bytes of W, the streaming kernel of gemm_stream.h.
-// More: tiles of 128 x 128 by block_gemm.h, from 250 rows an expert on of 256 x 256 by
-// ring_gemm.h; the gated form takes half of a tile's columns from each half of W, arranged
-// so that a wave holds the gate and the up sum of the same output.
+// More: ring_gemm.h's tiles of 128 x 128 to 256 x 256; the gated form takes half of a tile's
+// columns from each half of W, arranged so that a wave holds the gate and the up sum of the
+// same output.
 //
 // Measured, 8 experts of 14336 x 4096 (two experts a token, MI355X): a layer's three
-// products and its routing, 33 tokens 723 -> 452 us (4.7 -> 6.2 TB/s), 2949 tokens 1950 (256 x
-// 256 by block_gemm.h) -> 1707 us (1.22 PFLOP/s; the second product's 400 tiles are 1.6 rounds
+// products and its routing, 33 tokens 723 -> 452 us (4.7 -> 6.2 TB/s), 2949 tokens 1950 (eight
+// waves on 256 x 256) -> 1707 us (1.22 PFLOP/s; the second product's 400 tiles are 1.6 rounds
 // of 256 CUs).
 
-#include "block_gemm.h"
 #include "gemm_stream.h"
 #include "ring_gemm.h"
 
 namespace {
 
-using block_gemm::Block;
-using block_gemm::f32x4_t;
+using ring_gemm::f32x4_t;
 
-template <int BM, int BN, int WM, int WN, int STAGES, int MODE>
-__global__ __launch_bounds__(WM * WN * 64, 1) void moe_block_kernel(
+template <int BM, int BN, int SLOTS, int OCC, int MODE>
+__global__ __launch_bounds__(256, OCC) void moe_ring_kernel(
     __hip_bfloat16* __restrict__ y,        // [T, N]
     const __hip_bfloat16* __restrict__ x,  // [T, K] sorted by expert, or what segs.rows lists
     const __hip_bfloat16* __restrict__ w,  // [E, (gated ? 2 N : N), K]
     const moe::Segments segs, const int N, const int K, const float limit) {
-  using B = Block<BM, BN, WM, WN, STAGES>;
+  using R = ring_gemm::Ring<BM, BN, 2, 2, SLOTS>;
   constexpr bool GATED = moe::gated(MODE);
-  constexpr int COLS = GATED ? BN / 2 : BN;        // outputs of a block
-  constexpr int WCOLS = BN / WN, HALF = WCOLS / 2; // W rows of a wave
-  static_assert(!GATED || B::kTN % 2 == 0, "gate and up tiles in pairs");
-  __shared__ __align__(16) char lds[B::kLds];
-
-  const moe::Tile at = moe::find_tile(segs, BM, N / COLS);
-  if (at.rows == 0) return;
-  const int n0 = at.n * COLS;
-  const unsigned row_bytes = K * 2;
-
-  f32x4_t acc[B::kTM][B::kTN];
-#pragma unroll
-  for (int i = 0; i < B::kTM; ++i)
-#pragma unroll
-    for (int j = 0; j < B::kTN; ++j) acc[i][j] = f32x4_t{};
-
-  const char* xa = reinterpret_cast<const char*>(x);
-  const char* wb =
-      reinterpret_cast<const char*>(w + ((long)at.expert * (GATED ? 2 : 1) * N + n0) * K);
-  B::run(acc, lds, xa, wb, K,
-         // rows past the segment: its last one, whose results are not written
-         [&](int r) {
-           const int row = at.row0 + min(r, at.rows - 1);
-           return (segs.rows != nullptr ? segs.rows[row] : row) * row_bytes;
-         },
-         [&](int r) {
-           if constexpr (!GATED) return r * row_bytes;
-           const int wave = r / WCOLS, in = r % WCOLS;
-           const int row = in < HALF ? wave * HALF + in : N + wave * HALF + in - HALF;
-           return row * row_bytes;
-         });
-
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int col = lane & 15, quad = lane >> 4;
-  const int wm = wave / WN, wn = wave % WN;
-  constexpr int OUT = GATED ? B::kTN / 2 : B::kTN;
-#pragma unroll
-  for (int i = 0; i < B::kTM; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = (wm * B::kTM + i) * 16 + quad * 4 + r;
-      if (m >= at.rows) continue;
-      __hip_bfloat16* to = y + (long)(at.row0 + m) * N + n0 + wn * OUT * 16 + col;
-#pragma unroll
-      for (int j = 0; j < OUT; ++j)
-        to[j * 16] = __float2bfloat16(
-            moe::finish<MODE>(acc[i][j][r], acc[i][GATED ? OUT + j : j][r], limit));
-    }
-}
-
-template <int MODE>
-__global__ __launch_bounds__(256, 1) void moe_ring_kernel(
-    __hip_bfloat16* __restrict__ y,        // [T, N]
-    const __hip_bfloat16* __restrict__ x,  // [T, K] sorted by expert, or what segs.rows lists
-    const __hip_bfloat16* __restrict__ w,  // [E, (gated ? 2 N : N), K]
-    const moe::Segments segs, const int N, const int K, const float limit) {
-  using R = ring_gemm::Ring<256, 256, 2, 2, 4>;
-  constexpr bool GATED = moe::gated(MODE);
-  constexpr int COLS = GATED ? 128 : 256;          // outputs of a block
-  constexpr int OUT = GATED ? 4 : 8;               // output tiles of a wave
+  constexpr int COLS = GATED ? BN / 2 : BN;              // outputs of a block
+  constexpr int OUT = GATED ? R::kTN / 2 : R::kTN;       // output tiles of a wave
   __shared__ __align__(16) char lds[R::kLds];
 
-  const moe::Tile at = moe::find_tile(segs, 256, N / COLS);
+  const moe::Tile at = moe::find_tile(segs, BM, N / COLS);
   if (at.rows == 0) return;
   const int n0 = at.n * COLS;
   const unsigned row_bytes = K * 2;
@@ -113,7 +53,7 @@ __global__ __launch_bounds__(256, 1) void moe_ring_kernel(
            return (segs.rows != nullptr ? segs.rows[row] : row) * row_bytes;
          },
          [&](int r) {   // a wave's output tiles of gates, then of the other half
-           const int wave = r / 128, in = r % 128;
+           const int wave = r / (R::kTN * 16), in = r % (R::kTN * 16);
            const int half = in / (OUT * 16);
            return (half * N + wave * (OUT * 16) + R::out_col(in % (OUT * 16))) * row_bytes;
          });
@@ -147,18 +87,22 @@ void launch_mode(__hip_bfloat16* y, const __hip_bfloat16* x, const __hip_bfloat1
   hipLaunchKernelGGL((gemm_stream::gemm_stream_kernel<16, MT, 1, WN, WK, MODE, true>),        \
                      dim3(moe::max_blocks(T, E, 16 * MT, N / (16 * WN))), dim3(64 * WN * WK), \
                      0, stream, y, nullptr, x, w, nullptr, 0, N, K, segs, limit)
-#define BLOCK(BM, BN, WM, WN, ST)                                                             \
-  hipLaunchKernelGGL((moe_block_kernel<BM, BN, WM, WN, ST, MODE>),                            \
-                     dim3(moe::max_blocks(T, E, BM, N * cols / BN)), dim3(WM * WN * 64), 0,   \
-                     stream, y, x, w, segs, N, K, limit)
+#define TILES(BM, BN, SLOTS, OCC)                                                             \
+  hipLaunchKernelGGL((moe_ring_kernel<BM, BN, SLOTS, OCC, MODE>),                             \
+                     dim3(moe::max_blocks(T, E, BM, N * cols / BN)), dim3(256), 0, stream, y, \
+                     x, w, segs, N, K, limit)
   // Rows an expert, us gated / plain of what is chosen and its neighbour (8 experts, 4096 in
   // and 14336 between; rows are spread at random):
   //    8: <1,1,4> 270, <1,2,2> 144 (<2,2,2> 271, <4,4,2> 143);
   //   17: <2,2,2> 278, <4,4,2> 144 (<4,4,2> 301, <2,2,2> 170);  25: <4,4,2> 305, 156
-  //       (<2,2,2> 316, 197);  50: <4,4,2> 323, 173 (128 x 128: 351, 228);
-  //   64: 128 x 128 349, 232 (<4,4,2> 480, 332);  125: 128 x 128 449, 299 (256 x 256: 458,
-  //       335);  250: 256 x 256 609, 382 (128 x 128: 671, 480);  737: 1258, 726 (1442, 738).
-  // (256 x 256 there with block_gemm.h's loop; ring_gemm.h's takes a fifth less.)
+  //       (<2,2,2> 316, 197);  52: <4,4,2> 335, 171 (128 x 128 333, 166).
+  // Tiles, 128 x 128 | 128 x 256 | 256 x 256, * is chosen:
+  //   56: 327* 336* - / 163* 215 -;  100: 347 345* 387 / 179* 235 248;  125: 421 395 403* / 295
+  //       244* 253;  200: 543 464 412* / 269 234* 285;  249: 629 591 505* / 391 426 311*;
+  //   400: 908 836 705* / 505 429 331*.
+  // and with 16 experts, 2048 in and between, where 128 x 256 are too few:
+  //   64: 59* 66 - / 33* 37 -;  125: 69* 79 74 / 42 41* 46;  200: 89 81 78* / 43 42* 50.
+  // (The eight-wave tiles before these took, gated / plain, 64: 357 / 227, 200: 529 / 269.)
   //
   // That is with even loads.  The streaming form's workgroups, a chunk of 64 rows an expert and
   // two a CU, fill whole rounds at usual widths, and a few experts with more rows start another
@@ -176,12 +120,18 @@ void launch_mode(__hip_bfloat16* y, const __hip_bfloat16* x, const __hip_bfloat1
   else if (mean <= 9) STREAM(1, 2, 2);
   else if (mean <= 18 && moe::gated(MODE)) STREAM(2, 2, 2);
   else if (far || (mean <= 52 && !brim)) STREAM(4, 4, 2);
-  else if (mean < 250 || N * cols % 256 != 0) BLOCK(128, 128, 2, 2, 2);
-  else
-    hipLaunchKernelGGL(moe_ring_kernel<MODE>, dim3(moe::max_blocks(T, E, 256, N * cols / 256)),
-                       dim3(256), 0, stream, y, x, w, segs, N, K, limit);
+  else if (N * cols % 256 != 0) TILES(128, 128, 5, 2);
+  else if (moe::gated(MODE)) {
+    if (mean > (K >= 4096 ? 110 : 150)) TILES(256, 256, 4, 1);
+    else if (mean > 52 && K >= 4096) TILES(128, 256, 4, 1);
+    else TILES(128, 128, 5, 2);
+  } else {
+    if (mean > 220) TILES(256, 256, 4, 1);
+    else if (mean > 110) TILES(128, 256, 4, 1);
+    else TILES(128, 128, 5, 2);
+  }
 #undef STREAM
-#undef BLOCK
+#undef TILES
 }
 
 }  // namespace

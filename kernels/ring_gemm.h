@@ -3,8 +3,8 @@
 //
 // Bound by the matrix unit and, before it, by the chip's power: the clock falls to 1.7 GHz
 // under it.  What counts is to keep the unit busy with as few bytes moved as possible:
-//  - four waves of 128 x 128 read 128 KB of LDS a tile of 64 inputs, eight of 128 x 64 (the
-//    loop of block_gemm.h) 192 KB; the sums fill all accumulation registers.
+//  - four waves of 128 x 128 read 128 KB of LDS a tile of 64 inputs, eight of 128 x 64 192 KB;
+//    the sums fill all accumulation registers.
 //  - Rows of 64 inputs, whole cache lines: with 32 (half lines; as much in flight, half of
 //    the registers' turnover) every byte is asked for in two requests and the same loop
 //    ran at 1.25 PFLOP/s instead of 1.5.
@@ -15,7 +15,7 @@
 //    products reads one half of an operand into the registers of one that is done with.
 //  - One barrier a half tile.  Reads and loads stand between the products in source order.
 // The accumulation registers are named in the products themselves (multiply below).
-// Measured alone, us, the library | block_gemm.h's 256 x 256 | here, 4 slots (5 slots):
+// Measured alone, us, the library | eight waves, two whole tiles in LDS | here, 4 slots (5):
 //   rows x N (K): 8192 x 28672 (4096) 1412 | 1483 | 1325 (1351); 8192 x 4096 (14336) 609 |
 //   722 | 618 (645); 8192 x 6144 (4096) 268 | 313 | 274 (286); 2949 x 28672 (4096) 531 | 600
 //   | 527 (549); 512 x 28672 (4096) 91 | 115 | 96 (101).

@@ -1,0 +1,45 @@
+"""Expert products by large tiles: rows an expert at each line of the rule that chooses them,
+uneven and empty segments, against float64."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# means below and above 52, 110, 150, 220, with edges of 128 and 256 rows
+COUNTS = [[52, 53], [53, 53], [129, 91], [111, 111], [0, 255, 45], [256, 45, 0], [151, 151],
+          [300, 140], [221, 221], [257, 0, 511]]
+
+
+@pytest.mark.parametrize("mode", ["plain", "silu", "relu2"])
+@pytest.mark.parametrize("counts", COUNTS, ids=str)
+@pytest.mark.parametrize(("n", "k"), [(128, 192), (512, 64), (256, 4096)])
+def test_tiles(mode, counts, n, k):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from vllm_tgis_adapter_amd import ops
+
+    g = torch.Generator("cuda").manual_seed(sum(counts) + n)
+    seg = torch.zeros(len(counts) + 1, dtype=torch.int32)
+    seg[1:] = torch.tensor(counts).cumsum(0)
+    total, gated = int(seg[-1]), mode == "silu"
+    w = (torch.randn((len(counts), (1 + gated) * n, k), generator=g, device="cuda")
+         / k ** 0.5).bfloat16()
+    x = torch.randn((total // 2, k), generator=g, device="cuda").bfloat16()
+    rows = torch.randint(len(x), (total,), generator=g, device="cuda", dtype=torch.int32)
+    got = ops.moe_gemm(x, w, seg.cuda(), gated, act="relu2" if mode == "relu2" else None,
+                       rows=rows)
+    for e in range(len(counts)):
+        lo, hi = int(seg[e]), int(seg[e + 1])
+        s = x[rows[lo:hi].long()].double() @ w[e].double().t()
+        if gated:
+            a, u = s.chunk(2, dim=1)
+            s = torch.nn.functional.silu(a) * u
+        elif mode == "relu2":
+            s = s.clamp(min=0).square()
+        # one rounding to bf16; float32 sums of up to 4096 terms and exp below 1e-4
+        err = (got[lo:hi].double() - s).abs()
+        assert (err <= 2 ** -8 * s.abs() + 2e-4).all(), (e, err.max().item())
