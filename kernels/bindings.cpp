@@ -521,6 +521,10 @@ void gemm_skinny_gated(torch::Tensor y, torch::Tensor x, torch::Tensor w13) {
   TORCH_CHECK(y.size(0) == M && y.size(1) == I);
   torch::Tensor part;
   if (M <= 64) {
+    if (gemm_ring_wins(M, I, K, true) && on16(x) && on16(w13) && on16(y)) {
+      run_ring(y, x, w13, M, I, K, true, gemm_ring_plan(M, I, K, true));
+      return;
+    }
     const int parts = gemm_stream_parts(16, M, I, K, true);
     launch_gemm_stream_gated(ptr<__hip_bfloat16>(y),
                              stream_parts(part, x, parts, (int64_t)2 * M * I),

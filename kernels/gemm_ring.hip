@@ -49,7 +49,8 @@ __global__ __launch_bounds__(256, OCC) void gemm_ring_kernel(
          [&](int r) { return min(r, M - 1 - m0) * row_bytes; },
          [&](int r) {
            const int wave = r / (R::kTN * 16), at = r % (R::kTN * 16), half = at / (OUT * 16);
-           return (half * N + wave * (OUT * 16) + R::out_col(at % (OUT * 16))) * row_bytes;
+           const int col = at % (OUT * 16);
+           return (half * N + wave * (OUT * 16) + (OUT > 1 ? R::out_col(col) : col)) * row_bytes;
          });
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -58,9 +59,16 @@ __global__ __launch_bounds__(256, OCC) void gemm_ring_kernel(
   for (int i = 0; i < R::kTM; ++i) {
     const int m = m0 + (wm * R::kTM + i) * 16 + col;
     if (m >= M) continue;
-    const long at = (long)m * N + n0 + wn * OUT * 16 + quad * 8;
+    const long at = (long)m * N + n0 + wn * OUT * 16 + quad * (OUT > 1 ? 8 : 4);
+    if constexpr (OUT == 1) {
+      union { __hip_bfloat16 h[4]; uint2 u; } o;
 #pragma unroll
-    for (int j = 0; j < OUT; j += 2) {
+      for (int r = 0; r < 4; ++r)
+        o.h[r] = __float2bfloat16(moe::finish<moe::kSilu>(acc[i][0][r], acc[i][1][r], 0.f));
+      *reinterpret_cast<uint2*>(y + at) = o.u;
+    }
+#pragma unroll
+    for (int j = 0; j + 1 < OUT; j += 2) {
       if (!GATED && gridDim.y > 1) {
         float* to = part + blockIdx.y * ((long)M * N) + at + j * 16;
         *reinterpret_cast<f32x4_t*>(to) = acc[i][j];
@@ -91,7 +99,7 @@ constexpr Form kForms[] = {
     {128, 128, 2, 1.5, 0.3, 0.48, 1.00, 3.9, 0.20, 0.21},
     {64, 128, 2, 2.3, 0.0, 0.34, 0.77, 3.2, 0.21, 0.20},
 };
-// The fifth form, 64 x 64 for up to 64 rows, is not fitted: few_rows below.
+// The fifth form, 64 x 64 for up to 64 rows, is not fitted: few_rows below (gated: not cut).
 constexpr int kFew = 4, kForm4Cols = 64;
 
 struct Plan {
@@ -123,6 +131,7 @@ int few_rows(int M, int N, int K) {
 // The form and the parts of K (of six tiles at least) that the model gives the least time.  It
 // picks what is 3 % slower than the best of all at the mean of the measured sizes, 1 % gated.
 Plan plan_of(int M, int N, int K, bool gated) {
+  if (gated && M <= 64) return Plan{kFew, 1, 0.0};
   if (const int parts = gated ? 0 : few_rows(M, N, K)) return Plan{kFew, parts, 0.0};
   Plan best{0, 1, 1e30};
   const double cols = gated ? 2.0 * N : N, w_mb = cols * K * 2e-6;
@@ -170,13 +179,13 @@ void launch_plan(__hip_bfloat16* y, float* part, const __hip_bfloat16* x, const 
     case 2: launch_form<128, 128, 4, 2, GATED>(y, part, x, w, M, N, K, parts, stream); break;
     case 3: launch_form<64, 128, 6, 2, GATED>(y, part, x, w, M, N, K, parts, stream); break;
     default:
-      if constexpr (!GATED) {
+      {
         // W that is read once and is large goes past the caches (24 rows: 28672 x 4096 46.4 ->
         // 39.9 us, 8192 x 3584 15.6 -> 13.8, 4096 x 4096 11.5 -> 11.5; 64 rows 12.6 -> 13.5)
-        if (M <= 64 && (long)N * K >= 20000000)
-          launch_form<64, 64, 8, 2, false, 2>(y, part, x, w, M, N, K, parts, stream);
+        if (M <= 64 && (GATED ? 2L : 1L) * N * K >= 20000000)
+          launch_form<64, 64, 8, 2, GATED, 2>(y, part, x, w, M, N, K, parts, stream);
         else
-          launch_form<64, 64, 8, 2, false>(y, part, x, w, M, N, K, parts, stream);
+          launch_form<64, 64, 8, 2, GATED>(y, part, x, w, M, N, K, parts, stream);
       }
   }
 }
@@ -201,7 +210,7 @@ int gemm_ring_plan(int M, int N, int K, bool gated) {
 // Whether a plan is one: a tile's columns fit, no part of K is empty.
 bool gemm_ring_takes(int N, int K, int plan, bool gated) {
   const int form = plan >> 4, parts = plan & 15;
-  if (plan < 0 || form > (gated ? 3 : kFew) || parts < 1 || parts > (gated ? 1 : 8)) return false;
+  if (plan < 0 || form > kFew || parts < 1 || parts > (gated ? 1 : 8)) return false;
   const int depth = (K / 64 + parts - 1) / parts;
   const int bn = form == kFew ? kForm4Cols : kForms[form].bn;
   return (gated ? 2L : 1L) * N % bn == 0 && (K / 64 + depth - 1) / depth == parts;
@@ -219,13 +228,20 @@ bool gemm_ring_takes(int N, int K, int plan, bool gated) {
 //   0.88 to 1.10, 28672 x 4096 0.99 to 1.14, 3072 x 2048 0.82 to 1.27, 1024 x 4096 1.11 to 1.25.
 //   301 to 1024, long K: 4096 x 14336 0.81 to 0.97; 2048 x 8192 0.89 to 1.00; 8192 x 28672 0.63
 //   to 1.12; others around 1: 4096 x 4096 0.97 to 1.16, 6144 x 4096 1.01 to 1.17.
-//  Gated, against the library's and its gate, where the model is below 0.92 of the library's
+//  Gated, against gemm_stream.hip's, 17 | 64 rows: 14336 x 4096 0.91 | 0.92, 6144 x 4096 0.86 |
+//   0.82, 8192 x 2048 0.85 | 0.83, 7168 x 8192 1.01 | 0.79, 8192 x 8192 1.06 | 0.75, 11008 x 4096
+//   1.07 | 0.80, 28672 x 8192 0.92 | 1.06; against the library's and its gate, where the model is below 0.92 of the library's
 //   (fitted likewise): 8192 x 2048 0.78 to 0.93; 14336 x 4096 0.88 to 0.99 (768 rows: 1.07);
 //   28672 x 8192 0.88 to 0.97 (256: 1.05); 4096 x 2048 0.54 to 0.94; 1024 x 2048 0.68 to 1.14.
 bool gemm_ring_wins(long M, long N, long K, bool gated) {
   if (!fits(M, N, K, gated)) return false;
   if (gated) {
-    if (M <= 64 || N * K < 4000000) return false;
+    if (M <= 64) {
+      if (M <= 16 || N < 6144 || (M > 48 && N * K > 150000000)) return false;
+      const long blocks = N / 32;   // one a CU, or nearly two
+      return M > 32 || (blocks <= 256 ? K < 8192 : blocks >= 400);
+    }
+    if (N * K < 4000000) return false;
     const double tf = 4e-9 * M * N * K / 1.334;
     const double mb = (4e-6 * N * K + 2e-6 * M * (2.0 * N + K)) * 0.202;
     const double library = 12.9 + sqrt(tf * tf + mb * mb) + 0.6e-6 * M * N;

@@ -46,8 +46,6 @@ def test_forms(form, gated, k):
     from vllm_tgis_adapter_amd.ops import _C
 
     bm, bn = FORMS[form]
-    if gated and form == 4:
-        pytest.skip("plain only")
     for m in (1, bm - 1, bm, bm + 1, 9 * bm + 17):      # nine tiles: a band and one more
         for cols in (1, 2, 3):
             n = bn * cols if not gated else bn * cols // 2
@@ -99,6 +97,7 @@ def test_rule(m, n, k, own):
 
 
 @pytest.mark.parametrize(("m", "n", "k", "own"), [
+    (17, 8192, 2048, True), (64, 14336, 4096, True), (24, 4096, 2048, True),
     (65, 8192, 2048, True), (512, 2048, 2048, True), (65, 3584, 8192, False)])
 def test_gated_rule(m, n, k, own):
     from vllm_tgis_adapter_amd import ops
