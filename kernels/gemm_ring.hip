@@ -218,10 +218,11 @@ bool gemm_ring_takes(int N, int K, int plan, bool gated) {
 
 // Whether these tiles take a product from what would run it otherwise.  Time over that one's,
 // cold weights, N x K: rows.
-//  Against gemm_stream.hip's, 17 to 64 rows: 28672 x 4096 0.90 to 0.94; 4096 x 14336 0.77 to
+//  Against gemm_stream.hip's, 9 to 64 rows: 28672 x 4096 0.90 to 0.94; 4096 x 14336 0.77 to
 //   0.90; 4096 x 4096 17 0.98, 64 0.76; 512 x 4096 0.96 to 0.66; 3072 x 2048 17 1.08, 40 0.95, 64
-//   0.91; 2048 x 2048 32 1.12, 40 0.97; 12 rows: 6144 x 4096 1.08, 4096 x 4096 1.09, 28672 x 4096
-//   0.93.
+//   0.91; 2048 x 2048 32 1.12, 40 0.97.  2 | 12 rows: 28672 x 4096 0.99 | 0.94, 10240 x 8192 0.89 |
+//   0.86, 2048 x 8192 0.96 | 0.94, 16384 x 2048 0.98 | 0.93, 4096 x 14336 1.02 | 0.97, 14336 x 4096
+//   1.04 | 0.97; 6144 x 4096 1.13 | 1.10, 4096 x 7168 1.13 | 1.06, 8192 x 3584 1.07 | 1.03.
 //  Against the library's:
 //   65 to 256 rows: 4096 x 4096 0.60 to 0.99; 6144 x 4096 0.76 to 1.00; 4096 x 14336 0.82 to
 //   0.97; 8192 x 8192 0.89 to 1.02; 2560 x 8192 0.54 to 0.90; 12288 and 14336 x 4096 and 8192
@@ -247,8 +248,9 @@ bool gemm_ring_wins(long M, long N, long K, bool gated) {
     const double library = 12.9 + sqrt(tf * tf + mb * mb) + 0.6e-6 * M * N;
     return plan_of(M, N, K, true).us < 0.92 * library;
   }
+  if (M <= 16) return M > 8 && (K >= 8192 ? N * K >= 16000000 : N * K >= 33000000);
   if (M <= 64)
-    return M > 16 && N * K >= 2000000 && (K >= 4096 || N * K >= 16000000 || M >= 40);
+    return N * K >= 2000000 && (K >= 4096 || N * K >= 16000000 || M >= 40);
   if (N * K < 6000000) return false;
   if (M <= 256) return K >= 3584 && N <= 10240;
   return M <= 1024 && 2 * K >= 7 * N;

@@ -79,7 +79,8 @@ def test_plans_that_are_none():
 
 
 # first and last rows of the rule and the ones beside them: rows, N, K, whether it takes them
-LINES = [(16, 4096, 4096, False), (17, 4096, 4096, True), (64, 4096, 4096, True),
+LINES = [(8, 16384, 2048, False), (9, 16384, 2048, True), (9, 2048, 8192, True),
+         (16, 8192, 3584, False), (16, 4096, 4096, False), (17, 4096, 4096, True), (64, 4096, 4096, True),
          (33, 128, 8192, False), (17, 512, 4096, True), (39, 3072, 2048, False),
          (40, 3072, 2048, True), (64, 8192, 28672, True), (64, 28672, 4096, True),
          (17, 28672, 4096, True), (65, 28672, 4096, False), (256, 4096, 4096, True),
