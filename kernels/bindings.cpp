@@ -42,6 +42,8 @@ int gemm_stream_parts(int qbits, int M, int N, int K, bool gated);
 void launch_rotary_cache(const long*, __hip_bfloat16*, const __hip_bfloat16*,
                          const __hip_bfloat16*, const __hip_bfloat16*, const float*, void*, void*,
                          const long*, int, int, int, int, long, long, long, bool, hipStream_t);
+void launch_decode_inputs(const long*, long*, long*, long*, int*, int*, int*, int, int, int, int,
+                          hipStream_t);
 int gemm_ring_plan(int M, int N, int K, bool gated);
 void launch_gemm_ring_parts(__hip_bfloat16*, float*, const __hip_bfloat16*,
                             const __hip_bfloat16*, int, int, int, int, hipStream_t);
@@ -716,6 +718,32 @@ void lora_product(torch::Tensor out, torch::Tensor x, c10::optional<torch::Tenso
                      cols, T, R, PR, V, W, cuts, parts, gated, current_stream());
 }
 
+// A captured step's static buffers from a packed pinned host buffer (decode_inputs.hip) of n rows
+// and tables of w blocks; rows: of the graph
+void decode_inputs(torch::Tensor packed, torch::Tensor ids, torch::Tensor positions,
+                   torch::Tensor slots, torch::Tensor lens, c10::optional<torch::Tensor> states,
+                   torch::Tensor tables, int64_t n, int64_t w, int64_t rows) {
+  TORCH_CHECK(packed.is_pinned() && packed.is_contiguous() &&
+              packed.scalar_type() == at::ScalarType::Byte && on16(packed));
+  TORCH_CHECK(n >= 1 && w >= 0 && n <= rows && packed.numel() >= n * (32 + 4 * w));
+  for (const auto& t : {ids, positions, slots})
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::ScalarType::Long && t.is_contiguous() &&
+                t.numel() >= rows);
+  TORCH_CHECK(lens.is_cuda() && lens.scalar_type() == at::ScalarType::Int &&
+              lens.is_contiguous() && lens.numel() >= rows);
+  TORCH_CHECK(tables.is_cuda() && tables.scalar_type() == at::ScalarType::Int &&
+              tables.is_contiguous() && tables.dim() == 2 && tables.size(0) >= rows &&
+              tables.size(1) >= w);
+  if (states.has_value())
+    TORCH_CHECK(states->is_cuda() && states->scalar_type() == at::ScalarType::Int &&
+                states->is_contiguous() && states->numel() >= rows);
+  launch_decode_inputs(reinterpret_cast<const long*>(packed.data_ptr()), ids.data_ptr<long>(),
+                       positions.data_ptr<long>(), slots.data_ptr<long>(), lens.data_ptr<int>(),
+                       states.has_value() ? states->data_ptr<int>() : nullptr,
+                       tables.data_ptr<int>(), (int)n, (int)w, (int)rows, (int)tables.size(1),
+                       current_stream());
+}
+
 // slots[t] = the place of token_ids[t] among ids (64 at most), or -1
 void lora_slots(torch::Tensor slots, torch::Tensor token_ids, const std::vector<int>& ids) {
   for (const auto& t : {slots, token_ids})
@@ -905,6 +933,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_ring", &gemm_ring, "product of many rows, large tiles, also gated", py::arg("y"),
         py::arg("x"), py::arg("w"), py::arg("gated") = false, py::arg("plan") = 0);
   m.def("gemm_ring_wins", &gemm_ring_wins, "whether the large tiles are the faster product");
+  m.def("decode_inputs", &decode_inputs, "a captured step's inputs from a packed host buffer");
   m.def("lora_product", &lora_product, "a product with its LoRA deltas, also gated");
   m.def("lora_delta", &lora_delta,
         "bf16 multi-LoRA of up to three projections of one input");

@@ -127,3 +127,23 @@ class DecodeGraphRunner:
             self.in_block_tables[:n, w:].zero_()
         self.graphs[b].replay()
         return self.out_logits[b][:n]
+
+    @staticmethod
+    def packed_bytes(n: int, w: int) -> int:
+        """Of the host buffer that run_packed takes for n sequences and w blocks."""
+        return n * (32 + 4 * w)
+
+    @torch.inference_mode()
+    def run_packed(self, packed: torch.Tensor, n: int, w: int) -> torch.Tensor:
+        """run() with the inputs in one pinned uint8 buffer: int64 ids, positions and slots [n]
+        each, int32 lengths [n], state slots [n] (unused without sequence state) and block
+        tables [n, w].  The buffer is read when the stream gets there."""
+        from .. import ops
+
+        b = self.bucket_for(n)
+        assert b is not None
+        ops.decode_inputs(
+            packed, self.in_ids, self.in_pos, self.in_slots, self.in_seq_lens,
+            self.in_state_slots if self.with_seq_state else None, self.in_block_tables, n, w, b)
+        self.graphs[b].replay()
+        return self.out_logits[b][:n]

@@ -215,6 +215,9 @@ class Worker:
         # launch phase behind the previous step's GPU work)
         self._pin: dict[str, torch.Tensor] = {}
         self._pin_flip = 0
+        # decode steps: all inputs in one buffer, which the GPU reads (an event each: a
+        # buffer is written again when its step has read it)
+        self._packed: list = [None, None]
 
         if self.tp > 1 and self.device == "cuda":
             from ..parallel import init_xgmi_allreduce
@@ -622,13 +625,37 @@ class Worker:
         staging.copy_(torch.from_numpy(np.ascontiguousarray(arr)).view(-1).to(dtype))
         return staging.to(self.device, non_blocking=True).view(*arr.shape)
 
+    def _replay_packed(self, batch: dict, n: int) -> torch.Tensor:
+        """A decode step by its captured graph, its inputs by one launch."""
+        tables = _pad_np_tables(batch["decode_tables"])
+        w = tables.shape[1]
+        need = self.graph_runner.packed_bytes(n, w)
+        held = self._packed[self._pin_flip]
+        if held is not None:
+            held[2].synchronize()
+        if held is None or held[0].numel() < need:
+            buf = torch.empty(max(2 * need, 4096), dtype=torch.uint8, pin_memory=True)
+            held = (buf, buf.numpy(), torch.cuda.Event())
+            self._packed[self._pin_flip] = held
+        buf, host, read = held
+        longs = host[:24 * n].view(np.int64).reshape(3, n)
+        longs[0] = batch["token_ids"]
+        longs[1] = batch["positions"]
+        longs[2] = batch["slot_mapping"]
+        ints = host[24 * n:need].view(np.int32)
+        ints[:n] = batch["decode_seq_lens"]
+        if self.uses_seq_state:
+            ints[n:2 * n] = batch["state_slots"]
+        ints[2 * n:].reshape(n, w)[:] = tables
+        logits = self.graph_runner.run_packed(buf, n, w)
+        read.record()
+        return logits
+
     @torch.inference_mode()
     def execute_batch(self, batch: dict) -> Optional[torch.Tensor]:
         """All ranks: run the forward; returns logits rows on every rank."""
         dev = self.device
         self._pin_flip ^= 1
-        ids = self._h2d("ids", np.asarray(batch["token_ids"], dtype=np.int64), torch.int64)
-        pos = self._h2d("pos", np.asarray(batch["positions"], dtype=np.int64), torch.int64)
         np_seqs = len(batch["prefill_seq_lens"])
 
         # hipGraph replay path: pure-decode batch, every row samples, no LoRA
@@ -641,6 +668,10 @@ class Worker:
             and list(batch["logit_rows"]) == list(range(n))
             and self.graph_runner.bucket_for(n) is not None
         ):
+            if ops.has_native():
+                return self._replay_packed(batch, n)
+            ids = self._h2d("ids", np.asarray(batch["token_ids"], dtype=np.int64), torch.int64)
+            pos = self._h2d("pos", np.asarray(batch["positions"], dtype=np.int64), torch.int64)
             slots = self._h2d("slots", np.asarray(batch["slot_mapping"], dtype=np.int64), torch.int64)
             seq_lens = self._h2d("dsl", np.asarray(batch["decode_seq_lens"], dtype=np.int32), torch.int32)
             bt = self._h2d("dbt", _pad_np_tables(batch["decode_tables"]), torch.int32)
@@ -649,6 +680,8 @@ class Worker:
                 st = self._h2d("sts", np.asarray(batch["state_slots"], dtype=np.int32), torch.int32)
             return self.graph_runner.run(ids, pos, slots, seq_lens, bt, st)
 
+        ids = self._h2d("ids", np.asarray(batch["token_ids"], dtype=np.int64), torch.int64)
+        pos = self._h2d("pos", np.asarray(batch["positions"], dtype=np.int64), torch.int64)
         npt = batch["qsl"][-1] if np_seqs else 0
         meta = AttnMetadata(
             num_prefill_seqs=np_seqs,

@@ -585,6 +585,14 @@ def lora_product(
     return out
 
 
+def decode_inputs(packed, ids, positions, slots, lens, states, tables, n: int, w: int,
+                  rows: int) -> None:
+    """A captured step's static buffers from a packed pinned host buffer
+    (DecodeGraphRunner.run_packed), the rows from n to ``rows`` as padding."""
+    assert _native(ids), "decode_inputs is the GPU path"
+    _C.decode_inputs(packed, ids, positions, slots, lens, states, tables, n, w, rows)
+
+
 def lora_slots(token_ids: torch.Tensor, ids: tuple[int, ...]) -> torch.Tensor:
     """Place of every token's adapter id among ``ids``, -1 where it is none of them."""
     if native_enabled(token_ids) and token_ids.dtype == torch.int32 and len(ids) <= 64:
