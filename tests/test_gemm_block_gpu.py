@@ -1,4 +1,4 @@
-"""bf16 products by large tiles with a cut K (gemm_block.hip) against float64: rows around
+"""bf16 products by large tiles with a cut K (gemm_ring.hip) against float64: rows around
 the tiles of 128, a K of one tile, of uneven and of equal parts, and the rule that sends a
 product there."""
 

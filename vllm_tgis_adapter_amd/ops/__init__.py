@@ -302,7 +302,8 @@ def _plain_tensors(*tensors: torch.Tensor) -> bool:
 def _block_rows(n: int, k: int) -> range:
     """Rows of a product past 64 that the tiles with a cut K take from the library: where K
     is so long, and 128 x 128 tiles so few, that K can be cut over three workgroups and
-    more.  Time over the library's, cold weights, N x K: rows:
+    more.  Time over the library's, cold weights (with 128 x 128 tiles only; gemm_ring.hip's
+    choice is faster at every size measured, 4096 x 14336: 128 0.46, 512 0.78), N x K: rows:
       1024 x 8192: 160 1.13, 257 0.94, 512 1.04, 700 0.86;  2048 x 8192: 128 1.11, 129 0.91,
       700 0.87;  2560 x 8192: 160 1.00, 200 0.91, 512 0.85, 513 1.16;  4096 x 14336: 65 0.84,
       128 0.56, 512 0.96, 640 0.83, 700 1.15;  5120 x 8192: 65 1.06, 129 1.03, 256 0.60, 512
