@@ -297,6 +297,8 @@ int gemm_panel_plan(int M, int N, int K) {
   float least = 0.f;
   for (int i = 0; i < (int)(sizeof(kPanels) / sizeof(kPanels[0])); ++i) {
     if (N % (kPanels[i].tn * 64) != 0) continue;
+    // a panel's rows of x and of W lie inside 4 GB
+    if (32L * kPanels[i].tm * K >= 1L << 32 || 64L * kPanels[i].tn * K >= 1L << 32) continue;
     for (int parts = 1; parts <= 8 && (parts == 1 || K / parts >= 512); ++parts) {
       const int depth = (K / 64 + parts - 1) / parts;
       if ((K / 64 + depth - 1) / depth != parts) continue;   // no part is empty

@@ -55,17 +55,18 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, quad = lane >> 4;
 
-  // (where there are fewer loads than waves some are made twice: all waves wait alike)
+  // (where there are fewer loads than waves some are made twice: all waves wait alike; rows
+  // of a panel are found by 32 bits, see gemm_panel_plan)
   unsigned x_off[X_PASS], w_off[W_PASS];
 #pragma unroll
   for (int p = 0; p < X_PASS; ++p) {
     const int r = (p * kWaves + wave) % X_LOADS * 8 + lane / 8;
-    x_off[p] = min(r, M - 1 - m0) * (K * 2) + ((lane % 8) ^ (r / 2 % 8)) * 16;
+    x_off[p] = (unsigned)min(r, M - 1 - m0) * (K * 2u) + ((lane % 8) ^ (r / 2 % 8)) * 16;
   }
 #pragma unroll
   for (int p = 0; p < W_PASS; ++p) {
     const int r = (p * kWaves + wave) * 16 + lane / 4;
-    w_off[p] = r * K + ((lane % 4) ^ (r / 4 % 4)) * 16;
+    w_off[p] = (unsigned)r * K + ((lane % 4) ^ (r / 4 % 4)) * 16;
   }
   const auto x_from = block_gemm::resource(x + (long)m0 * K + k0);
   const auto w_from = block_gemm::resource(w + (long)n0 * K + k0);
