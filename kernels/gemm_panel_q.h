@@ -17,6 +17,8 @@ using block_gemm::bf16x8_t;
 using block_gemm::f32x4_t;
 
 typedef __attribute__((ext_vector_type(4))) unsigned int u32x4_t;
+// scales start at any float
+typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4_any_t;
 
 constexpr int kDepth = 64;    // inputs of a tile
 constexpr int kWaves = 4;     // along N
@@ -171,7 +173,7 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
     const int n = n0 + (wave * TN + j) * 16 + quad * 4;
-    const f32x4_t s = *reinterpret_cast<const f32x4_t*>(scale + n);
+    const f32x4_t s = *reinterpret_cast<const f32x4_any_t*>(scale + n);
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const int m = m0 + i * 16 + col;

@@ -144,7 +144,7 @@ def _at_odd_offset(t):
 
 
 @pytest.mark.parametrize("qbits", [8, 4])
-@pytest.mark.parametrize("which", ["x", "codes"])
+@pytest.mark.parametrize("which", ["x", "codes", "scales"])
 @pytest.mark.parametrize("m", [65, 300, 1200])
 def test_rounded_many_rows_from_any_address(qbits, which, m):
     """Tensors that start off a 16-byte boundary, in both forms of the product."""
@@ -156,8 +156,10 @@ def test_rounded_many_rows_from_any_address(qbits, which, m):
     want = ops.linear_quant(x, wq, scale, qbits)
     if which == "x":
         x = _at_odd_offset(x)
-    else:
+    elif which == "codes":
         wq = _at_odd_offset(wq)
+    else:
+        scale = _at_odd_offset(scale)
     got = ops.linear_quant(x, wq, scale, qbits)
     exact = x.double() @ ops.dequantize_weight(wq, scale, qbits, torch.float32).double().t()
     terms = x.double().abs() @ ops.dequantize_weight(wq, scale, qbits, torch.float32).double(
