@@ -773,10 +773,9 @@ void moe_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w,
   TORCH_CHECK(N % 128 == 0 && K % 64 == 0 && w.size(2) == K);
   TORCH_CHECK(y.size(0) == T && y.size(1) == N);
   TORCH_CHECK(x.is_contiguous() && w.is_contiguous() && y.is_contiguous());
-  // rows reach LDS, and results memory, in 16-byte pieces
+  // rows reach LDS in 16-byte pieces
   TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
-              reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0 &&
-              reinterpret_cast<uintptr_t>(y.data_ptr()) % 16 == 0, "x, w and y start at 16 bytes");
+              reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0, "x and w start at 16 bytes");
   const int* rp = nullptr;
   if (rows.has_value()) {
     TORCH_CHECK(rows->is_cuda() && rows->scalar_type() == at::ScalarType::Int &&

@@ -111,8 +111,10 @@ void launch_mode(__hip_bfloat16* y, const __hip_bfloat16* x, const __hip_bfloat1
   // by rank^-0.6: <4,4,2> 83 | 112, 128 x 128 85 | 85; 2048 and 2048: 33 | 47, 37 | 36; 8 of
   // 4096 and 3584, 128 x 128 at one workgroup a CU: <4,4,2> 46 | 49, 66 | 66.
   const int mean = T / E;
-  // rows of a block are found by 32 bits
-  const bool far = (long)N * cols * K * 2 >= 1L << 32 || (long)T * K * 2 >= 1L << 32;
+  // what the tiles do not take: rows of a block are found by 32 bits, results are stored by 16
+  // bytes (the streaming form stores them one by one)
+  const bool far = (long)N * cols * K * 2 >= 1L << 32 || (long)T * K * 2 >= 1L << 32 ||
+                   reinterpret_cast<uintptr_t>(y) % 16 != 0;
   const long one = (long)E * (N / 64), last = one % 512;   // streaming workgroups
   const bool brim = !moe::gated(MODE) && (last == 0 || last > 460) &&
                     (K <= 2048 || (one >= 1024 && K <= 8192));

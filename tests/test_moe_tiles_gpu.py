@@ -43,3 +43,36 @@ def test_tiles(mode, counts, n, k):
         # one rounding to bf16; float32 sums of up to 4096 terms and exp below 1e-4
         err = (got[lo:hi].double() - s).abs()
         assert (err <= 2 ** -8 * s.abs() + 2e-4).all(), (e, err.max().item())
+
+
+@pytest.mark.parametrize("module", ["_C", "_C_seq"])
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize("counts", [[5, 3], [60, 70], [300, 0, 141]], ids=str)
+def test_results_at_any_address(module, mode, counts):
+    """Results that start off a 16-byte boundary, rows past the last segment left as they are."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import importlib
+
+    moe_gemm = importlib.import_module(f"vllm_tgis_adapter_amd.{module}").moe_gemm
+    g = torch.Generator("cuda").manual_seed(len(counts))
+    n, k, total = 256, 128, sum(counts)
+    seg = torch.zeros(len(counts) + 1, dtype=torch.int32)
+    seg[1:] = torch.tensor(counts).cumsum(0)
+    w = torch.randn((len(counts), (1 + (mode == 1)) * n, k), generator=g, device="cuda")
+    w = (w / k ** 0.5).bfloat16()
+    x = torch.randn((total + 2, k), generator=g, device="cuda").bfloat16()
+    got = torch.full(((total + 2) * n + 1,), 7.0, dtype=torch.bfloat16, device="cuda")
+    moe_gemm(got[1:].view(total + 2, n), x, w, seg.cuda(), mode)
+    assert (got[:1] == 7).all() and (got[1 + total * n:] == 7).all()
+    for e in range(len(counts)):
+        lo, hi = int(seg[e]), int(seg[e + 1])
+        s = x[lo:hi].double() @ w[e].double().t()
+        if mode == 1:
+            a, u = s.chunk(2, dim=1)
+            s = torch.nn.functional.silu(a) * u
+        elif mode == 2:
+            s = s.clamp(min=0).square()
+        # as in test_tiles
+        err = (got[1:].view(-1, n)[lo:hi].double() - s).abs()
+        assert (err <= 2 ** -8 * s.abs() + 2e-4).all(), (e, err.max().item())
