@@ -68,6 +68,18 @@ def test_parts(form, parts, k):
     _check(y, x, w, False)
 
 
+@pytest.mark.parametrize("entry", ["gemm_block", "gemm_ring"])
+def test_results_at_any_address(entry):
+    """Results that start off a 16-byte boundary."""
+    from vllm_tgis_adapter_amd.ops import _C
+
+    x, w = _inputs(130, 384, 832)
+    got = torch.full((130 * 384 + 1,), 7.0, dtype=torch.bfloat16, device="cuda")
+    getattr(_C, entry)(got[1:].view(130, 384), x, w)
+    assert got[0] == 7
+    _check(got[1:].view(130, 384), x, w, False)
+
+
 def test_plans_that_are_none():
     from vllm_tgis_adapter_amd.ops import _C
 
