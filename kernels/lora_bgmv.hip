@@ -231,9 +231,30 @@ __global__ __launch_bounds__(64 * kShrinkWaves) void lora_shrink_tile_kernel(
   }
 }
 
-// grid (ceil(V / 256), ceil(T / TOKENS)).  Few tokens are a chain of latencies: what was in
-// out, the cuts' sums and, where they fit, the rows of B for all tokens are asked for at once
-// (61 tokens, rank 16, 4096 columns: 6.5 -> 4.0 us).
+// The cuts' sums of a workgroup's tokens.  FEW: eight parts are asked for at once.
+template <int R, int TOKENS, bool FEW>
+DEVINLINE void add_cuts(float (&sums)[TOKENS][3 * R], const float* __restrict__ tmp, const int T,
+                        const int t0, const int tokens, const int PR, const int cuts) {
+  for (int i = threadIdx.x; i < tokens * PR; i += 256) {
+    float s = 0.f;
+    if constexpr (FEW) {
+      for (int c0 = 0; c0 < cuts; c0 += 8) {
+        float part[8];
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+          part[c] = tmp[((long)min(c0 + c, cuts - 1) * T + t0) * PR + i];
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+          if (c0 + c < cuts) s += part[c];
+      }
+    } else {
+      for (int c = 0; c < cuts; ++c) s += tmp[((long)c * T + t0) * PR + i];
+    }
+    sums[i / PR][i % PR] = s;
+  }
+}
+
+// grid (ceil(V / 256), ceil(T / TOKENS))
 template <int R, int TOKENS>
 __global__ __launch_bounds__(256) void lora_expand_tile_kernel(
     __hip_bfloat16* __restrict__ out,            // [T, out_w]
@@ -241,6 +262,61 @@ __global__ __launch_bounds__(256) void lora_expand_tile_kernel(
     const __hip_bfloat16* __restrict__ b_stack,  // [L, V, R]
     const int* __restrict__ slots, const float* __restrict__ scales, const LoraCols cols,
     const int T, const int PR, const int V, const int out_w, const int cuts) {
+  __shared__ float sums[TOKENS][3 * R];
+  __shared__ int own[TOKENS];
+  const int t0 = blockIdx.y * TOKENS, v = blockIdx.x * 256 + threadIdx.x;
+  const int tokens = min(TOKENS, T - t0);
+  if (threadIdx.x < TOKENS)
+    own[threadIdx.x] = threadIdx.x < tokens ? slots[t0 + threadIdx.x] : -1;
+  __syncthreads();
+  for (int i = threadIdx.x; i < tokens * PR; i += 256) {
+    const int t = i / PR;
+    float s = 0.f;
+    if (own[t] >= 0)
+      for (int c = 0; c < cuts; ++c) s += tmp[((long)c * T + t0) * PR + i];
+    sums[t][i % PR] = s;
+  }
+  __syncthreads();
+  if (v >= V) return;
+  const int p = v < cols.end[0] ? 0 : v < cols.end[1] ? 1 : 2;
+  __hip_bfloat16* o = out + (long)t0 * out_w + v + cols.shift[p];
+  float was[TOKENS];
+#pragma unroll
+  for (int t = 0; t < TOKENS; ++t)
+    was[t] = t < tokens ? __bfloat162float(o[(long)t * out_w]) : 0.f;
+
+  Vec16<__hip_bfloat16> b[R / 8];
+  float scale = 0.f;
+  int cur = -1;
+#pragma unroll
+  for (int t = 0; t < TOKENS; ++t) {
+    const int slot = __builtin_amdgcn_readfirstlane(own[t]);
+    if (slot < 0) continue;
+    if (slot != cur) {
+      cur = slot;
+      scale = scales[slot];
+#pragma unroll
+      for (int j = 0; j < R / 8; ++j) b[j] = load16(b_stack + ((long)slot * V + v) * R + j * 8);
+    }
+    float acc = 0.f;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      acc = __builtin_fmaf(__bfloat162float(b[r / 8].data[r % 8]), sums[t][p * R + r], acc);
+    o[(long)t * out_w] = __float2bfloat16(was[t] + acc * scale);
+  }
+}
+
+// The same for few tokens, which are a chain of latencies: what was in out, the cuts' sums and,
+// where they fit, the rows of B for all tokens are asked for at once (61 tokens, rank 16, 4096
+// columns, K in 16 cuts: 4.5 -> 3.4 us).
+template <int R>
+__global__ __launch_bounds__(256) void lora_expand_few_kernel(
+    __hip_bfloat16* __restrict__ out,            // [T, out_w]
+    const float* __restrict__ tmp,               // [cuts, T, PR]
+    const __hip_bfloat16* __restrict__ b_stack,  // [L, V, R]
+    const int* __restrict__ slots, const float* __restrict__ scales, const LoraCols cols,
+    const int T, const int PR, const int V, const int out_w, const int cuts) {
+  constexpr int TOKENS = 2;
   constexpr bool AHEAD = TOKENS * R <= 64;
   __shared__ float sums[TOKENS][3 * R];
   const int t0 = blockIdx.y * TOKENS, v = blockIdx.x * 256 + threadIdx.x;
@@ -266,19 +342,7 @@ __global__ __launch_bounds__(256) void lora_expand_tile_kernel(
     }
   }
   // (tokens without an adapter: whatever is there, which is not used)
-  for (int i = threadIdx.x; i < tokens * PR; i += 256) {
-    float s = 0.f;
-    for (int c0 = 0; c0 < cuts; c0 += 8) {
-      float part[8];
-#pragma unroll
-      for (int c = 0; c < 8; ++c)
-        part[c] = tmp[((long)min(c0 + c, cuts - 1) * T + t0) * PR + i];
-#pragma unroll
-      for (int c = 0; c < 8; ++c)
-        if (c0 + c < cuts) s += part[c];
-    }
-    sums[i / PR][i % PR] = s;
-  }
+  add_cuts<R, TOKENS, true>(sums, tmp, T, t0, tokens, PR, cuts);
   __syncthreads();
   if (v >= V) return;
   int cur = -1;
@@ -313,8 +377,13 @@ void launch_expand(__hip_bfloat16* out, const float* tmp, const __hip_bfloat16* 
   // the rows of B.  Rank 16, by 256-column tiles of all tokens (us at 2, 4, 8, 16 tokens):
   // 976 3.7 4.4 5.6 8.2, 6832 7.0 5.9 6.6 9.7, 14336 12.1 9.6 8.7 11.5, 67200 67 50 41 44,
   // 229376 157 123 106 102; ranks 8 and 64 cross at the same places.
+  // The form for few tokens, us there | here at two tokens: rank 16, 8 cuts of K, 976 tiles 3.1 |
+  // 3.7, 2560 3.7 | 4.0, 3840 4.5 | 4.7, 4800 5.3 | 5.0 (at four); 4 cuts, 1600 3.3 | 3.5, 2400 3.9 |
+  // 3.7; rank 64, 8 cuts, 976 6.7 | 7.2, 1600 7.0 | 7.4, 2400 9.3 | 9.4; 4 cuts, 1200 7.0 | 6.8; rank
+  // 8, 16384 tiles 9.9 | 6.4 (at eight).
   const long tiles = (V + 255L) / 256 * T;
-  if (tiles <= 2560) go(lora_expand_tile_kernel<R, 2>, 2);
+  if (tiles <= (R <= 16 ? 2048 : 1024) * (cuts >= 8 ? 2 : 1)) go(lora_expand_few_kernel<R>, 2);
+  else if (tiles <= 2560) go(lora_expand_tile_kernel<R, 2>, 2);
   else if (tiles <= 8192) go(lora_expand_tile_kernel<R, 4>, 4);
   else if (tiles <= 98304) go(lora_expand_tile_kernel<R, 8>, 8);
   else go(lora_expand_tile_kernel<R, 16>, 16);
@@ -325,8 +394,10 @@ void launch_expand(__hip_bfloat16* out, const float* tmp, const __hip_bfloat16* 
 // times the second.  One launch for what were two or three (a merge, expand, a gate), results
 // rounded once.  grid (ceil(columns of out / 256), ceil(T / TOKENS)); bound as expand is.
 // 61 tokens of 4 adapters of rank 16: merge and expand into 4096 columns 3.9 + 4.0 -> 5.0 us,
-// expand into 28672 and the gate 7.8 + 4.1 -> 8.9.
-template <int R, int TOKENS, bool GATE>
+// expand into 28672 and the gate 8.5 -> 7.5.  With the gate two columns' rows of B are held, from
+// rank 32 on at the cost of waves (136 to 256 registers): engine/lora.py says up to how many tokens
+// it is the faster way.
+template <int R, int TOKENS, bool GATE, bool FEW>
 __global__ __launch_bounds__(256) void lora_finish_kernel(
     __hip_bfloat16* __restrict__ out,            // [T, GATE ? W / 2 : W]
     const __hip_bfloat16* __restrict__ base,     // [T, W] (parts == 0)
@@ -336,7 +407,7 @@ __global__ __launch_bounds__(256) void lora_finish_kernel(
     const int* __restrict__ slots, const float* __restrict__ scales, const LoraCols cols,
     const int T, const int PR, const int V, const int W, const int cuts, const int parts) {
   constexpr int H = GATE ? 2 : 1;
-  constexpr bool AHEAD = TOKENS * R * H <= 64;
+  constexpr bool AHEAD = FEW && TOKENS * R * H <= 64;
   __shared__ float sums[TOKENS][3 * R];
   const int OW = W / H, t0 = blockIdx.y * TOKENS, n = blockIdx.x * 256 + threadIdx.x;
   const int tokens = min(TOKENS, T - t0);
@@ -391,18 +462,7 @@ __global__ __launch_bounds__(256) void lora_finish_kernel(
 #pragma unroll
   for (int t = 0; t < TOKENS; ++t) scale[t] = own[t] >= 0 ? scales[own[t]] : 0.f;
   // (tokens without an adapter: whatever is there, which is not used)
-  for (int i = threadIdx.x; i < tokens * PR; i += 256) {
-    float s = 0.f;
-    for (int c0 = 0; c0 < cuts; c0 += 8) {
-      float v[8];
-#pragma unroll
-      for (int c = 0; c < 8; ++c) v[c] = tmp[((long)min(c0 + c, cuts - 1) * T + t0) * PR + i];
-#pragma unroll
-      for (int c = 0; c < 8; ++c)
-        if (c0 + c < cuts) s += v[c];
-    }
-    sums[i / PR][i % PR] = s;
-  }
+  add_cuts<R, TOKENS, FEW>(sums, tmp, T, t0, tokens, PR, cuts);
   __syncthreads();
   if (n >= OW) return;
   int cur = -1;
@@ -449,11 +509,13 @@ void launch_finish(__hip_bfloat16* out, const __hip_bfloat16* base, const float*
                        stream, out, base, part, tmp, b, slots, scales, cols, T, PR, V, W, cuts,
                        parts);
   };
-  // as in launch_expand, by what a thread has to do
+  // as in launch_expand, by what a thread has to do (many tokens: B is read where an adapter
+  // begins, rank 8, 57344 tiles with the gate 39.7 -> 30.2 us)
   const long tiles = (W + 255L) / 256 * T;
-  if (tiles <= 2560) go(lora_finish_kernel<R, 2, GATE>, 2);
-  else if (tiles <= 98304) go(lora_finish_kernel<R, 4, GATE>, 4);
-  else go(lora_finish_kernel<R, 8, GATE>, 8);
+  if (tiles <= 2560) go(lora_finish_kernel<R, 2, GATE, true>, 2);
+  else if (tiles <= 8192) go(lora_finish_kernel<R, 4, GATE, true>, 4);
+  else if (tiles <= 98304) go(lora_finish_kernel<R, 4, GATE, false>, 4);
+  else go(lora_finish_kernel<R, 8, GATE, false>, 8);
 }
 
 // slot of every token: the place of its adapter's id among `ids`, or -1
