@@ -152,17 +152,30 @@ def _batched(x: torch.Tensor) -> bool:
     )
 
 
+# Most tokens, times a layer's 256-column pieces, up to which the gate is taken in the launch that
+# adds the deltas, by rank (us there | deltas and gate apart; tokens x columns): rank 8, 1024 x
+# 16384 29 | 36, 2048 x 28672 82 | 93, 4096 x 28672 198 | 184; 16, 301 x 28672 18 | 19, 700 x 16384
+# 26 | 22; 32, 33 x 28672 8.1 | 8.6, 61 x 28672 12.9 | 12.2, 512 x 28672 77 | 53; 64, 16 x 16384 8.2 |
+# 9.0, 16 x 28672 14.8 | 11.5, 2048 x 28672 869 | 270.
+_GATE_TILES = {8: 131072, 16: 32768, 32: 4096, 64: 1024}
+
+
+def gate_with_deltas(tokens: int, width: int, rank: int) -> bool:
+    """Whether the launch that adds the deltas to a gate and up product takes the gate too."""
+    return tokens * ((width + 255) // 256) <= _GATE_TILES.get(rank, 0)
+
+
 def lora_linear(
     layer_idx: int,
     projs: list[tuple[str, int, int]],
     x: torch.Tensor,
     weight: Optional[torch.Tensor],  # of the base linear, without a bias; None: not as it is
-    base,                            # () -> its product, for a weight that is None
+    base,                            # () -> its product
     gated: bool = False,
 ) -> Optional[torch.Tensor]:
-    """The base linear's product and the adapters' deltas made together, gated: and silu of
-    the first half of its columns times the second.  None where that does not apply: the
-    caller has the product made, then apply_lora."""
+    """The base linear's product with the adapters' deltas, made together where that is
+    faster, gated: silu of the first half of its columns times the second.  None where the
+    batched bf16 kernels do not apply: the caller has the product made, then apply_lora."""
     if not (CTX.active and x.dim() == 2 and x.dtype == torch.bfloat16 and len(projs) <= 3
             and _batched(x)):
         return None
@@ -172,16 +185,26 @@ def lora_linear(
     from .. import ops
 
     a_stack, b_stack, scales, spans = stacks
+    slots = CTX.token_slots
+    gate = False
+    if gated:
+        width = projs[-1][2]
+        gate = gate_with_deltas(x.shape[0], width, b_stack.shape[2])
     out = None
     if weight is not None:
-        out = ops.lora_product(x, weight, None, a_stack, b_stack, CTX.token_slots, scales, spans,
-                               gated)
-    if out is None and gated:
+        out = ops.lora_product(x, weight, None, a_stack, b_stack, slots, scales, spans, gate)
+    if out is None:
         y = base()
-        out = ops.lora_product(x, None, y, a_stack, b_stack, CTX.token_slots, scales, spans, True)
+        if gate:
+            out = ops.lora_product(x, None, y, a_stack, b_stack, slots, scales, spans, True)
         if out is None:
-            out = ops.silu_and_mul(apply_lora(layer_idx, projs, x, y))
-    return out
+            gate = False
+            if y.is_contiguous():
+                ops.lora_delta(y, x, a_stack, b_stack, slots, scales, spans)
+                out = y
+            else:
+                out = apply_lora(layer_idx, projs, x, y)
+    return ops.silu_and_mul(out) if gated and not gate else out
 
 
 def apply_lora(

@@ -97,7 +97,7 @@ class MergedColumnParallelLinear(nn.Module):
 
             layer_idx, projs = lora
             y = lora_linear(layer_idx, projs, x, _as_it_is(self) if self.bias is None else None,
-                            None)
+                            lambda: _linear_fwd(self, x))
             if y is None:
                 y = apply_lora(layer_idx, projs, x, _linear_fwd(self, x))
             return y
@@ -136,23 +136,24 @@ class RowParallelLinear(nn.Module):
         self.weight = _init_weight((out_size, self.in_per_rank), dtype)
         self.bias = _init_weight((out_size,), dtype, std=0.0) if bias else None
 
+    def _product(self, x: torch.Tensor) -> torch.Tensor:
+        qbits = getattr(self, "quant_bits", None)
+        if qbits is not None:
+            return ops.linear_quant(x, self.weight_q, self.weight_scale, qbits)
+        return ops.linear(x, self.weight)
+
     def forward(self, x: torch.Tensor, lora=None) -> torch.Tensor:
-        y = None
         if lora is not None:
             # delta added BEFORE the all-reduce: A is input-sharded, so the
             # per-rank partial deltas sum to the full LoRA delta
             from ..engine.lora import apply_lora, lora_linear
 
             layer_idx, projs = lora
-            y = lora_linear(layer_idx, projs, x, _as_it_is(self), None)
-        if y is None:
-            qbits = getattr(self, "quant_bits", None)
-            if qbits is not None:
-                y = ops.linear_quant(x, self.weight_q, self.weight_scale, qbits)
-            else:
-                y = ops.linear(x, self.weight)
-            if lora is not None:
-                apply_lora(layer_idx, projs, x, y)
+            y = lora_linear(layer_idx, projs, x, _as_it_is(self), lambda: self._product(x))
+            if y is None:
+                y = apply_lora(layer_idx, projs, x, self._product(x))
+        else:
+            y = self._product(x)
         y = tp_all_reduce(y)
         if self.bias is not None:
             y = y + self.bias
