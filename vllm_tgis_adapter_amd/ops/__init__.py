@@ -299,6 +299,15 @@ def _plain_tensors(*tensors: torch.Tensor) -> bool:
                for t in tensors)
 
 
+def _tiles_take(m: int, n: int, k: int) -> bool:
+    """Whether ``linear`` has the tiles of gemm_ring.hip make an aligned product."""
+    max_m = int(os.environ.get("VTA_GEMM_MAX_M", "64"))
+    if m <= 64:
+        return m <= max_m and _C.gemm_ring_wins(m, n, k, False)
+    return m > max_m and (_C.gemm_ring_wins(m, n, k, False)
+                          or m in _block_rows(n, k) and n % 128 == 0 and k % 64 == 0)
+
+
 def _block_rows(n: int, k: int) -> range:
     """Rows of a product past 64 that the tiles with a cut K take from the library: where K
     is so long, and 128 x 128 tiles so few, that K can be cut over three workgroups and
@@ -572,13 +581,11 @@ def lora_product(
     product, or where tensors do not suit."""
     given = weight if y is None else y
     rows, width = x.shape[0], given.shape[0 if y is None else 1]
-    if (not native_enabled(x) or given.dtype != torch.bfloat16 or not given.is_contiguous()
+    if not native_enabled(x) or (y is None and not _tiles_take(rows, width, x.shape[1])):
+        return None
+    if (given.dtype != torch.bfloat16 or not given.is_contiguous()
             or width % 2 or not slots.is_contiguous() or not scales.is_contiguous()
             or not _plain_tensors(x, given, a_stack, b_stack)):
-        return None
-    if y is None and not (_C.gemm_ring_wins(rows, width, x.shape[1], False)
-                          or (rows > 64 and rows in _block_rows(width, x.shape[1])
-                              and width % 128 == 0 and x.shape[1] % 64 == 0)):
         return None
     out = torch.empty((rows, width // 2 if gated else width), dtype=x.dtype, device=x.device)
     _C.lora_product(out, x, None if y is not None else weight, y, a_stack, b_stack, slots, scales,
