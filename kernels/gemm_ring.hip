@@ -9,8 +9,8 @@
 // 14336: our 128 x 128 tiles before) -> here, cold weights, rows x N x K:
 //   gated 8192 x 14336 x 4096 1426 -> 1316; 2049 x 14336 x 4096 413 -> 382; 512 x 14336 x 4096
 //     108 -> 96; 512 x 8192 x 2048 43 -> 35; 192 x 2048 x 2048 16 -> 10
-//   plain 512 x 4096 x 14336 85 -> 70; 65 x 4096 x 14336 38 -> 29; 192 x 4096 x 4096 33 -> 20;
-//     128 x 6144 x 4096 27 -> 20
+//   plain 512 x 4096 x 14336 84 -> 69; 65 x 4096 x 14336 37 -> 26; 192 x 4096 x 4096 33 -> 19;
+//     128 x 6144 x 4096 26 -> 20; 128 x 8192 x 28672 113 -> 93
 // What did not pay: tiles of 256 x 128 beside 128 x 256 (within 1 %), five slots of 128 x 128
 // (2 % here and there), 64 x 256.
 
@@ -85,74 +85,95 @@ __global__ __launch_bounds__(256, OCC) void gemm_ring_kernel(
   }
 }
 
-// A tile's form and what its time is made of, in us, fitted to some 2000 measured products
-// (24 shapes of W of the presets and their shards, 17 to 8192 rows; standard deviation 8 to
-// 12 %): the start, a workgroup's start and end and its tiles of 64 inputs, alone on its CU and
-// in pairs, and a second launch for parts of K.
+// A tile's form and what its time is made of, in us, fitted to some 25000 measured products of 65
+// to 4096 rows (50 shapes of W of the presets and their shards, weights from HBM; standard
+// deviation 6 %), then moved a little towards the better choices: the start; a workgroup's start
+// and end and its tiles of 64 inputs, alone on its CU and in pairs, less a share for rows that
+// do not exist; the reading of W, more with every further tile of rows up to five; and a second
+// launch for parts of K.  The share of empty rows and `again` are of the whole.
 struct Form {
   int bm, bn, pairs;
-  double start, own, one, two, merge, merge_mb, w_mb;
+  double start, own, one, two, merge, merge_mb, merge_part, w_mb, again, empty;
 };
 constexpr Form kForms[] = {
-    {256, 256, 1, 0.0, 8.3, 1.13, 1.13, 4.1, 0.16, 0.24},
-    {128, 256, 1, 0.0, 2.4, 0.76, 0.76, 4.4, 0.21, 0.21},
-    {128, 128, 2, 1.5, 0.3, 0.48, 1.00, 3.9, 0.20, 0.21},
-    {64, 128, 2, 2.3, 0.0, 0.34, 0.77, 3.2, 0.21, 0.20},
+    {256, 256, 1, 0.14, 12.0, 1.07, 1.07, 2.3, 0.125, 1.10, 0.186, 0.52, 0.0},
+    {128, 256, 1, 0.20, 5.4, 0.77, 0.77, 4.9, 0.120, 0.55, 0.170, 0.31, 0.39},
+    {128, 128, 2, 2.46, 2.0, 0.53, 0.97, 2.8, 0.142, 0.26, 0.167, 0.36, 0.30},
+    {64, 128, 2, 3.00, 0.4, 0.38, 0.74, 3.1, 0.154, 0.16, 0.180, 0.23, 0.60},
+    {64, 64, 2, 2.83, 0.5, 0.27, 0.53, 2.1, 0.202, 0.14, 0.205, 0.07, 0.60},
 };
-// The fifth form, 64 x 64 for up to 64 rows, is not fitted: few_rows below (gated: not cut).
-constexpr int kFew = 4, kForm4Cols = 64;
+constexpr int kNarrow = 3, kFew = 4, kFormCount = 5;   // 64 x 128, 64 x 64
 
 struct Plan {
   int form, parts;
   double us;
 };
 
+// parts of K without an empty one
+int even_parts(int K, int parts) {
+  const int depth = (K / 64 + parts - 1) / parts;
+  return (K / 64 + depth - 1) / depth;
+}
+
 // Up to 64 rows x is one tile and W comes by once: workgroups of 64 rows of W, as many as there
 // are CUs (K cut), or two a CU where that leaves a quarter of them idle or K stays long, and W
-// past the caches.  us, the streaming kernel | 64 x 128 by the model below | here, N x K, 24 |
+// past the caches.  us, the streaming kernel | 64 x 128 by a cost model | here, N x K, 24 |
 // 64 rows: 28672 x 4096 44.7 48.8 39.9 | 52.2 49.9 47.3; 4096 x 14336 26.8 27.7 24.1 | 37.3 29.4
 // 28.8; 6144 x 4096 15.9 15.4 14.8 | 21.6 17.3 18.1; 4096 x 4096 12.1 12.7 11.5 | 16.5 14.2 12.6;
 // 16384 x 2048 16.6 17.1 15.5 | 20.6 19.2 16.5; 8192 x 28672 83 83 75 | 101 90 96.  Workgroups 128,
-// 256, 512 at 8192 x 28672, 24 rows: 130, 90, 75; at 4096 x 14336 64, 128, 256, 512: 54, 33, 24, 27.
-int few_rows(int M, int N, int K) {
-  if (M > 64 || (M > 48 && K >= 8192 && (long)N * K > 80000000)) return 0;
+// 256, 512 at 8192 x 28672, 24 rows: 130, 90, 75; at 4096 x 14336 64, 128, 256, 512: 54, 33, 24, 27;
+// 172 and 344 at 11008 x 4096: 20.2, 24.2.
+// Short K is cut less, eight tiles a part: 40 rows, 3072 x 2048 in 4 8.9 (in 5 9.4, whole 10.7), 8192
+// x 1024 whole 7.3 (in 2 8.0).  Past 48 rows of very many weights the tile of 128 columns reads x half
+// as often: 64 rows, 57344 x 8192 175 | 183, 8192 x 28672 in 4 90 | 96 (14336 x 8192 60 | 47, 28672 x
+// 8192 98 | 89, 10240 x 8192 in 3 37 | 38).
+Plan few_rows(int M, int N, int K) {
   const int cols = N / 64, tiles = K / 64;
   int parts = 256 / cols;
   if (parts < 1) parts = 1;
-  if (cols * parts < 192) parts = 512 / cols;
+  if (cols * parts < 192 && 512 / cols > 2) parts = 512 / cols;
   if (tiles / parts > 128 && cols * parts <= 256) parts *= 2;
   if (parts > 8) parts = 8;
-  if (parts > tiles / 6) parts = tiles / 6;
+  const int most = tiles < 32 ? 1 : tiles < 64 ? tiles / 8 : tiles / 6;
+  if (parts > most) parts = most;
   if (parts < 1) parts = 1;
-  const int depth = (tiles + parts - 1) / parts;
-  return (tiles + depth - 1) / depth;
+  const bool wide = M > 48 && K >= 8192 && (K >= 16384 || (long)N * K > 400000000);
+  return Plan{wide && N % 128 == 0 ? kNarrow : kFew, even_parts(K, parts), 0.0};
 }
 
 // The form and the parts of K (of six tiles at least) that the model gives the least time.  It
-// picks what is 3 % slower than the best of all at the mean of the measured sizes, 1 % gated.
+// picks what is 0.5 % slower than the best of all at the mean of the measured sizes, 6 % at one in
+// a hundred.  A cut tile's workgroups go where blockIdx.x does, eight XCDs of 32 CUs in turn:
+// rounds are counted there (84 tiles in three parts are 33 workgroups on some XCDs, two rounds,
+// though all are 252: 1.5 times the time of 80 tiles).
 Plan plan_of(int M, int N, int K, bool gated) {
-  if (gated && M <= 64) return Plan{kFew, 1, 0.0};
-  if (const int parts = gated ? 0 : few_rows(M, N, K)) return Plan{kFew, parts, 0.0};
+  if (M <= 64) return gated ? Plan{kFew, 1, 0.0} : few_rows(M, N, K);
   Plan best{0, 1, 1e30};
   const double cols = gated ? 2.0 * N : N, w_mb = cols * K * 2e-6;
-  for (int f = 0; f < 4; ++f) {
+  for (int f = 0; f < kFormCount; ++f) {
     const Form& form = kForms[f];
     if ((long)(gated ? 2 : 1) * N % form.bn) continue;
-    const long blocks = (M + form.bm - 1) / form.bm * (long)(cols / form.bn);
+    const long m_tiles = (M + form.bm - 1) / form.bm, blocks = m_tiles * (long)(cols / form.bn);
+    const double full_rows = 1.0 - form.empty * (1.0 - (double)M / (m_tiles * form.bm));
+    const double read =
+        w_mb * form.w_mb * (1.0 + form.again * (m_tiles > 5 ? 4 : m_tiles - 1));
     for (int parts = 1; parts <= 8; ++parts) {
       const int depth = (K / 64 + parts - 1) / parts;
-      if (parts > 1 && (gated || depth < 6 || (K / 64 + depth - 1) / depth != parts ||
-                        blocks * parts > 1024 || (double)parts * M * N > 64e6))
+      if (parts > 1 && (gated || depth < 6 || even_parts(K, parts) != parts ||
+                        blocks * parts > 1400 || (double)parts * M * N > 64e6))
         continue;
-      const long all = blocks * parts, round = 256 * form.pairs;
+      const long all = (blocks + 7) / 8 * parts, round = 32 * form.pairs;   // of an XCD
       const long full = all / round, rest = all % round;
-      const bool alone = rest > 0 && rest <= 256;
-      const double work =
-          (alone ? form.own + depth * form.one : 0.0) +
-          (full + (rest > 0 && !alone)) * (form.own + depth * form.two);
-      const double read = w_mb * form.w_mb, w2 = work * work, r2 = read * read;
-      const double us = form.start + sqrt(sqrt(w2 * w2 + r2 * r2)) +
-                        (parts > 1 ? form.merge + form.merge_mb * parts * M * (double)N * 8e-6 : 0);
+      const bool alone = rest > 0 && rest <= 32;
+      const double work = full_rows * ((alone ? form.own + depth * form.one : 0.0) +
+                                       (full + (rest > 0 && !alone)) *
+                                           (form.own + depth * form.two));
+      const double w2 = work * work, r2 = read * read;
+      const double us =
+          form.start + sqrt(sqrt(w2 * w2 + r2 * r2)) +
+          (parts > 1 ? form.merge + form.merge_mb * parts * M * (double)N * 8e-6 +
+                           form.merge_part * (parts - 2)
+                     : 0);
       if (us < best.us) best = Plan{f, parts, us};
     }
   }
@@ -172,22 +193,25 @@ void launch_form(__hip_bfloat16* y, float* part, const __hip_bfloat16* x, const 
 template <bool GATED>
 void launch_plan(__hip_bfloat16* y, float* part, const __hip_bfloat16* x, const __hip_bfloat16* w,
                  int M, int N, int K, int plan, hipStream_t stream) {
-  const int parts = plan & 15;
-  switch (plan >> 4) {
-    case 0: launch_form<256, 256, 4, 1, GATED>(y, part, x, w, M, N, K, parts, stream); break;
-    case 1: launch_form<128, 256, 4, 1, GATED>(y, part, x, w, M, N, K, parts, stream); break;
-    case 2: launch_form<128, 128, 4, 2, GATED>(y, part, x, w, M, N, K, parts, stream); break;
-    case 3: launch_form<64, 128, 6, 2, GATED>(y, part, x, w, M, N, K, parts, stream); break;
-    default:
-      {
-        // W that is read once and is large goes past the caches (24 rows: 28672 x 4096 46.4 ->
-        // 39.9 us, 8192 x 3584 15.6 -> 13.8, 4096 x 4096 11.5 -> 11.5; 64 rows 12.6 -> 13.5)
-        if (M <= 64 && (GATED ? 2L : 1L) * N * K >= 20000000)
-          launch_form<64, 64, 8, 2, GATED, 2>(y, part, x, w, M, N, K, parts, stream);
-        else
-          launch_form<64, 64, 8, 2, GATED>(y, part, x, w, M, N, K, parts, stream);
-      }
+  const int parts = plan & 15, form = plan >> 4;
+  // W that is read once and is large goes past the caches (24 rows by 64 x 64: 28672 x 4096 46.4 ->
+  // 39.9 us, 8192 x 3584 15.6 -> 13.8, 4096 x 4096 11.5 -> 11.5, 64 rows 12.6 -> 13.5; larger tiles, all
+  // rows in one: 8192 x 8192 by 128 x 128 0.88 of the time, 4096 x 14336 0.91, 5120 x 8192 0.97, but
+  // 7168 x 4096 1.02, 6144 x 4096 1.05)
+  const bool once = M <= kForms[form].bm &&
+                    (GATED ? 2L : 1L) * N * K >= (form == kFew ? 20000000 : 40000000);
+#define GO(BM, BN, SLOTS, OCC)                                                         \
+  if (once) launch_form<BM, BN, SLOTS, OCC, GATED, 2>(y, part, x, w, M, N, K, parts, stream); \
+  else launch_form<BM, BN, SLOTS, OCC, GATED>(y, part, x, w, M, N, K, parts, stream); \
+  break
+  switch (form) {
+    case 0: GO(256, 256, 4, 1);
+    case 1: GO(128, 256, 4, 1);
+    case 2: GO(128, 128, 4, 2);
+    case 3: GO(64, 128, 6, 2);
+    default: GO(64, 64, 8, 2);
   }
+#undef GO
 }
 
 // rows of W are found by 32 bits
@@ -210,30 +234,52 @@ int gemm_ring_plan(int M, int N, int K, bool gated) {
 // Whether a plan is one: a tile's columns fit, no part of K is empty.
 bool gemm_ring_takes(int N, int K, int plan, bool gated) {
   const int form = plan >> 4, parts = plan & 15;
-  if (plan < 0 || form > kFew || parts < 1 || parts > (gated ? 1 : 8)) return false;
-  const int depth = (K / 64 + parts - 1) / parts;
-  const int bn = form == kFew ? kForm4Cols : kForms[form].bn;
-  return (gated ? 2L : 1L) * N % bn == 0 && (K / 64 + depth - 1) / depth == parts;
+  if (plan < 0 || form >= kFormCount || parts < 1 || parts > (gated ? 1 : 8)) return false;
+  return (gated ? 2L : 1L) * N % kForms[form].bn == 0 && even_parts(K, parts) == parts;
+}
+
+// Rows of a plain product past 64 that the tiles take because K is so long, and tiles of 128 x
+// 128 so few, that K can be cut over three workgroups and more.  Time over the library's, weights
+// from HBM, N x K: first and last row of the rule, and the one past it:
+//   1280 x 8192: 257 0.73, 700 0.84; 2048 x 8192: 129 0.65, 700 0.83; 2560 x 8192: 224 0.73, 512
+//   0.86, 513 0.85; 4096 x 14336: 65 0.58, 640 0.77, 700 0.86; 5120 x 8192: 65 0.82, 512 0.81, 513
+//   1.06; 7168 x 8192: 65 0.87, 384 0.94, 448 0.87; 8192 x 8192: 65 0.87, 256 0.69, 340 1.12; 8192 x
+//   14336: 65 0.69, 256 0.59, 340 0.92; 10240 x 8192: 65 0.45, 256 0.65, 257 1.02.
+// (7168 x 8192, 301 to 384 rows, are 4 to 10 % slower than eight-wave tiles with two whole tiles of
+// K in LDS were there.)
+bool gemm_block_takes(long M, long N, long K) {
+  if (K < 8192 || N > 12288 || N < 128) return false;
+  if (N < 2048) return M >= 257 && M <= 700;
+  if (N < 2560) return M >= 129 && M <= 700;
+  if (N < 3072) return M >= 200 && M <= 512;
+  const long last = 168 / (N / 128) * 128;
+  return M >= 65 && M <= (last < 700 ? last : 700);
 }
 
 // Whether these tiles take a product from what would run it otherwise.  Time over that one's,
-// cold weights, N x K: rows.
-//  Against gemm_stream.hip's, 9 to 64 rows: 28672 x 4096 0.90 to 0.94; 4096 x 14336 0.77 to
-//   0.90; 4096 x 4096 17 0.98, 64 0.76; 512 x 4096 0.96 to 0.66; 3072 x 2048 17 1.08, 40 0.95, 64
-//   0.91; 2048 x 2048 32 1.12, 40 0.97.  2 | 12 rows: 28672 x 4096 0.99 | 0.94, 10240 x 8192 0.89 |
-//   0.86, 2048 x 8192 0.96 | 0.94, 16384 x 2048 0.98 | 0.93, 4096 x 14336 1.02 | 0.97, 14336 x 4096
-//   1.04 | 0.97; 6144 x 4096 1.13 | 1.10, 4096 x 7168 1.13 | 1.06, 8192 x 3584 1.07 | 1.03.
-//  Against the library's:
-//   65 to 256 rows: 4096 x 4096 0.60 to 0.99; 6144 x 4096 0.76 to 1.00; 4096 x 14336 0.82 to
-//   0.97; 8192 x 8192 0.89 to 1.02; 2560 x 8192 0.54 to 0.90; 12288 and 14336 x 4096 and 8192
-//   0.88 to 1.10, 28672 x 4096 0.99 to 1.14, 3072 x 2048 0.82 to 1.27, 1024 x 4096 1.11 to 1.25.
-//   301 to 1024, long K: 4096 x 14336 0.81 to 0.97; 2048 x 8192 0.89 to 1.00; 8192 x 28672 0.63
-//   to 1.12; others around 1: 4096 x 4096 0.97 to 1.16, 6144 x 4096 1.01 to 1.17.
+// weights from HBM, N x K: rows.
+//  Against gemm_stream.hip's, 9 to 64 rows: 28672 x 4096 0.94 to 0.92; 4096 x 14336 12 1.03, 17
+//   0.93, 64 0.79; 4096 x 4096 17 1.04, 32 0.97, 64 0.82; 2048 x 4096 17 1.06, 32 1.0, 64 0.85; 8192 x
+//   2048 17 0.83; 16384 x 2048 12 0.83; 10240 x 8192 12 0.83, 64 0.96; 14336 x 8192 0.90 to 0.85; 8192
+//   x 28672 0.89 to 0.91.  Left there: 12 rows of 6144 x 4096 1.05, 8192 x 4096 1.05 to 1.12 (half of
+//   the CUs without a tile, or K cut), 8192 x 3584 1.08; short K, 40 | 64 rows: 4096 x 1024 1.08 |
+//   1.05, 4096 x 1792 1.15 | 1.13, 2048 x 1024 1.15 | 1.13, where 8192 x 1024 has 0.74 | 0.69 and
+//   4864 x 896 0.88 | 0.87 (past 4096 columns the streaming workgroups are more than CUs).
+//   (Taken with K of 2048: 3072 x 2048 1.06 | 1.02, 4096 x 2048 1.06 | 1.04.)
+//  Against the library's, plain:
+//   65 to 256 rows, K from 3584 on: 4096 x 4096 0.58 to 0.95; 6144 x 4096 0.64 to 0.93; 4096 x 14336
+//   0.41 to 0.78; 8192 x 4096 0.75 to 1.01; 2048 x 4096 0.84 to 0.96; 14336 x 4096 0.90 to 1.04.
+//   257 to 1024, long K: 4096 x 14336 0.64 to 0.86; 2048 x 8192 0.74 to 0.91; 1280 x 8192 0.71 to
+//   0.89; 8192 x 28672 0.59 to 1.00, 513 to 768 rows 0.99 to 1.09, 900 0.96, 1024 0.93; others around 1: 4096 x 4096 0.91 to
+//   1.17, 6144 x 4096 0.92 to 1.13.
 //  Gated, against gemm_stream.hip's, 17 | 64 rows: 14336 x 4096 0.91 | 0.92, 6144 x 4096 0.86 |
 //   0.82, 8192 x 2048 0.85 | 0.83, 7168 x 8192 1.01 | 0.79, 8192 x 8192 1.06 | 0.75, 11008 x 4096
-//   1.07 | 0.80, 28672 x 8192 0.92 | 1.06; against the library's and its gate, where the model is below 0.92 of the library's
-//   (fitted likewise): 8192 x 2048 0.78 to 0.93; 14336 x 4096 0.88 to 0.99 (768 rows: 1.07);
-//   28672 x 8192 0.88 to 0.97 (256: 1.05); 4096 x 2048 0.54 to 0.94; 1024 x 2048 0.68 to 1.14.
+//   1.07 | 0.80, 28672 x 8192 0.92 | 1.06.
+//  Gated, past 64 rows, against the library's product (or the plain one by these tiles, where they
+//   take it) and its gate: where the model is below 1.05 of a model of the library's fitted likewise
+//   (14 %), below 0.98 for tiles of 256 x 256, whose last round costs most, and below 0.9 of its own
+//   for the plain one.  8192 x 2048 0.78 to 0.93; 14336 x 4096 0.88 to 0.99 (340 rows: 1.04); 28672
+//   x 8192 0.80 to 0.99; 4096 x 2048 0.54 to 1.00; 2048 x 2048 0.55 to 0.94.
 bool gemm_ring_wins(long M, long N, long K, bool gated) {
   if (!fits(M, N, K, gated)) return false;
   if (gated) {
@@ -243,17 +289,22 @@ bool gemm_ring_wins(long M, long N, long K, bool gated) {
       return M > 32 || (blocks <= 256 ? K < 8192 : blocks >= 400);
     }
     if (N * K < 4000000) return false;
-    const double tf = 4e-9 * M * N * K / 1.334;
-    const double mb = (4e-6 * N * K + 2e-6 * M * (2.0 * N + K)) * 0.202;
-    const double library = 12.9 + sqrt(tf * tf + mb * mb) + 0.6e-6 * M * N;
-    return plan_of(M, N, K, true).us < 0.92 * library;
+    const Plan plan = plan_of(M, N, K, true);
+    if (gemm_block_takes(M, 2 * N, K) || gemm_ring_wins(M, 2 * N, K, false))
+      return plan.us < 0.9 * (plan_of(M, 2 * N, K, false).us + 2.5 + 1.2e-6 * M * N);
+    const double products = 4e-9 * M * N * K / 1.294;
+    const double bytes = 4e-6 * N * K * 0.179 + 2e-6 * M * (2.0 * N + K) * 0.39;
+    const double library = 12.9 + sqrt(products * products + bytes * bytes);
+    return plan.us < (plan.form == 0 ? 0.98 : 1.05) * library;
   }
-  if (M <= 16) return M > 8 && (K >= 8192 ? N * K >= 16000000 : N * K >= 33000000);
-  if (M <= 64)
-    return N * K >= 2000000 && (K >= 4096 || N * K >= 16000000 || M >= 40);
+  if (M <= 16) return M > 8 && (K >= 8192 ? N * K >= 16000000 : N * K >= 33000000 && N >= 12288);
+  if (M <= 64) {
+    if (K >= 4096 || N * K >= 16000000) return N * K >= 2000000;
+    return M >= 40 && (N > 4096 ? N * K >= 2000000 : K >= 2048 && N * K >= 6000000);
+  }
   if (N * K < 6000000) return false;
   if (M <= 256) return K >= 3584 && N <= 10240;
-  return M <= 1024 && 2 * K >= 7 * N;
+  return M <= 1024 && 2 * K >= 7 * N && (N * K <= 100000000 || M <= 512 || M > 832);
 }
 
 // N % 128 == 0, K % 64 == 0, 0 < K < 2^23, x, W and y from 16-byte boundaries on

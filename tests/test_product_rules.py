@@ -21,3 +21,44 @@ def test_int8_panels_lie_inside_32_bits(n, k):
         assert plan > 1
         rows, cols = PANELS[(plan >> 8) - 1]
         assert 16 * rows * k * 2 < 1 << 32 and 64 * cols * k < 1 << 32
+
+
+# sizes at which the model's first form was off by 4 to 25 %, and the tiles (form << 4 | parts of K)
+# that measured within 4 % of the best
+PLANS = [
+    (96, 8192, 28672, False, {24, 36}), (128, 8192, 28672, False, {24, 36}),
+    (301, 1280, 8192, False, {39, 40}), (640, 1280, 8192, False, {36}),
+    (256, 8192, 8192, False, {6, 20, 34}), (340, 7168, 8192, False, {35}),
+    (96, 8192, 14336, False, {36}), (384, 5120, 8192, False, {20}), (128, 2048, 4096, False, {68}),
+    (160, 1536, 4096, False, {67}), (1024, 4096, 14336, False, {4}),
+    (512, 4096, 14336, False, {6, 7, 20}), (56, 14336, 8192, False, {65}),
+    (40, 3072, 2048, False, {67, 68}), (40, 8192, 1024, False, {65}),
+    (24, 11008, 4096, False, {65}), (24, 10240, 4096, False, {51, 65, 67}),
+    (224, 28672, 8192, True, {1}), (128, 3584, 4096, True, {65})]
+
+
+@pytest.mark.parametrize(("m", "n", "k", "gated", "plans"), PLANS)
+def test_plans_that_measured_well(m, n, k, gated, plans):
+    assert ops._C.gemm_ring_plan(m, n, k, gated) in plans
+
+
+@pytest.mark.parametrize(("m", "n", "k"), [
+    (640, 8192, 28672),                                    # the library is faster
+    (48, 4096, 1024), (64, 4096, 1792), (40, 2048, 1024),  # the streaming kernel is: short K
+    (12, 8192, 4096), (16, 8192, 4096)])                   # a K that would be cut
+def test_products_the_tiles_leave(m, n, k):
+    assert not ops._C.gemm_ring_wins(m, n, k, False) and not ops._C.gemm_block_takes(m, n, k)
+
+
+@pytest.mark.parametrize("gated", [False, True])
+def test_plans_are_plans(gated):
+    """Columns in whole tiles, no empty part, whatever the sizes."""
+    bn = [256, 256, 128, 128, 64]
+    for m in (1, 9, 64, 65, 129, 300, 1024, 5000):
+        for n in (128, 384, 640, 1280, 4096, 28672):
+            for k in (64, 128, 448, 832, 2112, 4096, 12352, 28672):
+                plan = ops._C.gemm_ring_plan(m, n, k, gated)
+                form, parts = plan >> 4, plan & 15
+                assert (1 + gated) * n % bn[form] == 0 and 1 <= parts <= (1 if gated else 8)
+                depth = -(-(k // 64) // parts)
+                assert -(-(k // 64) // depth) == parts

@@ -240,8 +240,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
     roofline (tools/gemm_bench.py); the hand-written MFMA kernel streams the
     weight matrix once with waves splitting K in-workgroup.  Larger M stays
     on hipBLASLt (VTA_GEMM_MAX_M raises the cutover for experiments) but for
-    the rows and inputs of ``_block_rows`` and where ``gemm_ring_wins``
-    (gemm_ring.hip) says that the tiles here are faster.
+    what ``gemm_block_takes`` and ``gemm_ring_wins`` (gemm_ring.hip) say that
+    the tiles here do faster.
     """
     max_m = int(os.environ.get("VTA_GEMM_MAX_M", "64"))
     tile_max_m = int(os.environ.get("VTA_GEMM_TILE_MAX_M", "0"))
@@ -269,7 +269,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
             )
             _C.gemm_tile(out, x, weight)
             return out
-        if (m > max_m and m in _block_rows(weight.shape[0], x.shape[1])
+        if (m > max_m and _C.gemm_block_takes(m, weight.shape[0], x.shape[1])
                 and _plain_tensors(x, weight)):
             out = torch.empty(
                 (m, weight.shape[0]), dtype=x.dtype, device=x.device
@@ -305,27 +305,7 @@ def _tiles_take(m: int, n: int, k: int) -> bool:
     if m <= 64:
         return m <= max_m and _C.gemm_ring_wins(m, n, k, False)
     return m > max_m and (_C.gemm_ring_wins(m, n, k, False)
-                          or m in _block_rows(n, k) and n % 128 == 0 and k % 64 == 0)
-
-
-def _block_rows(n: int, k: int) -> range:
-    """Rows of a product past 64 that the tiles with a cut K take from the library: where K
-    is so long, and 128 x 128 tiles so few, that K can be cut over three workgroups and
-    more.  Time over the library's, cold weights (with 128 x 128 tiles only; gemm_ring.hip's
-    choice is faster at every size measured, 4096 x 14336: 128 0.46, 512 0.78), N x K: rows:
-      1024 x 8192: 160 1.13, 257 0.94, 512 1.04, 700 0.86;  2048 x 8192: 128 1.11, 129 0.91,
-      700 0.87;  2560 x 8192: 160 1.00, 200 0.91, 512 0.85, 513 1.16;  4096 x 14336: 65 0.84,
-      128 0.56, 512 0.96, 640 0.83, 700 1.15;  5120 x 8192: 65 1.06, 129 1.03, 256 0.60, 512
-      0.95, 513 1.24;  8192 x 8192: 65 0.99, 144 1.05, 256 0.72, 300 1.10;  8192 x 28672: 65
-      0.54, 256 0.53, 384 1.20;  10240 x 8192: 128 0.85, 256 0.77, 257 1.17;  12288 x 8192:
-      128 0.90, 129 1.08;  14336 x 8192: 65 1.07, 128 1.13;  57344 x 8192: 160 1.32."""
-    if k < 8192 or n > 12288:
-        return range(0)
-    if n < 2048:
-        return range(257, 701)
-    if n < 3072:
-        return range(129, 701) if n < 2560 else range(200, 513)
-    return range(65, min(700, 168 // (n // 128) * 128) + 1)
+                          or _C.gemm_block_takes(m, n, k) and n % 128 == 0 and k % 64 == 0)
 
 
 def gemm_tile(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
