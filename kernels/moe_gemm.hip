@@ -77,6 +77,34 @@ __global__ __launch_bounds__(256, OCC) void moe_ring_kernel(
   }
 }
 
+}  // namespace
+
+// Which tile the products of more than some 52 rows an expert take: 0 256 x 256, 1 128 x 256, 2
+// 128 x 128 (rows x columns of W), by the mean of the rows and, since a tile that runs alone on
+// its CU takes as long as a full round of them, by how many tiles there are: us, 256 x 256 | 128 x 256
+// | 128 x 128, experts x between (in), rows an expert, evenly spread, tiles of 256 x 256:
+//   gated: 8 x 1792 (4096), 125, 112: 72 | 44 | 55; 4 x 512 (1024), 160, 16: 25 | 15 | 11; 8 x 3584
+//   (4096), 160, 224: 117 | 129 | 140 (unevenly, 200: 173 | 135 | 153); 8 x 7168 (4096), 448, 200: 204 |
+//   251 | 268.
+//   plain: 8 of 4096 (14336), 222, 128: 298 | 235 | 281 (unevenly 294 | 402 | 369), 249, 256: 299 | 418
+//   | 390; 8 of 4096 (3584), 222, 128: 65 | 49 | 53; 16 of 2048 (2048), 222, 128: 43 | 31 | 33; 4 of 1024
+//   (512), 160, 16: 16 | 10 | 8; 16 of 4096 (3584), 222, 256: 107 | 133 | 145.
+int moe_tile(int mean, int experts, long columns, int K, bool gated) {
+  if (columns % 256 != 0) return 2;
+  auto tiles = [&](long mean, long rows) {
+    return (mean + rows - 1) / rows * experts * (columns / 256);
+  };
+  if (gated) {
+    if (mean > (K >= 4096 ? 110 : 150) && tiles(mean, 256) >= 192) return 0;
+    return mean > 52 && K >= 4096 ? 1 : 2;
+  }
+  // some experts have more rows than the mean: from 228 on they are counted as two tiles
+  if (mean > 220 && tiles(mean * 9L / 8, 256) >= 192) return 0;
+  return mean > 110 && tiles(mean, 128) >= 128 ? 1 : 2;
+}
+
+namespace {
+
 template <int MODE>
 void launch_mode(__hip_bfloat16* y, const __hip_bfloat16* x, const __hip_bfloat16* w,
                  const int* seg_off, const int* x_rows, int E, int N, int K, int T,
@@ -103,6 +131,7 @@ void launch_mode(__hip_bfloat16* y, const __hip_bfloat16* x, const __hip_bfloat1
   // and with 16 experts, 2048 in and between, where 128 x 256 are too few:
   //   64: 59* 66 - / 33* 37 -;  125: 69* 79 74 / 42 41* 46;  200: 89 81 78* / 43 42* 50.
   // (The eight-wave tiles before these took, gated / plain, 64: 357 / 227, 200: 529 / 269.)
+  // Which of the tiles, and where they are too few for the chip: moe_tile below.
   //
   // That is with even loads.  The streaming form's workgroups, a chunk of 64 rows an expert and
   // two a CU, fill whole rounds at usual widths, and a few experts with more rows start another
@@ -122,15 +151,10 @@ void launch_mode(__hip_bfloat16* y, const __hip_bfloat16* x, const __hip_bfloat1
   else if (mean <= 9) STREAM(1, 2, 2);
   else if (mean <= 18 && moe::gated(MODE)) STREAM(2, 2, 2);
   else if (far || (mean <= 52 && !brim)) STREAM(4, 4, 2);
-  else if (N * cols % 256 != 0) TILES(128, 128, 5, 2);
-  else if (moe::gated(MODE)) {
-    if (mean > (K >= 4096 ? 110 : 150)) TILES(256, 256, 4, 1);
-    else if (mean > 52 && K >= 4096) TILES(128, 256, 4, 1);
-    else TILES(128, 128, 5, 2);
-  } else {
-    if (mean > 220) TILES(256, 256, 4, 1);
-    else if (mean > 110) TILES(128, 256, 4, 1);
-    else TILES(128, 128, 5, 2);
+  else switch (moe_tile(mean, E, N * cols, K, moe::gated(MODE))) {
+    case 0: TILES(256, 256, 4, 1); break;
+    case 1: TILES(128, 256, 4, 1); break;
+    default: TILES(128, 128, 5, 2);
   }
 #undef STREAM
 #undef TILES
