@@ -267,7 +267,10 @@ void launch_block(__hip_bfloat16* y, const __hip_bfloat16* x, const unsigned cha
 // Panels (gemm_panel_q.h) and how their time adds up, us: what a tile of 64 inputs takes with
 // one workgroup on a CU and with as many as share one.  Fitted to some 5000 times (ten matrices
 // from 1024 x 4096 to 28672 x 4096, 70 to 2048 rows, K cut over one to eight workgroups; 7 % rms);
-// what it chooses is 1.1 % off the fastest panel in the mean.
+// what it chooses is 0.9 % off the fastest panel in the mean (over 420 sizes, weights from memory).
+// Workgroups are dealt to XCDs of 32 CUs, so rounds are counted there: over the whole chip a few
+// more workgroups than CUs look like a second round that no XCD need have, and the other way
+// around (1.2 % in the mean; 1280 x 8192, 800 rows 45 | 32 us, 1536 x 4096, 560 rows 20.6 | 18.1).
 struct Panel {
   int tm, tn, per_cu;
   float one, full;
@@ -278,10 +281,11 @@ constexpr Panel kPanels[] = {{5, 1, 2, .232f, .423f}, {5, 2, 2, .347f, .598f},
                              {10, 2, 1, .550f, .550f}, {10, 4, 1, .985f, .985f}};
 
 float panel_us(const Panel& p, int M, int N, int K, int parts) {
-  const int wgs = (M + p.tm * 16 - 1) / (p.tm * 16) * (N / (p.tn * 64)) * parts;
-  const int tiles = (K / 64 + parts - 1) / parts, round = 256 * p.per_cu, left = wgs % round;
+  const int blocks = (M + p.tm * 16 - 1) / (p.tm * 16) * (N / (p.tn * 64));
+  const int wgs = (blocks + 7) / 8 * parts;   // of an XCD
+  const int tiles = (K / 64 + parts - 1) / parts, round = 32 * p.per_cu, left = wgs % round;
   float us = 2.6f + wgs / round * (p.full * tiles + 3.4f);
-  if (left > 0) us += (left > 256 ? p.full : p.one) * tiles + 3.4f;
+  if (left > 0) us += (left > 32 ? p.full : p.one) * tiles + 3.4f;
   if (parts > 1) us += 2.1f + 1.6e-6f * parts * M * N;   // their merge
   return us;
 }

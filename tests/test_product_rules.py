@@ -23,6 +23,15 @@ def test_int8_panels_lie_inside_32_bits(n, k):
         assert 16 * rows * k * 2 < 1 << 32 and 64 * cols * k < 1 << 32
 
 
+@pytest.mark.parametrize(("m", "n", "k", "plans"), [
+    # rounds of an XCD, of which counting the chip's took the slower: panel, parts of K
+    (800, 1280, 8192, {(1, 4), (6, 4), (5, 3), (1, 2)}), (560, 1536, 4096, {(0, 3), (2, 3)}),
+    (1100, 768, 4096, {(2, 3), (3, 2)})])
+def test_int8_panels_are_counted_by_xcd(m, n, k, plans):
+    plan = ops._C.gemm_panel_plan(m, n, k)
+    assert ((plan >> 8) - 1, plan & 255) in plans
+
+
 # sizes at which the model's first form was off by 4 to 25 %, and the tiles (form << 4 | parts of K)
 # that measured within 4 % of the best
 PLANS = [

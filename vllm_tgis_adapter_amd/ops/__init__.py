@@ -357,9 +357,12 @@ def dequantize_weight(wq: torch.Tensor, scales: torch.Tensor, qbits: int,
 def _quant_rows(qbits: int, n: int, k: int) -> int:
     """Most rows of a product that widens its weights itself.  Above, the second pass
     over the widened matrix costs less than the library's faster product saves (us, own
-    | widened for the library): int8 28672 x 4096 900 rows 225 | 245, 1200 rows 294 | 295,
-    6144 x 4096 900 rows 54 | 71, 2048 rows 113 | 98, 16384 x 2048 900 rows 74 | 75,
-    2048 x 2048 1500 rows 23 | 28; 4 bits 28672 x 4096 301 rows 129 | 136, 448 rows
+    | widened for the library): int8 28672 x 4096 900 rows 227 | 236, 1200 rows 294 | 300,
+    8192 x 8192 1200 rows 141 | 161, 1400 rows 198 | 185, 6144 x 4096 900 rows 54 | 71, 2048
+    rows 113 | 98, 2048 x 2048 1500 rows 23 | 28; below the line some large ones lose, but
+    with weights as they are instead of rounded to bf16: 10240 x 8192 900 rows 146 | 175,
+    1000 rows 190 | 180, 1200 rows 222 | 199, 14336 x 8192 900 rows 240 | 227, 1100 rows
+    254 | 279, 32000 x 2048 1000 rows 151 | 141; 4 bits 28672 x 4096 301 rows 129 | 136, 448 rows
     176 | 157, 4096 x 14336 80 rows 58 | 67, 150 rows 78 | 72."""
     if n * k <= 1 << 23:
         return 1500 if qbits == 8 else 1000
