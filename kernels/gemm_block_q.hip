@@ -290,13 +290,27 @@ float panel_us(const Panel& p, int M, int N, int K, int parts) {
   return us;
 }
 
+// Small matrices of short K stay with the tiles of launch_block while those are at most one to a CU,
+// or three to nearly every one (as many as fit): there is nothing to share that a panel would save.
+// us, tiles | panels: 768 x 768, 430 rows 5.5 | 6.6, 1000 rows 6.6 | 6.9; 128 x 512, 1000 rows
+// 4.6 | 5.5; 3072 x 768, 1000 rows (768 tiles) 10.8 | 12.7.  Past one to a CU panels are up to 25 %
+// faster (2048 x 1024, 640 rows, 320 tiles 9.7 | 8.0), and with few tiles of longer K, which
+// panels cut, 10 % (128 x 2048).  (Below 256 inputs and past 320 rows panels are taken as before.)
+bool small_tiles(int M, int N, int K) {
+  if (K > 2048 || (long)N * K > 1 << 23) return false;
+  if (M <= 320) return true;
+  const long tiles = (M + 63L) / 64 * (N / 64);
+  if (tiles > 736 && tiles <= 768) return K >= 256 && K <= 1024;
+  return K >= 256 && tiles <= 256 && (K <= 1536 || tiles > 64);
+}
+
 }  // namespace
 
 // Which panel, and how many workgroups K is cut over (each leaves a part of the result in f32),
 // of eight tiles of 64 inputs at least: (panel << 8 | parts), or 1 where tiles of
-// gemm_block_q_kernel do.  A function of shapes.
+// gemm_block_q_kernel do (small_tiles).  A function of shapes.
 int gemm_panel_plan(int M, int N, int K) {
-  if (K <= 2048 && (long)N * K <= 1 << 23 && M <= 320) return 1;
+  if (small_tiles(M, N, K)) return 1;
   int plan = 0;
   float least = 0.f;
   for (int i = 0; i < (int)(sizeof(kPanels) / sizeof(kPanels[0])); ++i) {

@@ -32,6 +32,15 @@ def test_int8_panels_are_counted_by_xcd(m, n, k, plans):
     assert ((plan >> 8) - 1, plan & 255) in plans
 
 
+@pytest.mark.parametrize(("m", "n", "k", "tiles"), [
+    (430, 768, 768, True), (1000, 768, 768, True), (1000, 128, 512, True), (1000, 3072, 768, True),
+    (400, 2048, 1024, True), (640, 2048, 1024, False), (800, 3072, 768, False),
+    (512, 128, 2048, False), (512, 4096, 2048, False)])
+def test_int8_small_matrices(m, n, k, tiles):
+    """Tiles of the whole K while they are one round."""
+    assert (ops._C.gemm_panel_plan(m, n, k) == 1) == tiles
+
+
 # sizes at which the model's first form was off by 4 to 25 %, and the tiles (form << 4 | parts of K)
 # that measured within 4 % of the best
 PLANS = [
