@@ -55,7 +55,7 @@ void launch_gemm_ring(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hi
                       int, int, int, bool, hipStream_t);
 void launch_gemm_stream(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hip_bfloat16*,
                         int, int, int, int, hipStream_t);
-bool gemm_row_fits(int qbits, int K);
+bool gemm_row_fits(int K);
 void launch_gemm_row_norm_gated(__hip_bfloat16*, __hip_bfloat16*, const __hip_bfloat16*,
                                 const __hip_bfloat16*, const __hip_bfloat16*, float, const void*,
                                 const float*, int, int, int, hipStream_t);
@@ -451,7 +451,7 @@ __hip_bfloat16* check_row_norm(const torch::Tensor& x, const c10::optional<torch
     row(*sum);
     TORCH_CHECK(sum->data_ptr() != residual->data_ptr() && sum->data_ptr() != x.data_ptr());
   }
-  TORCH_CHECK(rows % 128 == 0 && K % 64 == 0 && gemm_row_fits((int)qbits, (int)K));
+  TORCH_CHECK(rows % 128 == 0 && K % 64 == 0 && gemm_row_fits((int)K));
   TORCH_CHECK(w.is_cuda() && w.dim() == 2 && w.size(0) == rows && w.is_contiguous() &&
               reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0);
   if (qbits == 16) {

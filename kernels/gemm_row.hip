@@ -429,7 +429,7 @@ void launch_bits(const RowCall& c, int qbits) {
 }  // namespace
 
 // x is kept in LDS
-bool gemm_row_fits(int qbits, int K) { return K <= 28672; }
+bool gemm_row_fits(int K) { return K <= 28672; }
 
 // N % 128 == 0, K % 64 == 0 (rounded weights: K % 128 == 0)
 void launch_gemm_row(__hip_bfloat16* y, const __hip_bfloat16* x, const void* w,

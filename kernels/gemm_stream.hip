@@ -181,7 +181,7 @@ int gemm_stream_parts(int qbits, int M, int N, int K, bool gated) {
   return parts;
 }
 
-bool gemm_row_fits(int qbits, int K);
+bool gemm_row_fits(int K);
 void launch_gemm_row(__hip_bfloat16* y, const __hip_bfloat16* x, const void* w,
                      const float* scale, int qbits, int N, int K, bool gated,
                      hipStream_t stream);
@@ -190,7 +190,7 @@ void launch_gemm_row(__hip_bfloat16* y, const __hip_bfloat16* x, const void* w,
 void launch_gemm_stream(__hip_bfloat16* y, float* part, const __hip_bfloat16* x,
                         const __hip_bfloat16* w, int M, int N, int K, int parts,
                         hipStream_t stream) {
-  if (M == 1 && gemm_row_fits(16, K))
+  if (M == 1 && gemm_row_fits(K))
     launch_gemm_row(y, x, w, nullptr, 16, N, K, false, stream);
   else
     launch_q<16, false>(y, part, x, w, nullptr, M, N, K, parts, stream);
@@ -199,7 +199,7 @@ void launch_gemm_stream(__hip_bfloat16* y, float* part, const __hip_bfloat16* x,
 void launch_gemm_stream_gated(__hip_bfloat16* y, float* part, const __hip_bfloat16* x,
                               const __hip_bfloat16* w13, int M, int I, int K, int parts,
                               hipStream_t stream) {
-  if (M == 1 && gemm_row_fits(16, K))
+  if (M == 1 && gemm_row_fits(K))
     launch_gemm_row(y, x, w13, nullptr, 16, I, K, true, stream);
   else
     launch_q<16, true>(y, part, x, w13, nullptr, M, I, K, parts, stream);
@@ -208,7 +208,10 @@ void launch_gemm_stream_gated(__hip_bfloat16* y, float* part, const __hip_bfloat
 void launch_gemm_stream_q(__hip_bfloat16* y, float* part, const __hip_bfloat16* x,
                           const unsigned char* wq, const float* scale, int qbits, int M, int N,
                           int K, int parts, hipStream_t stream) {
-  if (M == 1 && gemm_row_fits(qbits, K))
+  // int8 of short K: a workgroup of gemm_row.hip has one segment of a row or less (us, here |
+  // there: 768 x 768 2.7 | 3.0, 4096 x 1024 3.2 | 3.5, 2048 x 1024 3.0 | 3.2; 1024 x 2048
+  // 3.7 | 3.2, 2048 x 2048 3.8 | 3.5)
+  if (M == 1 && gemm_row_fits(K) && !(qbits == 8 && K <= 1024))
     launch_gemm_row(y, x, wq, scale, qbits, N, K, false, stream);
   else if (qbits == 8)
     launch_q<8, false>(y, part, x, wq, scale, M, N, K, parts, stream);

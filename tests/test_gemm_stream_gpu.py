@@ -137,6 +137,19 @@ def test_one_row(n, k):
            5 * (x.double().abs() @ exact.abs().t() + size))
 
 
+@pytest.mark.parametrize(("n", "k"), [(128, 128), (768, 768), (4096, 1024), (128, 1152),
+                                      (768, 28672), (128, 28800)])
+def test_one_row_of_int8(n, k):
+    """Both sides of the shortest and the longest rows of the kernel for one."""
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    x, w = _x(1, k, 28), _x(n, k, 29)
+    wq, scale = ops.quantize_weight(w, 8)
+    exact = (wq.double() * scale.double()[:, None]).t()
+    _check(ops.linear_quant(x, wq, scale, 8), x.double() @ exact, x.double().abs() @ exact.abs())
+
+
 def _at_odd_offset(t):
     flat = torch.zeros(t.numel() + 1, dtype=t.dtype, device=t.device)
     out = flat[1:].view(t.shape)
