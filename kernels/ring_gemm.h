@@ -47,13 +47,24 @@ struct Ring {
   static_assert((SLOTS - 1) * kLoads < 64, "vmcnt has six bits");
 
   // A sum stays in its accumulation registers: all 256 are in use, and the compiler's own
-  // choice copies some of them in every turn.
+  // choice copies some of them in every turn.  Written out, a product is no matrix instruction
+  // to the compiler, which adds no wait states: a form is sound only if between the products
+  // sums are neither copied nor spilled and fragments come from LDS alone, and if `settle` is
+  // the first to follow the last product.  tests/test_ring_products.py looks for that in the
+  // built code; a new form, or a new compiler, has to pass it.
   static DEVINLINE void multiply(f32x4_t& acc, const bf16x8_t& a, const bf16x8_t& b) {
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
   }
-  // 18 wait states lie between a product and what reads its sum without the matrix unit
-  static DEVINLINE void settle(f32x4_t (&acc)[kTM][kTN]) {
-    asm volatile("s_nop 15\n\ts_nop 7");
+  // 18 wait states at most lie between a product and what reads its sum without the matrix
+  // unit.  They are taken in the loop, behind the last product of the last turn: on the way out
+  // of it the compiler copies sums.  One block, since a branch of its own would be moved there too.
+  static DEVINLINE void settle(int turn, int turns) {
+    asm volatile("s_cmp_lt_i32 %0, %1\n\ts_cbranch_scc1 1f\n\ts_nop 15\n\ts_nop 7\n1:"
+                 ::"s"(turn), "s"(turns) : "scc");
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // (the compiler would spill some of 256 that it takes to be wanted elsewhere)
+  static DEVINLINE void keep(f32x4_t (&acc)[kTM][kTN]) {
 #pragma unroll
     for (int i = 0; i < kTM; ++i)
 #pragma unroll
@@ -224,11 +235,13 @@ struct Ring {
                 ask1);
         quarter(kHM, kHN, fa1, fb1, 2 * kHN, [&](int q) { read_b(fb0, there1, q); }, kLoads / 2,
                 kLoads, ask1);
+        __builtin_amdgcn_sched_barrier(0);
+        settle(t + 2, n);
         advance();
       }
     }
     block_gemm::wait_loads<0>();
-    settle(acc);
+    keep(acc);
   }
 };
 

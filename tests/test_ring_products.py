@@ -1,0 +1,71 @@
+"""Products written in assembly (ring_gemm.h) get no wait states from the compiler: in the built
+kernels nothing but the products touches a sum between the first and the last of them, and a
+fragment comes from LDS, not from another vector instruction right ahead of its product."""
+
+from __future__ import annotations
+
+import os
+import re
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+
+ROCM = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
+PACKAGE = Path(__file__).resolve().parent.parent / "vllm_tgis_adapter_amd"
+OBJDUMP = shutil.which("llvm-objdump", path=f"{ROCM}/llvm/bin:{os.environ.get('PATH', '')}")
+PRODUCT = "v_mfma_f32_16x16x32_bf16"
+
+
+def _registers(operand: str) -> set[int]:
+    found = re.fullmatch(r"v\[(\d+):(\d+)\]|v(\d+)", operand.strip())
+    if not found:
+        return set()
+    if found[3]:
+        return {int(found[3])}
+    return set(range(int(found[1]), int(found[2]) + 1))
+
+
+def _kernels(name: str, tmp_path: Path):
+    shutil.copy(PACKAGE / name, tmp_path / name)
+    subprocess.run([OBJDUMP, "--offloading", name], cwd=tmp_path, check=True, capture_output=True)
+    for code in sorted(tmp_path.glob(f"{name}.*gfx950")):
+        listing = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", "--no-leading-addr", code],
+                                 check=True, capture_output=True, text=True).stdout
+        for part in re.split(r"^<(?=\w*_ring_kernel)", listing, flags=re.M)[1:]:
+            lines = [line.split("//")[0].strip() for line in part.splitlines()]
+            end = lines.index("") if "" in lines else len(lines)
+            yield lines[0].rstrip(">:"), lines[1:end]
+
+
+@pytest.mark.skipif(OBJDUMP is None, reason="no llvm-objdump")
+@pytest.mark.parametrize(("name", "least"), [("_C.so", 32), ("_C_seq.so", 12)])
+def test_sums_and_fragments_stay_in_place(name, least, tmp_path):
+    if not (PACKAGE / name).exists():
+        pytest.skip("the extension is not built")
+    kernels = 0
+    for kernel, body in _kernels(name, tmp_path):
+        at = [i for i, line in enumerate(body) if line.startswith(PRODUCT)]
+        assert at, kernel
+        kernels += 1
+        for line in body[at[0]:at[-1]]:
+            assert "accvgpr" not in line and "scratch_" not in line, (kernel, line)
+        for i in at:
+            to, a, b, c = (o.strip() for o in body[i][len(PRODUCT):].split(",")[:4])
+            assert to == c and c.startswith("a["), (kernel, body[i])
+            # two wait states lie between a vector instruction and the product that reads what
+            # it wrote; here four instructions, whatever they are
+            read = _registers(a) | _registers(b)
+            assert len(read) in (4, 8), (kernel, body[i])
+            for line in body[max(0, i - 4):i]:
+                if line.startswith("v_") and not line.startswith((PRODUCT, "v_cmp")):
+                    wrote = _registers(line.split(None, 1)[1].split(",")[0])
+                    assert not read & wrote, (kernel, line, body[i])
+        # what reads a sum first waits for the last product
+        behind = body[at[-1] + 1:]
+        behind = behind[:next(i for i, line in enumerate(behind) if re.search(r"\ba\[?\d", line))]
+        waits = sum(int(line.split()[1], 0) + 1 if line.startswith("s_nop") else 1
+                    for line in behind)
+        assert waits >= 18, (kernel, behind)
+    assert kernels >= least
