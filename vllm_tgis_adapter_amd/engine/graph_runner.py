@@ -134,10 +134,12 @@ class DecodeGraphRunner:
         return n * (32 + 4 * w)
 
     @torch.inference_mode()
-    def run_packed(self, packed: torch.Tensor, n: int, w: int) -> torch.Tensor:
+    def run_packed(self, packed: torch.Tensor, n: int, w: int,
+                   read: "torch.cuda.Event | None" = None) -> torch.Tensor:
         """run() with the inputs in one pinned uint8 buffer: int64 ids, positions and slots [n]
         each, int32 lengths [n], state slots [n] (unused without sequence state) and block
-        tables [n, w].  The buffer is read when the stream gets there."""
+        tables [n, w].  The buffer is read when the stream gets there: `read` says so, ahead
+        of the step itself."""
         from .. import ops
 
         b = self.bucket_for(n)
@@ -145,5 +147,7 @@ class DecodeGraphRunner:
         ops.decode_inputs(
             packed, self.in_ids, self.in_pos, self.in_slots, self.in_seq_lens,
             self.in_state_slots if self.with_seq_state else None, self.in_block_tables, n, w, b)
+        if read is not None:
+            read.record()
         self.graphs[b].replay()
         return self.out_logits[b][:n]

@@ -647,9 +647,7 @@ class Worker:
         if self.uses_seq_state:
             ints[n:2 * n] = batch["state_slots"]
         ints[2 * n:].reshape(n, w)[:] = tables
-        logits = self.graph_runner.run_packed(buf, n, w)
-        read.record()
-        return logits
+        return self.graph_runner.run_packed(buf, n, w, read)
 
     @torch.inference_mode()
     def execute_batch(self, batch: dict) -> Optional[torch.Tensor]:
