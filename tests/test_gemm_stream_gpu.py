@@ -245,6 +245,53 @@ def test_parts_of_k(m, n, k):
                5 * (x.double().abs() @ exact.abs().t() + size))
 
 
+# what aligned tensors still reach of the cuts for more than 16 rows in bf16 (the rest of
+# test_plain, test_gated_cuts and test_parts_of_k has the tiles of gemm_ring.hip): K over several
+# workgroups, over one, and the gated cut for many columns
+@pytest.mark.parametrize(("m", "n", "k", "gated"), [
+    (33, 4096, 3072, False), (39, 5120, 2944, False), (33, 5120, 1792, False),
+    (39, 12288, 1024, False), (17, 12288, 640, True), (49, 12288, 12288, True)])
+def test_cuts_of_aligned_tensors(m, n, k, gated):
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    assert not ops._C.gemm_ring_wins(m, n, k, gated)
+    x, w = _x(m, k, 30), _x(n * (1 + gated), k, 31) / k ** 0.5
+    want, terms = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    if gated:
+        g, u = want.chunk(2, dim=1)
+        _check(ops.gated_mlp_up(x, w), torch.nn.functional.silu(g) * u,
+               30 * (1 + g.abs()) * (1 + u.abs()))
+    else:
+        _check(ops.linear(x, w), want, terms)
+
+
+# and the same cuts where the tiles refuse a tensor, which starts four bytes off their boundary
+@pytest.mark.parametrize("which", ["x", "w"])
+@pytest.mark.parametrize(("m", "n", "k", "gated"), [
+    (17, 6144, 4096, False), (25, 7168, 4224, False), (17, 10240, 3200, False),
+    (49, 5120, 8192, False), (49, 16384, 2048, False), (17, 20480, 8192, True),
+    (25, 7168, 4096, True), (49, 14336, 4096, True)])
+def test_cuts_of_tensors_off_a_boundary(which, m, n, k, gated):
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    assert ops._C.gemm_ring_wins(m, n, k, gated)
+    x, w = _x(m, k, 32), _x(n * (1 + gated), k, 33) / k ** 0.5
+    flat = torch.zeros((x if which == "x" else w).numel() + 2, dtype=x.dtype, device="cuda")[2:]
+    if which == "x":
+        x = flat.view(x.shape).copy_(x)
+    else:
+        w = flat.view(w.shape).copy_(w)
+    want, terms = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    if gated:
+        g, u = want.chunk(2, dim=1)
+        _check(ops.gated_mlp_up(x, w), torch.nn.functional.silu(g) * u,
+               30 * (1 + g.abs()) * (1 + u.abs()))
+    else:
+        _check(ops.linear(x, w), want, terms)
+
+
 @pytest.mark.parametrize("m", [1025, 1041])
 def test_rounded_largest_tiles(m):
     """Wide matrices of few inputs, past 4096 blocks of 64 x 128."""
