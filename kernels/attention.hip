@@ -1,4 +1,4 @@
-// Paged-KV attention kernels (SURVEY.md E3/E4).
+// Paged-KV attention kernels.
 //
 // Cache layout: [num_blocks, block_size, kv_heads, head_dim]; a (slot, head)
 // row is head_dim contiguous elements (256 B at hd=128 bf16).

@@ -1,5 +1,5 @@
 // Prompt attention with a window, sinks, chunks, prefixes or capped scores over the paged
-// KV cache (SURVEY.md E3; plain causal attention: attention_prefill_tile.hip): KVBLK=64
+// KV cache (plain causal attention: attention_prefill_tile.hip): KVBLK=64
 // tiles, a zero-conflict XOR-16 K image, hardware transpose reads (ds_read_b64_tr_b16) for
 // the V fragments, async staging (global loads issued under softmax+PV), defer-max
 // rescaling, and exp2 with the softmax scale folded into the logits.

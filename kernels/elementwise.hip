@@ -1,6 +1,5 @@
 // SiLU-mul activation, NeoX rotary embedding, paged-KV cache write
-// (SURVEY.md E6 / E3-E4 support ops).  All memory-bound: 16-B vector
-// accesses, f32 math, grid-stride loops.
+// support.  All memory-bound: 16-B vector accesses, f32 math.
 
 #include "common.h"
 
@@ -124,7 +123,7 @@ void launch_reshape_and_cache(const T* k, const T* v, T* kc, T* vc,
                      0, s, k, v, kc, vc, slots, row_elems, k_stride, v_stride);
 }
 
-// fp8 KV cache (SURVEY E5 + E18 adjacency): bf16 K/V quantized to OCP e4m3
+// fp8 KV cache: bf16 K/V quantized to OCP e4m3
 // at cache-write time; halves the decode-attention HBM stream and doubles
 // KV capacity in the 288 GB pool.
 __global__ void reshape_and_cache_fp8_kernel(

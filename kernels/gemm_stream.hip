@@ -1,5 +1,6 @@
 // Products of few rows with a whole weight matrix (decode, M <= 64; a single row:
-// gemm_row.hip):
+// gemm_row.hip; aligned bf16 of more than 8 rows, where they are faster: the tiles of
+// gemm_ring.hip):
 //   y[m, n] = sum_k x[m, k] W[n, k],  or  silu(x Wg^T) * (x Wu^T) for W = [Wg; Wu],
 // with W in bf16, in int8 (a scale per row) or in 4 bits (offset 8, a scale per row
 // and 128 inputs).
@@ -27,6 +28,8 @@
 //   23 rows, 14336 x 4096 gated 55.2 -> 43.4; the mean of 6144 x 4096, 4096 x 4096 and
 //     4096 x 14336 23.9 -> 17.5 (a llama-3-8b layer reads W at 4.5 TB/s);
 //   61 rows, the mean of these three and 28672 x 4096: 38.1 -> 30.
+// (In bf16 the tiles have taken over from there at 23 and 61 rows; in rounded weights, up to 16
+// rows, short K and small matrices these kernels are what runs.)
 
 #include "gemm_stream.h"
 

@@ -1,4 +1,4 @@
-// Decode-batch tile GEMMs (SURVEY.md E6): y[M,N] = x[M,K] @ W[N,K]^T, bf16.
+// Decode-batch tile GEMMs: y[M,N] = x[M,K] @ W[N,K]^T, bf16.
 //
 // Two tilings:
 //  * gemm_tile_kernel   — 128x128 macro-tile, 4 waves, glds-staged (r2 first

@@ -1,4 +1,4 @@
-// Batched multi-LoRA products (SURVEY.md E12).
+// Batched multi-LoRA products.
 //
 // Mixed-adapter batches carry a per-token adapter slot (-1 = no adapter); weights of the
 // active adapters are stacked host-side, for up to three projections of one input side

@@ -1,4 +1,4 @@
-// Grouped products over experts' segments (SURVEY.md E16): one launch covers every
+// Grouped products over experts' segments: one launch covers every
 // expert's rows of the batch sorted by expert,
 //
 //   h[r, :]  = silu(x[r]·Wg_e^T) * (x[r]·Wu_e^T)   (gated, w13 = [E, 2I, H])

@@ -1,5 +1,5 @@
-// Fused RMSNorm kernels (SURVEY.md E6).
-// Memory-bound: one workgroup per row, 16-B vector loads (guide G13 — scalar
+// Fused RMSNorm kernels.
+// Memory-bound: one workgroup per row, 16-B vector loads (scalar
 // bf16 loads cost ~2x), sum-of-squares in f32, one pass read + one pass write.
 //
 // Of a step's rows what counts is the chain of latencies.  Rows of up to 8192 (f32: 4096)

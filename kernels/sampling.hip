@@ -1,4 +1,4 @@
-// Fused sampling kernel (SURVEY.md E7).
+// Fused sampling kernel.
 //
 // For rows without top-k/top-p filtering (the serving common case), sampling
 // from softmax(logits/T) with per-request exponential noise q reduces to

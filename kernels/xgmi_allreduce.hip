@@ -1,4 +1,4 @@
-// Direct-xGMI one-shot all-reduce (SURVEY.md E15).
+// Direct-xGMI one-shot all-reduce.
 //
 // MI355X xGMI is point-to-point (7 links x ~153 GB/s per GPU), so a ring
 // all-reduce pays 2*S*(N-1)/N bytes per link; the one-shot form — every rank

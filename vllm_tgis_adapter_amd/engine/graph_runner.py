@@ -1,4 +1,4 @@
-"""hipGraph capture of the decode step (SURVEY.md E24).
+"""hipGraph capture of the decode step.
 
 Steady-state decode batches are launch-bound (dozens of small kernels per
 layer); capturing the whole forward + logits computation per batch-size

@@ -1,4 +1,4 @@
-"""Multi-LoRA runtime (SURVEY.md E12).
+"""Multi-LoRA runtime.
 
 Hot-loads PEFT LoRA adapters (adapter_config.json + adapter_model.safetensors)
 onto the serving model and applies them per request in mixed batches.

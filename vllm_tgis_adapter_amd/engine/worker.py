@@ -1,6 +1,6 @@
 """GPU worker: owns the model, the paged KV cache, and step execution.
 
-One worker per GPU (one process per GPU for TP>1; SURVEY.md E14/E15).  Rank 0
+One worker per GPU (one process per GPU for TP>1).  Rank 0
 drives: it turns a SchedulerOutput into a flat token batch, broadcasts it to
 the other TP ranks (torch.distributed over RCCL/gloo), runs the forward, and
 samples.  Non-zero ranks sit in ``worker_loop`` executing broadcast commands.

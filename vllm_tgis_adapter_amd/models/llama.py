@@ -1,4 +1,4 @@
-"""Llama-3-class decoder (SURVEY.md E6): RMSNorm + rotary GQA attention over
+"""Llama-3-class decoder: RMSNorm + rotary GQA attention over
 the paged KV cache + SwiGLU MLP, TP-sharded.
 
 Hot elementwise/normalisation work goes through the fused HIP ops

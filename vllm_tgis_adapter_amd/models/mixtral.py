@@ -1,4 +1,4 @@
-"""Mixtral-class MoE decoder (SURVEY.md E6/E16).
+"""Mixtral-class MoE decoder.
 
 Same attention stack as llama; the MLP is a top-k routed mixture of SwiGLU
 experts.  Experts are TP-sharded on the intermediate dimension (every rank

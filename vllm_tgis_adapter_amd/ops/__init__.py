@@ -3,8 +3,7 @@
 GPU tensors run the hand-written CDNA4 HIP kernels from the in-tree ``_C``
 extension (kernels/ — built by ``__graft_entry__.build()`` for gfx950).  CPU
 tensors run the plain-PyTorch reference (ops/reference.py), which keeps the
-full engine runnable in CPU-only CI like the reference's CPU vLLM build
-(SURVEY.md §4).  On a GPU box a missing extension is a hard error — there is
+full engine runnable in CPU-only CI like the reference's CPU vLLM build.  On a GPU box a missing extension is a hard error — there is
 deliberately no silent eager fallback.
 """
 
@@ -317,7 +316,7 @@ def gemm_tile(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 
 
 # ---------------------------------------------------------------------------
-# Weight-only quantization (SURVEY.md E18): RTN into int8 (per-out-channel
+# Weight-only quantization: RTN into int8 (per-out-channel
 # scale) or packed int4 with group-128 scales (the --quantize awq/gptq/
 # squeezellm 4-bit surface; offline RTN since checkpoint-specific scales
 # don't exist in this environment).

@@ -1,4 +1,4 @@
-"""TP-sharded layers (SURVEY.md E14).
+"""TP-sharded layers.
 
 Column-parallel linears hold an [out/tp, in] shard and emit parallel
 activations; row-parallel linears hold [out, in/tp] and all-reduce their
@@ -44,7 +44,7 @@ def _as_it_is(mod: nn.Module) -> torch.Tensor | None:
 
 
 def _init_weight(shape, dtype, std: float = 0.006) -> nn.Parameter:
-    # Random-init path for synthetic benchmarking (BASELINE measures on
+    # Random-init path for synthetic benchmarking (which measures on
     # random-init weights); real checkpoints overwrite via load_weights.
     w = torch.empty(shape, dtype=dtype)
     w.normal_(mean=0.0, std=std)
