@@ -50,6 +50,7 @@ void launch_gemm_ring_parts(__hip_bfloat16*, float*, const __hip_bfloat16*,
 bool gemm_ring_takes(int N, int K, int plan, bool gated);
 bool gemm_ring_wins(long M, long N, long K, bool gated);
 bool gemm_block_takes(long M, long N, long K);
+int gemm_tiles_route(long M, long N, long K);
 int moe_tile(int mean, int experts, long columns, int K, bool gated);
 void launch_gemm_ring(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hip_bfloat16*, int,
                       int, int, int, bool, hipStream_t);
@@ -938,6 +939,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("x"), py::arg("w"), py::arg("gated") = false, py::arg("plan") = 0);
   m.def("gemm_ring_wins", &gemm_ring_wins, "whether the large tiles are the faster product");
   m.def("moe_tile", &moe_tile, "which tile expert products of many rows take");
+  m.def("gemm_tiles_route", &gemm_tiles_route,
+        "past 64 rows: 1 for their cut K, 2 otherwise, 0 where the library is faster");
   m.def("gemm_block_takes", &gemm_block_takes, "whether they are for their cut K");
   m.def("gemm_ring_plan", &gemm_ring_plan, "which tile a product takes, and parts of K (form << 4 | parts)");
   m.def("decode_inputs", &decode_inputs, "a captured step's inputs from a packed host buffer");

@@ -307,6 +307,12 @@ bool gemm_ring_wins(long M, long N, long K, bool gated) {
   return M <= 1024 && 2 * K >= 7 * N && (N * K <= 100000000 || M <= 512 || M > 832);
 }
 
+// Both questions of a plain product past 64 rows: 1 gemm_block_takes, 2 gemm_ring_wins, 0 neither
+int gemm_tiles_route(long M, long N, long K) {
+  if (M <= 64) return 0;
+  return gemm_block_takes(M, N, K) ? 1 : gemm_ring_wins(M, N, K, false) ? 2 : 0;
+}
+
 // N % 128 == 0, K % 64 == 0, 0 < K < 2^23, x, W and y from 16-byte boundaries on
 void launch_gemm_ring(__hip_bfloat16* y, float* part, const __hip_bfloat16* x,
                       const __hip_bfloat16* w, int M, int N, int K, int plan, bool gated,

@@ -92,3 +92,13 @@ def test_plans_are_plans(gated):
 def test_expert_tiles_fill_the_chip(mean, experts, columns, k, gated, tile):
     """Large tiles only where there are enough of them."""
     assert ops._C.moe_tile(mean, experts, columns, k, gated) == tile
+
+
+def test_one_question_for_both_rules():
+    """What linear asks says what the two rules say, the cut first, and nothing up to 64 rows."""
+    for m in (1, 17, 64, 65, 129, 300, 640, 1024, 5000):
+        for n in (128, 1280, 2048, 4096, 8192, 28672):
+            for k in (64, 2048, 4096, 8192, 28672):
+                block, ring = ops._C.gemm_block_takes(m, n, k), ops._C.gemm_ring_wins(m, n, k, False)
+                want = 0 if m <= 64 else 1 if block else 2 if ring else 0
+                assert ops._C.gemm_tiles_route(m, n, k) == want

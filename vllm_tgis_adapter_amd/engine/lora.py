@@ -23,6 +23,7 @@ from typing import Optional
 
 import torch
 
+from .. import ops
 from ..parallel import get_tp_rank, get_tp_world_size
 
 # projection name -> (parallel kind, hf targets)
@@ -90,8 +91,6 @@ def set_context(token_lora_ids: Optional[torch.Tensor], adapters: dict[int, LoRA
     CTX.slot_ids = new_slot_ids
     CTX.token_slots = None
     if token_lora_ids is not None and adapters:
-        from .. import ops
-
         CTX.token_slots = ops.lora_slots(token_lora_ids, CTX.slot_ids)
 
 
@@ -119,8 +118,6 @@ def _get_stacks(layer_idx: int, projs: list[tuple[str, int, int]], in_size: int,
         return None
     rank = max(a.weights[(layer_idx, name)][0].shape[0]
                for a in adapters for name, _, _ in have if (layer_idx, name) in a.weights)
-    from .. import ops
-
     rank = next((r for r in ops.LORA_RANKS if r >= rank), rank)
     L, width = len(adapters), sum(hi - lo for _, lo, hi in have)
     a_stack = torch.zeros((L, len(have) * rank, in_size), dtype=dtype, device=device)
@@ -141,8 +138,6 @@ def _get_stacks(layer_idx: int, projs: list[tuple[str, int, int]], in_size: int,
 
 def _batched(x: torch.Tensor) -> bool:
     """Whether the batched kernels take the deltas of this input."""
-    from .. import ops
-
     return (
         CTX.token_slots is not None
         and ops.native_enabled(x)
@@ -182,8 +177,6 @@ def lora_linear(
     stacks = _get_stacks(layer_idx, projs, x.shape[1], x.dtype, x.device)
     if stacks is None:
         return None
-    from .. import ops
-
     a_stack, b_stack, scales, spans = stacks
     slots = CTX.token_slots
     gate = False
@@ -215,8 +208,6 @@ def apply_lora(
 ) -> torch.Tensor:
     if not CTX.active:
         return out
-    from .. import ops
-
     # GPU: batched BGMV shrink/expand HIP kernels over the mixed batch (E12)
     if _batched(x) and out.is_contiguous():
         if x.dtype == torch.bfloat16 and len(projs) <= 3:

@@ -23,13 +23,8 @@ from ..parallel.layers import (
     ParallelLMHead,
     RowParallelLinear,
     VocabParallelEmbedding,
+    lora_active,
 )
-
-
-def lora_active() -> bool:
-    from ..engine.lora import CTX
-
-    return CTX.active
 
 
 def stored_weight(linear: nn.Module):
@@ -94,7 +89,7 @@ class Attention(nn.Module):
         """The norm, the projections, the rotation and the cache write of a step of one row
         in one launch: (q, residual), or None where that doesn't apply."""
         qkv = self.qkv_proj
-        if hidden.shape[0] != 1 or qkv.bias is not None or lora_active():
+        if qkv.bias is not None or lora_active():
             return None
         return ops.row_norm_qkv(
             hidden, residual, norm.weight, norm.eps, *stored_weight(qkv), self.num_heads,
@@ -147,7 +142,7 @@ class LlamaMLP(nn.Module):
     def row(self, hidden, residual, norm):
         """The norm and the feed-forward of a step of one row, the norm and the gate in the
         first product's launch: (hidden, residual), or None where that doesn't apply."""
-        if hidden.shape[0] != 1 or self.gate_up.bias is not None or lora_active():
+        if self.gate_up.bias is not None or lora_active():
             return None
         made = ops.row_norm_gated(hidden, residual, norm.weight, norm.eps,
                                   *stored_weight(self.gate_up))
@@ -158,10 +153,11 @@ class LlamaMLP(nn.Module):
 
 def attention_sublayer(layer, hidden, residual, positions, kv_cache, meta, cos_sin_cache):
     """A layer's first norm and attention: (hidden, residual) for the second norm."""
-    made = layer.attn.row_inputs(hidden, residual, layer.input_norm, positions, kv_cache, meta,
-                                 cos_sin_cache)
-    if made is not None:
-        return layer.attn.attend(made[0], kv_cache, meta), made[1]
+    if hidden.shape[0] == 1:
+        made = layer.attn.row_inputs(hidden, residual, layer.input_norm, positions, kv_cache,
+                                     meta, cos_sin_cache)
+        if made is not None:
+            return layer.attn.attend(made[0], kv_cache, meta), made[1]
     if residual is None:
         residual = hidden
         hidden = layer.input_norm(hidden)
@@ -181,9 +177,10 @@ class LlamaDecoderLayer(nn.Module):
     def forward(self, hidden, residual, positions, kv_cache, meta, cos_sin_cache):
         hidden, residual = attention_sublayer(
             self, hidden, residual, positions, kv_cache, meta, cos_sin_cache)
-        made = self.mlp.row(hidden, residual, self.post_norm)
-        if made is not None:
-            return made
+        if hidden.shape[0] == 1:
+            made = self.mlp.row(hidden, residual, self.post_norm)
+            if made is not None:
+                return made
         hidden, residual = self.post_norm(hidden, residual)
         hidden = self.mlp(hidden)
         return hidden, residual

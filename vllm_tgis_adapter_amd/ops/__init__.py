@@ -3,8 +3,9 @@
 GPU tensors run the hand-written CDNA4 HIP kernels from the in-tree ``_C``
 extension (kernels/ — built by ``__graft_entry__.build()`` for gfx950).  CPU
 tensors run the plain-PyTorch reference (ops/reference.py), which keeps the
-full engine runnable in CPU-only CI like the reference's CPU vLLM build.  On a GPU box a missing extension is a hard error — there is
-deliberately no silent eager fallback.
+full engine runnable in CPU-only CI like the reference's CPU vLLM build.  On a
+GPU box a missing extension is a hard error — there is deliberately no silent
+eager fallback.
 """
 
 from __future__ import annotations
@@ -239,10 +240,9 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
     roofline (tools/gemm_bench.py); the hand-written MFMA kernel streams the
     weight matrix once with waves splitting K in-workgroup.  Larger M stays
     on hipBLASLt (VTA_GEMM_MAX_M raises the cutover for experiments) but for
-    what ``gemm_block_takes`` and ``gemm_ring_wins`` (gemm_ring.hip) say that
-    the tiles here do faster.
+    what ``gemm_tiles_route`` (gemm_ring.hip) says that the tiles here do faster.
     """
-    max_m = int(os.environ.get("VTA_GEMM_MAX_M", "64"))
+    max_m = _gemm_max_m()
     tile_max_m = int(os.environ.get("VTA_GEMM_TILE_MAX_M", "0"))
     if (
         bias is None
@@ -268,19 +268,16 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
             )
             _C.gemm_tile(out, x, weight)
             return out
-        if (m > max_m and _C.gemm_block_takes(m, weight.shape[0], x.shape[1])
-                and _plain_tensors(x, weight)):
+        # (asked once: small steps are bound by the host, a question takes 0.3 us)
+        route = _C.gemm_tiles_route(m, weight.shape[0], x.shape[1]) if m > max_m else 0
+        if route and _plain_tensors(x, weight):
             out = torch.empty(
                 (m, weight.shape[0]), dtype=x.dtype, device=x.device
             )
-            _C.gemm_block(out, x, weight)
-            return out
-        if (m > max(max_m, 64) and _C.gemm_ring_wins(m, weight.shape[0], x.shape[1], False)
-                and _plain_tensors(x, weight)):
-            out = torch.empty(
-                (m, weight.shape[0]), dtype=x.dtype, device=x.device
-            )
-            _C.gemm_ring(out, x, weight)
+            if route == 1:
+                _C.gemm_block(out, x, weight)
+            else:
+                _C.gemm_ring(out, x, weight)
             return out
     return torch.nn.functional.linear(x, weight, bias)
 
@@ -300,11 +297,15 @@ def _plain_tensors(*tensors: torch.Tensor) -> bool:
 
 def _tiles_take(m: int, n: int, k: int) -> bool:
     """Whether ``linear`` has the tiles of gemm_ring.hip make an aligned product."""
-    max_m = int(os.environ.get("VTA_GEMM_MAX_M", "64"))
+    # (the rule first: reading the environment takes three times as long)
     if m <= 64:
-        return m <= max_m and _C.gemm_ring_wins(m, n, k, False)
-    return m > max_m and (_C.gemm_ring_wins(m, n, k, False)
-                          or _C.gemm_block_takes(m, n, k) and n % 128 == 0 and k % 64 == 0)
+        return _C.gemm_ring_wins(m, n, k, False) and m <= _gemm_max_m()
+    return (n % 128 == 0 and k % 64 == 0 and _C.gemm_tiles_route(m, n, k) != 0
+            and m > _gemm_max_m())
+
+
+def _gemm_max_m() -> int:
+    return int(os.environ.get("VTA_GEMM_MAX_M", "64"))
 
 
 def gemm_tile(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
@@ -405,7 +406,7 @@ def gated_mlp_up(x: torch.Tensor, w13: torch.Tensor) -> torch.Tensor | None:
     Returns None when the fused CDNA4 path doesn't apply (caller falls back
     to linear + silu_and_mul).
     """
-    max_m = int(os.environ.get("VTA_GEMM_MAX_M", "64"))
+    max_m = _gemm_max_m()
     if (
         x.dim() == 2
         and x.shape[0] >= 1
@@ -434,7 +435,7 @@ def _row_norm_usable(x, residual, norm_weight, weight, scales, qbits: int) -> bo
     """Whether a norm and the product of its one row are one launch: what the kernels of a
     single row take, and where gated_mlp_up and linear_quant would take their kernels too."""
     if (x.dim() != 2 or x.shape[0] != 1 or not native_enabled(x)
-            or int(os.environ.get("VTA_GEMM_MAX_M", "64")) < 1):
+            or _gemm_max_m() < 1):
         return False
     k = x.shape[1]
     rows = [x, norm_weight] if residual is None else [x, norm_weight, residual]

@@ -38,6 +38,18 @@ def _linear_fwd(mod: nn.Module, x: torch.Tensor) -> torch.Tensor:
     return ops.linear(x, mod.weight, mod.bias)
 
 
+_lora_context = None   # engine.lora.CTX; that module imports this package
+
+
+def lora_active() -> bool:
+    """Whether this step has adapters: asked ahead of everything else about them, as a small
+    step is bound by the host."""
+    global _lora_context
+    if _lora_context is None:
+        from ..engine.lora import CTX as _lora_context
+    return _lora_context.active
+
+
 def _as_it_is(mod: nn.Module) -> torch.Tensor | None:
     """A layer's weight unless it is rounded."""
     return mod.weight if getattr(mod, "quant_bits", None) is None else None
@@ -92,7 +104,7 @@ class MergedColumnParallelLinear(nn.Module):
         self.bias = _init_weight((total,), dtype, std=0.0) if bias else None
 
     def forward(self, x: torch.Tensor, lora=None) -> torch.Tensor:
-        if lora is not None:
+        if lora is not None and lora_active():
             from ..engine.lora import apply_lora, lora_linear
 
             layer_idx, projs = lora
@@ -105,7 +117,7 @@ class MergedColumnParallelLinear(nn.Module):
 
     def gated(self, x: torch.Tensor, lora=None) -> torch.Tensor:
         """silu of the first half of the outputs times the second."""
-        if lora is not None:
+        if lora is not None and lora_active():
             from ..engine.lora import lora_linear
 
             layer_idx, projs = lora
@@ -143,7 +155,7 @@ class RowParallelLinear(nn.Module):
         return ops.linear(x, self.weight)
 
     def forward(self, x: torch.Tensor, lora=None) -> torch.Tensor:
-        if lora is not None:
+        if lora is not None and lora_active():
             # delta added BEFORE the all-reduce: A is input-sharded, so the
             # per-rank partial deltas sum to the full LoRA delta
             from ..engine.lora import apply_lora, lora_linear
