@@ -102,3 +102,11 @@ def test_one_question_for_both_rules():
                 block, ring = ops._C.gemm_block_takes(m, n, k), ops._C.gemm_ring_wins(m, n, k, False)
                 want = 0 if m <= 64 else 1 if block else 2 if ring else 0
                 assert ops._C.gemm_tiles_route(m, n, k) == want
+
+
+def test_few_rows_are_not_asked_for():
+    """Adapters' products of up to eight rows go past the question."""
+    for m in range(1, 9):
+        for n in (128, 2048, 14336, 28672):
+            for k in (64, 2048, 8192, 28672):
+                assert not ops._tiles_take(m, n, k)
