@@ -85,21 +85,32 @@ __global__ __launch_bounds__(256, OCC) void moe_ring_kernel(
 // | 128 x 128, experts x between (in), rows an expert, evenly spread, tiles of 256 x 256:
 //   gated: 8 x 1792 (4096), 125, 112: 72 | 44 | 55; 4 x 512 (1024), 160, 16: 25 | 15 | 11; 8 x 3584
 //   (4096), 160, 224: 117 | 129 | 140 (unevenly, 200: 173 | 135 | 153); 8 x 7168 (4096), 448, 200: 204 |
-//   251 | 268.
+//   251 | 268.  About 240 rows some experts have more than 256, and one round of tiles becomes two:
+//   8 x 3584 (4096), 249: 189 | 140 | 159, 16 x 2048 (2048), 249: 98 | 99 | 91.
 //   plain: 8 of 4096 (14336), 222, 128: 298 | 235 | 281 (unevenly 294 | 402 | 369), 249, 256: 299 | 418
 //   | 390; 8 of 4096 (3584), 222, 128: 65 | 49 | 53; 16 of 2048 (2048), 222, 128: 43 | 31 | 33; 4 of 1024
 //   (512), 160, 16: 16 | 10 | 8; 16 of 4096 (3584), 222, 256: 107 | 133 | 145.
+//   Short K (evenly, unevenly), where two tiles of 128 x 128 share a CU for less: 32 of 2048 (1024),
+//   118: 34 | 37 | 31, 35 | 40 | 33; 245: 56 | 56 | 47, 59 | 55 | 48; 280: 66 | 59 | 56, 60 | 59 | 55;
+//   420: 67 | 78 | 73, 86 | 76 | 72; 64 of 2048 (768), 140: 57 | 67 | 61, 55 | 63 | 55, 180: 58 | 72 |
+//   66, 74 | 71 | 64 (256 x 256 are one tile an expert there, but two of the experts with more);
+//   48 of 2048 (768), 280: 80 | 75 | 66, 75 | 78 | 66; 16 of 2048 (2048), whose 128 x 256 are one
+//   round, 118: 44 | 28 | 35, 44 | 29 | 36, 245: 50 | 53 | 48, 51 | 55 | 48.
 int moe_tile(int mean, int experts, long columns, int K, bool gated) {
   if (columns % 256 != 0) return 2;
   auto tiles = [&](long mean, long rows) {
     return (mean + rows - 1) / rows * experts * (columns / 256);
   };
   if (gated) {
-    if (mean > (K >= 4096 ? 110 : 150) && tiles(mean, 256) >= 192) return 0;
+    const long large = tiles(mean, 256);
+    if (mean > (K >= 4096 ? 110 : 150) && large >= 192 && (large > 256 || mean <= 236 || mean > 256))
+      return 0;
     return mean > 52 && K >= 4096 ? 1 : 2;
   }
   // some experts have more rows than the mean: from 228 on they are counted as two tiles
-  if (mean > 220 && tiles(mean * 9L / 8, 256) >= 192) return 0;
+  const long more = mean * 9L / 8;
+  if (mean > (K <= 2048 ? 300 : 220) && tiles(more, 256) >= 192) return 0;
+  if (K <= 2048 && tiles(more, 128) > 256) return 2;
   return mean > 110 && tiles(mean, 128) >= 128 ? 1 : 2;
 }
 

@@ -45,6 +45,26 @@ def test_tiles(mode, counts, n, k):
         assert (err <= 2 ** -8 * s.abs() + 2e-4).all(), (e, err.max().item())
 
 
+# what has enough of them for 256 x 256 (short and long K, gated) and for 128 x 256: segments of one
+# row more and less than tiles, of none, and of several tiles
+@pytest.mark.parametrize(("mode", "counts", "n", "k", "tile"), [
+    ("plain", [511, 0, 257, 256, 255, 1, 700, 512] * 3, 2048, 64, 0),
+    ("relu2", [513, 300, 257, 256, 255, 129, 400, 512] * 3, 2048, 192, 0),
+    ("plain", [257, 200, 256, 255, 222, 129, 213, 255] * 2, 4096, 2112, 0),
+    ("silu", [257, 0, 256, 255, 1, 129, 127, 255] * 2, 1536, 192, 0),
+    ("silu", [256, 100, 129, 128, 127, 70, 1, 257] * 2, 1536, 4096, 0),
+    ("plain", [129, 128, 127, 1, 0, 257, 160, 110] * 2, 2048, 64, 1),
+    ("relu2", [129, 128, 127, 1, 0, 257, 160, 110] * 2, 2048, 128, 1)])
+def test_many_large_tiles(mode, counts, n, k, tile):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from vllm_tgis_adapter_amd import ops
+
+    gated = mode == "silu"
+    assert ops._C.moe_tile(sum(counts) // len(counts), len(counts), n * (1 + gated), k, gated) == tile
+    test_tiles(mode, counts, n, k)
+
+
 @pytest.mark.parametrize("module", ["_C", "_C_seq"])
 @pytest.mark.parametrize("mode", [0, 1, 2])
 @pytest.mark.parametrize("counts", [[5, 3], [60, 70], [300, 0, 141]], ids=str)

@@ -85,10 +85,13 @@ def test_plans_are_plans(gated):
 # 0: 256 x 256, 1: 128 x 256, 2: 128 x 128; rows an expert, experts, columns of W, K
 @pytest.mark.parametrize(("mean", "experts", "columns", "k", "gated", "tile"), [
     (737, 8, 28672, 4096, True, 0), (737, 8, 4096, 14336, False, 0), (125, 8, 28672, 4096, True, 0),
-    (100, 8, 28672, 4096, True, 1), (222, 8, 4096, 14336, False, 1), (249, 8, 4096, 14336, False, 0), (300, 8, 4096, 14336, False, 0),
-    (125, 8, 3584, 4096, True, 1), (249, 8, 3584, 4096, True, 1), (160, 4, 1024, 1024, True, 2),
-    (222, 4, 1024, 512, False, 2), (400, 4, 1024, 512, False, 2), (222, 8, 4096, 3584, False, 1),
-    (222, 16, 2048, 2048, False, 1), (222, 16, 4096, 3584, False, 0), (160, 8, 2048 + 128, 4096, True, 2)])
+    (100, 8, 28672, 4096, True, 1), (249, 8, 28672, 4096, True, 0), (125, 8, 3584, 4096, True, 1),
+    (230, 8, 7168, 4096, True, 0), (249, 8, 7168, 4096, True, 1), (260, 8, 7168, 4096, True, 0),
+    (160, 4, 1024, 1024, True, 2), (160, 8, 2048 + 128, 4096, True, 2),
+    (222, 8, 4096, 14336, False, 1), (230, 8, 4096, 14336, False, 0), (300, 8, 4096, 14336, False, 0),
+    (222, 8, 4096, 3584, False, 1), (222, 16, 4096, 3584, False, 0), (222, 4, 1024, 512, False, 2),
+    (400, 4, 1024, 512, False, 2), (222, 16, 2048, 2048, False, 1), (245, 16, 2048, 2048, False, 2),
+    (118, 32, 2048, 1024, False, 2), (280, 32, 2048, 1024, False, 2), (420, 32, 2048, 1024, False, 0)])
 def test_expert_tiles_fill_the_chip(mean, experts, columns, k, gated, tile):
     """Large tiles only where there are enough of them."""
     assert ops._C.moe_tile(mean, experts, columns, k, gated) == tile
