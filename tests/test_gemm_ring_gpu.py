@@ -68,6 +68,20 @@ def test_parts(form, parts, k):
     _check(y, x, w, False)
 
 
+# weights of 40 million and more that one tile of rows reads go past the caches, 64 x 64 from 20
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("form", range(5))
+def test_weights_read_once(form, gated):
+    from vllm_tgis_adapter_amd.ops import _C
+
+    n, k = 15872 // (1 + gated), 2560
+    for m in (FORMS[form][0] - 1, FORMS[form][0] + 1):   # read once, and twice
+        x, w = _inputs(m, n * (1 + gated), k)
+        y = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+        _C.gemm_ring(y, x, w, gated, form << 4 | 1)
+        _check(y, x, w, gated)
+
+
 @pytest.mark.parametrize("entry", ["gemm_block", "gemm_ring"])
 def test_results_at_any_address(entry):
     """Results that start off a 16-byte boundary."""
