@@ -9,22 +9,34 @@
 // v_mfma_f32_32x32x16_bf16 takes S^T = K Q^T, so a lane keeps one query's statistics and
 // accumulators; 16 keys of the scores enter the second product in the order the score
 // layout has them, so probabilities are packed where they are, and the values come back
-// transposed (ds_read_b64_tr_b16).  The products of the next tile's scores alternate with
-// this tile's exponentials: keys are staged a tile ahead of values.
+// transposed (ds_read_b64_tr_b16).
 //
-// Bound by the matrix unit and the vector unit taking turns (heads of 128: 1024 and 1060
-// cycles of a wave and tile, 2270 taken) where the chip is full; by a wave's own chain,
-// 1.6 us a tile, where it is not, hence the cut over keys.
+// Bound by what a SIMD issues: a tile of 64 keys (heads of 128) takes a wave 32 products of 32
+// clocks, of which each keeps the vector unit for about 12, and some 1050 clocks of exponentials
+// (16 each), sums and packing.  With eight waves the two of a SIMD take turns, one making
+// probabilities while the other multiplies: 2 x 1550 clocks of 2 x 1050 + 64 x 12.  What that took:
+//  - block ids and addresses on the scalar unit.  By the lanes they were 500 clocks a tile,
+//    and ids that went through vector memory had the compiler wait for the whole next tile.
+//  - three tiles of keys and of values in LDS, so that a turn's first fragments are read ahead of
+//    its barrier; addresses are constants then, no vector instruction lies between the products.
+//  - reads in batches: with transposed ones among them the compiler waits for all.
+//  - chunks of values turned so that sixteen lanes of a transposed read lie in different banks
+//    (2.7 -> 1.9 clocks a read of a full LDS).
+// Fewer waves, where a workgroup's are alone or two workgroups share a CU: products of the next
+// tile's scores between this one's exponentials.
 //
-// Measured (MI355X, 32/8 heads of 128, before -> after): 3500 tokens of 7 prompts after
-// 700 each, bf16: 182 -> 84 us, 645 TFLOP/s; one prompt of 8192 tokens 975 TFLOP/s, 512
-// tokens after 5000 65 us.  On the way: eight waves of one head (256 tokens) leave early
-// rows' waves idle; the second product a tile behind the first, both among the exponentials,
-// 564 -> 590 us at 8192 tokens, with register staging 630; transposed reads as asm 584;
-// results stored in 8 bytes a lane instead of 16: 24 tokens 7.0 us instead of 6.2.
+// Measured (MI355X, 32/8 heads of 128, keys and queries of variance 1, before -> after): 3500
+// tokens of 7 prompts after 700 each, bf16: 86 -> 74 us; one prompt of 8192 tokens 580 -> 522 us (1050
+// TFLOP/s; e4m3 605 -> 560), 3000 tokens 114 -> 100, 512 tokens after 5000 75 -> 67.  Turns alone, with
+// the lanes' addresses, were worth 1 %.  Left: ids of blocks that a wave's load does not fit
+// (under 4 to 8 rows), for which the lanes still work: 100 tokens after 200 by 2 %, 17 by 4.
+// On the way here: eight waves of one head (256 tokens) leave early rows' waves idle; register
+// staging 630 us of 564; transposed reads as asm 584; results stored in 8 bytes a lane instead of
+// 16: 24 tokens 7.0 us instead of 6.2.
 
 #include "common.h"
 #include <float.h>
+#include <type_traits>
 
 typedef __attribute__((ext_vector_type(8))) short bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) short s16x4_t;
@@ -61,7 +73,7 @@ DEVINLINE s16x4_t read_transposed(lds_s16x4_t* __restrict__ at) {
 // transposed read lie in different banks.
 template <int HD> DEVINLINE int k_swizzle(int r) { return HD == 128 ? r & 15 : (r >> 1) & 7; }
 template <int HD> DEVINLINE int v_swizzle(int r) {
-  return HD == 128 ? (r & 7) * 2 : ((r >> 1) & 3) * 2;
+  return HD == 128 ? (r & 3) * 4 : (r & 2) * 2;
 }
 
 // tiles of keys that one part takes
@@ -69,7 +81,12 @@ DEVINLINE int tiles_per_part(int tiles, int parts) {
   return max(kMinTiles, (tiles + parts - 1) / parts);
 }
 
-template <int HD, typename CT, int NW>
+// Tiles of keys, and of values, that LDS holds
+constexpr int prefill_buffers(int waves) { return waves == 8 ? 3 : 2; }
+
+// EVEN: cache blocks are a multiple of the rows of a wave's load (and a power of two), so that
+// these have one block
+template <int HD, typename CT, int NW, bool EVEN>
 __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
     __hip_bfloat16* __restrict__ out,         // [total_q, nheads, HD]
     const __hip_bfloat16* __restrict__ q,     // [total_q, nheads, HD]
@@ -102,6 +119,7 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
   if (tile < 0) return;
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int scalar_wave = __builtin_amdgcn_readfirstlane(wave);
   const int col = lane & 31, half = lane >> 5;
   const int group = nheads / kvh, per_kv = group / heads;   // workgroups of a key head
   const int kv_head = blockIdx.x / per_kv;
@@ -120,9 +138,10 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
   const int wave_min = past + token0 - origin;
   const int wave_max = token0 < q_len ? past + min(token0 + 31, q_len - 1) - origin : -1;
 
-  extern __shared__ __align__(16) char lds_all[];   // keys twice, values twice
+  constexpr int BUFS = prefill_buffers(NW);
+  __shared__ __align__(16) char lds_all[2 * BUFS * BYTES];   // tiles of keys, then of values
   char* const k_lds[2] = {lds_all, lds_all + BYTES};
-  char* const v_lds[2] = {lds_all + 2 * BYTES, lds_all + 3 * BYTES};
+  char* const v_lds[2] = {lds_all + BUFS * BYTES, lds_all + (BUFS + 1) * BYTES};
 
   const __hip_bfloat16* q_row = q + ((long)(q_start + token) * nheads + head) * HD + half * 8;
   bf16x8_t qf[KS];
@@ -135,37 +154,59 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
   const char* k_at = reinterpret_cast<const char*>(k_cache) + kv_head * HD * sizeof(CT);
   const char* v_at = reinterpret_cast<const char*>(v_cache) + kv_head * HD * sizeof(CT);
   auto row_of = [&](int ps) { return (ps * NW + wave) * RPP + lane / LPR; };
-  // block ids of a tile's keys (past the end: of the last key), and the cache rows that
-  // they lead to: apart, so that nothing waits for the ids before the next step
-  auto pos_of = [&](int ps, int t) { return min(origin + t * kTile + row_of(ps), keys - 1); };
+  // Block ids of a tile's keys (past the end: of the last key), and what they lead to: apart, so
+  // that nothing waits for the ids before the next step.  With EVEN blocks both are the wave's, on
+  // the scalar unit: a lane by itself takes 500 of the vector unit's clocks a tile for them,
+  // half as much as for its probabilities.
+  struct Place {       // of a wave's load in the cache
+    long at;    // EVEN: where its first row begins; else: the lane's row
+    int last;   // EVEN: rows past it are this one again
+  };
+  auto pos_of = [&](int ps, int t) {
+    return min(origin + t * kTile + (EVEN ? (ps * NW + scalar_wave) * RPP : row_of(ps)), keys - 1);
+  };
   auto page_of = [&](int pos) {
-    return block_shift >= 0 ? pos >> block_shift : pos / block_size;
+    return EVEN || block_shift >= 0 ? pos >> block_shift : pos / block_size;
   };
   auto ids_of = [&](int (&ids)[PASS], int t) {
 #pragma unroll
     for (int ps = 0; ps < PASS; ++ps) ids[ps] = table[page_of(pos_of(ps, t))];
   };
-  auto slots_of = [&](int (&slots)[PASS], const int (&ids)[PASS], int t) {
+  // (ahead of a tile's loads: behind them the compiler has all of these land before it touches
+  // the ids, a memory latency in every tile)
+  auto places_of = [&](Place (&places)[PASS], const int (&ids)[PASS], int t) {
 #pragma unroll
     for (int ps = 0; ps < PASS; ++ps) {
-      const int pos = pos_of(ps, t);
-      slots[ps] = ids[ps] * block_size + (pos - page_of(pos) * block_size);
+      const int pos = pos_of(ps, t), in = pos - page_of(pos) * block_size;
+      if constexpr (EVEN) {
+        places[ps] = Place{(((long)ids[ps] << block_shift) + in) * row_bytes, keys - 1 - pos};
+      } else {
+        int row = ids[ps] * block_size + in;
+        if constexpr (NW == 8) asm volatile("" : "+v"(row));
+        places[ps] = Place{row, 0};
+      }
     }
   };
   u32x4_t kr[FP8 ? PASS : 1], vr[FP8 ? PASS : 1];
-  auto issue = [&](const char* cache, const int (&slots)[PASS], char* lds, auto& regs,
+  auto issue = [&](const char* cache, const Place (&places)[PASS], char* lds, auto& regs,
                    auto swizzle) {
 #pragma unroll
     for (int ps = 0; ps < PASS; ++ps) {
-      const char* row = cache + slots[ps] * row_bytes;
+      const char* row;
+      unsigned in = (FP8 ? lane % LPR : (lane % LPR) ^ swizzle(row_of(ps))) * 16;
+      if constexpr (EVEN) {
+        row = cache + places[ps].at;
+        in += __umul24(min(lane / LPR, places[ps].last), (unsigned)row_bytes);
+      } else {
+        row = cache + places[ps].at * row_bytes;
+      }
       if constexpr (FP8)
-        regs[ps] = *reinterpret_cast<const u32x4_t*>(row + lane % LPR * 16);
+        regs[ps] = *reinterpret_cast<const u32x4_t*>(row + in);
       else
         __builtin_amdgcn_global_load_lds(
-            (const __attribute__((address_space(1))) unsigned*)(row + ((lane % LPR) ^
-                                                                       swizzle(row_of(ps))) * 16),
-            (__attribute__((address_space(3))) unsigned*)(lds + (ps * NW + wave) * 1024), 16, 0,
-            0);
+            (const __attribute__((address_space(1))) unsigned*)(row + in),
+            (__attribute__((address_space(3))) unsigned*)(lds + (ps * NW + scalar_wave) * 1024), 16,
+            0, 0);
     }
   };
   auto unpack = [&](char* lds, const auto& regs, auto swizzle) {
@@ -183,15 +224,18 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
   };
   auto k_swz = [](int r) { return k_swizzle<HD>(r); };
   auto v_swz = [](int r) { return v_swizzle<HD>(r); };
+  auto block_meet = [&] {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
   // own loads have landed (or are written to LDS), everybody's have
   auto meet = [&] {
     if constexpr (FP8) {
       __syncthreads();
     } else {
       __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
+      block_meet();
     }
   };
 
@@ -204,16 +248,17 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
   // LDS addresses in the first tile of keys and of values; kept out of the compiler's sight,
   // which would rather compute them again than keep them (where there are registers for it)
   constexpr bool KEEP = !FP8 && NW == 8;
+  const unsigned lds_at = (unsigned)(__SIZE_TYPE__)(__attribute__((address_space(3))) char*)lds_all;
   unsigned k_lane[KS], v_lane[DT];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
-    k_lane[ks] = col * HD * 2 + ((ks * 2 + half) ^ k_swizzle<HD>(col)) * 16;
+    k_lane[ks] = lds_at + col * HD * 2 + ((ks * 2 + half) ^ k_swizzle<HD>(col)) * 16;
     if constexpr (KEEP) asm volatile("" : "+v"(k_lane[ks]));
   }
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) {
     const int i = lane & 15, side = lane >> 4 & 1, r = half * 4 + (i >> 2);
-    v_lane[dt] = 2 * BYTES + r * HD * 2 +
+    v_lane[dt] = lds_at + BUFS * BYTES + r * HD * 2 +
                  (((dt * 2 + side) * 2 + ((i & 3) >> 1)) ^ v_swizzle<HD>(r)) * 16 + (i & 1) * 8;
     if constexpr (KEEP) asm volatile("" : "+v"(v_lane[dt]));
   }
@@ -273,71 +318,208 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
     l_state += a + b;
     p[i / 4].u[i % 4] = pack_bf16(a, b);
   };
+  auto value_frag = [&](int at, int c, int dt) {   // 16 keys, 32 dims
+    union { s16x4_t h[2]; bf16x8_t v; } vf;
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+      vf.h[x] = read_transposed((lds_s16x4_t*)(v_lane[dt] + (at + (2 * c + x) * 8 * HD * 2)));
+    return vf.v;
+  };
   auto values = [&](const Probs (&p)[4], int buf) {
 #pragma unroll
     for (int c = 0; c < 4; ++c)
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        union { s16x4_t h[2]; bf16x8_t v; } vf;
-#pragma unroll
-        for (int x = 0; x < 2; ++x)
-          vf.h[x] = read_transposed(
-              (lds_s16x4_t*)(v_lane[dt] + (buf * BYTES + (2 * c + x) * 8 * HD * 2)));
-        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.v, p[c].v, acc[dt], 0, 0, 0);
-      }
+      for (int dt = 0; dt < DT; ++dt)
+        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(value_frag(buf * BYTES, c, dt), p[c].v,
+                                                          acc[dt], 0, 0, 0);
   };
 
-  f32x16_t s0[2], s1[2];
-  int slots[PASS], ids[PASS];   // rows of tile t + 1, block ids of tile t + 2
-  auto step = [&](int t, f32x16_t (&now)[2], f32x16_t (&next)[2], int buf) {
-    meet();
-    const bool more_k = t + 2 < n, more_v = t + 1 < n;
-    if (more_v) issue(v_at, slots, v_lds[buf ^ 1], vr, v_swz);
-    if (more_k) {
-      slots_of(slots, ids, t + 2);
-      issue(k_at, slots, k_lds[buf], kr, k_swz);
-      if (t + 3 < n) ids_of(ids, t + 3);
-    }
-    // wave-uniform: the matrix unit wants all lanes
-    if (t * kTile <= wave_max) {
-      Probs p[4];
-      follow(now, t * kTile);
-      bias = m_state == -FLT_MAX ? 0.f : -m_state * scale_log2;
-      auto work = [&](int i) { weigh(now, p, i); };
-      if (more_v && (t + 1) * kTile <= wave_max) {
-        scores(next, (buf ^ 1) * BYTES, work);
-      } else {
+  int ids[PASS];         // block ids of the tile after the next to be asked for
+  Place places[PASS];    // of the values that are asked for next
+  if constexpr (NW == 8) {
+    // Two waves of a SIMD take turns: while one's probabilities are made, the other multiplies.
+    // Both run the same program, waves 4 to 7 a barrier later: with barriers counted from the
+    // first scores on, tile t's probabilities lie behind barrier 2 t + 1 (late: + 2), its values
+    // and the next one's scores behind 2 t + 2 (+ 3).
+    f32x16_t s[2];
+    Probs p[4];
+    const bool late = wave >= 4;
+    auto turn = [&] {
+      __builtin_amdgcn_sched_barrier(0);
+      block_meet();
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    // Fragments are read a batch ahead, behind the first products of the batch before (the
+    // compiler waits for all reads that are on their way, wherever it waits), the first batch
+    // ahead of the barrier.
+    constexpr int COUNT = HD / 8, BATCH = 4;   // products of values, of scores
+    bf16x8_t kf[2 * BATCH], vf[2 * BATCH];
+    auto fetch = [&](auto at, int g, bool keys) {
+      constexpr int k_buf = (at + 1) % 3 * BYTES, v_buf = at * BYTES;
+      if (keys) kf[g % (2 * BATCH)] = key_frag(k_buf, g);
+      vf[g % (2 * BATCH)] = value_frag(v_buf, g / DT, g % DT);
+    };
+    auto multiply = [&](auto at, auto more, auto between) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) work(i);
+      for (int g = 0; g < COUNT; ++g) {
+        if constexpr (more)
+          s[g & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              kf[g % (2 * BATCH)], qf[g >> 1], g < 2 ? f32x16_t{} : s[g & 1], 0, 0, 0);
+        acc[g % DT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[g % (2 * BATCH)], p[g / DT].v,
+                                                              acc[g % DT], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (g % BATCH < 2 && g / BATCH + 1 < COUNT / BATCH) {
+          fetch(at, (g / BATCH + 1) * BATCH + g % BATCH * 2, more);
+          fetch(at, (g / BATCH + 1) * BATCH + g % BATCH * 2 + 1, more);
+        }
+        if (g == 2) between();
+        __builtin_amdgcn_sched_barrier(0);
       }
-      values(p, buf);
-    }
-    if constexpr (FP8) {
-      if (more_v) unpack(v_lds[buf ^ 1], vr, v_swz);
-      if (more_k) unpack(k_lds[buf], kr, k_swz);
-    }
-  };
-  if (n > 0) {
-    ids_of(ids, 0);
-    slots_of(slots, ids, 0);
-    issue(k_at, slots, k_lds[0], kr, k_swz);
-    issue(v_at, slots, v_lds[0], vr, v_swz);
-    if constexpr (FP8) {
-      unpack(k_lds[0], kr, k_swz);
-      unpack(v_lds[0], vr, v_swz);
-    }
-    if (n > 1) {
+    };
+    // Behind barrier 2 u + 2 tile u + 3 of keys and u + 2 of values: their places were last read
+    // ahead of it, in the late waves' products of tile u - 1.  They have landed ahead of barrier
+    // 2 u + 4 and are first read behind 2 u + 5.
+    auto plan = [&](Place (&ahead)[PASS], int u) {
+      if (EVEN || u + 3 < n) places_of(ahead, ids, u + 3);
+      if (EVEN || u + 4 < n) ids_of(ids, u + 4);
+    };
+    auto ask = [&](int u, auto at, Place (&ahead)[PASS]) {
+      if constexpr (!EVEN) plan(ahead, u);
+      if (u + 2 < n) issue(v_at, places, lds_all + (3 + (at + 2) % 3) * BYTES, vr, v_swz);
+      if (u + 3 < n) issue(k_at, ahead, lds_all + at * BYTES, kr, k_swz);
+    };
+    auto landed = [&](int u, auto at) {
+      if constexpr (FP8) {
+        if (u + 2 < n) unpack(lds_all + (3 + (at + 2) % 3) * BYTES, vr, v_swz);
+        if (u + 3 < n) unpack(lds_all + at * BYTES, kr, k_swz);
+        __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0), lgkmcnt(0)
+      } else {
+        __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+      }
+    };
+    auto step = [&](int t, auto at) {   // at: t % 3
+      Place ahead[PASS];
+      if constexpr (EVEN) plan(ahead, t);   // where all waves come by: the scalar unit's
+      turn();
+      if (late) ask(t, at, ahead);
+      const bool active = t * kTile <= wave_max;   // wave-uniform: the matrix unit wants all lanes
+      if (active) {
+        follow(s, t * kTile);
+        bias = m_state == -FLT_MAX ? 0.f : -m_state * scale_log2;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) weigh(s, p, i);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int g = 0; g < BATCH; ++g) fetch(at, g, true);
+      }
+      if (!late && t > 0) landed(t - 1, std::integral_constant<int, (at + 2) % 3>{});
+      turn();
+      auto between = [&] {
+        if (!late) ask(t, at, ahead);
+      };
+      if (active) {
+        __builtin_amdgcn_s_setprio(1);
+        if (t + 1 < n && (t + 1) * kTile <= wave_max)
+          multiply(at, std::true_type{}, between);
+        else
+          multiply(at, std::false_type{}, between);
+        __builtin_amdgcn_s_setprio(0);
+      } else {
+        between();
+      }
+      if (late) landed(t, at);
+#pragma unroll
+      for (int ps = 0; ps < PASS; ++ps) places[ps] = ahead[ps];
+    };
+    if (n > 0) {
+      auto first_keys = [&](int t) {
+        issue(k_at, places, lds_all + t * BYTES, kr, k_swz);
+        if constexpr (FP8) unpack(lds_all + t * BYTES, kr, k_swz);
+      };
+      auto first_values = [&](int t) {
+        issue(v_at, places, lds_all + (3 + t) * BYTES, vr, v_swz);
+        if constexpr (FP8) unpack(lds_all + (3 + t) * BYTES, vr, v_swz);
+      };
+      ids_of(ids, 0);
+      places_of(places, ids, 0);
       ids_of(ids, 1);
-      slots_of(slots, ids, 1);
-      issue(k_at, slots, k_lds[1], kr, k_swz);
-      if constexpr (FP8) unpack(k_lds[1], kr, k_swz);
-      if (n > 2) ids_of(ids, 2);
+      first_keys(0);
+      first_values(0);
+      if (n > 1) {
+        places_of(places, ids, 1);
+        ids_of(ids, 2);
+        first_keys(1);
+        first_values(1);
+        if (n > 2) {
+          places_of(places, ids, 2);
+          first_keys(2);
+        }
+        ids_of(ids, 3);
+      }
+      meet();
+      if (late) turn();
+      if (0 <= wave_max) scores(s, 0, [](int) {});
+      for (int t = 0; t < n; t += 3) {
+        step(t, std::integral_constant<int, 0>{});
+        if (t + 1 < n) step(t + 1, std::integral_constant<int, 1>{});
+        if (t + 2 < n) step(t + 2, std::integral_constant<int, 2>{});
+      }
+      if (!late) turn();
     }
-    meet();
-    if (0 <= wave_max) scores(s0, 0, [](int) {});
-    for (int t = 0; t < n; t += 2) {
-      step(t, s0, s1, 0);
-      if (t + 1 < n) step(t + 1, s1, s0, 1);
+  } else {
+    f32x16_t s0[2], s1[2];
+    auto step = [&](int t, f32x16_t (&now)[2], f32x16_t (&next)[2], int buf) {
+      meet();
+      const bool more_k = t + 2 < n, more_v = t + 1 < n;
+      Place ahead[PASS];
+      if (EVEN || more_k) places_of(ahead, ids, t + 2);
+      if (more_v) issue(v_at, places, v_lds[buf ^ 1], vr, v_swz);
+      if (more_k) issue(k_at, ahead, k_lds[buf], kr, k_swz);
+      if (EVEN || t + 3 < n) ids_of(ids, t + 3);
+      if (EVEN || more_k)
+#pragma unroll
+        for (int ps = 0; ps < PASS; ++ps) places[ps] = ahead[ps];
+      // wave-uniform: the matrix unit wants all lanes
+      if (t * kTile <= wave_max) {
+        Probs p[4];
+        follow(now, t * kTile);
+        bias = m_state == -FLT_MAX ? 0.f : -m_state * scale_log2;
+        auto work = [&](int i) { weigh(now, p, i); };
+        if (more_v && (t + 1) * kTile <= wave_max) {
+          scores(next, (buf ^ 1) * BYTES, work);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) work(i);
+        }
+        values(p, buf);
+      }
+      if constexpr (FP8) {
+        if (more_v) unpack(v_lds[buf ^ 1], vr, v_swz);
+        if (more_k) unpack(k_lds[buf], kr, k_swz);
+      }
+    };
+    if (n > 0) {
+      ids_of(ids, 0);
+      places_of(places, ids, 0);
+      issue(k_at, places, k_lds[0], kr, k_swz);
+      issue(v_at, places, v_lds[0], vr, v_swz);
+      if constexpr (FP8) {
+        unpack(k_lds[0], kr, k_swz);
+        unpack(v_lds[0], vr, v_swz);
+      }
+      if (n > 1) {
+        ids_of(ids, 1);
+        places_of(places, ids, 1);
+        issue(k_at, places, k_lds[1], kr, k_swz);
+        if constexpr (FP8) unpack(k_lds[1], kr, k_swz);
+        if (EVEN || n > 2) ids_of(ids, 2);
+      }
+      meet();
+      if (0 <= wave_max) scores(s0, 0, [](int) {});
+      for (int t = 0; t < n; t += 2) {
+        step(t, s0, s1, 0);
+        if (t + 1 < n) step(t + 1, s1, s0, 1);
+      }
     }
   }
 
@@ -471,13 +653,18 @@ void launch(__hip_bfloat16* out, float* part_acc, float* part_ml, const __hip_bf
   const int tiles = (max_query_len + c.tokens - 1) / c.tokens;
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(nheads / c.heads, nseq, tiles * c.parts),
-                       dim3(c.waves * 64), 4 * kTile * HD * 2, stream, out, q, kc, vc, bt, qsl,
+                       dim3(c.waves * 64), 0, stream, out, q, kc, vc, bt, qsl,
                        sl, scale * kLog2e, nheads, kvh, c.heads, block_size, shift, max_blocks,
                        c.parts, part_acc, part_ml);
   };
-  if (c.waves == 8) go(paged_prefill_tile_kernel<HD, CT, 8>);
-  else if (c.waves == 4) go(paged_prefill_tile_kernel<HD, CT, 4>);
-  else go(paged_prefill_tile_kernel<HD, CT, 2>);
+  constexpr int kLoad = 1024 / (HD * sizeof(CT));   // rows of a wave's load
+  const bool even = shift >= 0 && block_size % kLoad == 0 && (long)kvh * HD * sizeof(CT) < 1 << 24;
+  if (c.waves == 8 && even) go(paged_prefill_tile_kernel<HD, CT, 8, true>);
+  else if (c.waves == 8) go(paged_prefill_tile_kernel<HD, CT, 8, false>);
+  else if (c.waves == 4 && even) go(paged_prefill_tile_kernel<HD, CT, 4, true>);
+  else if (c.waves == 4) go(paged_prefill_tile_kernel<HD, CT, 4, false>);
+  else if (even) go(paged_prefill_tile_kernel<HD, CT, 2, true>);
+  else go(paged_prefill_tile_kernel<HD, CT, 2, false>);
   if (c.parts > 1)
     hipLaunchKernelGGL((prefill_tile_merge_kernel<HD>), dim3(max_query_len, nseq, (nheads + 3) / 4),
                        dim3(256), 0, stream, out, part_acc, part_ml, qsl, sl, nheads, c.tokens, c.parts);

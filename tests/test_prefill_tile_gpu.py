@@ -251,3 +251,32 @@ def test_waves(heads, kv_heads, dim, fp8, seqs, longest, past):
 
     v = vc.float().cpu().nan_to_num()
     _close(got, plain(v), plain(v.abs()))
+
+
+# eight waves, whose tiles go round in three places of LDS: first to last place, once and twice round,
+# a last tile of one key and a full one; blocks that a wave's load fits, that it does not, and of
+# a size that is no power of two
+@pytest.mark.parametrize("block", [32, 8, 4, 24])
+@pytest.mark.parametrize(("dim", "fp8"), [(128, False), (64, False), (128, True)])
+@pytest.mark.parametrize("keys", [65, 128, 129, 192, 193, 256, 321, 384, 449])
+def test_places_of_tiles(block, dim, fp8, keys):
+    _need()
+    from vllm_tgis_adapter_amd import ops
+    from vllm_tgis_adapter_amd.ops import reference as R
+
+    gen = torch.Generator("cuda").manual_seed(keys)
+    lens, new, heads = [keys] * 5, [64, 33, 1, 64, 50], 64
+    (kc, vc), tables = _paged(lens, 8, dim, gen, block=block, fp8=fp8,
+                              unowned=0x7f if fp8 else float("nan"))
+    q = torch.randn((sum(new), heads, dim), generator=gen, device="cuda").bfloat16()
+    start = [sum(new[:i]) for i in range(6)]
+    kb, vb = (c.view(torch.uint8) if fp8 else c for c in (kc, vc))
+    got = ops.paged_attention_prefill(q, kb, vb, tables.cuda(), _ints(start), _ints(lens), 0.1,
+                                      64, keys)
+
+    def plain(v):
+        return R.paged_attention(q.float().cpu(), kc.float().cpu().nan_to_num(), v, tables,
+                                 torch.tensor(start), torch.tensor(lens), 0.1)
+
+    v = vc.float().cpu().nan_to_num()
+    _close(got, plain(v), plain(v.abs()))
