@@ -75,6 +75,9 @@ void launch_gemm_skinny_gated(__hip_bfloat16*, float*, const __hip_bfloat16*,
                               const __hip_bfloat16*, int, int, int, int,
                               hipStream_t);
 int gemm_panel_plan(int M, int N, int K);
+int gemm_panel_gated_plan(int M, int N, int K);
+void launch_gemm_panel_gated(__hip_bfloat16*, const __hip_bfloat16*, const unsigned char*,
+                             const float*, int, int, int, int, hipStream_t);
 void launch_gemm_block_q(__hip_bfloat16*, float*, const __hip_bfloat16*, const unsigned char*,
                          const float*, int, int, int, int, int, hipStream_t);
 void launch_widen_weight(__hip_bfloat16*, const unsigned char*, const float*, int, long, int,
@@ -473,6 +476,26 @@ const float* optional_scales(const c10::optional<torch::Tensor>& t, int64_t qbit
 }
 
 // y [1, I] = silu(n Wg^T) * (n Wu^T), n = rmsnorm(x + residual), sum = x + residual
+// y = silu(x Wg^T) * (x Wu^T) for int8 [Wg; Wu] and more than 64 rows, by one launch; false:
+// nothing was done, the product's plan has no room for the gate
+bool gemm_q_gated(torch::Tensor y, torch::Tensor x, torch::Tensor wq, torch::Tensor wscale) {
+  const int64_t M = x.size(0), K = x.size(1), N = wq.size(0) / 2;
+  const int plan = gemm_panel_gated_plan((int)M, (int)N, (int)K);
+  if (plan == 0) return false;
+  check_rounded(wq, wscale, 8, 2 * N, K);
+  TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::ScalarType::BFloat16 &&
+              y.scalar_type() == at::ScalarType::BFloat16);
+  TORCH_CHECK(x.is_contiguous() && y.is_contiguous() && y.size(0) == M && y.size(1) == N);
+  TORCH_CHECK((int64_t)128 * K < (1LL << 31));
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+              reinterpret_cast<uintptr_t>(wq.data_ptr()) % 16 == 0 &&
+              reinterpret_cast<uintptr_t>(y.data_ptr()) % 8 == 0);
+  launch_gemm_panel_gated(ptr<__hip_bfloat16>(y), cptr<__hip_bfloat16>(x),
+                          cptr<unsigned char>(wq), wscale.data_ptr<float>(), (int)M, (int)N, (int)K,
+                          plan, current_stream());
+  return true;
+}
+
 void row_norm_gated(torch::Tensor y, c10::optional<torch::Tensor> sum, torch::Tensor x,
                     c10::optional<torch::Tensor> residual, torch::Tensor weight, double eps,
                     torch::Tensor w, c10::optional<torch::Tensor> scales, int64_t qbits) {
@@ -914,6 +937,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("widen_weight", &widen_weight, "int8 / 4-bit weights to bf16");
   m.def("gemm_skinny", &gemm_skinny,
         "skinny decode GEMM y = x @ w^T, M <= 64 (CDNA4 MFMA)");
+  m.def("gemm_q_gated", &gemm_q_gated, "gated int8 product of many rows, where it is one launch");
+  m.def("gemm_panel_gated_plan", &gemm_panel_gated_plan, "its plan, or 0");
   m.def("gemm_panel_plan", &gemm_panel_plan,
         "which panel int8 products of many rows take, and parts of K (panel << 8 | parts)");
   m.def("row_norm_gated", &row_norm_gated, "norm and gated product of one row (CDNA4)");

@@ -18,7 +18,8 @@
 // turned by the row: x by r (256-byte rows) or r / 2 (128), W by r / 2 (128) or r / 4 (64).
 //
 // Measured: four llama-3-8b layers around attention, 301 rows, int8: 5101 -> 1064 us with tiles of
-// up to 64 x 128 whose weights every 64 rows widened again, -> 739 us with panels.
+// up to 64 x 128 whose weights every 64 rows widened again, -> 739 us with panels, -> 692 with the
+// gate in the panel and widening spread over its products.
 // Widening 28672 x 4096: 61 us (5.8 TB/s).
 
 #include "gemm_panel_q.h"
@@ -335,6 +336,8 @@ void launch_gemm_merge(__hip_bfloat16* y, const float* part, long plane, int par
 
 namespace {
 
+// Without GATED: N columns of y; with it N / 2, of a plan for N with whole K and even panels
+template <bool GATED>
 void launch_panel(__hip_bfloat16* y, float* part, const __hip_bfloat16* x, const unsigned char* w,
                   const float* scale, int M, int N, int K, int plan, hipStream_t stream) {
   const int parts = plan & 255, panel = (plan >> 8) - 1;
@@ -342,10 +345,11 @@ void launch_panel(__hip_bfloat16* y, float* part, const __hip_bfloat16* x, const
 #define GO(I, STAGES)                                                                         \
   case I: {                                                                                   \
     constexpr Panel p = kPanels[I];                                                           \
+    constexpr bool gate = GATED && p.tn % 2 == 0;                                             \
     const int blocks = (M + p.tm * 16 - 1) / (p.tm * 16) * (N / (p.tn * 64));                 \
-    hipLaunchKernelGGL((gemm_panel::gemm_panel_q_kernel<p.tm, p.tn, STAGES, p.per_cu>),       \
+    hipLaunchKernelGGL((gemm_panel::gemm_panel_q_kernel<p.tm, p.tn, STAGES, p.per_cu, gate>), \
                        dim3((blocks + 7) / 8 * 8, parts), dim3(64 * gemm_panel::kWaves), 0,   \
-                       stream, y, part, x, w, scale, M, N, K, depth);                         \
+                       stream, y, part, x, w, scale, M, GATED ? N / 2 : N, K, depth);         \
     break;                                                                                    \
   }
   switch (panel) {
@@ -364,9 +368,24 @@ void launch_gemm_block_q(__hip_bfloat16* y, float* part, const __hip_bfloat16* x
   if (qbits == 4)
     launch_block<4>(y, x, w, scale, M, N, K, stream);
   else if (plan > 1)
-    launch_panel(y, part, x, w, scale, M, N, K, plan, stream);
+    launch_panel<false>(y, part, x, w, scale, M, N, K, plan, stream);
   else
     launch_block<8>(y, x, w, scale, M, N, K, stream);
+}
+
+// The plan of a gated int8 product of M > 64 rows with [2 N, K], or 0 where the plain one's cuts K or
+// takes columns one tile a wave: the gate is not in the panel then.
+int gemm_panel_gated_plan(int M, int N, int K) {
+  if (M <= 64 || N % 128 != 0 || K % 128 != 0 || (long)(N + 128) * K >= 1L << 32) return 0;
+  const int plan = gemm_panel_plan(M, 2 * N, K);
+  return plan > 1 && (plan & 255) == 1 && kPanels[(plan >> 8) - 1].tn % 2 == 0 ? plan : 0;
+}
+
+// y [M, N] = silu(x Wg^T) * (x Wu^T), W = [Wg; Wu] in int8, plan of gemm_panel_gated_plan
+void launch_gemm_panel_gated(__hip_bfloat16* y, const __hip_bfloat16* x, const unsigned char* w,
+                             const float* scale, int M, int N, int K, int plan,
+                             hipStream_t stream) {
+  launch_panel<true>(y, nullptr, x, w, scale, M, 2 * N, K, plan, stream);
 }
 
 // total = N * K, K % 128 == 0

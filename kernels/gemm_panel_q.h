@@ -7,9 +7,22 @@
 // weights are on their way or widened before the tile begins, and a tile's loads are asked for
 // one by one between the products (a burst keeps all waves from them).  Neighbouring columns
 // start a tile of K apart (4096 x 4096, 301 rows 20.0 -> 18.8 us).
+//
+// In large panels a pair of weights is widened behind each product of the step before: one more
+// instruction hides behind v_mfma_f32_16x16x32_bf16 (16 clocks), each further one adds four to a
+// lone wave's time (28672 x 4096, 301 rows: 80 -> 77 us, and 2 % over four layers under sustained load;
+// 96 x 128, two a CU, 4096 x 14336, 700 rows 107 | 110, as before.  Products of 32 x
+// 32, which hide five, take 69 us alone but more power: the clock falls from 2360 to 2180 MHz, four
+// layers 718 | 727).  LDS serves 16-byte reads sixteen lanes at a time, half of them of one quarter of
+// the wave and half of the next (0..3, 12..15, 20..27 | 4..11, 16..19, 28..31): chunks lie so that these
+// are in different banks (half of all LDS cycles were conflicts).
+//
+// Gated, half of a wave's columns are gates and half what they multiply, and the launch that did
+// that (6 us at 301 x 28672) with its reads of the product falls away.
 #pragma once
 
 #include "block_gemm.h"
+#include "moe_tiles.h"
 
 namespace gemm_panel {
 
@@ -24,14 +37,14 @@ constexpr int kDepth = 64;    // inputs of a tile
 constexpr int kWaves = 4;     // along N
 
 // grid (tiles of y, parts of K); part [parts, M, N] (gridDim.y > 1); depth: inputs of a part
-// PER_CU: workgroups that share a CU
-template <int TM, int TN, int STAGES, int PER_CU>
+// PER_CU: workgroups that share a CU.  GATED: N outputs of 2 N rows of W, K in one part.
+template <int TM, int TN, int STAGES, int PER_CU, bool GATED>
 __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
     __hip_bfloat16* __restrict__ y,         // [M, N]
     float* __restrict__ part,
     const __hip_bfloat16* __restrict__ x,   // [M, K]
-    const unsigned char* __restrict__ w,    // int8 [N, K]
-    const float* __restrict__ scale,        // [N]
+    const unsigned char* __restrict__ w,    // int8 [N, K] | [2 N, K]
+    const float* __restrict__ scale,        // [N] | [2 N]
     const int M, const int N, const int K, const int depth) {
   constexpr int BM = TM * 16, BN = TN * 16 * kWaves;
   constexpr int X_BYTES = BM * kDepth * 2, W_BYTES = BN * kDepth, STAGE = X_BYTES + W_BYTES;
@@ -39,17 +52,20 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
   constexpr int X_PASS = (X_LOADS + kWaves - 1) / kWaves, W_PASS = W_LOADS / kWaves;
   constexpr int LOADS = X_PASS + W_PASS;
   constexpr int AHEAD = 3;                // fragments of x on their way
+  constexpr bool SPREAD = TM >= 8;        // widening over the products
+  constexpr int OUT = GATED ? TN / 2 : TN, COLS = OUT * 16 * kWaves;   // of results
+  static_assert(!GATED || TN % 2 == 0, "as many gates");
   static_assert(TM >= TN && 2 * TM > AHEAD && STAGES >= 3, "what a tile's products hide");
   static_assert(STAGES * STAGE * PER_CU <= 160 * 1024, "LDS of a CU");
   __shared__ __align__(16) char lds[STAGES * STAGE];
 
   // neighbours in a run of blocks that one XCD gets share their columns of W
-  const int m_tiles = (M + BM - 1) / BM, blocks = m_tiles * (N / BN);
+  const int m_tiles = (M + BM - 1) / BM, blocks = m_tiles * (N / COLS);
   const int per_xcd = (blocks + 7) / 8, slot = blockIdx.x / 8;
   const int id = (blockIdx.x % 8) * per_xcd + slot;
   if (slot >= per_xcd || id >= blocks) return;
   const int k0 = blockIdx.y * depth;
-  const int m0 = id % m_tiles * BM, n0 = id / m_tiles * BN;
+  const int m0 = id % m_tiles * BM, n0 = id / m_tiles * COLS;
   const int tiles = min(depth, K - k0) / kDepth;
   const int start = id / m_tiles % tiles;
 
@@ -57,18 +73,22 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, quad = lane >> 4;
 
+  auto w_turn = [](int r) { return SPREAD ? -(r / 4) & 3 : r / 4 % 4; };
   // (where there are fewer loads than waves some are made twice: all waves wait alike; rows
   // of a panel are found by 32 bits, see gemm_panel_plan)
   unsigned x_off[X_PASS], w_off[W_PASS];
 #pragma unroll
   for (int p = 0; p < X_PASS; ++p) {
     const int r = (p * kWaves + wave) % X_LOADS * 8 + lane / 8;
-    x_off[p] = (unsigned)min(r, M - 1 - m0) * (K * 2u) + ((lane % 8) ^ (r / 2 % 8)) * 16;
+    const int at = (lane % 8) ^ (r / 2 % 8);   // large: of the chunks 0 2 4 6 1 3 5 7
+    x_off[p] = (unsigned)min(r, M - 1 - m0) * (K * 2u) + (SPREAD ? at % 4 * 2 + at / 4 : at) * 16;
   }
 #pragma unroll
   for (int p = 0; p < W_PASS; ++p) {
     const int r = (p * kWaves + wave) * 16 + lane / 4;
-    w_off[p] = (unsigned)r * K + ((lane % 4) ^ (r / 4 % 4)) * 16;
+    const int own = r / (TN * 16), in = r % (TN * 16), half = in / (OUT * 16);
+    w_off[p] = (unsigned)(half * N + own * (OUT * 16) + in % (OUT * 16)) * K +
+               ((lane % 4) ^ w_turn(r)) * 16;
   }
   const auto x_from = block_gemm::resource(x + (long)m0 * K + k0);
   const auto w_from = block_gemm::resource(w + (long)n0 * K + k0);
@@ -96,23 +116,20 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
   auto x_frag = [&](const char* at, int s, int i) {
     const int r = i * 16 + col;
     return *reinterpret_cast<const bf16x8_t*>(at + r * (kDepth * 2) +
-                                              ((quad * 2 + s) ^ (r / 2 % 8)) * 16);
+                                              ((SPREAD ? s * 4 + quad : quad * 2 + s) ^
+                                               (r / 2 % 8)) * 16);
   };
   auto w_chunk = [&](const char* at, int j) {
     const int r = (wave * TN + j) * 16 + col;
-    return *reinterpret_cast<const u32x4_t*>(at + X_BYTES + r * kDepth + (quad ^ (r / 4 % 4)) * 16);
+    return *reinterpret_cast<const u32x4_t*>(at + X_BYTES + r * kDepth +
+                                               (quad ^ w_turn(r)) * 16);
   };
-  auto unpack = [&](const u32x4_t& c, int s) {
-    union { unsigned u[4]; bf16x8_t v; } o;
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      const unsigned four = c[2 * s + d / 2] >> (d % 2 * 16);
-      const float a = (float)(signed char)(four & 0xff);
-      const float b = (float)(signed char)((four >> 8) & 0xff);
-      // whole numbers of 8 bits: the upper half of the float is all of it
-      o.u[d] = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302);
-    }
-    return o.v;
+  auto unpack = [&](const u32x4_t& c, int s, int d) {   // pair d of a column's weights of step s
+    const unsigned four = c[2 * s + d / 2] >> (d % 2 * 16);
+    const float a = (float)(signed char)(four & 0xff);
+    const float b = (float)(signed char)((four >> 8) & 0xff);
+    // whole numbers of 8 bits: the upper half of the float is all of it
+    return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302);
   };
 
 #pragma unroll
@@ -122,11 +139,14 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
   block_gemm::wait_loads<(STAGES - 2) * LOADS>();
   block_gemm::meet();
   u32x4_t c[TN];
-  bf16x8_t wf[2][TN], xf[AHEAD];
+  u32x4_t wf[2][TN];
+  bf16x8_t xf[AHEAD];
 #pragma unroll
   for (int j = 0; j < TN; ++j) c[j] = w_chunk(lds, j);
 #pragma unroll
-  for (int j = 0; j < TN; ++j) wf[0][j] = unpack(c[j], 0);
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int d = 0; d < 4; ++d) wf[0][j][d] = unpack(c[j], 0, d);
 #pragma unroll
   for (int q = 0; q < AHEAD; ++q) xf[q] = x_frag(lds, q / TM, q % TM);
 
@@ -154,13 +174,27 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
       const int f = q + AHEAD;
       xr[f] = f < 2 * TM ? x_frag(here, f / TM, f % TM)
                          : x_frag(there, (f - 2 * TM) / TM, (f - 2 * TM) % TM);
-      // the weights of the next step, a column at a time
-      if (s == 0 && i < TN) wf[1][i] = unpack(c[i], 1);
-      if (s == 1 && i >= TM - TN) wf[0][i - (TM - TN)] = unpack(c[i - (TM - TN)], 0);
+      // the weights of the next step, a column at a time or a pair behind each product (of the
+      // next tile two rows of products late: its weights are on their way)
+      constexpr int PAIRS = 4 * TN, LATE = 2 * TN;
+      const int room = s == 0 ? TM * TN : TM * TN - LATE;
+      if (!SPREAD && (s == 0 ? i < TN : i >= TM - TN)) {
+        const int j = s == 0 ? i : i - (TM - TN);
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
-        acc[i][j] =
-            __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[s][j], xr[q], acc[i][j], 0, 0, 0);
+        for (int d = 0; d < 4; ++d) wf[1 - s][j][d] = unpack(c[j], 1 - s, d);
+      }
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(bf16x8_t, wf[s][j]), xr[q], acc[i][j], 0, 0, 0);
+        const int at = i * TN + j - (s == 0 ? 0 : LATE);
+        if (SPREAD && at >= 0) {
+#pragma unroll
+          for (int u = at * PAIRS / room; u < (at + 1) * PAIRS / room; ++u)
+            wf[1 - s][u / 4][u % 4] = unpack(c[u / 4], 1 - s, u % 4);
+        }
+        if (SPREAD) __builtin_amdgcn_sched_barrier(0);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
@@ -171,17 +205,23 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
 
   const bool cut = gridDim.y > 1;
 #pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int n = n0 + (wave * TN + j) * 16 + quad * 4;
+  for (int j = 0; j < OUT; ++j) {
+    const int n = n0 + (wave * OUT + j) * 16 + quad * 4;
     const f32x4_t s = *reinterpret_cast<const f32x4_any_t*>(scale + n);
+    f32x4_t su{};
+    if constexpr (GATED) su = *reinterpret_cast<const f32x4_any_t*>(scale + N + n);
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const int m = m0 + i * 16 + col;
       if (m >= M) continue;
       f32x4_t v;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = acc[i][j][r] * s[r];
-      if (cut) {
+      for (int r = 0; r < 4; ++r) {
+        v[r] = acc[i][j][r] * s[r];
+        if constexpr (GATED)
+          v[r] = moe::finish<moe::kSilu>(v[r], acc[i][OUT + j][r] * su[r], 0.f);
+      }
+      if (!GATED && cut) {
         *reinterpret_cast<f32x4_t*>(part + (blockIdx.y * (long)M + m) * N + n) = v;
       } else {
         union { __hip_bfloat16 h[4]; uint2 u; } o;

@@ -324,3 +324,27 @@ def test_int8_panels(m, n, k, panel, parts):
     wq, scale = ops.quantize_weight(w, 8)
     exact = (wq.double() * scale.double()[:, None]).t().contiguous()
     _check(ops.linear_quant(x, wq, scale, 8), x.double() @ exact, x.double().abs() @ exact.abs())
+
+
+# every panel that takes the gate in, whole and with rows missing; the last is refused: K is cut
+@pytest.mark.parametrize(("m", "n", "k", "panel"), [
+    (65, 14336, 384, 1), (321, 4096, 128, 2), (511, 8192, 128, 4), (97, 14336, 384, 5),
+    (129, 14336, 384, 6), (301, 14336, 4096, 7), (1199, 4096, 128, 7), (301, 3072, 8192, None)])
+def test_int8_gated_panels(m, n, k, panel):
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    plan = ops._C.gemm_panel_gated_plan(m, n, k)
+    assert plan == (0 if panel is None else (panel + 1) << 8 | 1)
+    x, w = _x(m, k, 28), _x(2 * n, k, 29) / k ** 0.5
+    wq, scale = ops.quantize_weight(w, 8)
+    got = ops.gated_quant(x, wq, scale, 8)
+    if panel is None:
+        assert got is None
+        return
+    exact = (wq.double() * scale.double()[:, None]).t().contiguous()
+    g, u = (x.double() @ exact).chunk(2, dim=1)
+    _check(got, torch.nn.functional.silu(g) * u, 30 * (1 + g.abs()) * (1 + u.abs()))
+    # as by two launches, to the roundings in between
+    two = ops.silu_and_mul(ops.linear_quant(x, wq, scale, 8))
+    assert (got.float() - two.float()).norm() <= 2 ** -6 * two.float().norm()

@@ -400,6 +400,23 @@ def linear_quant(x: torch.Tensor, wq: torch.Tensor, scales: torch.Tensor,
     return torch.nn.functional.linear(x, w, bias)
 
 
+def gated_quant(x: torch.Tensor, wq: torch.Tensor, scales: torch.Tensor,
+                qbits: int) -> torch.Tensor | None:
+    """silu(x Wg^T) * (x Wu^T) for int8 [gate; up] weights as ``quantize_weight`` makes them, where
+    the product of so many rows takes the gate into its launch; None elsewhere (the caller has
+    linear_quant and silu_and_mul)."""
+    if (qbits != 8 or x.dim() != 2 or x.shape[0] <= 64 or x.dtype != torch.bfloat16
+            or not native_enabled(x) or not x.is_contiguous()):
+        return None
+    m, n, k = x.shape[0], wq.shape[0], x.shape[1]
+    if (n % 256 or k % 128 or m > _quant_rows(8, n, k) or wq.dtype != torch.int8
+            or scales.dtype != torch.float32 or not wq.is_contiguous()
+            or not scales.is_contiguous() or not _plain_tensors(x, wq)):
+        return None
+    out = torch.empty((m, n // 2), dtype=x.dtype, device=x.device)
+    return out if _C.gemm_q_gated(out, x, wq, scales) else None
+
+
 def gated_mlp_up(x: torch.Tensor, w13: torch.Tensor) -> torch.Tensor | None:
     """Fused silu(x@Wg^T) * (x@Wu^T) for merged [gate; up] weights.
 

@@ -131,6 +131,10 @@ class MergedColumnParallelLinear(nn.Module):
                             lambda: _linear_fwd(self, x), gated=True)
             if h is not None:
                 return h
+        elif self.quant_bits is not None and self.bias is None:
+            h = ops.gated_quant(x, self.weight_q, self.weight_scale, self.quant_bits)
+            if h is not None:
+                return h
         return ops.silu_and_mul(self(x, lora=lora))
 
     def load_full_weights(self, ws: list[torch.Tensor]) -> None:
