@@ -48,6 +48,10 @@ int gemm_ring_plan(int M, int N, int K, bool gated);
 void launch_gemm_ring_parts(__hip_bfloat16*, float*, const __hip_bfloat16*,
                             const __hip_bfloat16*, int, int, int, int, hipStream_t);
 bool gemm_ring_takes(int N, int K, int plan, bool gated);
+int gemm_ring_lora_cuts(int M, int K, int L, int PR, int plan);
+void launch_gemm_ring_lora(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hip_bfloat16*,
+                           int, int, int, int, float*, const __hip_bfloat16*, const int*, int, int,
+                           int, hipStream_t);
 bool gemm_ring_wins(long M, long N, long K, bool gated);
 bool gemm_block_takes(long M, long N, long K);
 int gemm_tiles_route(long M, long N, long K);
@@ -718,8 +722,8 @@ void lora_product(torch::Tensor out, torch::Tensor x, c10::optional<torch::Tenso
   const LoraCols cols = lora_cols(spans, V, W);
   if (T == 0) return;
   const auto f32 = x.options().dtype(at::ScalarType::Float);
-  torch::Tensor base, part;
-  int parts = 0;
+  torch::Tensor base, part, tmp;
+  int parts = 0, cuts = lora_shrink_cuts(T, K);
   if (y.has_value()) {
     TORCH_CHECK(y->size(0) == T);
     base = *y;
@@ -732,15 +736,25 @@ void lora_product(torch::Tensor out, torch::Tensor x, c10::optional<torch::Tenso
     } else {
       base = at::empty({T, W}, x.options());
     }
-    launch_gemm_ring_parts(parts ? nullptr : ptr<__hip_bfloat16>(base),
-                           parts ? part.data_ptr<float>() : nullptr, cptr<__hip_bfloat16>(x),
-                           cptr<__hip_bfloat16>(*w), T, W, K, plan, current_stream());
+    auto* to = parts ? nullptr : ptr<__hip_bfloat16>(base);
+    float* sums = parts ? part.data_ptr<float>() : nullptr;
+    if (const int ahead = gemm_ring_lora_cuts(T, K, L, PR, plan)) {
+      cuts = ahead;
+      tmp = at::empty({cuts, T, PR}, f32);
+      launch_gemm_ring_lora(to, sums, cptr<__hip_bfloat16>(x), cptr<__hip_bfloat16>(*w), T, W, K,
+                            plan, tmp.data_ptr<float>(), cptr<__hip_bfloat16>(a),
+                            slots.data_ptr<int>(), L, PR, cuts, current_stream());
+    } else {
+      launch_gemm_ring_parts(to, sums, cptr<__hip_bfloat16>(x), cptr<__hip_bfloat16>(*w), T, W, K,
+                             plan, current_stream());
+    }
   }
-  const int cuts = lora_shrink_cuts(T, K);
-  auto tmp = at::empty({cuts, T, PR}, f32);
-  launch_lora_shrink_tiles(tmp.data_ptr<float>(), cptr<__hip_bfloat16>(x),
-                           cptr<__hip_bfloat16>(a), slots.data_ptr<int>(), T, L, PR, K, cuts,
-                           current_stream());
+  if (!tmp.defined()) {
+    tmp = at::empty({cuts, T, PR}, f32);
+    launch_lora_shrink_tiles(tmp.data_ptr<float>(), cptr<__hip_bfloat16>(x),
+                             cptr<__hip_bfloat16>(a), slots.data_ptr<int>(), T, L, PR, K, cuts,
+                             current_stream());
+  }
   launch_lora_finish(ptr<__hip_bfloat16>(out), parts ? nullptr : cptr<__hip_bfloat16>(base),
                      parts ? part.data_ptr<float>() : nullptr, tmp.data_ptr<float>(),
                      cptr<__hip_bfloat16>(b), slots.data_ptr<int>(), scales.data_ptr<float>(),

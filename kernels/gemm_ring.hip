@@ -14,31 +14,33 @@
 // What did not pay: tiles of 256 x 128 beside 128 x 256 (within 1 %), five slots of 128 x 128
 // (2 % here and there), 64 x 256.
 
+#include <algorithm>
+
 #include "ring_gemm.h"
+#include "lora_shrink.h"
 #include "moe_tiles.h"
 
 namespace {
 
 using ring_gemm::f32x4_t;
 
-// grid (tiles of y, parts of K); part [parts, M, N] (gridDim.y > 1); depth: K of a part
-template <int BM, int BN, int SLOTS, int OCC, bool GATED, int HINT = 0>
-__global__ __launch_bounds__(256, OCC) void gemm_ring_kernel(
-    __hip_bfloat16* __restrict__ y, float* __restrict__ part,
-    const __hip_bfloat16* __restrict__ x, const __hip_bfloat16* __restrict__ w, const int M,
-    const int N, const int K, const int depth) {
+// Tile `tile` of y, part `own` of K; part [parts, M, N] (parts > 1); depth: K of a part
+template <int BM, int BN, int SLOTS, bool GATED, int HINT>
+DEVINLINE void product(char* lds, __hip_bfloat16* __restrict__ y, float* __restrict__ part,
+                       const __hip_bfloat16* __restrict__ x, const __hip_bfloat16* __restrict__ w,
+                       const int M, const int N, const int K, const int depth, const int tile,
+                       const int own, const int parts) {
   using R = ring_gemm::Ring<BM, BN, 2, 2, SLOTS, HINT>;
   constexpr int COLS = GATED ? BN / 2 : BN;              // outputs of a block
   constexpr int OUT = GATED ? R::kTN / 2 : R::kTN;       // output tiles of a wave
-  __shared__ __align__(16) char lds[R::kLds];
   // Each XCD has a run of neighbours: bands of up to eight tiles of rows, column by column,
   // so that the tiles that run at a time share rows of x and of W in its L2
   const int m_tiles = (M + BM - 1) / BM, n_tiles = N / COLS, blocks = m_tiles * n_tiles;
-  const int per_xcd = (blocks + 7) / 8, slot = blockIdx.x / 8;
-  const int id = (blockIdx.x % 8) * per_xcd + slot;
+  const int per_xcd = (blocks + 7) / 8, slot = tile / 8;
+  const int id = (tile % 8) * per_xcd + slot;
   if (slot >= per_xcd || id >= blocks) return;
   const int band = id / (8 * n_tiles), in = id % (8 * n_tiles), high = min(8, m_tiles - band * 8);
-  const int m0 = (band * 8 + in % high) * BM, n0 = in / high * COLS, k0 = blockIdx.y * depth;
+  const int m0 = (band * 8 + in % high) * BM, n0 = in / high * COLS, k0 = own * depth;
 
   f32x4_t acc[R::kTM][R::kTN];
   R::clear(acc);
@@ -69,8 +71,8 @@ __global__ __launch_bounds__(256, OCC) void gemm_ring_kernel(
     }
 #pragma unroll
     for (int j = 0; j + 1 < OUT; j += 2) {
-      if (!GATED && gridDim.y > 1) {
-        float* to = part + blockIdx.y * ((long)M * N) + at + j * 16;
+      if (!GATED && parts > 1) {
+        float* to = part + own * ((long)M * N) + at + j * 16;
         *reinterpret_cast<f32x4_t*>(to) = acc[i][j];
         *reinterpret_cast<f32x4_t*>(to + 4) = acc[i][j + 1];
         continue;
@@ -83,6 +85,49 @@ __global__ __launch_bounds__(256, OCC) void gemm_ring_kernel(
       *reinterpret_cast<uint4*>(y + at + j * 16) = o.u;
     }
   }
+}
+
+// grid (tiles of y, parts of K)
+template <int BM, int BN, int SLOTS, int OCC, bool GATED, int HINT = 0>
+__global__ __launch_bounds__(256, OCC) void gemm_ring_kernel(
+    __hip_bfloat16* __restrict__ y, float* __restrict__ part,
+    const __hip_bfloat16* __restrict__ x, const __hip_bfloat16* __restrict__ w, const int M,
+    const int N, const int K, const int depth) {
+  __shared__ __align__(16) char lds[ring_gemm::Ring<BM, BN, 2, 2, SLOTS, HINT>::kLds];
+  product<BM, BN, SLOTS, GATED, HINT>(lds, y, part, x, w, M, N, K, depth, blockIdx.x, blockIdx.y,
+                                      gridDim.y);
+}
+
+// The same, and beside it what the adapters of its rows need of x: `ahead` workgroups (a multiple of
+// eight, so that tiles stay on their XCDs) that begin first, on CUs that the product's leave
+// free or beside them.  In a launch of their own they took 4.0 to 5.2 us and a gap, all of it latency;
+// here the product's weights go by meanwhile.  With expand, us, 61 rows, 4 adapters of rank 16, in two
+// launches and in one: 6144 x 4096 24.6 20.0, 4096 x 4096 18.3 16.3, gated 28672 x 4096 66.9 63.2, 4096 x 14336
+// 36.0 33.6; 24 rows 4096 x 4096 16.2 14.5, 32 rows 3072 x 2048 14.4 10.6.
+constexpr int kShrinkTiles = 2;   // 16-wide tiles of a workgroup: one form for all ranks
+
+template <int BM, int BN, int SLOTS, int OCC, int HINT>
+__global__ __launch_bounds__(256, OCC) void gemm_ring_lora(
+    __hip_bfloat16* __restrict__ y, float* __restrict__ part,
+    const __hip_bfloat16* __restrict__ x, const __hip_bfloat16* __restrict__ w, const int M,
+    const int N, const int K, const int depth, const int parts, const int tiles,
+    const lora::Shrink shrink, const int adapters, const int ahead) {
+  using R = ring_gemm::Ring<BM, BN, 2, 2, SLOTS, HINT>;
+  static_assert(R::kLds >= lora::shrink_lds(kShrinkTiles) && lora::kShrinkWaves == 4, "shared");
+  __shared__ __align__(16) char lds[R::kLds];
+  int id = blockIdx.x;
+  if (id < ahead) {
+    const int wide = (shrink.PR + 16 * kShrinkTiles - 1) / (16 * kShrinkTiles);
+    const int cut = id % shrink.cuts, row = id / shrink.cuts % wide;
+    id /= shrink.cuts * wide;
+    const int groups = lora::groups_of(lora::kWindow, adapters);   // of a window
+    lora::shrink<kShrinkTiles, true>(shrink, cut, adapters, id / groups * lora::kWindow,
+                                     id % groups, row * 16 * kShrinkTiles, lds);
+    return;
+  }
+  id -= ahead;
+  product<BM, BN, SLOTS, false, HINT>(lds, y, part, x, w, M, N, K, depth, id % tiles, id / tiles,
+                                      parts);
 }
 
 // A tile's form and what its time is made of, in us, fitted to some 25000 measured products of 65
@@ -180,6 +225,14 @@ Plan plan_of(int M, int N, int K, bool gated) {
   return best;
 }
 
+// W that is read once and is large goes past the caches (24 rows by 64 x 64: 28672 x 4096 46.4 ->
+// 39.9 us, 8192 x 3584 15.6 -> 13.8, 4096 x 4096 11.5 -> 11.5, 64 rows 12.6 -> 13.5; larger tiles, all
+// rows in one: 8192 x 8192 by 128 x 128 0.88 of the time, 4096 x 14336 0.91, 5120 x 8192 0.97, but
+// 7168 x 4096 1.02, 6144 x 4096 1.05)
+bool read_once(int M, long weights, int form) {
+  return M <= kForms[form].bm && weights >= (form == kFew ? 20000000 : 40000000);
+}
+
 template <int BM, int BN, int SLOTS, int OCC, bool GATED, int HINT = 0>
 void launch_form(__hip_bfloat16* y, float* part, const __hip_bfloat16* x, const __hip_bfloat16* w,
                  int M, int N, int K, int parts, hipStream_t stream) {
@@ -190,16 +243,31 @@ void launch_form(__hip_bfloat16* y, float* part, const __hip_bfloat16* x, const 
                      K, depth);
 }
 
+// The workgroups that shrink M rows beside a product
+int beside(int M, int PR, int adapters, int cuts) {
+  const int wide = (PR + 16 * kShrinkTiles - 1) / (16 * kShrinkTiles);
+  const int groups = M / lora::kWindow * lora::groups_of(lora::kWindow, adapters) +
+                     lora::groups_of(M % lora::kWindow, adapters);
+  return (cuts * wide * groups + 7) / 8 * 8;
+}
+
+template <int BM, int BN, int SLOTS, int OCC, int HINT>
+void launch_lora_form(__hip_bfloat16* y, float* part, const __hip_bfloat16* x,
+                      const __hip_bfloat16* w, int M, int N, int K, int parts,
+                      const lora::Shrink& shrink, int adapters, hipStream_t stream) {
+  const long tiles = ((M + BM - 1) / BM * (long)(N / BN) + 7) / 8 * 8;
+  const int ahead = beside(M, shrink.PR, adapters, shrink.cuts);
+  const int depth = (K / 64 + parts - 1) / parts * 64;
+  hipLaunchKernelGGL((gemm_ring_lora<BM, BN, SLOTS, OCC, HINT>), dim3(ahead + tiles * parts),
+                     dim3(256), 0, stream, y, part, x, w, M, N, K, depth, parts, (int)tiles, shrink,
+                     adapters, ahead);
+}
+
 template <bool GATED>
 void launch_plan(__hip_bfloat16* y, float* part, const __hip_bfloat16* x, const __hip_bfloat16* w,
                  int M, int N, int K, int plan, hipStream_t stream) {
   const int parts = plan & 15, form = plan >> 4;
-  // W that is read once and is large goes past the caches (24 rows by 64 x 64: 28672 x 4096 46.4 ->
-  // 39.9 us, 8192 x 3584 15.6 -> 13.8, 4096 x 4096 11.5 -> 11.5, 64 rows 12.6 -> 13.5; larger tiles, all
-  // rows in one: 8192 x 8192 by 128 x 128 0.88 of the time, 4096 x 14336 0.91, 5120 x 8192 0.97, but
-  // 7168 x 4096 1.02, 6144 x 4096 1.05)
-  const bool once = M <= kForms[form].bm &&
-                    (GATED ? 2L : 1L) * N * K >= (form == kFew ? 20000000 : 40000000);
+  const bool once = read_once(M, (GATED ? 2L : 1L) * N * K, form);
 #define GO(BM, BN, SLOTS, OCC)                                                         \
   if (once) launch_form<BM, BN, SLOTS, OCC, GATED, 2>(y, part, x, w, M, N, K, parts, stream); \
   else launch_form<BM, BN, SLOTS, OCC, GATED>(y, part, x, w, M, N, K, parts, stream); \
@@ -327,4 +395,37 @@ void launch_gemm_ring_parts(__hip_bfloat16* y, float* part, const __hip_bfloat16
                             const __hip_bfloat16* w, int M, int N, int K, int plan,
                             hipStream_t stream) {
   launch_plan<false>(y, part, x, w, M, N, K, plan, stream);
+}
+
+// Parts of K for the adapters' shrink beside a product by `plan`, 0: in a launch of its own.  There
+// is time beside a product, so K is cut less than it is alone and expand has fewer sums to add, but
+// a wave's eight steps are short of the shortest product (K 8192, 40 rows, rank 64: four parts 22.1 us,
+// eight 18.9, alone 21.4).  Each of its workgroups holds the LDS of one of the product's, two a CU:
+// up to one a CU they are done when the product's later ones would begin; more keep it waiting
+// (sides: alone, beside; 4096 x 14336, 96 rows, 32 adapters of rank 8: 481 workgroups 38.9 52.9; 4096 x
+// 4096, 512 rows, 8 of rank 64: 384 70.9 83.6; but 256 rows, 2 of rank 64: 144 42.6 40.3).
+int gemm_ring_lora_cuts(int M, int K, int L, int PR, int plan) {
+  const int cuts = std::min(lora_shrink_cuts(M, K), std::max(4, K / 1024));
+  return plan >> 4 >= 2 && beside(M, PR, L, cuts) <= 256 ? cuts : 0;
+}
+
+// launch_gemm_ring_parts and, in the same launch, tmp [cuts, M, PR] = the rows of A x of each
+// row's adapter, in parts
+void launch_gemm_ring_lora(__hip_bfloat16* y, float* part, const __hip_bfloat16* x,
+                           const __hip_bfloat16* w, int M, int N, int K, int plan, float* tmp,
+                           const __hip_bfloat16* a, const int* slots, int L, int PR, int cuts,
+                           hipStream_t stream) {
+  const int parts = plan & 15, form = plan >> 4;
+  const lora::Shrink shrink{tmp, x, a, slots, M, PR, K, cuts};
+  const bool once = read_once(M, (long)N * K, form);
+#define GO(BM, BN, SLOTS, OCC)                                                              \
+  if (once) launch_lora_form<BM, BN, SLOTS, OCC, 2>(y, part, x, w, M, N, K, parts, shrink, L, stream); \
+  else launch_lora_form<BM, BN, SLOTS, OCC, 0>(y, part, x, w, M, N, K, parts, shrink, L, stream); \
+  break
+  switch (form) {
+    case 2: GO(128, 128, 4, 2);
+    case 3: GO(64, 128, 6, 2);
+    default: GO(64, 64, 8, 2);
+  }
+#undef GO
 }

@@ -17,7 +17,8 @@
 // read and write of out.
 //
 // Layers of 4096 wide rows, 61 tokens of 4 adapters of rank 16: 7 + 7 launches of 25 and
-// 5 us were 4 + 4 of 4.6 and 4.0 to 7.8.  2048 tokens: shrink 23 us, expand into 4096 columns 14
+// 5 us were 4 + 4 of 4.6 and 4.0 to 7.8; of these the shrinks go beside their products now
+// (gemm_ring_lora), a pass of 604 us is one of 548.  2048 tokens: shrink 23 us, expand into 4096 columns 14
 // and into 28672 102, where reading and writing out takes 51.
 //
 // f32 and f16: one token per workgroup in both,
@@ -26,7 +27,7 @@
 //   expand: R <= 64 fits a lane-resident tmp row; each thread owns one
 //           output column and walks r with the B row loads coalesced.
 
-#include "common.h"
+#include "lora_shrink.h"
 
 // ---------------------------------------------------------------------------
 // shrink: tmp[T, R] (f32) = A[slot(t)] · x[t]
@@ -136,9 +137,6 @@ void launch_lora_expand(T* out, const float* tmp, const T* b_stack,
 // bf16
 // ---------------------------------------------------------------------------
 
-typedef __attribute__((ext_vector_type(8))) short bf16x8_t;
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-
 // virtual column v of projection p (v < end[p]) is column v + shift[p] of out
 struct LoraCols {
   int end[3], shift[3];
@@ -146,89 +144,20 @@ struct LoraCols {
 
 namespace {
 
-constexpr int kShrinkWaves = 4;
-constexpr int kWindow = 256;   // tokens that are grouped by adapter
+using lora::kShrinkWaves;
 
-// grid (cuts of K, adapters, windows of kWindow tokens x kWindow / 16 groups): a group is 16
-// tokens of the window that have the adapter, in any order, and ends at once where there
-// are no more.  Groups are numbered slowest, so that the ones that have tokens lie next to
-// each other and on all XCDs.  tmp [cuts, T, PR]; tokens without an adapter are left unwritten.
-//
-// Groups of neighbours instead read every adapter of a mixed batch's 16 tokens for one or
-// two of them.  32 adapters of rank 8 dealt out at random, 1024 x 4096, us with expand, a
-// token a workgroup, neighbours, windows: 256 tokens 10.3 17.4 9.5, 1000 14.4 33.9 15.1.
+// grid (cuts, adapters, windows x kWindow / 16 groups): groups are numbered slowest, so that the
+// ones that have tokens lie next to each other and on all XCDs
 template <int TILES>   // 16-wide tiles of PR
 __global__ __launch_bounds__(64 * kShrinkWaves) void lora_shrink_tile_kernel(
     float* __restrict__ tmp, const __hip_bfloat16* __restrict__ x,
     const __hip_bfloat16* __restrict__ a_stack, const int* __restrict__ slots, const int T,
     const int PR, const int K) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int col = lane & 15, quad = lane >> 4;
-  const int cut = blockIdx.x, slot = blockIdx.y;
-  const int t0 = blockIdx.z / (kWindow / 16) * kWindow;
-  const int first = blockIdx.z % (kWindow / 16) * 16;   // of the window's tokens of this slot
-  __shared__ int group[kShrinkWaves][16];
-  int slot_of[kWindow / 64], found = 0;
-#pragma unroll
-  for (int i = 0; i < kWindow / 64; ++i)
-    slot_of[i] = t0 + i * 64 + lane < T ? slots[t0 + i * 64 + lane] : -1;
-#pragma unroll
-  for (int i = 0; i < kWindow / 64; ++i) {
-    const unsigned long long has = __ballot(slot_of[i] == slot);
-    const int at = found + __popcll(has & ((1ull << lane) - 1)) - first;
-    if (slot_of[i] == slot && at >= 0 && at < 16) group[wave][at] = t0 + i * 64 + lane;
-    found += __popcll(has);
-  }
-  const int tokens = min(found - first, 16);
-  if (tokens <= 0) return;
-  // other lanes of this wave read it: LDS keeps a wave's order, the compiler has to
-  asm volatile("" ::: "memory");
-  const int own = group[wave][min(col, tokens - 1)];
-
-  const __hip_bfloat16* xr = x + (long)own * K + quad * 8;
-  const __hip_bfloat16* ar[TILES];
-#pragma unroll
-  for (int j = 0; j < TILES; ++j)
-    ar[j] = a_stack + ((long)slot * PR + min(j * 16 + col, PR - 1)) * K + quad * 8;
-  f32x4_t acc[TILES];
-#pragma unroll
-  for (int j = 0; j < TILES; ++j) acc[j] = f32x4_t{};
-
-  const int steps = (K + 31) / 32, stride = gridDim.x * kShrinkWaves;
-  constexpr int AHEAD = TILES <= 4 ? 4 : 2;
-  for (int s0 = cut * kShrinkWaves + wave; s0 < steps; s0 += AHEAD * stride) {
-    bf16x8_t xf[AHEAD], af[AHEAD][TILES];
-#pragma unroll
-    for (int u = 0; u < AHEAD; ++u) {
-      const int k = (s0 + u * stride) * 32;
-      const bool in = k + quad * 8 < K;   // K % 8 == 0: a lane's eight inputs are in or out
-      xf[u] = in ? *reinterpret_cast<const bf16x8_t*>(xr + k) : bf16x8_t{};
-#pragma unroll
-      for (int j = 0; j < TILES; ++j)
-        af[u][j] = in ? *reinterpret_cast<const bf16x8_t*>(ar[j] + k) : bf16x8_t{};
-    }
-#pragma unroll
-    for (int u = 0; u < AHEAD; ++u)
-#pragma unroll
-      for (int j = 0; j < TILES; ++j)
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[u], af[u][j], acc[j], 0, 0, 0);
-  }
-
-  __shared__ f32x4_t all[kShrinkWaves][TILES][64];
-#pragma unroll
-  for (int j = 0; j < TILES; ++j) all[wave][j][lane] = acc[j];
-  __syncthreads();
-  for (int j = wave; j < TILES; j += kShrinkWaves) {
-    f32x4_t v = all[0][j][lane];
-#pragma unroll
-    for (int w = 1; w < kShrinkWaves; ++w) v += all[w][j][lane];
-    const int r = j * 16 + col;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = quad * 4 + i, t = __shfl(own, m, 64);
-      if (m < tokens && r < PR) tmp[((long)cut * T + t) * PR + r] = v[i];
-    }
-  }
+  __shared__ __align__(16) char lds[lora::shrink_lds(TILES)];
+  constexpr int GROUPS = lora::kWindow / 16;
+  lora::shrink<TILES, false>(lora::Shrink{tmp, x, a_stack, slots, T, PR, K, (int)gridDim.x},
+                             blockIdx.x, blockIdx.y, blockIdx.z / GROUPS * lora::kWindow,
+                             blockIdx.z % GROUPS * 16, 0, lds);
 }
 
 // The cuts' sums of a workgroup's tokens.  FEW: eight parts are asked for at once.

@@ -62,3 +62,46 @@ def test_product(t, k, width, spans, rank, gated, given):
         off = 1.1 * (og * (up.abs() + ou)) + ou * gate.abs() + 1e-5 * want.abs()
     err = (out.double() - want).abs()
     assert (err <= 2 ** -8 * want.abs() + off + 1e-7).all(), err.max().item()
+
+
+# rows, adapters, K, rank: edges of the 16 tokens of a group and the 256 of a window, more adapters
+# than rows, K that its parts do not divide; up to 256 workgroups go beside the product
+@pytest.mark.parametrize(("t", "adapters", "k", "rank"), [
+    (1, 40, 4096, 16), (15, 1, 4160, 8), (16, 16, 1024, 64), (17, 3, 14336, 32), (63, 60, 4096, 8),
+    (64, 4, 64, 64), (255, 2, 2048, 64), (256, 1, 4096, 8), (257, 3, 1088, 16), (272, 30, 1024, 8),
+    (513, 1, 4096, 32), (600, 2, 4096, 8), (600, 9, 4096, 64),
+])
+@pytest.mark.parametrize("some", [False, True])
+def test_adapters_beside_the_product(t, adapters, k, rank, some):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from vllm_tgis_adapter_amd.ops import _C
+
+    g = torch.Generator("cuda").manual_seed(t + k + rank)
+
+    def normal(*shape, by=1.0):
+        return (torch.randn(shape, generator=g, device="cuda") * by).bfloat16()
+
+    width, spans = 384, [(0, 256), (256, 384)]
+    x, w = normal(t, k), normal(width, k, by=k ** -0.5)
+    a, b = normal(adapters, 2 * rank, k, by=k ** -0.5), normal(adapters, width, rank)
+    slots = torch.randint(-1, adapters, (t,), generator=g, device="cuda").int()
+    if not some:   # the last one alone, then a row without
+        slots[:] = adapters - 1
+        slots[t - 1] = -1
+    scales = torch.linspace(0.5, 2.0, adapters, device="cuda")
+    out = torch.full((t, width), float("nan"), device="cuda").bfloat16()
+    _C.lora_product(out, x, w, None, a, b, slots, scales, spans, False)
+
+    x, w, a, b = x.double(), w.double(), a.double(), b.double()
+    want = x @ w.t()
+    # a product of one part is rounded to bf16, sums are in float32
+    off = 2 ** -8 * want.abs() + 2 ** -20 * (x.abs() @ w.abs().t())
+    for s in slots.unique().tolist():
+        rows = (slots == s).nonzero().view(-1)
+        for p, (lo, hi) in enumerate(spans if s >= 0 else []):
+            aa, bb, scale = a[s, p * rank:(p + 1) * rank], b[s, lo:hi], scales[s].double()
+            want[rows, lo:hi] += scale * (x[rows] @ aa.t()) @ bb.t()
+            off[rows, lo:hi] += 2 ** -20 * scale * (x[rows].abs() @ aa.abs().t()) @ bb.abs().t()
+    err = (out.double() - want).abs()
+    assert (err <= 2 ** -8 * want.abs() + off + 1e-7).all(), err.max().item()
