@@ -60,3 +60,18 @@ def test_matches_the_reference(fp8, kvh, group, hd, block, lens, width):
     assert (out[live] - want).abs().max() <= bound
     assert torch.equal(out[[i for i, n in enumerate(lens) if not n]],
                        torch.zeros(len(lens) - len(live), kvh * group, hd))
+
+
+def test_every_byte_of_a_cache():
+    """One key: the result is its value, exactly, for all codes of e4m3."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from vllm_tgis_adapter_amd import ops
+
+    codes = torch.arange(256, dtype=torch.uint8, device="cuda").view(1, 1, 2, 128)
+    out = ops.paged_attention_decode(
+        torch.ones((1, 2, 128), device="cuda").bfloat16(), torch.zeros_like(codes), codes,
+        torch.zeros((1, 1), dtype=torch.int32, device="cuda"),
+        torch.ones(1, dtype=torch.int32, device="cuda"), 0.1, 1)
+    want = codes.view(torch.float8_e4m3fn).bfloat16().view(-1)
+    torch.testing.assert_close(out.view(-1), want, rtol=0, atol=0, equal_nan=True)
