@@ -109,7 +109,8 @@ template <typename T>
 void launch_sample_argmax(long*, const T*, const float*, const float*, int,
                           int, hipStream_t);
 void launch_moe_gemm(__hip_bfloat16*, const __hip_bfloat16*, const __hip_bfloat16*, const int*,
-                     const int*, int, int, int, int, int, hipStream_t);
+                     const int*, int, int, int, int, int, float*, hipStream_t);
+long moe_gemm_scratch(int E, int N, int K, int T, int mode);
 int moe_topk_max_experts();
 int moe_topk_max_top();
 void launch_moe_topk(int*, float*, const __hip_bfloat16*, const __hip_bfloat16*, int, int, int,
@@ -826,8 +827,12 @@ void moe_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w,
     rp = rows->data_ptr<int>();
   }
   if (T == 0) return;
+  torch::Tensor scratch;
+  if (const long floats = moe_gemm_scratch(E, N, K, T, (int)mode))
+    scratch = at::empty({floats}, x.options().dtype(at::ScalarType::Float));
   launch_moe_gemm(ptr<__hip_bfloat16>(y), cptr<__hip_bfloat16>(x), cptr<__hip_bfloat16>(w),
-                  seg_off.data_ptr<int>(), rp, E, N, K, T, (int)mode, current_stream());
+                  seg_off.data_ptr<int>(), rp, E, N, K, T, (int)mode,
+                  scratch.defined() ? scratch.data_ptr<float>() : nullptr, current_stream());
 }
 
 void moe_topk(torch::Tensor ids, torch::Tensor weights, torch::Tensor x, torch::Tensor gate) {

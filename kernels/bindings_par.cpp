@@ -34,7 +34,8 @@ template <typename T>
 void launch_moe_sort(T*, int*, int*, int*, const T*, long, const int*, int, int,
                      int, int, const float*, hipStream_t);
 void launch_moe_gemm(__hip_bfloat16*, const __hip_bfloat16*, const __hip_bfloat16*, const int*,
-                     const int*, int, int, int, int, int, hipStream_t);
+                     const int*, int, int, int, int, int, float*, hipStream_t);
+long moe_gemm_scratch(int E, int N, int K, int T, int mode);
 void launch_moe_gemm_clamped(__hip_bfloat16*, const __hip_bfloat16*, const __hip_bfloat16*,
                              const int*, int, int, int, int, float, hipStream_t);
 
@@ -342,9 +343,12 @@ void moe_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w,
   TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
               reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0, "x and w start at 16 bytes");
   if (T == 0) return;
+  torch::Tensor scratch;
+  if (const long floats = moe_gemm_scratch(E, N, K, T, (int)mode))
+    scratch = at::empty({floats}, x.options().dtype(at::ScalarType::Float));
   launch_moe_gemm(ptr<__hip_bfloat16>(y), ptr<__hip_bfloat16>(x),
                   ptr<__hip_bfloat16>(w), ptr<int>(seg_off), nullptr, E, N, K, T, (int)mode,
-                  stream());
+                  scratch.defined() ? scratch.data_ptr<float>() : nullptr, stream());
 }
 
 // clamped gate of the halves, see common.h

@@ -17,8 +17,8 @@
 //
 // Measured, 8 experts of 14336 x 4096 (two experts a token, MI355X): a layer's three
 // products and its routing, 33 tokens 723 -> 452 us (4.7 -> 6.2 TB/s), 2949 tokens 1950 (eight
-// waves on 256 x 256) -> 1707 us (1.22 PFLOP/s; the second product's 400 tiles are 1.6 rounds
-// of 256 CUs).
+// waves on 256 x 256) -> 1670 us (1.25 PFLOP/s; of the second product's 384 tiles, one and a half
+// rounds of 256 CUs, the last 128 have K cut in two; with 400, 144 are left, which stay whole).
 
 #include "gemm_stream.h"
 #include "ring_gemm.h"
@@ -27,26 +27,99 @@ namespace {
 
 using ring_gemm::f32x4_t;
 
+// Tiles that do not fill a last round of the chip leave CUs idle for as long as a whole one: 400
+// tiles of 256 x 256 are 1.6 rounds of 256 CUs.  So K of the tiles behind the last whole round is
+// cut in parts, a workgroup each, and the launch behind adds them up.
+constexpr int kCus = 256;
+constexpr int kMostParts = 2 * kCus - 1;   // of all those tiles
+
+struct Rounds {
+  int whole;          // tiles of one workgroup each
+  int parts, depth;   // of the others: parts of K, steps of a part
+};
+
+// A step takes 0.95 us where a workgroup has the chip's caches to itself and 1.5 beside 255 others
+// (the smaller tiles are hardly faster: 128 x 256 stay whole), a part 0.22 us to store and to add, the
+// launch 8.  4096 x 14336, 8 experts, tiles: whole tiles | with parts, us: 288 578 | 456, 384 620 | 578,
+// 576 899 | 790; 16 experts, 6144 x 8192: 792 744 | 685.  432, whose last 176 tiles are left whole: 650 | 652.
+// (Equal shares of all steps instead, whatever tile they belong to: 384 610 | 560, but 432
+// 622 | 710: workgroups at different inputs find nothing of each other's in the caches.)
+DEVINLINE Rounds rounds_of(int tiles, int steps, bool parted) {
+  const int rest = tiles % kCus;
+  Rounds best{tiles, 1, steps};
+  if (!parted || rest == 0) return best;
+  auto round = [](int blocks) { return blocks > 0 ? 0.95f + 0.55f / kCus * blocks : 0.f; };
+  float least = steps * round(rest);
+  for (int parts = 2; parts <= 8 && parts * rest <= kMostParts && parts * 8 <= steps; ++parts) {
+    const int depth = ((steps + parts - 1) / parts + 1) / 2 * 2, blocks = rest * parts;
+    const float us =
+        depth * (round(min(blocks, kCus)) + round(blocks - kCus)) + 8.f + blocks * 0.22f;
+    if (us < least) {
+      least = us;
+      best = Rounds{tiles - rest, parts, depth};
+    }
+  }
+  return best;
+}
+
+// What a lane holds of a tile: row i * 16 + lane % 16 of its wave's, columns in eights
+template <typename R, int OUT, int MODE>
+DEVINLINE void store(__hip_bfloat16* y, const moe::Tile& at, int N, int n0, int i,
+                     const f32x4_t (&acc)[R::kTN], float limit) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wm = wave / 2, wn = wave % 2, m = (wm * R::kTM + i) * 16 + (lane & 15);
+  if (m >= at.rows) return;
+  __hip_bfloat16* to = y + (long)(at.row0 + m) * N + n0 + wn * OUT * 16 + lane / 16 * 8;
+#pragma unroll
+  for (int j = 0; j < OUT; j += 2) {
+    union { __hip_bfloat16 h[8]; uint4 u; } o;
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+      o.h[r] = __float2bfloat16(moe::finish<MODE>(
+          acc[j + r / 4][r % 4], acc[(moe::gated(MODE) ? OUT : 0) + j + r / 4][r % 4], limit));
+    *reinterpret_cast<uint4*>(to + j * 16) = o.u;
+  }
+}
+
+// part: null, or room for kMostParts tiles of f32
 template <int BM, int BN, int SLOTS, int OCC, int MODE>
 __global__ __launch_bounds__(256, OCC) void moe_ring_kernel(
     __hip_bfloat16* __restrict__ y,        // [T, N]
     const __hip_bfloat16* __restrict__ x,  // [T, K] sorted by expert, or what segs.rows lists
     const __hip_bfloat16* __restrict__ w,  // [E, (gated ? 2 N : N), K]
-    const moe::Segments segs, const int N, const int K, const float limit) {
+    f32x4_t* __restrict__ part, const moe::Segments segs, const int N, const int K,
+    const float limit) {
   using R = ring_gemm::Ring<BM, BN, 2, 2, SLOTS>;
-  constexpr bool GATED = moe::gated(MODE);
+  constexpr bool GATED = moe::gated(MODE), PARTED = !GATED && BM == 256;
   constexpr int COLS = GATED ? BN / 2 : BN;              // outputs of a block
   constexpr int OUT = GATED ? R::kTN / 2 : R::kTN;       // output tiles of a wave
   __shared__ __align__(16) char lds[R::kLds];
 
-  const moe::Tile at = moe::find_tile(segs, BM, N / COLS);
-  if (at.rows == 0) return;
-  const int n0 = at.n * COLS;
+  const int steps = K / ring_gemm::kDepth, n_tiles = N / COLS;
+  const int tiles = moe::count_chunks(segs, BM) * n_tiles;
+  const Rounds rounds = rounds_of(tiles, steps, PARTED && part != nullptr);
+  const int per_xcd = (rounds.whole + 7) / 8, xcd = blockIdx.x % 8;
+  const int slot = blockIdx.x / 8 - per_xcd;
+  int id = xcd * per_xcd + blockIdx.x / 8, piece = -1, first = 0, own = steps;
+  if (slot < 0) {
+    if (id >= rounds.whole) return;
+  } else {   // part by part, so that what is read at a time is of the same inputs
+    if constexpr (!PARTED) return;
+    const int rest = tiles - rounds.whole, per = (rest * rounds.parts + 7) / 8;
+    piece = xcd * per + slot;
+    if (slot >= per || piece >= rest * rounds.parts) return;
+    id = rounds.whole + piece % rest;
+    first = piece / rest * rounds.depth;
+    own = min(rounds.depth, steps - first);
+  }
+  const moe::Tile at = moe::tile_of(segs, BM, n_tiles, id);
+  const int n0 = at.n * COLS, k0 = first * ring_gemm::kDepth;
   const unsigned row_bytes = K * 2;
   f32x4_t acc[R::kTM][R::kTN];
   R::clear(acc);
-  R::run(acc, lds, reinterpret_cast<const char*>(x),
-         reinterpret_cast<const char*>(w + ((long)at.expert * (GATED ? 2 : 1) * N + n0) * K), K,
+  R::run(acc, lds, reinterpret_cast<const char*>(x + k0),
+         reinterpret_cast<const char*>(w + ((long)at.expert * (GATED ? 2 : 1) * N + n0) * K + k0),
+         own * ring_gemm::kDepth,
          // rows past the segment: its last one, whose results are not written
          [&](int r) {
            const int row = at.row0 + min(r, at.rows - 1);
@@ -57,23 +130,41 @@ __global__ __launch_bounds__(256, OCC) void moe_ring_kernel(
            const int half = in / (OUT * 16);
            return (half * N + wave * (OUT * 16) + R::out_col(in % (OUT * 16))) * row_bytes;
          });
+  if (!PARTED || piece < 0) {
+#pragma unroll
+    for (int i = 0; i < R::kTM; ++i) store<R, OUT, MODE>(y, at, N, n0, i, acc[i], limit);
+  } else {
+    f32x4_t* to = part + (long)piece * (BM * BN / 4) + threadIdx.x;
+#pragma unroll
+    for (int i = 0; i < R::kTM; ++i)
+#pragma unroll
+      for (int j = 0; j < R::kTN; ++j) to[(i * R::kTN + j) * 256] = acc[i][j];
+  }
+}
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int col = lane & 15, quad = lane >> 4, wm = wave / 2, wn = wave % 2;
+// The parts of a tile become its results.  Grid (any, sixteenths of half of a tile's rows)
+template <int BM, int BN, int MODE>
+__global__ __launch_bounds__(256) void moe_parts_kernel(
+    __hip_bfloat16* __restrict__ y, const f32x4_t* __restrict__ part, const moe::Segments segs,
+    const int N, const int K, const float limit) {
+  using R = ring_gemm::Ring<BM, BN, 2, 2, 4>;
+  const int n_tiles = N / BN, i = blockIdx.y;
+  const int tiles = moe::count_chunks(segs, BM) * n_tiles;
+  const Rounds rounds = rounds_of(tiles, K / ring_gemm::kDepth, true);
+  const int rest = tiles - rounds.whole;
+  for (int own = blockIdx.x; own < rest; own += gridDim.x) {
+    const moe::Tile at = moe::tile_of(segs, BM, n_tiles, rounds.whole + own);
+    if (i * 16 >= at.rows) continue;   // (of the first half of its rows)
+    f32x4_t acc[R::kTN];
 #pragma unroll
-  for (int i = 0; i < R::kTM; ++i) {
-    const int m = (wm * R::kTM + i) * 16 + col;
-    if (m >= at.rows) continue;
-    __hip_bfloat16* to = y + (long)(at.row0 + m) * N + n0 + wn * OUT * 16 + quad * 8;
+    for (int j = 0; j < R::kTN; ++j) acc[j] = f32x4_t{};
+    for (int p = 0; p < rounds.parts; ++p) {
+      const f32x4_t* from =
+          part + (long)(p * rest + own) * (BM * BN / 4) + i * (R::kTN * 256) + threadIdx.x;
 #pragma unroll
-    for (int j = 0; j < OUT; j += 2) {
-      union { __hip_bfloat16 h[8]; uint4 u; } o;
-#pragma unroll
-      for (int r = 0; r < 8; ++r)
-        o.h[r] = __float2bfloat16(moe::finish<MODE>(
-            acc[i][j + r / 4][r % 4], acc[i][(GATED ? OUT : 0) + j + r / 4][r % 4], limit));
-      *reinterpret_cast<uint4*>(to + j * 16) = o.u;
+      for (int j = 0; j < R::kTN; ++j) acc[j] += from[j * 256];
     }
+    store<R, R::kTN, MODE>(y, at, N, at.n * BN, i, acc, limit);
   }
 }
 
@@ -119,8 +210,9 @@ namespace {
 template <int MODE>
 void launch_mode(__hip_bfloat16* y, const __hip_bfloat16* x, const __hip_bfloat16* w,
                  const int* seg_off, const int* x_rows, int E, int N, int K, int T,
-                 float limit, hipStream_t stream) {
+                 float limit, float* scratch, hipStream_t stream) {
   const moe::Segments segs{seg_off, E, x_rows};
+  f32x4_t* part = reinterpret_cast<f32x4_t*>(scratch);
   const int cols = moe::gated(MODE) ? 2 : 1;
 #define STREAM(MT, WN, WK)                                                                    \
   hipLaunchKernelGGL((gemm_stream::gemm_stream_kernel<16, MT, 1, WN, WK, MODE, true>),        \
@@ -128,8 +220,8 @@ void launch_mode(__hip_bfloat16* y, const __hip_bfloat16* x, const __hip_bfloat1
                      0, stream, y, nullptr, x, w, nullptr, 0, N, K, segs, limit)
 #define TILES(BM, BN, SLOTS, OCC)                                                             \
   hipLaunchKernelGGL((moe_ring_kernel<BM, BN, SLOTS, OCC, MODE>),                             \
-                     dim3(moe::max_blocks(T, E, BM, N * cols / BN)), dim3(256), 0, stream, y, \
-                     x, w, segs, N, K, limit)
+                     dim3(moe::max_blocks(T, E, BM, N * cols / BN) + (part ? kMostParts + 1 : 0)), \
+                     dim3(256), 0, stream, y, x, w, part, segs, N, K, limit)
   // Rows an expert, us gated / plain of what is chosen and its neighbour (8 experts, 4096 in
   // and 14336 between; rows are spread at random):
   //    8: <1,1,4> 270, <1,2,2> 144 (<2,2,2> 271, <4,4,2> 143);
@@ -163,7 +255,13 @@ void launch_mode(__hip_bfloat16* y, const __hip_bfloat16* x, const __hip_bfloat1
   else if (mean <= 18 && moe::gated(MODE)) STREAM(2, 2, 2);
   else if (far || (mean <= 52 && !brim)) STREAM(4, 4, 2);
   else switch (moe_tile(mean, E, N * cols, K, moe::gated(MODE))) {
-    case 0: TILES(256, 256, 4, 1); break;
+    case 0:
+      TILES(256, 256, 4, 1);
+      if constexpr (!moe::gated(MODE))
+        if (part)
+          hipLaunchKernelGGL((moe_parts_kernel<256, 256, MODE>), dim3(kCus / 2, 8), dim3(256), 0,
+                             stream, y, part, segs, N, K, limit);
+      break;
     case 1: TILES(128, 256, 4, 1); break;
     default: TILES(128, 128, 5, 2);
   }
@@ -173,19 +271,27 @@ void launch_mode(__hip_bfloat16* y, const __hip_bfloat16* x, const __hip_bfloat1
 
 }  // namespace
 
+// Floats of scratch that launch_moe_gemm wants, 0: none.  From 8192 inputs on: below, parts save no
+// more than they cost (7168, 416 tiles 323 | 330 us) and the launch that finds nothing to add is 2 to 4 us.
+long moe_gemm_scratch(int E, int N, int K, int T, int mode) {
+  const bool large =
+      mode != 1 && K >= 8192 && T / E > 52 && moe_tile(T / E, E, N, K, false) == 0;
+  return large ? (long)kMostParts * 256 * 256 : 0;
+}
+
 void launch_moe_gemm(__hip_bfloat16* y, const __hip_bfloat16* x, const __hip_bfloat16* w,
                      const int* seg_off, const int* x_rows, int E, int N, int K, int T,
-                     int mode, hipStream_t stream) {
+                     int mode, float* scratch, hipStream_t stream) {
   if (mode == 1)
-    launch_mode<moe::kSilu>(y, x, w, seg_off, x_rows, E, N, K, T, 0.f, stream);
+    launch_mode<moe::kSilu>(y, x, w, seg_off, x_rows, E, N, K, T, 0.f, scratch, stream);
   else if (mode == 2)
-    launch_mode<moe::kRelu2>(y, x, w, seg_off, x_rows, E, N, K, T, 0.f, stream);
+    launch_mode<moe::kRelu2>(y, x, w, seg_off, x_rows, E, N, K, T, 0.f, scratch, stream);
   else
-    launch_mode<moe::kPlain>(y, x, w, seg_off, x_rows, E, N, K, T, 0.f, stream);
+    launch_mode<moe::kPlain>(y, x, w, seg_off, x_rows, E, N, K, T, 0.f, scratch, stream);
 }
 
 void launch_moe_gemm_clamped(__hip_bfloat16* y, const __hip_bfloat16* x,
                              const __hip_bfloat16* w, const int* seg_off, int E, int N, int K,
                              int T, float limit, hipStream_t stream) {
-  launch_mode<moe::kClamped>(y, x, w, seg_off, nullptr, E, N, K, T, limit, stream);
+  launch_mode<moe::kClamped>(y, x, w, seg_off, nullptr, E, N, K, T, limit, nullptr, stream);
 }

@@ -36,9 +36,8 @@ struct Tile {
 // (blockIdx.x % 8) has a run of neighbours: chunks that read the same columns of W, and
 // columns that read the same rows, meet in one L2.  Segment sizes stay on the device;
 // the launch covers the most blocks there can be (max_blocks) and the rest end here.
-DEVINLINE Tile find_tile(const Segments& s, int chunk, int n_tiles) {
+DEVINLINE int count_chunks(const Segments& s, int chunk) {   // of all experts
   const int lane = threadIdx.x & 63;
-  // chunks of all experts
   int total = 0;
   for (int e0 = 0; e0 < s.experts; e0 += 64) {
     const int e = e0 + lane;
@@ -48,11 +47,12 @@ DEVINLINE Tile find_tile(const Segments& s, int chunk, int n_tiles) {
     for (int d = 32; d > 0; d >>= 1) c += __shfl_xor(c, d, 64);
     total += c;
   }
-  total = __builtin_amdgcn_readfirstlane(total);
-  const int blocks = total * n_tiles, per_xcd = (blocks + 7) / 8;
-  const int slot = blockIdx.x / 8;
-  int id = (blockIdx.x % 8) * per_xcd + slot;
-  if (slot >= per_xcd || id >= blocks) return Tile{0, 0, 0, 0};
+  return __builtin_amdgcn_readfirstlane(total);
+}
+
+// The tile of number `id`, which is one of count_chunks(s, chunk) * n_tiles
+DEVINLINE Tile tile_of(const Segments& s, int chunk, int n_tiles, int id) {
+  const int lane = threadIdx.x & 63;
   for (int e0 = 0; e0 < s.experts; e0 += 64) {
     const int e = e0 + lane;
     int lo = 0, rows = 0;
@@ -83,6 +83,13 @@ DEVINLINE Tile find_tile(const Segments& s, int chunk, int n_tiles) {
     return Tile{e0 + at, n, lo_e + m * chunk, min(chunk, rows_e - m * chunk)};
   }
   return Tile{0, 0, 0, 0};
+}
+
+DEVINLINE Tile find_tile(const Segments& s, int chunk, int n_tiles) {
+  const int blocks = count_chunks(s, chunk) * n_tiles, per_xcd = (blocks + 7) / 8;
+  const int slot = blockIdx.x / 8, id = (blockIdx.x % 8) * per_xcd + slot;
+  if (slot >= per_xcd || id >= blocks) return Tile{0, 0, 0, 0};
+  return tile_of(s, chunk, n_tiles, id);
 }
 
 // The most blocks that rows of these many experts can make, a multiple of eight.
