@@ -18,7 +18,7 @@
 //
 // Measured (MI355X, 32/8 heads of 128, two layers with their cache writes): 512
 // sequences of ~520 keys, bf16: 794 -> 361 us (2.8 -> 6.1 TB/s; a plain read
-// reaches 6.3); 41 of ~4800 keys, e4m3: 1365 -> 167 us (the former kernel ran 328
+// reaches 6.3); 41 of ~4800 keys, e4m3: 1365 -> 165 us (the former kernel ran 328
 // workgroups there).  On the way: three workgroups a CU instead of two spill, 427;
 // cached loads, 407; keys loaded straight into the operand's layout, 398.
 
@@ -50,6 +50,11 @@ DEVINLINE int tiles_per_part(int tiles, int npart) {
   return max(kMinTiles, (per + kWaves - 1) / kWaves * kWaves);
 }
 
+// A load that is asked for where it stands: the compiler would move it behind a branch
+template <typename T> DEVINLINE T load_here(const T* at) {
+  return __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+
 template <int HD, typename CT>
 __global__ __launch_bounds__(256, 2) void paged_decode_stream_kernel(
     __hip_bfloat16* __restrict__ out,       // [nseq, nheads, HD]
@@ -72,6 +77,19 @@ __global__ __launch_bounds__(256, 2) void paged_decode_stream_kernel(
 
   const int seq = blockIdx.x, kv_head = blockIdx.y, part = blockIdx.z;
   const int npart = gridDim.z;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int* table = block_tables + (long)seq * max_blocks;
+
+  // Where a launch is short, and a workgroup's first tile does not depend on the length, block ids
+  // are asked for beside it (with the merge's loads, us: one sequence of 230 keys of 64 6.8 -> 6.5, of
+  // 700 keys of 128 8.4 -> 8.0, of 8000 in e4m3 16.8 -> 15.1; 512 of 520, uncut, 183.3 -> 184.1).
+  // Past the end of the sequence, but not of its table, they may be anything.
+  const int most = max_blocks * block_size;
+  const bool early = npart > 1 && (part == 0 || most <= npart * (kMinTiles * kTile));
+  auto page_of = [&](int pos) { return block_shift >= 0 ? pos >> block_shift : pos / block_size; };
+  const int pos0 = (part * kMinTiles + wave) * kTile + (lane & 31);
+  int entry0 = 0;
+  if (early) entry0 = load_here(table + page_of(min(pos0, most - 1)));
   const int seq_len = seq_lens[seq];
   const int tiles = (seq_len + kTile - 1) / kTile;
   const int tpp = tiles_per_part(tiles, npart);
@@ -80,10 +98,8 @@ __global__ __launch_bounds__(256, 2) void paged_decode_stream_kernel(
   if (lo >= tiles && part > 0) return;
   const int hi = min(lo + tpp, tiles);
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 15, quad = lane >> 4;
   const int head0 = kv_head * group;
-  const int* table = block_tables + (long)seq * max_blocks;
   const long row_elems = (long)kvh * HD;
 
   __shared__ __align__(16) __hip_bfloat16 tile_all[kWaves][kTile * HD];
@@ -102,7 +118,7 @@ __global__ __launch_bounds__(256, 2) void paged_decode_stream_kernel(
   // cache row of key (tile * 32 + lane % 32); past the end: of the last key
   auto slot_of = [&](int tile) {
     const int pos = min(tile * kTile + (lane & 31), seq_len - 1);
-    const int page = block_shift >= 0 ? pos >> block_shift : pos / block_size;
+    const int page = page_of(pos);
     return table[page] * block_size + (pos - page * block_size);
   };
 
@@ -151,7 +167,15 @@ __global__ __launch_bounds__(256, 2) void paged_decode_stream_kernel(
 
   int t = lo + wave, slot_next = 0;
   if (t < hi) {
-    issue(slot_of(t));
+    int slot;
+    if (early) {   // past the end: of the tile's first key
+      slot = (unsigned)entry0 * block_size + (pos0 - page_of(pos0) * block_size);
+      const int begin = __shfl(slot, 0, 64);
+      if (pos0 >= seq_len) slot = begin;
+    } else {
+      slot = slot_of(t);
+    }
+    issue(slot);
     if (t + kWaves < hi) slot_next = slot_of(t + kWaves);
   }
   for (; t < hi; t += kWaves) {
@@ -279,27 +303,34 @@ __global__ __launch_bounds__(HD) void decode_stream_merge_kernel(
     const float* __restrict__ part_ml, const int* __restrict__ seq_lens,
     const int nheads, const int npart) {
   const int seq = blockIdx.x, d = threadIdx.x;
+  const long row = (long)seq * nheads + blockIdx.y;
+  const int lane = d & 63;
+  const float* ml = part_ml + row * npart * 2;
+  const float* acc = part_acc + row * npart * HD + d;
+  // asked for beside the length: parts that are not used hold anything, and are not
+  const float m0 = load_here(ml + 2 * min(lane, npart - 1));
+  const float l0 = load_here(ml + 2 * min(lane, npart - 1) + 1);
+  float v[8];   // eight loads on their way at a time
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = load_here(acc + (long)min(i, npart - 1) * HD);
   const int tiles = (seq_lens[seq] + kTile - 1) / kTile;
   const int tpp = tiles_per_part(tiles, npart);
   if (tpp >= tiles) return;
   const int used = (tiles + tpp - 1) / tpp;   // <= npart <= 64
-  const long row = (long)seq * nheads + blockIdx.y;
-  const int lane = d & 63;
-  const float* ml = part_ml + row * npart * 2;
-  const float m = lane < used ? ml[2 * lane] : -FLT_MAX;
-  const float l = lane < used ? ml[2 * lane + 1] : 0.f;
+  const float m = lane < used ? m0 : -FLT_MAX;
+  const float l = lane < used ? l0 : 0.f;
   const float M = wave_reduce_max(m);
   const float f = lane < used ? __builtin_amdgcn_exp2f(m - M) : 0.f;
   const float L = wave_reduce_sum(f * l);
-  const float* acc = part_acc + row * npart * HD + d;
   float a = 0.f;
-  for (int p0 = 0; p0 < used; p0 += 8) {   // eight loads on their way at a time
-    float v[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = acc[(long)min(p0 + i, used - 1) * HD];
+  for (int p0 = 0;;) {
 #pragma unroll
     for (int i = 0; i < 8; ++i)
       if (p0 + i < used) a += __shfl(f, p0 + i, 64) * v[i];
+    p0 += 8;
+    if (p0 >= used) break;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = acc[(long)min(p0 + i, used - 1) * HD];
   }
   out[row * HD + d] = __float2bfloat16(a * (L > 0.f ? 1.f / L : 0.f));
 }

@@ -75,3 +75,23 @@ def test_every_byte_of_a_cache():
         torch.ones(1, dtype=torch.int32, device="cuda"), 0.1, 1)
     want = codes.view(torch.float8_e4m3fn).bfloat16().view(-1)
     torch.testing.assert_close(out.view(-1), want, rtol=0, atol=0, equal_nan=True)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize(("block", "lens", "width"), [
+    (16, EDGES, 512), (16, [130, 640, 641, 1900], 160), (24, [3, 25, 1000, 3840], 160),
+    (1, [1, 33, 129, 300], 320)])
+def test_block_ids_past_the_end_say_nothing(fp8, block, lens, width):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from vllm_tgis_adapter_amd import ops
+
+    kc, vc, tables = (t.cuda() for t in _caches(lens, block, 2, 128, fp8, 5, width))
+    q = torch.randn(len(lens), 8, 128, generator=torch.Generator().manual_seed(6)).bfloat16().cuda()
+    seq_lens = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    want = ops.paged_attention_decode(q, kc, vc, tables, seq_lens, 0.1, max(lens))
+    used = (seq_lens + block - 1) // block
+    past = torch.arange(width, device="cuda")[None] >= used[:, None]
+    got = ops.paged_attention_decode(
+        q, kc, vc, tables.masked_fill(past, 2 ** 31 - 1), seq_lens, 0.1, max(lens))
+    assert torch.equal(got, want)
