@@ -93,7 +93,7 @@ int lora_shrink_cuts(int T, int K);
 void launch_lora_shrink_tiles(float*, const __hip_bfloat16*, const __hip_bfloat16*, const int*,
                               int, int, int, int, int, hipStream_t);
 void launch_lora_finish(__hip_bfloat16*, const __hip_bfloat16*, const float*, const float*,
-                        const __hip_bfloat16*, const int*, const float*, const LoraCols&, int, int,
+                        const __hip_bfloat16*, const int*, const float*, const LoraCols&, int, int, int,
                         int, int, int, int, int, bool, hipStream_t);
 void launch_lora_tiles(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hip_bfloat16*,
                        const __hip_bfloat16*, const int*, const float*, const LoraCols&, int,
@@ -759,7 +759,7 @@ void lora_product(torch::Tensor out, torch::Tensor x, c10::optional<torch::Tenso
   launch_lora_finish(ptr<__hip_bfloat16>(out), parts ? nullptr : cptr<__hip_bfloat16>(base),
                      parts ? part.data_ptr<float>() : nullptr, tmp.data_ptr<float>(),
                      cptr<__hip_bfloat16>(b), slots.data_ptr<int>(), scales.data_ptr<float>(),
-                     cols, T, R, PR, V, W, cuts, parts, gated, current_stream());
+                     cols, T, L, R, PR, V, W, cuts, parts, gated, current_stream());
 }
 
 // A captured step's static buffers from a packed pinned host buffer (decode_inputs.hip) of n rows

@@ -19,7 +19,7 @@
 // Layers of 4096 wide rows, 61 tokens of 4 adapters of rank 16: 7 + 7 launches of 25 and
 // 5 us were 4 + 4 of 4.6 and 4.0 to 7.8; of these the shrinks go beside their products now
 // (gemm_ring_lora), a pass of 604 us is one of 548.  2048 tokens: shrink 23 us, expand into 4096 columns 14
-// and into 28672 102, where reading and writing out takes 51.
+// and into 28672 102 (by the matrix unit some 75), where reading and writing out takes 51.
 //
 // f32 and f16: one token per workgroup in both,
 //   shrink: 4 waves split K; each (wave, r) pair accumulates a partial dot,
@@ -141,6 +141,8 @@ void launch_lora_expand(T* out, const float* tmp, const T* b_stack,
 struct LoraCols {
   int end[3], shift[3];
 };
+
+bool lora_tiles_win(int T, int L, int R, int W);
 
 namespace {
 
@@ -427,12 +429,229 @@ __global__ __launch_bounds__(256) void lora_finish_kernel(
   }
 }
 
+// The same by the matrix unit, 16 tokens of one adapter (or of none) at a time: products of B's
+// rows, which are bf16, and the tokens' f32 sums of the shrink in three terms of eight bits, which
+// are all 24 of them, with sums in f32.  Bound by the reads and writes of the product; a wave takes
+// 32 columns at a time, its lanes eight neighbours of a token each.  us with the shrink, a column a
+// thread | here: 1464 x 28672 rank 64 with the gate 971 | 140, 948 x 28672 rank 64 in place 314 | 69,
+// 868 x 28672 rank 32 119 | 50, 1582 x 28672 rank 8 107 | 63, 359 x 2048 rank 64 21.9 | 15.5, 107 x 4096
+// rank 64 15.8 | 13.6.
+// grid (ceil(columns of out / (128 chunks)), windows x groups_of(kWindow, L + 1))
+template <int R, bool GATE>
+__global__ __launch_bounds__(256) void lora_finish_tile_kernel(
+    __hip_bfloat16* out,                         // [T, GATE ? W / 2 : W]
+    const __hip_bfloat16* base,                  // [T, W] (parts == 0); may be out
+    const float* __restrict__ part,              // [parts, T, W]
+    const float* __restrict__ tmp,               // [cuts, T, PR]
+    const __hip_bfloat16* __restrict__ b_stack,  // [L, V, R]
+    const int* __restrict__ slots, const float* __restrict__ scales, const LoraCols cols,
+    const int T, const int L, const int PR, const int V, const int W, const int cuts,
+    const int parts, const int chunks) {
+  using lora::bf16x8_t;
+  using lora::f32x4_t;
+  constexpr int H = GATE ? 2 : 1, KS = (R + 31) / 32, PAD = 3 * R + 4, WINDOW = lora::kWindow;
+  __shared__ __align__(16) float sums[16][PAD];
+  __shared__ int groups[4][16];
+  const int OW = W / H;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, quad = lane >> 4;
+  const int per = lora::groups_of(WINDOW, L + 1), t0 = blockIdx.y / per * WINDOW;
+
+  // the group: as in the shrink, but that -1 is an adapter too
+  int first = blockIdx.y % per, slot, slot_of[WINDOW / 64];
+#pragma unroll
+  for (int i = 0; i < WINDOW / 64; ++i)
+    slot_of[i] = t0 + i * 64 + lane < T ? max(slots[t0 + i * 64 + lane], -1) : -2;
+  for (slot = -1; slot < L; ++slot) {
+    int n = 15;
+#pragma unroll
+    for (int i = 0; i < WINDOW / 64; ++i) n += __popcll(__ballot(slot_of[i] == slot));
+    if (first < n / 16) break;
+    first -= n / 16;
+  }
+  if (slot == L) return;
+  first *= 16;
+  int* group = groups[wave];
+  int found = 0;
+#pragma unroll
+  for (int i = 0; i < WINDOW / 64; ++i) {
+    const unsigned long long has = __ballot(slot_of[i] == slot);
+    const int at = found + __popcll(has & ((1ull << lane) - 1)) - first;
+    if (slot_of[i] == slot && at >= 0 && at < 16) group[at] = t0 + i * 64 + lane;
+    found += __popcll(has);
+  }
+  const int tokens = min(found - first, 16);
+  // other lanes of this wave read it: LDS keeps a wave's order, the compiler has to
+  asm volatile("" ::: "memory");
+  const int own = group[min(col, tokens - 1)];
+
+  // projections with columns among [c, c + n)
+  auto meets = [&](int p, int c, int n) {
+    const int v0 = p > 0 ? cols.end[p - 1] : 0;
+    return v0 < cols.end[p] && c < cols.end[p] + cols.shift[p] && c + n > v0 + cols.shift[p];
+  };
+  const int c_wg = blockIdx.x * chunks * 128;
+  int lo = 3, hi = -1;
+  if (slot >= 0)
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+      if (meets(p, c_wg, min(chunks * 128, OW - c_wg)) ||
+          (GATE && meets(p, c_wg + OW, min(chunks * 128, OW - c_wg)))) {
+        lo = min(lo, p);
+        hi = max(hi, p);
+      }
+  if (base == out && hi < 0) return;
+
+  float sum[H][8];
+  auto load = [&](int c) {
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      const long at = (long)own * W + c + h * OW + quad * 8;
+      if (parts == 0) {
+        const Vec16<__hip_bfloat16> v = load16(base + at);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sum[h][i] = __bfloat162float(v.data[i]);
+        continue;
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) sum[h][i] = 0.f;
+      for (int p0 = 0; p0 < parts; p0 += 4) {
+        f32x4_t v[4][2];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+          const f32x4_t* from = reinterpret_cast<const f32x4_t*>(
+              part + (long)min(p0 + p, parts - 1) * T * W + at);
+          v[p][0] = from[0];
+          v[p][1] = from[1];
+        }
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+          if (p0 + p < parts)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) sum[h][i] += v[p][i / 4][i % 4];
+      }
+    }
+  };
+  float scale = 0.f;
+  if (hi >= 0) {
+    scale = scales[slot];
+    // the shrink's sums of the tokens: of the projections that are met
+    const int width = (hi - lo + 1) * R;
+    for (int i = threadIdx.x; i < 16 * width; i += 256) {
+      const int m = i / width, r = lo * R + i % width;
+      const float* from = tmp + (long)group[min(m, tokens - 1)] * PR + r;
+      float s = 0.f;
+      for (int q0 = 0; q0 < cuts; q0 += 4) {
+        float v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = from[(long)min(q0 + q, cuts - 1) * T * PR];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (q0 + q < cuts) s += v[q];
+      }
+      sums[m][r] = s;
+    }
+    __syncthreads();
+  }
+
+  for (int u = 0; u < chunks; ++u) {
+    const int c = c_wg + u * 128 + wave * 32;
+    if (c >= OW) break;
+    load(c);
+    if (hi >= 0) {
+      for (int p = lo; p <= hi; ++p) {
+        const int v0 = p > 0 ? cols.end[p - 1] : 0;
+        bf16x8_t x[KS][3];
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          union { unsigned short u[8]; bf16x8_t v; } o[3];
+          const int r = ks * 32 + quad * 8;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            float f = r < R ? sums[col][p * R + r + i] : 0.f;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {   // cut off, not rounded: infinity stays the first term
+              const unsigned bits = __float_as_uint(f);
+              o[k].u[i] = bits >> 16;
+              f = (bits & 0x7fffffff) == 0x7f800000 ? 0.f
+                                                     : f - __uint_as_float(bits & 0xffff0000);
+            }
+          }
+#pragma unroll
+          for (int k = 0; k < 3; ++k) x[ks][k] = o[k].v;
+        }
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+          if (!meets(p, c + h * OW, 32)) continue;
+          f32x4_t acc[2] = {f32x4_t{}, f32x4_t{}};
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            // a lane's sums are of eight neighbouring columns
+            const int v = c + h * OW + col / 4 * 8 + j * 4 + col % 4 - cols.shift[p];
+            const bool in = v >= v0 && v < cols.end[p];
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+              bf16x8_t w = bf16x8_t{};
+              if (in && ks * 32 + quad * 8 < R)
+                w = *reinterpret_cast<const bf16x8_t*>(b_stack + ((long)slot * V + v) * R +
+                                                       ks * 32 + quad * 8);
+#pragma unroll
+              for (int k = 2; k >= 0; --k)
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x[ks][k], acc[j], 0, 0, 0);
+            }
+          }
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {   // (an infinite sum is no zero beside the projection)
+            const int v = c + h * OW + quad * 8 + i - cols.shift[p];
+            if (v >= v0 && v < cols.end[p]) sum[h][i] += acc[i / 4][i % 4] * scale;
+          }
+        }
+      }
+    }
+    if (col >= tokens) continue;
+    union { __hip_bfloat16 h[8]; uint4 u; } o;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float y = sum[0][i];
+      if constexpr (GATE) y = y / (1.f + __expf(-y)) * sum[H - 1][i];
+      o.h[i] = __float2bfloat16(y);
+    }
+    *reinterpret_cast<uint4*>(out + (long)own * OW + c + quad * 8) = o.u;
+  }
+}
+
+// Groups of 16 tokens that T tokens of L adapters, and some of none, leave at most
+long finish_groups(int T, int L) {
+  return T / lora::kWindow * (long)lora::groups_of(lora::kWindow, L + 1) +
+         lora::groups_of(T % lora::kWindow, L + 1);
+}
+
+template <int R, bool GATE>
+void launch_finish_tiles(__hip_bfloat16* out, const __hip_bfloat16* base, const float* part,
+                         const float* tmp, const __hip_bfloat16* b, const int* slots,
+                         const float* scales, const LoraCols& cols, int T, int L, int PR, int V,
+                         int W, int cuts, int parts, hipStream_t stream) {
+  const int OW = GATE ? W / 2 : W;
+  const long groups = finish_groups(T, L), all = (OW + 127L) / 128 * groups;
+  const int chunks = all > 8192 ? 4 : all > 4096 ? 2 : 1;   // of 128 columns, a workgroup
+  hipLaunchKernelGGL((lora_finish_tile_kernel<R, GATE>),
+                     dim3((OW + 128 * chunks - 1) / (128 * chunks), groups), dim3(256), 0, stream,
+                     out, base, part, tmp, b, slots, scales, cols, T, L, PR, V, W, cuts, parts,
+                     chunks);
+}
+
 template <int R, bool GATE>
 void launch_finish(__hip_bfloat16* out, const __hip_bfloat16* base, const float* part,
                    const float* tmp, const __hip_bfloat16* b, const int* slots,
-                   const float* scales, const LoraCols& cols, int T, int PR, int V, int W,
+                   const float* scales, const LoraCols& cols, int T, int L, int PR, int V, int W,
                    int cuts, int parts, hipStream_t stream) {
   const int OW = GATE ? W / 2 : W;
+  if (lora_tiles_win(T, L, R, W) && OW % 32 == 0) {
+    launch_finish_tiles<R, GATE>(out, base, part, tmp, b, slots, scales, cols, T, L, PR, V, W, cuts,
+                                 parts, stream);
+    return;
+  }
   auto go = [&](auto kernel, int tokens) {
     hipLaunchKernelGGL(kernel, dim3((OW + 255) / 256, (T + tokens - 1) / tokens), dim3(256), 0,
                        stream, out, base, part, tmp, b, slots, scales, cols, T, PR, V, W, cuts,
@@ -475,6 +694,15 @@ void launch_lora_slots(int* slots, const int* token_ids, const int* ids, int n, 
                      token_ids, by_value, T);
 }
 
+// Whether deltas of T tokens into W columns are added by the matrix unit: where products are many
+// (below, the search for a group's tokens shows, us by column a thread | matrix unit: 61 x 28672 ranks 16
+// and 32 13.0 | 13.2, 21.2 | 15.1; 61 x 6144 32 and 64 10.9 | 11.9, 19.1 | 17.3; 200 x 4096 8 and 64
+// 9.2 | 9.2, 18.7 | 14.0; 9 x 4096 64 9.6 | 10.4) and groups of 16 are not mostly empty (32 adapters
+// of rank 8, 200 x 28672 23 | 35, 1000 x 4096 21.6 | 29.0).
+bool lora_tiles_win(int T, int L, int R, int W) {
+  return (long)T * W * R >= 28000000 && (long)T * R >= 80 * finish_groups(T, L);
+}
+
 // Workgroups K is cut over: enough for one a CU, four steps a wave at least (K 14336, rank
 // 16, 61 tokens: 29.5 us uncut, 6.1 in 8, 4.2 in 16; K 4096: 12.5, 3.7, 3.1, and as much
 // again in expand's sums; 2048 tokens: 23 us uncut and in 16).
@@ -510,12 +738,20 @@ void launch_lora_tiles(__hip_bfloat16* out, float* tmp, const __hip_bfloat16* x,
                        const float* scales, const LoraCols& cols, int T, int L, int R, int PR,
                        int V, int K, int out_w, int cuts, hipStream_t stream) {
   launch_lora_shrink_tiles(tmp, x, a, slots, T, L, PR, K, cuts, stream);
-#define EXPAND(RR) \
-  launch_expand<RR>(out, tmp, b, slots, scales, cols, T, PR, V, out_w, cuts, stream)
-  if (R == 8) EXPAND(8);
-  else if (R == 16) EXPAND(16);
-  else if (R == 32) EXPAND(32);
-  else EXPAND(64);
+  const bool tiles = lora_tiles_win(T, L, R, V) && out_w % 32 == 0 &&
+                     reinterpret_cast<uintptr_t>(out) % 16 == 0;
+#define EXPAND(RR)                                                                            \
+  if (tiles)                                                                                  \
+    launch_finish_tiles<RR, false>(out, out, nullptr, tmp, b, slots, scales, cols, T, L, PR,  \
+                                   V, out_w, cuts, 0, stream);                                \
+  else                                                                                        \
+    launch_expand<RR>(out, tmp, b, slots, scales, cols, T, PR, V, out_w, cuts, stream)
+  switch (R) {
+    case 8: EXPAND(8); break;
+    case 16: EXPAND(16); break;
+    case 32: EXPAND(32); break;
+    default: EXPAND(64);
+  }
 #undef EXPAND
 }
 
@@ -523,15 +759,15 @@ void launch_lora_tiles(__hip_bfloat16* out, float* tmp, const __hip_bfloat16* x,
 // gated: silu of the first half of the columns times the second
 void launch_lora_finish(__hip_bfloat16* out, const __hip_bfloat16* base, const float* part,
                         const float* tmp, const __hip_bfloat16* b, const int* slots,
-                        const float* scales, const LoraCols& cols, int T, int R, int PR, int V,
-                        int W, int cuts, int parts, bool gated, hipStream_t stream) {
+                        const float* scales, const LoraCols& cols, int T, int L, int R, int PR,
+                        int V, int W, int cuts, int parts, bool gated, hipStream_t stream) {
 #define FINISH(RR)                                                                             \
   if (R == RR && gated)                                                                        \
-    launch_finish<RR, true>(out, base, part, tmp, b, slots, scales, cols, T, PR, V, W, cuts,   \
-                            parts, stream);                                                    \
+    launch_finish<RR, true>(out, base, part, tmp, b, slots, scales, cols, T, L, PR, V, W,      \
+                            cuts, parts, stream);                                                    \
   else if (R == RR)                                                                            \
-    launch_finish<RR, false>(out, base, part, tmp, b, slots, scales, cols, T, PR, V, W, cuts,  \
-                             parts, stream)
+    launch_finish<RR, false>(out, base, part, tmp, b, slots, scales, cols, T, L, PR, V, W,     \
+                             cuts, parts, stream)
   FINISH(8);
   FINISH(16);
   FINISH(32);

@@ -105,3 +105,73 @@ def test_adapters_beside_the_product(t, adapters, k, rank, some):
             off[rows, lo:hi] += 2 ** -20 * scale * (x[rows].abs() @ aa.abs().t()) @ bb.abs().t()
     err = (out.double() - want).abs()
     assert (err <= 2 ** -8 * want.abs() + off + 1e-7).all(), err.max().item()
+
+
+# deltas by the matrix unit: spans off its 32 columns, columns without an adapter, ragged windows
+TILES = [(257, 64, 1792, [(3, 700), (701, 1792)], 5, 64), (1000, 128, 3584, [(0, 3584)], 1, 8),
+         (520, 64, 3392, [(1000, 1033), (1050, 2000), (2000, 3392)], 9, 16),
+         (450, 64, 4160, [(0, 2080), (2080, 4160)], 3, 16), (130, 2048, 7168, [(0, 7168)], 2, 32),
+         (900, 64, 2064, [(0, 2064)], 2, 16)]   # (half a tile of columns: a column a thread)
+
+
+@pytest.mark.parametrize(("t", "k", "width", "spans", "adapters", "rank"), TILES)
+@pytest.mark.parametrize("way", ["product", "gated", "in place"])
+def test_deltas_by_the_matrix_unit(t, k, width, spans, adapters, rank, way):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from vllm_tgis_adapter_amd.ops import _C
+
+    g = torch.Generator("cuda").manual_seed(t + rank)
+
+    def normal(*shape, by=1.0):
+        return (torch.randn(shape, generator=g, device="cuda") * by).bfloat16()
+
+    cols = sum(hi - lo for lo, hi in spans)
+    x, y = normal(t, k), normal(t, width)
+    a, b = normal(adapters, len(spans) * rank, k, by=k ** -0.5), normal(adapters, cols, rank)
+    # tokens 0 and 1, alone in rank 0: a sum past float32 and one just inside it
+    x[:2], a[:, :, 0] = 0, 0
+    x[0, 0], x[1, 0] = 3e38, 3e38
+    a[:, ::rank, 0] = 1.0625
+    a[0, ::rank, 0] = 16
+    slots = torch.randint(-1, adapters, (t,), generator=g, device="cuda").int()
+    slots[0], slots[1] = 0, adapters - 1
+    scales = torch.linspace(0.5, 1.0, adapters, device="cuda")
+    scales[0] = 0.5
+    if way == "in place":
+        out = y.clone()
+        _C.lora_delta(out, x, a, b, slots, scales, spans)
+    else:
+        out = torch.full((t, width // (1 + (way == "gated"))), float("nan"), device="cuda").bfloat16()
+        _C.lora_product(out, x, None, y, a, b, slots, scales, spans, way == "gated")
+
+    want = y.double()
+    off = torch.zeros_like(want)
+    for s in range(adapters):
+        rows, v = (slots == s).nonzero().view(-1), 0
+        for p, (lo, hi) in enumerate(spans):
+            aa, bb = a[s, p * rank:(p + 1) * rank].double(), b[s, v:v + hi - lo].double()
+            xr, scale = x[rows].double(), scales[s].double()
+            want[rows, lo:hi] += scale * (xr @ aa.t()) @ bb.t()
+            off[rows, lo:hi] += 2 ** -20 * scale * (xr.abs() @ aa.abs().t()) @ bb.abs().t()
+            v += hi - lo
+    # 16 * 3e38 is infinite in float32, whatever B makes of it
+    past = torch.zeros_like(want, dtype=torch.bool)
+    for lo, hi in spans:
+        past[0, lo:hi] = True
+        if adapters == 1:
+            past[1, lo:hi] = True
+    if way == "gated":
+        (gate, up), (og, ou) = want.chunk(2, 1), off.chunk(2, 1)
+        want = torch.nn.functional.silu(gate) * up
+        off = 1.1 * (og * (up.abs() + ou)) + ou * gate.abs() + 1e-5 * want.abs()
+        p0, p1 = past.chunk(2, 1)
+        past = p0 | p1
+        past[:2] = True   # (products of two sums of that size)
+        assert not out[2:].isnan().any()
+    else:
+        assert not out.isnan().any()
+        assert (out.double()[past] == float("inf") * want[past].sign()).all()
+    past |= want.abs() + off > 2.0 ** 127   # (rounded to what is infinite in bf16)
+    err = (out.double() - want).abs()
+    assert (err <= 2 ** -8 * want.abs() + off + 1e-7)[~past].all(), err[~past].max().item()
