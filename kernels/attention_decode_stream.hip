@@ -55,7 +55,8 @@ template <typename T> DEVINLINE T load_here(const T* at) {
   return __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
 
-template <int HD, typename CT>
+// CUT: npart > 1
+template <int HD, typename CT, bool CUT>
 __global__ __launch_bounds__(256, 2) void paged_decode_stream_kernel(
     __hip_bfloat16* __restrict__ out,       // [nseq, nheads, HD]
     float* __restrict__ part_acc,           // [nseq, nheads, npart, HD] (npart > 1)
@@ -80,12 +81,12 @@ __global__ __launch_bounds__(256, 2) void paged_decode_stream_kernel(
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int* table = block_tables + (long)seq * max_blocks;
 
-  // Where a launch is short, and a workgroup's first tile does not depend on the length, block ids
+  // Where a sequence is cut, and so the launch short, and a workgroup's first tile does not depend on the length, block ids
   // are asked for beside it (with the merge's loads, us: one sequence of 230 keys of 64 6.8 -> 6.5, of
   // 700 keys of 128 8.4 -> 8.0, of 8000 in e4m3 16.8 -> 15.1; 512 of 520, uncut, 183.3 -> 184.1).
   // Past the end of the sequence, but not of its table, they may be anything.
   const int most = max_blocks * block_size;
-  const bool early = npart > 1 && (part == 0 || most <= npart * (kMinTiles * kTile));
+  const bool early = CUT && (part == 0 || most <= npart * (kMinTiles * kTile));
   auto page_of = [&](int pos) { return block_shift >= 0 ? pos >> block_shift : pos / block_size; };
   const int pos0 = (part * kMinTiles + wave) * kTile + (lane & 31);
   int entry0 = 0;
@@ -342,9 +343,13 @@ void launch(__hip_bfloat16* out, float* part_acc, float* part_ml, const __hip_bf
             hipStream_t stream) {
   int shift = -1;
   if ((block_size & (block_size - 1)) == 0) shift = __builtin_ctz(block_size);
-  hipLaunchKernelGGL((paged_decode_stream_kernel<HD, CT>), dim3(nseq, kvh, npart), dim3(256), 0,
-                     stream, out, part_acc, part_ml, q, kc, vc, bt, sl, scale * kLog2e, nheads,
-                     kvh, nheads / kvh, block_size, shift, max_blocks);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(nseq, kvh, npart), dim3(256), 0, stream, out, part_acc, part_ml,
+                       q, kc, vc, bt, sl, scale * kLog2e, nheads, kvh, nheads / kvh, block_size,
+                       shift, max_blocks);
+  };
+  if (npart > 1) go(paged_decode_stream_kernel<HD, CT, true>);
+  else go(paged_decode_stream_kernel<HD, CT, false>);
   if (npart > 1)
     hipLaunchKernelGGL((decode_stream_merge_kernel<HD>), dim3(nseq, nheads), dim3(HD), 0, stream,
                        out, part_acc, part_ml, sl, nheads, npart);
