@@ -3,69 +3,62 @@
 // bf16 loads cost ~2x), sum-of-squares in f32, one pass read + one pass write.
 //
 // Of a step's rows what counts is the chain of latencies.  Rows of up to 8192 (f32: 4096)
-// stay in registers, CHUNKS vectors a thread, the weight is asked for with the row, and the
-// waves' sums meet once: 61 rows of 4096 4.3 -> 3.7 us, 8192 rows 44.5 -> 42.8 (they were read
-// again after the sum, which waited for the store and then for a cold weight).
+// stay in registers, a vector a thread, the weight is asked for with the row, and the waves'
+// sums meet once, which no store is waited for at: us at 256 threads, the sum stored first |
+// here: 1 row of 4096 2.4 | 2.0, 61 3.3 | 2.8, 1000 9.9 | 9.1, 8192 50.7 | 49.1; 64 of 8192 4.6 | 3.4.
+// (Rows read again after the sum, which waited for a cold weight: 61 of 4096 4.3 where 3.7.)
 
 #include "common.h"
 
 namespace {
 
-constexpr int kThreads = 256;
-
-// the workgroup's sum, in one meeting
+// the workgroup's sum, in one meeting of its WAVES
+template <int WAVES>
 DEVINLINE float sum_of_waves(float x, float* lds) {
   x = wave_reduce_sum(x);
   if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = x;
   __syncthreads();
-  return (lds[0] + lds[1]) + (lds[2] + lds[3]);
+  float sum = 0.f;
+#pragma unroll
+  for (int w = 0; w < WAVES; w += 4) sum += (lds[w] + lds[w + 1]) + (lds[w + 2] + lds[w + 3]);
+  return sum;
 }
 
 // x <- rmsnorm(x + residual) w, residual <- x + residual, or (ADD false) out <- rmsnorm(x) w;
-// hidden is a multiple of a vector and at most CHUNKS of them a thread
-template <typename T, int CHUNKS, bool ADD>
-__global__ __launch_bounds__(kThreads) void rms_norm_row_kernel(
+// hidden is a multiple of a vector and at most one of them a thread
+template <typename T, int THREADS, bool ADD>
+__global__ __launch_bounds__(THREADS) void rms_norm_row_kernel(
     T* out, const T* x, T* residual, const T* __restrict__ weight, const float eps,
     const int hidden) {
   constexpr int V = Vec16<T>::kElems;
-  const long row = (long)blockIdx.x * hidden;
-  Vec16<T> v[CHUNKS], r[CHUNKS], w[CHUNKS];
-#pragma unroll
-  for (int c = 0; c < CHUNKS; ++c) {
-    const int i = (c * kThreads + threadIdx.x) * V;
-    if (i >= hidden) continue;
-    v[c] = load16(x + row + i);
-    if (ADD) r[c] = load16(residual + row + i);
-    w[c] = load16(weight + i);
-  }
+  const int i = threadIdx.x * V;
+  const long at = (long)blockIdx.x * hidden + i;
+  const bool in = i < hidden;
+  Vec16<T> v, r, w;
   float ss = 0.f;
-#pragma unroll
-  for (int c = 0; c < CHUNKS; ++c) {
-    const int i = (c * kThreads + threadIdx.x) * V;
-    if (i >= hidden) continue;
+  if (in) {
+    v = load16(x + at);
+    if (ADD) r = load16(residual + at);
+    w = load16(weight + i);
 #pragma unroll
     for (int j = 0; j < V; ++j) {
       // the norm is of the rounded sum, which is what is stored
       if (ADD)
-        v[c].data[j] = ScalarOps<T>::from_f32(ScalarOps<T>::to_f32(v[c].data[j]) +
-                                              ScalarOps<T>::to_f32(r[c].data[j]));
-      const float s = ScalarOps<T>::to_f32(v[c].data[j]);
+        v.data[j] = ScalarOps<T>::from_f32(ScalarOps<T>::to_f32(v.data[j]) +
+                                           ScalarOps<T>::to_f32(r.data[j]));
+      const float s = ScalarOps<T>::to_f32(v.data[j]);
       ss += s * s;
     }
-    if (ADD) store16(residual + row + i, v[c]);
   }
-  __shared__ float lds[kThreads / 64];
-  const float inv = rsqrtf(sum_of_waves(ss, lds) / hidden + eps);
+  __shared__ float lds[THREADS / 64];
+  const float inv = rsqrtf(sum_of_waves<THREADS / 64>(ss, lds) / hidden + eps);
+  if (!in) return;
+  if (ADD) store16(residual + at, v);   // (the meeting would wait for it)
 #pragma unroll
-  for (int c = 0; c < CHUNKS; ++c) {
-    const int i = (c * kThreads + threadIdx.x) * V;
-    if (i >= hidden) continue;
-#pragma unroll
-    for (int j = 0; j < V; ++j)
-      v[c].data[j] = ScalarOps<T>::from_f32(ScalarOps<T>::to_f32(v[c].data[j]) * inv *
-                                            ScalarOps<T>::to_f32(w[c].data[j]));
-    store16(out + row + i, v[c]);
-  }
+  for (int j = 0; j < V; ++j)
+    v.data[j] = ScalarOps<T>::from_f32(ScalarOps<T>::to_f32(v.data[j]) * inv *
+                                       ScalarOps<T>::to_f32(w.data[j]));
+  store16(out + at, v);
 }
 
 template <typename T, bool ADD>
@@ -73,15 +66,14 @@ bool launch_row(T* out, const T* x, T* residual, const T* w, float eps, int rows
                 hipStream_t stream) {
   constexpr int V = Vec16<T>::kElems;
   if (hidden % V != 0) return false;
-  auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(rows), dim3(kThreads), 0, stream, out, x, residual, w, eps,
+  auto go = [&](auto kernel, int threads) {
+    hipLaunchKernelGGL(kernel, dim3(rows), dim3(threads), 0, stream, out, x, residual, w, eps,
                        hidden);
     return true;
   };
-  const int chunks = (hidden / V + kThreads - 1) / kThreads;
-  if (chunks <= 1) return go(rms_norm_row_kernel<T, 1, ADD>);
-  if (chunks <= 2) return go(rms_norm_row_kernel<T, 2, ADD>);
-  if (chunks <= 4) return go(rms_norm_row_kernel<T, 4, ADD>);
+  if (hidden <= 256 * V) return go(rms_norm_row_kernel<T, 256, ADD>, 256);
+  if (hidden <= 512 * V) return go(rms_norm_row_kernel<T, 512, ADD>, 512);
+  if (hidden <= 1024 * V) return go(rms_norm_row_kernel<T, 1024, ADD>, 1024);
   return false;
 }
 
