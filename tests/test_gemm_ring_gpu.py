@@ -94,6 +94,11 @@ def test_results_at_any_address(entry):
     _check(got[1:].view(130, 384), x, w, False)
 
 
+@pytest.mark.parametrize("parts", [4, 6, 7])
+def test_counts_of_parts_that_are_added_at_once(parts):
+    test_parts(4, parts, 64 * parts)
+
+
 def test_plans_that_are_none():
     from vllm_tgis_adapter_amd.ops import _C
 
