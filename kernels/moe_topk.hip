@@ -11,14 +11,33 @@
 
 namespace {
 
-constexpr int kTokens = 4;        // tokens of a workgroup
 constexpr int kMaxExperts = 64;
 constexpr int kMaxTop = 8;
+
+// Eight values of every lane summed over the wave, each in the order of wave_reduce_sum: at every
+// step half of them go to half of the lanes, 10 exchanges instead of 48.  Lane l has value l / 8.
+DEVINLINE float sums_of_wave(float (&v)[8]) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int s = 0; s < 3; ++s) {
+    const int half = 4 >> s, mask = 32 >> s;
+    const bool up = lane & mask;
+#pragma unroll
+    for (int i = 0; i < half; ++i) {
+      const float send = up ? v[i] : v[i + half], keep = up ? v[i + half] : v[i];
+      v[i] = keep + __shfl_xor(send, mask, 64);
+    }
+  }
+#pragma unroll
+  for (int mask = 4; mask >= 1; mask >>= 1) v[0] += __shfl_xor(v[0], mask, 64);
+  return v[0];
+}
 
 // ids, weights [T, top]: the top largest x[t]·gate[e] and their softmax among themselves.
 // The four waves cut K; a workgroup's tokens share what it reads of the gate matrix.
 // Bound by the latency of a few dependent loads at decode sizes, by x and the gate
 // matrix from L2 at prompt sizes.
+template <int kTokens>   // of a workgroup
 __global__ __launch_bounds__(256) void moe_topk_kernel(
     int* __restrict__ ids, float* __restrict__ weights,
     const __hip_bfloat16* __restrict__ x,     // [T, K]
@@ -32,11 +51,9 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(
   const int per = ((K / 8 + 3) / 4) * 8;      // inputs of a wave, in runs of 8
   const int lo = wave * per, hi = min(lo + per, K);
   for (int e0 = 0; e0 < E; e0 += 8) {
-    float acc[kTokens][8];
+    float acc[kTokens * 8];
 #pragma unroll
-    for (int t = 0; t < kTokens; ++t)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) acc[t][e] = 0.f;
+    for (int i = 0; i < kTokens * 8; ++i) acc[i] = 0.f;
     for (int k = lo + lane * 8; k < hi; k += 512) {
       Vec16<__hip_bfloat16> xv[kTokens], gv[8];
 #pragma unroll
@@ -52,17 +69,20 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(
         for (int e = 0; e < 8; ++e) {
           const float g = __bfloat162float(gv[e].data[j]);
 #pragma unroll
-          for (int t = 0; t < kTokens; ++t) acc[t][e] = __builtin_fmaf(xf[t], g, acc[t][e]);
+          for (int t = 0; t < kTokens; ++t) acc[t * 8 + e] = __builtin_fmaf(xf[t], g, acc[t * 8 + e]);
         }
       }
     }
+    if constexpr (kTokens == 1) {
+      const float v = sums_of_wave(acc);
+      if (lane % 8 == 0) part[wave][0][lane / 8] = v;
+    } else {
 #pragma unroll
-    for (int t = 0; t < kTokens; ++t)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float v = wave_reduce_sum(acc[t][e]);
-        if (lane == 0) part[wave][t][e] = v;
+      for (int i = 0; i < kTokens * 8; ++i) {
+        const float v = wave_reduce_sum(acc[i]);
+        if (lane == 0) part[wave][i / 8][i % 8] = v;
       }
+    }
     __syncthreads();
     if (threadIdx.x < kTokens * 8) {
       const int t = threadIdx.x / 8, e = threadIdx.x % 8;
@@ -193,8 +213,15 @@ int moe_topk_max_top() { return kMaxTop; }
 void launch_moe_topk(int* ids, float* weights, const __hip_bfloat16* x,
                      const __hip_bfloat16* gate, int T, int E, int K, int top,
                      hipStream_t stream) {
-  hipLaunchKernelGGL(moe_topk_kernel, dim3((T + kTokens - 1) / kTokens), dim3(256), 0, stream,
-                     ids, weights, x, gate, T, E, K, top);
+  auto go = [&](auto kernel, int tokens) {
+    hipLaunchKernelGGL(kernel, dim3((T + tokens - 1) / tokens), dim3(256), 0, stream, ids, weights,
+                       x, gate, T, E, K, top);
+  };
+  // A token a workgroup is the shorter chain, four read the gate matrix once.  us, four | one, 8 experts
+  // of 4096 inputs: 1 token 11.1 | 4.9, 33 11.3 | 5.2, 1024 11.9 | 7.7, 2048 12.8 | 11.1, 2949 14.2 | 14.4; 64
+  // of 2048: 33 95 | 46, 2000 104 | 78.  (Two: 33 tokens 7.6, 2949 14.2.)
+  if (T <= 2048) go(moe_topk_kernel<1>, 1);
+  else go(moe_topk_kernel<4>, 4);
 }
 
 void launch_moe_group(int* rows, int* pos, int* seg, const int* ids, int pairs, int E, int top,

@@ -202,3 +202,9 @@ def test_products_that_fill_whole_rounds(mode, experts, n, k, mean):
         err = (got[lo:hi].double() - s).abs()
         # one rounding to bf16; float32 sums of up to 2112 terms of size 1 / sqrt(k)
         assert (err <= 2 ** -8 * s.abs() + 1e-4).all(), (e, err.max().item())
+
+
+# a token a workgroup up to 2048 tokens, then four
+@pytest.mark.parametrize("tokens", [2048, 2049])
+def test_router_of_many_tokens(tokens):
+    test_router_grouping_and_sum(tokens, 9, 2, 1000)
