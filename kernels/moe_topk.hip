@@ -134,31 +134,17 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(
 
 // Pairs p = t * top + j grouped by expert: seg [E + 1], pos[p] the sorted row of a pair,
 // rows[pos[p]] = t.  One workgroup: a few thousand pairs are less than a second launch.
-// A wave counts and claims places for all its lanes of one expert at a time.
+// Counts and places are claimed in LDS, a pair a lane: a wave that did so for all its lanes of one
+// expert at a time took, with a round trip for each, us: 33 tokens, 2 of 8 experts 3.7 where 2.1, 2949
+// 15.0 (4.8), 8192 38 (10.6); 33 tokens, 8 of 64 11.8 (2.5), 1000 85 (6.7).
 __global__ __launch_bounds__(1024) void moe_group_kernel(
     int* __restrict__ rows, int* __restrict__ pos, int* __restrict__ seg,
     const int* __restrict__ ids, const int pairs, const int E, const int top) {
   __shared__ int count[kMaxExperts], next[kMaxExperts];
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x;
   for (int e = tid; e < E; e += 1024) count[e] = 0;
   __syncthreads();
-  auto for_each = [&](auto take) {
-    for (int base = 0; base < pairs; base += 1024) {
-      const int p = base + tid;
-      const int e = p < pairs ? ids[p] : -1;
-      unsigned long long left = __ballot(e >= 0);
-      while (left) {
-        const int lead = __builtin_ctzll(left);
-        const int which = __shfl(e, lead, 64);
-        const unsigned long long same = __ballot(e == which);
-        take(p, e == which, which, same, lead);
-        left &= ~same;
-      }
-    }
-  };
-  for_each([&](int, bool, int which, unsigned long long same, int lead) {
-    if (lane == lead) atomicAdd(&count[which], __popcll(same));
-  });
+  for (int p = tid; p < pairs; p += 1024) atomicAdd(&count[ids[p]], 1);
   __syncthreads();
   if (tid == 0) {
     int at = 0;
@@ -170,16 +156,11 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(
     seg[E] = at;
   }
   __syncthreads();
-  for_each([&](int p, bool mine, int which, unsigned long long same, int lead) {
-    int at = 0;
-    if (lane == lead) at = atomicAdd(&next[which], __popcll(same));
-    at = __shfl(at, lead, 64);
-    if (mine) {
-      const int row = at + __popcll(same & ((1ull << lane) - 1));
-      pos[p] = row;
-      rows[row] = p / top;
-    }
-  });
+  for (int p = tid; p < pairs; p += 1024) {
+    const int row = atomicAdd(&next[ids[p]], 1);
+    pos[p] = row;
+    rows[row] = p / top;
+  }
 }
 
 // out[t] = sum_j weights[t, j] ye[pos[t, j]], in f32, rounded once.  Bound by the bytes
