@@ -163,21 +163,32 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(
   }
 }
 
-// out[t] = sum_j weights[t, j] ye[pos[t, j]], in f32, rounded once.  Bound by the bytes
-// of ye and out.
-__global__ __launch_bounds__(256) void moe_sum_kernel(
+// out[t] = sum_j weights[t, j] ye[pos[t, j]], in f32, rounded once.  Bound by the bytes of ye and
+// out, few tokens by the chain from places to rows: eight results a thread, the rows of AHEAD pairs
+// asked for at once.  us, 256 threads and a pair after the other | here: 33 x 4096 of 2 2.3 | 1.9, 256
+// 3.6 | 2.9, 2949 14.4 | 14.4, 33 x 8192 3.5 | 2.3.  (Four of 8 pairs at once: 33 x 2048 3.0 | 3.2.)
+template <int AHEAD>
+__global__ __launch_bounds__(1024) void moe_sum_kernel(
     __hip_bfloat16* __restrict__ out,       // [T, H]
     const __hip_bfloat16* __restrict__ ye,  // [T * top, H]
     const int* __restrict__ pos, const float* __restrict__ weights, const int H,
     const int top) {
   const long t = blockIdx.x;
-  for (int h = threadIdx.x * 8; h < H; h += 2048) {
+  for (int h = threadIdx.x * 8; h < H; h += blockDim.x * 8) {
     float acc[8] = {};
-    for (int j = 0; j < top; ++j) {
-      const float w = weights[t * top + j];
-      const Vec16<__hip_bfloat16> v = load16(ye + (long)pos[t * top + j] * H + h);
+    for (int j0 = 0; j0 < top; j0 += AHEAD) {
+      Vec16<__hip_bfloat16> v[AHEAD];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) acc[i] = __builtin_fmaf(w, __bfloat162float(v.data[i]), acc[i]);
+      for (int j = 0; j < AHEAD; ++j)
+        v[j] = load16(ye + (long)pos[t * top + min(j0 + j, top - 1)] * H + h);
+#pragma unroll
+      for (int j = 0; j < AHEAD; ++j) {
+        if (j0 + j >= top) break;
+        const float w = weights[t * top + j0 + j];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          acc[i] = __builtin_fmaf(w, __bfloat162float(v[j].data[i]), acc[i]);
+      }
     }
     Vec16<__hip_bfloat16> o;
 #pragma unroll
@@ -213,6 +224,10 @@ void launch_moe_group(int* rows, int* pos, int* seg, const int* ids, int pairs, 
 
 void launch_moe_sum(__hip_bfloat16* out, const __hip_bfloat16* ye, const int* pos,
                     const float* weights, int T, int H, int top, hipStream_t stream) {
-  hipLaunchKernelGGL(moe_sum_kernel, dim3(T), dim3(256), 0, stream, out, ye, pos, weights, H,
-                     top);
+  const int threads = H >= 8192 ? 1024 : (H / 8 + 63) / 64 * 64;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(T), dim3(threads), 0, stream, out, ye, pos, weights, H, top);
+  };
+  if (top <= 2) go(moe_sum_kernel<2>);
+  else go(moe_sum_kernel<1>);
 }

@@ -208,3 +208,20 @@ def test_products_that_fill_whole_rounds(mode, experts, n, k, mean):
 @pytest.mark.parametrize("tokens", [2048, 2049])
 def test_router_of_many_tokens(tokens):
     test_router_grouping_and_sum(tokens, 9, 2, 1000)
+
+
+# results of the weighted sum: less than a wave's, a workgroup's, more
+@pytest.mark.parametrize("width", [8, 520, 8192, 8200])
+@pytest.mark.parametrize("top", [1, 2, 3])
+def test_sums_of_any_width(width, top):
+    from vllm_tgis_adapter_amd.ops import _C
+
+    g = torch.Generator("cuda").manual_seed(width)
+    ye = torch.randn((5 * top, width), generator=g, device="cuda").bfloat16()
+    pos = torch.randperm(5 * top, generator=g, device="cuda").int().view(5, top)
+    weights = torch.rand((5, top), generator=g, device="cuda")
+    out = torch.full((5, width), float("nan"), device="cuda").bfloat16()
+    _C.moe_sum(out, ye, pos, weights)
+    want = (weights.double()[..., None] * ye.double()[pos.long()]).sum(dim=1)
+    # one rounding to bf16 of a float32 sum of three
+    assert ((out.double() - want).abs() <= 2 ** -8 * want.abs() + 1e-6).all()
