@@ -33,9 +33,13 @@ using ring_gemm::f32x4_t;
 constexpr int kCus = 256;
 constexpr int kMostParts = 2 * kCus - 1;   // of all those tiles
 
+// A row's results are not to depend on its place among its expert's rows, which callers leave to
+// the order of atomics: where the line falls between the chunks of an expert's rows in one column
+// tile, the ones ahead of it are sums of the same parts too, made by one workgroup one after the other.
 struct Rounds {
   int whole;          // tiles of one workgroup each
-  int parts, depth;   // of the others: parts of K, steps of a part
+  int summed;         // tiles from here on are sums of parts
+  int parts, depth;   // of these: parts of K, steps of a part
 };
 
 // A step takes 0.95 us where a workgroup has the chip's caches to itself and 1.5 beside 255 others
@@ -44,22 +48,31 @@ struct Rounds {
 // 576 899 | 790; 16 experts, 6144 x 8192: 792 744 | 685.  432, whose last 176 tiles are left whole: 650 | 652.
 // (Equal shares of all steps instead, whatever tile they belong to: 384 610 | 560, but 432
 // 622 | 710: workgroups at different inputs find nothing of each other's in the caches.)
-DEVINLINE Rounds rounds_of(int tiles, int steps, bool parted) {
+// shared: tiles ahead of the line whose chunks are of the same expert and column tile as one behind it
+DEVINLINE Rounds rounds_of(int tiles, int steps, int shared) {
   const int rest = tiles % kCus;
-  Rounds best{tiles, 1, steps};
-  if (!parted || rest == 0) return best;
+  Rounds best{tiles, tiles, 1, steps};
+  if (rest == 0) return best;
   auto round = [](int blocks) { return blocks > 0 ? 0.95f + 0.55f / kCus * blocks : 0.f; };
   float least = steps * round(rest);
-  for (int parts = 2; parts <= 8 && parts * rest <= kMostParts && parts * 8 <= steps; ++parts) {
+  for (int parts = 2; parts <= 8 && parts * (rest + shared) <= kMostParts && parts * 8 <= steps;
+       ++parts) {
     const int depth = ((steps + parts - 1) / parts + 1) / 2 * 2, blocks = rest * parts;
     const float us =
         depth * (round(min(blocks, kCus)) + round(blocks - kCus)) + 8.f + blocks * 0.22f;
     if (us < least) {
       least = us;
-      best = Rounds{tiles - rest, parts, depth};
+      best = Rounds{tiles - rest, tiles - rest - shared, parts, depth};
     }
   }
   return best;
+}
+
+DEVINLINE Rounds rounds_of(const moe::Segments& segs, int chunk, int n_tiles, int tiles, int steps) {
+  const int line = tiles - tiles % kCus;
+  if (line == tiles) return rounds_of(tiles, steps, 0);
+  const moe::Tile at = moe::tile_of(segs, chunk, n_tiles, line);
+  return rounds_of(tiles, steps, (at.row0 - segs.off[at.expert]) / chunk);
 }
 
 // What a lane holds of a tile: row i * 16 + lane % 16 of its wave's, columns in eights
@@ -97,49 +110,57 @@ __global__ __launch_bounds__(256, OCC) void moe_ring_kernel(
 
   const int steps = K / ring_gemm::kDepth, n_tiles = N / COLS;
   const int tiles = moe::count_chunks(segs, BM) * n_tiles;
-  const Rounds rounds = rounds_of(tiles, steps, PARTED && part != nullptr);
+  Rounds rounds{tiles, tiles, 1, steps};
+  if (PARTED && part != nullptr) rounds = rounds_of(segs, BM, n_tiles, tiles, steps);
   const int per_xcd = (rounds.whole + 7) / 8, xcd = blockIdx.x % 8;
   const int slot = blockIdx.x / 8 - per_xcd;
-  int id = xcd * per_xcd + blockIdx.x / 8, piece = -1, first = 0, own = steps;
+  int id = xcd * per_xcd + blockIdx.x / 8, own = 0, end = 1;   // parts of K
   if (slot < 0) {
     if (id >= rounds.whole) return;
+    if (id >= rounds.summed) end = rounds.parts;
   } else {   // part by part, so that what is read at a time is of the same inputs
     if constexpr (!PARTED) return;
     const int rest = tiles - rounds.whole, per = (rest * rounds.parts + 7) / 8;
-    piece = xcd * per + slot;
+    const int piece = xcd * per + slot;
     if (slot >= per || piece >= rest * rounds.parts) return;
     id = rounds.whole + piece % rest;
-    first = piece / rest * rounds.depth;
-    own = min(rounds.depth, steps - first);
+    own = piece / rest;
+    end = own + 1;
   }
+  const bool summed = PARTED && id >= rounds.summed;
   const moe::Tile at = moe::tile_of(segs, BM, n_tiles, id);
-  const int n0 = at.n * COLS, k0 = first * ring_gemm::kDepth;
+  const int n0 = at.n * COLS;
   const unsigned row_bytes = K * 2;
   f32x4_t acc[R::kTM][R::kTN];
-  R::clear(acc);
-  R::run(acc, lds, reinterpret_cast<const char*>(x + k0),
-         reinterpret_cast<const char*>(w + ((long)at.expert * (GATED ? 2 : 1) * N + n0) * K + k0),
-         own * ring_gemm::kDepth,
-         // rows past the segment: its last one, whose results are not written
-         [&](int r) {
-           const int row = at.row0 + min(r, at.rows - 1);
-           return (segs.rows != nullptr ? segs.rows[row] : row) * row_bytes;
-         },
-         [&](int r) {   // a wave's output tiles of gates, then of the other half
-           const int wave = r / (R::kTN * 16), in = r % (R::kTN * 16);
-           const int half = in / (OUT * 16);
-           return (half * N + wave * (OUT * 16) + R::out_col(in % (OUT * 16))) * row_bytes;
-         });
-  if (!PARTED || piece < 0) {
-#pragma unroll
-    for (int i = 0; i < R::kTM; ++i) store<R, OUT, MODE>(y, at, N, n0, i, acc[i], limit);
-  } else {
-    f32x4_t* to = part + (long)piece * (BM * BN / 4) + threadIdx.x;
+  for (;;) {
+    const int first = own * rounds.depth, k0 = first * ring_gemm::kDepth;
+    R::clear(acc);
+    R::run(acc, lds, reinterpret_cast<const char*>(x + k0),
+           reinterpret_cast<const char*>(w + ((long)at.expert * (GATED ? 2 : 1) * N + n0) * K + k0),
+           (summed ? min(rounds.depth, steps - first) : steps) * ring_gemm::kDepth,
+           // rows past the segment: its last one, whose results are not written
+           [&](int r) {
+             const int row = at.row0 + min(r, at.rows - 1);
+             return (segs.rows != nullptr ? segs.rows[row] : row) * row_bytes;
+           },
+           [&](int r) {   // a wave's output tiles of gates, then of the other half
+             const int wave = r / (R::kTN * 16), in = r % (R::kTN * 16);
+             const int half = in / (OUT * 16);
+             return (half * N + wave * (OUT * 16) + R::out_col(in % (OUT * 16))) * row_bytes;
+           });
+    if (!summed) break;
+    f32x4_t* to = part +
+                  ((long)own * (tiles - rounds.summed) + id - rounds.summed) * (BM * BN / 4) +
+                  threadIdx.x;
 #pragma unroll
     for (int i = 0; i < R::kTM; ++i)
 #pragma unroll
       for (int j = 0; j < R::kTN; ++j) to[(i * R::kTN + j) * 256] = acc[i][j];
+    if (++own == end) return;
+    block_gemm::meet();   // all have read what LDS holds
   }
+#pragma unroll
+  for (int i = 0; i < R::kTM; ++i) store<R, OUT, MODE>(y, at, N, n0, i, acc[i], limit);
 }
 
 // The parts of a tile become its results.  Grid (any, sixteenths of half of a tile's rows)
@@ -150,10 +171,10 @@ __global__ __launch_bounds__(256) void moe_parts_kernel(
   using R = ring_gemm::Ring<BM, BN, 2, 2, 4>;
   const int n_tiles = N / BN, i = blockIdx.y;
   const int tiles = moe::count_chunks(segs, BM) * n_tiles;
-  const Rounds rounds = rounds_of(tiles, K / ring_gemm::kDepth, true);
-  const int rest = tiles - rounds.whole;
+  const Rounds rounds = rounds_of(segs, BM, n_tiles, tiles, K / ring_gemm::kDepth);
+  const int rest = tiles - rounds.summed;
   for (int own = blockIdx.x; own < rest; own += gridDim.x) {
-    const moe::Tile at = moe::tile_of(segs, BM, n_tiles, rounds.whole + own);
+    const moe::Tile at = moe::tile_of(segs, BM, n_tiles, rounds.summed + own);
     if (i * 16 >= at.rows) continue;   // (of the first half of its rows)
     f32x4_t acc[R::kTN];
 #pragma unroll

@@ -112,3 +112,27 @@ def test_last_rounds_in_parts(mode, counts, n, k):
 
     assert ops._C.moe_tile(sum(counts) // len(counts), len(counts), n, k, False) == 0
     test_tiles(mode, counts, n, k)
+
+
+# the line between whole tiles and those whose K is cut (in 6, 8, 4 and 2) falls between the chunks of
+# an expert's rows in one column tile: on the second of three, the fifth of six; and on the first
+@pytest.mark.parametrize(("mode", "counts", "n", "k"), [
+    ("plain", [700] * 9, 2560, 8192), ("relu2", [600] * 3 + [700] * 4 + [513], 2816, 8192),
+    ("plain", [500] * 2 + [900] * 5 + [1300], 2560, 8192), ("plain", [600] * 8, 4096, 14336),
+    ("plain", [400] * 9, 4096, 8192)])
+def test_a_rows_results_do_not_depend_on_its_place(mode, counts, n, k):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from vllm_tgis_adapter_amd import ops
+
+    assert ops._C.moe_tile(sum(counts) // len(counts), len(counts), n, k, False) == 0
+    g = torch.Generator("cuda").manual_seed(n + len(counts))
+    total = sum(counts)
+    seg = torch.tensor([0, *counts]).cumsum(0).int().cuda()
+    w = (torch.randn((len(counts), n, k), generator=g, device="cuda") / k ** 0.5).bfloat16()
+    x = torch.randn((total, k), generator=g, device="cuda").bfloat16()
+    order = torch.cat([lo + torch.randperm(m, generator=g, device="cuda")
+                       for lo, m in zip(seg.tolist(), counts)])
+    act = "relu2" if mode == "relu2" else None
+    first = ops.moe_gemm(x, w, seg, False, act=act)
+    assert torch.equal(ops.moe_gemm(x, w, seg, False, act=act, rows=order.int()), first[order])
