@@ -48,20 +48,22 @@ struct Rounds {
 // 576 899 | 790; 16 experts, 6144 x 8192: 792 744 | 685.  432, whose last 176 tiles are left whole: 650 | 652.
 // (Equal shares of all steps instead, whatever tile they belong to: 384 610 | 560, but 432
 // 622 | 710: workgroups at different inputs find nothing of each other's in the caches.)
+// Two launches decide alike, so the times are whole numbers, of 1 / 25600 us: there are ties (8192
+// inputs, 120 tiles).
 // shared: tiles ahead of the line whose chunks are of the same expert and column tile as one behind it
 DEVINLINE Rounds rounds_of(int tiles, int steps, int shared) {
   const int rest = tiles % kCus;
   Rounds best{tiles, tiles, 1, steps};
   if (rest == 0) return best;
-  auto round = [](int blocks) { return blocks > 0 ? 0.95f + 0.55f / kCus * blocks : 0.f; };
-  float least = steps * round(rest);
+  auto round = [](int blocks) { return blocks > 0 ? 24320L + 55 * blocks : 0; };   // a step of all
+  long least = steps * round(rest);
   for (int parts = 2; parts <= 8 && parts * (rest + shared) <= kMostParts && parts * 8 <= steps;
        ++parts) {
     const int depth = ((steps + parts - 1) / parts + 1) / 2 * 2, blocks = rest * parts;
-    const float us =
-        depth * (round(min(blocks, kCus)) + round(blocks - kCus)) + 8.f + blocks * 0.22f;
-    if (us < least) {
-      least = us;
+    const long time =
+        depth * (round(min(blocks, kCus)) + round(blocks - kCus)) + 204800 + blocks * 5632;
+    if (time < least) {
+      least = time;
       best = Rounds{tiles - rest, tiles - rest - shared, parts, depth};
     }
   }

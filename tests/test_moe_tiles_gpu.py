@@ -99,12 +99,13 @@ def test_results_at_any_address(module, mode, counts):
 
 
 # tiles of 256 x 256 behind whole rounds of 256 whose K is cut: 16 by 8 with one row in the last,
-# 32, 128 by 2 with an odd last part, one alone; 144 and none stay whole
+# 32, 128 by 2 with an odd last part, one alone; 144 and none stay whole, and 120, as long in two parts
 @pytest.mark.parametrize(("mode", "counts", "n", "k"), [
     ("plain", [400] * 7 + [513], 4096, 8192), ("relu2", [400] * 7 + [513], 4096, 8256),
     ("plain", [256] * 16 + [257], 4096, 8192), ("plain", [600] * 8, 4096, 8256),
     ("relu2", [600, 0] + [700] * 7, 4096, 8320), ("plain", [256] * 257, 256, 8192),
-    ("plain", [600] * 7 + [769], 4096, 8192), ("plain", [400] * 8, 4096, 8192)])
+    ("plain", [600] * 7 + [769], 4096, 8192), ("plain", [400] * 8, 4096, 8192),
+    ("plain", [256] * 47, 2048, 8192)])
 def test_last_rounds_in_parts(mode, counts, n, k):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
