@@ -20,6 +20,8 @@
 // waves on 256 x 256) -> 1670 us (1.25 PFLOP/s; of the second product's 384 tiles, one and a half
 // rounds of 256 CUs, the last 128 have K cut in two; with 400, 144 are left, which stay whole).
 
+#include <algorithm>
+
 #include "gemm_stream.h"
 #include "ring_gemm.h"
 
@@ -51,7 +53,7 @@ struct Rounds {
 // Two launches decide alike, so the times are whole numbers, of 1 / 25600 us: there are ties (8192
 // inputs, 120 tiles).
 // shared: tiles ahead of the line whose chunks are of the same expert and column tile as one behind it
-DEVINLINE Rounds rounds_of(int tiles, int steps, int shared) {
+__host__ __device__ inline Rounds rounds_of(int tiles, int steps, int shared) {
   const int rest = tiles % kCus;
   Rounds best{tiles, tiles, 1, steps};
   if (rest == 0) return best;
@@ -61,7 +63,7 @@ DEVINLINE Rounds rounds_of(int tiles, int steps, int shared) {
        ++parts) {
     const int depth = ((steps + parts - 1) / parts + 1) / 2 * 2, blocks = rest * parts;
     const long time =
-        depth * (round(min(blocks, kCus)) + round(blocks - kCus)) + 204800 + blocks * 5632;
+        depth * (round(blocks < kCus ? blocks : kCus) + round(blocks - kCus)) + 204800 + blocks * 5632;
     if (time < least) {
       least = time;
       best = Rounds{tiles - rest, tiles - rest - shared, parts, depth};
@@ -96,7 +98,7 @@ DEVINLINE void store(__hip_bfloat16* y, const moe::Tile& at, int N, int n0, int 
   }
 }
 
-// part: null, or room for kMostParts tiles of f32
+// part: null, or room for the parts that moe_gemm_scratch counts
 template <int BM, int BN, int SLOTS, int OCC, int MODE>
 __global__ __launch_bounds__(256, OCC) void moe_ring_kernel(
     __hip_bfloat16* __restrict__ y,        // [T, N]
@@ -294,12 +296,23 @@ void launch_mode(__hip_bfloat16* y, const __hip_bfloat16* x, const __hip_bfloat1
 
 }  // namespace
 
-// Floats of scratch that launch_moe_gemm wants, 0: none.  From 8192 inputs on: below, parts save no
-// more than they cost (7168, 416 tiles 323 | 330 us) and the launch that finds nothing to add is 2 to 4 us.
+// Floats of scratch that launch_moe_gemm wants, 0: none, whatever the segments hold.  From 8192 inputs
+// on: below, parts save no more than they cost (7168, 416 tiles 323 | 330 us) and the launch that finds
+// nothing to add is 2 to 4 us.  The segments' chunks of rows, at most T / 256 and one an expert, are not
+// known here, so it is the most that any number of them wants: 8 experts of 14336 x 4096, 2949 tokens 87 MiB.
 long moe_gemm_scratch(int E, int N, int K, int T, int mode) {
-  const bool large =
-      mode != 1 && K >= 8192 && T / E > 52 && moe_tile(T / E, E, N, K, false) == 0;
-  return large ? (long)kMostParts * 256 * 256 : 0;
+  if (mode == 1 || K < 8192 || T / E <= 52 || moe_tile(T / E, E, N, K, false) != 0) return 0;
+  const int n_tiles = N / 256, most = T / 256 + std::min(T, E);
+  const int shared = (long)most * n_tiles > kCus ? (T + 255) / 256 - 1 : 0;
+  int pieces = 0;
+  for (int chunks = 1; chunks <= std::min(most, kCus); ++chunks) {   // (what is left of a round repeats)
+    const int rest = chunks * n_tiles % kCus;
+    const Rounds rounds = rounds_of(rest, K / ring_gemm::kDepth, 0);
+    // (chunks that share a line make no more parts of it)
+    if (rounds.parts > 1)
+      pieces = std::max(pieces, std::min(kMostParts, rounds.parts * (rest + shared)));
+  }
+  return pieces * (256L * 256);
 }
 
 void launch_moe_gemm(__hip_bfloat16* y, const __hip_bfloat16* x, const __hip_bfloat16* w,

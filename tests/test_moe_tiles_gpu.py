@@ -137,3 +137,22 @@ def test_a_rows_results_do_not_depend_on_its_place(mode, counts, n, k):
     act = "relu2" if mode == "relu2" else None
     first = ops.moe_gemm(x, w, seg, False, act=act)
     assert torch.equal(ops.moe_gemm(x, w, seg, False, act=act, rows=order.int()), first[order])
+
+
+# a whole round whatever the counts are; at most 6 chunks of rows by 32 tiles of columns, of which three
+# (96 tiles) in two parts are the most
+@pytest.mark.parametrize(("counts", "n", "parts"), [([300], 65536, 0), ([600, 600], 8192, 192)])
+def test_room_for_parts(counts, n, parts):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from vllm_tgis_adapter_amd import ops
+
+    assert ops._C.moe_tile(sum(counts) // len(counts), len(counts), n, 8192, False) == 0
+    w = torch.zeros((len(counts), n, 8192), device="cuda").bfloat16()
+    x = torch.zeros((sum(counts), 8192), device="cuda").bfloat16()
+    seg = torch.tensor([0, *counts]).cumsum(0).int().cuda()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    out = ops.moe_gemm(x, w, seg, False)
+    most = out.numel() * 2 + parts * 256 * 256 * 4
+    assert torch.cuda.max_memory_allocated() - before <= most + (1 << 20)
