@@ -65,6 +65,27 @@ def test_engine_quantized_generates(method):
     assert steps < 40
 
 
+def test_hooks_of_a_gate_and_up_layer_run(monkeypatch):
+    """The gate taken into the product goes past the layer's call, which hooks ask for."""
+    from vllm_tgis_adapter_amd.parallel.layers import MergedColumnParallelLinear, quantize_module_
+
+    layer = MergedColumnParallelLinear(128, [64, 64], dtype=torch.bfloat16)
+    quantize_module_(layer, 8)
+    x = torch.randn(70, 128).bfloat16()
+    made = torch.zeros(70, 64).bfloat16()
+    monkeypatch.setattr(ops, "gated_quant", lambda *a: made)
+    assert layer.gated(x) is made
+    seen = []
+    for hook in (layer.register_forward_hook(lambda m, i, o: seen.append(o.shape)),
+                 layer.register_forward_pre_hook(lambda m, i: seen.append(i[0].shape)),
+                 torch.nn.modules.module.register_module_forward_hook(
+                     lambda m, i, o: seen.append(o.shape))):
+        assert layer.gated(x) is not made and len(seen) == 1
+        hook.remove()
+        seen.clear()
+    assert layer.gated(x) is made
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("qbits", [8, 4])
 @pytest.mark.parametrize("m", [1, 16, 64])

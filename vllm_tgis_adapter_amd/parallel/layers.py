@@ -11,6 +11,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules import module as modules
 
 from .. import ops
 from . import divide, get_tp_rank, get_tp_world_size, tp_all_gather, tp_all_reduce
@@ -48,6 +49,12 @@ def lora_active() -> bool:
     if _lora_context is None:
         from ..engine.lora import CTX as _lora_context
     return _lora_context.active
+
+
+def _hooked(mod: nn.Module) -> bool:
+    """Whether calling a layer does more than its forward."""
+    return bool(mod._forward_hooks or mod._forward_pre_hooks
+                or modules._global_forward_hooks or modules._global_forward_pre_hooks)
 
 
 def _as_it_is(mod: nn.Module) -> torch.Tensor | None:
@@ -131,7 +138,7 @@ class MergedColumnParallelLinear(nn.Module):
                             lambda: _linear_fwd(self, x), gated=True)
             if h is not None:
                 return h
-        elif self.quant_bits is not None and self.bias is None:
+        elif self.quant_bits is not None and self.bias is None and not _hooked(self):
             h = ops.gated_quant(x, self.weight_q, self.weight_scale, self.quant_bits)
             if h is not None:
                 return h
