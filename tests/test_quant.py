@@ -76,11 +76,13 @@ def test_hooks_of_a_gate_and_up_layer_run(monkeypatch):
     monkeypatch.setattr(ops, "gated_quant", lambda *a: made)
     assert layer.gated(x) is made
     seen = []
-    for hook in (layer.register_forward_hook(lambda m, i, o: seen.append(o.shape)),
-                 layer.register_forward_pre_hook(lambda m, i: seen.append(i[0].shape)),
-                 torch.nn.modules.module.register_module_forward_hook(
-                     lambda m, i, o: seen.append(o.shape))):
-        assert layer.gated(x) is not made and len(seen) == 1
+    for register, hook in (
+            (layer.register_forward_hook, lambda m, i, o: seen.append(m)),
+            (layer.register_forward_pre_hook, lambda m, i: seen.append(m)),
+            (torch.nn.modules.module.register_module_forward_hook,
+             lambda m, i, o: seen.append(m))):
+        hook = register(hook)
+        assert layer.gated(x) is not made and seen == [layer]
         hook.remove()
         seen.clear()
     assert layer.gated(x) is made
