@@ -851,7 +851,7 @@ void moe_topk(torch::Tensor ids, torch::Tensor weights, torch::Tensor x, torch::
 }
 
 void moe_group(torch::Tensor rows, torch::Tensor pos, torch::Tensor seg, torch::Tensor ids) {
-  // ids hold experts 0 .. seg.numel() - 2 only
+  // pairs with ids other than experts 0 .. seg.numel() - 2 are left out
   const int pairs = ids.numel(), E = seg.numel() - 1;
   for (const auto& t : {rows, pos, seg, ids})
     TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::ScalarType::Int && t.is_contiguous());

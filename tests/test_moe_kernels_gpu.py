@@ -225,3 +225,23 @@ def test_sums_of_any_width(width, top):
     want = (weights.double()[..., None] * ye.double()[pos.long()]).sum(dim=1)
     # one rounding to bf16 of a float32 sum of three
     assert ((out.double() - want).abs() <= 2 ** -8 * want.abs() + 1e-6).all()
+
+
+@pytest.mark.parametrize(("tokens", "top", "experts"), [(3, 2, 1), (40, 2, 8), (700, 3, 64)])
+def test_pairs_without_an_expert(tokens, top, experts):
+    from vllm_tgis_adapter_amd.ops import _C
+
+    g = torch.Generator("cuda").manual_seed(tokens)
+    ids = torch.randint(-2, experts + 2, (tokens, top), generator=g, device="cuda").int()
+    rows, pos = torch.full((tokens * top,), -7).int().cuda(), torch.full_like(ids, -7)
+    seg = torch.empty(experts + 1, dtype=torch.int32, device="cuda")
+    _C.moe_group(rows, pos, seg, ids)
+    real = (ids >= 0) & (ids < experts)
+    count = torch.bincount(ids[real].long(), minlength=experts)
+    assert torch.equal(seg[1:].long(), count.cumsum(0)) and seg[0] == 0
+    at, e = pos[real].long(), ids[real].long()
+    assert (at >= seg[e]).all() and (at < seg[e + 1]).all()
+    assert torch.equal(at.sort().values, torch.arange(len(at), device="cuda"))
+    token = torch.arange(tokens, device="cuda")[:, None].expand(-1, top)
+    assert torch.equal(rows[at].long(), token[real])
+    assert (pos[~real] == -7).all() and (rows[len(at):] == -7).all()
