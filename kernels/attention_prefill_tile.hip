@@ -22,14 +22,16 @@
 //  - reads in batches: with transposed ones among them the compiler waits for all.
 //  - chunks of values turned so that sixteen lanes of a transposed read lie in different banks
 //    (2.7 -> 1.9 clocks a read of a full LDS).
-// Fewer waves, where a workgroup's are alone or two workgroups share a CU: products of the next
-// tile's scores between this one's exponentials.
+// Fewer waves, where a workgroup's are alone or two workgroups share a CU, and eight that find their
+// rows by the lanes, but in bf16 heads of 128: products of the next tile's scores between this
+// one's exponentials.
 //
 // Measured (MI355X, 32/8 heads of 128, keys and queries of variance 1, before -> after): 3500
 // tokens of 7 prompts after 700 each, bf16: 86 -> 74 us; one prompt of 8192 tokens 580 -> 522 us (1050
-// TFLOP/s; e4m3 605 -> 560), 3000 tokens 114 -> 100, 512 tokens after 5000 75 -> 67.  Turns alone, with
-// the lanes' addresses, were worth 1 %.  Left: ids of blocks that a wave's load does not fit
-// (under 4 to 8 rows), for which the lanes still work: 100 tokens after 200 by 2 %, 17 by 4.
+// TFLOP/s; e4m3 605 -> 555), 3000 tokens 114 -> 100, 512 tokens after 5000 75 -> 67.  Turns alone, with
+// the lanes' addresses, were worth 1 %.  Blocks that a wave's load does not fit (under 4 to 16 rows, or
+// no power of two) leave the addresses to the lanes: blocks of 24, 3000 tokens 120 -> 111, e4m3 121 ->
+// 120, 33 tokens 7.0 -> 7.1.
 // On the way here: eight waves of one head (256 tokens) leave early rows' waves idle; register
 // staging 630 us of 564; transposed reads as asm 584; results stored in 8 bytes a lane instead of
 // 16: 24 tokens 7.0 us instead of 6.2.
@@ -70,9 +72,11 @@ DEVINLINE s16x4_t read_transposed(lds_s16x4_t* __restrict__ at) {
 
 // 16-byte chunk c of row r of a tile lies at chunk c ^ swizzle(r).  Keys: the 16 rows of
 // equal chunks cover all banks.  Values: pairs of chunks stay pairs, the four rows of a
-// transposed read lie in different banks.
+// transposed read lie in different banks; PAIRS: two by two only, which is as good where rows found by
+// the lanes are widened on their way to LDS (4 prompts of 500 after 700, e4m3, blocks of 24: 76.1 | 73.0).
 template <int HD> DEVINLINE int k_swizzle(int r) { return HD == 128 ? r & 15 : (r >> 1) & 7; }
-template <int HD> DEVINLINE int v_swizzle(int r) {
+template <int HD, bool PAIRS> DEVINLINE int v_swizzle(int r) {
+  if (PAIRS) return HD == 128 ? (r & 7) * 2 : ((r >> 1) & 3) * 2;
   return HD == 128 ? (r & 3) * 4 : (r & 2) * 2;
 }
 
@@ -81,8 +85,25 @@ DEVINLINE int tiles_per_part(int tiles, int parts) {
   return max(kMinTiles, (tiles + parts - 1) / parts);
 }
 
-// Tiles of keys, and of values, that LDS holds
-constexpr int prefill_buffers(int waves) { return waves == 8 ? 3 : 2; }
+// Whether the two waves of a SIMD take turns: not where the lanes find their rows and little is won by
+// it (us, two tiles in LDS | in turns, blocks of 24: e4m3, 512 tokens after 5000 80 | 82, 4 prompts of
+// 500 after 700 76 | 79; heads of 64 21.4 | 22.6; bf16 heads of 128 76 | 72)
+template <int HD, typename CT, int NW, bool EVEN>
+constexpr bool kTurns = NW == 8 && (EVEN || (sizeof(CT) == 2 && HD == 128));
+
+// The LDS of a workgroup, an array of BYTES or, FROM_0, of the launch's size, which has the address 0: a
+// static array's is not known to be that, and is added to the lanes' (rows found by the lanes, us, static |
+// from 0: 33 tokens e4m3 8.2 | 7.8, 100 after 200 17.2 | 16.2, bf16 14.1 | 13.8; but in turns, where no
+// addresses are left, e4m3, 512 after 5000 70 | 71, 4 prompts of 500 after 700 66 | 67).
+template <int BYTES, bool FROM_0> DEVINLINE char* shared_bytes() {
+  if constexpr (FROM_0) {
+    extern __shared__ __align__(16) char given[];
+    return given;
+  } else {
+    __shared__ __align__(16) char own[BYTES];
+    return own;
+  }
+}
 
 // EVEN: cache blocks are a multiple of the rows of a wave's load (and a power of two), so that
 // these have one block
@@ -108,6 +129,7 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
   constexpr int PASS = kTile / RPP / NW;      // loads of a thread, keys or values
   constexpr int BYTES = kTile * HD * 2;
   static_assert(PASS * RPP * NW == kTile, "whole passes");
+  constexpr bool TURNS = kTurns<HD, CT, NW, EVEN>;
 
   const int seq = blockIdx.y;
   const int q_start = query_start_loc[seq];
@@ -138,8 +160,8 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
   const int wave_min = past + token0 - origin;
   const int wave_max = token0 < q_len ? past + min(token0 + 31, q_len - 1) - origin : -1;
 
-  constexpr int BUFS = prefill_buffers(NW);
-  __shared__ __align__(16) char lds_all[2 * BUFS * BYTES];   // tiles of keys, then of values
+  constexpr int BUFS = TURNS ? 3 : 2;
+  char* const lds_all = shared_bytes<2 * BUFS * BYTES, !TURNS>();   // tiles of keys, then of values
   char* const k_lds[2] = {lds_all, lds_all + BYTES};
   char* const v_lds[2] = {lds_all + BUFS * BYTES, lds_all + (BUFS + 1) * BYTES};
 
@@ -159,7 +181,7 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
   // the scalar unit: a lane by itself takes 500 of the vector unit's clocks a tile for them,
   // half as much as for its probabilities.
   struct Place {       // of a wave's load in the cache
-    long at;    // EVEN: where its first row begins; else: the lane's row
+    std::conditional_t<EVEN, long, int> at;   // where its first row begins; else: the lane's row
     int last;   // EVEN: rows past it are this one again
   };
   auto pos_of = [&](int ps, int t) {
@@ -182,7 +204,7 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
         places[ps] = Place{(((long)ids[ps] << block_shift) + in) * row_bytes, keys - 1 - pos};
       } else {
         int row = ids[ps] * block_size + in;
-        if constexpr (NW == 8) asm volatile("" : "+v"(row));
+        if constexpr (TURNS) asm volatile("" : "+v"(row));
         places[ps] = Place{row, 0};
       }
     }
@@ -223,7 +245,7 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
       }
   };
   auto k_swz = [](int r) { return k_swizzle<HD>(r); };
-  auto v_swz = [](int r) { return v_swizzle<HD>(r); };
+  auto v_swz = [](int r) { return v_swizzle<HD, FP8 && !EVEN>(r); };
   auto block_meet = [&] {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -248,8 +270,9 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
   // LDS addresses in the first tile of keys and of values; kept out of the compiler's sight,
   // which would rather compute them again than keep them (where there are registers for it)
   constexpr bool KEEP = !FP8 && NW == 8;
-  const unsigned lds_at = (unsigned)(__SIZE_TYPE__)(__attribute__((address_space(3))) char*)lds_all;
-  unsigned k_lane[KS], v_lane[DT];
+  unsigned k_lane[KS], v_lane[DT], lds_at = 0;
+  if constexpr (TURNS)
+    lds_at = (unsigned)(__SIZE_TYPE__)(__attribute__((address_space(3))) char*)lds_all;
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
     k_lane[ks] = lds_at + col * HD * 2 + ((ks * 2 + half) ^ k_swizzle<HD>(col)) * 16;
@@ -259,7 +282,7 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
   for (int dt = 0; dt < DT; ++dt) {
     const int i = lane & 15, side = lane >> 4 & 1, r = half * 4 + (i >> 2);
     v_lane[dt] = lds_at + BUFS * BYTES + r * HD * 2 +
-                 (((dt * 2 + side) * 2 + ((i & 3) >> 1)) ^ v_swizzle<HD>(r)) * 16 + (i & 1) * 8;
+                 (((dt * 2 + side) * 2 + ((i & 3) >> 1)) ^ v_swizzle<HD, FP8 && !EVEN>(r)) * 16 + (i & 1) * 8;
     if constexpr (KEEP) asm volatile("" : "+v"(v_lane[dt]));
   }
   auto key_frag = [&](int at, int g) {   // g: 32-key half g % 2, 16 dims g / 2
@@ -336,7 +359,7 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
 
   int ids[PASS];         // block ids of the tile after the next to be asked for
   Place places[PASS];    // of the values that are asked for next
-  if constexpr (NW == 8) {
+  if constexpr (TURNS) {
     // Two waves of a SIMD take turns: while one's probabilities are made, the other multiplies.
     // Both run the same program, waves 4 to 7 a barrier later: with barriers counted from the
     // first scores on, tile t's probabilities lie behind barrier 2 t + 1 (late: + 2), its values
@@ -471,14 +494,22 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
     auto step = [&](int t, f32x16_t (&now)[2], f32x16_t (&next)[2], int buf) {
       meet();
       const bool more_k = t + 2 < n, more_v = t + 1 < n;
-      Place ahead[PASS];
-      if (EVEN || more_k) places_of(ahead, ids, t + 2);
-      if (more_v) issue(v_at, places, v_lds[buf ^ 1], vr, v_swz);
-      if (more_k) issue(k_at, ahead, k_lds[buf], kr, k_swz);
-      if (EVEN || t + 3 < n) ids_of(ids, t + 3);
-      if (EVEN || more_k)
+      if constexpr (EVEN) {
+        Place ahead[PASS];
+        places_of(ahead, ids, t + 2);
+        if (more_v) issue(v_at, places, v_lds[buf ^ 1], vr, v_swz);
+        if (more_k) issue(k_at, ahead, k_lds[buf], kr, k_swz);
+        ids_of(ids, t + 3);
 #pragma unroll
         for (int ps = 0; ps < PASS; ++ps) places[ps] = ahead[ps];
+      } else {
+        if (more_v) issue(v_at, places, v_lds[buf ^ 1], vr, v_swz);
+        if (more_k) {
+          places_of(places, ids, t + 2);
+          issue(k_at, places, k_lds[buf], kr, k_swz);
+          if (t + 3 < n) ids_of(ids, t + 3);
+        }
+      }
       // wave-uniform: the matrix unit wants all lanes
       if (t * kTile <= wave_max) {
         Probs p[4];
@@ -651,20 +682,22 @@ void launch(__hip_bfloat16* out, float* part_acc, float* part_ml, const __hip_bf
             int max_query_len, const Cut& c, hipStream_t stream) {
   const int shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz(block_size) : -1;
   const int tiles = (max_query_len + c.tokens - 1) / c.tokens;
-  auto go = [&](auto kernel) {
+  auto go = [&](auto kernel, bool turns) {
     hipLaunchKernelGGL(kernel, dim3(nheads / c.heads, nseq, tiles * c.parts),
-                       dim3(c.waves * 64), 0, stream, out, q, kc, vc, bt, qsl,
+                       dim3(c.waves * 64), turns ? 0 : 4 * kTile * HD * 2, stream, out, q, kc, vc, bt, qsl,
                        sl, scale * kLog2e, nheads, kvh, c.heads, block_size, shift, max_blocks,
                        c.parts, part_acc, part_ml);
   };
   constexpr int kLoad = 1024 / (HD * sizeof(CT));   // rows of a wave's load
   const bool even = shift >= 0 && block_size % kLoad == 0 && (long)kvh * HD * sizeof(CT) < 1 << 24;
-  if (c.waves == 8 && even) go(paged_prefill_tile_kernel<HD, CT, 8, true>);
-  else if (c.waves == 8) go(paged_prefill_tile_kernel<HD, CT, 8, false>);
-  else if (c.waves == 4 && even) go(paged_prefill_tile_kernel<HD, CT, 4, true>);
-  else if (c.waves == 4) go(paged_prefill_tile_kernel<HD, CT, 4, false>);
-  else if (even) go(paged_prefill_tile_kernel<HD, CT, 2, true>);
-  else go(paged_prefill_tile_kernel<HD, CT, 2, false>);
+#define GO(NW, EVEN) go(paged_prefill_tile_kernel<HD, CT, NW, EVEN>, kTurns<HD, CT, NW, EVEN>)
+  if (c.waves == 8 && even) GO(8, true);
+  else if (c.waves == 8) GO(8, false);
+  else if (c.waves == 4 && even) GO(4, true);
+  else if (c.waves == 4) GO(4, false);
+  else if (even) GO(2, true);
+  else GO(2, false);
+#undef GO
   if (c.parts > 1)
     hipLaunchKernelGGL((prefill_tile_merge_kernel<HD>), dim3(max_query_len, nseq, (nheads + 3) / 4),
                        dim3(256), 0, stream, out, part_acc, part_ml, qsl, sl, nheads, c.tokens, c.parts);
