@@ -90,6 +90,7 @@ struct LoraCols {
   int end[3], shift[3];
 };
 int lora_shrink_cuts(int T, int K);
+bool lora_tiles_win(int T, int L, int R, int W);
 void launch_lora_shrink_tiles(float*, const __hip_bfloat16*, const __hip_bfloat16*, const int*,
                               int, int, int, int, int, hipStream_t);
 void launch_lora_finish(__hip_bfloat16*, const __hip_bfloat16*, const float*, const float*,
@@ -989,6 +990,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_ring_plan", &gemm_ring_plan, "which tile a product takes, and parts of K (form << 4 | parts)");
   m.def("decode_inputs", &decode_inputs, "a captured step's inputs from a packed host buffer");
   m.def("lora_product", &lora_product, "a product with its LoRA deltas, also gated");
+  m.def("lora_tiles_win", &lora_tiles_win, "whether its deltas are added by the matrix unit");
   m.def("lora_delta", &lora_delta,
         "bf16 multi-LoRA of up to three projections of one input");
   m.def("lora_slots", &lora_slots, "adapter slot of every token");

@@ -694,13 +694,16 @@ void launch_lora_slots(int* slots, const int* token_ids, const int* ids, int n, 
                      token_ids, by_value, T);
 }
 
-// Whether deltas of T tokens into W columns are added by the matrix unit: where products are many
-// (below, the search for a group's tokens shows, us by column a thread | matrix unit: 61 x 28672 ranks 16
-// and 32 13.0 | 13.2, 21.2 | 15.1; 61 x 6144 32 and 64 10.9 | 11.9, 19.1 | 17.3; 200 x 4096 8 and 64
-// 9.2 | 9.2, 18.7 | 14.0; 9 x 4096 64 9.6 | 10.4) and groups of 16 are not mostly empty (32 adapters
-// of rank 8, 200 x 28672 23 | 35, 1000 x 4096 21.6 | 29.0).
+// Whether deltas of T tokens into W columns are added by the matrix unit: where the products are more
+// than a launch's chain of loads, and than what every group that there may be, empty or not, takes for
+// its columns, which grows with the adapters that it looks through.  us, a column a thread | matrix unit:
+// 61 x 28672, 4 adapters of rank 16 13.0 | 13.2, 61 x 6144, 4 of 64 19.1 | 17.3, 436 x 2048, one of 32 8.5 |
+// 9.0, 872 x 4096, 5 of 8 12.6 | 13.5; 1069 x 2048, 32 of 64 in four runs 38.6 | 41.3; 60 of 32, 200 x 6144
+// 14.8 | 35.3, 599 x 2048 20.0 | 38.5; taken: 109 x 4096, 4 of 64 12.6 | 11.9, 458 x 28672, 60 of 64
+// 243 | 126.  Of 1205 sizes of 1 to 60 adapters none is slower by more than 3 %, and of what all would
+// gain 4 % is left.
 bool lora_tiles_win(int T, int L, int R, int W) {
-  return (long)T * W * R >= 28000000 && (long)T * R >= 80 * finish_groups(T, L);
+  return (long)T * W * R >= 28000000 + 7 * (L + 4) * finish_groups(T, L) * W;
 }
 
 // Workgroups K is cut over: enough for one a CU, four steps a wave at least (K 14336, rank

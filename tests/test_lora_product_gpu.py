@@ -108,10 +108,10 @@ def test_adapters_beside_the_product(t, adapters, k, rank, some):
 
 
 # deltas by the matrix unit: spans off its 32 columns, columns without an adapter, ragged windows
-TILES = [(257, 64, 1792, [(3, 700), (701, 1792)], 5, 64), (1000, 128, 3584, [(0, 3584)], 1, 8),
-         (520, 64, 3392, [(1000, 1033), (1050, 2000), (2000, 3392)], 9, 16),
-         (450, 64, 4160, [(0, 2080), (2080, 4160)], 3, 16), (130, 2048, 7168, [(0, 7168)], 2, 32),
-         (900, 64, 2064, [(0, 2064)], 2, 16)]   # (half a tile of columns: a column a thread)
+TILES = [(257, 64, 2048, [(3, 700), (701, 2043)], 5, 64), (1000, 128, 5792, [(0, 5792)], 1, 8),
+         (520, 64, 4800, [(1000, 1033), (1050, 2400), (2600, 4800)], 9, 32),
+         (450, 64, 5376, [(0, 2688), (2688, 5376)], 3, 16), (130, 2048, 8192, [(0, 8192)], 2, 32),
+         (900, 64, 2064, [(0, 2064)], 2, 32)]   # (half a tile of columns: a column a thread)
 
 
 @pytest.mark.parametrize(("t", "k", "width", "spans", "adapters", "rank"), TILES)
@@ -127,6 +127,7 @@ def test_deltas_by_the_matrix_unit(t, k, width, spans, adapters, rank, way):
         return (torch.randn(shape, generator=g, device="cuda") * by).bfloat16()
 
     cols = sum(hi - lo for lo, hi in spans)
+    assert _C.lora_tiles_win(t, adapters, rank, cols)   # (the gate of rank 64: a column a thread)
     x, y = normal(t, k), normal(t, width)
     a, b = normal(adapters, len(spans) * rank, k, by=k ** -0.5), normal(adapters, cols, rank)
     # tokens 0 and 1, alone in rank 0: a sum past float32 and one just inside it
@@ -175,3 +176,15 @@ def test_deltas_by_the_matrix_unit(t, k, width, spans, adapters, rank, way):
     past |= want.abs() + off > 2.0 ** 127   # (rounded to what is infinite in bf16)
     err = (out.double() - want).abs()
     assert (err <= 2 ** -8 * want.abs() + off + 1e-7)[~past].all(), err[~past].max().item()
+
+
+def test_many_adapters_of_few_tokens_take_a_column_a_thread():
+    """Groups of 16 tokens are mostly empty there, and each looks through all adapters."""
+    from vllm_tgis_adapter_amd.ops import _C
+
+    if _C is None:
+        pytest.skip("the extension is not built")
+    for t, adapters, rank, width in [(200, 60, 32, 6144), (599, 60, 32, 2048), (150, 60, 64, 4096),
+                                     (1197, 32, 16, 2048), (300, 32, 32, 4096), (291, 16, 16, 6144)]:
+        assert not _C.lora_tiles_win(t, adapters, rank, width)
+        assert _C.lora_tiles_win(t, 1, rank, 4 * width)
