@@ -433,9 +433,9 @@ __global__ __launch_bounds__(256) void lora_finish_kernel(
 // rows, which are bf16, and the tokens' f32 sums of the shrink in three terms of eight bits, which
 // are all 24 of them, with sums in f32.  Bound by the reads and writes of the product; a wave takes
 // 32 columns at a time, its lanes eight neighbours of a token each.  us with the shrink, a column a
-// thread | here: 1464 x 28672 rank 64 with the gate 971 | 140, 948 x 28672 rank 64 in place 314 | 69,
-// 868 x 28672 rank 32 119 | 50, 1582 x 28672 rank 8 107 | 63, 359 x 2048 rank 64 21.9 | 15.5, 107 x 4096
-// rank 64 15.8 | 13.6.
+// thread | here: 948 x 28672 rank 64 in place 314 | 69, 868 x 28672 rank 32 119 | 50, 1582 x 28672 rank 8
+// 107 | 63, 359 x 2048 rank 64 21.9 | 15.5, 107 x 4096 rank 64 15.8 | 13.6; with the gate 2048 x 28672 rank
+// 8 151 | 104, 1000 x 28672 rank 16 106 | 61.
 // grid (ceil(columns of out / (128 chunks)), windows x groups_of(kWindow, L + 1))
 template <int R, bool GATE>
 __global__ __launch_bounds__(256) void lora_finish_tile_kernel(
@@ -647,10 +647,13 @@ void launch_finish(__hip_bfloat16* out, const __hip_bfloat16* base, const float*
                    const float* scales, const LoraCols& cols, int T, int L, int PR, int V, int W,
                    int cuts, int parts, hipStream_t stream) {
   const int OW = GATE ? W / 2 : W;
-  if (lora_tiles_win(T, L, R, W) && OW % 32 == 0) {
-    launch_finish_tiles<R, GATE>(out, base, part, tmp, b, slots, scales, cols, T, L, PR, V, W, cuts,
-                                 parts, stream);
-    return;
+  // (with the gate rank 64 is asked for where products are few: engine/lora.py, _GATE_TILES)
+  if constexpr (!GATE || R < 64) {
+    if (lora_tiles_win(T, L, R, W) && OW % 32 == 0) {
+      launch_finish_tiles<R, GATE>(out, base, part, tmp, b, slots, scales, cols, T, L, PR, V, W,
+                                   cuts, parts, stream);
+      return;
+    }
   }
   auto go = [&](auto kernel, int tokens) {
     hipLaunchKernelGGL(kernel, dim3((OW + 255) / 256, (T + tokens - 1) / tokens), dim3(256), 0,

@@ -148,10 +148,11 @@ def _batched(x: torch.Tensor) -> bool:
 
 
 # Most tokens, times a layer's 256-column pieces, up to which the gate is taken in the launch that
-# adds the deltas, by rank (us there | deltas and gate apart; tokens x columns): rank 8, 1024 x
-# 16384 29 | 36, 2048 x 28672 82 | 93, 4096 x 28672 198 | 184; 16, 301 x 28672 18 | 19, 700 x 16384
-# 26 | 22; 32, 33 x 28672 8.1 | 8.6, 61 x 28672 12.9 | 12.2, 512 x 28672 77 | 53; 64, 16 x 16384 8.2 |
-# 9.0, 16 x 28672 14.8 | 11.5, 2048 x 28672 869 | 270.
+# adds the deltas, by rank (us there | deltas and gate apart; tokens x columns, 4 adapters): rank 8, 1024 x
+# 16384 41 | 43, 2048 x 28672 104 | 113, 4096 x 28672 198 | 217; 16, 301 x 28672 26.7 | 27.3, 700 x 16384
+# 36.0 | 36.2, 1000 x 28672 61.1 | 60.8; 32, 33 x 28672 13.9 | 15.3, 36 x 28672 15.1 | 16.3; past the line 61 x
+# 28672 15.3 | 16.0, 512 x 28672 42 | 41, 1024 x 28672 74 | 75; 64, 16 x 16384 15.1 | 15.9; past the line,
+# where the gate would be a column a thread, 16 x 28672 22.4 | 20.2, 512 x 28672 413 | 54.
 _GATE_TILES = {8: 131072, 16: 32768, 32: 4096, 64: 1024}
 
 
