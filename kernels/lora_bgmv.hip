@@ -28,6 +28,7 @@
 //           output column and walks r with the B row loads coalesced.
 
 #include "lora_shrink.h"
+#include <float.h>
 
 // ---------------------------------------------------------------------------
 // shrink: tmp[T, R] (f32) = A[slot(t)] · x[t]
@@ -449,8 +450,8 @@ __global__ __launch_bounds__(256) void lora_finish_tile_kernel(
     const int parts, const int chunks) {
   using lora::bf16x8_t;
   using lora::f32x4_t;
-  constexpr int H = GATE ? 2 : 1, KS = (R + 31) / 32, PAD = 3 * R + 4, WINDOW = lora::kWindow;
-  __shared__ __align__(16) float sums[16][PAD];
+  constexpr int H = GATE ? 2 : 1, KS = (R + 31) / 32, PAD = 3 * R + 8, WINDOW = lora::kWindow;
+  __shared__ __align__(16) unsigned short terms[3][16][PAD];   // of the tokens' sums
   __shared__ int groups[4][16];
   const int OW = W / H;
   const int lane = threadIdx.x & 63;
@@ -550,7 +551,16 @@ __global__ __launch_bounds__(256) void lora_finish_tile_kernel(
         for (int q = 0; q < 4; ++q)
           if (q0 + q < cuts) s += v[q];
       }
-      sums[m][r] = s;
+      // cut off, not rounded: infinity stays the first term, the others have its sign; none of a sum
+      // that is not 0 is 0, which infinities in B would make NaN, but a least number
+      const float sign = s, least = s == 0.f ? 0.f : FLT_MIN;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const unsigned bits = __float_as_uint(s);
+        terms[k][m][r] =
+            (k == 0 ? bits : __float_as_uint(copysignf(fmaxf(fabsf(s), least), sign))) >> 16;
+        s = (bits & 0x7fffffff) == 0x7f800000 ? 0.f : s - __uint_as_float(bits & 0xffff0000);
+      }
     }
     __syncthreads();
   }
@@ -565,21 +575,11 @@ __global__ __launch_bounds__(256) void lora_finish_tile_kernel(
         bf16x8_t x[KS][3];
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-          union { unsigned short u[8]; bf16x8_t v; } o[3];
           const int r = ks * 32 + quad * 8;
 #pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            float f = r < R ? sums[col][p * R + r + i] : 0.f;
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {   // cut off, not rounded: infinity stays the first term
-              const unsigned bits = __float_as_uint(f);
-              o[k].u[i] = bits >> 16;
-              f = (bits & 0x7fffffff) == 0x7f800000 ? 0.f
-                                                     : f - __uint_as_float(bits & 0xffff0000);
-            }
-          }
-#pragma unroll
-          for (int k = 0; k < 3; ++k) x[ks][k] = o[k].v;
+          for (int k = 0; k < 3; ++k)
+            x[ks][k] = r < R ? *reinterpret_cast<const bf16x8_t*>(&terms[k][col][p * R + r])
+                             : bf16x8_t{};
         }
 #pragma unroll
         for (int h = 0; h < H; ++h) {

@@ -178,6 +178,34 @@ def test_deltas_by_the_matrix_unit(t, k, width, spans, adapters, rank, way):
     assert (err <= 2 ** -8 * want.abs() + off + 1e-7)[~past].all(), err[~past].max().item()
 
 
+def test_infinite_adapters_by_the_matrix_unit():
+    """An infinity in B times a sum is one, of the sum's sign, whatever terms the sum enters in."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from vllm_tgis_adapter_amd.ops import _C
+
+    t, k, width, rank = 1000, 128, 5792, 8
+    g = torch.Generator("cuda").manual_seed(4)
+    x, a = (torch.randn(s, generator=g, device="cuda").bfloat16() for s in ((t, k), (1, rank, k)))
+    b = torch.randn((1, width, rank), generator=g, device="cuda").bfloat16()
+    # sums that are 0, that bf16 holds, one that is infinite itself
+    x[:3] = 0
+    x[1, 3], x[2, 5], a[0, :, 5], a[0, 2, 5] = 1, 3e38, 0.25, 4
+    b[0, 7, 2], b[0, 40, 5], b[0, 41, 0] = float("inf"), -float("inf"), float("nan")
+    b[0, 40, 2] = -1
+    slots = torch.zeros(t, dtype=torch.int32, device="cuda")
+    assert _C.lora_tiles_win(t, 1, rank, width)
+    out = torch.zeros((t, width), device="cuda").bfloat16()
+    _C.lora_delta(out, x, a, b, slots, torch.ones(1, device="cuda"), [(0, width)])
+    s = x.double() @ a[0].double().t()
+    assert (s[1:, [2, 5]].abs() > 1e-3).all()   # (no sum of float32 is of another sign)
+    assert torch.equal(out[1:, 7].double(), float("inf") * s[1:, 2].sign())
+    assert torch.equal(out[1:, 40].double(), -float("inf") * s[1:, 5].sign())
+    assert out[0, [7, 40]].isnan().all() and out[:, 41].isnan().all()
+    rest = [v for v in range(width) if v not in (7, 40, 41)]
+    assert out[:2, rest].isfinite().all() and out[3:, rest].isfinite().all()
+
+
 def test_many_adapters_of_few_tokens_take_a_column_a_thread():
     """Groups of 16 tokens are mostly empty there, and each looks through all adapters."""
     from vllm_tgis_adapter_amd.ops import _C
