@@ -81,10 +81,10 @@ __global__ __launch_bounds__(256, 2) void paged_decode_stream_kernel(
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int* table = block_tables + (long)seq * max_blocks;
 
-  // Where a sequence is cut, and so the launch short, and a workgroup's first tile does not depend on the length, block ids
-  // are asked for beside it (with the merge's loads, us: one sequence of 230 keys of 64 6.8 -> 6.5, of
-  // 700 keys of 128 8.4 -> 8.0, of 8000 in e4m3 16.8 -> 15.1; 512 of 520, uncut, 183.3 -> 184.1).
-  // Past the end of the sequence, but not of its table, they may be anything.
+  // Where a sequence is cut, and so the launch short, and a workgroup's first tile does not depend on
+  // the length, block ids are asked for beside it (with the merge's loads, us: one sequence of 230 keys
+  // of 64 6.8 -> 6.5, of 700 keys of 128 8.4 -> 8.0, of 8000 in e4m3 16.8 -> 15.1).  Past the end of the
+  // sequence, but not of its table, they may be anything.
   const int most = max_blocks * block_size;
   const bool early = CUT && (part == 0 || most <= npart * (kMinTiles * kTile));
   auto page_of = [&](int pos) { return block_shift >= 0 ? pos >> block_shift : pos / block_size; };

@@ -481,7 +481,6 @@ const float* optional_scales(const c10::optional<torch::Tensor>& t, int64_t qbit
   return qbits == 16 ? nullptr : t->data_ptr<float>();
 }
 
-// y [1, I] = silu(n Wg^T) * (n Wu^T), n = rmsnorm(x + residual), sum = x + residual
 // y = silu(x Wg^T) * (x Wu^T) for int8 [Wg; Wu] and more than 64 rows, by one launch; false:
 // nothing was done, the product's plan has no room for the gate
 bool gemm_q_gated(torch::Tensor y, torch::Tensor x, torch::Tensor wq, torch::Tensor wscale) {
@@ -502,6 +501,7 @@ bool gemm_q_gated(torch::Tensor y, torch::Tensor x, torch::Tensor wq, torch::Ten
   return true;
 }
 
+// y [1, I] = silu(n Wg^T) * (n Wu^T), n = rmsnorm(x + residual), sum = x + residual
 void row_norm_gated(torch::Tensor y, c10::optional<torch::Tensor> sum, torch::Tensor x,
                     c10::optional<torch::Tensor> residual, torch::Tensor weight, double eps,
                     torch::Tensor w, c10::optional<torch::Tensor> scales, int64_t qbits) {

@@ -217,7 +217,8 @@ void launch_moe_topk(int* ids, float* weights, const __hip_bfloat16* x,
   };
   // A token a workgroup is the shorter chain, four read the gate matrix once.  us, four | one, 8 experts
   // of 4096 inputs: 1 token 11.1 | 4.9, 33 11.3 | 5.2, 1024 11.9 | 7.7, 2048 12.8 | 11.1, 2949 14.2 | 14.4; 64
-  // of 2048: 33 95 | 46, 2000 104 | 78.  (Two: 33 tokens 7.6, 2949 14.2.)
+  // of 2048: 33 95 | 46, 2000 104 | 78.  (Two: 33 tokens 7.6, 2949 14.2.)  The line is where 8 experts
+  // cross; more of them have more sums of a wave to make, which four tokens make one after the other.
   if (T <= 2048) go(moe_topk_kernel<1>, 1);
   else go(moe_topk_kernel<4>, 4);
 }
