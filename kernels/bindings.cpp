@@ -990,6 +990,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_ring_plan", &gemm_ring_plan, "which tile a product takes, and parts of K (form << 4 | parts)");
   m.def("decode_inputs", &decode_inputs, "a captured step's inputs from a packed host buffer");
   m.def("lora_product", &lora_product, "a product with its LoRA deltas, also gated");
+  m.def("gemm_ring_lora_cuts", &gemm_ring_lora_cuts,
+        "parts of K of the adapters' shrink beside a product, 0: in a launch of its own");
   m.def("lora_tiles_win", &lora_tiles_win, "whether its deltas are added by the matrix unit");
   m.def("lora_delta", &lora_delta,
         "bf16 multi-LoRA of up to three projections of one input");

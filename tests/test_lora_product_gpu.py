@@ -73,6 +73,25 @@ def test_product(t, k, width, spans, rank, gated, given):
 ])
 @pytest.mark.parametrize("some", [False, True])
 def test_adapters_beside_the_product(t, adapters, k, rank, some):
+    _beside_the_product(t, adapters, k, rank, some, 384, [(0, 256), (256, 384)])
+
+
+# every form of tile, weights that stay in the caches and that go past them, K whole and in parts
+@pytest.mark.parametrize(("t", "width", "k", "form", "parts"), [
+    (61, 28672, 4096, 4, 1), (9, 5120, 4096, 4, 3), (61, 1408, 28672, 3, 8), (65, 15360, 512, 3, 1),
+    (129, 2688, 8192, 3, 4), (120, 28672, 4096, 2, 1), (65, 5120, 8192, 2, 6),
+    (129, 11264, 2048, 2, 1), (200, 2816, 14336, 2, 5)])
+def test_adapters_beside_every_form_of_product(t, width, k, form, parts):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from vllm_tgis_adapter_amd.ops import _C
+
+    plan = _C.gemm_ring_plan(t, width, k, False)
+    assert plan == form << 4 | parts and _C.gemm_ring_lora_cuts(t, k, 3, 32, plan) > 0
+    _beside_the_product(t, 3, k, 16, True, width, [(0, 256), (256, width)])
+
+
+def _beside_the_product(t, adapters, k, rank, some, width, spans):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
     from vllm_tgis_adapter_amd.ops import _C
@@ -82,7 +101,6 @@ def test_adapters_beside_the_product(t, adapters, k, rank, some):
     def normal(*shape, by=1.0):
         return (torch.randn(shape, generator=g, device="cuda") * by).bfloat16()
 
-    width, spans = 384, [(0, 256), (256, 384)]
     x, w = normal(t, k), normal(width, k, by=k ** -0.5)
     a, b = normal(adapters, 2 * rank, k, by=k ** -0.5), normal(adapters, width, rank)
     slots = torch.randint(-1, adapters, (t,), generator=g, device="cuda").int()
