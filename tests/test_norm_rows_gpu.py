@@ -33,3 +33,11 @@ def test_rows(dtype, hidden, rows):
     normed, residual = ops.fused_add_rms_norm(x.clone(), r.clone(), w, 1e-5)
     assert torch.equal(residual, summed)
     check(normed, summed)
+
+
+# more rows, without a sum, have two or four vectors a thread
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("hidden", [1024, 1032, 2056, 4096, 4104, 8192])
+@pytest.mark.parametrize("rows", [768, 769])
+def test_many_rows(dtype, hidden, rows):
+    test_rows(dtype, hidden, rows)
