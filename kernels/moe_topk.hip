@@ -135,20 +135,32 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(
 // Pairs p = t * top + j grouped by expert: seg [E + 1], pos[p] the sorted row of a pair,
 // rows[pos[p]] = t; pairs of no expert, whose id is any other, get no row and no pos.  One workgroup:
 // a few thousand pairs are less than a second launch.
-// Counts and places are claimed in LDS, a pair a lane: a wave that did so for all its lanes of one
-// expert at a time took, with a round trip for each, us: 33 tokens, 2 of 8 experts 3.7 where 2.1, 2949
-// 15.0 (4.8), 8192 38 (10.6); 33 tokens, 8 of 64 11.8 (2.5), 1000 85 (6.7).
+// Counts and places are claimed in LDS, a pair a lane, but for the lanes of the first one's expert, which
+// claims for all of them: where most pairs are of one expert each would wait for the others.  us, a
+// wave that claims for the lanes of one expert after the other, a round trip each | each lane for itself |
+// here: 33 tokens, 2 of 8 experts 3.7 | 2.2 | 2.2, 2949 15.1 | 4.9 | 5.2, 1000, 8 of 64 87 | 6.7 | 7.5; all of
+// one expert, 512 2.4 | 2.8 | 2.3, 4000 4.1 | 8.6 | 3.9; of two 4000 8.4 | 8.6 | 8.8.
 __global__ __launch_bounds__(1024) void moe_group_kernel(
     int* __restrict__ rows, int* __restrict__ pos, int* __restrict__ seg,
     const int* __restrict__ ids, const int pairs, const int E, const int top) {
   __shared__ int count[kMaxExperts], next[kMaxExperts];
   const int tid = threadIdx.x;
+  const int lane = tid & 63;
   for (int e = tid; e < E; e += 1024) count[e] = 0;
   __syncthreads();
-  for (int p = tid; p < pairs; p += 1024) {
-    const int e = ids[p];
-    if ((unsigned)e < (unsigned)E) atomicAdd(&count[e], 1);
-  }
+  // the lane's place among those of its expert
+  auto claim = [&](int* at, int e) {
+    const unsigned long long some = __ballot((unsigned)e < (unsigned)E);
+    if (some == 0) return 0;
+    const int lead = __builtin_ctzll(some), common = __builtin_amdgcn_readlane(e, lead);
+    const unsigned long long same = __ballot(e == common);
+    int place = 0;
+    if (lane == lead || ((unsigned)e < (unsigned)E && e != common))
+      place = atomicAdd(&at[e], lane == lead ? __popcll(same) : 1);
+    const int ahead = __popcll(same & ((1ull << lane) - 1));
+    return e == common ? __builtin_amdgcn_readlane(place, lead) + ahead : place;
+  };
+  for (int p = tid; p < pairs; p += 1024) claim(count, ids[p]);
   __syncthreads();
   if (tid == 0) {
     int at = 0;
@@ -161,9 +173,8 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(
   }
   __syncthreads();
   for (int p = tid; p < pairs; p += 1024) {
-    const int e = ids[p];
+    const int e = ids[p], row = claim(next, e);
     if ((unsigned)e >= (unsigned)E) continue;
-    const int row = atomicAdd(&next[e], 1);
     pos[p] = row;
     rows[row] = p / top;
   }

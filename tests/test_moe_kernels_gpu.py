@@ -227,7 +227,9 @@ def test_sums_of_any_width(width, top):
     assert ((out.double() - want).abs() <= 2 ** -8 * want.abs() + 1e-6).all()
 
 
-@pytest.mark.parametrize(("tokens", "top", "experts"), [(3, 2, 1), (40, 2, 8), (700, 3, 64)])
+# parts of a wave and of a round of pairs, all of one expert
+@pytest.mark.parametrize(("tokens", "top", "experts"), [
+    (3, 2, 1), (40, 2, 8), (700, 3, 64), (1024, 1, 5), (1025, 1, 33), (2100, 2, 9), (5000, 3, 1)])
 def test_pairs_without_an_expert(tokens, top, experts):
     from vllm_tgis_adapter_amd.ops import _C
 
