@@ -14,7 +14,8 @@
 // The keys of a sequence are cut over up to npart workgroups (a pure function of
 // shapes, so that a captured launch stays valid) of at least four tiles each, the
 // four waves merge in LDS, and only a sequence that was cut goes through the merge
-// kernel.
+// kernel.  Of many short sequences a wave takes a key head by itself (decode_alone_tiles): the
+// lengths say so on the device, so that a captured launch serves both.
 //
 // Measured (MI355X, 32/8 heads of 128, two layers with their cache writes): 512
 // sequences of ~520 keys, bf16: 794 -> 361 us (2.8 -> 6.1 TB/s; a plain read
@@ -55,95 +56,62 @@ template <typename T> DEVINLINE T load_here(const T* at) {
   return __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
 
-// CUT: npart > 1
-template <int HD, typename CT, bool CUT>
-__global__ __launch_bounds__(256, 2) void paged_decode_stream_kernel(
-    __hip_bfloat16* __restrict__ out,       // [nseq, nheads, HD]
-    float* __restrict__ part_acc,           // [nseq, nheads, npart, HD] (npart > 1)
-    float* __restrict__ part_ml,            // [nseq, nheads, npart, 2]  (npart > 1)
-    const __hip_bfloat16* __restrict__ q,   // [nseq, nheads, HD]
-    const CT* __restrict__ k_cache,         // [blocks, block_size, kvh, HD]
-    const CT* __restrict__ v_cache,
-    const int* __restrict__ block_tables,   // [nseq, max_blocks]
-    const int* __restrict__ seq_lens,       // [nseq]
-    const float scale_log2, const int nheads, const int kvh, const int group,
-    const int block_size, const int block_shift, const int max_blocks) {
-  constexpr bool FP8 = sizeof(CT) == 1;
-  constexpr int KS = HD / 32;              // contraction steps of a score tile
-  constexpr int DT = HD / 16;              // 16-wide tiles of the result
-  constexpr int PER = 16 / sizeof(CT);     // elements of a 16-byte load
-  constexpr int LPR = HD / PER;            // lanes per value row
-  constexpr int RPP = 64 / LPR;            // value rows per pass
-  constexpr int VP = kTile / RPP;          // passes
+// What a wave does with its tiles of 32 keys of one key head.
+template <int HD, typename CT> struct Walk {
+  static constexpr bool FP8 = sizeof(CT) == 1;
+  static constexpr int KS = HD / 32;              // contraction steps of a score tile
+  static constexpr int DT = HD / 16;              // 16-wide tiles of the result
+  static constexpr int PER = 16 / sizeof(CT);     // elements of a 16-byte load
+  static constexpr int LPR = HD / PER;            // lanes per value row
+  static constexpr int RPP = 64 / LPR;            // value rows per pass
+  static constexpr int VP = kTile / RPP;          // passes
 
-  const int seq = blockIdx.x, kv_head = blockIdx.y, part = blockIdx.z;
-  const int npart = gridDim.z;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int* table = block_tables + (long)seq * max_blocks;
-
-  // Where a sequence is cut, and so the launch short, and a workgroup's first tile does not depend on
-  // the length, block ids are asked for beside it (with the merge's loads, us: one sequence of 230 keys
-  // of 64 6.8 -> 6.5, of 700 keys of 128 8.4 -> 8.0, of 8000 in e4m3 16.8 -> 15.1).  Past the end of the
-  // sequence, but not of its table, they may be anything.
-  const int most = max_blocks * block_size;
-  const bool early = CUT && (part == 0 || most <= npart * (kMinTiles * kTile));
-  auto page_of = [&](int pos) { return block_shift >= 0 ? pos >> block_shift : pos / block_size; };
-  const int pos0 = (part * kMinTiles + wave) * kTile + (lane & 31);
-  int entry0 = 0;
-  if (early) entry0 = load_here(table + page_of(min(pos0, most - 1)));
-  const int seq_len = seq_lens[seq];
-  const int tiles = (seq_len + kTile - 1) / kTile;
-  const int tpp = tiles_per_part(tiles, npart);
-  const int lo = part * tpp;
-  // a sequence without keys (padding) still gets its zeros from part 0
-  if (lo >= tiles && part > 0) return;
-  const int hi = min(lo + tpp, tiles);
-
-  const int col = lane & 15, quad = lane >> 4;
-  const int head0 = kv_head * group;
-  const long row_elems = (long)kvh * HD;
-
-  __shared__ __align__(16) __hip_bfloat16 tile_all[kWaves][kTile * HD];
-  __shared__ float ml_all[kWaves][2][16];
-  __hip_bfloat16* tile_lds = tile_all[wave];
-
+  char* lds;                                 // the wave's tile
+  int lane, col, quad;
   bf16x8_t qf[KS];
+  u32x4_t kr[VP], vr[VP];                    // the tile that is on its way
+  float m_state, l_state;                    // of query `col`; l: this lane's keys
+  f32x4_t acc[DT];
+
+  DEVINLINE void begin() {
+    m_state = -FLT_MAX;
+    l_state = 0.f;
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    qf[ks] = bf16x8_t{};
-    if (col < group)
-      qf[ks] = *reinterpret_cast<const bf16x8_t*>(
-          q + ((long)seq * nheads + head0 + col) * HD + ks * 32 + quad * 8);
+    for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x4_t{};
   }
-
-  // cache row of key (tile * 32 + lane % 32); past the end: of the last key
-  auto slot_of = [&](int tile) {
-    const int pos = min(tile * kTile + (lane & 31), seq_len - 1);
-    const int page = page_of(pos);
-    return table[page] * block_size + (pos - page * block_size);
-  };
-
-  u32x4_t kr[VP], vr[VP];
-  auto issue = [&](int slot) {
+  // queries of `group` heads from `from` on
+  DEVINLINE void ask_queries(bf16x8_t (&to)[KS], const __hip_bfloat16* from, int group) const {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      to[ks] = bf16x8_t{};
+      if (col < group)
+        to[ks] = *reinterpret_cast<const bf16x8_t*>(from + col * HD + ks * 32 + quad * 8);
+    }
+  }
+  // slot: cache row of the tile's key lane % 32
+  DEVINLINE void issue(const CT* k_cache, const CT* v_cache, int slot, int kv_head,
+                       long row_elems) {
     long at[VP];
 #pragma unroll
     for (int ps = 0; ps < VP; ++ps)
       at[ps] = __shfl(slot, ps * RPP + lane / LPR, 64) * row_elems + kv_head * HD +
                (lane % LPR) * PER;
 #pragma unroll
-    for (int ps = 0; ps < VP; ++ps) kr[ps] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(k_cache + at[ps]));
+    for (int ps = 0; ps < VP; ++ps)
+      kr[ps] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(k_cache + at[ps]));
 #pragma unroll
-    for (int ps = 0; ps < VP; ++ps) vr[ps] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(v_cache + at[ps]));
-  };
+    for (int ps = 0; ps < VP; ++ps)
+      vr[ps] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(v_cache + at[ps]));
+  }
   // 16-byte chunk c of row r lies at chunk c ^ swizzle(r): a pair of chunks stays a
   // pair, the 16 rows of a transposed read cover all banks twice, and eight rows'
   // equal chunks lie in different banks
-  auto swizzle = [](int r) { return HD == 128 ? (r & 7) * 2 : ((r >> 1) & 3) * 2; };
-  auto stage = [&](const u32x4_t (&from)[VP]) {
+  static DEVINLINE int swizzle(int r) { return HD == 128 ? (r & 7) * 2 : ((r >> 1) & 3) * 2; }
+  DEVINLINE void stage(const u32x4_t (&from)[VP]) const {
 #pragma unroll
     for (int ps = 0; ps < VP; ++ps) {
       const int r = ps * RPP + lane / LPR;
-      char* row = reinterpret_cast<char*>(tile_lds) + r * HD * 2;
+      char* row = lds + r * HD * 2;
       if constexpr (FP8) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -159,27 +127,10 @@ __global__ __launch_bounds__(256, 2) void paged_decode_stream_kernel(
     }
     // other lanes of this wave read it: LDS keeps a wave's order, the compiler has to
     asm volatile("" ::: "memory");
-  };
-
-  float m_state = -FLT_MAX, l_state = 0.f;   // of query `col`; l: this lane's keys
-  f32x4_t acc[DT];
-#pragma unroll
-  for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x4_t{};
-
-  int t = lo + wave, slot_next = 0;
-  if (t < hi) {
-    int slot;
-    if (early) {   // past the end: of the tile's first key
-      slot = (unsigned)entry0 * block_size + (pos0 - page_of(pos0) * block_size);
-      const int begin = __shfl(slot, 0, 64);
-      if (pos0 >= seq_len) slot = begin;
-    } else {
-      slot = slot_of(t);
-    }
-    issue(slot);
-    if (t + kWaves < hi) slot_next = slot_of(t + kWaves);
   }
-  for (; t < hi; t += kWaves) {
+  // The tile on its way, of keys key0 .. key0 + 31; `next` asks for the one after it.
+  template <typename Next>
+  DEVINLINE void work(const int key0, const int seq_len, const float scale_log2, Next next) {
     f32x4_t s[2] = {f32x4_t{}, f32x4_t{}};
     stage(kr);
 #pragma unroll
@@ -188,19 +139,15 @@ __global__ __launch_bounds__(256, 2) void paged_decode_stream_kernel(
       for (int rt = 0; rt < 2; ++rt) {
         const int r = rt * 16 + col;
         const bf16x8_t kf = *reinterpret_cast<const bf16x8_t*>(
-            reinterpret_cast<const char*>(tile_lds) + r * HD * 2 +
-            ((ks * 4 + quad) ^ swizzle(r)) * 16);
+            lds + r * HD * 2 + ((ks * 4 + quad) ^ swizzle(r)) * 16);
         s[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[ks], s[rt], 0, 0, 0);
       }
     asm volatile("" ::: "memory");
     stage(vr);
-    if (t + kWaves < hi) {
-      issue(slot_next);
-      if (t + 2 * kWaves < hi) slot_next = slot_of(t + 2 * kWaves);
-    }
+    next();
 
     // ---- softmax: lane has keys rt*16 + quad*4 + r of query col ----------
-    const int base = t * kTile + quad * 4;
+    const int base = key0 + quad * 4;
     float big = -FLT_MAX;
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt)
@@ -243,33 +190,137 @@ __global__ __launch_bounds__(256, 2) void paged_decode_stream_kernel(
 #pragma unroll
       for (int rt = 0; rt < 2; ++rt) {
         const int r = rt * 16 + quad * 4 + (col >> 2);
-        char* at = reinterpret_cast<char*>(tile_lds) + r * HD * 2 +
-                   ((dt * 2 + ((col & 3) >> 1)) ^ swizzle(r)) * 16 + (col & 1) * 8;
+        char* at = lds + r * HD * 2 + ((dt * 2 + ((col & 3) >> 1)) ^ swizzle(r)) * 16 +
+                   (col & 1) * 8;
         vf.h[rt] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)at);
       }
       acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, p.v, acc[dt], 0, 0, 0);
     }
     asm volatile("" ::: "memory");
   }
+  // l of all of the tiles' keys
+  DEVINLINE void end() {
+    l_state += __shfl_xor(l_state, 16, 64);
+    l_state += __shfl_xor(l_state, 32, 64);
+  }
+};
+
+// CUT: npart > 1
+template <int HD, typename CT, bool CUT>
+__global__ __launch_bounds__(256, 2) void paged_decode_stream_kernel(
+    __hip_bfloat16* __restrict__ out,       // [nseq, nheads, HD]
+    float* __restrict__ part_acc,           // [nseq, nheads, npart, HD] (npart > 1)
+    float* __restrict__ part_ml,            // [nseq, nheads, npart, 2]  (npart > 1)
+    const __hip_bfloat16* __restrict__ q,   // [nseq, nheads, HD]
+    const CT* __restrict__ k_cache,         // [blocks, block_size, kvh, HD]
+    const CT* __restrict__ v_cache,
+    const int* __restrict__ block_tables,   // [nseq, max_blocks]
+    const int* __restrict__ seq_lens,       // [nseq]
+    const float scale_log2, const int nheads, const int kvh, const int group,
+    const int block_size, const int block_shift, const int max_blocks,
+    const int alone_tiles) {   // see decode_alone_tiles
+  using W = Walk<HD, CT>;
+  const int seq = blockIdx.x, part = blockIdx.z;
+  int kv_head = blockIdx.y;
+  const int npart = gridDim.z;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int* table = block_tables + (long)seq * max_blocks;
+
+  // Where a sequence is cut, and so the launch short, and a workgroup's first tile does not depend on
+  // the length, block ids are asked for beside it (with the merge's loads, us: one sequence of 230 keys
+  // of 64 6.8 -> 6.5, of 700 keys of 128 8.4 -> 8.0, of 8000 in e4m3 16.8 -> 15.1).  Past the end of the
+  // sequence, but not of its table, they may be anything.
+  const int most = max_blocks * block_size;
+  const bool early = CUT && (part == 0 || most <= npart * (kMinTiles * kTile));
+  auto page_of = [&](int pos) { return block_shift >= 0 ? pos >> block_shift : pos / block_size; };
+  const int pos0 = (part * kMinTiles + wave) * kTile + (lane & 31);
+  int entry0 = 0;
+  if (early) entry0 = load_here(table + page_of(min(pos0, most - 1)));
+  const int seq_len = seq_lens[seq];
+  const int tiles = (seq_len + kTile - 1) / kTile;
+  const int tpp = tiles_per_part(tiles, npart);
+  const int lo = part * tpp;
+  // a sequence without keys (padding) still gets its zeros from part 0
+  if (lo >= tiles && part > 0) return;
+  const int hi = min(lo + tpp, tiles);
+  // Few keys: a wave takes a key head by itself, every fourth workgroup four of them.
+  const bool alone = tiles <= alone_tiles;
+  if (alone) {
+    if (kv_head % kWaves != 0) return;
+    kv_head += wave;
+  }
+
+  const int head0 = kv_head * group;
+  const long row_elems = (long)kvh * HD;
+
+  __shared__ __align__(16) __hip_bfloat16 tile_all[kWaves][kTile * HD];
+  __shared__ float ml_all[kWaves][2][16];
+  W walk;
+  walk.lds = reinterpret_cast<char*>(tile_all[wave]);
+  walk.lane = lane;
+  walk.col = lane & 15;
+  walk.quad = lane >> 4;
+  const int col = walk.col, quad = walk.quad;
+  walk.ask_queries(walk.qf, q + ((long)seq * nheads + head0) * HD, group);
+
+  // cache row of key (tile * 32 + lane % 32); past the end: of the last key
+  auto slot_of = [&](int tile) {
+    const int pos = min(tile * kTile + (lane & 31), seq_len - 1);
+    const int page = page_of(pos);
+    return table[page] * block_size + (pos - page * block_size);
+  };
+  walk.begin();
+
+  int t = alone ? 0 : lo + wave, slot_next = 0;
+  const int stride = alone ? 1 : kWaves;
+  if (t < hi) {
+    int slot;
+    if (early && !alone) {   // past the end: of the tile's first key
+      slot = (unsigned)entry0 * block_size + (pos0 - page_of(pos0) * block_size);
+      const int begin = __shfl(slot, 0, 64);
+      if (pos0 >= seq_len) slot = begin;
+    } else {
+      slot = slot_of(t);
+    }
+    walk.issue(k_cache, v_cache, slot, kv_head, row_elems);
+    if (t + stride < hi) slot_next = slot_of(t + stride);
+  }
+  for (; t < hi; t += stride)
+    walk.work(t * kTile, seq_len, scale_log2, [&] {
+      if (t + stride < hi) {
+        walk.issue(k_cache, v_cache, slot_next, kv_head, row_elems);
+        if (t + 2 * stride < hi) slot_next = slot_of(t + 2 * stride);
+      }
+    });
+  walk.end();
+  if (alone) {
+    if (col >= group) return;
+    const float inv = walk.l_state > 0.f ? 1.f / walk.l_state : 0.f;
+    __hip_bfloat16* o = out + ((long)seq * nheads + head0 + col) * HD + quad * 4;
+#pragma unroll
+    for (int dt = 0; dt < W::DT; ++dt)
+      *reinterpret_cast<uint2*>(o + dt * 16) =
+          uint2{pack_bf16(walk.acc[dt][0] * inv, walk.acc[dt][1] * inv),
+                pack_bf16(walk.acc[dt][2] * inv, walk.acc[dt][3] * inv)};
+    return;
+  }
 
   // ---- the waves' results become one ---------------------------------------
-  l_state += __shfl_xor(l_state, 16, 64);
-  l_state += __shfl_xor(l_state, 32, 64);
   if (lane < 16) {
-    ml_all[wave][0][lane] = m_state;
-    ml_all[wave][1][lane] = l_state;
+    ml_all[wave][0][lane] = walk.m_state;
+    ml_all[wave][1][lane] = walk.l_state;
   }
   __syncthreads();
   float M = ml_all[0][0][col];
 #pragma unroll
   for (int w = 1; w < kWaves; ++w) M = fmaxf(M, ml_all[w][0][col]);
-  const float f = __builtin_amdgcn_exp2f(m_state - M);
+  const float f = __builtin_amdgcn_exp2f(walk.m_state - M);
   float* mine = reinterpret_cast<float*>(tile_all[wave]);   // [16][HD]
   static_assert(kTile * 2 >= 16 * 4, "a wave's tile holds its result");
   if (col < group) {
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-      *reinterpret_cast<f32x4_t*>(mine + col * HD + dt * 16 + quad * 4) = acc[dt] * f;
+    for (int dt = 0; dt < W::DT; ++dt)
+      *reinterpret_cast<f32x4_t*>(mine + col * HD + dt * 16 + quad * 4) = walk.acc[dt] * f;
   }
   __syncthreads();
   const bool whole = tpp >= tiles;
@@ -343,6 +394,22 @@ __global__ __launch_bounds__(HD) void decode_stream_merge_kernel(
   out[row * HD + d] = __float2bfloat16(a * (L > 0.f ? 1.f / L : 0.f));
 }
 
+// Up to how many tiles a sequence's key heads are a wave's each instead of a workgroup's, -1: never.
+// With a tile or two most waves of a workgroup have none, and what it takes is its chain of loads
+// and the waves' meeting: worth it where the workgroups are more than are resident at a time (two or
+// three a CU).  Two layers with their cache writes, us, a head a workgroup | up to 1, 2, 4, 6 tiles a head a
+// wave; 32/8 heads of 128, sequences x mean keys: 453 x 34 75.8 | 68.1, 51.2, 51.1, 51.1 (e4m3 60.1 |
+// 51.6, 39.1, 39.0, 38.7); 194 x 62 47.1 | 46.4, 43.3, 42.5, 42.4; 190 x 90 64.3 | 64.8, 64.8, 60.9, 69.0;
+// 400 x 128 105.6 | 105.5, 104.8, 101.6, 98.9; 100 x 60 36.9 | 36.7, 35.3, 35.9, 35.9; 50 x 60 27.4 |
+// 27.3, 29.7, 33.4, 33.5; 64 x 30 26.4 | 26.5, 31.6; 64/8 heads, 81 x 22 35.3 | 28.8, 30.6, 30.5; heads of
+// 64, 512 x 50 48.5 | 48.1, 42.7, 39.8, 39.7.  (The workgroups that work first instead of every fourth:
+// the same there, and 512 x 520 0.8 % slower.)
+int decode_alone_tiles(int nseq, int kvh) {
+  if (kvh % kWaves != 0) return -1;
+  const long heads = (long)nseq * kvh;
+  return heads >= 1536 ? 4 : heads >= 640 ? 2 : -1;
+}
+
 template <int HD, typename CT>
 void launch(__hip_bfloat16* out, float* part_acc, float* part_ml, const __hip_bfloat16* q,
             const CT* kc, const CT* vc, const int* bt, const int* sl, float scale, int nseq,
@@ -350,10 +417,11 @@ void launch(__hip_bfloat16* out, float* part_acc, float* part_ml, const __hip_bf
             hipStream_t stream) {
   int shift = -1;
   if ((block_size & (block_size - 1)) == 0) shift = __builtin_ctz(block_size);
+  const int alone = decode_alone_tiles(nseq, kvh);
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(nseq, kvh, npart), dim3(256), 0, stream, out, part_acc, part_ml,
                        q, kc, vc, bt, sl, scale * kLog2e, nheads, kvh, nheads / kvh, block_size,
-                       shift, max_blocks);
+                       shift, max_blocks, alone);
   };
   if (npart > 1) go(paged_decode_stream_kernel<HD, CT, true>);
   else go(paged_decode_stream_kernel<HD, CT, false>);

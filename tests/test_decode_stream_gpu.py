@@ -95,3 +95,36 @@ def test_block_ids_past_the_end_say_nothing(fp8, block, lens, width):
     got = ops.paged_attention_decode(
         q, kc, vc, tables.masked_fill(past, 2 ** 31 - 1), seq_lens, 0.1, max(lens))
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize(("kvh", "group", "hd", "nseq", "width"), [
+    (8, 4, 128, 80, 40),       # 640 heads: up to two tiles a wave's each, sequences are cut
+    (8, 1, 64, 81, 16),
+    (8, 8, 128, 192, 512),     # 1536: up to four tiles, uncut
+    (4, 3, 64, 400, 9),
+    (6, 2, 128, 300, 9),       # key heads are no whole workgroups: never
+])
+def test_heads_of_short_sequences_are_a_waves_each(fp8, kvh, group, hd, nseq, width):
+    """Lengths on both sides of two and four tiles of 32 keys beside each other."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from vllm_tgis_adapter_amd import ops
+    from vllm_tgis_adapter_amd.ops import reference as R
+
+    edges = [1, 31, 33, 0, 64, 65, 128, 129]
+    lens = [edges[i % 8] for i in range(nseq)]
+    kc, vc, tables = _caches(lens, 16, kvh, hd, fp8, 5, width)
+    q = torch.randn(nseq, kvh * group, hd, generator=torch.Generator().manual_seed(6)).bfloat16()
+    seq_lens = torch.tensor(lens, dtype=torch.int32)
+    out = ops.paged_attention_decode(q.cuda(), kc.cuda(), vc.cuda(), tables.cuda(),
+                                     seq_lens.cuda(), hd ** -0.5, max(lens)).float().cpu()
+    if fp8:
+        kc, vc = (c.view(torch.float8_e4m3fn) for c in (kc, vc))
+    live = [i for i, n in enumerate(lens) if n]
+    want = R.paged_attention(
+        q[live].float(), kc.float(), vc.float(), tables[live],
+        torch.arange(len(live) + 1, dtype=torch.int32), seq_lens[live], hd ** -0.5)
+    # as above
+    assert (out[live] - want).abs().max() <= 2 ** -8 * vc.float().abs().max()
+    assert not out[[i for i, n in enumerate(lens) if not n]].any()
