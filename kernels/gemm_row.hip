@@ -18,11 +18,11 @@
 // us over 1 GB of weights in turn, gemm_stream.h -> here (at 6.2 TB/s; reads in sequence
 // reach 6.4), N x K:
 //   4 bits: 28672 x 4096 23.7 -> 15.9 (10.1), 6144 x 4096 8.9 -> 6.0 (2.2), 4096 x 4096 6.7 ->
-//     4.9 (1.4), 4096 x 14336 17.4 -> 11.5 (5.0);
+//     4.9 (1.4), 4096 x 14336 17.4 -> 10.5 (5.0);
 //   int8: 28672 x 4096 26.5 -> 22.0 (18.9), 6144 x 4096 9.6 -> 7.3 (4.1), 4096 x 14336 16.0 ->
-//     12.8 (9.5), 2048 x 8192 8.6 -> 6.1 (2.7), 32000 x 2048 15.0 -> 13.7 (10.6);
-//   bf16: 14336 x 4096 gated 41.7 -> 36.9 (37.9), 8192 x 2048 gated 15.7 -> 13.4 (10.8), 2048 x
-//     8192 11.4 -> 8.8 (5.4), 2048 x 2048 5.1 -> 4.0 (1.4), 32000 x 2048 27.8 -> 22.5 (21.1).
+//     12.2 (9.5), 2048 x 8192 8.6 -> 5.8 (2.7), 32000 x 2048 15.0 -> 13.7 (10.6);
+//   bf16: 14336 x 4096 gated 41.7 -> 36.9 (37.9), 8192 x 2048 gated 15.7 -> 13.0 (10.8), 2048 x
+//     8192 11.4 -> 7.7 (5.4), 2048 x 2048 5.1 -> 4.0 (1.4), 32000 x 2048 27.8 -> 22.5 (21.1).
 // With the norm a product takes 0.3 to 0.7 us more, with rotation and cache write 0.5 to 1.3,
 // where launches of their own took 2 to 4 each: a llama-1b step 412 -> 365 us, a llama-3-8b
 // one in 4 bits, whose gate is in the product now, 604 -> 451.
@@ -38,7 +38,6 @@ typedef __attribute__((ext_vector_type(4))) unsigned int u32x4_t;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf2_t;
 
 constexpr int kRows = 4;    // of W, a wave
-constexpr int kWaves = 4;
 
 DEVINLINE float dot2(unsigned a, unsigned b, float c) {
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf2_t, a),
@@ -72,7 +71,7 @@ enum RowMode { kRowPlain = 0, kRowGated = 1, kRowTurn = 2 };
 
 // MODE: plain takes four neighbouring rows of W a wave, gated two of each half of W, turn two
 // of each half of a head.  KS: waves that K is dealt to, the others take other rows of W.
-template <int QB, int MODE, int KS, bool NORM>
+template <int QB, int MODE, int KS, bool NORM, int kWaves>
 __global__ __launch_bounds__(64 * kWaves, 4) void gemm_row_kernel(
     __hip_bfloat16* __restrict__ y,         // [N] (turn: the queries)
     const __hip_bfloat16* __restrict__ x,   // [K]
@@ -401,29 +400,75 @@ struct RowCall {
   hipStream_t stream;
 };
 
-template <int QB, int MODE, int KS, bool NORM>
+template <int QB, int MODE, int KS, bool NORM, int kWaves>
 void launch(const RowCall& c) {
   constexpr int SEG = 64 * 128 / QB, COLS = kWaves / KS * (MODE == kRowPlain ? kRows : kRows / 2);
   static_assert(128 % COLS == 0 && 16 % COLS == 0, "whole workgroups, inside half a head");
-  // four workgroups a CU walk the rows (28672 x 4096 4 bits: 17.0 us, two 19.1, all 19.2)
+  // sixteen waves a CU walk the rows (28672 x 4096 4 bits: 17.0 us, eight 19.1, all 19.2)
+  constexpr int MOST = 256 * 16 / kWaves;
   const int blocks = (MODE == kRowTurn ? c.N / 2 : c.N) / COLS;
-  hipLaunchKernelGGL((gemm_row_kernel<QB, MODE, KS, NORM>), dim3(blocks < 1024 ? blocks : 1024),
-                     dim3(64 * kWaves), (c.K + SEG - 1) / SEG * SEG * 2, c.stream, c.y, c.x,
+  hipLaunchKernelGGL((gemm_row_kernel<QB, MODE, KS, NORM, kWaves>),
+                     dim3(blocks < MOST ? blocks : MOST), dim3(64 * kWaves), (c.K + SEG - 1) / SEG * SEG * 2, c.stream, c.y, c.x,
                      static_cast<const unsigned char*>(c.w), c.scale, c.N, c.K, c.norm, c.turns);
 }
 
-// K is dealt to all four waves in bf16 (2048 x 8192 8.8 us, to two 10.0, to one 14.2); in 4
-// bits a load covers 2048 inputs, and rows go first where they are many (28672 x 4096: one
-// 17.0, two 21.7; 2048 x 8192: four 6.0, two 7.0, one 9.9).
+// Waves of a workgroup, and over how many of them K is dealt (us, N x K, W/KS).  With eight waves half
+// as many workgroups stage x, and of long K more is asked for at once; K dealt to more waves leaves
+// shorter chains where rows are few, to fewer less to add up and more rows that share x.
+//   bf16, 4/4 | 8/8: 2048 x 8192 8.43 | 7.65, 4096 x 14336 21.7 | 20.7, 8192 x 28672 77.4 | 74.9, 4096 x 7168
+//     11.74 | 11.40, 768 x 8192 5.90 | 5.04; 2560 x 8192 9.85 | 10.04 (640 blocks, 512 workgroups); 8192 x
+//     8192 24.4 | 24.6, 8/4 24.0; 16384 x 8192 44.9 | 46.6, 8/4 44.5; to 4096 inputs 8/8 loses 6 %.
+//     Gated, 4/4 | 4/2 | 8/4: 8192 x 2048 13.71 | 13.03 | 13.40, 3072 x 1024 5.63 | 5.19, 28672 x 8192 147.0 |
+//     149.3 | 145.2, 7168 x 8192 42.3 | 42.5 | 41.1, 14336 x 4096 38.8 | 39.2 | 38.6.  Turned, 4/4 | 8/8 | 8/4:
+//     1280 x 8192 8.86 | 7.83 | 8.24, 5120 x 8192 18.8 | 17.8 | 18.5, 10240 x 8192 31.6 | 31.2 | 30.8, 6144 x 4096
+//     10.8 | 11.2 | 11.2.
+//   int8, 4/4 | 8/4: 8192 x 28672 46.1 | 40.5, 4096 x 14336 12.6 | 12.2, 2048 x 8192 6.09 | 5.78, 4096 x 4096
+//     5.79 | 5.83.  Gated, 4/4 | 4/2 | 8/4: 14336 x 4096 24.0 | 22.0 | 23.3, 7168 x 4096 13.4 | 12.9 | 13.6, 28672 x
+//     8192 78.7 | 80.0 | 76.3; 4/2 | 4/1: 8192 x 2048 9.06 | 8.63, 2048 x 2048 4.92 | 4.84.  Turned, 4/4 |
+//     8/4: 6144 x 4096 8.25 | 7.78, 10240 x 8192 18.6 | 17.5, 3072 x 4096 6.36 | 6.52.
+//   4 bits (a load covers 2048 inputs), plain, 4/4 | 8/2 | 8/4 | 8/8: 8192 x 28672 34.5 | 27.6 | 29.8 | 31.0,
+//     4096 x 14336 11.08 | 10.51 | 10.92 | 11.32, 8192 x 8192 11.7 | 11.6 | 11.6 | 11.8, 4096 x 7168 7.20 | 7.11 |
+//     6.65 | 7.39, 2048 x 8192 5.38 | 6.47 | 4.98 | 5.06, 1024 x 8192 4.12 | 5.86 | 4.25 | 3.88.  Shorter
+//     K, and with pairs: rows go first where they are many (14336 x 4096 gated 4/1 16.9, 4/2 17.9; 2048 x
+//     8192 4/1 7.0, 4/2 5.5).
 template <int MODE, bool NORM>
 void launch_bits(const RowCall& c, int qbits) {
   const int rows = MODE == kRowGated ? 2 * c.N : c.N;
-  if (qbits == 16) launch<16, MODE, 4, NORM>(c);
-  else if (qbits == 8 && c.K > 2048) launch<8, MODE, 4, NORM>(c);
-  else if (qbits == 8) launch<8, MODE, 2, NORM>(c);
-  else if (c.K > 2048 * 3 && rows <= 8192) launch<4, MODE, 4, NORM>(c);
-  else if (c.K > 2048 && rows <= 16384) launch<4, MODE, 2, NORM>(c);
-  else launch<4, MODE, 1, NORM>(c);
+#define GO(QB, W, KS) launch<QB, MODE, KS, NORM, W>(c)
+  if (qbits == 16) {
+    if constexpr (MODE == kRowPlain) {
+      if (c.K >= 7168 && (c.N <= 2048 || (c.N >= 4096 && (c.N < 8192 || c.K > 8192))))
+        return GO(16, 8, 8);
+      if (c.K >= 7168 && c.N >= 8192) return GO(16, 8, 4);
+    } else if constexpr (MODE == kRowGated) {
+      if (c.K <= 2048) return GO(16, 4, 2);
+      if (c.K >= 8192) return GO(16, 8, 4);
+    } else if (c.K >= 8192) {
+      return c.N <= 5120 ? GO(16, 8, 8) : GO(16, 8, 4);
+    }
+    return GO(16, 4, 4);
+  }
+  if (qbits == 8) {
+    if constexpr (MODE == kRowGated) {
+      if (c.K <= 2048) return GO(8, 4, 1);
+      if (c.K < 8192) return GO(8, 4, 2);
+      return GO(8, 8, 4);
+    } else {
+      if (c.K <= 2048) return GO(8, 4, 2);
+      if (MODE == kRowTurn ? c.K >= 4096 && c.N >= 6144 : c.K >= 7168) return GO(8, 8, 4);
+      return GO(8, 4, 4);
+    }
+  }
+  if constexpr (MODE == kRowPlain) {
+    if (c.K > 2048 * 3) {
+      if (c.N < 2048) return GO(4, 8, 8);
+      return c.N > 4096 || (c.N == 4096 && c.K > 8192) ? GO(4, 8, 2) : GO(4, 8, 4);
+    }
+  }
+  if (MODE != kRowPlain && c.K > 2048 * 3 && rows <= 8192) return GO(4, 4, 4);
+  if (c.K > 2048 && rows <= 16384) return GO(4, 4, 2);
+  GO(4, 4, 1);
+#undef GO
 }
 
 }  // namespace

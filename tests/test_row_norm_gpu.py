@@ -117,6 +117,55 @@ def test_int8_products_of_one_row(n, k):
     _close(ops.linear_quant(x, w, s, 8), x.double() @ value.t())
 
 
+@pytest.mark.parametrize("bits", [16, 8, 4])
+@pytest.mark.parametrize(("n", "k"), [
+    (128, 7168), (2048, 7296),       # a K that ends inside a wave's load
+    (2176, 8320), (4096, 8192), (4096, 14464), (4224, 6400), (8192, 7168), (8320, 8320),
+    (16512, 7168)])                  # more rows than the workgroups take at a time
+def test_long_rows(bits, n, k):
+    """Plain products on both sides of where workgroups of eight waves begin."""
+    from vllm_tgis_adapter_amd import ops
+
+    gen = torch.Generator("cuda").manual_seed(n + k + bits)
+    w, s, value = _weights(n, k, bits, gen)
+    x = torch.randn((1, k), generator=gen, device="cuda").bfloat16()
+    got = ops.linear(x, w) if bits == 16 else ops.linear_quant(x, w, s, bits)
+    _close(got, x.double() @ value.t())
+
+
+@pytest.mark.parametrize("bits", [16, 8, 4])
+@pytest.mark.parametrize(("k", "inter"), [(1920, 640), (2176, 1280), (8320, 4224), (8192, 14336)])
+def test_gates_of_long_rows(bits, k, inter):
+    from vllm_tgis_adapter_amd import ops
+
+    gen = torch.Generator("cuda").manual_seed(k + bits)
+    x, r, g, total, n = _row(k, gen, True)
+    w, s, value = _weights(2 * inter, k, bits, gen)
+    out, rest = ops.row_norm_gated(x, r, g, EPS, w, s, bits)
+    assert torch.equal(rest, total)
+    _close_gated(out, *(n @ value.t()).chunk(2, dim=1))
+
+
+@pytest.mark.parametrize("bits", [16, 8])
+@pytest.mark.parametrize(("k", "heads", "kv_heads"), [(8192, 38, 2), (8192, 40, 2), (4096, 44, 2)])
+def test_rotation_of_long_rows(bits, k, heads, kv_heads):
+    """Heads of 128, around the widths where K is dealt to fewer of eight waves."""
+    from vllm_tgis_adapter_amd import ops
+
+    gen = torch.Generator("cuda").manual_seed(k + heads + bits)
+    x, r, g, total, n = _row(k, gen, True)
+    w, s, value = _weights((heads + 2 * kv_heads) * 128, k, bits, gen)
+    cos_sin = torch.cat([torch.ones(500, 64), torch.zeros(500, 64)], dim=1).cuda()
+    kc, vc = (torch.zeros((4, 16, kv_heads, 128), device="cuda", dtype=torch.bfloat16)
+              for _ in "kv")
+    q, rest = ops.row_norm_qkv(x, r, g, EPS, w, s, bits, heads, torch.tensor([7], device="cuda"),
+                               cos_sin, kc, vc, torch.tensor([20], device="cuda"))
+    assert torch.equal(rest, total)
+    y = (n @ value.t()).view(heads + 2 * kv_heads, 128)
+    _close(torch.cat([q.view(heads, 128), kc.view(-1, kv_heads, 128)[20],
+                      vc.view(-1, kv_heads, 128)[20]]), y, ulps=4.0)
+
+
 def test_what_stays_with_the_launches_apart(monkeypatch):
     from vllm_tgis_adapter_amd import ops
 
