@@ -78,10 +78,10 @@ void launch_gemm_skinny(__hip_bfloat16*, float*, const __hip_bfloat16*,
 void launch_gemm_skinny_gated(__hip_bfloat16*, float*, const __hip_bfloat16*,
                               const __hip_bfloat16*, int, int, int, int,
                               hipStream_t);
-int gemm_panel_plan(int M, int N, int K);
-int gemm_panel_gated_plan(int M, int N, int K);
+int gemm_panel_plan(int M, int N, int K, int qbits);
+int gemm_panel_gated_plan(int M, int N, int K, int qbits);
 void launch_gemm_panel_gated(__hip_bfloat16*, const __hip_bfloat16*, const unsigned char*,
-                             const float*, int, int, int, int, hipStream_t);
+                             const float*, int, int, int, int, int, hipStream_t);
 void launch_gemm_block_q(__hip_bfloat16*, float*, const __hip_bfloat16*, const unsigned char*,
                          const float*, int, int, int, int, int, hipStream_t);
 void launch_widen_weight(__hip_bfloat16*, const unsigned char*, const float*, int, long, int,
@@ -416,7 +416,7 @@ void gemm_q(torch::Tensor y, torch::Tensor x, torch::Tensor wq, torch::Tensor ws
     // both reach LDS in 16-byte pieces
     TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
                 reinterpret_cast<uintptr_t>(wq.data_ptr()) % 16 == 0);
-    const int plan = qbits == 8 ? gemm_panel_plan(M, N, K) : 1;
+    const int plan = gemm_panel_plan(M, N, K, (int)qbits);
     torch::Tensor part;
     launch_gemm_block_q(ptr<__hip_bfloat16>(y), stream_parts(part, x, plan & 255, (int64_t)M * N),
                         cptr<__hip_bfloat16>(x), cptr<unsigned char>(wq),
@@ -481,13 +481,14 @@ const float* optional_scales(const c10::optional<torch::Tensor>& t, int64_t qbit
   return qbits == 16 ? nullptr : t->data_ptr<float>();
 }
 
-// y = silu(x Wg^T) * (x Wu^T) for int8 [Wg; Wu] and more than 64 rows, by one launch; false:
+// y = silu(x Wg^T) * (x Wu^T) for rounded [Wg; Wu] and more than 64 rows, by one launch; false:
 // nothing was done, the product's plan has no room for the gate
-bool gemm_q_gated(torch::Tensor y, torch::Tensor x, torch::Tensor wq, torch::Tensor wscale) {
+bool gemm_q_gated(torch::Tensor y, torch::Tensor x, torch::Tensor wq, torch::Tensor wscale,
+                  int64_t qbits) {
   const int64_t M = x.size(0), K = x.size(1), N = wq.size(0) / 2;
-  const int plan = gemm_panel_gated_plan((int)M, (int)N, (int)K);
+  const int plan = gemm_panel_gated_plan((int)M, (int)N, (int)K, (int)qbits);
   if (plan == 0) return false;
-  check_rounded(wq, wscale, 8, 2 * N, K);
+  check_rounded(wq, wscale, qbits, 2 * N, K);
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::ScalarType::BFloat16 &&
               y.scalar_type() == at::ScalarType::BFloat16);
   TORCH_CHECK(x.is_contiguous() && y.is_contiguous() && y.size(0) == M && y.size(1) == N);
@@ -496,8 +497,8 @@ bool gemm_q_gated(torch::Tensor y, torch::Tensor x, torch::Tensor wq, torch::Ten
               reinterpret_cast<uintptr_t>(wq.data_ptr()) % 16 == 0 &&
               reinterpret_cast<uintptr_t>(y.data_ptr()) % 8 == 0);
   launch_gemm_panel_gated(ptr<__hip_bfloat16>(y), cptr<__hip_bfloat16>(x),
-                          cptr<unsigned char>(wq), wscale.data_ptr<float>(), (int)M, (int)N, (int)K,
-                          plan, current_stream());
+                          cptr<unsigned char>(wq), wscale.data_ptr<float>(), (int)qbits, (int)M,
+                          (int)N, (int)K, plan, current_stream());
   return true;
 }
 
@@ -957,10 +958,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("widen_weight", &widen_weight, "int8 / 4-bit weights to bf16");
   m.def("gemm_skinny", &gemm_skinny,
         "skinny decode GEMM y = x @ w^T, M <= 64 (CDNA4 MFMA)");
-  m.def("gemm_q_gated", &gemm_q_gated, "gated int8 product of many rows, where it is one launch");
-  m.def("gemm_panel_gated_plan", &gemm_panel_gated_plan, "its plan, or 0");
+  m.def("gemm_q_gated", &gemm_q_gated,
+        "gated product of many rows with rounded weights, where it is one launch", py::arg("y"),
+        py::arg("x"), py::arg("wq"), py::arg("wscale"), py::arg("qbits") = 8);
+  m.def("gemm_panel_gated_plan", &gemm_panel_gated_plan, "its plan, or 0", py::arg("m"),
+        py::arg("n"), py::arg("k"), py::arg("qbits") = 8);
   m.def("gemm_panel_plan", &gemm_panel_plan,
-        "which panel int8 products of many rows take, and parts of K (panel << 8 | parts)");
+        "which panel products of many rows with rounded weights take, and parts of K (panel << 8 | "
+        "parts)", py::arg("m"), py::arg("n"), py::arg("k"), py::arg("qbits") = 8);
   m.def("row_norm_gated", &row_norm_gated, "norm and gated product of one row (CDNA4)");
   m.def("row_norm_turn", &row_norm_turn,
         "norm, query / key / value product, rotation and cache write of one row (CDNA4)");

@@ -5,14 +5,14 @@
 // two products, all in f32 in memory) ahead of a library product: 1.0 ms of 1.3 ms a
 // llama-3-8b layer at 301 rows.  Now
 //  - up to some hundreds of rows the product widens a tile's weights itself, between LDS
-//    and the matrix unit: W crosses memory once, at its own size (int8: gemm_panel_q.h, but
+//    and the matrix unit: W crosses memory once, at its own size (gemm_panel_q.h, but
 //    for small matrices);
 //  - above, one kernel writes the widened matrix (bf16(q scale), bound by its bytes) for
 //    the library's product, which is then the larger part and the faster one.
 //
 // In the product weights are whole numbers and scales are applied to 32-bit sums, as in
-// gemm_stream.hip: int8 by conversion to f32 of which the upper half is all; 4 bits as the
-// bf16 pattern of 8 + n/2, with -12 times the sum of x added by a constant operand and the
+// gemm_stream.hip: int8 by conversion to f32 of which the upper half is all; 4 bits (in tiles; panels
+// have n - 8 itself) as the bf16 pattern of 8 + n/2, with -12 times the sum of x added by a constant operand and the
 // scale doubled.  A lane's 16 bytes of W hold the inputs of two matrix steps in int8, of four
 // in 4 bits, and x is read to match.  x and W reach LDS without registers; chunks of a row are
 // turned by the row: x by r (256-byte rows) or r / 2 (128), W by r / 2 (128) or r / 4 (64).
@@ -20,6 +20,8 @@
 // Measured: four llama-3-8b layers around attention, 301 rows, int8: 5101 -> 1064 us with tiles of
 // up to 64 x 128 whose weights every 64 rows widened again, -> 739 us with panels, -> 692 with the
 // gate in the panel and widening spread over its products.
+// 4 bits, in the same four layers, 196 rows: 932 -> 662 us with panels and the gate in them, 841 rows
+// (widened for the library before) 2018 -> 1789.
 // Widening 28672 x 4096: 61 us (5.8 TB/s).
 
 #include "gemm_panel_q.h"
@@ -239,14 +241,9 @@ __global__ __launch_bounds__(256) void widen_weight_kernel(
   }
 }
 
-// Tiles by how many blocks there are to fill 256 CUs with (us of what is chosen and the
-// next best; columns x inputs 6144 x 4096, 4096 x 4096, 28672 x 4096, 4096 x 14336):
-//   4 bits, 100 rows: 32x64 24.5 (64x64 23.9), 18.4 (23.4), 64x128 53, 32x64 56.4 (74.7)
-//         301 rows: 64x128 34.1, 32x64 31.2 (33.2), 64x128 123, 32x64 101 (107)
-//         700 rows: 64x128 77, 48.5, 247, 167
-//   int8, small matrices of short K (64x64, and 32x64 where fewer, | panels): 2048 x 2048, 100
-//         rows 10.3 | 10.2, 256 rows 10.5 | 12.3; 3072 x 2048, 128 rows 10.5 | 12.0, 301 rows
-//         12.6 | 12.8, 384 rows 15.5 | 13.2
+// Tiles for small matrices, which panels have nothing to share over (int8: 64x64, and 32x64 where
+// fewer; 4 bits: 32x64).  us, tiles | panels, columns x inputs: int8 2048 x 2048, 100 rows 10.3 | 10.2,
+// 256 rows 10.5 | 12.3; 3072 x 2048, 128 rows 10.5 | 12.0, 301 rows 12.6 | 12.8, 384 rows 15.5 | 13.2
 template <int QB>
 void launch_block(__hip_bfloat16* y, const __hip_bfloat16* x, const unsigned char* w,
                   const float* scale, int M, int N, int K, hipStream_t stream) {
@@ -254,12 +251,10 @@ void launch_block(__hip_bfloat16* y, const __hip_bfloat16* x, const unsigned cha
   hipLaunchKernelGGL((gemm_block_q_kernel<QB, DEPTH, BM, BN, WM, WN, ST>),                   \
                      dim3(((M + BM - 1) / BM * (N / BN) + 7) / 8 * 8), dim3(WM * WN * 64), 0, \
                      stream, y, x, w, scale, M, N, K)
-  const long wide = (M + 63L) / 64 * (N / 128);   // blocks of 64x128
   if constexpr (QB == 4) {
-    if (wide >= 230) GO(128, 64, 128, 1, 4, 3);
-    else GO(128, 32, 64, 1, 4, 3);
+    GO(128, 32, 64, 1, 4, 3);
   } else {
-    if (wide >= 150) GO(128, 64, 64, 1, 4, 2);
+    if ((M + 63L) / 64 * (N / 128) >= 150) GO(128, 64, 64, 1, 4, 2);
     else GO(128, 32, 64, 1, 4, 3);
   }
 #undef GO
@@ -280,6 +275,37 @@ constexpr Panel kPanels[] = {{5, 1, 2, .232f, .423f}, {5, 2, 2, .347f, .598f},
                              {6, 2, 2, .373f, .648f}, {8, 1, 2, .319f, .551f},
                              {8, 2, 2, .582f, .784f}, {8, 2, 1, .482f, .482f},
                              {10, 2, 1, .550f, .550f}, {10, 4, 1, .985f, .985f}};
+
+// Panels for 4 bits, likewise, over 1800 times (eleven matrices, 65 to 1000 rows; 6 % rms; the choice
+// is 0.5 % off the fastest in the mean): weights are a quarter of what x is in LDS, so that panels of
+// few rows of x and many columns pay, and two workgroups a CU, whose products hide the scaling of
+// each other's sums.  us, tiles of up to 64 x 128 before | panels: 28672 x 4096, 128 rows 53 | 46, 196
+// 97 | 67, 301 125 | 82, 600 229 | 161; 4096 x 14336, 80 rows 51 | 23, 196 72 | 43, 301 102 | 51; 6144 x
+// 4096, 196 rows 32 | 27, 420 49 | 36; 4096 x 4096, 80 rows 17.1 | 12.9, 301 31 | 23; 1024 x 4096, 65 rows
+// 17 | 8.2.
+constexpr Panel kPanels4[] = {
+    {5, 1, 2, .259f, .515f}, {5, 2, 2, .426f, .693f}, {6, 2, 2, .451f, .725f},
+    {8, 1, 2, .350f, .619f}, {8, 2, 2, .623f, .867f}, {5, 4, 2, .679f, 1.076f},
+    {4, 2, 2, .371f, .628f}};
+
+float panel4_us(const Panel& p, int M, int N, int K, int parts) {
+  const int blocks = (M + p.tm * 16 - 1) / (p.tm * 16) * (N / (p.tn * 64));
+  const int wgs = (blocks + 7) / 8 * parts;   // of an XCD
+  const int tiles = (K / 128 + parts - 1) / parts * 2, round = 32 * p.per_cu, left = wgs % round;
+  float us = 4.3f + wgs / round * (p.full * tiles);
+  if (left > 0) us += (left > 32 ? p.full : p.one) * tiles;
+  if (parts > 1) us += 1.8f + 1.65e-6f * parts * M * N;
+  return us;
+}
+
+// 32 x 64 tiles of 4 bits while they are at most two a CU and K is short: us, tiles | panels, 768 x 768,
+// 301 rows 4.9 | 6.6; 4096 x 1024, 65 rows 6.0 | 8.3, 160 7.7 | 8.0, 301 (640 tiles) 10.1 | 8.4; 2048 x
+// 2048, 65 rows 9.1 | 8.1, 224 9.5 | 11.4, 384 12.5 | 12.4; 512 x 2048, 301 rows 9.3 | 8.4, 700 9.5 | 10.7
+float tiles4_us(int M, int N, int K) {
+  const int all = ((M + 31) / 32 * (N / 64) + 7) / 8;   // of an XCD
+  if (K > 2048 || all > 64) return 1e30f;
+  return all <= 32 ? 2.4f + K / 128 * 0.44f : 2.6f + K / 128 * 0.62f;
+}
 
 float panel_us(const Panel& p, int M, int N, int K, int parts) {
   const int blocks = (M + p.tm * 16 - 1) / (p.tm * 16) * (N / (p.tn * 64));
@@ -307,10 +333,40 @@ bool small_tiles(int M, int N, int K) {
 
 }  // namespace
 
+namespace {
+
+// The same for 4 bits; a gated one (N of both halves) has whole K and even panels
+int panel4_plan(int M, int N, int K, bool gated, float& least) {
+  int plan = gated ? 0 : 1;
+  least = gated ? 1e30f : tiles4_us(M, N, K);
+  for (int i = 0; i < (int)(sizeof(kPanels4) / sizeof(kPanels4[0])); ++i) {
+    const Panel& p = kPanels4[i];
+    if (N % (p.tn * 64) != 0 || (gated && p.tn % 2 != 0)) continue;
+    // a panel's rows of x and of W lie inside 4 GB
+    if (32L * p.tm * K >= 1L << 32 || 32L * p.tn * K >= 1L << 32) continue;
+    for (int parts = 1; parts <= (gated ? 1 : 8) && (parts == 1 || K / parts >= 512); ++parts) {
+      const int depth = (K / 128 + parts - 1) / parts;
+      if ((K / 128 + depth - 1) / depth != parts) continue;   // no part is empty
+      const float us = panel4_us(p, M, N, K, parts);
+      if (us < least) {
+        plan = (i + 1) << 8 | parts;
+        least = us;
+      }
+    }
+  }
+  return plan;
+}
+
+}  // namespace
+
 // Which panel, and how many workgroups K is cut over (each leaves a part of the result in f32),
 // of eight tiles of 64 inputs at least: (panel << 8 | parts), or 1 where tiles of
 // gemm_block_q_kernel do (small_tiles).  A function of shapes.
-int gemm_panel_plan(int M, int N, int K) {
+int gemm_panel_plan(int M, int N, int K, int qbits) {
+  if (qbits == 4) {
+    float us;
+    return panel4_plan(M, N, K, false, us);
+  }
   if (small_tiles(M, N, K)) return 1;
   int plan = 0;
   float least = 0.f;
@@ -337,23 +393,30 @@ void launch_gemm_merge(__hip_bfloat16* y, const float* part, long plane, int par
 namespace {
 
 // Without GATED: N columns of y; with it N / 2, of a plan for N with whole K and even panels
-template <bool GATED>
+template <int QB, bool GATED>
 void launch_panel(__hip_bfloat16* y, float* part, const __hip_bfloat16* x, const unsigned char* w,
                   const float* scale, int M, int N, int K, int plan, hipStream_t stream) {
+  constexpr int kGroup = QB == 4 ? 128 : 64;
   const int parts = plan & 255, panel = (plan >> 8) - 1;
-  const int depth = (K / 64 + parts - 1) / parts * 64;
-#define GO(I, STAGES)                                                                         \
-  case I: {                                                                                   \
-    constexpr Panel p = kPanels[I];                                                           \
-    constexpr bool gate = GATED && p.tn % 2 == 0;                                             \
-    const int blocks = (M + p.tm * 16 - 1) / (p.tm * 16) * (N / (p.tn * 64));                 \
-    hipLaunchKernelGGL((gemm_panel::gemm_panel_q_kernel<p.tm, p.tn, STAGES, p.per_cu, gate>), \
-                       dim3((blocks + 7) / 8 * 8, parts), dim3(64 * gemm_panel::kWaves), 0,   \
-                       stream, y, part, x, w, scale, M, GATED ? N / 2 : N, K, depth);         \
-    break;                                                                                    \
+  const int depth = (K / kGroup + parts - 1) / parts * kGroup;
+#define GO(I, STAGES)                                                                             \
+  case I: {                                                                                       \
+    constexpr Panel p = QB == 4 ? kPanels4[I < 7 ? I : 0] : kPanels[I];                           \
+    constexpr bool gate = GATED && p.tn % 2 == 0;                                                 \
+    const int blocks = (M + p.tm * 16 - 1) / (p.tm * 16) * (N / (p.tn * 64));                     \
+    hipLaunchKernelGGL((gemm_panel::gemm_panel_q_kernel<QB, p.tm, p.tn, STAGES, p.per_cu, gate>), \
+                       dim3((blocks + 7) / 8 * 8, parts), dim3(64 * gemm_panel::kWaves), 0,       \
+                       stream, y, part, x, w, scale, M, GATED ? N / 2 : N, K, depth);             \
+    break;                                                                                        \
   }
-  switch (panel) {
-    GO(0, 5) GO(1, 4) GO(2, 4) GO(3, 4) GO(4, 3) GO(5, 5) GO(6, 4) GO(7, 4)
+  if constexpr (QB == 4) {
+    switch (panel) {
+      GO(0, 5) GO(1, 5) GO(2, 4) GO(3, 4) GO(4, 3) GO(5, 4) GO(6, 6)
+    }
+  } else {
+    switch (panel) {
+      GO(0, 5) GO(1, 4) GO(2, 4) GO(3, 4) GO(4, 3) GO(5, 5) GO(6, 4) GO(7, 4)
+    }
   }
 #undef GO
   if (parts > 1) launch_gemm_merge(y, part, (long)M * N, parts, false, stream);
@@ -361,31 +424,44 @@ void launch_panel(__hip_bfloat16* y, float* part, const __hip_bfloat16* x, const
 
 }  // namespace
 
-// M >= 1, N % 128 == 0, K % 128 == 0; int8: plan of gemm_panel_plan, its parts [parts, M, N]
+// M >= 1, N % 128 == 0, K % 128 == 0; plan of gemm_panel_plan, its parts [parts, M, N]
 void launch_gemm_block_q(__hip_bfloat16* y, float* part, const __hip_bfloat16* x,
                          const unsigned char* w, const float* scale, int qbits, int M, int N,
                          int K, int plan, hipStream_t stream) {
-  if (qbits == 4)
-    launch_block<4>(y, x, w, scale, M, N, K, stream);
+  if (plan > 1 && qbits == 4)
+    launch_panel<4, false>(y, part, x, w, scale, M, N, K, plan, stream);
   else if (plan > 1)
-    launch_panel<false>(y, part, x, w, scale, M, N, K, plan, stream);
+    launch_panel<8, false>(y, part, x, w, scale, M, N, K, plan, stream);
+  else if (qbits == 4)
+    launch_block<4>(y, x, w, scale, M, N, K, stream);
   else
     launch_block<8>(y, x, w, scale, M, N, K, stream);
 }
 
-// The plan of a gated int8 product of M > 64 rows with [2 N, K], or 0 where the plain one's cuts K or
-// takes columns one tile a wave: the gate is not in the panel then.
-int gemm_panel_gated_plan(int M, int N, int K) {
+// The plan of a gated product of M > 64 rows with [2 N, K], or 0 where the plain one and a launch for
+// the gate are faster.  int8: where the plain one's plan cuts K or takes columns one tile a wave, as
+// the gate is not in the panel then; 4 bits: the best panel that can take it, against those two (the
+// gate 2.5 us and 4 bytes read, 2 written an output).
+int gemm_panel_gated_plan(int M, int N, int K, int qbits) {
   if (M <= 64 || N % 128 != 0 || K % 128 != 0 || (long)(N + 128) * K >= 1L << 32) return 0;
-  const int plan = gemm_panel_plan(M, 2 * N, K);
+  if (qbits == 4) {
+    float us, plain;
+    const int plan = panel4_plan(M, 2 * N, K, true, us);
+    panel4_plan(M, 2 * N, K, false, plain);
+    return us < plain + 2.5f + 1.2e-6f * M * N ? plan : 0;
+  }
+  const int plan = gemm_panel_plan(M, 2 * N, K, 8);
   return plan > 1 && (plan & 255) == 1 && kPanels[(plan >> 8) - 1].tn % 2 == 0 ? plan : 0;
 }
 
-// y [M, N] = silu(x Wg^T) * (x Wu^T), W = [Wg; Wu] in int8, plan of gemm_panel_gated_plan
+// y [M, N] = silu(x Wg^T) * (x Wu^T), W = [Wg; Wu] rounded, plan of gemm_panel_gated_plan
 void launch_gemm_panel_gated(__hip_bfloat16* y, const __hip_bfloat16* x, const unsigned char* w,
-                             const float* scale, int M, int N, int K, int plan,
+                             const float* scale, int qbits, int M, int N, int K, int plan,
                              hipStream_t stream) {
-  launch_panel<true>(y, nullptr, x, w, scale, M, 2 * N, K, plan, stream);
+  if (qbits == 4)
+    launch_panel<4, true>(y, nullptr, x, w, scale, M, 2 * N, K, plan, stream);
+  else
+    launch_panel<8, true>(y, nullptr, x, w, scale, M, 2 * N, K, plan, stream);
 }
 
 // total = N * K, K % 128 == 0

@@ -1,4 +1,4 @@
-// Products of 65 to some hundreds of rows with int8 weights (see gemm_block_q.hip): panels of
+// Products of 65 to some hundreds of rows with rounded weights (see gemm_block_q.hip): panels of
 // 16 TM rows of x against 64 TN columns of W.  The waves lie along the columns, so that every
 // weight of a panel is widened by one wave only, once for all its rows.
 //
@@ -17,9 +17,19 @@
 // the wave and half of the next (0..3, 12..15, 20..27 | 4..11, 16..19, 28..31): chunks lie so that these
 // are in different banks (half of all LDS cycles were conflicts).
 //
+// 4 bits: a nibble less its offset becomes a float in one instruction (v_cvt_off_f32_i4, of two's
+// complement), whose upper half is all of it, so that there is no offset to take from the sums (8 + n/2
+// by bit patterns, cheaper by a third, needs the sum of x of every row and group).  Sums of a group of 128
+// inputs are apart: its first product begins them and a row late each is multiplied by its column's
+// scale into the whole ones, four instructions for every four products of 16 x 16 x 32, beside those
+// that widen.  With two workgroups a CU they hide behind the other's products: 28672 x 4096, 196
+// rows 0.69 PFLOP/s, 900 rows 0.88 (int8 0.76, 0.98).  W's rows of a tile are 32 bytes.
+//
 // Gated, half of a wave's columns are gates and half what they multiply, and the launch that did
 // that (6 us at 301 x 28672) with its reads of the product falls away.
 #pragma once
+
+#include <type_traits>
 
 #include "block_gemm.h"
 #include "moe_tiles.h"
@@ -30,26 +40,52 @@ using block_gemm::bf16x8_t;
 using block_gemm::f32x4_t;
 
 typedef __attribute__((ext_vector_type(4))) unsigned int u32x4_t;
+typedef __attribute__((ext_vector_type(2))) unsigned int u32x2_t;
 // scales start at any float
 typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4_any_t;
 
 constexpr int kDepth = 64;    // inputs of a tile
 constexpr int kWaves = 4;     // along N
 
-// grid (tiles of y, parts of K); part [parts, M, N] (gridDim.y > 1); depth: inputs of a part
+// A wave's loads of n tiles, of `each` and, for 4 bits, the scales of a group of two with its
+// first; half: of the first tile
+template <int QB> constexpr int loads_of(int each, int half, int n) {
+  return n * each + (QB == 4 ? (n + 1 - half % 2) / 2 : 0);
+}
+
+// The low nibble of byte d as a whole number of two's complement, over 16.  (VALU only, and all of
+// the result's bits are written: nothing for the compiler to wait for.)
+DEVINLINE unsigned nibble(unsigned v, int d) {
+  unsigned f;
+#define CVT(B)                                                                      \
+  asm("v_cvt_off_f32_i4_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_" #B \
+      : "=v"(f) : "v"(v))
+  if (d == 0) CVT(0);
+  else if (d == 1) CVT(1);
+  else if (d == 2) CVT(2);
+  else CVT(3);
+#undef CVT
+  return f;
+}
+
+// grid (tiles of y, parts of K); part [parts, M, N] (gridDim.y > 1); depth: inputs of a part (4
+// bits: whole groups of 128)
 // PER_CU: workgroups that share a CU.  GATED: N outputs of 2 N rows of W, K in one part.
-template <int TM, int TN, int STAGES, int PER_CU, bool GATED>
+template <int QB, int TM, int TN, int STAGES, int PER_CU, bool GATED>
 __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
     __hip_bfloat16* __restrict__ y,         // [M, N]
     float* __restrict__ part,
     const __hip_bfloat16* __restrict__ x,   // [M, K]
-    const unsigned char* __restrict__ w,    // int8 [N, K] | [2 N, K]
-    const float* __restrict__ scale,        // [N] | [2 N]
+    const unsigned char* __restrict__ w,    // int8 [N, K] | [2 N, K]; 4 bits [.., K / 2]
+    const float* __restrict__ scale,        // [N] | [2 N]; 4 bits [.., K / 128]
     const int M, const int N, const int K, const int depth) {
   constexpr int BM = TM * 16, BN = TN * 16 * kWaves;
-  constexpr int X_BYTES = BM * kDepth * 2, W_BYTES = BN * kDepth, STAGE = X_BYTES + W_BYTES;
-  constexpr int X_LOADS = BM / 8, W_LOADS = BN / 16;   // 1 KB each: 8 rows of x, 16 of W
-  constexpr int X_PASS = (X_LOADS + kWaves - 1) / kWaves, W_PASS = W_LOADS / kWaves;
+  constexpr int W_ROW = kDepth * QB / 8, WL = W_ROW / 16;   // bytes and lanes of a W row
+  constexpr int X_BYTES = BM * kDepth * 2, W_BYTES = BN * W_ROW;
+  constexpr int STAGE = X_BYTES + W_BYTES + (QB == 4 ? BN * 4 : 0);
+  constexpr int X_LOADS = BM / 8, W_LOADS = W_BYTES / 1024;   // 1 KB each
+  constexpr int X_PASS = (X_LOADS + kWaves - 1) / kWaves;
+  constexpr int W_PASS = (W_LOADS + kWaves - 1) / kWaves;
   constexpr int LOADS = X_PASS + W_PASS;
   constexpr int AHEAD = 3;                // fragments of x on their way
   constexpr bool SPREAD = TM >= 8;        // widening over the products
@@ -67,13 +103,14 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
   const int k0 = blockIdx.y * depth;
   const int m0 = id % m_tiles * BM, n0 = id / m_tiles * COLS;
   const int tiles = min(depth, K - k0) / kDepth;
-  const int start = id / m_tiles % tiles;
+  const int start = QB == 4 ? id / m_tiles % (tiles / 2) * 2 : id / m_tiles % tiles;
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, quad = lane >> 4;
 
-  auto w_turn = [](int r) { return SPREAD ? -(r / 4) & 3 : r / 4 % 4; };
+  // (4 bits: the reads of a wave are one run of bytes)
+  auto w_turn = [](int r) { return QB == 4 ? 0 : SPREAD ? -(r / 4) & 3 : r / 4 % 4; };
   // (where there are fewer loads than waves some are made twice: all waves wait alike; rows
   // of a panel are found by 32 bits, see gemm_panel_plan)
   unsigned x_off[X_PASS], w_off[W_PASS];
@@ -83,15 +120,21 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
     const int at = (lane % 8) ^ (r / 2 % 8);   // large: of the chunks 0 2 4 6 1 3 5 7
     x_off[p] = (unsigned)min(r, M - 1 - m0) * (K * 2u) + (SPREAD ? at % 4 * 2 + at / 4 : at) * 16;
   }
+  auto w_row = [&](int r) {   // of W from n0 on, for row r of the panel's
+    const int own = r / (TN * 16), in = r % (TN * 16), half = in / (OUT * 16);
+    return (unsigned)(half * N + own * (OUT * 16) + in % (OUT * 16));
+  };
 #pragma unroll
   for (int p = 0; p < W_PASS; ++p) {
-    const int r = (p * kWaves + wave) * 16 + lane / 4;
-    const int own = r / (TN * 16), in = r % (TN * 16), half = in / (OUT * 16);
-    w_off[p] = (unsigned)(half * N + own * (OUT * 16) + in % (OUT * 16)) * K +
-               ((lane % 4) ^ w_turn(r)) * 16;
+    const int r = (p * kWaves + wave) % W_LOADS * (64 / WL) + lane / WL;
+    w_off[p] = w_row(r) * (unsigned)(K * QB / 8) + ((lane % WL) ^ w_turn(r)) * 16;
   }
   const auto x_from = block_gemm::resource(x + (long)m0 * K + k0);
-  const auto w_from = block_gemm::resource(w + (long)n0 * K + k0);
+  const auto w_from = block_gemm::resource(w + ((long)n0 * K + k0) * QB / 8);
+  unsigned s_off = 0;
+  if constexpr (QB == 4) s_off = w_row(wave % TN * 64 + lane) * (unsigned)(K / 128 * 4);
+  const auto s_from =
+      block_gemm::resource(QB == 4 ? scale + (long)n0 * (K / 128) + k0 / 128 : scale);
   // load p of a tile (past the last tile it is the last one again)
   auto load = [&](int buf, int tile, int p) {
     char* to = lds + buf * STAGE;
@@ -100,9 +143,11 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
     if (p < X_PASS)
       block_gemm::load_lds(to + (p * kWaves + wave) % X_LOADS * 1024, x_from, x_off[p],
                            tile * (kDepth * 2));
+    else if (p < LOADS)
+      block_gemm::load_lds(to + X_BYTES + ((p - X_PASS) * kWaves + wave) % W_LOADS * 1024, w_from,
+                           w_off[p < LOADS ? p - X_PASS : 0], tile * W_ROW);
     else
-      block_gemm::load_lds(to + X_BYTES + ((p - X_PASS) * kWaves + wave) * 1024, w_from,
-                           w_off[p - X_PASS], tile * kDepth);
+      block_gemm::load_lds4(to + X_BYTES + W_BYTES + wave % TN * 256, s_from, s_off, tile / 2 * 4);
   };
 
   f32x4_t acc[TM][TN];
@@ -110,6 +155,8 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = f32x4_t{};
+  // 4 bits: sums of a group, ahead of its scales
+  f32x4_t part_sum[QB == 4 ? TM : 1][QB == 4 ? TN : 1], group_scale[QB == 4 ? TN : 1];
 
   // A lane's 16 weights of a column (chunk quad of its row) are its inputs of two matrix steps,
   // and x is read to match.
@@ -121,10 +168,18 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
   };
   auto w_chunk = [&](const char* at, int j) {
     const int r = (wave * TN + j) * 16 + col;
-    return *reinterpret_cast<const u32x4_t*>(at + X_BYTES + r * kDepth +
+    if constexpr (QB == 4)
+      return *reinterpret_cast<const u32x2_t*>(at + X_BYTES + r * W_ROW + quad * 8);
+    else
+      return *reinterpret_cast<const u32x4_t*>(at + X_BYTES + r * W_ROW +
                                                (quad ^ w_turn(r)) * 16);
   };
-  auto unpack = [&](const u32x4_t& c, int s, int d) {   // pair d of a column's weights of step s
+  using Chunk = decltype(w_chunk(lds, 0));
+  auto unpack = [&](const Chunk& c, int s, int d) {   // pair d of a column's weights of step s
+    if constexpr (QB == 4) {
+      const unsigned eight = c[s] ^ 0x88888888u;   // n - 8 in two's complement
+      return __builtin_amdgcn_perm(nibble(eight >> 4, d), nibble(eight, d), 0x07060302);
+    }
     const unsigned four = c[2 * s + d / 2] >> (d % 2 * 16);
     const float a = (float)(signed char)(four & 0xff);
     const float b = (float)(signed char)((four >> 8) & 0xff);
@@ -135,10 +190,10 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
 #pragma unroll
   for (int s = 0; s < STAGES - 1; ++s)
 #pragma unroll
-    for (int p = 0; p < LOADS; ++p) load(s, s, p);
-  block_gemm::wait_loads<(STAGES - 2) * LOADS>();
+    for (int p = 0; p < loads_of<QB>(LOADS, s, 1); ++p) load(s, s, p);
+  block_gemm::wait_loads<loads_of<QB>(LOADS, 1, STAGES - 2)>();
   block_gemm::meet();
-  u32x4_t c[TN];
+  Chunk c[TN];
   u32x4_t wf[2][TN];
   bf16x8_t xf[AHEAD];
 #pragma unroll
@@ -150,8 +205,16 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
 #pragma unroll
   for (int q = 0; q < AHEAD; ++q) xf[q] = x_frag(lds, q / TM, q % TM);
 
+  auto finish = [&](int i, int j) {
+    if constexpr (QB == 4) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        acc[i][j][r] = __builtin_fmaf(group_scale[j][r], part_sum[i][j][r], acc[i][j][r]);
+    }
+  };
   int buf = 0;
-  for (int t = 0; t < tiles; ++t) {
+  auto turn = [&](int t, auto which) {
+    constexpr int HALF = decltype(which)::value;   // 4 bits: of a group
     const int after = buf + 1 == STAGES ? 0 : buf + 1, before = buf == 0 ? STAGES - 1 : buf - 1;
     const char* here = lds + buf * STAGE;
     const char* there = lds + after * STAGE;
@@ -163,14 +226,21 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
       const int s = q / TM, i = q % TM;
       if (q == TM) {
         // the next tile is here, and all have read the one before this one
-        block_gemm::wait_loads<(STAGES - 3) * LOADS>();
+        block_gemm::wait_loads<loads_of<QB>(LOADS, HALF, STAGES - 3)>();
         block_gemm::meet();
 #pragma unroll
         for (int j = 0; j < TN; ++j) c[j] = w_chunk(there, j);
       }
+      constexpr int ASKED = loads_of<QB>(LOADS, HALF + STAGES - 1, 1);
 #pragma unroll
-      for (int p = 0; p < LOADS; ++p)
-        if (s == 1 && p * TM / LOADS == i) load(before, t + STAGES - 1, p);
+      for (int p = 0; p < ASKED; ++p)
+        if (s == 1 && p * TM / ASKED == i) load(before, t + STAGES - 1, p);
+      if constexpr (QB == 4 && HALF == 0)
+        if (q == 0)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            group_scale[j] = *reinterpret_cast<const f32x4_t*>(
+                here + X_BYTES + W_BYTES + ((wave * TN + j) * 16 + quad * 4) * 4);
       const int f = q + AHEAD;
       xr[f] = f < 2 * TM ? x_frag(here, f / TM, f % TM)
                          : x_frag(there, (f - 2 * TM) / TM, (f - 2 * TM) % TM);
@@ -185,8 +255,16 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
       }
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            __builtin_bit_cast(bf16x8_t, wf[s][j]), xr[q], acc[i][j], 0, 0, 0);
+        if constexpr (QB == 4) {
+          part_sum[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8_t, wf[s][j]), xr[q],
+              HALF == 0 && s == 0 ? f32x4_t{} : part_sum[i][j], 0, 0, 0);
+          // a row late: its sums are there
+          if (HALF == 1 && s == 1 && i > 0) finish(i - 1, j);
+        } else {
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8_t, wf[s][j]), xr[q], acc[i][j], 0, 0, 0);
+        }
         const int at = i * TN + j - (s == 0 ? 0 : LATE);
         if (SPREAD && at >= 0) {
 #pragma unroll
@@ -199,7 +277,18 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
     }
 #pragma unroll
     for (int q = 0; q < AHEAD; ++q) xf[q] = xr[2 * TM + q];
+    if constexpr (QB == 4 && HALF == 1)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) finish(TM - 1, j);
     buf = after;
+  };
+  if constexpr (QB == 4) {
+    for (int t = 0; t < tiles; t += 2) {
+      turn(t, std::integral_constant<int, 0>{});
+      turn(t + 1, std::integral_constant<int, 1>{});
+    }
+  } else {
+    for (int t = 0; t < tiles; ++t) turn(t, std::integral_constant<int, 0>{});
   }
   block_gemm::wait_loads<0>();   // LDS is not given back ahead of them
 
@@ -207,9 +296,11 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
 #pragma unroll
   for (int j = 0; j < OUT; ++j) {
     const int n = n0 + (wave * OUT + j) * 16 + quad * 4;
-    const f32x4_t s = *reinterpret_cast<const f32x4_any_t*>(scale + n);
-    f32x4_t su{};
-    if constexpr (GATED) su = *reinterpret_cast<const f32x4_any_t*>(scale + N + n);
+    f32x4_t s{16.f, 16.f, 16.f, 16.f}, su = s;   // (4 bits: what `nibble` leaves)
+    if constexpr (QB == 8) {
+      s = *reinterpret_cast<const f32x4_any_t*>(scale + n);
+      if constexpr (GATED) su = *reinterpret_cast<const f32x4_any_t*>(scale + N + n);
+    }
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const int m = m0 + i * 16 + col;

@@ -326,6 +326,50 @@ def test_int8_panels(m, n, k, panel, parts):
     _check(ops.linear_quant(x, wq, scale, 8), x.double() @ exact, x.double().abs() @ exact.abs())
 
 
+def _exact4(wq, scale):
+    q = torch.stack([wq & 0xF, wq >> 4], dim=2).view(wq.shape[0], -1, 128).double() - 8.0
+    return (q * scale.double()[:, :, None]).view(wq.shape[0], -1).t().contiguous()
+
+
+# the same for 4 bits, one group and parts of unequal numbers of groups among them
+@pytest.mark.parametrize(("m", "n", "k", "panel", "parts"), [
+    (257, 4096, 128, 0, 1), (65, 128, 2176, 0, 4), (65, 28672, 128, 1, 1), (65, 6144, 4224, 1, 5),
+    (321, 8192, 128, 2, 1), (161, 2048, 6272, 2, 7), (161, 6144, 128, 3, 1), (161, 2048, 2176, 3, 4),
+    (511, 16384, 384, 4, 1), (97, 8192, 8192, 4, 8), (129, 28672, 128, 5, 1), (129, 6144, 6272, 5, 5),
+    (257, 6144, 2176, 6, 1), (161, 2048, 4224, 6, 5)])
+def test_4_bit_panels(m, n, k, panel, parts):
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    assert m <= ops._quant_rows(4, n, k)
+    assert ops._C.gemm_panel_plan(m, n, k, 4) == (panel + 1) << 8 | parts
+    x, w = _x(m, k, 30), _x(n, k, 31)
+    w[0], w[n // 2:n // 2 + 2] = 0.0, 8.0     # least scales; the largest weight
+    wq, scale = ops.quantize_weight(w, 4)
+    wq[n // 2 + 1] = 0                        # -8, which rounding to the nearest does not give
+    exact = _exact4(wq, scale)
+    _check(ops.linear_quant(x, wq, scale, 4), x.double() @ exact, x.double().abs() @ exact.abs())
+
+
+@pytest.mark.parametrize(("m", "n", "k", "panel"), [
+    (65, 14336, 128, 1), (321, 4096, 384, 2), (511, 3072, 128, 4), (301, 14336, 4096, 5),
+    (257, 8192, 128, 5), (161, 3072, 384, 6), (65, 1024, 8192, None)])
+def test_4_bit_gated_panels(m, n, k, panel):
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    plan = ops._C.gemm_panel_gated_plan(m, n, k, 4)
+    assert plan == (0 if panel is None else (panel + 1) << 8 | 1)
+    x, w = _x(m, k, 32), _x(2 * n, k, 33) / k ** 0.5
+    wq, scale = ops.quantize_weight(w, 4)
+    got = ops.gated_quant(x, wq, scale, 4)
+    if panel is None:
+        assert got is None
+        return
+    g, u = (x.double() @ _exact4(wq, scale)).chunk(2, dim=1)
+    _check(got, torch.nn.functional.silu(g) * u, 30 * (1 + g.abs()) * (1 + u.abs()))
+
+
 # every panel that takes the gate in, whole and with rows missing; the last is refused: K is cut
 @pytest.mark.parametrize(("m", "n", "k", "panel"), [
     (65, 14336, 384, 1), (321, 4096, 128, 2), (511, 8192, 128, 4), (97, 14336, 384, 5),

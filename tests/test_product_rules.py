@@ -23,6 +23,28 @@ def test_int8_panels_lie_inside_32_bits(n, k):
         assert 16 * rows * k * 2 < 1 << 32 and 64 * cols * k < 1 << 32
 
 
+# the same of 4 bits
+PANELS4 = [(5, 1), (5, 2), (6, 2), (8, 1), (8, 2), (5, 4), (4, 2)]
+
+
+@pytest.mark.parametrize("k", [128, 2048, 14336, 13 << 20, (1 << 24) - 128])
+@pytest.mark.parametrize("n", [128, 512, 768, 4096, 28672])
+def test_4_bit_panels_fit(n, k):
+    """Whole columns, no part of K without a group, rows of a panel inside 32 bits; a gated
+    product's panels have both halves and all of K."""
+    for m in (65, 129, 160, 257, 300, 513, 899, 1200):
+        for plan, gated in ((ops._C.gemm_panel_plan(m, n, k, 4), False),
+                            (ops._C.gemm_panel_gated_plan(m, n // 2, k, 4), True)):
+            if plan <= 1:
+                assert plan == (0 if gated else 1) and (gated or k <= 2048)
+                continue
+            (rows, cols), parts = PANELS4[(plan >> 8) - 1], plan & 255
+            assert n % (64 * cols) == 0 and not (gated and (cols % 2 or parts > 1))
+            assert 16 * rows * k * 2 < 1 << 32 and 64 * cols * k // 2 < 1 << 32
+            groups = -(-(k // 128) // parts)
+            assert (parts - 1) * groups < k // 128 <= parts * groups
+
+
 @pytest.mark.parametrize(("m", "n", "k", "plans"), [
     # rounds of an XCD, of which counting the chip's took the slower: panel, parts of K
     (800, 1280, 8192, {(1, 4), (6, 4), (5, 3), (1, 2)}), (560, 1536, 4096, {(0, 3), (2, 3)}),

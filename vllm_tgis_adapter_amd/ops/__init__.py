@@ -362,13 +362,14 @@ def _quant_rows(qbits: int, n: int, k: int) -> int:
     rows 113 | 98, 2048 x 2048 1500 rows 23 | 28; below the line some large ones lose, but
     with weights as they are instead of rounded to bf16: 10240 x 8192 900 rows 146 | 175,
     1000 rows 190 | 180, 1200 rows 222 | 199, 14336 x 8192 900 rows 240 | 227, 1100 rows
-    254 | 279, 32000 x 2048 1000 rows 151 | 141; 4 bits 28672 x 4096 301 rows 129 | 136, 448 rows
-    176 | 157, 4096 x 14336 80 rows 58 | 67, 150 rows 78 | 72."""
+    254 | 279, 32000 x 2048 1000 rows 151 | 141; 4 bits 28672 x 4096 gated 800
+    rows 201 | 263, 1200 rows 288 | 311, 1500 rows 365 | 332, 4096 x 14336 800 rows 112 | 130, 1200
+    rows 158 | 155, 6144 x 4096 800 rows 53 | 55, 1000 rows 64 | 61, 10240 x 8192 800 rows
+    152 | 163, 1000 rows 199 | 172, 8192 x 28672 1200 rows 566 | 576, 1500 rows 721 | 635, 2048 x
+    2048 1500 rows 20 | 28."""
     if n * k <= 1 << 23:
-        return 1500 if qbits == 8 else 1000
-    if qbits == 8:
-        return 1200
-    return 320 if k < 8192 else 128
+        return 1500
+    return 1200 if qbits == 8 or n >= 16384 or k > 8192 else 900
 
 
 def linear_quant(x: torch.Tensor, wq: torch.Tensor, scales: torch.Tensor,
@@ -402,19 +403,20 @@ def linear_quant(x: torch.Tensor, wq: torch.Tensor, scales: torch.Tensor,
 
 def gated_quant(x: torch.Tensor, wq: torch.Tensor, scales: torch.Tensor,
                 qbits: int) -> torch.Tensor | None:
-    """silu(x Wg^T) * (x Wu^T) for int8 [gate; up] weights as ``quantize_weight`` makes them, where
+    """silu(x Wg^T) * (x Wu^T) for [gate; up] weights as ``quantize_weight`` makes them, where
     the product of so many rows takes the gate into its launch; None elsewhere (the caller has
     linear_quant and silu_and_mul)."""
-    if (qbits != 8 or x.dim() != 2 or x.shape[0] <= 64 or x.dtype != torch.bfloat16
+    if (qbits not in (4, 8) or x.dim() != 2 or x.shape[0] <= 64 or x.dtype != torch.bfloat16
             or not native_enabled(x) or not x.is_contiguous()):
         return None
     m, n, k = x.shape[0], wq.shape[0], x.shape[1]
-    if (n % 256 or k % 128 or m > _quant_rows(8, n, k) or wq.dtype != torch.int8
+    if (n % 256 or k % 128 or m > _quant_rows(qbits, n, k)
+            or wq.dtype != (torch.int8 if qbits == 8 else torch.uint8)
             or scales.dtype != torch.float32 or not wq.is_contiguous()
             or not scales.is_contiguous() or not _plain_tensors(x, wq)):
         return None
     out = torch.empty((m, n // 2), dtype=x.dtype, device=x.device)
-    return out if _C.gemm_q_gated(out, x, wq, scales) else None
+    return out if _C.gemm_q_gated(out, x, wq, scales, qbits) else None
 
 
 def gated_mlp_up(x: torch.Tensor, w13: torch.Tensor) -> torch.Tensor | None:
