@@ -80,6 +80,7 @@ void launch_gemm_skinny_gated(__hip_bfloat16*, float*, const __hip_bfloat16*,
                               hipStream_t);
 int gemm_panel_plan(int M, int N, int K, int qbits);
 int gemm_panel_gated_plan(int M, int N, int K, int qbits);
+int gemm_panel_few_plan(int M, int N, int K, int qbits);
 void launch_gemm_panel_gated(__hip_bfloat16*, const __hip_bfloat16*, const unsigned char*,
                              const float*, int, int, int, int, int, hipStream_t);
 void launch_gemm_block_q(__hip_bfloat16*, float*, const __hip_bfloat16*, const unsigned char*,
@@ -412,11 +413,14 @@ void gemm_q(torch::Tensor y, torch::Tensor x, torch::Tensor wq, torch::Tensor ws
   TORCH_CHECK(y.size(0) == M && y.size(1) == N);
   // rows of a block of W are found by 32 bits
   TORCH_CHECK((int64_t)128 * K < (1LL << 31));
-  if (M > 64) {
-    // both reach LDS in 16-byte pieces
-    TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
-                reinterpret_cast<uintptr_t>(wq.data_ptr()) % 16 == 0);
-    const int plan = gemm_panel_plan(M, N, K, (int)qbits);
+  // x and W reach LDS in 16-byte pieces by panels and tiles
+  const bool aligned = reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+                       reinterpret_cast<uintptr_t>(wq.data_ptr()) % 16 == 0;
+  const int plan = M > 64 ? gemm_panel_plan(M, N, K, (int)qbits)
+                   : aligned && reinterpret_cast<uintptr_t>(y.data_ptr()) % 8 == 0
+                       ? gemm_panel_few_plan(M, N, K, (int)qbits) : 0;
+  if (plan > 0) {
+    TORCH_CHECK(aligned);
     torch::Tensor part;
     launch_gemm_block_q(ptr<__hip_bfloat16>(y), stream_parts(part, x, plan & 255, (int64_t)M * N),
                         cptr<__hip_bfloat16>(x), cptr<unsigned char>(wq),
@@ -481,7 +485,7 @@ const float* optional_scales(const c10::optional<torch::Tensor>& t, int64_t qbit
   return qbits == 16 ? nullptr : t->data_ptr<float>();
 }
 
-// y = silu(x Wg^T) * (x Wu^T) for rounded [Wg; Wu] and more than 64 rows, by one launch; false:
+// y = silu(x Wg^T) * (x Wu^T) for rounded [Wg; Wu] and more than one row, by one launch; false:
 // nothing was done, the product's plan has no room for the gate
 bool gemm_q_gated(torch::Tensor y, torch::Tensor x, torch::Tensor wq, torch::Tensor wscale,
                   int64_t qbits) {
@@ -959,13 +963,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_skinny", &gemm_skinny,
         "skinny decode GEMM y = x @ w^T, M <= 64 (CDNA4 MFMA)");
   m.def("gemm_q_gated", &gemm_q_gated,
-        "gated product of many rows with rounded weights, where it is one launch", py::arg("y"),
+        "gated product with rounded weights, where it is one launch", py::arg("y"),
         py::arg("x"), py::arg("wq"), py::arg("wscale"), py::arg("qbits") = 8);
   m.def("gemm_panel_gated_plan", &gemm_panel_gated_plan, "its plan, or 0", py::arg("m"),
         py::arg("n"), py::arg("k"), py::arg("qbits") = 8);
   m.def("gemm_panel_plan", &gemm_panel_plan,
         "which panel products of many rows with rounded weights take, and parts of K (panel << 8 | "
         "parts)", py::arg("m"), py::arg("n"), py::arg("k"), py::arg("qbits") = 8);
+  m.def("gemm_panel_few_plan", &gemm_panel_few_plan, "the same up to 64 rows, 0: no panel");
   m.def("row_norm_gated", &row_norm_gated, "norm and gated product of one row (CDNA4)");
   m.def("row_norm_turn", &row_norm_turn,
         "norm, query / key / value product, rotation and cache write of one row (CDNA4)");

@@ -1,4 +1,4 @@
-// Products of more than 64 rows with rounded weights: y[m, n] = sum_k x[m, k] W[n, k],
+// Products of more than one row with rounded weights: y[m, n] = sum_k x[m, k] W[n, k],
 // W in int8 (a scale per row) or in 4 bits (offset 8, a scale per row and 128 inputs).
 //
 // The weights used to be widened by tensor ops (for 4 bits: masks, shifts, casts, a stack,
@@ -23,6 +23,8 @@
 // 4 bits, in the same four layers, 196 rows: 932 -> 662 us with panels and the gate in them, 841 rows
 // (widened for the library before) 2018 -> 1789.
 // Widening 28672 x 4096: 61 us (5.8 TB/s).
+
+#include <cmath>
 
 #include "gemm_panel_q.h"
 
@@ -335,13 +337,58 @@ bool small_tiles(int M, int N, int K) {
 
 namespace {
 
-// The same for 4 bits; a gated one (N of both halves) has whole K and even panels
+// Panels for up to 64 rows, all of them in one: columns in K parts that fill the chip, as the
+// streaming kernels' (gemm_stream.hip), but x is read by four times as many columns at a time, loads
+// need no registers and weights no turn through LDS and back.  us, streaming | panels, int8: 28672 x
+// 4096, 9 rows 27.6 | 24.5, 24 27.1 | 25.5, 40 36.8 | 27.4, 64 42.6 | 30.1; 4096 x 14336, 24 rows 17.4 |
+// 16.6, 64 28.9 | 22.7; 6144 x 4096, 64 rows 18.9 | 14.8; 4096 x 4096, 40 rows 12.4 | 9.8; 2048 x 8192, 24 rows
+// 12.2 | 9.1.  4 bits: 28672 x 4096, 24 rows 32.1 | 26.4, 64 46.6 | 29.8; 4096 x 14336, 24 rows 20.4 | 17.1,
+// 64 33.0 | 20.6; 2048 x 8192, 24 rows 13.6 | 9.8; 8192 x 28672, 8 rows 62 | 45.
+// Their times, fitted as above (to sixteen matrices, 2 to 64 rows; 4.5 % rms; the choice is 0.3 % off the
+// best in the mean): as few rows are near the bytes of W, those at least.  int8, 4 bits:
+struct FewPanel {
+  int tm, tn;
+  float one[2], full[2];
+};
+constexpr FewPanel kFewPanels[] = {
+    {2, 1, {.198f, .219f}, {.347f, .458f}}, {2, 2, {.297f, .347f}, {.619f, .597f}},
+    {3, 1, {.198f, .239f}, {.411f, .492f}}, {3, 2, {.330f, .349f}, {.658f, .617f}},
+    {4, 1, {.231f, .249f}, {.436f, .494f}}, {4, 2, {.376f, .382f}, {.644f, .646f}}};
+constexpr int kFewAt = 16;   // their number in a plan
+
+int few_plan(int M, int N, int K, int qbits, bool gated, float& least) {
+  const int q = qbits == 4, group = q ? 128 : 64;
+  const float read = (q ? 0.269f * 0.5e-6f : 0.158f * 1e-6f) * N * K;
+  int plan = 0;
+  least = 1e30f;
+  for (int i = 0; i < (int)(sizeof(kFewPanels) / sizeof(kFewPanels[0])); ++i) {
+    const FewPanel& p = kFewPanels[i];
+    if (16 * p.tm < M || N % (p.tn * 64) != 0) continue;
+    for (int parts = 1; parts <= (gated ? 1 : 8) && (parts == 1 || K / parts >= 512); ++parts) {
+      const int depth = (K / group + parts - 1) / parts;
+      if ((K / group + depth - 1) / depth != parts) continue;   // no part is empty
+      const int wgs = (N / (p.tn * 64) + 7) / 8 * parts, left = wgs % 64;   // of an XCD
+      const int tiles = depth * (group / 64);
+      float work = wgs / 64 * p.full[q] * tiles;
+      if (left > 0) work += (left > 32 ? p.full[q] : p.one[q]) * tiles;
+      float us = 3.2f + sqrtf(sqrtf(work * work * work * work + read * read * read * read));
+      if (parts > 1) us += 1.75f + (q ? 2.7e-6f : 2.5e-6f) * parts * M * N;
+      if (us < least) {
+        plan = (kFewAt + i + 1) << 8 | parts;
+        least = us;
+      }
+    }
+  }
+  return plan;
+}
+
+// The same for 4 bits; a gated one (N of both halves) has whole K
 int panel4_plan(int M, int N, int K, bool gated, float& least) {
   int plan = gated ? 0 : 1;
   least = gated ? 1e30f : tiles4_us(M, N, K);
   for (int i = 0; i < (int)(sizeof(kPanels4) / sizeof(kPanels4[0])); ++i) {
     const Panel& p = kPanels4[i];
-    if (N % (p.tn * 64) != 0 || (gated && p.tn % 2 != 0)) continue;
+    if (N % (p.tn * 64) != 0) continue;
     // a panel's rows of x and of W lie inside 4 GB
     if (32L * p.tm * K >= 1L << 32 || 32L * p.tn * K >= 1L << 32) continue;
     for (int parts = 1; parts <= (gated ? 1 : 8) && (parts == 1 || K / parts >= 512); ++parts) {
@@ -387,44 +434,70 @@ int gemm_panel_plan(int M, int N, int K, int qbits) {
   return plan;
 }
 
+// The plan of a product of up to 64 rows by a panel, 0: the streaming kernels, which are as fast or
+// faster for small matrices of short K and, in int8, up to 11 rows (us, streaming | panels: 33 rows,
+// int8 4096 x 1024 6.2 | 7.2, 2048 x 2048 7.5 | 7.2, 8192 x 1024 9.3 | 6.5; 17 rows 4096 x 4096 8.7 | 8.8, 4
+// bits 8.3 | 9.4, 16384 x 2048 9.7 | 10.1, 4 bits 13.1 | 10.5; 9 rows 6144 x 4096 9.8 | 10.4, 4 bits 10.4 |
+// 11.3; 4 bits 2048 x 8192, 2 rows 9.9 | 9.1, 3584 x 8192 12.8 | 14.0, int8 2048 x 8192 8.3 | 8.5; int8 57344 x 8192, 8 rows 82 | 90, 14 rows
+// 101 | 93, 8192 x 28672, 2 rows 52 | 46).
+int gemm_panel_few_plan(int M, int N, int K, int qbits) {
+  const long size = (long)N * K;
+  bool takes;
+  if (M < 2 || M > 64) takes = false;
+  else if (M > 32) takes = K >= 2048 || size >= 8000000;
+  else if (qbits == 4 && M > 16) takes = K >= 8192 || size >= 20000000;
+  else if (qbits == 4)
+    takes = (K >= 8192 && (N <= 2048 || size >= 50000000)) || (M > 8 && size >= 100000000);
+  else if (M > 16) takes = K >= 8192 || (K >= 4096 && size >= 20000000);
+  else takes = K >= 16384 || (M > 11 && size >= 50000000);
+  float us;
+  return takes ? few_plan(M, N, K, qbits, false, us) : 0;
+}
+
 void launch_gemm_merge(__hip_bfloat16* y, const float* part, long plane, int parts, bool gated,
                        hipStream_t stream);
 
 namespace {
 
-// Without GATED: N columns of y; with it N / 2, of a plan for N with whole K and even panels
+// Without GATED: N columns of y; with it N / 2, of a plan for N with whole K
 template <int QB, bool GATED>
 void launch_panel(__hip_bfloat16* y, float* part, const __hip_bfloat16* x, const unsigned char* w,
                   const float* scale, int M, int N, int K, int plan, hipStream_t stream) {
   constexpr int kGroup = QB == 4 ? 128 : 64;
   const int parts = plan & 255, panel = (plan >> 8) - 1;
   const int depth = (K / kGroup + parts - 1) / parts * kGroup;
-#define GO(I, STAGES)                                                                             \
-  case I: {                                                                                       \
-    constexpr Panel p = QB == 4 ? kPanels4[I < 7 ? I : 0] : kPanels[I];                           \
-    constexpr bool gate = GATED && p.tn % 2 == 0;                                                 \
-    const int blocks = (M + p.tm * 16 - 1) / (p.tm * 16) * (N / (p.tn * 64));                     \
-    hipLaunchKernelGGL((gemm_panel::gemm_panel_q_kernel<QB, p.tm, p.tn, STAGES, p.per_cu, gate>), \
-                       dim3((blocks + 7) / 8 * 8, parts), dim3(64 * gemm_panel::kWaves), 0,       \
-                       stream, y, part, x, w, scale, M, GATED ? N / 2 : N, K, depth);             \
-    break;                                                                                        \
+#define GO(I, TM, TN, STAGES, PER_CU)                                                         \
+  case I: {                                                                                   \
+    const int blocks = (M + TM * 16 - 1) / (TM * 16) * (N / (TN * 64));                       \
+    hipLaunchKernelGGL((gemm_panel::gemm_panel_q_kernel<QB, TM, TN, STAGES, PER_CU, GATED>),  \
+                       dim3((blocks + 7) / 8 * 8, parts), dim3(64 * gemm_panel::kWaves), 0,   \
+                       stream, y, part, x, w, scale, M, GATED ? N / 2 : N, K, depth);         \
+    break;                                                                                    \
   }
-  if constexpr (QB == 4) {
-    switch (panel) {
-      GO(0, 5) GO(1, 5) GO(2, 4) GO(3, 4) GO(4, 3) GO(5, 4) GO(6, 6)
-    }
-  } else {
-    switch (panel) {
-      GO(0, 5) GO(1, 4) GO(2, 4) GO(3, 4) GO(4, 3) GO(5, 5) GO(6, 4) GO(7, 4)
-    }
+#define BOTH(I, ST4, ST8)                                                                     \
+  GO(I, kPanelOf(I).tm, kPanelOf(I).tn, (QB == 4 ? ST4 : ST8), kPanelOf(I).per_cu)
+#define FEW(I, ST4, ST8)                                                                      \
+  GO(kFewAt + I, kFewPanels[I].tm, kFewPanels[I].tn, (QB == 4 ? ST4 : ST8), 2)
+  constexpr auto kPanelOf = [](int i) constexpr { return QB == 4 ? kPanels4[i] : kPanels[i]; };
+  switch (panel) {
+    BOTH(0, 5, 5) BOTH(1, 5, 4) BOTH(2, 4, 4) BOTH(3, 4, 4) BOTH(4, 3, 3) BOTH(5, 4, 5) BOTH(6, 6, 4)
+    FEW(0, 8, 8) FEW(1, 6, 6) FEW(2, 6, 6) FEW(3, 5, 5) FEW(4, 6, 6) FEW(5, 6, 4)
+    default:
+      if constexpr (QB == 8)
+        switch (panel) {
+          BOTH(7, 4, 4)
+        }
   }
+#undef FEW
+#undef BOTH
 #undef GO
   if (parts > 1) launch_gemm_merge(y, part, (long)M * N, parts, false, stream);
 }
 
 }  // namespace
 
-// M >= 1, N % 128 == 0, K % 128 == 0; plan of gemm_panel_plan, its parts [parts, M, N]
+// M >= 1, N % 128 == 0, K % 128 == 0; plan of gemm_panel_plan or gemm_panel_few_plan, its parts
+// [parts, M, N]
 void launch_gemm_block_q(__hip_bfloat16* y, float* part, const __hip_bfloat16* x,
                          const unsigned char* w, const float* scale, int qbits, int M, int N,
                          int K, int plan, hipStream_t stream) {
@@ -438,20 +511,32 @@ void launch_gemm_block_q(__hip_bfloat16* y, float* part, const __hip_bfloat16* x
     launch_block<8>(y, x, w, scale, M, N, K, stream);
 }
 
-// The plan of a gated product of M > 64 rows with [2 N, K], or 0 where the plain one and a launch for
-// the gate are faster.  int8: where the plain one's plan cuts K or takes columns one tile a wave, as
-// the gate is not in the panel then; 4 bits: the best panel that can take it, against those two (the
-// gate 2.5 us and 4 bytes read, 2 written an output).
+// The plan of a gated product of M > 1 rows with [2 N, K], or 0 where the plain one and a launch for
+// the gate (2.5 us, 4 bytes read and 2 written an output) are faster.  int8 past 64 rows: where the
+// plain one's plan cuts K, as the gate is not in the panel then; others: the best panel with whole K
+// against those two.  Up to 64 rows only for matrices that panels take as fast as the streaming kernels
+// do (us, streaming and gate | gated panel, captured, int8: 28672 x 4096, 8 rows 27.9 | 26.4, 32 rows
+// 31.2 | 27.9, 64 46.5 | 31.6; 16384 x 2048, 8 rows 11.7 | 9.9, 32 13.1 | 10.1; 4096 x 1024, 8 rows 5.9 | 6.1, 33
+// rows 8.7 | 6.9; 4 bits 28672 x 4096, 2 rows 26.8 | 27.6, 4 rows 27.1 | 26.5, 16 rows 34.0 | 26.3).
 int gemm_panel_gated_plan(int M, int N, int K, int qbits) {
-  if (M <= 64 || N % 128 != 0 || K % 128 != 0 || (long)(N + 128) * K >= 1L << 32) return 0;
-  if (qbits == 4) {
-    float us, plain;
-    const int plan = panel4_plan(M, 2 * N, K, true, us);
+  if (M < 2 || N % 128 != 0 || K % 128 != 0 || (long)(N + 128) * K >= 1L << 32) return 0;
+  float us, plain;
+  int plan;
+  if (M <= 64) {
+    const long size = 2L * N * K;
+    if ((size < 24000000 && (K > 1024 || M <= 32)) || (qbits == 4 && M < 4) ||
+        (qbits == 8 && M < 12 && size >= 300000000))
+      return 0;
+    plan = few_plan(M, 2 * N, K, qbits, true, us);
+    few_plan(M, 2 * N, K, qbits, false, plain);
+  } else if (qbits == 4) {
+    plan = panel4_plan(M, 2 * N, K, true, us);
     panel4_plan(M, 2 * N, K, false, plain);
-    return us < plain + 2.5f + 1.2e-6f * M * N ? plan : 0;
+  } else {
+    plan = gemm_panel_plan(M, 2 * N, K, 8);
+    return plan > 1 && (plan & 255) == 1 ? plan : 0;
   }
-  const int plan = gemm_panel_plan(M, 2 * N, K, 8);
-  return plan > 1 && (plan & 255) == 1 && kPanels[(plan >> 8) - 1].tn % 2 == 0 ? plan : 0;
+  return us < plain + 2.5f + 1.2e-6f * M * N ? plan : 0;
 }
 
 // y [M, N] = silu(x Wg^T) * (x Wu^T), W = [Wg; Wu] rounded, plan of gemm_panel_gated_plan

@@ -87,11 +87,15 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
   constexpr int X_PASS = (X_LOADS + kWaves - 1) / kWaves;
   constexpr int W_PASS = (W_LOADS + kWaves - 1) / kWaves;
   constexpr int LOADS = X_PASS + W_PASS;
-  constexpr int AHEAD = 3;                // fragments of x on their way
+  // fragments of x on their way; those of the next tile are asked for behind the barrier
+  constexpr int AHEAD = TM < 3 ? TM : 3;
   constexpr bool SPREAD = TM >= 8;        // widening over the products
-  constexpr int OUT = GATED ? TN / 2 : TN, COLS = OUT * 16 * kWaves;   // of results
-  static_assert(!GATED || TN % 2 == 0, "as many gates");
-  static_assert(TM >= TN && 2 * TM > AHEAD && STAGES >= 3, "what a tile's products hide");
+  // results of a wave and of a panel; one tile a wave has eight gates and eight of the others
+  constexpr int WIDE = TN * (GATED ? 8 : 16), COLS = WIDE * kWaves;
+  constexpr bool HALVES = GATED && TN == 1;
+  constexpr int OUT = GATED && !HALVES ? TN / 2 : TN;
+  static_assert(!GATED || HALVES || TN % 2 == 0, "as many gates");
+  static_assert(TM >= TN && TM >= AHEAD && STAGES >= 3, "what a tile's products hide");
   static_assert(STAGES * STAGE * PER_CU <= 160 * 1024, "LDS of a CU");
   __shared__ __align__(16) char lds[STAGES * STAGE];
 
@@ -121,8 +125,8 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
     x_off[p] = (unsigned)min(r, M - 1 - m0) * (K * 2u) + (SPREAD ? at % 4 * 2 + at / 4 : at) * 16;
   }
   auto w_row = [&](int r) {   // of W from n0 on, for row r of the panel's
-    const int own = r / (TN * 16), in = r % (TN * 16), half = in / (OUT * 16);
-    return (unsigned)(half * N + own * (OUT * 16) + in % (OUT * 16));
+    const int own = r / (TN * 16), in = r % (TN * 16);
+    return (unsigned)(in / WIDE * N + own * WIDE + in % WIDE);
   };
 #pragma unroll
   for (int p = 0; p < W_PASS; ++p) {
@@ -295,23 +299,25 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
   const bool cut = gridDim.y > 1;
 #pragma unroll
   for (int j = 0; j < OUT; ++j) {
-    const int n = n0 + (wave * OUT + j) * 16 + quad * 4;
+    const int n = n0 + wave * WIDE + j * 16 + (HALVES ? quad % 2 : quad) * 4;
     f32x4_t s{16.f, 16.f, 16.f, 16.f}, su = s;   // (4 bits: what `nibble` leaves)
     if constexpr (QB == 8) {
-      s = *reinterpret_cast<const f32x4_any_t*>(scale + n);
-      if constexpr (GATED) su = *reinterpret_cast<const f32x4_any_t*>(scale + N + n);
+      s = *reinterpret_cast<const f32x4_any_t*>(scale + n + (HALVES && quad >= 2 ? N : 0));
+      if constexpr (GATED && !HALVES) su = *reinterpret_cast<const f32x4_any_t*>(scale + N + n);
     }
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const int m = m0 + i * 16 + col;
-      if (m >= M) continue;
       f32x4_t v;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         v[r] = acc[i][j][r] * s[r];
-        if constexpr (GATED)
+        if constexpr (HALVES)
+          v[r] = moe::finish<moe::kSilu>(v[r], __shfl_xor(v[r], 32), 0.f);
+        else if constexpr (GATED)
           v[r] = moe::finish<moe::kSilu>(v[r], acc[i][OUT + j][r] * su[r], 0.f);
       }
+      if (m >= M || (HALVES && quad >= 2)) continue;
       if (!GATED && cut) {
         *reinterpret_cast<f32x4_t*>(part + (blockIdx.y * (long)M + m) * N + n) = v;
       } else {

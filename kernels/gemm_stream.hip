@@ -28,8 +28,9 @@
 //   23 rows, 14336 x 4096 gated 55.2 -> 43.4; the mean of 6144 x 4096, 4096 x 4096 and
 //     4096 x 14336 23.9 -> 17.5 (a llama-3-8b layer reads W at 4.5 TB/s);
 //   61 rows, the mean of these three and 28672 x 4096: 38.1 -> 30.
-// (In bf16 the tiles have taken over from there at 23 and 61 rows; in rounded weights, up to 16
-// rows, short K and small matrices these kernels are what runs.)
+// (In bf16 the tiles have taken over from there at 23 and 61 rows, in rounded weights past 32 rows, and
+// fewer where the matrix is large, the panels of gemm_block_q.hip; up to 16 rows, at short K, for
+// small matrices and for rounded weights' operands off a 16-byte boundary these kernels are what runs.)
 
 #include "gemm_stream.h"
 

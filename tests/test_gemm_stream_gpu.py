@@ -352,8 +352,8 @@ def test_4_bit_panels(m, n, k, panel, parts):
 
 
 @pytest.mark.parametrize(("m", "n", "k", "panel"), [
-    (65, 14336, 128, 1), (321, 4096, 384, 2), (511, 3072, 128, 4), (301, 14336, 4096, 5),
-    (257, 8192, 128, 5), (161, 3072, 384, 6), (65, 1024, 8192, None)])
+    (65, 4096, 128, 0), (65, 14336, 128, 1), (321, 4096, 384, 2), (161, 3072, 384, 3),
+    (511, 8192, 384, 4), (301, 14336, 4096, 5), (257, 8192, 128, 5), (65, 1024, 8192, None)])
 def test_4_bit_gated_panels(m, n, k, panel):
     _need()
     from vllm_tgis_adapter_amd import ops
@@ -370,8 +370,54 @@ def test_4_bit_gated_panels(m, n, k, panel):
     _check(got, torch.nn.functional.silu(g) * u, 30 * (1 + g.abs()) * (1 + u.abs()))
 
 
+# panels of up to 64 rows, with whole K and with K cut evenly and unevenly, and with the gate
+@pytest.mark.parametrize("qbits", [8, 4])
+@pytest.mark.parametrize(("m", "n", "k", "panel", "parts"), [
+    (2, 128, 16512, 0, 8), (32, 28672, 4096, 1, 1), (17, 4096, 14336, 1, 8), (33, 4096, 2048, 2, 4), (48, 16384, 1024, 2, 1),
+    (33, 28672, 4096, 3, 1), (64, 2048, 2304, 4, 4), (49, 16384, 1024, 4, 1), (49, 6144, 14464, 5, 5),
+    (64, 28672, 2048, 5, 1)])
+def test_panels_of_few_rows(qbits, m, n, k, panel, parts):
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    assert ops._C.gemm_panel_few_plan(m, n, k, qbits) == (panel + 17) << 8 | parts
+    x, w = _x(m, k, 34), _x(n, k, 35)
+    wq, scale = ops.quantize_weight(w, qbits)
+    exact = _exact4(wq, scale) if qbits == 4 else (
+        wq.double() * scale.double()[:, None]).t().contiguous()
+    want, terms = x.double() @ exact, x.double().abs() @ exact.abs()
+    _check(ops.linear_quant(x, wq, scale, qbits), want, terms)
+    # off a 16-byte boundary: the streaming kernels
+    odd = torch.empty(m * k + 1, dtype=x.dtype, device="cuda")[1:].view(m, k).copy_(x)
+    _check(ops.linear_quant(odd, wq, scale, qbits), want, 20 * (terms + 1))
+
+
+@pytest.mark.parametrize("qbits", [8, 4])
+@pytest.mark.parametrize(("m", "n", "k", "panel"), [
+    (4, 8192, 2048, 0), (32, 8192, 2048, 0), (9, 14336, 4096, 1), (33, 128, 128, 2),
+    (47, 14336, 1024, 3), (64, 4096, 128, 4), (49, 14336, 2048, 5),
+    (2, 128, 2048, None)])
+def test_gated_panels_of_few_rows(qbits, m, n, k, panel):
+    _need()
+    from vllm_tgis_adapter_amd import ops
+
+    plan = ops._C.gemm_panel_gated_plan(m, n, k, qbits)
+    if panel is None:
+        assert plan == 0
+        return
+    assert plan == (panel + 17) << 8 | 1
+    x, w = _x(m, k, 36), _x(2 * n, k, 37) / k ** 0.5
+    wq, scale = ops.quantize_weight(w, qbits)
+    exact = _exact4(wq, scale) if qbits == 4 else (
+        wq.double() * scale.double()[:, None]).t().contiguous()
+    g, u = (x.double() @ exact).chunk(2, dim=1)
+    _check(ops.gated_quant(x, wq, scale, qbits), torch.nn.functional.silu(g) * u,
+           30 * (1 + g.abs()) * (1 + u.abs()))
+
+
 # every panel that takes the gate in, whole and with rows missing; the last is refused: K is cut
 @pytest.mark.parametrize(("m", "n", "k", "panel"), [
+    (511, 128, 128, 0), (511, 2048, 128, 3),
     (65, 14336, 384, 1), (321, 4096, 128, 2), (511, 8192, 128, 4), (97, 14336, 384, 5),
     (129, 14336, 384, 6), (301, 14336, 4096, 7), (1199, 4096, 128, 7), (301, 3072, 8192, None)])
 def test_int8_gated_panels(m, n, k, panel):

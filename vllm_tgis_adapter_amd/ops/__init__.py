@@ -406,7 +406,7 @@ def gated_quant(x: torch.Tensor, wq: torch.Tensor, scales: torch.Tensor,
     """silu(x Wg^T) * (x Wu^T) for [gate; up] weights as ``quantize_weight`` makes them, where
     the product of so many rows takes the gate into its launch; None elsewhere (the caller has
     linear_quant and silu_and_mul)."""
-    if (qbits not in (4, 8) or x.dim() != 2 or x.shape[0] <= 64 or x.dtype != torch.bfloat16
+    if (qbits not in (4, 8) or x.dim() != 2 or x.shape[0] < 2 or x.dtype != torch.bfloat16
             or not native_enabled(x) or not x.is_contiguous()):
         return None
     m, n, k = x.shape[0], wq.shape[0], x.shape[1]
