@@ -49,6 +49,7 @@ void launch_gemm_ring_parts(__hip_bfloat16*, float*, const __hip_bfloat16*,
                             const __hip_bfloat16*, int, int, int, int, hipStream_t);
 bool gemm_ring_takes(int N, int K, int plan, bool gated);
 int gemm_ring_lora_cuts(int M, int K, int L, int PR, int plan);
+bool gemm_ring_lora_wins(long M, long N, long K);
 void launch_gemm_ring_lora(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hip_bfloat16*,
                            int, int, int, int, float*, const __hip_bfloat16*, const int*, int, int,
                            int, hipStream_t);
@@ -1000,6 +1001,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_ring_plan", &gemm_ring_plan, "which tile a product takes, and parts of K (form << 4 | parts)");
   m.def("decode_inputs", &decode_inputs, "a captured step's inputs from a packed host buffer");
   m.def("lora_product", &lora_product, "a product with its LoRA deltas, also gated");
+  m.def("gemm_ring_lora_wins", &gemm_ring_lora_wins, "whether the tiles take a product with adapters");
   m.def("gemm_ring_lora_cuts", &gemm_ring_lora_cuts,
         "parts of K of the adapters' shrink beside a product, 0: in a launch of its own");
   m.def("lora_tiles_win", &lora_tiles_win, "whether its deltas are added by the matrix unit");

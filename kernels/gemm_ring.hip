@@ -409,6 +409,36 @@ int gemm_ring_lora_cuts(int M, int K, int L, int PR, int plan) {
   return plan >> 4 >= 2 && beside(M, PR, L, cuts) <= 256 ? cuts : 0;
 }
 
+// Whether these tiles take a product that has adapters, whatever takes it without them: beside other
+// products the shrink is a launch of its own, the deltas go over their rounded results, and where K is
+// cut the sum of the parts is one more; here it is two launches.  us with the deltas, otherwise |
+// here, 4 adapters of rank 16 (captured, cold weights), N x K: rows
+//   up to 16 rows: 6144 x 4096 2 19.2 | 15.8, 16 21.7 | 16.8; 28672 x 4096 gated 2 49.7 | 45.3; 4096 x 14336
+//    8 30.5 | 26.6; 2048 x 2048 12 11.3 | 8.8; 57344 x 8192 gated 2 174 | 163; 768 x 768 2 8.8 | 9.0; not
+//    4096 x 1792 12.3 | 13.7 (too short to be cut, 64 workgroups); of one row 6144 x 4096 16.4 | 15.0, 2048
+//    x 2048 9.3 | 7.8, but 4096 x 4096 12.5 | 13.3, 57344 x 8192 153 | 161;
+//   17 to 128: 2048 x 2048 64 16.2 | 9.2; 3072 x 2048 32 15.1 | 10.1, 65 20.7 | 12.7; 16384 x 2048 gated
+//    128 35.5 | 32.2; 28672 x 4096 gated 80 81.8 | 62.7, 128 73.2 | 65.9, 160 76.4 | 82.8; 57344 x 8192
+//    gated 65 207 | 172;
+//   up to 256: 3072 x 2048 24.3 | 19.4; 16384 x 2048 gated 44.7 | 38.5; 57344 x 8192 gated 269 | 234;
+//   up to 512: 4096 x 4096 301 37.8 | 33.3, 512 43.0 | 40.4; 2048 x 2048 512 22.3 | 16.9; 10240 x 8192 400
+//    110 | 100; 1536 x 4096 301 26.8 | 20.5; 3072 x 2048 400 28.1 | 28.5, 512 29.6 | 32.4; 6144 x 4096
+//    400 50.5 | 55.4; 16384 x 2048 gated 301 46.8 | 48.8.
+// (Of other ranks and numbers of adapters: as far or further apart but for rank 64 at 400 to 512 rows,
+// 0.98 to 1.03 of the others.)
+bool gemm_ring_lora_wins(long M, long N, long K) {
+  if (!fits(M, N, K, false)) return false;
+  if (M <= 64 ? gemm_ring_wins(M, N, K, false) : gemm_tiles_route(M, N, K) != 0) return true;
+  const long size = N * K;
+  if (M == 1) return size <= 6000000 || (size <= 300000000 && (K >= 8192 || N > 4096));
+  if (M <= 16) return K <= 1024 || K >= 2048 || N > 4096;
+  if (M <= 128) return true;
+  if (M <= 256) return size <= 34000000 || K >= 8192;
+  if (M > 512) return false;
+  return (K >= 8192 && size <= 100000000) ||
+         size <= (M <= 320 || K >= 4096 ? 17000000 : 5000000);
+}
+
 // launch_gemm_ring_parts and, in the same launch, tmp [cuts, M, PR] = the rows of A x of each
 // row's adapter, in parts
 void launch_gemm_ring_lora(__hip_bfloat16* y, float* part, const __hip_bfloat16* x,

@@ -91,6 +91,21 @@ def test_adapters_beside_every_form_of_product(t, width, k, form, parts):
     _beside_the_product(t, 3, k, 16, True, width, [(0, 256), (256, width)])
 
 
+# sizes at which the tiles take a product for its adapters' sake only
+@pytest.mark.parametrize(("t", "width", "k"), [
+    (1, 2048, 2048), (2, 28672, 4096), (8, 384, 64), (16, 6144, 4096), (17, 768, 768),
+    (64, 2048, 2048), (65, 16384, 2048), (128, 28672, 4096), (256, 3072, 2048), (320, 4096, 4096),
+    (512, 1536, 4096)])
+@pytest.mark.parametrize("rank", [8, 64])
+def test_products_that_adapters_bring(t, width, k, rank):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from vllm_tgis_adapter_amd import ops
+
+    assert ops._lora_tiles_take(t, width, k) and not ops._tiles_take(t, width, k)
+    _beside_the_product(t, 3, k, rank, True, width, [(0, 256), (256, width)])
+
+
 def _beside_the_product(t, adapters, k, rank, some, width, spans):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")

@@ -130,7 +130,7 @@ def test_one_question_for_both_rules():
 
 
 def test_few_rows_are_not_asked_for():
-    """Adapters' products of up to eight rows go past the question."""
+    """Products of up to eight rows are none of the tiles', but with adapters."""
     for m in range(1, 9):
         for n in (128, 2048, 14336, 28672):
             for k in (64, 2048, 8192, 28672):

@@ -185,7 +185,7 @@ def lora_linear(
         width = projs[-1][2]
         gate = gate_with_deltas(x.shape[0], width, b_stack.shape[2])
     out = None
-    if weight is not None and x.shape[0] > 8:   # (the tiles take none of fewer rows)
+    if weight is not None:
         out = ops.lora_product(x, weight, None, a_stack, b_stack, slots, scales, spans, gate)
     if out is None:
         y = base()

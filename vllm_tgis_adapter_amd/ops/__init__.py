@@ -304,6 +304,12 @@ def _tiles_take(m: int, n: int, k: int) -> bool:
             and m > _gemm_max_m())
 
 
+def _lora_tiles_take(m: int, n: int, k: int) -> bool:
+    """The same of a product with adapters."""
+    return (_C.gemm_ring_lora_wins(m, n, k)
+            and (m <= _gemm_max_m() if m <= 64 else m > _gemm_max_m()))
+
+
 def _gemm_max_m() -> int:
     return int(os.environ.get("VTA_GEMM_MAX_M", "64"))
 
@@ -579,11 +585,11 @@ def lora_product(
     gated: bool = False,
 ) -> torch.Tensor | None:
     """A product and its LoRA deltas in one, gated: and silu of the first half of its columns
-    times the second.  None where the tiles of gemm_ring.hip are not what would run the
-    product, or where tensors do not suit."""
+    times the second.  None where the tiles of gemm_ring.hip are slower than what would run the
+    product and the deltas, or where tensors do not suit."""
     given = weight if y is None else y
     rows, width = x.shape[0], given.shape[0 if y is None else 1]
-    if not native_enabled(x) or (y is None and not _tiles_take(rows, width, x.shape[1])):
+    if not native_enabled(x) or (y is None and not _lora_tiles_take(rows, width, x.shape[1])):
         return None
     if (given.dtype != torch.bfloat16 or not given.is_contiguous()
             or width % 2 or not slots.is_contiguous() or not scales.is_contiguous()
