@@ -31,7 +31,7 @@ PANELS4 = [(5, 1), (5, 2), (6, 2), (8, 1), (8, 2), (5, 4), (4, 2)]
 @pytest.mark.parametrize("n", [128, 512, 768, 4096, 28672])
 def test_4_bit_panels_fit(n, k):
     """Whole columns, no part of K without a group, rows of a panel inside 32 bits; a gated
-    product's panels have both halves and all of K."""
+    product's panels have all of K."""
     for m in (65, 129, 160, 257, 300, 513, 899, 1200):
         for plan, gated in ((ops._C.gemm_panel_plan(m, n, k, 4), False),
                             (ops._C.gemm_panel_gated_plan(m, n // 2, k, 4), True)):
@@ -39,10 +39,33 @@ def test_4_bit_panels_fit(n, k):
                 assert plan == (0 if gated else 1) and (gated or k <= 2048)
                 continue
             (rows, cols), parts = PANELS4[(plan >> 8) - 1], plan & 255
-            assert n % (64 * cols) == 0 and not (gated and (cols % 2 or parts > 1))
+            assert n % (64 * cols) == 0 and not (gated and parts > 1)
             assert 16 * rows * k * 2 < 1 << 32 and 64 * cols * k // 2 < 1 << 32
             groups = -(-(k // 128) // parts)
             assert (parts - 1) * groups < k // 128 <= parts * groups
+
+
+# of up to 64 rows
+FEW_PANELS = [(2, 1), (2, 2), (3, 1), (3, 2), (4, 1), (4, 2)]
+
+
+@pytest.mark.parametrize("qbits", [8, 4])
+@pytest.mark.parametrize("k", [128, 2048, 14336, 28672, (1 << 24) - 128])
+@pytest.mark.parametrize("n", [128, 512, 768, 4096, 28672, 57344])
+def test_panels_of_few_rows_fit(qbits, n, k):
+    """The same for these, which have all rows in one panel."""
+    for m in (2, 4, 9, 16, 17, 32, 33, 48, 49, 64):
+        for plan, gated in ((ops._C.gemm_panel_few_plan(m, n, k, qbits), False),
+                            (ops._C.gemm_panel_gated_plan(m, n // 2, k, qbits), True)):
+            if plan == 0:
+                continue
+            (rows, cols), parts = FEW_PANELS[(plan >> 8) - 17], plan & 255
+            assert 16 * rows >= m and n % (64 * cols) == 0 and not (gated and parts > 1)
+            assert 16 * rows * k * 2 < 1 << 32 and 64 * cols * k < 1 << 32
+            depth = -(-(k // (128 if qbits == 4 else 64)) // parts)
+            assert (parts - 1) * depth < k // (128 if qbits == 4 else 64) <= parts * depth
+    assert ops._C.gemm_panel_few_plan(1, n, k, qbits) == 0
+    assert ops._C.gemm_panel_gated_plan(1, n // 2, k, qbits) == 0
 
 
 @pytest.mark.parametrize(("m", "n", "k", "plans"), [
