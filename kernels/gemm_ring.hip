@@ -171,7 +171,13 @@ int even_parts(int K, int parts) {
 // Short K is cut less, eight tiles a part: 40 rows, 3072 x 2048 in 4 8.9 (in 5 9.4, whole 10.7), 8192
 // x 1024 whole 7.3 (in 2 8.0).  Past 48 rows of very many weights the tile of 128 columns reads x half
 // as often: 64 rows, 57344 x 8192 175 | 183, 8192 x 28672 in 4 90 | 96 (14336 x 8192 60 | 47, 28672 x
-// 8192 98 | 89, 10240 x 8192 in 3 37 | 38).
+// 8192 98 | 89).
+// For fewer rows too it is faster where columns of 64 would be cut and still be two a CU (one a CU then),
+// and, with K cut further, where they would be cut in two (half the barriers for as many bytes).  us, 64 |
+// 128 columns, 17 rows, 64 rows: 10240 x 8192 in 3 32.2 | 30.5, 38.7 | 33.7; 10240 x 2048 in 3 12.6 | 11.8,
+// 17.4 | 15.8; 14336 x 14336 in 2 75.9 | 63.3, 94.2 | 72.6; in 2 | in 4: 6144 x 4096 13.7 | 12.7, 17.2 | 16.7;
+// 8192 x 4096 16.5 | 14.6, 18.2 | 16.4; 6144 x 14336 33.1 | 31.5, 43.4 | 38.5; but 6144 x 2048 8.9 | 9.6;
+// in 2 | in 3: 8192 x 8192 27.3 | 25.1, 29.8 | 28.7; but 6144 x 8192 22.2 | 22.8, 27.5 | 28.0.
 Plan few_rows(int M, int N, int K) {
   const int cols = N / 64, tiles = K / 64;
   int parts = 256 / cols;
@@ -182,7 +188,13 @@ Plan few_rows(int M, int N, int K) {
   const int most = tiles < 32 ? 1 : tiles < 64 ? tiles / 8 : tiles / 6;
   if (parts > most) parts = most;
   if (parts < 1) parts = 1;
-  const bool wide = M > 48 && K >= 8192 && (K >= 16384 || (long)N * K > 400000000);
+  bool wide = (M > 48 && K >= 8192 && (K >= 16384 || (long)N * K > 400000000)) ||
+              (parts > 1 && cols * parts > 256);
+  if (parts == 2 && cols <= 128 && K >= 4096) {
+    const int more = K <= 6144 || K >= 12288 ? 4 : cols >= 120 ? 3 : 2;
+    wide = wide || more > 2;
+    parts = more;
+  }
   return Plan{wide && N % 128 == 0 ? kNarrow : kFew, even_parts(K, parts), 0.0};
 }
 
@@ -192,7 +204,9 @@ Plan few_rows(int M, int N, int K) {
 // rounds are counted there (84 tiles in three parts are 33 workgroups on some XCDs, two rounds,
 // though all are 252: 1.5 times the time of 80 tiles).
 Plan plan_of(int M, int N, int K, bool gated) {
-  if (M <= 64) return gated ? Plan{kFew, 1, 0.0} : few_rows(M, N, K);
+  // (gated, past one and a half rounds of two a CU, of 64 | 128 rows of W, us at 17, 40, 64 rows: 28672 x
+  // 8192 146 | 142, 155 | 145, 174 | 152; but 20480 x 5120 76 | 84, 94 | 96)
+  if (M <= 64) return gated ? Plan{N > 24576 ? kNarrow : kFew, 1, 0.0} : few_rows(M, N, K);
   Plan best{0, 1, 1e30};
   const double cols = gated ? 2.0 * N : N, w_mb = cols * K * 2e-6;
   for (int f = 0; f < kFormCount; ++f) {
@@ -230,7 +244,7 @@ Plan plan_of(int M, int N, int K, bool gated) {
 // rows in one: 8192 x 8192 by 128 x 128 0.88 of the time, 4096 x 14336 0.91, 5120 x 8192 0.97, but
 // 7168 x 4096 1.02, 6144 x 4096 1.05)
 bool read_once(int M, long weights, int form) {
-  return M <= kForms[form].bm && weights >= (form == kFew ? 20000000 : 40000000);
+  return M <= kForms[form].bm && weights >= (form >= kNarrow ? 20000000 : 40000000);
 }
 
 template <int BM, int BN, int SLOTS, int OCC, bool GATED, int HINT = 0>
@@ -342,7 +356,7 @@ bool gemm_block_takes(long M, long N, long K) {
 //   1.17, 6144 x 4096 0.92 to 1.13.
 //  Gated, against gemm_stream.hip's, 17 | 64 rows: 14336 x 4096 0.91 | 0.92, 6144 x 4096 0.86 |
 //   0.82, 8192 x 2048 0.85 | 0.83, 7168 x 8192 1.01 | 0.79, 8192 x 8192 1.06 | 0.75, 11008 x 4096
-//   1.07 | 0.80, 28672 x 8192 0.92 | 1.06.
+//   1.07 | 0.80, 28672 x 8192 0.89 | 0.94.
 //  Gated, past 64 rows, against the library's product (or the plain one by these tiles, where they
 //   take it) and its gate: where the model is below 1.05 of a model of the library's fitted likewise
 //   (14 %), below 0.98 for tiles of 256 x 256, whose last round costs most, and below 0.9 of its own
@@ -352,7 +366,7 @@ bool gemm_ring_wins(long M, long N, long K, bool gated) {
   if (!fits(M, N, K, gated)) return false;
   if (gated) {
     if (M <= 64) {
-      if (M <= 16 || N < 6144 || (M > 48 && N * K > 150000000)) return false;
+      if (M <= 16 || N < 6144 || (M > 48 && N * K > 150000000 && N <= 24576)) return false;
       const long blocks = N / 32;   // one a CU, or nearly two
       return M > 32 || (blocks <= 256 ? K < 8192 : blocks >= 400);
     }
