@@ -38,6 +38,7 @@
 
 #include "common.h"
 #include <float.h>
+#include <algorithm>
 #include <type_traits>
 
 typedef __attribute__((ext_vector_type(8))) short bf16x8_t;
@@ -50,7 +51,10 @@ typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
 namespace {
 
 constexpr int kTile = 64;   // keys of a step
-constexpr int kMinTiles = 6;   // a part is no shorter
+// A part is no shorter: few tokens after a long context are a chain of tiles, and what a part leaves is
+// little (8 prompts of 2 tokens after 600 in 1 | 3 parts: 18.4 | 13.3 us, 64 after 2000 in 5 | 8: 22.0 |
+// 20.7); e4m3, whose first tile is widened ahead of all, was not measured for less.
+template <typename CT> constexpr int kMinTiles = sizeof(CT) == 2 ? 3 : 6;
 constexpr float kLog2e = 1.4426950408889634f;
 // A maximum that grew by less than this (log2) is not followed: sums and probabilities
 // stay in range, their relative precision is the same.
@@ -81,8 +85,8 @@ template <int HD, bool PAIRS> DEVINLINE int v_swizzle(int r) {
 }
 
 // tiles of keys that one part takes
-DEVINLINE int tiles_per_part(int tiles, int parts) {
-  return max(kMinTiles, (tiles + parts - 1) / parts);
+template <typename CT> DEVINLINE int tiles_per_part(int tiles, int parts) {
+  return max(kMinTiles<CT>, (tiles + parts - 1) / parts);
 }
 
 // Whether the two waves of a SIMD take turns: not where the lanes find their rows and little is won by
@@ -150,7 +154,7 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
   const int token = min(token0 + col, q_len - 1);
   const int past = seq_len - q_len;
   const int keys = min(seq_len, past + min((tile + 1) * tokens, q_len));
-  const int tiles = (keys + kTile - 1) / kTile, per = tiles_per_part(tiles, parts);
+  const int tiles = (keys + kTile - 1) / kTile, per = tiles_per_part<CT>(tiles, parts);
   const int first = blockIdx.z % parts * per;
   // no keys at all: part 0 writes the zeros
   if (first >= tiles && first > 0) return;
@@ -596,7 +600,7 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
 
 // Tokens whose keys were cut: out = sum_p f_p acc_p / sum_p f_p l_p.  grid (tokens of the
 // longest prompt, sequences, heads / 4), a wave a head; parts <= 16.
-template <int HD>
+template <int HD, typename CT>
 __global__ __launch_bounds__(256) void prefill_tile_merge_kernel(
     __hip_bfloat16* __restrict__ out, const float* __restrict__ part_acc,
     const float* __restrict__ part_ml, const int* __restrict__ query_start_loc,
@@ -607,7 +611,7 @@ __global__ __launch_bounds__(256) void prefill_tile_merge_kernel(
   if (token >= q_len || head >= nheads) return;
   const int seq_len = seq_lens[seq], past = seq_len - q_len;
   const int keys = min(seq_len, past + min((token / tokens + 1) * tokens, q_len));
-  const int tiles = (keys + kTile - 1) / kTile, per = tiles_per_part(tiles, parts);
+  const int tiles = (keys + kTile - 1) / kTile, per = tiles_per_part<CT>(tiles, parts);
   if (per >= tiles) return;
   const int used = (tiles + per - 1) / per;
   const long rows = (long)query_start_loc[gridDim.y] * nheads;
@@ -641,6 +645,17 @@ struct Cut {
   int waves, heads, tokens, parts;   // of a workgroup; workgroups a tile's keys are cut over
 };
 
+void shape(Cut& c, int waves, int group) {
+  c.waves = c.heads = waves;
+  while (group % c.heads) c.heads /= 2;
+  c.tokens = waves / c.heads * 32;
+}
+
+long blocks_of(const Cut& c, int nseq, int nheads, int max_query_len) {
+  const long n = (long)nheads / c.heads * nseq * ((max_query_len + c.tokens - 1) / c.tokens);
+  return n > 0 ? n : 1;
+}
+
 // Eight waves share every tile of keys where their workgroups, with the keys cut into parts
 // where there are few, fill more than half the chip; else four do, two such workgroups a
 // CU.  Measured, heads 32/8 of 128 (us, waves/parts): 3500 tokens of 7 prompts after 700
@@ -655,16 +670,13 @@ struct Cut {
 // long contexts all eight are worth it (16/16 heads of 128, 64 tokens after 4000 22.6 | 24.2),
 // two do for a few tiles only (16/8, 100 of 5 after 500 | 55 | 66), and e4m3 keys, which are
 // widened, take more (16/16, 16 of 128 11.5 | 12.6, 8 of 30 | 7.2 | 8.5).
-Cut cut_of(bool fp8, int nseq, int nheads, int kvh, int max_query_len, int max_keys) {
-  const int group = nheads / kvh, most = max_keys / (kTile * kMinTiles);
+Cut waves_of(bool fp8, int nseq, int nheads, int kvh, int max_query_len, int max_keys) {
+  const int group = nheads / kvh, most = max_keys / (kTile * 6);
   Cut c{};
   for (c.waves = 8;; c.waves /= 2) {
-    c.heads = c.waves;
-    while (group % c.heads) c.heads /= 2;
-    c.tokens = c.waves / c.heads * 32;
-    const long blocks =
-        (long)nheads / c.heads * nseq * ((max_query_len + c.tokens - 1) / c.tokens);
-    const long fit = 256 * 8 / c.waves / (blocks > 0 ? blocks : 1);
+    shape(c, c.waves, group);
+    const long blocks = blocks_of(c, nseq, nheads, max_query_len);
+    const long fit = 256 * 8 / c.waves / blocks;
     c.parts = fit < 16 ? (int)fit : 16;
     if (c.parts > most) c.parts = most;
     if (c.parts < 1) c.parts = 1;
@@ -673,6 +685,51 @@ Cut cut_of(bool fp8, int nseq, int nheads, int kvh, int max_query_len, int max_k
     const bool least = c.waves == (fp8 || max_keys > 2 * kTile ? 4 : 2);
     if (least || (!idle && (c.waves == 4 || blocks * c.parts > 128))) return c;
   }
+}
+
+// bf16 keys and four or eight query heads a key head: the parts again, and four waves instead of
+// eight, by what a launch takes, us: its start, the longest chain of tiles, and for parts their launch,
+// their sums written and read.  Fitted to some 700 times (heads 32/8 of 128 and 64, 64/8 of 128; one to
+// sixteen prompts of 2 to 8192 tokens, after none to 6000).
+//  - Parts pay for their sums only where tokens are few: one prompt of 1000 in 8 waves, 2 parts 37.8, 1
+//    part 30.9, by 4 waves 29.0; heads of 64 29.0 | 20.3; after 1000 tokens, heads of 64, 40.9 | 35.4; 64/8
+//    heads, 512 after 1000 46.7 | 41.6; but 1000 after 3000 78.6 | 96.
+//  - Uncut, four waves end a workgroup's last tiles sooner, where they are one a CU, or, where many keys
+//    are the prompts' own, two and their tiles few (heads of 64: up to three): 8 | 4 waves, 32/8 heads
+//    of 128, 2 prompts of 1000 33.3 | 32.4, 8 of 256 16.6 | 15.1; of 64, one of 2000 40.4 | 36.6, 4 of 500
+//    after 700 28.8 | 26.4; past that 7 of 500 after 700 67.6 | 70.1, one of 4000 132 | 145; 64/8 heads,
+//    8 of 128 after 600 31.3 | 34.1, one of 2000 73.8 | 79.3.
+Cut cut_of(bool fp8, int nseq, int nheads, int kvh, int head_dim, int max_query_len,
+           int max_keys) {
+  Cut c = waves_of(fp8, nseq, nheads, kvh, max_query_len, max_keys);
+  const int group = nheads / kvh;
+  if (fp8 || group % 4 != 0 || c.waves < 4) return c;
+  const bool wide = head_dim == 128;
+  const int tiles = (max_keys + kTile - 1) / kTile, least = kMinTiles<__hip_bfloat16>;
+  const double mb = 8e-6 * nseq * max_query_len * nheads * head_dim;   // of a part, there and back
+  auto us = [&](int waves, int parts) {
+    const int per = parts == 1 || tiles <= least ? tiles : std::max(least, (tiles + parts - 1) / parts);
+    return (wide ? (waves == 8 ? 8.1 : 6.1) : waves == 8 ? 5.7 : 4.6) +
+           (wide ? (waves == 8 ? 1.44 : 1.42) : waves == 8 ? 1.3 : 0.95) * per +
+           (parts > 1 ? 3.5 + 0.3 * parts + (wide ? 0.21 : 0.35) * mb * parts : 0.0);
+  };
+  const long fit = 256 * 8 / c.waves / blocks_of(c, nseq, nheads, max_query_len);
+  const int most = max_keys / (kTile * least);
+  c.parts = 1;
+  for (int p = 2; p <= 16 && p <= fit && p <= most; ++p)
+    if (us(c.waves, p) < us(c.waves, c.parts)) c.parts = p;
+  if (c.waves == 8) {
+    Cut four{};
+    shape(four, 4, group);
+    four.parts = 1;
+    const long blocks = blocks_of(four, nseq, nheads, max_query_len);
+    const bool short_chain =
+        2L * max_keys <= 5L * max_query_len && (wide ? blocks <= 512 && tiles <= 16 : blocks <= 768);
+    if (c.parts == 1 ? blocks <= 256 || short_chain
+                     : blocks <= 512 && us(4, 1) < 0.95 * us(8, c.parts))
+      c = four;
+  }
+  return c;
 }
 
 template <int HD, typename CT>
@@ -699,7 +756,7 @@ void launch(__hip_bfloat16* out, float* part_acc, float* part_ml, const __hip_bf
   else GO(2, false);
 #undef GO
   if (c.parts > 1)
-    hipLaunchKernelGGL((prefill_tile_merge_kernel<HD>), dim3(max_query_len, nseq, (nheads + 3) / 4),
+    hipLaunchKernelGGL((prefill_tile_merge_kernel<HD, CT>), dim3(max_query_len, nseq, (nheads + 3) / 4),
                        dim3(256), 0, stream, out, part_acc, part_ml, qsl, sl, nheads, c.tokens, c.parts);
 }
 
@@ -708,9 +765,9 @@ void launch(__hip_bfloat16* out, float* part_acc, float* part_ml, const __hip_bf
 // Workgroups that a prompt's keys may be cut over (a function of shapes only): 1, or the
 // launch needs part_acc [parts, tokens, nheads, head_dim] and part_ml [parts, tokens,
 // nheads, 2].
-int prefill_tile_parts(bool fp8, int nseq, int nheads, int kvh, int max_query_len,
+int prefill_tile_parts(bool fp8, int nseq, int nheads, int kvh, int head_dim, int max_query_len,
                        int max_keys) {
-  return cut_of(fp8, nseq, nheads, kvh, max_query_len, max_keys).parts;
+  return cut_of(fp8, nseq, nheads, kvh, head_dim, max_query_len, max_keys).parts;
 }
 
 void launch_paged_prefill_tile(__hip_bfloat16* out, float* part_acc, float* part_ml,
@@ -719,7 +776,7 @@ void launch_paged_prefill_tile(__hip_bfloat16* out, float* part_acc, float* part
                                const int* sl, float scale, int nseq, int nheads, int kvh,
                                int head_dim, int block_size, int max_blocks, int max_query_len,
                                int max_keys, hipStream_t stream) {
-  const Cut c = cut_of(false, nseq, nheads, kvh, max_query_len, max_keys);
+  const Cut c = cut_of(false, nseq, nheads, kvh, head_dim, max_query_len, max_keys);
   auto go = [&](auto launch) {
     launch(out, part_acc, part_ml, q, kc, vc, bt, qsl, sl, scale, nseq, nheads, kvh, block_size,
            max_blocks, max_query_len, c, stream);
@@ -737,5 +794,5 @@ void launch_paged_prefill_tile_fp8(__hip_bfloat16* out, float* part_acc, float* 
                                    int max_keys, hipStream_t stream) {
   launch<128, unsigned char>(out, part_acc, part_ml, q, kc, vc, bt, qsl, sl, scale, nseq, nheads,
                              kvh, block_size, max_blocks, max_query_len,
-                             cut_of(true, nseq, nheads, kvh, max_query_len, max_keys), stream);
+                             cut_of(true, nseq, nheads, kvh, 128, max_query_len, max_keys), stream);
 }

@@ -17,7 +17,7 @@ template <typename T>
 void launch_paged_prefill(T*, const T*, const T*, const T*, const int*,
                           const int*, const int*, float, int, int, int, int,
                           int, int, int, hipStream_t);
-int prefill_tile_parts(bool fp8, int nseq, int nheads, int kvh, int max_query_len,
+int prefill_tile_parts(bool fp8, int nseq, int nheads, int kvh, int head_dim, int max_query_len,
                        int max_keys);
 void launch_paged_prefill_tile(__hip_bfloat16*, float*, float*, const __hip_bfloat16*,
                                const __hip_bfloat16*, const __hip_bfloat16*, const int*,
@@ -222,7 +222,7 @@ void paged_attention_prefill(torch::Tensor out, torch::Tensor q,
   const int64_t parts =
       tiles && (!force_valu || k_cache.scalar_type() == at::ScalarType::Byte)
           ? prefill_tile_parts(k_cache.scalar_type() == at::ScalarType::Byte, nseq, nheads, kvh,
-                               (int)max_query_len, max_keys)
+                               head_dim, (int)max_query_len, max_keys)
           : 1;
   torch::Tensor part_acc, part_ml;
   float *acc = nullptr, *ml = nullptr;

@@ -280,3 +280,13 @@ def test_places_of_tiles(block, dim, fp8, keys):
 
     v = vc.float().cpu().nan_to_num()
     _close(got, plain(v), plain(v.abs()))
+
+
+# parts of three tiles and more, of a sequence that has fewer too, four waves where eight were
+@pytest.mark.parametrize("shape", [
+    [(2, 600)] * 8, [(64, 500), (3, 190), (1, 0)], [(1000, 0)], [(256, 1000), (5, 190)],
+    [(256, 0)] * 8], ids=str)
+@pytest.mark.parametrize(("heads", "kv_heads"), [(32, 8), (64, 8)])
+@pytest.mark.parametrize("dim", [64, 128])
+def test_prefill_of_served_heads(shape, heads, kv_heads, dim):
+    test_prefill(shape, heads, kv_heads, dim, torch.bfloat16, 16)
