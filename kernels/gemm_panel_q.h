@@ -1,4 +1,4 @@
-// Products of 65 to some hundreds of rows with rounded weights (see gemm_block_q.hip): panels of
+// Products of 2 to some hundreds of rows with rounded weights (see gemm_block_q.hip): panels of
 // 16 TM rows of x against 64 TN columns of W.  The waves lie along the columns, so that every
 // weight of a panel is widened by one wave only, once for all its rows.
 //
