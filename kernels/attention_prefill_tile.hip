@@ -52,9 +52,9 @@ namespace {
 
 constexpr int kTile = 64;   // keys of a step
 // A part is no shorter: few tokens after a long context are a chain of tiles, and what a part leaves is
-// little (8 prompts of 2 tokens after 600 in 1 | 3 parts: 18.4 | 13.3 us, 64 after 2000 in 5 | 8: 22.0 |
-// 20.7); e4m3, whose first tile is widened ahead of all, was not measured for less.
-template <typename CT> constexpr int kMinTiles = sizeof(CT) == 2 ? 3 : 6;
+// little (8 prompts of 2 tokens after 600 in 1 | 3 parts: 18.4 | 13.3 us, e4m3 21.3 | 14.6; 64 after 2000
+// in 5 | 8: 22.0 | 20.7, e4m3 23.7 | 22.0)
+constexpr int kMinTiles = 3;
 constexpr float kLog2e = 1.4426950408889634f;
 // A maximum that grew by less than this (log2) is not followed: sums and probabilities
 // stay in range, their relative precision is the same.
@@ -85,8 +85,8 @@ template <int HD, bool PAIRS> DEVINLINE int v_swizzle(int r) {
 }
 
 // tiles of keys that one part takes
-template <typename CT> DEVINLINE int tiles_per_part(int tiles, int parts) {
-  return max(kMinTiles<CT>, (tiles + parts - 1) / parts);
+DEVINLINE int tiles_per_part(int tiles, int parts) {
+  return max(kMinTiles, (tiles + parts - 1) / parts);
 }
 
 // Whether the two waves of a SIMD take turns: not where the lanes find their rows and little is won by
@@ -154,7 +154,7 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
   const int token = min(token0 + col, q_len - 1);
   const int past = seq_len - q_len;
   const int keys = min(seq_len, past + min((tile + 1) * tokens, q_len));
-  const int tiles = (keys + kTile - 1) / kTile, per = tiles_per_part<CT>(tiles, parts);
+  const int tiles = (keys + kTile - 1) / kTile, per = tiles_per_part(tiles, parts);
   const int first = blockIdx.z % parts * per;
   // no keys at all: part 0 writes the zeros
   if (first >= tiles && first > 0) return;
@@ -600,7 +600,7 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_tile_kernel(
 
 // Tokens whose keys were cut: out = sum_p f_p acc_p / sum_p f_p l_p.  grid (tokens of the
 // longest prompt, sequences, heads / 4), a wave a head; parts <= 16.
-template <int HD, typename CT>
+template <int HD>
 __global__ __launch_bounds__(256) void prefill_tile_merge_kernel(
     __hip_bfloat16* __restrict__ out, const float* __restrict__ part_acc,
     const float* __restrict__ part_ml, const int* __restrict__ query_start_loc,
@@ -611,7 +611,7 @@ __global__ __launch_bounds__(256) void prefill_tile_merge_kernel(
   if (token >= q_len || head >= nheads) return;
   const int seq_len = seq_lens[seq], past = seq_len - q_len;
   const int keys = min(seq_len, past + min((token / tokens + 1) * tokens, q_len));
-  const int tiles = (keys + kTile - 1) / kTile, per = tiles_per_part<CT>(tiles, parts);
+  const int tiles = (keys + kTile - 1) / kTile, per = tiles_per_part(tiles, parts);
   if (per >= tiles) return;
   const int used = (tiles + per - 1) / per;
   const long rows = (long)query_start_loc[gridDim.y] * nheads;
@@ -687,30 +687,33 @@ Cut waves_of(bool fp8, int nseq, int nheads, int kvh, int max_query_len, int max
   }
 }
 
-// bf16 keys and four or eight query heads a key head: the parts again, and four waves instead of
+// Four or eight query heads a key head: the parts again, and for bf16 keys four waves instead of
 // eight, by what a launch takes, us: its start, the longest chain of tiles, and for parts their launch,
-// their sums written and read.  Fitted to some 700 times (heads 32/8 of 128 and 64, 64/8 of 128; one to
+// their sums written and read.  Fitted to some 1000 times (heads 32/8 of 128 and 64, 64/8 of 128; one to
 // sixteen prompts of 2 to 8192 tokens, after none to 6000).
 //  - Parts pay for their sums only where tokens are few: one prompt of 1000 in 8 waves, 2 parts 37.8, 1
-//    part 30.9, by 4 waves 29.0; heads of 64 29.0 | 20.3; after 1000 tokens, heads of 64, 40.9 | 35.4; 64/8
+//    part 30.9, by 4 waves 29.0; heads of 64 29.0 | 20.3, e4m3 40.0 | 33.3 by 8; after 1000 tokens, heads of 64, 40.9 | 35.4; 64/8
 //    heads, 512 after 1000 46.7 | 41.6; but 1000 after 3000 78.6 | 96.
 //  - Uncut, four waves end a workgroup's last tiles sooner, where they are one a CU, or, where many keys
 //    are the prompts' own, two and their tiles few (heads of 64: up to three): 8 | 4 waves, 32/8 heads
 //    of 128, 2 prompts of 1000 33.3 | 32.4, 8 of 256 16.6 | 15.1; of 64, one of 2000 40.4 | 36.6, 4 of 500
 //    after 700 28.8 | 26.4; past that 7 of 500 after 700 67.6 | 70.1, one of 4000 132 | 145; 64/8 heads,
-//    8 of 128 after 600 31.3 | 34.1, one of 2000 73.8 | 79.3.
+//    8 of 128 after 600 31.3 | 34.1, one of 2000 73.8 | 79.3; e4m3, 2 prompts of 1000 37.0 | 37.6.
 Cut cut_of(bool fp8, int nseq, int nheads, int kvh, int head_dim, int max_query_len,
            int max_keys) {
   Cut c = waves_of(fp8, nseq, nheads, kvh, max_query_len, max_keys);
   const int group = nheads / kvh;
-  if (fp8 || group % 4 != 0 || c.waves < 4) return c;
+  if (group % 4 != 0 || c.waves < 4) return c;
   const bool wide = head_dim == 128;
-  const int tiles = (max_keys + kTile - 1) / kTile, least = kMinTiles<__hip_bfloat16>;
+  const int tiles = (max_keys + kTile - 1) / kTile, least = kMinTiles;
   const double mb = 8e-6 * nseq * max_query_len * nheads * head_dim;   // of a part, there and back
   auto us = [&](int waves, int parts) {
     const int per = parts == 1 || tiles <= least ? tiles : std::max(least, (tiles + parts - 1) / parts);
-    return (wide ? (waves == 8 ? 8.1 : 6.1) : waves == 8 ? 5.7 : 4.6) +
-           (wide ? (waves == 8 ? 1.44 : 1.42) : waves == 8 ? 1.3 : 0.95) * per +
+    const double start = fp8    ? (waves == 8 ? 7.0 : 4.5)
+                         : wide ? (waves == 8 ? 8.1 : 6.1) : (waves == 8 ? 5.7 : 4.6);
+    const double tile = fp8    ? (waves == 8 ? 1.65 : 1.83)
+                        : wide ? (waves == 8 ? 1.44 : 1.42) : (waves == 8 ? 1.3 : 0.95);
+    return start + tile * per +
            (parts > 1 ? 3.5 + 0.3 * parts + (wide ? 0.21 : 0.35) * mb * parts : 0.0);
   };
   const long fit = 256 * 8 / c.waves / blocks_of(c, nseq, nheads, max_query_len);
@@ -718,7 +721,7 @@ Cut cut_of(bool fp8, int nseq, int nheads, int kvh, int head_dim, int max_query_
   c.parts = 1;
   for (int p = 2; p <= 16 && p <= fit && p <= most; ++p)
     if (us(c.waves, p) < us(c.waves, c.parts)) c.parts = p;
-  if (c.waves == 8) {
+  if (c.waves == 8 && !fp8) {
     Cut four{};
     shape(four, 4, group);
     four.parts = 1;
@@ -756,7 +759,7 @@ void launch(__hip_bfloat16* out, float* part_acc, float* part_ml, const __hip_bf
   else GO(2, false);
 #undef GO
   if (c.parts > 1)
-    hipLaunchKernelGGL((prefill_tile_merge_kernel<HD, CT>), dim3(max_query_len, nseq, (nheads + 3) / 4),
+    hipLaunchKernelGGL((prefill_tile_merge_kernel<HD>), dim3(max_query_len, nseq, (nheads + 3) / 4),
                        dim3(256), 0, stream, out, part_acc, part_ml, qsl, sl, nheads, c.tokens, c.parts);
 }
 

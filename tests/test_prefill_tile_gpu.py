@@ -287,6 +287,7 @@ def test_places_of_tiles(block, dim, fp8, keys):
     [(2, 600)] * 8, [(64, 500), (3, 190), (1, 0)], [(1000, 0)], [(256, 1000), (5, 190)],
     [(256, 0)] * 8], ids=str)
 @pytest.mark.parametrize(("heads", "kv_heads"), [(32, 8), (64, 8)])
-@pytest.mark.parametrize("dim", [64, 128])
-def test_prefill_of_served_heads(shape, heads, kv_heads, dim):
-    test_prefill(shape, heads, kv_heads, dim, torch.bfloat16, 16)
+@pytest.mark.parametrize(("dim", "dtype"), [
+    (64, torch.bfloat16), (128, torch.bfloat16), (128, torch.uint8)])
+def test_prefill_of_served_heads(shape, heads, kv_heads, dim, dtype):
+    test_prefill(shape, heads, kv_heads, dim, dtype, 16)
