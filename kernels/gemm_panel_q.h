@@ -115,12 +115,21 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
 
   // (4 bits: the reads of a wave are one run of bytes)
   auto w_turn = [](int r) { return QB == 4 ? 0 : SPREAD ? -(r / 4) & 3 : r / 4 % 4; };
-  // (where there are fewer loads than waves some are made twice: all waves wait alike; rows
-  // of a panel are found by 32 bits, see gemm_panel_plan)
+  // Pass p of the waves' over a tile's loads.  (Where the last has fewer than waves some are made twice: all
+  // waves wait alike.)  Only there is a remainder taken past 64 rows: other places are the wave's own
+  // and a literal.  With remainders everywhere the loop of 160 x 256 had 282 instructions, now 271, each four
+  // clocks of a wave alone on its SIMD: four layers of llama-3-8b in int8, 150 rows 506 -> 492 us, 301
+  // rows 716 -> 706; of 80 x 64, 4096 x 4096, 257 rows 21.0 -> 19.1.  (Panels of fewer rows, of which two
+  // share a SIMD, gain nothing: 40 rows 326 as they are, 330.)
+  auto pass = [&](int p, int loads) {
+    const int at = p * kWaves + wave;
+    return TM > 4 && (p + 1) * kWaves <= loads ? at : at % loads;
+  };
+  // (rows of a panel are found by 32 bits, see gemm_panel_plan)
   unsigned x_off[X_PASS], w_off[W_PASS];
 #pragma unroll
   for (int p = 0; p < X_PASS; ++p) {
-    const int r = (p * kWaves + wave) % X_LOADS * 8 + lane / 8;
+    const int r = pass(p, X_LOADS) * 8 + lane / 8;
     const int at = (lane % 8) ^ (r / 2 % 8);   // large: of the chunks 0 2 4 6 1 3 5 7
     x_off[p] = (unsigned)min(r, M - 1 - m0) * (K * 2u) + (SPREAD ? at % 4 * 2 + at / 4 : at) * 16;
   }
@@ -130,7 +139,7 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
   };
 #pragma unroll
   for (int p = 0; p < W_PASS; ++p) {
-    const int r = (p * kWaves + wave) % W_LOADS * (64 / WL) + lane / WL;
+    const int r = pass(p, W_LOADS) * (64 / WL) + lane / WL;
     w_off[p] = w_row(r) * (unsigned)(K * QB / 8) + ((lane % WL) ^ w_turn(r)) * 16;
   }
   const auto x_from = block_gemm::resource(x + (long)m0 * K + k0);
@@ -139,19 +148,24 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
   if constexpr (QB == 4) s_off = w_row(wave % TN * 64 + lane) * (unsigned)(K / 128 * 4);
   const auto s_from =
       block_gemm::resource(QB == 4 ? scale + (long)n0 * (K / 128) + k0 / 128 : scale);
-  // load p of a tile (past the last tile it is the last one again)
-  auto load = [&](int buf, int tile, int p) {
-    char* to = lds + buf * STAGE;
+  // load p of a tile (past the last tile it is the last one again) to the buffer of which `own` is the
+  // wave's first KB: places are that and a literal, or a register where a remainder is taken
+  auto load = [&](int& own, int tile, int p) {
     tile = min(tile, tiles - 1) + start;
     if (tile >= tiles) tile -= tiles;
+    // Added as the load is made, in one instruction: where loads are many the compiler adds all ahead and
+    // copies each.  (Elsewhere it does well alone, and keeping the order costs: 4 bits 28672 x 4096, 129
+    // rows 47.8 us, 59.6 with it; int8 4096 x 4096, 196 rows 18.9, 20.9)
+    if constexpr (QB == 8 && TN == 4) asm volatile("" : "+s"(own));
+    auto place = [&](int q, int loads) { return lds + own + (pass(q, loads) - wave) * 1024; };
     if (p < X_PASS)
-      block_gemm::load_lds(to + (p * kWaves + wave) % X_LOADS * 1024, x_from, x_off[p],
-                           tile * (kDepth * 2));
+      block_gemm::load_lds(place(p, X_LOADS), x_from, x_off[p], tile * (kDepth * 2));
     else if (p < LOADS)
-      block_gemm::load_lds(to + X_BYTES + ((p - X_PASS) * kWaves + wave) % W_LOADS * 1024, w_from,
+      block_gemm::load_lds(place(p - X_PASS, W_LOADS) + X_BYTES, w_from,
                            w_off[p < LOADS ? p - X_PASS : 0], tile * W_ROW);
     else
-      block_gemm::load_lds4(to + X_BYTES + W_BYTES + wave % TN * 256, s_from, s_off, tile / 2 * 4);
+      block_gemm::load_lds4(lds + own + (X_BYTES + W_BYTES + wave % TN * 256 - wave * 1024), s_from,
+                            s_off, tile / 2 * 4);
   };
 
   f32x4_t acc[TM][TN];
@@ -192,9 +206,11 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
   };
 
 #pragma unroll
-  for (int s = 0; s < STAGES - 1; ++s)
+  for (int s = 0; s < STAGES - 1; ++s) {
+    int own = s * STAGE + wave * 1024;
 #pragma unroll
-    for (int p = 0; p < loads_of<QB>(LOADS, s, 1); ++p) load(s, s, p);
+    for (int p = 0; p < loads_of<QB>(LOADS, s, 1); ++p) load(own, s, p);
+  }
   block_gemm::wait_loads<loads_of<QB>(LOADS, 1, STAGES - 2)>();
   block_gemm::meet();
   Chunk c[TN];
@@ -222,6 +238,7 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
     const int after = buf + 1 == STAGES ? 0 : buf + 1, before = buf == 0 ? STAGES - 1 : buf - 1;
     const char* here = lds + buf * STAGE;
     const char* there = lds + after * STAGE;
+    int own = before * STAGE + wave * 1024;   // of the tile that is asked for
     bf16x8_t xr[2 * TM + AHEAD];
 #pragma unroll
     for (int q = 0; q < AHEAD; ++q) xr[q] = xf[q];
@@ -238,7 +255,7 @@ __global__ __launch_bounds__(64 * kWaves, PER_CU) void gemm_panel_q_kernel(
       constexpr int ASKED = loads_of<QB>(LOADS, HALF + STAGES - 1, 1);
 #pragma unroll
       for (int p = 0; p < ASKED; ++p)
-        if (s == 1 && p * TM / ASKED == i) load(before, t + STAGES - 1, p);
+        if (s == 1 && p * TM / ASKED == i) load(own, t + STAGES - 1, p);
       if constexpr (QB == 4 && HALF == 0)
         if (q == 0)
 #pragma unroll

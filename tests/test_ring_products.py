@@ -86,3 +86,33 @@ def test_sums_and_fragments_stay_in_place(name, least, tmp_path):
                     for line in behind)
         assert waits >= 18, (kernel, behind)
     assert kernels >= least
+
+
+@pytest.mark.skipif(OBJDUMP is None, reason="no llvm-objdump")
+def test_a_large_panel_computes_no_places_for_its_loads(tmp_path):
+    """In int8 panels of 160 x 256 (gemm_panel_q.h) a wave is alone on its SIMD, and every instruction
+    beyond those that hide behind the products takes its four clocks: a load's place in LDS is a
+    register and a literal, one instruction each.  (Of remainders, copied: 282 instructions.)"""
+    if not (PACKAGE / "_C.so").exists():
+        pytest.skip("the extension is not built")
+    shutil.copy(PACKAGE / "_C.so", tmp_path / "_C.so")
+    subprocess.run([OBJDUMP, "--offloading", "_C.so"], cwd=tmp_path, check=True,
+                   capture_output=True)
+    loops = []
+    for code in sorted(tmp_path.glob("_C.so.*gfx950")):
+        listing = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", code],
+                                 check=True, capture_output=True, text=True).stdout
+        for part in re.split(r"^\w+ <(?=\w*gemm_panel_q_kernelILi8ELi10ELi4E)", listing,
+                             flags=re.M)[1:]:
+            found = re.findall(r"^\s+(\w[^/]*?)\s*// ([0-9A-F]+):", part.split("\n\n")[0], flags=re.M)
+            at = {int(address, 16): i for i, (_, address) in enumerate(found)}
+            for i, (line, address) in enumerate(found):
+                if branch := re.match(r"s_cbranch\w* (\d+)", line):
+                    words = (int(branch[1]) ^ 0x8000) - 0x8000   # of 16 bits, from behind it on
+                    loop = [line for line, _ in found[at.get(int(address, 16) + 4 + 4 * words, i):i + 1]]
+                    if sum(line.startswith(PRODUCT) for line in loop) == 80:
+                        loops.append(loop)
+    assert len(loops) == 2   # without and with the gate
+    for loop in loops:
+        assert sum(line.startswith("buffer_load") for line in loop) == 9
+        assert len(loop) <= 272, "\n".join(loop)
