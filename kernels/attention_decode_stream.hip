@@ -417,7 +417,8 @@ void launch(__hip_bfloat16* out, float* part_acc, float* part_ml, const __hip_bf
             hipStream_t stream) {
   int shift = -1;
   if ((block_size & (block_size - 1)) == 0) shift = __builtin_ctz(block_size);
-  const int alone = decode_alone_tiles(nseq, kvh);
+  // (a wave's results of a head by itself are stored by 8 bytes, a workgroup's one by one)
+  const int alone = reinterpret_cast<uintptr_t>(out) % 8 == 0 ? decode_alone_tiles(nseq, kvh) : -1;
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(nseq, kvh, npart), dim3(256), 0, stream, out, part_acc, part_ml,
                        q, kc, vc, bt, sl, scale * kLog2e, nheads, kvh, nheads / kvh, block_size,

@@ -128,3 +128,32 @@ def test_heads_of_short_sequences_are_a_waves_each(fp8, kvh, group, hd, nseq, wi
     # as above
     assert (out[live] - want).abs().max() <= 2 ** -8 * vc.float().abs().max()
     assert not out[[i for i, n in enumerate(lens) if not n]].any()
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize(("dim", "off"), [(64, 1), (128, 2), (128, 3), (128, 4)])
+def test_results_off_an_8_byte_boundary_are_stored_one_by_one(fp8, dim, off):
+    """Short sequences, so many that elsewhere a wave has a key head; `off` results into the
+    buffer a workgroup does, as in batches of half the size, whose bits these are."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from vllm_tgis_adapter_amd import ops
+
+    lens = [(17, 33, 50, 64)[i % 4] for i in range(80)]
+    kc, vc, tables = (t.cuda() for t in _caches(lens, 16, 8, dim, fp8, 7, 4))
+    q = torch.randn(80, 32, dim, generator=torch.Generator().manual_seed(8)).bfloat16().cuda()
+    seq_lens = torch.tensor(lens, dtype=torch.int32, device="cuda")
+
+    def decode(out, rows):
+        ops._C.paged_attention_decode(out, q[rows], kc, vc, tables[rows], seq_lens[rows],
+                                      dim ** -0.5)
+        return out
+
+    halves = torch.cat([decode(torch.empty_like(q[:40]), slice(i, i + 40)) for i in (0, 40)])
+    whole = torch.full((q.numel() + 8,), 7.0, dtype=q.dtype, device="cuda")
+    got = decode(whole[off:off + q.numel()].view_as(q), slice(0, 80))
+    if off % 4:
+        assert torch.equal(got, halves)
+    else:   # on such a boundary; sums in another order, rounded to 8 bits
+        assert (got - halves).abs().max() <= 2 ** -8 * halves.abs().max()
+    assert (whole[:off] == 7).all() and (whole[off + q.numel():] == 7).all()
