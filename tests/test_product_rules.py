@@ -45,6 +45,14 @@ def test_4_bit_panels_fit(n, k):
             assert (parts - 1) * groups < k // 128 <= parts * groups
 
 
+@pytest.mark.parametrize("qbits", [8, 4])
+def test_longest_rows_are_widened(qbits):
+    """Past the longest K that the kernels take (gemm_q) only the pass over a widened matrix is left."""
+    for n in (128, 512, 16384):
+        assert ops._quant_rows(qbits, n, (1 << 24) - 128) >= 900
+        assert ops._quant_rows(qbits, n, 1 << 24) <= 64
+
+
 # of up to 64 rows
 FEW_PANELS = [(2, 1), (2, 2), (3, 1), (3, 2), (4, 1), (4, 2)]
 

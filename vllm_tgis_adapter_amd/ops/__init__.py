@@ -372,7 +372,9 @@ def _quant_rows(qbits: int, n: int, k: int) -> int:
     rows 201 | 263, 1200 rows 288 | 311, 1500 rows 365 | 332, 4096 x 14336 800 rows 112 | 130, 1200
     rows 158 | 155, 6144 x 4096 800 rows 53 | 55, 1000 rows 64 | 61, 10240 x 8192 800 rows
     152 | 163, 1000 rows 199 | 172, 8192 x 28672 1200 rows 566 | 576, 1500 rows 721 | 635, 2048 x
-    2048 1500 rows 20 | 28."""
+    2048 1500 rows 20 | 28.  (Rows of W of 2^24 weights are past the kernels' 32-bit places.)"""
+    if k >= 1 << 24:
+        return 64
     if n * k <= 1 << 23:
         return 1500
     return 1200 if qbits == 8 or n >= 16384 or k > 8192 else 900
