@@ -62,6 +62,7 @@ void launch_gemm_ring(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hi
 void launch_gemm_stream(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hip_bfloat16*,
                         int, int, int, int, hipStream_t);
 bool gemm_row_fits(int K);
+int gemm_row_form(int qbits, int mode, int N, int K);
 void launch_gemm_row_norm_gated(__hip_bfloat16*, __hip_bfloat16*, const __hip_bfloat16*,
                                 const __hip_bfloat16*, const __hip_bfloat16*, float, const void*,
                                 const float*, int, int, int, hipStream_t);
@@ -972,6 +973,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "which panel products of many rows with rounded weights take, and parts of K (panel << 8 | "
         "parts)", py::arg("m"), py::arg("n"), py::arg("k"), py::arg("qbits") = 8);
   m.def("gemm_panel_few_plan", &gemm_panel_few_plan, "the same up to 64 rows, 0: no panel");
+  m.def("gemm_row_form", &gemm_row_form,
+        "waves of a workgroup for products of one row, and those K is dealt to (waves << 4 | those); "
+        "mode 0 plain, 1 gated, 2 turned", py::arg("qbits"), py::arg("mode"), py::arg("n"), py::arg("k"));
   m.def("row_norm_gated", &row_norm_gated, "norm and gated product of one row (CDNA4)");
   m.def("row_norm_turn", &row_norm_turn,
         "norm, query / key / value product, rotation and cache write of one row (CDNA4)");

@@ -412,62 +412,113 @@ void launch(const RowCall& c) {
                      static_cast<const unsigned char*>(c.w), c.scale, c.N, c.K, c.norm, c.turns);
 }
 
-// Waves of a workgroup, and over how many of them K is dealt (us, N x K, W/KS).  With eight waves half
-// as many workgroups stage x, and of long K more is asked for at once; K dealt to more waves leaves
-// shorter chains where rows are few, to fewer less to add up and more rows that share x.
-//   bf16, 4/4 | 8/8: 2048 x 8192 8.43 | 7.65, 4096 x 14336 21.7 | 20.7, 8192 x 28672 77.4 | 74.9, 4096 x 7168
-//     11.74 | 11.40, 768 x 8192 5.90 | 5.04; 2560 x 8192 9.85 | 10.04 (640 blocks, 512 workgroups); 8192 x
-//     8192 24.4 | 24.6, 8/4 24.0; 16384 x 8192 44.9 | 46.6, 8/4 44.5; to 4096 inputs 8/8 loses 6 %.
-//     Gated, 4/4 | 4/2 | 8/4: 8192 x 2048 13.71 | 13.03 | 13.40, 3072 x 1024 5.63 | 5.19, 28672 x 8192 147.0 |
-//     149.3 | 145.2, 7168 x 8192 42.3 | 42.5 | 41.1, 14336 x 4096 38.8 | 39.2 | 38.6.  Turned, 4/4 | 8/8 | 8/4:
-//     1280 x 8192 8.86 | 7.83 | 8.24, 5120 x 8192 18.8 | 17.8 | 18.5, 10240 x 8192 31.6 | 31.2 | 30.8, 6144 x 4096
-//     10.8 | 11.2 | 11.2.
-//   int8, 4/4 | 8/4: 8192 x 28672 46.1 | 40.5, 4096 x 14336 12.6 | 12.2, 2048 x 8192 6.09 | 5.78, 4096 x 4096
-//     5.79 | 5.83.  Gated, 4/4 | 4/2 | 8/4: 14336 x 4096 24.0 | 22.0 | 23.3, 7168 x 4096 13.4 | 12.9 | 13.6, 28672 x
-//     8192 78.7 | 80.0 | 76.3; 4/2 | 4/1: 8192 x 2048 9.06 | 8.63, 2048 x 2048 4.92 | 4.84.  Turned, 4/4 |
-//     8/4: 6144 x 4096 8.25 | 7.78, 10240 x 8192 18.6 | 17.5, 3072 x 4096 6.36 | 6.52.
-//   4 bits (a load covers 2048 inputs), plain, 4/4 | 8/2 | 8/4 | 8/8: 8192 x 28672 34.5 | 27.6 | 29.8 | 31.0,
-//     4096 x 14336 11.08 | 10.51 | 10.92 | 11.32, 8192 x 8192 11.7 | 11.6 | 11.6 | 11.8, 4096 x 7168 7.20 | 7.11 |
-//     6.65 | 7.39, 2048 x 8192 5.38 | 6.47 | 4.98 | 5.06, 1024 x 8192 4.12 | 5.86 | 4.25 | 3.88.  Shorter
-//     K, and with pairs: rows go first where they are many (14336 x 4096 gated 4/1 16.9, 4/2 17.9; 2048 x
-//     8192 4/1 7.0, 4/2 5.5).
-template <int MODE, bool NORM>
-void launch_bits(const RowCall& c, int qbits) {
-  const int rows = MODE == kRowGated ? 2 * c.N : c.N;
-#define GO(QB, W, KS) launch<QB, MODE, KS, NORM, W>(c)
+// The rows of W that the busiest CU has when workgroups take `cols` of N at a time.
+int busiest(int N, int cols) { return (N / cols + 255) / 256 * cols; }
+
+// How many workgroups share a CU's LDS, for the row that each keeps there, and whether that is fewer than
+// four of four waves.
+int resident(int K) { return 80 * 1024 / (K + 64); }
+bool crowded(int K) { return resident(K) < 4; }
+
+}  // namespace
+
+// Waves of a workgroup, and over how many of them K is dealt: waves << 4 | those.  A function of sizes.
+// With eight waves half as many workgroups stage x, and of long K more is asked for at once; K dealt to
+// more waves leaves shorter chains where rows are few, to fewer less to add up and more rows that share
+// x.  Workgroups that take more rows (16 by 8/2 and 4/1, 8 by 8/4 and 4/2, 4 by 4/4 and 8/8) leave CUs
+// with fewer rows than others: `busiest`.  us, N x K, W/KS:
+//   bf16, plain: up to 2048 rows all workgroups of 8/8 are there at once, 4/4 | 8/8: 2048 x 8192 8.70 | 7.78,
+//     768 x 8192 6.01 | 4.97, 128 x 7168 5.46 | 4.17 (to 4096 inputs 8/8 loses 6 %); up to 4096 only
+//     those of 4/4 are: 2176 x 10240 10.54 | 11.09, 2560 x 14336 14.5 | 14.8, 3072 x 8192 11.1 | 10.9, but
+//     crowded, 2560 x 28672 33.8 | 26.1; past that neither are: 5120 x 8192 16.6 | 16.0, 4608 x 14336 24.7 |
+//     23.0, 9216 x 14336 41.6 | 40.1, 7168 x 9216 22.2 | 22.7.  Many sums of eight waves are seen while K
+//     is short, 4/4 | 8/8 | 8/4: 16384 x 8192 42.8 | 44.3 | 42.7, 8192 x 8192 23.3 | 23.4 | 23.1, 20480 x
+//     7168 45.7 | .. | 44.5, 6144 x 8192 18.5 | 18.3 | 18.3, 16384 x 9216 47.2 | 46.8 | 45.7.
+//     Gated, 4/4 | 4/2, two loads of K: 3072 x 1024 5.77 | 5.18; four: 8192 x 2048 13.5 | 12.4, 2048 x 2048
+//     6.05 | 5.88, but 1024 x 2048 4.73 | 5.16; three, of which one of two waves has two: 8192 x 1280
+//     10.3 | 9.6, 5120 x 1280 7.40 | 7.72, 2048 x 1280 5.14 | 5.37.  Long K, 4/4 | 8/4: 28672 x 8192 147.0 | 145.2,
+//     2048 x 8192 15.2 | 13.4, 128 x 8192 7.00 | 6.78 (14336 x 4096 38.8 | 38.6).
+//     Turned, 4/4 | 8/8 | 8/4: 1280 x 8192 8.52 | 7.69 | 8.24, 5120 x 8192 17.9 | 17.2 | 18.5, 6144 x 10240 23.8 |
+//     22.6 | 22.4, 10240 x 8192 31.6 | 31.2 | 30.8 (6144 x 4096 10.8 | 11.2 | 11.2).
+//   int8, plain, 4/4 | 8/4: 4096 x 14336 12.5 | 12.1, 2048 x 8192 6.2 | 5.8, 1280 x 14336 7.7 | 7.1, 10240 x
+//     14336 25.7 | 24.6 (4096 x 4096 5.79 | 5.83); a CU with more rows: 256 x 14336 5.80 | 6.42, 2560 x
+//     14336 9.6 | 10.2, 4608 x 8192 8.55 | 8.89; crowded, 3328 x 20480 17.6 | 13.4, 2560 x 28672
+//     19.9 | 17.0.
+//     Gated, a load of K, 4/2 | 4/1: 14336 x 1024 9.7 | 8.4, 512 x 1024 3.72 | 3.66; two: 8192 x 2048 9.0 |
+//     8.5, 4096 x 2048 6.6 | 6.1, 5120 x 1280 6.0 | 6.6, 1024 x 2048 4.1 | 4.5.  Longer, 4/4 | 4/2: 14336 x 4096
+//     22.2 | 20.8, 2048 x 4096 7.0 | 6.5, 512 x 4096 4.3 | 4.8, 1152 x 2560 5.2 | 5.4; 4/4 | 8/4: 28672 x
+//     8192 73.4 | 72.0, 2048 x 8192 10.5 | 8.7, 128 x 8192 5.5 | 5.4.  Turned, 4/4 | 8/4: 6144 x 4096 8.0 |
+//     7.4, 10240 x 8192 17.4 | 16.2, 3072 x 4096 6.36 | 6.52.
+//   4 bits (a load covers 2048 inputs), plain, K past three loads.  Up to 2047 rows, 4/4 | 8/8: 1024 x 8192
+//     4.30 | 4.02, 128 x 28672 7.3 | 6.5.  Four loads, 4/4 | 8/4, all workgroups there at once: 4096 x 8192
+//     7.31 | 6.75, 2048 x 8192 5.44 | 5.02; more rows, 4/4 | 4/2 | 8/2: 5120 x 8192 8.4 | 8.8 | 9.7, 6144 x
+//     7168 9.0 | 8.8 | 9.3, 8192 x 8192 11.1 | 10.5 | 10.8, 10240 x 8192 12.9 | 12.1 | 13.6, 28672 x 8192
+//     27.0 by 4/1 | 25.4 | 27.6.  Longer, 8/2 where CUs have as many rows as with fewer a workgroup, 4/4 | 4/2 | 8/2:
+//     4096 x 14336 10.4 | 10.0 | 10.2, 7680 x 14336 16.1 | .. | 14.6, 8192 x 14336 16.2 | 15.6 | 14.9, but
+//     4608 x 14336 11.5 | 12.2 | 13.5, 5120 x 10240 9.6 | 10.2 | 10.7, 10240 x 14336 18.0 | 17.6 | 18.6, 14336 x 14336 22.9 | 22.9 |
+//     24.5, 2560 x 14336 8.8 by 4/4 | 9.1; past 16384, 4/1 | 8/2: 57344 x 14336 71 | 75, 28672 x 14336 39.1 | 39.2.
+//     Crowded, 4/4 | 8/2 | 8/4 | 8/8: 8192 x 28672 31 | 24.6 | 26.6 | 27.3, 4096 x 28672 19.7 | 14.9 | 16.3 | 16.8,
+//     6144 x 28672 25.1 | 23.0 | 20.7 | 22.3, 5120 x 28672 22.8 | 22.8 | 20.1 | 19.0.
+//     Shorter K, and with pairs: rows go first where they are many (14336 x 4096 gated 4/1 16.9, 4/2 17.9;
+//     2048 x 8192 4/1 7.0, 4/2 5.5).
+int gemm_row_form(int qbits, int mode, int N, int K) {
+  constexpr int k41 = 0x41, k42 = 0x42, k44 = 0x44, k82 = 0x82, k84 = 0x84, k88 = 0x88;
+  const int r4 = busiest(N, 4), r8 = busiest(N, 8), r16 = busiest(N, 16);
   if (qbits == 16) {
-    if constexpr (MODE == kRowPlain) {
-      if (c.K >= 7168 && (c.N <= 2048 || (c.N >= 4096 && (c.N < 8192 || c.K > 8192))))
-        return GO(16, 8, 8);
-      if (c.K >= 7168 && c.N >= 8192) return GO(16, 8, 4);
-    } else if constexpr (MODE == kRowGated) {
-      if (c.K <= 2048) return GO(16, 4, 2);
-      if (c.K >= 8192) return GO(16, 8, 4);
-    } else if (c.K >= 8192) {
-      return c.N <= 5120 ? GO(16, 8, 8) : GO(16, 8, 4);
-    }
-    return GO(16, 4, 4);
+    if (mode == kRowGated)
+      return K >= 8192 ? k84
+             : K <= 1024 || (K <= 2048 && N >= (K > 1536 ? 2048 : 8192)) ? k42 : k44;
+    if (mode == kRowTurn) return K < 8192 ? k44 : N <= 5120 ? k88 : k84;
+    if (K < 7168 || (N > 2048 && N < 4096 && !crowded(K))) return k44;
+    return N >= 8192 && K <= 8192 ? k84 : k88;
   }
   if (qbits == 8) {
-    if constexpr (MODE == kRowGated) {
-      if (c.K <= 2048) return GO(8, 4, 1);
-      if (c.K < 8192) return GO(8, 4, 2);
-      return GO(8, 8, 4);
-    } else {
-      if (c.K <= 2048) return GO(8, 4, 2);
-      if (MODE == kRowTurn ? c.K >= 4096 && c.N >= 6144 : c.K >= 7168) return GO(8, 8, 4);
-      return GO(8, 4, 4);
+    if (mode == kRowGated) {
+      if (K <= 2048) return K <= 1024 || N >= (K > 1792 ? 3584 : 8192) ? k41 : k42;
+      return K >= 8192 ? k84 : N >= 1280 ? k42 : k44;
     }
+    if (K <= 2048) return k42;
+    if (mode == kRowTurn) return K >= 4096 && N >= 6144 ? k84 : k44;
+    return K >= 7168 && (r8 <= r4 || (crowded(K) && r4 > 4 * resident(K))) ? k84 : k44;
+  }
+  const int rows = mode == kRowGated ? 2 * N : N;
+  if (mode != kRowPlain || K <= 2048 * 3)
+    return mode != kRowPlain && K > 2048 * 3 && rows <= 8192 ? k44
+           : K > 2048 && rows <= 16384                       ? k42 : k41;
+  if (N < 2048) return k88;
+  if (K <= 8192) return N <= 4096 ? k84 : N > 8192 || r8 <= r4 ? k42 : k44;
+  if (crowded(K)) return r16 <= r8 ? k82 : r8 <= r4 ? k84 : k88;
+  if (N > 16384) return k41;
+  if (r16 <= r8 && (N > 4096 || r16 <= r4)) return k82;
+  if (N <= 4096) return r8 <= r4 ? k84 : k44;
+  return N > 8192 || r8 <= r4 ? k42 : k44;
+}
+
+namespace {
+
+template <int MODE, bool NORM>
+void launch_bits(const RowCall& c, int qbits) {
+  const int form = gemm_row_form(qbits, MODE, c.N, c.K);
+#define GO(QB, W, KS) if (qbits == QB && form == (W << 4 | KS)) return launch<QB, MODE, KS, NORM, W>(c)
+  GO(16, 4, 4);
+  GO(16, 8, 4);
+  GO(8, 4, 4);
+  GO(8, 4, 2);
+  GO(8, 8, 4);
+  GO(4, 4, 4);
+  GO(4, 4, 2);
+  if constexpr (MODE == kRowGated) {
+    GO(16, 4, 2);
+    GO(8, 4, 1);
+  } else {
+    GO(16, 8, 8);
   }
   if constexpr (MODE == kRowPlain) {
-    if (c.K > 2048 * 3) {
-      if (c.N < 2048) return GO(4, 8, 8);
-      return c.N > 4096 || (c.N == 4096 && c.K > 8192) ? GO(4, 8, 2) : GO(4, 8, 4);
-    }
+    GO(4, 8, 2);
+    GO(4, 8, 4);
+    GO(4, 8, 8);
   }
-  if (MODE != kRowPlain && c.K > 2048 * 3 && rows <= 8192) return GO(4, 4, 4);
-  if (c.K > 2048 && rows <= 16384) return GO(4, 4, 2);
-  GO(4, 4, 1);
+  launch<4, MODE, 1, NORM, 4>(c);
 #undef GO
 }
 

@@ -166,3 +166,38 @@ def test_few_rows_are_not_asked_for():
         for n in (128, 2048, 14336, 28672):
             for k in (64, 2048, 8192, 28672):
                 assert not ops._tiles_take(m, n, k)
+
+
+# waves, and those that K is dealt to: forms within 4 % of the fastest at sizes around every line of the rule
+@pytest.mark.parametrize(("bits", "mode", "n", "k", "forms"), [
+    (4, 0, 128, 8192, {0x88}), (4, 0, 1024, 28672, {0x88}), (4, 0, 2048, 8192, {0x84, 0x88}),
+    (4, 0, 2560, 14336, {0x44, 0x88, 0x82}), (4, 0, 3072, 10240, {0x44, 0x88}),
+    (4, 0, 3584, 7168, {0x84}), (4, 0, 3584, 14336, {0x82, 0x42, 0x84}), (4, 0, 3968, 14336, {0x82, 0x42, 0x84}),
+    (4, 0, 4096, 8192, {0x84}), (4, 0, 4096, 14336, {0x82, 0x42}), (4, 0, 4096, 28672, {0x82}),
+    (4, 0, 4224, 7168, {0x44, 0x88}), (4, 0, 4608, 7168, {0x44, 0x88}), (4, 0, 4608, 14336, {0x44}),
+    (4, 0, 5120, 8192, {0x44, 0x88}), (4, 0, 5120, 14336, {0x44}), (4, 0, 5120, 28672, {0x88}),
+    (4, 0, 6144, 8192, {0x42, 0x84, 0x88, 0x44}), (4, 0, 6144, 28672, {0x84}), (4, 0, 7680, 14336, {0x82}),
+    (4, 0, 8192, 8192, {0x42, 0x82}), (4, 0, 8192, 28672, {0x82}), (4, 0, 9216, 8192, {0x42, 0x88}),
+    (4, 0, 10240, 8192, {0x42}), (4, 0, 10240, 14336, {0x42, 0x44}), (4, 0, 14336, 8192, {0x42}),
+    (4, 0, 28672, 8192, {0x42}), (4, 0, 57344, 14336, {0x41}), (4, 0, 57344, 28672, {0x82}),
+    (8, 0, 256, 14336, {0x44}), (8, 0, 1280, 14336, {0x84}), (8, 0, 2560, 14336, {0x44, 0x82}),
+    (8, 0, 4096, 8192, {0x84}), (8, 0, 4608, 8192, {0x44}), (8, 0, 2560, 28672, {0x84}),
+    (8, 0, 3328, 20480, {0x84}), (8, 0, 8192, 28672, {0x84}),
+    (8, 1, 512, 1024, {0x41, 0x42}), (8, 1, 768, 2048, {0x42}), (8, 1, 8192, 2048, {0x41}),
+    (8, 1, 5120, 1280, {0x42}), (8, 1, 512, 4096, {0x44}), (8, 1, 14336, 4096, {0x42}),
+    (16, 1, 768, 2048, {0x44, 0x84}), (16, 1, 3072, 1024, {0x42}), (16, 1, 2048, 1280, {0x44, 0x84}),
+    (16, 1, 8192, 2048, {0x42}), (16, 0, 2176, 10240, {0x44}), (16, 0, 2048, 8192, {0x88}),
+    (16, 0, 2560, 28672, {0x88}), (16, 0, 5120, 14336, {0x88}), (16, 0, 16384, 8192, {0x44, 0x84})])
+def test_one_row_forms_that_measured_well(bits, mode, n, k, forms):
+    assert ops._C.gemm_row_form(bits, mode, n, k) in forms
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize(("bits", "made"), [
+    (16, [{0x44, 0x84, 0x88}, {0x44, 0x84, 0x42}, {0x44, 0x84, 0x88}]),
+    (8, [{0x44, 0x42, 0x84}, {0x44, 0x42, 0x84, 0x41}, {0x44, 0x42, 0x84}]),
+    (4, [{0x44, 0x42, 0x41, 0x82, 0x84, 0x88}, {0x44, 0x42, 0x41}, {0x44, 0x42, 0x41}])])
+def test_one_row_forms_are_built(bits, mode, made):
+    for n in (128, 384, 1152, 2048, 2176, 3072, 4096, 4224, 6144, 8192, 9216, 14336, 16512, 57344):
+        for k in (128, 1024, 1280, 2048, 2176, 6144, 6272, 7168, 8192, 8320, 14336, 20480, 28672):
+            assert ops._C.gemm_row_form(bits, mode, n, k) in made[mode]

@@ -121,9 +121,10 @@ def test_int8_products_of_one_row(n, k):
 @pytest.mark.parametrize(("n", "k"), [
     (128, 7168), (2048, 7296),       # a K that ends inside a wave's load
     (2176, 8320), (4096, 8192), (4096, 14464), (4224, 6400), (8192, 7168), (8320, 8320),
-    (16512, 7168)])                  # more rows than the workgroups take at a time
+    (16512, 7168), (16512, 8320),    # more rows than the workgroups take at a time
+    (256, 28672), (2688, 28672), (6144, 20480), (4608, 20480)])   # rows that fill LDS
 def test_long_rows(bits, n, k):
-    """Plain products on both sides of where workgroups of eight waves begin."""
+    """Plain products of every form, on both sides of where workgroups of eight waves begin."""
     from vllm_tgis_adapter_amd import ops
 
     gen = torch.Generator("cuda").manual_seed(n + k + bits)
@@ -134,7 +135,9 @@ def test_long_rows(bits, n, k):
 
 
 @pytest.mark.parametrize("bits", [16, 8, 4])
-@pytest.mark.parametrize(("k", "inter"), [(1920, 640), (2176, 1280), (8320, 4224), (8192, 14336)])
+@pytest.mark.parametrize(("k", "inter"), [
+    (1024, 640), (1920, 640), (2048, 4224), (1280, 8320), (2176, 1152), (2176, 1280), (8320, 4224),
+    (8192, 14336)])
 def test_gates_of_long_rows(bits, k, inter):
     from vllm_tgis_adapter_amd import ops
 
