@@ -48,6 +48,7 @@ int gemm_ring_plan(int M, int N, int K, bool gated);
 void launch_gemm_ring_parts(__hip_bfloat16*, float*, const __hip_bfloat16*,
                             const __hip_bfloat16*, int, int, int, int, hipStream_t);
 bool gemm_ring_takes(int N, int K, int plan, bool gated);
+bool gemm_ring_reads_once(int M, int N, int K, int plan, bool gated);
 int gemm_ring_lora_cuts(int M, int K, int L, int PR, int plan);
 bool gemm_ring_lora_wins(long M, long N, long K);
 void launch_gemm_ring_lora(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hip_bfloat16*,
@@ -1003,6 +1004,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "past 64 rows: 1 for their cut K, 2 otherwise, 0 where the library is faster");
   m.def("gemm_block_takes", &gemm_block_takes, "whether they are for their cut K");
   m.def("gemm_ring_plan", &gemm_ring_plan, "which tile a product takes, and parts of K (form << 4 | parts)");
+  m.def("gemm_ring_reads_once", &gemm_ring_reads_once, "whether its weights go past the caches",
+        py::arg("m"), py::arg("n"), py::arg("k"), py::arg("plan"), py::arg("gated") = false);
   m.def("decode_inputs", &decode_inputs, "a captured step's inputs from a packed host buffer");
   m.def("lora_product", &lora_product, "a product with its LoRA deltas, also gated");
   m.def("gemm_ring_lora_wins", &gemm_ring_lora_wins, "whether the tiles take a product with adapters");

@@ -164,18 +164,19 @@ int even_parts(int K, int parts) {
 // are CUs (K cut), or two a CU where that leaves a quarter of them idle or K stays long, and W
 // past the caches.  us, the streaming kernel | 64 x 128 by a cost model | here, N x K, 24 |
 // 64 rows: 28672 x 4096 44.7 48.8 39.9 | 52.2 49.9 47.3; 4096 x 14336 26.8 27.7 24.1 | 37.3 29.4
-// 28.8; 6144 x 4096 15.9 15.4 14.8 | 21.6 17.3 18.1; 4096 x 4096 12.1 12.7 11.5 | 16.5 14.2 12.6;
-// 16384 x 2048 16.6 17.1 15.5 | 20.6 19.2 16.5; 8192 x 28672 83 83 75 | 101 90 96.  Workgroups 128,
-// 256, 512 at 8192 x 28672, 24 rows: 130, 90, 75; at 4096 x 14336 64, 128, 256, 512: 54, 33, 24, 27;
-// 172 and 344 at 11008 x 4096: 20.2, 24.2.
+// 28.8; 4096 x 4096 12.1 12.7 11.5 | 16.5 14.2 12.6; 16384 x 2048 16.6 17.1 15.5 | 20.6 19.2 16.5.
+// Workgroups 128, 256, 512 of 64 columns at 8192 x 28672, 24 rows: 130, 90, 75; at 4096 x 14336 64, 128,
+// 256, 512: 54, 33, 24, 27; 172 and 344 at 11008 x 4096: 20.2, 24.2.
 // Short K is cut less, eight tiles a part: 40 rows, 3072 x 2048 in 4 8.9 (in 5 9.4, whole 10.7), 8192
 // x 1024 whole 7.3 (in 2 8.0).  Past 48 rows of very many weights the tile of 128 columns reads x half
-// as often: 64 rows, 57344 x 8192 175 | 183, 8192 x 28672 in 4 90 | 96 (14336 x 8192 60 | 47, 28672 x
-// 8192 98 | 89).
+// as often, 128 | 64 columns: 64 rows, 57344 x 8192 175 | 183, 8192 x 28672 in 4 90 | 96 (14336 x 8192
+// 60 | 47, 28672 x 8192 98 | 89).
 // For fewer rows too it is faster where columns of 64 would be cut and still be two a CU (one a CU then),
 // and, with K cut further, where they would be cut in two (half the barriers for as many bytes).  us, 64 |
 // 128 columns, 17 rows, 64 rows: 10240 x 8192 in 3 32.2 | 30.5, 38.7 | 33.7; 10240 x 2048 in 3 12.6 | 11.8,
-// 17.4 | 15.8; 14336 x 14336 in 2 75.9 | 63.3, 94.2 | 72.6; in 2 | in 4: 6144 x 4096 13.7 | 12.7, 17.2 | 16.7;
+// 17.4 | 15.8; 14336 x 14336 in 2 75.9 | 63.3, 94.2 | 72.6; 9, 24, 48 rows, 8192 x 28672 in 4 72.2 | 71.2, 76.2 |
+// 72.6, 87.2 | 77.4; 5120 x 28672 in 6 49.3 | 48.0, 52.3 | 49.3, 60.7 | 52.3; 10240 x 28672 in 3 97 | 91, 104 |
+// 93, 118 | 97; of 23 such matrices, 9 to 64 rows, none is 1 % slower; in 2 | in 4: 6144 x 4096 13.7 | 12.7, 17.2 | 16.7;
 // 8192 x 4096 16.5 | 14.6, 18.2 | 16.4; 6144 x 14336 33.1 | 31.5, 43.4 | 38.5; but 6144 x 2048 8.9 | 9.6;
 // in 2 | in 3: 8192 x 8192 27.3 | 25.1, 29.8 | 28.7; but 6144 x 8192 22.2 | 22.8, 27.5 | 28.0.
 Plan few_rows(int M, int N, int K) {
@@ -204,8 +205,11 @@ Plan few_rows(int M, int N, int K) {
 // rounds are counted there (84 tiles in three parts are 33 workgroups on some XCDs, two rounds,
 // though all are 252: 1.5 times the time of 80 tiles).
 Plan plan_of(int M, int N, int K, bool gated) {
-  // (gated, past one and a half rounds of two a CU, of 64 | 128 rows of W, us at 17, 40, 64 rows: 28672 x
-  // 8192 146 | 142, 155 | 145, 174 | 152; but 20480 x 5120 76 | 84, 94 | 96)
+  // (gated: past one and a half rounds of two a CU of 64 rows of W, which are two then, 128 are one.  us, 64 |
+  // 128 at 17, 40, 64 rows, up to the line and past it: 24576 x 2048 36.7 | 39.9, 37.3 | 41.1, 39.7 | 42.8, 24704
+  // x 2048 43.4 | 40.6, 44.5 | 42.0, 48.1 | 43.5; 24576 x 4096 63 | 70, 66 | 73, 71 | 76, 24704 x 4096 75 | 71, 79 |
+  // 74, 87 | 78; 24576 x 5120 80 | 88, 90 | 93, 99 | 100, 24704 x 5120 96 | 87, 109 | 93, 122 | 100; farther off,
+  // 20480 x 5120 76 | 84, 94 | 96, 28672 x 8192 146 | 142, 155 | 145, 174 | 152)
   if (M <= 64) return gated ? Plan{N > 24576 ? kNarrow : kFew, 1, 0.0} : few_rows(M, N, K);
   Plan best{0, 1, 1e30};
   const double cols = gated ? 2.0 * N : N, w_mb = cols * K * 2e-6;
@@ -239,10 +243,14 @@ Plan plan_of(int M, int N, int K, bool gated) {
   return best;
 }
 
-// W that is read once and is large goes past the caches (24 rows by 64 x 64: 28672 x 4096 46.4 ->
-// 39.9 us, 8192 x 3584 15.6 -> 13.8, 4096 x 4096 11.5 -> 11.5, 64 rows 12.6 -> 13.5; larger tiles, all
-// rows in one: 8192 x 8192 by 128 x 128 0.88 of the time, 4096 x 14336 0.91, 5120 x 8192 0.97, but
-// 7168 x 4096 1.02, 6144 x 4096 1.05)
+// W that is read once and is large goes past the caches, by tiles of up to 64 rows from 20 million weights
+// on, by larger ones from 40 (64 x 64, 24 rows: 28672 x 4096 46.4 -> 39.9 us, 8192 x 3584 15.6 -> 13.8, 4096 x
+// 4096 11.5 -> 11.5, 64 rows 12.6 -> 13.5; 64 x 128, 17, 40, 64 rows: 8192 x 4096 17.3 -> 14.6, 17.8 -> 15.4, 18.7 ->
+// 16.4, 6144 x 4096 13.6 -> 13.0, 15.8 -> 14.8, 17.2 -> 16.9, 5120 x 4096 12.6 -> 12.0, 13.8 -> 13.7, 15.1 -> 15.5,
+// 3072 x 8192 18.4 -> 17.6, 21.4 -> 19.4, 22.5 -> 21.3, but 10240 x 2048 12.6 -> 12.2, 13.8 -> 14.1, 14.8 -> 16.1,
+// and below the line 4096 x 4096 11.7 -> 11.4, 13.0 -> 12.8, 14.2 -> 14.5; larger tiles, all rows in one: 8192
+// x 8192 by 128 x 128 0.88 of the time, 4096 x 14336 0.91, 5120 x 8192 0.97, but 7168 x 4096 1.02, 6144 x
+// 4096 1.05)
 bool read_once(int M, long weights, int form) {
   return M <= kForms[form].bm && weights >= (form >= kNarrow ? 20000000 : 40000000);
 }
@@ -311,6 +319,11 @@ void launch_gemm_merge(__hip_bfloat16* y, const float* part, long plane, int par
 int gemm_ring_plan(int M, int N, int K, bool gated) {
   const Plan p = plan_of(M, N, K, gated);
   return p.form << 4 | p.parts;
+}
+
+// Whether a product's weights go past the caches.
+bool gemm_ring_reads_once(int M, int N, int K, int plan, bool gated) {
+  return read_once(M, (gated ? 2L : 1L) * N * K, plan >> 4);
 }
 
 // Whether a plan is one: a tile's columns fit, no part of K is empty.
@@ -425,8 +438,9 @@ int gemm_ring_lora_cuts(int M, int K, int L, int PR, int plan) {
 
 // Whether these tiles take a product that has adapters, whatever takes it without them: beside other
 // products the shrink is a launch of its own, the deltas go over their rounded results, and where K is
-// cut the sum of the parts is one more; here it is two launches.  us with the deltas, otherwise |
-// here, 4 adapters of rank 16 (captured, cold weights), N x K: rows
+// cut the sum of the parts is one more; here it is two launches, three where the shrink has no room beside
+// the product (gemm_ring_lora_cuts: many adapters or tokens, high ranks).  The rule sees sizes of the product
+// only.  us with the deltas, otherwise | here, 4 adapters of rank 16 (captured, cold weights), N x K: rows
 //   up to 16 rows: 6144 x 4096 2 19.2 | 15.8, 16 21.7 | 16.8; 28672 x 4096 gated 2 49.7 | 45.3; 4096 x 14336
 //    8 30.5 | 26.6; 2048 x 2048 12 11.3 | 8.8; 57344 x 8192 gated 2 174 | 163; 768 x 768 2 8.8 | 9.0; not
 //    4096 x 1792 12.3 | 13.7 (too short to be cut, 64 workgroups); of one row 6144 x 4096 16.4 | 15.0, 2048

@@ -68,14 +68,17 @@ def test_parts(form, parts, k):
     _check(y, x, w, False)
 
 
-# weights of 40 million and more that one tile of rows reads go past the caches, 64 x 64 from 20
+# weights that one tile of rows reads go past the caches: tiles of 64 rows 20 million and more, larger
+# ones 40
 @pytest.mark.parametrize("gated", [False, True])
-@pytest.mark.parametrize("form", range(5))
-def test_weights_read_once(form, gated):
+@pytest.mark.parametrize(("form", "n"), [
+    (0, 15872), (1, 15872), (2, 15872), (3, 15872), (4, 15872), (3, 8192), (4, 8192)])
+def test_weights_read_once(form, n, gated):
     from vllm_tgis_adapter_amd.ops import _C
 
-    n, k = 15872 // (1 + gated), 2560
+    n, k = n // (1 + gated), 2560
     for m in (FORMS[form][0] - 1, FORMS[form][0] + 1):   # read once, and twice
+        assert _C.gemm_ring_reads_once(m, n, k, form << 4 | 1, gated) == (m < FORMS[form][0])
         x, w = _inputs(m, n * (1 + gated), k)
         y = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
         _C.gemm_ring(y, x, w, gated, form << 4 | 1)

@@ -105,12 +105,31 @@ PLANS = [
     (512, 4096, 14336, False, {6, 7, 20}), (56, 14336, 8192, False, {65}),
     (40, 3072, 2048, False, {67, 68}), (40, 8192, 1024, False, {65}),
     (24, 11008, 4096, False, {65}), (24, 10240, 4096, False, {51, 65, 67}),
-    (224, 28672, 8192, True, {1}), (128, 3584, 4096, True, {65})]
+    (224, 28672, 8192, True, {1}), (128, 3584, 4096, True, {65}),
+    # columns of 64 where they fill the chip as they are, of 128 where they would be cut and two a CU
+    (24, 4096, 14336, False, {68}), (24, 8192, 28672, False, {52}), (9, 5120, 28672, False, {54}),
+    (17, 10240, 8192, False, {51}), (24, 14336, 14336, False, {50}), (40, 6144, 4096, False, {52}),
+    (64, 8192, 8192, False, {51}), (17, 6144, 2048, False, {66}), (24, 6144, 8192, False, {66}),
+    # gated, one and a half rounds of columns of 64, and more
+    (17, 24576, 4096, True, {65}), (17, 24704, 4096, True, {49}), (40, 28672, 2048, True, {49})]
 
 
 @pytest.mark.parametrize(("m", "n", "k", "gated", "plans"), PLANS)
 def test_plans_that_measured_well(m, n, k, gated, plans):
     assert ops._C.gemm_ring_plan(m, n, k, gated) in plans
+
+
+@pytest.mark.parametrize(("form", "rows", "least"), [
+    (0, 256, 40), (1, 128, 40), (2, 128, 40), (3, 64, 20), (4, 64, 20)])
+def test_weights_that_go_past_the_caches(form, rows, least):
+    """Millions of weights from which on they do, while all rows are one tile."""
+    for gated in (False, True):
+        def once(m, cols):   # 10240 weights a column
+            return ops._C.gemm_ring_reads_once(m, cols, 10240 // (1 + gated), form << 4 | 1, gated)
+
+        cols = -(-least * 10**6 // 10240)
+        assert once(1, cols) and once(rows, cols)
+        assert not once(rows, cols - 1) and not once(rows + 1, cols)
 
 
 @pytest.mark.parametrize(("m", "n", "k"), [
