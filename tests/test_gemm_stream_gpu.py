@@ -353,7 +353,8 @@ def test_4_bit_panels(m, n, k, panel, parts):
 
 @pytest.mark.parametrize(("m", "n", "k", "panel"), [
     (65, 4096, 128, 0), (65, 14336, 128, 1), (321, 4096, 384, 2), (161, 3072, 384, 3),
-    (511, 8192, 384, 4), (301, 14336, 4096, 5), (257, 8192, 128, 5), (65, 1024, 8192, None)])
+    (511, 8192, 384, 4), (301, 14336, 4096, 5), (257, 8192, 128, 5), (513, 3584, 4096, 6),
+    (131, 4224, 128, 6), (65, 1024, 8192, None)])
 def test_4_bit_gated_panels(m, n, k, panel):
     _need()
     from vllm_tgis_adapter_amd import ops
