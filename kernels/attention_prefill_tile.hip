@@ -693,7 +693,9 @@ Cut waves_of(bool fp8, int nseq, int nheads, int kvh, int max_query_len, int max
 // sixteen prompts of 2 to 8192 tokens, after none to 6000).
 //  - Parts pay for their sums only where tokens are few: one prompt of 1000 in 8 waves, 2 parts 37.8, 1
 //    part 30.9, by 4 waves 29.0; heads of 64 29.0 | 20.3, e4m3 40.0 | 33.3 by 8; after 1000 tokens, heads of 64, 40.9 | 35.4; 64/8
-//    heads, 512 after 1000 46.7 | 41.6; but 1000 after 3000 78.6 | 96.
+//    heads, 512 after 1000 46.7 | 41.6; but 1000 after 3000 78.6 | 96.  Fewer parts than fill the chip,
+//    but some, are never faster: what few tokens leave stays in the caches (10 | 8 parts, e4m3, 2 prompts of
+//    64 after 4000 33.8 | 36.1, 64/8 heads, 64 after 4000 32.1 | 33.7; 15 | 12, 30 after 6000 26.2 | 26.6).
 //  - Uncut, four waves end a workgroup's last tiles sooner, where they are one a CU, or, where many keys
 //    are the prompts' own, two and their tiles few (heads of 64: up to three): 8 | 4 waves, 32/8 heads
 //    of 128, 2 prompts of 1000 33.3 | 32.4, 8 of 256 16.6 | 15.1; of 64, one of 2000 40.4 | 36.6, 4 of 500
@@ -717,9 +719,9 @@ Cut cut_of(bool fp8, int nseq, int nheads, int kvh, int head_dim, int max_query_
            (parts > 1 ? 3.5 + 0.3 * parts + (wide ? 0.21 : 0.35) * mb * parts : 0.0);
   };
   const long fit = 256 * 8 / c.waves / blocks_of(c, nseq, nheads, max_query_len);
-  const int most = max_keys / (kTile * least);
+  const int most = max_keys / (kTile * least), filling = std::max(2, c.parts);
   c.parts = 1;
-  for (int p = 2; p <= 16 && p <= fit && p <= most; ++p)
+  for (int p = filling; p <= 16 && p <= fit && p <= most; ++p)
     if (us(c.waves, p) < us(c.waves, c.parts)) c.parts = p;
   if (c.waves == 8 && !fp8) {
     Cut four{};
@@ -765,12 +767,13 @@ void launch(__hip_bfloat16* out, float* part_acc, float* part_ml, const __hip_bf
 
 }  // namespace
 
-// Workgroups that a prompt's keys may be cut over (a function of shapes only): 1, or the
-// launch needs part_acc [parts, tokens, nheads, head_dim] and part_ml [parts, tokens,
+// Waves of a workgroup << 8 | workgroups that a prompt's keys may be cut over (a function of shapes
+// only): 1, or the launch needs part_acc [parts, tokens, nheads, head_dim] and part_ml [parts, tokens,
 // nheads, 2].
-int prefill_tile_parts(bool fp8, int nseq, int nheads, int kvh, int head_dim, int max_query_len,
-                       int max_keys) {
-  return cut_of(fp8, nseq, nheads, kvh, head_dim, max_query_len, max_keys).parts;
+int prefill_tile_plan(bool fp8, int nseq, int nheads, int kvh, int head_dim, int max_query_len,
+                      int max_keys) {
+  const Cut c = cut_of(fp8, nseq, nheads, kvh, head_dim, max_query_len, max_keys);
+  return c.waves << 8 | c.parts;
 }
 
 void launch_paged_prefill_tile(__hip_bfloat16* out, float* part_acc, float* part_ml,
