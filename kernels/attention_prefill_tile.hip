@@ -701,7 +701,12 @@ Cut waves_of(bool fp8, int nseq, int nheads, int kvh, int max_query_len, int max
 //    of 128, 2 prompts of 1000 33.3 | 32.4, 8 of 256 16.6 | 15.1; of 64, one of 2000 40.4 | 36.6, 4 of 500
 //    after 700 28.8 | 26.4; past that 7 of 500 after 700 67.6 | 70.1, one of 4000 132 | 145; 64/8 heads,
 //    8 of 128 after 600 31.3 | 34.1, one of 2000 73.8 | 79.3; e4m3, 2 prompts of 1000 37.0 | 37.6.
-Cut cut_of(bool fp8, int nseq, int nheads, int kvh, int head_dim, int max_query_len,
+//  - Where lanes find their rows (not `even`: blocks of 24) a tile takes longer, by four waves more so: four
+//    where they are the faster by times of their own (8 | 4 waves, 32/8 heads of 128, one of 512 23.1 | 21.7, 8
+//    of 256 18.3 | 17.3, but one of 1000 36.8 | 37.4, 2 of 1000 38.8 | 39.9, 1000 after 500 in 2 parts 48.3 |
+//    53.4; of 64, one of 1000 25.9 | 24.6, 700 after 700 33.9 | 32.0, but 512 after 1000 in 3 parts 29.4 |
+//    34.1, 3 of 1000 27.2 | 28.4, 64/8 heads, 1500 after 1500 93 | 104).
+Cut cut_of(bool fp8, bool even, int nseq, int nheads, int kvh, int head_dim, int max_query_len,
            int max_keys) {
   Cut c = waves_of(fp8, nseq, nheads, kvh, max_query_len, max_keys);
   const int group = nheads / kvh;
@@ -709,12 +714,15 @@ Cut cut_of(bool fp8, int nseq, int nheads, int kvh, int head_dim, int max_query_
   const bool wide = head_dim == 128;
   const int tiles = (max_keys + kTile - 1) / kTile, least = kMinTiles;
   const double mb = 8e-6 * nseq * max_query_len * nheads * head_dim;   // of a part, there and back
+  const bool lanes = !even && !fp8 && c.waves == 8;   // (e4m3 keys stay with eight waves or four)
   auto us = [&](int waves, int parts) {
     const int per = parts == 1 || tiles <= least ? tiles : std::max(least, (tiles + parts - 1) / parts);
     const double start = fp8    ? (waves == 8 ? 7.0 : 4.5)
                          : wide ? (waves == 8 ? 8.1 : 6.1) : (waves == 8 ? 5.7 : 4.6);
-    const double tile = fp8    ? (waves == 8 ? 1.65 : 1.83)
-                        : wide ? (waves == 8 ? 1.44 : 1.42) : (waves == 8 ? 1.3 : 0.95);
+    const double tile = fp8             ? (waves == 8 ? 1.65 : 1.83)
+                        : lanes && wide ? (waves == 8 ? 1.8 : 1.95)
+                        : lanes         ? (waves == 8 ? 1.25 : 1.22)
+                        : wide          ? (waves == 8 ? 1.44 : 1.42) : (waves == 8 ? 1.3 : 0.95);
     return start + tile * per +
            (parts > 1 ? 3.5 + 0.3 * parts + (wide ? 0.21 : 0.35) * mb * parts : 0.0);
   };
@@ -728,13 +736,20 @@ Cut cut_of(bool fp8, int nseq, int nheads, int kvh, int head_dim, int max_query_
     shape(four, 4, group);
     four.parts = 1;
     const long blocks = blocks_of(four, nseq, nheads, max_query_len);
-    const bool short_chain =
-        2L * max_keys <= 5L * max_query_len && (wide ? blocks <= 512 && tiles <= 16 : blocks <= 768);
-    if (c.parts == 1 ? blocks <= 256 || short_chain
-                     : blocks <= 512 && us(4, 1) < 0.95 * us(8, c.parts))
+    const bool own = 2L * max_keys <= 5L * max_query_len;
+    const bool short_chain = own && (wide ? blocks <= 512 && tiles <= 16 : blocks <= 768);
+    if (lanes          ? blocks <= (own || c.parts > 1 ? 512 : 256) && us(4, 1) < us(8, c.parts)
+        : c.parts == 1 ? blocks <= 256 || short_chain
+                       : blocks <= 512 && us(4, 1) < 0.95 * us(8, c.parts))
       c = four;
   }
   return c;
+}
+
+// Whether a wave's loads lie inside cache blocks and are found by the scalar unit: see the kernel.
+bool even_blocks(int block_size, int kvh, int head_dim, int bytes) {
+  return (block_size & (block_size - 1)) == 0 && block_size % (1024 / (head_dim * bytes)) == 0 &&
+         (long)kvh * head_dim * bytes < 1 << 24;
 }
 
 template <int HD, typename CT>
@@ -750,8 +765,7 @@ void launch(__hip_bfloat16* out, float* part_acc, float* part_ml, const __hip_bf
                        sl, scale * kLog2e, nheads, kvh, c.heads, block_size, shift, max_blocks,
                        c.parts, part_acc, part_ml);
   };
-  constexpr int kLoad = 1024 / (HD * sizeof(CT));   // rows of a wave's load
-  const bool even = shift >= 0 && block_size % kLoad == 0 && (long)kvh * HD * sizeof(CT) < 1 << 24;
+  const bool even = even_blocks(block_size, kvh, HD, sizeof(CT));
 #define GO(NW, EVEN) go(paged_prefill_tile_kernel<HD, CT, NW, EVEN>, kTurns<HD, CT, NW, EVEN>)
   if (c.waves == 8 && even) GO(8, true);
   else if (c.waves == 8) GO(8, false);
@@ -770,9 +784,10 @@ void launch(__hip_bfloat16* out, float* part_acc, float* part_ml, const __hip_bf
 // Waves of a workgroup << 8 | workgroups that a prompt's keys may be cut over (a function of shapes
 // only): 1, or the launch needs part_acc [parts, tokens, nheads, head_dim] and part_ml [parts, tokens,
 // nheads, 2].
-int prefill_tile_plan(bool fp8, int nseq, int nheads, int kvh, int head_dim, int max_query_len,
-                      int max_keys) {
-  const Cut c = cut_of(fp8, nseq, nheads, kvh, head_dim, max_query_len, max_keys);
+int prefill_tile_plan(bool fp8, int block_size, int nseq, int nheads, int kvh, int head_dim,
+                      int max_query_len, int max_keys) {
+  const Cut c = cut_of(fp8, even_blocks(block_size, kvh, head_dim, fp8 ? 1 : 2), nseq, nheads, kvh,
+                       head_dim, max_query_len, max_keys);
   return c.waves << 8 | c.parts;
 }
 
@@ -782,7 +797,8 @@ void launch_paged_prefill_tile(__hip_bfloat16* out, float* part_acc, float* part
                                const int* sl, float scale, int nseq, int nheads, int kvh,
                                int head_dim, int block_size, int max_blocks, int max_query_len,
                                int max_keys, hipStream_t stream) {
-  const Cut c = cut_of(false, nseq, nheads, kvh, head_dim, max_query_len, max_keys);
+  const Cut c = cut_of(false, even_blocks(block_size, kvh, head_dim, 2), nseq, nheads, kvh, head_dim,
+                       max_query_len, max_keys);
   auto go = [&](auto launch) {
     launch(out, part_acc, part_ml, q, kc, vc, bt, qsl, sl, scale, nseq, nheads, kvh, block_size,
            max_blocks, max_query_len, c, stream);
@@ -800,5 +816,6 @@ void launch_paged_prefill_tile_fp8(__hip_bfloat16* out, float* part_acc, float* 
                                    int max_keys, hipStream_t stream) {
   launch<128, unsigned char>(out, part_acc, part_ml, q, kc, vc, bt, qsl, sl, scale, nseq, nheads,
                              kvh, block_size, max_blocks, max_query_len,
-                             cut_of(true, nseq, nheads, kvh, 128, max_query_len, max_keys), stream);
+                             cut_of(true, even_blocks(block_size, kvh, 128, 1), nseq, nheads, kvh,
+                                    128, max_query_len, max_keys), stream);
 }

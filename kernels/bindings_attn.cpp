@@ -17,8 +17,8 @@ template <typename T>
 void launch_paged_prefill(T*, const T*, const T*, const T*, const int*,
                           const int*, const int*, float, int, int, int, int,
                           int, int, int, hipStream_t);
-int prefill_tile_plan(bool fp8, int nseq, int nheads, int kvh, int head_dim, int max_query_len,
-                      int max_keys);
+int prefill_tile_plan(bool fp8, int block_size, int nseq, int nheads, int kvh, int head_dim,
+                      int max_query_len, int max_keys);
 void launch_paged_prefill_tile(__hip_bfloat16*, float*, float*, const __hip_bfloat16*,
                                const __hip_bfloat16*, const __hip_bfloat16*, const int*,
                                const int*, const int*, float, int, int, int, int, int, int, int,
@@ -221,8 +221,8 @@ void paged_attention_prefill(torch::Tensor out, torch::Tensor q,
   const int max_keys = (int)std::min<int64_t>(max_seq_len, (int64_t)max_blocks * block_size);
   const int64_t parts =
       tiles && (!force_valu || k_cache.scalar_type() == at::ScalarType::Byte)
-          ? prefill_tile_plan(k_cache.scalar_type() == at::ScalarType::Byte, nseq, nheads, kvh,
-                              head_dim, (int)max_query_len, max_keys) & 255
+          ? prefill_tile_plan(k_cache.scalar_type() == at::ScalarType::Byte, block_size, nseq, nheads,
+                              kvh, head_dim, (int)max_query_len, max_keys) & 255
           : 1;
   torch::Tensor part_acc, part_ml;
   float *acc = nullptr, *ml = nullptr;
@@ -639,8 +639,14 @@ void register_attention_ops(pybind11::module& m) {
         "paged decode attention (CDNA4)");
   m.def("paged_attention_prefill", &paged_attention_prefill,
         "paged causal prefill attention (CDNA4)");
-  m.def("prefill_tile_plan", &prefill_tile_plan,
+  m.def("prefill_tile_plan",
+        [](bool fp8, int block_size, int nseq, int nheads, int kvh, int head_dim, int max_query_len,
+           int max_keys) {
+          TORCH_CHECK(block_size > 0 && nseq > 0 && kvh > 0 && nheads >= kvh && nheads % kvh == 0 &&
+                      (head_dim == 128 || (head_dim == 64 && !fp8)) && max_query_len > 0 && max_keys > 0);
+          return prefill_tile_plan(fp8, block_size, nseq, nheads, kvh, head_dim, max_query_len, max_keys);
+        },
         "how prompt attention is cut: waves of a workgroup << 8 | parts of the keys", pybind11::arg("fp8"),
-        pybind11::arg("nseq"), pybind11::arg("nheads"), pybind11::arg("kvh"), pybind11::arg("head_dim"),
-        pybind11::arg("max_query_len"), pybind11::arg("max_keys"));
+        pybind11::arg("block_size"), pybind11::arg("nseq"), pybind11::arg("nheads"), pybind11::arg("kvh"),
+        pybind11::arg("head_dim"), pybind11::arg("max_query_len"), pybind11::arg("max_keys"));
 }
