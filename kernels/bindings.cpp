@@ -50,7 +50,7 @@ void launch_gemm_ring_parts(__hip_bfloat16*, float*, const __hip_bfloat16*,
 bool gemm_ring_takes(int N, int K, int plan, bool gated);
 bool gemm_ring_reads_once(int M, int N, int K, int plan, bool gated);
 int gemm_ring_lora_cuts(int M, int K, int L, int PR, int plan);
-bool gemm_ring_lora_wins(long M, long N, long K);
+bool gemm_ring_lora_wins(long M, long N, long K, int rank);
 void launch_gemm_ring_lora(__hip_bfloat16*, float*, const __hip_bfloat16*, const __hip_bfloat16*,
                            int, int, int, int, float*, const __hip_bfloat16*, const int*, int, int,
                            int, hipStream_t);
@@ -1008,7 +1008,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("m"), py::arg("n"), py::arg("k"), py::arg("plan"), py::arg("gated") = false);
   m.def("decode_inputs", &decode_inputs, "a captured step's inputs from a packed host buffer");
   m.def("lora_product", &lora_product, "a product with its LoRA deltas, also gated");
-  m.def("gemm_ring_lora_wins", &gemm_ring_lora_wins, "whether the tiles take a product with adapters");
+  m.def("gemm_ring_lora_wins", &gemm_ring_lora_wins, "whether the tiles take a product with adapters",
+        py::arg("m"), py::arg("n"), py::arg("k"), py::arg("rank") = 16);
   m.def("gemm_ring_lora_cuts", &gemm_ring_lora_cuts,
         "parts of K of the adapters' shrink beside a product, 0: in a launch of its own");
   m.def("lora_tiles_win", &lora_tiles_win, "whether its deltas are added by the matrix unit");

@@ -439,12 +439,13 @@ int gemm_ring_lora_cuts(int M, int K, int L, int PR, int plan) {
 // Whether these tiles take a product that has adapters, whatever takes it without them: beside other
 // products the shrink is a launch of its own, the deltas go over their rounded results, and where K is
 // cut the sum of the parts is one more; here it is two launches, three where the shrink has no room beside
-// the product (gemm_ring_lora_cuts: many adapters or tokens, high ranks).  The rule sees sizes of the product
-// only.  us with the deltas, otherwise | here, 4 adapters of rank 16 (captured, cold weights), N x K: rows
+// the product (gemm_ring_lora_cuts: many adapters or tokens, high ranks).  Of the adapters the rule sees their
+// rank, for one row of many columns.  us with the deltas, otherwise | here, 4 adapters of rank 16 (captured, cold weights), N x K: rows
 //   up to 16 rows: 6144 x 4096 2 19.2 | 15.8, 16 21.7 | 16.8; 28672 x 4096 gated 2 49.7 | 45.3; 4096 x 14336
 //    8 30.5 | 26.6; 2048 x 2048 12 11.3 | 8.8; 57344 x 8192 gated 2 174 | 163; 768 x 768 2 8.8 | 9.0; not
 //    4096 x 1792 12.3 | 13.7 (too short to be cut, 64 workgroups); of one row 6144 x 4096 16.4 | 15.0, 2048
-//    x 2048 9.3 | 7.8, but 4096 x 4096 12.5 | 13.3, 57344 x 8192 153 | 161;
+//    x 2048 9.3 | 7.8, but 4096 x 4096 12.5 | 13.3, 57344 x 8192 153 | 161; of one row and rank 8, whose
+//    expand is little, gated 16384 x 2048 18.8 | 19.5, 28672 x 4096 45.9 | 47.5, 7168 x 4096 16.9 | 15.7;
 //   17 to 128: 2048 x 2048 64 16.2 | 9.2; 3072 x 2048 32 15.1 | 10.1, 65 20.7 | 12.7; 16384 x 2048 gated
 //    128 35.5 | 32.2; 28672 x 4096 gated 80 81.8 | 62.7, 128 73.2 | 65.9, 160 76.4 | 82.8; 57344 x 8192
 //    gated 65 207 | 172;
@@ -454,11 +455,12 @@ int gemm_ring_lora_cuts(int M, int K, int L, int PR, int plan) {
 //    400 50.5 | 55.4; 16384 x 2048 gated 301 46.8 | 48.8.
 // (Of other ranks and numbers of adapters: as far or further apart but for rank 64 at 400 to 512 rows,
 // 0.98 to 1.03 of the others.)
-bool gemm_ring_lora_wins(long M, long N, long K) {
+bool gemm_ring_lora_wins(long M, long N, long K, int rank) {
   if (!fits(M, N, K, false)) return false;
   if (M <= 64 ? gemm_ring_wins(M, N, K, false) : gemm_tiles_route(M, N, K) != 0) return true;
   const long size = N * K;
-  if (M == 1) return size <= 6000000 || (size <= 300000000 && (K >= 8192 || N > 4096));
+  if (M == 1)
+    return size <= 6000000 || (size <= 300000000 && (K >= 8192 || (N > 4096 && (rank > 8 || N < 16384))));
   if (M <= 16) return K <= 1024 || K >= 2048 || N > 4096;
   if (M <= 128) return true;
   if (M <= 256) return size <= 34000000 || K >= 8192;

@@ -187,6 +187,14 @@ def test_few_rows_are_not_asked_for():
                 assert not ops._tiles_take(m, n, k)
 
 
+# adapters of rank 8 on one row leave little to add up
+@pytest.mark.parametrize(("m", "n", "k", "ranks"), [
+    (1, 28672, 4096, {16, 32, 64}), (1, 16384, 2048, {16, 32, 64}), (2, 28672, 4096, {8, 16, 32, 64}),
+    (1, 7168, 4096, {8, 16, 32, 64}), (1, 10240, 8192, {8, 16, 32, 64}), (1, 4096, 4096, set())])
+def test_products_with_adapters_by_rank(m, n, k, ranks):
+    assert {r for r in ops.LORA_RANKS if ops._lora_tiles_take(m, n, k, r)} == ranks
+
+
 # waves, and those that K is dealt to: forms within 4 % of the fastest at sizes around every line of the rule
 @pytest.mark.parametrize(("bits", "mode", "n", "k", "forms"), [
     (4, 0, 128, 8192, {0x88}), (4, 0, 1024, 28672, {0x88}), (4, 0, 2048, 8192, {0x84, 0x88}),

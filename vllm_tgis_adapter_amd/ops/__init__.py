@@ -304,9 +304,9 @@ def _tiles_take(m: int, n: int, k: int) -> bool:
             and m > _gemm_max_m())
 
 
-def _lora_tiles_take(m: int, n: int, k: int) -> bool:
+def _lora_tiles_take(m: int, n: int, k: int, rank: int = 16) -> bool:
     """The same of a product with adapters."""
-    return (_C.gemm_ring_lora_wins(m, n, k)
+    return (_C.gemm_ring_lora_wins(m, n, k, rank)
             and (m <= _gemm_max_m() if m <= 64 else m > _gemm_max_m()))
 
 
@@ -591,7 +591,8 @@ def lora_product(
     product and the deltas, or where tensors do not suit."""
     given = weight if y is None else y
     rows, width = x.shape[0], given.shape[0 if y is None else 1]
-    if not native_enabled(x) or (y is None and not _lora_tiles_take(rows, width, x.shape[1])):
+    if not native_enabled(x) or (
+            y is None and not _lora_tiles_take(rows, width, x.shape[1], b_stack.shape[2])):
         return None
     if (given.dtype != torch.bfloat16 or not given.is_contiguous()
             or width % 2 or not slots.is_contiguous() or not scales.is_contiguous()
