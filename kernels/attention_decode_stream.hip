@@ -14,7 +14,7 @@
 // The keys of a sequence are cut over up to npart workgroups (a pure function of
 // shapes, so that a captured launch stays valid) of at least four tiles each, the
 // four waves merge in LDS, and only a sequence that was cut goes through the merge
-// kernel.  Of many short sequences a wave takes a key head by itself (decode_alone_tiles): the
+// kernel.  Of many short sequences a wave takes a key head by itself (alone_tiles): the
 // lengths say so on the device, so that a captured launch serves both.
 //
 // Measured (MI355X, 32/8 heads of 128, two layers with their cache writes): 512
@@ -218,7 +218,7 @@ __global__ __launch_bounds__(256, 2) void paged_decode_stream_kernel(
     const int* __restrict__ seq_lens,       // [nseq]
     const float scale_log2, const int nheads, const int kvh, const int group,
     const int block_size, const int block_shift, const int max_blocks,
-    const int alone_tiles) {   // see decode_alone_tiles
+    const int alone_tiles) {   // see the rule of that name
   using W = Walk<HD, CT>;
   const int seq = blockIdx.x, part = blockIdx.z;
   int kv_head = blockIdx.y;
@@ -404,10 +404,19 @@ __global__ __launch_bounds__(HD) void decode_stream_merge_kernel(
 // 27.3, 29.7, 33.4, 33.5; 64 x 30 26.4 | 26.5, 31.6; 64/8 heads, 81 x 22 35.3 | 28.8, 30.6, 30.5; heads of
 // 64, 512 x 50 48.5 | 48.1, 42.7, 39.8, 39.7.  (The workgroups that work first instead of every fourth:
 // the same there, and 512 x 520 0.8 % slower.)
-int decode_alone_tiles(int nseq, int kvh) {
+// What there is to win grows with the queries of a head, whose sums the waves would meet over, and shrinks
+// with smaller tiles (heads of 64, e4m3), of which more workgroups are resident.  20 layers in turn, so many
+// that no cache holds them, tables of 2048 keys; us of a launch, a head a workgroup | a wave, sequences x
+// keys (up to), below the lines and past them: 32/8 heads of 64, 80 x 60 7.2 | 7.9, 192 x 120 in 4 tiles
+// 9.8 | 10.5, 320 x 90 12.6 | 11.1; e4m3, 80 x 60 8.6 | 9.6, 128 x 60 11.9 | 10.2; one query a head, 32/32 of 128,
+// 24 x 60 10.5 | 11.7, 48 x 180 22.3 | 25.7, 12/12 of 64, 64 x 60 6.7 | 9.1, 192 x 120 12.5 | 13.5.  With these lines
+// none of 1352 such launches is 3 % slower than a head a workgroup, and the mean is 0.875 of it.
+int alone_tiles(int nseq, int kvh, int group, int head_dim, bool fp8) {
   if (kvh % kWaves != 0) return -1;
   const long heads = (long)nseq * kvh;
-  return heads >= 1536 ? 4 : heads >= 640 ? 2 : -1;
+  if (group < 4) return heads >= 3072 ? 4 : heads >= (head_dim == 64 ? 1344 : 2560) ? 2 : -1;
+  if (head_dim == 64) return heads >= 2048 ? 4 : heads >= 1280 ? 2 : -1;
+  return heads >= 1536 ? 4 : heads >= (fp8 ? 896 : 640) ? 2 : -1;
 }
 
 template <int HD, typename CT>
@@ -418,7 +427,8 @@ void launch(__hip_bfloat16* out, float* part_acc, float* part_ml, const __hip_bf
   int shift = -1;
   if ((block_size & (block_size - 1)) == 0) shift = __builtin_ctz(block_size);
   // (a wave's results of a head by itself are stored by 8 bytes, a workgroup's one by one)
-  const int alone = reinterpret_cast<uintptr_t>(out) % 8 == 0 ? decode_alone_tiles(nseq, kvh) : -1;
+  const int alone = reinterpret_cast<uintptr_t>(out) % 8 == 0
+                        ? alone_tiles(nseq, kvh, nheads / kvh, HD, sizeof(CT) == 1) : -1;
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(nseq, kvh, npart), dim3(256), 0, stream, out, part_acc, part_ml,
                        q, kc, vc, bt, sl, scale * kLog2e, nheads, kvh, nheads / kvh, block_size,
@@ -432,6 +442,10 @@ void launch(__hip_bfloat16* out, float* part_acc, float* part_ml, const __hip_bf
 }
 
 }  // namespace
+
+int decode_alone_tiles(int nseq, int kvh, int group, int head_dim, bool fp8) {
+  return alone_tiles(nseq, kvh, group, head_dim, fp8);
+}
 
 // Workgroups a sequence and key head may be cut over: enough for some six per CU
 // where the batch alone has fewer (twice as many measured the same), at least four

@@ -17,6 +17,7 @@ template <typename T>
 void launch_paged_prefill(T*, const T*, const T*, const T*, const int*,
                           const int*, const int*, float, int, int, int, int,
                           int, int, int, hipStream_t);
+int decode_alone_tiles(int nseq, int kvh, int group, int head_dim, bool fp8);
 int prefill_tile_plan(bool fp8, int block_size, int nseq, int nheads, int kvh, int head_dim,
                       int max_query_len, int max_keys);
 void launch_paged_prefill_tile(__hip_bfloat16*, float*, float*, const __hip_bfloat16*,
@@ -639,6 +640,10 @@ void register_attention_ops(pybind11::module& m) {
         "paged decode attention (CDNA4)");
   m.def("paged_attention_prefill", &paged_attention_prefill,
         "paged causal prefill attention (CDNA4)");
+  m.def("decode_alone_tiles", &decode_alone_tiles,
+        "up to how many tiles of 32 keys a head is a wave's in decode attention, -1: never",
+        pybind11::arg("nseq"), pybind11::arg("kvh"), pybind11::arg("group"), pybind11::arg("head_dim"),
+        pybind11::arg("fp8"));
   m.def("prefill_tile_plan",
         [](bool fp8, int block_size, int nseq, int nheads, int kvh, int head_dim, int max_query_len,
            int max_keys) {

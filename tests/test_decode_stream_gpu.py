@@ -104,6 +104,8 @@ def test_block_ids_past_the_end_say_nothing(fp8, block, lens, width):
     (8, 8, 128, 192, 512),     # 1536: up to four tiles, uncut
     (4, 3, 64, 400, 9),
     (6, 2, 128, 300, 9),       # key heads are no whole workgroups: never
+    (8, 4, 128, 112, 40), (8, 4, 64, 160, 40), (8, 4, 64, 256, 40), (4, 1, 128, 640, 12),
+    (4, 1, 64, 336, 40), (8, 2, 128, 384, 12),
 ])
 def test_heads_of_short_sequences_are_a_waves_each(fp8, kvh, group, hd, nseq, width):
     """Lengths on both sides of two and four tiles of 32 keys beside each other."""
