@@ -436,10 +436,19 @@ int gemm_panel_plan(int M, int N, int K, int qbits) {
 
 // The plan of a product of up to 64 rows by a panel, 0: the streaming kernels, which are as fast or
 // faster for small matrices of short K and, in int8, up to 11 rows (us, streaming | panels: 33 rows,
-// int8 4096 x 1024 6.2 | 7.2, 2048 x 2048 7.5 | 7.2, 8192 x 1024 9.3 | 6.5; 17 rows 4096 x 4096 8.7 | 8.8, 4
-// bits 8.3 | 9.4, 16384 x 2048 9.7 | 10.1, 4 bits 13.1 | 10.5; 9 rows 6144 x 4096 9.8 | 10.4, 4 bits 10.4 |
+// int8 4096 x 1024 6.2 | 7.2, 2048 x 2048 7.5 | 7.2, 8192 x 1024 9.3 | 6.5; 17 rows 4 bits 4096 x 4096
+// 8.3 | 9.4, 16384 x 2048 13.1 | 10.5; 9 rows 6144 x 4096 9.8 | 10.4, 4 bits 10.4 |
 // 11.3; 4 bits 2048 x 8192, 2 rows 9.9 | 9.1, 3584 x 8192 12.8 | 14.0, int8 2048 x 8192 8.3 | 8.5; int8 57344 x 8192, 8 rows 82 | 90, 14 rows
 // 101 | 93, 8192 x 28672, 2 rows 52 | 46).
+// A panel takes as long for 2 rows as for 32, the streaming kernels for 16 (and for 32, nearly):
+//  - int8, 17 to 27 rows are as fast there but where W is so small that waves work alone in them (2^24: 1280 x 8192
+//    0.75 of it, 512 x 14336 0.64; 1536 x 14336 11.2 | 12.2, 57344 x 7168 76 | 91, 6144 x 14336 22.3 | 24.3, but 4096 x
+//    14336 1.00 to 0.97), shorter K up to 23 rows; from 28 on not where W is largest (57344 x 7168 86 | 93) or K is
+//    longest and columns few (768 x 28672 17.2 | 18.2);
+//  - up to 8 rows, many columns of long K: 4 bits 28672 x 8192 47 | 54, 16384 x 8192 27.7 | 31.0, but 16384 x 28672
+//    80 | 83, 8 rows 0.86 of it; int8 14336 x 28672 77 | 89.
+// Over 4698 products of 2 to 64 rows, 17 widths and 13 K, three are 3 % slower than streaming (by 4 at most), the
+// mean is 0.90 of it.
 int gemm_panel_few_plan(int M, int N, int K, int qbits) {
   const long size = (long)N * K;
   bool takes;
@@ -447,9 +456,16 @@ int gemm_panel_few_plan(int M, int N, int K, int qbits) {
   else if (M > 32) takes = K >= 2048 || size >= 8000000;
   else if (qbits == 4 && M > 16) takes = K >= 8192 || size >= 20000000;
   else if (qbits == 4)
-    takes = (K >= 8192 && (N <= 2048 || size >= 50000000)) || (M > 8 && size >= 100000000);
-  else if (M > 16) takes = K >= 8192 || (K >= 4096 && size >= 20000000);
-  else takes = K >= 16384 || (M > 11 && size >= 50000000);
+    takes = (K >= 8192 && (N <= 2048 || (size >= 50000000 && (M > 8 || N <= 12288 || K >= 16384)))) ||
+            (M > 8 && size >= 100000000);
+  else if (M > 16)
+    takes = (K >= 7168 && size <= 1 << 24) || (K >= 8192 && N >= 3584 && N <= 5120) ||
+            (M > 23 && K >= 4096 && K < 8192 && size >= 20000000 && size < 200000000 &&
+             (M > 27 || N < 14336)) ||
+            (M > 27 && K >= 8192 && (K < 16384 || N > 2048));
+  else
+    takes = (K >= 16384 && (M > 6 || size <= 300000000)) ||
+            (M > (K >= 5120 ? 11 : 13) && size >= 50000000);
   float us;
   return takes ? few_plan(M, N, K, qbits, false, us) : 0;
 }
@@ -518,14 +534,23 @@ void launch_gemm_block_q(__hip_bfloat16* y, float* part, const __hip_bfloat16* x
 // do (us, streaming and gate | gated panel, captured, int8: 28672 x 4096, 8 rows 27.9 | 26.4, 32 rows
 // 31.2 | 27.9, 64 46.5 | 31.6; 16384 x 2048, 8 rows 11.7 | 9.9, 32 13.1 | 10.1; 4096 x 1024, 8 rows 5.9 | 6.1, 33
 // rows 8.7 | 6.9; 4 bits 28672 x 4096, 2 rows 26.8 | 27.6, 4 rows 27.1 | 26.5, 16 rows 34.0 | 26.3).
+// Few rows leave the gate little to save: not int8 up to 9 rows of long K, of few columns, or of large W (2 N x
+// K: 57344 x 5120 53 | 71, 28672 x 7168 39 | 46, 10240 x 3584 12.6 | 14.0), nor 17 to 31 of the largest (57344 x 5120, 17
+// rows 63 | 74), nor 4 bits of few columns, which all of K leaves CUs without (10240 x 3584, 10 rows 13.7 | 15.8, 14336 x
+// 4096, 4 rows 16.4 | 18.1, 10 rows 18.3 | 18.2).  Of 4140 gated products twelve are 3 % slower than streaming and
+// gate (one by 10, others by 7 at most), the mean is 0.89.
 int gemm_panel_gated_plan(int M, int N, int K, int qbits) {
   if (M < 2 || N % 128 != 0 || K % 128 != 0 || (long)(N + 128) * K >= 1L << 32) return 0;
   float us, plain;
   int plan;
   if (M <= 64) {
     const long size = 2L * N * K;
-    if ((size < 24000000 && (K > 1024 || M <= 32)) || (qbits == 4 && M < 4) ||
-        (qbits == 8 && M < 12 && size >= 300000000))
+    if (size < 24000000 && (K > 1024 || M <= 32)) return 0;
+    if (qbits == 4
+            ? M < 4 || (K >= 3584 && 2 * N <= 16384 && M < (2 * N <= 12288 ? 17 : 10))
+            : (M < 10 && (size > 120000000 || K > 4096 || 2 * N < 14336)) ||
+                  (M < 24 && (M < 12 || M > 16) && size >= 140000000) ||
+                  (M > 16 && M < 32 && K >= 5120 && size >= 200000000))
       return 0;
     plan = few_plan(M, 2 * N, K, qbits, true, us);
     few_plan(M, 2 * N, K, qbits, false, plain);

@@ -187,6 +187,24 @@ def test_few_rows_are_not_asked_for():
                 assert not ops._tiles_take(m, n, k)
 
 
+# both sides of every line, where one way is at least 4 % faster; n: of [gate; up] where it is gated
+@pytest.mark.parametrize(("bits", "gated", "m", "n", "k", "panel"), [
+    (8, False, 17, 1280, 8192, True), (8, False, 17, 6144, 14336, False), (8, False, 20, 57344, 7168, False),
+    (8, False, 28, 57344, 7168, False), (8, False, 24, 5120, 8192, True), (8, False, 28, 768, 28672, False),
+    (8, False, 17, 1280, 14336, False), (8, False, 28, 6144, 14336, True),
+    (8, False, 2, 14336, 28672, False), (8, False, 2, 6144, 28672, True), (8, False, 12, 57344, 2560, False),
+    (8, False, 14, 28672, 2560, True), (4, False, 2, 28672, 8192, False), (4, False, 10, 28672, 8192, True),
+    (4, False, 2, 8192, 8192, True), (4, False, 8, 16384, 28672, True),
+    (8, True, 2, 57344, 5120, False), (8, True, 4, 14336, 4096, True), (8, True, 6, 28672, 7168, False),
+    (8, True, 3, 10240, 3584, False), (8, True, 17, 57344, 5120, False), (8, True, 32, 57344, 3584, True),
+    (8, True, 17, 14336, 7168, True), (4, True, 10, 10240, 3584, False), (4, True, 4, 14336, 4096, False),
+    (4, True, 12, 14336, 4096, True), (4, True, 4, 28672, 2560, True)])
+def test_few_rows_take_panels_where_they_are_faster(bits, gated, m, n, k, panel):
+    plan = (ops._C.gemm_panel_gated_plan(m, n // 2, k, bits) if gated
+            else ops._C.gemm_panel_few_plan(m, n, k, bits))
+    assert (plan > 0) == panel
+
+
 # adapters of rank 8 on one row leave little to add up
 @pytest.mark.parametrize(("m", "n", "k", "ranks"), [
     (1, 28672, 4096, {16, 32, 64}), (1, 16384, 2048, {16, 32, 64}), (2, 28672, 4096, {8, 16, 32, 64}),
