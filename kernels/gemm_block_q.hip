@@ -447,8 +447,7 @@ int gemm_panel_plan(int M, int N, int K, int qbits) {
 //    longest and columns few (768 x 28672 17.2 | 18.2);
 //  - up to 8 rows, many columns of long K: 4 bits 28672 x 8192 47 | 54, 16384 x 8192 27.7 | 31.0, but 16384 x 28672
 //    80 | 83, 8 rows 0.86 of it; int8 14336 x 28672 77 | 89.
-// Over 4698 products of 2 to 64 rows, 17 widths and 13 K, three are 3 % slower than streaming (by 4 at most), the
-// mean is 0.90 of it.
+// Over 4698 products of 2 to 64 rows, 17 widths and 13 K, one is 3 % slower than streaming, the mean is 0.90 of it.
 int gemm_panel_few_plan(int M, int N, int K, int qbits) {
   const long size = (long)N * K;
   bool takes;
@@ -537,8 +536,8 @@ void launch_gemm_block_q(__hip_bfloat16* y, float* part, const __hip_bfloat16* x
 // Few rows leave the gate little to save: not int8 up to 9 rows of long K, of few columns, or of large W (2 N x
 // K: 57344 x 5120 53 | 71, 28672 x 7168 39 | 46, 10240 x 3584 12.6 | 14.0), nor 17 to 31 of the largest (57344 x 5120, 17
 // rows 63 | 74), nor 4 bits of few columns, which all of K leaves CUs without (10240 x 3584, 10 rows 13.7 | 15.8, 14336 x
-// 4096, 4 rows 16.4 | 18.1, 10 rows 18.3 | 18.2).  Of 4140 gated products twelve are 3 % slower than streaming and
-// gate (one by 10, others by 7 at most), the mean is 0.89.
+// 4096, 4 rows 16.4 | 18.1, 10 rows 18.3 | 18.2).  Of 4140 gated products nine are 3 % slower than streaming and
+// gate (57344 x 1536, 2 rows, by 10, others by 5 at most), the mean is 0.89.
 int gemm_panel_gated_plan(int M, int N, int K, int qbits) {
   if (M < 2 || N % 128 != 0 || K % 128 != 0 || (long)(N + 128) * K >= 1L << 32) return 0;
   float us, plain;
