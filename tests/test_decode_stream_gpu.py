@@ -99,13 +99,14 @@ def test_block_ids_past_the_end_say_nothing(fp8, block, lens, width):
 
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize(("kvh", "group", "hd", "nseq", "width"), [
-    (8, 4, 128, 80, 40),       # 640 heads: up to two tiles a wave's each, sequences are cut
-    (8, 1, 64, 81, 16),
+    (8, 4, 128, 80, 40),       # 640 heads: up to two tiles a wave's each (bf16), sequences are cut
+    (8, 1, 64, 81, 16),        # never
     (8, 8, 128, 192, 512),     # 1536: up to four tiles, uncut
     (4, 3, 64, 400, 9),
     (6, 2, 128, 300, 9),       # key heads are no whole workgroups: never
-    (8, 4, 128, 112, 40), (8, 4, 64, 160, 40), (8, 4, 64, 256, 40), (4, 1, 128, 640, 12),
-    (4, 1, 64, 336, 40), (8, 2, 128, 384, 12),
+    # two tiles, four, of other heads and types
+    (8, 4, 128, 112, 40), (8, 4, 64, 160, 40), (4, 1, 128, 640, 12), (4, 1, 64, 336, 40),
+    (8, 4, 64, 256, 40), (8, 2, 128, 384, 12),
 ])
 def test_heads_of_short_sequences_are_a_waves_each(fp8, kvh, group, hd, nseq, width):
     """Lengths on both sides of two and four tiles of 32 keys beside each other."""
@@ -136,14 +137,14 @@ def test_heads_of_short_sequences_are_a_waves_each(fp8, kvh, group, hd, nseq, wi
 @pytest.mark.parametrize(("dim", "off"), [(64, 1), (128, 2), (128, 3), (128, 4)])
 def test_results_off_an_8_byte_boundary_are_stored_one_by_one(fp8, dim, off):
     """Short sequences, so many that elsewhere a wave has a key head; `off` results into the
-    buffer a workgroup does, as in batches of half the size, whose bits these are."""
+    buffer a workgroup does, as in batches of a quarter of the size, whose bits these are."""
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
     from vllm_tgis_adapter_amd import ops
 
-    lens = [(17, 33, 50, 64)[i % 4] for i in range(80)]
+    lens = [(17, 33, 50, 64)[i % 4] for i in range(160)]
     kc, vc, tables = (t.cuda() for t in _caches(lens, 16, 8, dim, fp8, 7, 4))
-    q = torch.randn(80, 32, dim, generator=torch.Generator().manual_seed(8)).bfloat16().cuda()
+    q = torch.randn(160, 32, dim, generator=torch.Generator().manual_seed(8)).bfloat16().cuda()
     seq_lens = torch.tensor(lens, dtype=torch.int32, device="cuda")
 
     def decode(out, rows):
@@ -151,11 +152,13 @@ def test_results_off_an_8_byte_boundary_are_stored_one_by_one(fp8, dim, off):
                                       dim ** -0.5)
         return out
 
-    halves = torch.cat([decode(torch.empty_like(q[:40]), slice(i, i + 40)) for i in (0, 40)])
+    assert ops._C.decode_alone_tiles(160, 8, 4, dim, fp8) == 2
+    assert ops._C.decode_alone_tiles(40, 8, 4, dim, fp8) == -1
+    few = torch.cat([decode(torch.empty_like(q[:40]), slice(i, i + 40)) for i in range(0, 160, 40)])
     whole = torch.full((q.numel() + 8,), 7.0, dtype=q.dtype, device="cuda")
-    got = decode(whole[off:off + q.numel()].view_as(q), slice(0, 80))
+    got = decode(whole[off:off + q.numel()].view_as(q), slice(0, 160))
     if off % 4:
-        assert torch.equal(got, halves)
+        assert torch.equal(got, few)
     else:   # on such a boundary; sums in another order, rounded to 8 bits
-        assert (got - halves).abs().max() <= 2 ** -8 * halves.abs().max()
+        assert (got - few).abs().max() <= 2 ** -8 * few.abs().max()
     assert (whole[:off] == 7).all() and (whole[off + q.numel():] == 7).all()
